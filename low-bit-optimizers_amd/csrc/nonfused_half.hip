@@ -17,6 +17,13 @@
 // The maxima of the new second moment over rows and columns are taken with integer atomics on the
 // float images of the half values in a float work array (a maximum of half values is a half value);
 // a last small kernel writes them out as halfs.
+//
+// Both passes are bound by their arithmetic (eleven roundings per element in the first), so what counts is
+// instructions per element.  Halfs stay in pairs, roundings are packed, products read halfs directly (below),
+// maxima over a lane's columns stay in registers through its passes instead of going to LDS one by one,
+// and addresses advance by one addition each.  Four decoder layers of width 4096 (8.1e8 values), update +
+// second pass: 1603 + 779 us (78 and 38 issue slots per element) -> 1240 + 498 us; 970 + 390 us would be the
+// memory system's.  Six waves per SIMD: with five the update takes 1295 us, with seven it spills.
 #include "rank1_tiles.hpp"
 
 namespace lpmm {
@@ -25,7 +32,6 @@ typedef _Float16 h16;
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ v4h load_h4(const h16 *p) { return __builtin_nontemporal_load(reinterpret_cast<const v4h *>(p)); }
-__device__ __forceinline__ void store_h4(h16 *p, v4h v) { __builtin_nontemporal_store(v, reinterpret_cast<v4h *>(p)); }
 
 // One rounding to half (nearest even, subnormals kept), as at the end of every op of the chain.  The
 // float result is pinned in a register first: otherwise the compiler merges the producing operation
@@ -38,67 +44,201 @@ __device__ __forceinline__ float rh(float x)
     return (float)(h16)x;
 }
 
-__device__ __forceinline__ void widen8(const v4h &a, const v4h &b, float (&o)[kEltsPerLane])
+// The chain works on pairs of halfs in one register each: two float results go back to halfs in one
+// instruction (v_cvt_pk_f16_f32), and a product or sum takes its half operands out of the pairs by itself
+// (v_fma_mix_f32: float arithmetic, one rounding, any operand a half of a register).  The compiler forms
+// that instruction from an fma of widened halfs only, so products and sums are written as fma(a, b, -0)
+// and fma(a, 1, b) -- exactly a * b and a + b, signs of zeros included -- with the two constants hidden
+// from it.  A rounding to half then costs half an instruction instead of two conversions; the update pass
+// is bound by its arithmetic.
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+typedef uint16_t v2u __attribute__((ext_vector_type(2)));
+constexpr int kPairs = kEltsPerLane / 2;
+
+struct MixConst {
+    float one, neg_zero;
+};
+
+__device__ __forceinline__ MixConst mix_const()
 {
-    o[0] = (float)a.x; o[1] = (float)a.y; o[2] = (float)a.z; o[3] = (float)a.w;
-    o[4] = (float)b.x; o[5] = (float)b.y; o[6] = (float)b.z; o[7] = (float)b.w;
+    MixConst c = {1.0f, -0.0f};
+    asm("" : "+v"(c.one), "+v"(c.neg_zero));
+    return c;
 }
 
-__device__ __forceinline__ v4h narrow4(const float (&x)[kEltsPerLane], int h)
+__device__ __forceinline__ float mix_mul(h16 a, float b, const MixConst &c) { return __builtin_fmaf((float)a, b, c.neg_zero); }
+__device__ __forceinline__ float mix_add(h16 a, float b, const MixConst &c) { return __builtin_fmaf((float)a, c.one, b); }
+
+// rh of two values; see rh for the pins
+__device__ __forceinline__ v2h round2(float a, float b)
 {
-    const v4h r = {(h16)x[4 * h], (h16)x[4 * h + 1], (h16)x[4 * h + 2], (h16)x[4 * h + 3]};
+    asm("" : "+v"(a), "+v"(b));
+    const v2f t = {a, b};
+    return __builtin_convertvector(t, v2h);
+}
+
+__device__ __forceinline__ v2h abs2(v2h x)
+{
+    return __builtin_bit_cast(v2h, __builtin_bit_cast(uint32_t, x) & 0x7fff7fffu);
+}
+
+// Larger of two halfs each, a NaN left out as by fmaxf.  (The compiler's own maximum canonicalises both
+// operands first; these come from a conversion and are canonical.)
+__device__ __forceinline__ v2h max2(v2h a, v2h b)
+{
+    v2h r;
+    asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
 
-// v.mul_(beta2).addcmul_(g, g, value=1 - beta2) on half tensors
-__device__ __forceinline__ void half_second_moment(float &v, float g, const NfHyper &h)
+// largest of a lane's eight values and zero; ABS: of their magnitudes (otherwise no value is negative)
+template <bool ABS>
+__device__ __forceinline__ float max8(const v2h (&x)[kPairs])
 {
-    v = rh(v * h.b2);
-    v = rh(v + (h.w2 * g) * g);
+    const v2h a = ABS ? max2(abs2(x[0]), abs2(x[1])) : max2(x[0], x[1]);
+    const v2h b = ABS ? max2(abs2(x[2]), abs2(x[3])) : max2(x[2], x[3]);
+    const v2h r = max2(a, b);
+    return fmaxf(fmaxf((float)r.x, (float)r.y), 0.0f);
 }
 
-// x / d for a denominator that may be zero: float16 rounds the default eps of 1e-8 to zero, so the
-// denominator of an element whose second moment is zero is zero and the parameter becomes infinite or
-// NaN, as in the reference.  The quotient of the approximate reciprocal is already the IEEE result then
-// (x * inf); elsewhere the residual correction makes it the correctly rounded quotient (div_fast).
-__device__ __forceinline__ float div_maybe_zero(float x, float d)
+// maxima and minima of non-negative halfs are those of their bit patterns
+__device__ __forceinline__ v2h max2_bits(v2h a, v2h b)
 {
-    const float rc = __builtin_amdgcn_rcpf(d);
+    return __builtin_bit_cast(v2h, __builtin_elementwise_max(__builtin_bit_cast(v2u, a), __builtin_bit_cast(v2u, b)));
+}
+__device__ __forceinline__ v2h min2_bits(v2h a, v2h b)
+{
+    return __builtin_bit_cast(v2h, __builtin_elementwise_min(__builtin_bit_cast(v2u, a), __builtin_bit_cast(v2u, b)));
+}
+
+__device__ __forceinline__ void pairs_of(const v4h &a, const v4h &b, v2h (&o)[kPairs])
+{
+    o[0] = a.xy; o[1] = a.zw; o[2] = b.xy; o[3] = b.zw;
+}
+
+// a lane's eight values of a group: four at p, four 64 further on
+__device__ __forceinline__ void store_pairs(h16 *p, const v2h (&x)[kPairs])
+{
+    typedef uint32_t v2w __attribute__((ext_vector_type(2)));
+    const v2w lo = {__builtin_bit_cast(uint32_t, x[0]), __builtin_bit_cast(uint32_t, x[1])};
+    const v2w hi = {__builtin_bit_cast(uint32_t, x[2]), __builtin_bit_cast(uint32_t, x[3])};
+    __builtin_nontemporal_store(lo, reinterpret_cast<v2w *>(p));
+    __builtin_nontemporal_store(hi, reinterpret_cast<v2w *>(p + 64));
+}
+
+// v.mul_(beta2).addcmul_(g, g, value=1 - beta2) on half tensors
+__device__ __forceinline__ v2h half_second_moment(v2h v, v2h g, const NfHyper &h, const MixConst &c)
+{
+    v = round2(mix_mul(v.x, h.b2, c), mix_mul(v.y, h.b2, c));
+    const float ax = mix_mul(g.x, mix_mul(g.x, h.w2, c), c), ay = mix_mul(g.y, mix_mul(g.y, h.w2, c), c);
+    return round2(mix_add(v.x, ax, c), mix_add(v.y, ay, c));
+}
+
+// m.lerp_(g, 1 - beta1); NEAR: the weight lies below 0.5 (lerp_w)
+template <bool NEAR>
+__device__ __forceinline__ float half_lerp(h16 m, h16 g, float w, const MixConst &c)
+{
+    const float d = __builtin_fmaf((float)g, c.one, -(float)m);
+    return NEAR ? __builtin_fmaf(w, d, (float)m) : __builtin_fmaf(w - 1.0f, d, (float)g);
+}
+
+// x / d, correctly rounded (div_fast).  ZERO: the denominator may be zero: float16 rounds the default eps of
+// 1e-8 to zero, so the denominator of an element whose second moment is zero is zero and the parameter
+// becomes infinite or NaN, as in the reference; the quotient of the approximate reciprocal is already the
+// IEEE result then (x * inf).
+template <bool ZERO>
+__device__ __forceinline__ float half_quotient(float x, h16 dh)
+{
+    const float d = (float)dh, rc = __builtin_amdgcn_rcpf(d);
     const float q = x * rc;
     const float r = __builtin_fmaf(-q, d, x);
     const float c = __builtin_fmaf(r, rc, q);
-    return d == 0.0f ? q : c;
+    return ZERO && d == 0.0f ? q : c;
 }
 
-// One element of the chain; p, m and v (halfs held as floats) are updated in place.
-__device__ __forceinline__ void half_elt(float &p, float g, float &m, float &v, const NfHyper &h)
+// The parameter of two elements from their updated moments.  The root of a half rounded to half lies at
+// least 0.5 ulp of a float away from a tie, and the hardware's float root (1 ulp) rounds to the same half as
+// the correctly rounded one for every half (all of them are compared by the tests).
+template <bool ZERO>
+__device__ __forceinline__ v2h half_param(v2h p, v2h m, v2h v, const NfHyper &h, const MixConst &c)
 {
-    const float pi = rh(p * h.decay);
-    m = rh(lerp_w(m, g, h.w1));
-    half_second_moment(v, g, h);
-    float d = rh(sqrt_fast(v));
-    d = rh(div_by_rc(d, h.bc2_sqrt, h.rbc2_sqrt));
-    d = rh(d + h.eps);
-    p = rh(pi + div_maybe_zero(h.neg_step_size * m, d));
+    const v2h pi = round2(mix_mul(p.x, h.decay, c), mix_mul(p.y, h.decay, c));
+    v2h d = round2(__builtin_amdgcn_sqrtf((float)v.x), __builtin_amdgcn_sqrtf((float)v.y));
+    float q[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // div_by_rc(d, bc2_sqrt, rbc2_sqrt)
+        q[i] = mix_mul(d[i], h.rbc2_sqrt, c);
+        q[i] = __builtin_fmaf(__builtin_fmaf(-q[i], h.bc2_sqrt, (float)d[i]), h.rbc2_sqrt, q[i]);
+    }
+    d = round2(q[0], q[1]);
+    d = round2(mix_add(d.x, h.eps, c), mix_add(d.y, h.eps, c));
+    const float ux = half_quotient<ZERO>(mix_mul(m.x, h.neg_step_size, c), d.x);
+    const float uy = half_quotient<ZERO>(mix_mul(m.y, h.neg_step_size, c), d.y);
+    return round2(mix_add(pi.x, ux, c), mix_add(pi.y, uy, c));
 }
 
-// Codes of rh(v[k] / scale) for a lane's 8 values; |v[k]| <= scale wherever the scale is finite and
+// A lane's eight elements through the chain; p, m and v are updated in place.  Both branches are uniform.
+__device__ __forceinline__ void half_elts8(v2h (&p)[kPairs], const v2h (&g)[kPairs], v2h (&m)[kPairs], v2h (&v)[kPairs],
+                                           const NfHyper &h, const MixConst &c)
+{
+    if (fabsf(h.w1) < 0.5f) {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
+            m[j] = round2(half_lerp<true>(m[j].x, g[j].x, h.w1, c), half_lerp<true>(m[j].y, g[j].y, h.w1, c));
+    } else {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
+            m[j] = round2(half_lerp<false>(m[j].x, g[j].x, h.w1, c), half_lerp<false>(m[j].y, g[j].y, h.w1, c));
+    }
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j)
+        v[j] = half_second_moment(v[j], g[j], h, c);
+    // an eps that is positive as a half keeps every denominator positive: rounding is monotonic
+    if (h.eps > 0x1p-25f) {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
+            p[j] = half_param<false>(p[j], m[j], v[j], h, c);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
+            p[j] = half_param<true>(p[j], m[j], v[j], h, c);
+    }
+}
+
+// rh(x / s) of two halfs given rc = RN(1 / s), s in the range in which that is exact, 0 <= |x| <= s: one
+// product.  With the significands as integers V, S in [1024, 2047] the quotient's distance from a rounding
+// boundary M of halfs (an odd integer below 4096) is |V 2^j - M S| / S >= 1 / S >= 1 / 2047 -- never zero, as
+// M would have to divide V -- and the product's error is at most M 2^-23 (1 + 2^-25) < 1 / 2047, so it
+// falls on the quotient's side of every boundary.  (Quotients below 2^-14, which have fewer bits as halfs, may
+// round otherwise; no map the closed forms serve has a midpoint there.)
+__device__ __forceinline__ v2h half_quotients(v2h x, float rcx, float rcy, const MixConst &c)
+{
+    return round2(mix_mul(x.x, rcx, c), mix_mul(x.y, rcy, c));
+}
+
+// Codes of rh(v / scale) for a lane's 8 values; |v| <= scale wherever the scale is finite and
 // positive (it is a maximum over the values it divides).
 __device__ __forceinline__ uint32_t encode8_scaled_h(const uint32_t *lds, uint32_t lds_map, int kind,
-                                                     const float (&v)[kEltsPerLane], float scale)
+                                                     const v2h (&v)[kPairs], float scale, const MixConst &c)
 {
     float x[kEltsPerLane];
     if (kind != kMapGeneric && rc_safe(scale)) {
         // quotients in [-1, 1], no NaN: the closed forms of the standard maps apply as they are
         const float rc = rcp_exact(scale);
 #pragma unroll
-        for (int k = 0; k < kEltsPerLane; ++k)
-            x[k] = rh(div_by_rc(v[k], scale, rc));
+        for (int j = 0; j < kPairs; ++j) {
+            const v2h q = half_quotients(v[j], rc, rc, c);
+            x[2 * j] = (float)q.x;
+            x[2 * j + 1] = (float)q.y;
+        }
         return kind == kMapStdM ? encode8_std_m(lds, x) : encode8_std_v(x);
     }
 #pragma unroll
-    for (int k = 0; k < kEltsPerLane; ++k)
-        x[k] = rh(v[k] / scale);
+    for (int j = 0; j < kPairs; ++j) {
+        x[2 * j] = rh((float)v[j].x / scale);
+        x[2 * j + 1] = rh((float)v[j].y / scale);
+    }
     return encode8_plain(lds, lds_map, kind, x);
 }
 
@@ -185,20 +325,20 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
     uint16_t *mcp = reinterpret_cast<uint16_t *>(t.mc + (gbase >> 1)) + lane16;
     uint16_t *vcp = reinterpret_cast<uint16_t *>(t.vc + (gbase >> 1)) + lane16;
     const LdsFill fill = lds_fill_load(qmap_m, qmap_v);
-    float pv[kEltsPerLane], gv[kEltsPerLane];
+    v2h p2[kPairs], g2[kPairs];
     uint32_t wm = 0, wv = 0;
     float sm = 0.0f, sv = 0.0f;
     if (full) {
         const h16 *gp = t.g + gbase + lane16 * 4;
         const v4h a0 = load_h4(pp), a1 = load_h4(pp + 64), b0 = load_h4(gp), b1 = load_h4(gp + 64);
-        widen8(a0, a1, pv);
-        widen8(b0, b1, gv);
+        pairs_of(a0, a1, p2);
+        pairs_of(b0, b1, g2);
     } else if (live) {
 #pragma unroll
         for (int k = 0; k < kEltsPerLane; ++k) {
             const int64_t i = gbase + elt_offset(lane16, k);
-            pv[k] = i < n ? (float)t.p[i] : 0.0f;
-            gv[k] = i < n ? (float)t.g[i] : 0.0f;
+            p2[k >> 1][k & 1] = i < n ? t.p[i] : (h16)0.0f;
+            g2[k >> 1][k & 1] = i < n ? t.g[i] : (h16)0.0f;
         }
     }
     if (live) {
@@ -244,42 +384,59 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
     h.bc2_sqrt = t.bc2_sqrt;
     h.rbc2_sqrt = t.rbc2_sqrt;
     const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
-    float m[kEltsPerLane], v[kEltsPerLane];
     float amax_m = 0.0f, amax_v = 0.0f;
+    uint32_t om, ov;
+    if constexpr (FUSED) {
+        float m[kEltsPerLane], v[kEltsPerLane];
 #pragma unroll
-    for (int k = 0; k < kEltsPerLane; ++k) {
-        if (FUSED) {
+        for (int k = 0; k < kEltsPerLane; ++k) {
             m[k] = rh(rh(decode_nibble(lds, kLdsQ0, nm, k)) * sm);
             v[k] = rh(rh(decode_nibble(lds, kLdsQ1, nv, k)) * sv);
-            adamw_moments(gv[k], m[k], v[k], fh);
+            adamw_moments((float)g2[k >> 1][k & 1], m[k], v[k], fh);
             m[k] = rh(m[k]);
             v[k] = rh(v[k]);
-            pv[k] = rh(adamw_param(pv[k], m[k], v[k], fh));
-        } else {
-            m[k] = rh(decode_nibble(lds, kLdsQ0, nm, k) * sm);
-            v[k] = rh(decode_nibble(lds, kLdsQ1, nv, k) * sv);
-            half_elt(pv[k], gv[k], m[k], v[k], h);
+            p2[k >> 1][k & 1] = (h16)rh(adamw_param((float)p2[k >> 1][k & 1], m[k], v[k], fh));
+            // elements past the end of the tensor: threads that the operator does not have
+            if (!full && gbase + elt_offset(lane16, k) >= n)
+                m[k] = v[k] = 0.0f;
+            amax_m = fmaxf(amax_m, fabsf(m[k]));
+            amax_v = fmaxf(amax_v, fabsf(v[k]));
         }
-        // elements past the end of the tensor: the zero padding of the chain's quantiser; threads that
-        // the fused operator does not have
-        if (!full && gbase + elt_offset(lane16, k) >= n)
-            m[k] = v[k] = 0.0f;
-        amax_m = fmaxf(amax_m, fabsf(m[k]));
-        amax_v = fmaxf(amax_v, fabsf(v[k]));
+        row16_max2(amax_m, amax_v);
+        // the fused operator normalises in float
+        om = encode8_scaled(lds, kLdsQ0, kind_m, m, amax_m);
+        ov = encode8_scaled(lds, kLdsQ1, kind_v, v, amax_v);
+    } else {
+        const MixConst c = mix_const();
+        v2h m[kPairs], v[kPairs];
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j) {
+            m[j] = round2(decode_nibble(lds, kLdsQ0, nm, 2 * j) * sm, decode_nibble(lds, kLdsQ0, nm, 2 * j + 1) * sm);
+            v[j] = round2(decode_nibble(lds, kLdsQ1, nv, 2 * j) * sv, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1) * sv);
+        }
+        half_elts8(p2, g2, m, v, h, c);
+        if (!full) {
+            // elements past the end of the tensor: the zero padding of the chain's quantiser
+#pragma unroll
+            for (int k = 0; k < kEltsPerLane; ++k)
+                if (gbase + elt_offset(lane16, k) >= n)
+                    m[k >> 1][k & 1] = v[k >> 1][k & 1] = (h16)0.0f;
+        }
+        amax_m = max8<true>(m);
+        amax_v = max8<false>(v);
+        row16_max2(amax_m, amax_v);
+        // the chain normalises in half (x.div(max1) on half tensors)
+        om = encode8_scaled_h(lds, kLdsQ0, kind_m, m, amax_m, c);
+        ov = encode8_scaled_h(lds, kLdsQ1, kind_v, v, amax_v, c);
     }
-    row16_max2(amax_m, amax_v);
-    // the chain normalises in half (x.div(max1) on half tensors), the fused operator in float
-    const uint32_t om = FUSED ? encode8_scaled(lds, kLdsQ0, kind_m, m, amax_m) : encode8_scaled_h(lds, kLdsQ0, kind_m, m, amax_m);
-    const uint32_t ov = FUSED ? encode8_scaled(lds, kLdsQ1, kind_v, v, amax_v) : encode8_scaled_h(lds, kLdsQ1, kind_v, v, amax_v);
     if (full) {
-        store_h4(pp, narrow4(pv, 0));
-        store_h4(pp + 64, narrow4(pv, 1));
+        store_pairs(pp, p2);
     } else {
 #pragma unroll
         for (int k = 0; k < kEltsPerLane; ++k) {
             const int64_t i = gbase + elt_offset(lane16, k);
             if (i < n)
-                t.p[i] = (h16)pv[k];
+                t.p[i] = p2[k >> 1][k & 1];
         }
     }
     if (!FUSED || full) {
@@ -302,19 +459,72 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
 // are MultiR1 with p, g, ms, row_old and col_old pointing at halfs; row_new and col_new are the float
 // work arrays.
 // ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void rank1_update_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
+// Where a lane stands in the operands; a pass moves every pointer on by the same distance, which costs an
+// addition each (recomputing them from the row took a tenth of the pass's instructions).
+struct HalfCursor {
+    h16 *p, *ms;
+    const h16 *g, *row_old;
+    uint16_t *mc, *vc;
+    int64_t row, rows_on, values_on;
+
+    __device__ __forceinline__ HalfCursor(const TensorR1 &t, const Geometry &q, int lane16)
+    {
+        const int64_t grp = q.row0 * t.col_blocks + q.cg, first = grp * kGroup + lane16 * 4;
+        p = reinterpret_cast<h16 *>(t.p) + first;
+        g = reinterpret_cast<const h16 *>(t.g) + first;
+        ms = reinterpret_cast<h16 *>(t.ms) + grp;
+        row_old = reinterpret_cast<const h16 *>(t.row_old) + q.row0;
+        mc = reinterpret_cast<uint16_t *>(t.mc) + grp * (kGroup / 4) + lane16;
+        vc = reinterpret_cast<uint16_t *>(t.vc) + grp * (kGroup / 4) + lane16;
+        row = q.row0;
+        rows_on = q.step;
+        values_on = (int64_t)q.step * t.col_blocks * kGroup;
+    }
+    __device__ __forceinline__ void advance()
+    {
+        p += values_on;
+        g += values_on;
+        ms += values_on / kGroup;
+        row_old += rows_on;
+        mc += values_on / 4;
+        vc += values_on / 4;
+        row += rows_on;
+    }
+};
+
+// larger of two non-negative floats that are numbers
+__device__ __forceinline__ float max_bits(float a, float b)
+{
+    return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
+}
+
+// The second pass's part of lds_fill: the second moment's map, and the first moment's encode table only where
+// the caller's map is that one.
+__device__ __forceinline__ void lds_fill_v(uint32_t *lds, int kind_v, const float *__restrict__ qmap_v)
+{
+    if (kind_v == kMapStdM)
+        lds_fill(lds, qmap_v, qmap_v);
+    else if (threadIdx.x < 16)
+        lds[kLdsQ1 / 4 + threadIdx.x] = __float_as_uint(qmap_v[threadIdx.x]);
+}
+
+// (co < ro) ? co : ro for two columns' statistics: non-negative halfs or NaN.  On bit patterns a NaN is the
+// largest, so a NaN column gives the row's statistic as the comparison does; a NaN row statistic is the result.
+__device__ __forceinline__ v2h rank1_scales(v2h co, h16 ro)
+{
+    const v2h rows = {ro, ro};
+    return ro == ro ? min2_bits(co, rows) : rows;
+}
+
+__global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                     const float *__restrict__ qmap_v)
 {
     __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
-    __shared__ __align__(16) float col_old[kMaxWide * kGroup];
+    __shared__ __align__(16) h16 col_old[kMaxWide * kGroup];
     __shared__ uint32_t colred[kMaxWide * kRedSlotWords];
     __shared__ uint32_t rowred[kRowSlots];
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    h16 *const P = reinterpret_cast<h16 *>(t.p);
-    const h16 *const G = reinterpret_cast<const h16 *>(t.g);
-    h16 *const MS = reinterpret_cast<h16 *>(t.ms);
-    const h16 *const ROW_OLD = reinterpret_cast<const h16 *>(t.row_old);
     const h16 *const COL_OLD = reinterpret_cast<const h16 *>(t.col_old);
     const uint32_t tl = blockIdx.x - args.tile_start[lo];
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
@@ -323,7 +533,7 @@ __global__ __launch_bounds__(kThreads) void rank1_update_half_kernel(const Multi
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
     lds_fill(lds, qmap_m, qmap_v);
     for (int j = threadIdx.x; j < kMaxWide * kGroup; j += kThreads)
-        col_old[j] = (j < q.wide * kGroup && tile_c0 + j < cols) ? (float)COL_OLD[tile_c0 + j] : 0.0f;
+        col_old[j] = (j < q.wide * kGroup && tile_c0 + j < cols) ? COL_OLD[tile_c0 + j] : (h16)0.0f;
     for (int j = threadIdx.x; j < kMaxWide * (int)kRedSlotWords; j += kThreads)
         colred[j] = 0u;
     if (threadIdx.x < kRowSlots)
@@ -338,6 +548,7 @@ __global__ __launch_bounds__(kThreads) void rank1_update_half_kernel(const Multi
     h.neg_step_size = t.neg_step_size;
     h.bc2_sqrt = t.bc2_sqrt;
     h.rbc2_sqrt = t.rbc2_sqrt;
+    const MixConst c = mix_const();
     __syncthreads();
 
     if (tl == 0) {
@@ -347,51 +558,51 @@ __global__ __launch_bounds__(kThreads) void rank1_update_half_kernel(const Multi
                       encode8_plain(lds, kLdsQ0, kind_m, z));
     }
     const int slot = drow & (q.wide - 1);
-    if (q.cg < t.col_blocks) {
-        const float *cop = col_old + slot * kGroup + lane16 * 4;
-        uint32_t *red = colred + slot * kRedSlotWords + lane16;
-        float co[kEltsPerLane];
-        unpack8(*reinterpret_cast<const float4 *>(cop), *reinterpret_cast<const float4 *>(cop + 64), co);
-#pragma unroll 1
-        for (int it = 0; it < q.passes; ++it) {
-            const int64_t r = q.row0 + it * q.step;
-            if (r >= t.rows)
-                break;
-            const int64_t grp = r * t.col_blocks + q.cg;
-            const int64_t gbase = grp * kGroup;
-            h16 *pp = P + gbase + lane16 * 4;
-            const h16 *gp = G + gbase + lane16 * 4;
-            uint16_t *mcp = reinterpret_cast<uint16_t *>(t.mc + (gbase >> 1)) + lane16;
-            const uint16_t *vcp = reinterpret_cast<const uint16_t *>(t.vc + (gbase >> 1)) + lane16;
-            const v4h a0 = load_h4(pp), a1 = load_h4(pp + 64), b0 = load_h4(gp), b1 = load_h4(gp + 64);
-            const uint32_t wm = load_u16(mcp) | (load_u16(mcp + 16) << 16);
-            const uint32_t wv = load_u16(vcp) | (load_u16(vcp + 16) << 16);
-            const float sm = (float)MS[grp], ro = (float)ROW_OLD[r];
-            float pv[kEltsPerLane], gv[kEltsPerLane], m[kEltsPerLane], v[kEltsPerLane];
-            widen8(a0, a1, pv);
-            widen8(b0, b1, gv);
-            const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
-            float amax_m = 0.0f, vmax = 0.0f;
+    if (q.cg < t.col_blocks && q.row0 < t.rows) {
+        const v4h *cop = reinterpret_cast<const v4h *>(col_old + slot * kGroup + lane16 * 4);
+        v2h co[kPairs], vtop[kPairs];  // the lane's columns: current statistics, maxima over its passes
+        pairs_of(cop[0], cop[16], co);
 #pragma unroll
-            for (int k = 0; k < kEltsPerLane; ++k) {
-                m[k] = rh(decode_nibble(lds, kLdsQ0, nm, k) * sm);
-                v[k] = rh(decode_nibble(lds, kLdsQ1, nv, k) * ((co[k] < ro) ? co[k] : ro));
-                half_elt(pv[k], gv[k], m[k], v[k], h);
-                amax_m = fmaxf(amax_m, fabsf(m[k]));
-                vmax = fmaxf(vmax, v[k]);
-                atomicMax(red + k * 16, __float_as_uint(v[k]));
+        for (int j = 0; j < kPairs; ++j)
+            vtop[j] = v2h{(h16)0.0f, (h16)0.0f};
+        HalfCursor at(t, q, lane16);
+#pragma unroll 1
+        for (int it = 0; it < q.passes && at.row < t.rows; ++it, at.advance()) {
+            const v4h a0 = load_h4(at.p), a1 = load_h4(at.p + 64), b0 = load_h4(at.g), b1 = load_h4(at.g + 64);
+            const uint32_t wm = load_u16(at.mc) | (load_u16(at.mc + 16) << 16);
+            const uint32_t wv = load_u16(at.vc) | (load_u16(at.vc + 16) << 16);
+            const float sm = (float)*at.ms;
+            const h16 ro = *at.row_old;
+            v2h p2[kPairs], g2[kPairs], m[kPairs], v[kPairs];
+            pairs_of(a0, a1, p2);
+            pairs_of(b0, b1, g2);
+            const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
+#pragma unroll
+            for (int j = 0; j < kPairs; ++j) {
+                m[j] = round2(decode_nibble(lds, kLdsQ0, nm, 2 * j) * sm, decode_nibble(lds, kLdsQ0, nm, 2 * j + 1) * sm);
+                const v2h s = rank1_scales(co[j], ro);
+                v[j] = round2(mix_mul(s.x, decode_nibble(lds, kLdsQ1, nv, 2 * j), c),
+                              mix_mul(s.y, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1), c));
             }
+            half_elts8(p2, g2, m, v, h, c);
+#pragma unroll
+            for (int j = 0; j < kPairs; ++j)
+                vtop[j] = max2_bits(vtop[j], v[j]);
+            float amax_m = max8<true>(m), vmax = max8<false>(v);
             row16_max2(amax_m, vmax);
-            const uint32_t om = encode8_scaled_h(lds, kLdsQ0, kind_m, m, amax_m);
-            store_h4(pp, narrow4(pv, 0));
-            store_h4(pp + 64, narrow4(pv, 1));
-            store_u16(mcp, om & 0xFFFFu);
-            store_u16(mcp + 16, om >> 16);
+            const uint32_t om = encode8_scaled_h(lds, kLdsQ0, kind_m, m, amax_m, c);
+            store_pairs(at.p, p2);
+            store_u16(at.mc, om & 0xFFFFu);
+            store_u16(at.mc + 16, om >> 16);
             if (lane16 == 0) {
-                MS[grp] = (h16)amax_m;
+                *at.ms = (h16)amax_m;
                 atomicMax(rowred + row_slot(t.tile, it, drow), __float_as_uint(vmax));
             }
         }
+        uint32_t *red = colred + slot * kRedSlotWords + lane16;
+#pragma unroll
+        for (int k = 0; k < kEltsPerLane; ++k)
+            atomicMax(red + k * 16, __float_as_uint((float)vtop[k >> 1][k & 1]));
     }
     __syncthreads();
     flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
@@ -404,31 +615,39 @@ __global__ __launch_bounds__(kThreads) void rank1_update_half_kernel(const Multi
     }
 }
 
-__global__ __launch_bounds__(kThreads) void rank1_requant_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
+__global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                      const float *__restrict__ qmap_v)
 {
     __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
-    __shared__ __align__(16) float col_old[kMaxWide * kGroup], col_new[kMaxWide * kGroup];
+    __shared__ __align__(16) h16 col_old[kMaxWide * kGroup];
+    __shared__ __align__(16) float col_new[kMaxWide * kGroup], col_rcp[kMaxWide * kGroup];
+    __shared__ uint32_t odd_columns;  // does the tile have a column statistic outside the reciprocal's exact range
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    const h16 *const G = reinterpret_cast<const h16 *>(t.g);
-    const h16 *const ROW_OLD = reinterpret_cast<const h16 *>(t.row_old);
     const h16 *const COL_OLD = reinterpret_cast<const h16 *>(t.col_old);
     const uint32_t tl = blockIdx.x - args.tile_start[lo];
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)t.col_blocks * kGroup;
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
-    lds_fill(lds, qmap_m, qmap_v);
+    const int kind_v = classify_map(qmap_v);
+    lds_fill_v(lds, kind_v, qmap_v);
+    if (threadIdx.x == 0)
+        odd_columns = 0u;
+    __syncthreads();
     for (int j = threadIdx.x; j < kMaxWide * kGroup; j += kThreads) {
         const bool in = j < q.wide * kGroup && tile_c0 + j < cols;
-        col_old[j] = in ? (float)COL_OLD[tile_c0 + j] : 0.0f;
-        col_new[j] = in ? t.col_new[tile_c0 + j] : 0.0f;
+        const float cn = in ? t.col_new[tile_c0 + j] : 1.0f;
+        col_old[j] = in ? COL_OLD[tile_c0 + j] : (h16)0.0f;
+        col_new[j] = cn;
+        col_rcp[j] = rcp_exact(cn);
+        if (!rc_safe(cn))
+            odd_columns = 1u;
     }
-    const int kind_v = classify_map(qmap_v);
     NfHyper h;
     h.b2 = args.b2;
     h.w2 = args.w2;
+    const MixConst c = mix_const();
     __syncthreads();
 
     if (tl == 0) {
@@ -440,55 +659,62 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_half_kernel(const Mult
     if (q.cg >= t.col_blocks)
         return;
     const int col_off = (drow & (q.wide - 1)) * kGroup + lane16 * 4;
-    float co[kEltsPerLane], cn[kEltsPerLane];
-    unpack8(*reinterpret_cast<const float4 *>(col_old + col_off), *reinterpret_cast<const float4 *>(col_old + col_off + 64), co);
-    unpack8(*reinterpret_cast<const float4 *>(col_new + col_off), *reinterpret_cast<const float4 *>(col_new + col_off + 64), cn);
+    const v4h *cop = reinterpret_cast<const v4h *>(col_old + col_off);
+    v2h co[kPairs];
     float rcn[kEltsPerLane];
-    bool cols_safe = true;
-#pragma unroll
-    for (int k = 0; k < kEltsPerLane; ++k) {
-        rcn[k] = rcp_exact(cn[k]);
-        cols_safe = cols_safe && rc_safe(cn[k]);
-    }
+    pairs_of(cop[0], cop[16], co);
+    unpack8(*reinterpret_cast<const float4 *>(col_rcp + col_off), *reinterpret_cast<const float4 *>(col_rcp + col_off + 64), rcn);
+    const bool even = kind_v == kMapStdV && __builtin_amdgcn_readfirstlane(odd_columns) == 0u;
+    const uint32_t code_dword = code_dword_of_lane(lane16), code_sel = code_swap_selector(lane16);
+    const int64_t first = (q.row0 * t.col_blocks + q.cg) * kGroup, values_on = (int64_t)q.step * t.col_blocks * kGroup;
+    const h16 *gp = reinterpret_cast<const h16 *>(t.g) + first + lane16 * 4;
+    uint32_t *vcp = reinterpret_cast<uint32_t *>(t.vc) + first / 8 + code_dword;
+    const h16 *row_old = reinterpret_cast<const h16 *>(t.row_old) + q.row0;
+    const float *row_new = t.row_new + q.row0;
+    const int64_t rows = t.rows;
 #pragma unroll 1
-    for (int it = 0; it < q.passes; ++it) {
-        const int64_t r = q.row0 + it * q.step;
-        if (r >= t.rows)
-            break;
-        const int64_t gbase = (r * t.col_blocks + q.cg) * kGroup;
-        const h16 *gp = G + gbase + lane16 * 4;
+    for (int64_t it = 0, r = q.row0; it < q.passes && r < rows; ++it, r += q.step, gp += values_on, vcp += values_on / 8,
+                 row_old += q.step, row_new += q.step) {
         const v4h b0 = load_h4(gp), b1 = load_h4(gp + 64);
-        uint16_t *vcp = reinterpret_cast<uint16_t *>(t.vc + (gbase >> 1)) + lane16;
-        const uint32_t wv = load_u16(vcp) | (load_u16(vcp + 16) << 16);
-        const float ro = (float)ROW_OLD[r], rn = t.row_new[r];
-        float gv[kEltsPerLane], v[kEltsPerLane], x[kEltsPerLane];
-        widen8(b0, b1, gv);
+        const uint32_t wv = swap_code_halves(load_u32(vcp), code_sel);
+        const h16 ro = *row_old;
+        const float rn = *row_new;
+        v2h g2[kPairs], v[kPairs];
+        pairs_of(b0, b1, g2);
         const Nibbles nv = split_nibbles(wv);
 #pragma unroll
-        for (int k = 0; k < kEltsPerLane; ++k) {
-            v[k] = rh(decode_nibble(lds, kLdsQ1, nv, k) * ((co[k] < ro) ? co[k] : ro));
-            half_second_moment(v[k], gv[k], h);
+        for (int j = 0; j < kPairs; ++j) {
+            const v2h s = rank1_scales(co[j], ro);
+            v[j] = round2(mix_mul(s.x, decode_nibble(lds, kLdsQ1, nv, 2 * j), c),
+                          mix_mul(s.y, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1), c));
+            v[j] = half_second_moment(v[j], g2[j], h, c);
         }
-        // every scale is a maximum over the values it divides: where all of the wave's scales lie in the
-        // range in which the reciprocal is exact, one multiply and two fmas give the correctly rounded quotient
+        float x[kEltsPerLane];
         uint32_t ov;
-        if (__all(cols_safe && rc_safe(rn))) {
+        // every scale is a maximum over the values it divides: where all of the wave's scales lie in the
+        // range in which the reciprocal is exact, one product gives the quotient as a half, and the reciprocal
+        // of the smaller statistic is the larger of the two reciprocals (rounding is monotonic)
+        if (even && __all(rc_safe(rn))) {
             const float rcr = rcp_exact(rn);
 #pragma unroll
-            for (int k = 0; k < kEltsPerLane; ++k) {
-                const bool by_col = cn[k] < rn;
-                x[k] = rh(div_by_rc(v[k], by_col ? cn[k] : rn, by_col ? rcn[k] : rcr));
+            for (int j = 0; j < kPairs; ++j) {
+                const v2h qt = half_quotients(v[j], max_bits(rcn[2 * j], rcr), max_bits(rcn[2 * j + 1], rcr), c);
+                // quotients in [0, 1]: the closed form of the standard map (encode8_std_v)
+                x[2 * j] = (float)qt.x;
+                x[2 * j + 1] = (float)qt.y;
             }
-            // quotients in [0, 1]: the closed form of the standard map applies as it is
-            ov = kind_v == kMapStdV ? encode8_std_v(x) : encode8_plain(lds, kLdsQ1, kind_v, x);
+            ov = encode8_std_v(x);
         } else {
 #pragma unroll
-            for (int k = 0; k < kEltsPerLane; ++k)
-                x[k] = rh(v[k] / ((cn[k] < rn) ? cn[k] : rn));
+            for (int k = 0; k < kEltsPerLane; ++k) {
+                v2h pair = v[k >> 1];
+                asm volatile("" : "+v"(pair));  // what only this branch needs stays in it
+                const float cn = col_new[col_off + (k & 3) + (k >> 2) * 64];
+                x[k] = rh((float)pair[k & 1] / ((cn < rn) ? cn : rn));
+            }
             ov = encode8_plain(lds, kLdsQ1, kind_v, x);
         }
-        store_u16(vcp, ov & 0xFFFFu);
-        store_u16(vcp + 16, ov >> 16);
+        store_u32(vcp, swap_code_halves(ov, code_sel));
     }
 }
 

@@ -506,8 +506,10 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     // served as double rows (rank1_tiles.hpp)
     const bool can_fold = MODE == kMCodes128 && bits_m == 4 && !half_io;
     // rows per tile: with an fp32 first moment a pass moves 24.5 instead of 13.5 bytes per element, and
-    // tiles of half the rows do better (LLaMA-7B-shaped set 29.3 -> 28.6 ms per step)
-    const uint32_t policy_rows = M32 ? kPolicyRowsM32 : kPolicyRows;
+    // tiles of half the rows do better (LLaMA-7B-shaped set 29.3 -> 28.6 ms per step); the passes on float16
+    // parameters are bound by their arithmetic, and taller tiles spread a tile's set-up over more rows (update
+    // and second pass of four decoder layers of width 4096: 1254 + 519 -> 1244 + 498 us)
+    const uint32_t policy_rows = M32 ? kPolicyRowsM32 : half_io ? kPolicyRowsHalf : kPolicyRows;
     // column counts that are no multiple of 128 (wide-group records only): every tensor of the call
     // then takes the kernels for ragged rows
     bool ragged = false;

@@ -24,6 +24,8 @@ constexpr int kR1Max = 32;               // tensors per launch
 constexpr int kPolicyLgWide = LPMM_R1_LG;
 constexpr uint32_t kPolicyRows = LPMM_R1_ROWS, kPolicyResident = LPMM_R1_RESIDENT;
 constexpr uint32_t kPolicyRowsM32 = LPMM_R1_ROWS / 2;  // fp32 first moment
+constexpr uint32_t kPolicyRowsHalf = LPMM_R1_ROWS * 2;  // float16 parameters
+constexpr uint32_t kPolicyRowsMost = kPolicyRowsHalf;
 static_assert(LPMM_R1_LG >= 1 && LPMM_R1_LG <= 3, "a tile is 256 to 1024 columns wide at most");
 constexpr int kMaxLgWide = kPolicyLgWide;   // the LDS column arrays hold 128 << kMaxLgWide columns
 constexpr int kMaxWide = 1 << kMaxLgWide;
@@ -175,7 +177,7 @@ __device__ __forceinline__ void fold_rows(const Fold &f, int64_t r, uint32_t cg,
 // the tile) + (tensor row of a double row: folded rows only) -- and one global atomic per row and
 // tile follows the passes, issued by neighbouring threads for neighbouring rows (LLaMA-7B-shaped
 // set 21.23 -> 20.85 ms per step, GPT-2-XL-shaped set 6.30 -> 5.71 ms).
-constexpr int kRowSlots = 2 * (int)kPolicyRows;
+constexpr int kRowSlots = 2 * (int)kPolicyRowsMost;
 static_assert(kRowSlots <= kThreads, "one thread per row slot");
 static_assert(kPolicyRows >= (uint32_t)kDppRows, "a tile holds the policy's rows: one slot pair per row");
 

@@ -321,3 +321,56 @@ def test_fused_operator_on_every_half_gradient_value(oracle, qmaps):
         _same_halfs(to_np(ms), hms, f"step {step}: m scales")
         _same_halfs(to_np(vs), hvs, f"step {step}: v scales")
         _same_halfs(to_np(p), hp, f"step {step}: p")
+
+
+def _one_step(nat, t, g, step, qmaps, beta1, beta2, lr, wd, eps):
+    dqm, dqv = (to_dev(q) for q in qmaps)
+    table = np.array([t.record(g, step)], dtype=nat.ADAMW4BIT_TENSOR)
+    st = nat.lib().lpmm_nonfused_adamw4bit_f16_step_multi(table.ctypes.data, 1, dqm.data_ptr(), dqv.data_ptr(), beta1,
+                                                          beta2, lr, wd, eps, nat.current_stream(torch.device("cuda:0")))
+    assert st == 0
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("eps", [1e-3, 1e-8])
+def test_half_root_of_every_second_moment(oracle, qmaps, eps):
+    """A step that starts from every finite positive half as the second moment of one group (code 15 is 1.0,
+    gradients are zero, beta2 = 1 - 2^-24 keeps the value): parameters show the root and the quotients."""
+    nat = _native()
+    rng = np.random.default_rng(71)
+    scales = np.arange(1, 0x7C00, dtype=np.uint16).view(f16)
+    t = _Flat(oracle, scales.size * 128, rng)
+    t.host_p[:] = 0
+    t.p.zero_()
+    codes = [np.zeros(_nbytes(t.n), np.uint8) for _ in range(2)]
+    codes[0][: t.n // 2] = rng.integers(0, 256, t.n // 2, dtype=np.uint8)
+    codes[1][: t.n // 2] = 0xFF
+    t.state.m, t.state.v = (codes[0], np.ones(scales.size, f16)), (codes[1], scales.copy())
+    t.mc, t.vc, t.ms, t.vs = to_dev(codes[0]), to_dev(codes[1]), to_dev(t.state.m[1]), to_dev(scales)
+    step = t.state.step = 300_000_000  # both bias corrections are 1 then
+    t.state.step -= 1
+    hyper = (0.9, 1 - 2.0 ** -24, 0.1, 0.0, eps)
+    g = np.zeros(t.n, f16)
+    _one_step(nat, t, g, step, qmaps, *hyper)
+    oracle.nonfused_step_f16(t.host_p, g, t.state, *qmaps, hyper[2], hyper[0], hyper[1], eps, 0.0)
+    assert np.array_equal(t.state.v[1], scales)
+    t.check("every second moment")
+
+
+def test_half_quotient_of_every_pair_of_significands(oracle, qmaps):
+    """Every significand over every group maximum's: the product by the reciprocal, rounded to half, gives the
+    codes of the correctly rounded quotient.  beta1 = 0 makes the gradients the first moment."""
+    nat = _native()
+    rng = np.random.default_rng(72)
+    sig = np.arange(1024, 2048, dtype=np.float32)
+    groups = np.zeros((1024, 9, 128), np.float32)  # 1024 values in 9 groups of 127 behind each maximum
+    groups[:, :, 0] = sig[:, None] / 1024
+    below = np.zeros(9 * 127, np.float32)
+    below[:1024] = sig / 2048
+    exponents = rng.integers(-8, 1, (1024, 9 * 127))
+    groups[:, :, 1:] = (below * 2.0 ** exponents).reshape(1024, 9, 127)
+    g = (groups.reshape(-1) * rng.choice([-1.0, 1.0], groups.size)).astype(f16)
+    t = _Flat(oracle, g.size, rng)
+    _one_step(nat, t, g, 1, qmaps, 0.0, 0.999, 1e-2, 0.01, 1e-3)
+    oracle.nonfused_step_f16(t.host_p, g, t.state, *qmaps, 1e-2, 0.0, 0.999, 1e-3, 0.01)
+    t.check("every pair of significands")
