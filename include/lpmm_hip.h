@@ -662,6 +662,20 @@ int lpmm_selftest_bucket_encoder(const float *qmap, int bits, unsigned long long
  *   LPMM_PROBE_READ       a read                                   4 B/element
  *   LPMM_PROBE_WRITE      a written                                4 B/element
  *   LPMM_PROBE_COPY       a = b                                    8 B/element
+/* The same chain on a float buffer (tensors whose buffer is not quantised): buf float[n], written
+ * only on the first step.  Pointers are 4-byte aligned. */
+typedef struct lpmm_sgd_fp32_tensor {
+    float *p;
+    const float *g;
+    float *buf;
+    int64_t n;
+    int32_t first_step;
+    int32_t reserved;
+} lpmm_sgd_fp32_tensor;
+
+int lpmm_sgd_fp32_step_multi(const lpmm_sgd_fp32_tensor *tensors, int64_t count, double momentum, double dampening,
+                             double lr, double weight_decay, int nesterov, int maximize, void *stream);
+
  *   LPMM_PROBE_UPDATE     a += b in place (2 reads : 1 write)     12 B/element
  *   LPMM_PROBE_FUSED_MIX  the seven streams of lpmm_adamw4bit_step: a, b read, a written,
  *                         codes0/1 (n/2 bytes each) and scale0/1 (n/128 floats each) read and

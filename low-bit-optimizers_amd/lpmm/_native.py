@@ -76,6 +76,7 @@ PROTOTYPES = {
     "lpmm_stream_probe": (_int, [_int] + [_vp] * 6 + [_i64, _i64, _vp]),
     "lpmm_selftest_encoders": (_int, [_vp, _vp]),
     "lpmm_selftest_bucket_encoder": (_int, [_vp, _int, _vp, _vp]),
+    "lpmm_sgd_fp32_step_multi": (_int, [_vp, _i64] + [_d] * 4 + [_int, _int, _vp]),
     "lpmm_selftest_arithmetic": (_int, [_vp, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_uint32, _vp]),
 }
 
@@ -117,6 +118,8 @@ _lib = None
 def lib():
     """The loaded library; raises RuntimeError when it has not been built."""
     global _lib
+SGD_FP32_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("buf", "<u8"), ("n", "<i8"), ("first_step", "<i4"),
+                            ("reserved", "<i4")])
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(

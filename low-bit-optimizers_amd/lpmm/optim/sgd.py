@@ -6,7 +6,8 @@ The momentum buffer uses the first-moment quantisation config (QUANT.M).  Contig
 tensors whose buffer is quantised with 4 bits, 'group' scaling over 128 values and round to
 nearest (the default configuration) take one HIP kernel per 64 tensors that reads p, g and the
 packed buffer once and writes p and the buffer back (lpmm_sgd4bit_step_multi: 13 bytes per
-parameter).  Every other case runs the reference's own chain of PyTorch ops on the device
+parameter); contiguous float32 tensors whose buffer is not quantised take the same chain on a
+float buffer, one kernel per 64 tensors.  Every other case runs the reference's own chain of PyTorch ops on the device
 (lpmm/optim/sgd.py:152-187) around the HIP dequantise / quantise kernels of lpmm.functional.
 Both produce the same state layout.
 """
@@ -67,6 +68,7 @@ class SGD(LowBitOptimizer):
         for group in self.param_groups:
             momentum, dampening = group["momentum"], group["dampening"]
             batched = {}  # (device, map address) -> records of the one-pass kernel
+            plain = {}  # device -> records of the kernel on float buffers
             for p in group["params"]:
                 if p.grad is None:
                     continue
@@ -79,8 +81,20 @@ class SGD(LowBitOptimizer):
                 qstate = state["momentum_buffer_qstate"]
                 enabled = self.override_q_enable.get(id(p), qstate["enable"])
 
-                if (one_pass_config and enabled and momentum != 0 and p.is_cuda and p.dtype is torch.float32
-                        and p.grad.dtype is torch.float32 and p.is_contiguous() and p.grad.is_contiguous()):
+                dense = (momentum != 0 and p.is_cuda and p.grad.is_cuda and p.dtype is torch.float32
+                         and p.grad.dtype is torch.float32 and p.is_contiguous() and p.grad.is_contiguous())
+                if dense and not enabled:
+                    buf = state["momentum_buffer"]
+                    first = buf.numel() <= 1
+                    if first:
+                        buf = torch.empty_like(p, memory_format=torch.contiguous_format)
+                    if buf.dtype is torch.float32 and buf.is_contiguous() and buf.shape == p.shape and buf.device == p.device:
+                        state["momentum_buffer"] = buf
+                        plain.setdefault(p.device, []).append(
+                            (p.data_ptr(), p.grad.data_ptr(), buf.data_ptr(), p.numel(), 1 if first else 0, 0))
+                        continue
+
+                if one_pass_config and enabled and dense:
                     first = state["momentum_buffer"].numel() <= 1
                     if first:
                         groups = (p.numel() + 127) // 128
@@ -129,4 +143,11 @@ class SGD(LowBitOptimizer):
                         group["weight_decay"], int(bool(group["nesterov"])), int(bool(group["maximize"])),
                         _native.current_stream(dev))
                 _native.check(st, "SGD step")
+            for dev, records in plain.items():
+                table = np.array(records, dtype=_native.SGD_FP32_TENSOR)
+                with torch.cuda.device(dev):
+                    st = _native.lib().lpmm_sgd_fp32_step_multi(
+                        table.ctypes.data, len(records), momentum, dampening, group["lr"], group["weight_decay"],
+                        int(bool(group["nesterov"])), int(bool(group["maximize"])), _native.current_stream(dev))
+                _native.check(st, "SGD step on float buffers")
         return loss

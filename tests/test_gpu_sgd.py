@@ -208,3 +208,34 @@ def test_sgd_argument_checks(qmaps):
     assert call([ok[:4] + (-5, 1, 0)]) != 0
     assert call([ok[:4] + (0, 1, 0)]) == 0  # an empty tensor is skipped
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("hyper", HYPERS)
+def test_sgd_on_float_buffers_matches_oracle(oracle, hyper):
+    """Tensors whose buffer is not quantised (lpmm_sgd_fp32_step_multi), through lpmm.optim.SGD: sizes around the
+    16-byte accesses and the 1024-value tiles, pointers off a 16-byte boundary, more tensors than one launch holds,
+    two steps after the one that creates the buffers.  A one-element buffer counts as not created, on every step
+    (the reference tells by numel() <= 1, lpmm/optim/sgd.py:161)."""
+    import lpmm
+
+    rng = np.random.default_rng(45)
+    sizes = [1, 2, 3, 4, 5, 1023, 1024, 1025, 4095, 4096] + [int(n) for n in rng.integers(1, 4097, 60)]
+    host = [(rng.standard_normal(n) * 0.02).astype(np.float32) for n in sizes]
+    stores = [to_dev(np.concatenate([np.zeros(i % 3, np.float32), h])) for i, h in enumerate(host)]
+    params = [torch.nn.Parameter(s[i % 3:]) for i, s in enumerate(stores)]
+    opt = lpmm.optim.SGD(params, lr=hyper["lr"], momentum=hyper["momentum"], dampening=hyper["dampening"],
+                         weight_decay=hyper["wd"], nesterov=hyper["nesterov"], maximize=hyper["maximize"])
+    bufs = [np.zeros(n, np.float32) for n in sizes]
+    for step in range(3):
+        grads = [(rng.standard_normal(n) * 1e-2).astype(np.float32) for n in sizes]
+        for p, g in zip(params, grads):
+            p.grad = to_dev(g)
+        opt.step()
+        torch.cuda.synchronize()
+        for i, (h, g, b) in enumerate(zip(host, grads, bufs)):
+            oracle.sgd_update(h, g, b, hyper["momentum"], hyper["dampening"], hyper["lr"], hyper["wd"], hyper["nesterov"],
+                              hyper["maximize"], step == 0 or h.size == 1)
+            got = opt.state[params[i]]["momentum_buffer"]
+            assert got.dtype == torch.float32 and got.shape == params[i].shape
+            assert np.array_equal(to_np(got), b) and np.array_equal(to_np(params[i]), h), (i, h.size, step)
+            assert not to_np(stores[i][: i % 3]).any()
