@@ -280,6 +280,11 @@ int lpmm_nonfused_update(float *p, const float *g, float *m, float *v, int64_t n
 int lpmm_nonfused_update_multi(const lpmm_adamw_fp32_tensor *tensors, int64_t count, double beta1,
                                double beta2, double lr, double weight_decay, double eps, void *stream);
 
+/* The same for IEEE half-precision tensors (p, g, m, v of the records point to fp16[n], 2-byte aligned): the
+ * chain of PyTorch's half ops, one rounding to half per op (lpmm/optim/adamw.py:367-369, :412-422). */
+int lpmm_nonfused_update_f16_multi(const lpmm_adamw_fp32_tensor *tensors, int64_t count, double beta1,
+                                   double beta2, double lr, double weight_decay, double eps, void *stream);
+
 /* The whole non-fused step on 4-bit states in one pass, for the configuration the reference
  * uses by default when fused=False is combined with block-wise second-moment scaling (both
  * moments 4-bit, 'group' scaling, gp_sz 128, real-nearest): dequantise m and v, the update
@@ -497,6 +502,47 @@ int lpmm_nonfused_adamw4bit_rank1_mgroup_step_multi(const lpmm_rank1_mgroup_tens
                                                     double beta1, double beta2, double lr,
                                                     double weight_decay, double eps, void *stream);
 
+/* The two passes for any column count and alignment (natural alignment of the types; code arrays 4-byte aligned),
+ * for every kind of state above.  kind: what m, m_max1 and the parameters are --
+ *   LPMM_RANK1_CODES4   4-bit codes, m_group_size 128, 256, ... 4096
+ *   LPMM_RANK1_FLOAT_M  m float[rows * cols], 4-bit second moment; qmap_m is not read
+ *   LPMM_RANK1_CODES8   one code of bits_m / bits_v (5 .. 8) bits per byte, m_group_size 128, code tables or NULL
+ *   LPMM_RANK1_HALF     p, g, scales and statistics binary16, 4-bit codes, m_group_size 128; work: rows + cols +
+ *                       ceil(rows * cols / 128) floats of scratch (not read for the other kinds)
+ * New codes, scales (not FLOAT_M, whose first moment is updated in place) and statistics go to the *_next arrays,
+ * which must not alias the current ones and are written in full.  passes: 3 both, 1 or 2 one at a time (as in
+ * lpmm_nonfused_adamw4bit_rank1_pass_multi, with the same records; not LPMM_RANK1_HALF).  Up to 32 tensors per
+ * launch. */
+#define LPMM_RANK1_CODES4 0
+#define LPMM_RANK1_FLOAT_M 1
+#define LPMM_RANK1_CODES8 2
+#define LPMM_RANK1_HALF 3
+typedef struct lpmm_rank1_any_tensor {
+    void *p;
+    const void *g;
+    void *m;
+    uint8_t *m_codes_next;
+    const void *m_max1;
+    void *m_max1_next;
+    const uint8_t *v_codes;
+    uint8_t *v_codes_next;
+    const void *v_rowmax;
+    const void *v_colmax;
+    void *v_rowmax_next;
+    void *v_colmax_next;
+    float *work;
+    int64_t rows;
+    int64_t cols;
+    float step;
+    float reserved;
+} lpmm_rank1_any_tensor;
+
+int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, int kind,
+                                             int64_t m_group_size, const float *qmap_m, int bits_m,
+                                             const void *table_m, const float *qmap_v, int bits_v,
+                                             const void *table_v, double beta1, double beta2, double lr,
+                                             double weight_decay, double eps, int passes, void *stream);
+
 /* lpmm_nonfused_adamw4bit_rank1_step_multi for code widths of 5 to 8 bits (lpmm/configs/
  * default_{5,6,7,8}b.yml): qmap_m / qmap_v hold 2^bits_m / 2^bits_v entries; the code arrays hold
  * one code per byte (lpmm/cpp_extension/quantization_kernel.cu:516-533, :656-669):
@@ -616,6 +662,20 @@ int lpmm_sgd4bit_step_multi(const lpmm_sgd4bit_tensor *tensors, int64_t count, c
                             double momentum, double dampening, double lr, double weight_decay,
                             int nesterov, int maximize, void *stream);
 
+/* The same chain on a float buffer (tensors whose buffer is not quantised): buf float[n], not
+ * read on the first step.  Pointers are 4-byte aligned. */
+typedef struct lpmm_sgd_fp32_tensor {
+    float *p;
+    const float *g;
+    float *buf;
+    int64_t n;
+    int32_t first_step;
+    int32_t reserved;
+} lpmm_sgd_fp32_tensor;
+
+int lpmm_sgd_fp32_step_multi(const lpmm_sgd_fp32_tensor *tensors, int64_t count, double momentum, double dampening,
+                             double lr, double weight_decay, int nesterov, int maximize, void *stream);
+
 /* ---------------------------------------------------------------------------------------
  * Diagnostic (no counterpart in the reference): compares the library's near-exact sqrt and
  * division sequences (hardware approximation + one fma correction of the residual) with the
@@ -662,20 +722,6 @@ int lpmm_selftest_bucket_encoder(const float *qmap, int bits, unsigned long long
  *   LPMM_PROBE_READ       a read                                   4 B/element
  *   LPMM_PROBE_WRITE      a written                                4 B/element
  *   LPMM_PROBE_COPY       a = b                                    8 B/element
-/* The same chain on a float buffer (tensors whose buffer is not quantised): buf float[n], written
- * only on the first step.  Pointers are 4-byte aligned. */
-typedef struct lpmm_sgd_fp32_tensor {
-    float *p;
-    const float *g;
-    float *buf;
-    int64_t n;
-    int32_t first_step;
-    int32_t reserved;
-} lpmm_sgd_fp32_tensor;
-
-int lpmm_sgd_fp32_step_multi(const lpmm_sgd_fp32_tensor *tensors, int64_t count, double momentum, double dampening,
-                             double lr, double weight_decay, int nesterov, int maximize, void *stream);
-
  *   LPMM_PROBE_UPDATE     a += b in place (2 reads : 1 write)     12 B/element
  *   LPMM_PROBE_FUSED_MIX  the seven streams of lpmm_adamw4bit_step: a, b read, a written,
  *                         codes0/1 (n/2 bytes each) and scale0/1 (n/128 floats each) read and

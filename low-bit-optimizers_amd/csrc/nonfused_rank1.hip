@@ -495,12 +495,15 @@ template <int MODE, class Record>
 static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
                             uint32_t m_lg, double beta1, double beta2, double lr, double weight_decay, double eps,
                             void *stream, int bits_m = 4, int bits_v = 4, const void *table_m = nullptr,
-                            const void *table_v = nullptr, int passes = 3, bool half_io = false)
+                            const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr)
 {
     // passes: 1 = the first pass alone (with the clearing of the next statistics), 2 = the second alone,
-    // 3 = both; one at a time only where the launches below are this file's own
-    if (passes < 1 || passes > 3 || (passes != 3 && (MODE != kMCodes128 || bits_m != 4 || half_io)))
+    // 3 = both; one at a time only where the launches below are this file's own, or general ones: any column count,
+    // any alignment (nonfused_rank1_any.hip; wide-group and fp32 records, at most one launch's worth, none empty).
+    const bool general = out != nullptr;
+    if (passes < 1 || passes > 3 || (passes != 3 && !general && (MODE != kMCodes128 || bits_m != 4 || half_io)))
         return LPMM_ERR_ARG;
+    const int64_t real_bytes = general && half_io ? 2 : 4, vec_bytes = general ? real_bytes : 16;
     constexpr bool M32 = MODE == kMFloat;
     // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
     // served as double rows (rank1_tiles.hpp)
@@ -526,7 +529,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         const Record &t = tensors[i];
         if (t.rows < 0 || t.cols < 0)
             return LPMM_ERR_SIZE;
-        if (t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && folds(t.rows, t.cols)))
+        if (!general && t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && folds(t.rows, t.cols)))
             return LPMM_ERR_SIZE;
         ragged = ragged || (MODE == kMCodesWide && t.cols % kGroup != 0);
         if (t.rows == 0 || t.cols == 0)
@@ -547,21 +550,21 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         LPMM_REQUIRE_PTR(t.v_colmax);
         LPMM_REQUIRE_PTR(t.v_rowmax_next);
         LPMM_REQUIRE_PTR(t.v_colmax_next);
-        LPMM_REQUIRE_ALIGN(t.p, 16);
-        LPMM_REQUIRE_ALIGN(t.g, 16);
-        LPMM_REQUIRE_ALIGN(first_moment(t), M32 ? 16 : 4);
+        LPMM_REQUIRE_ALIGN(t.p, vec_bytes);
+        LPMM_REQUIRE_ALIGN(t.g, vec_bytes);
+        LPMM_REQUIRE_ALIGN(first_moment(t), M32 && !general ? 16 : 4);
         LPMM_REQUIRE_ALIGN(t.v_codes, 4);
-        LPMM_REQUIRE_ALIGN(first_moment_scales(t), 4);
+        LPMM_REQUIRE_ALIGN(first_moment_scales(t), real_bytes);
         if (MODE == kMCodesWide) {
             LPMM_REQUIRE_PTR(next_scales(t));
             LPMM_REQUIRE_ALIGN(next_scales(t), 4);
             if (next_scales(t) == first_moment_scales(t))
                 return LPMM_ERR_ARG;
         }
-        LPMM_REQUIRE_ALIGN(t.v_rowmax, 4);
-        LPMM_REQUIRE_ALIGN(t.v_colmax, 16);
+        LPMM_REQUIRE_ALIGN(t.v_rowmax, real_bytes);
+        LPMM_REQUIRE_ALIGN(t.v_colmax, vec_bytes);
         LPMM_REQUIRE_ALIGN(t.v_rowmax_next, 4);
-        LPMM_REQUIRE_ALIGN(t.v_colmax_next, 16);
+        LPMM_REQUIRE_ALIGN(t.v_colmax_next, general ? 4 : 16);
         if (t.v_rowmax == t.v_rowmax_next || t.v_colmax == t.v_colmax_next)
             return LPMM_ERR_ARG;
     }
@@ -631,7 +634,11 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         if (passes & 1)
             hipLaunchKernelGGL(rank1_clear_kernel, dim3((uint32_t)clear_blocks, (uint32_t)k), dim3(kThreads), 0,
                                s, args);
-        if (half_io) {
+        if (general) {
+            const AnyKind kind = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
+            launch_rank1_any(args, *out, (uint32_t)tiles, qmap_m, qmap_v, kind, bits_m, bits_v,
+                             static_cast<const uint32_t *>(table_m), static_cast<const uint32_t *>(table_v), passes, s);
+        } else if (half_io) {
             launch_rank1_half(args, (uint32_t)tiles, qmap_m, qmap_v, s);
         } else if (ragged || (MODE == kMCodesWide && m_lg == 0)) {
             launch_rank1_ragged(args, (uint32_t)tiles, qmap_m, qmap_v, s);
@@ -735,4 +742,91 @@ extern "C" int lpmm_nonfused_adamw_bits_rank1_step_multi_table(const lpmm_nonfus
         LPMM_REQUIRE_ALIGN(table_v, 16);
     return rank1_step_multi<kMCodes128>(tensors, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream,
                                         bits_m, bits_v, table_m, table_v);
+}
+
+int lpmm::rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg,
+                               const float *qmap_m, int bits_m, const void *table_m, const float *qmap_v, int bits_v,
+                               const void *table_v, double beta1, double beta2, double lr, double weight_decay, double eps,
+                               int passes, void *stream)
+{
+    lpmm_rank1_mgroup_tensor wide[kR1Max];
+    lpmm_rank1_v4bit_tensor plain[kR1Max];
+    NewCodes out;
+    for (int64_t i = 0; i < count;) {
+        int k = 0;
+        for (; i < count && k < kR1Max; ++i) {
+            const lpmm_rank1_any_tensor &t = tensors[i];
+            if (t.rows == 0 || t.cols == 0)
+                continue;
+            lpmm_rank1_mgroup_tensor &w = wide[k];
+            lpmm_rank1_v4bit_tensor &f = plain[k];
+            f.p = w.p = static_cast<float *>(t.p);
+            f.g = w.g = static_cast<const float *>(t.g);
+            f.m = static_cast<float *>(t.m);
+            w.m_codes = static_cast<uint8_t *>(t.m);
+            w.m_max1 = static_cast<const float *>(t.m_max1);
+            w.m_max1_next = static_cast<float *>(t.m_max1_next);
+            f.v_codes = w.v_codes = const_cast<uint8_t *>(t.v_codes);
+            f.v_rowmax = w.v_rowmax = static_cast<const float *>(t.v_rowmax);
+            f.v_colmax = w.v_colmax = static_cast<const float *>(t.v_colmax);
+            f.v_rowmax_next = w.v_rowmax_next = static_cast<float *>(t.v_rowmax_next);
+            f.v_colmax_next = w.v_colmax_next = static_cast<float *>(t.v_colmax_next);
+            f.rows = w.rows = t.rows;
+            f.cols = w.cols = t.cols;
+            f.step = w.step = t.step;
+            f.reserved = w.reserved = 0.0f;
+            LPMM_REQUIRE_PTR(t.v_codes_next);
+            LPMM_REQUIRE_ALIGN(t.v_codes_next, 4);
+            if (t.v_codes_next == t.v_codes)
+                return LPMM_ERR_ARG;
+            if (kind != kAnyFloatM) {
+                LPMM_REQUIRE_PTR(t.m_codes_next);
+                LPMM_REQUIRE_ALIGN(t.m_codes_next, 4);
+                if (t.m_codes_next == t.m)
+                    return LPMM_ERR_ARG;
+            }
+            out.v[k] = t.v_codes_next;
+            out.m[k++] = t.m_codes_next;
+        }
+        const int st = kind == kAnyFloatM
+                           ? rank1_step_multi<kMFloat>(plain, k, qmap_v, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, 4,
+                                                       4, nullptr, nullptr, passes, false, &out)
+                           : rank1_step_multi<kMCodesWide>(wide, k, qmap_m, qmap_v, m_lg, beta1, beta2, lr, weight_decay, eps,
+                                                           stream, bits_m, bits_v, table_m, table_v, passes, kind == kAnyHalf, &out);
+        if (st != LPMM_OK)
+            return st;
+    }
+    return LPMM_OK;
+}
+
+extern "C" int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, int kind,
+                                                        int64_t m_group_size, const float *qmap_m, int bits_m,
+                                                        const void *table_m, const float *qmap_v, int bits_v,
+                                                        const void *table_v, double beta1, double beta2, double lr,
+                                                        double weight_decay, double eps, int passes, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    LPMM_REQUIRE_PTR(tensors);
+    if (kind < LPMM_RANK1_CODES4 || kind > LPMM_RANK1_HALF || passes < 1 || passes > 3)
+        return LPMM_ERR_ARG;
+    const bool bytes = kind == LPMM_RANK1_CODES8;
+    if (bytes ? bits_m < 5 || bits_m > 8 || bits_v < 5 || bits_v > 8 : bits_m != 4 || bits_v != 4)
+        return LPMM_ERR_ARG;
+    if (table_m != nullptr)
+        LPMM_REQUIRE_ALIGN(table_m, 16);
+    if (table_v != nullptr)
+        LPMM_REQUIRE_ALIGN(table_v, 16);
+    uint32_t m_lg = 0;
+    while (m_lg < 5 && ((int64_t)kGroup << m_lg) < m_group_size)
+        ++m_lg;
+    if (((int64_t)kGroup << m_lg) != m_group_size || (m_lg != 0 && kind != LPMM_RANK1_CODES4))
+        return LPMM_ERR_SIZE;  // 128; 4-bit codes also 256, 512, 1024, 2048, 4096
+    if (kind == LPMM_RANK1_HALF)
+        return passes == 3 ? rank1_any_half(tensors, count, qmap_m, qmap_v, beta1, beta2, lr, weight_decay, eps, stream)
+                           : LPMM_ERR_ARG;
+    return rank1_any_step_multi(tensors, count, (AnyKind)kind, m_lg, qmap_m, bits_m, table_m, qmap_v, bits_v, table_v, beta1,
+                                beta2, lr, weight_decay, eps, passes, stream);
 }

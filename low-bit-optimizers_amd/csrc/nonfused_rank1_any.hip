@@ -1,0 +1,601 @@
+// The two passes of the non-fused AdamW step with a rank-1 second moment for any column count and any
+// alignment, for every kind of state and parameter the tuned kernels serve: 4-bit states (what
+// nonfused_rank1_ragged.hip leaves: columns that are no multiple of 8), an fp32 first moment, 5-8-bit
+// codes and float16 parameters on columns that are no multiple of 128.  Tiles, records and statistics
+// as in nonfused_rank1.hip.
+//
+// What the tuned kernels rely on and these do not: rows that start on a 16-byte boundary and on a whole
+// code byte, and 128-value groups of the first moment that never straddle a row.  Here
+//   * a lane takes columns 16 apart (column block start + 16 k + lane), one value per access, so that
+//     neighbouring lanes touch neighbouring addresses whatever the row's first address is;
+//   * lanes beyond the end of the row work on the row's last value once more and store nothing: their
+//     maxima change nothing, and no access needs a branch;
+//   * the first moment's groups lie in up to two pieces in a DPP row's 128 values; its scale takes the
+//     route of the second moment's statistics (maxima merged by the first pass, codes written by the
+//     second), as in the ragged kernels;
+//   * the new codes go to arrays of their own, as on the staged path (the state's tensors are replaced); two codes
+//     that share a byte may belong to neighbouring lanes (they meet by a lane exchange) or, where the column
+//     count is odd, to different rows: the first pass clears such a byte, the second sets its halves by atomic or.
+// Before, these tensors took the staged path (dequantise, update, statistics, normalise: six to eight
+// launches a tensor and 50 bytes a value; float16: about thirty PyTorch ops a tensor).  One step on one tensor,
+// staged -> here: 4096 x 4100 default 224 -> 107 us, fp32 first moment 183 -> 104, 8 bits 221 -> 102, float16
+// 539 -> 151; 4095 x 4099 271 -> 159; 50000 x 34 122 -> 55 (4096 x 4096 on the tuned kernels: 74-84, float16 67).
+// What bounds them: instructions, the code bytes' extraction and one access per value (the tuned kernels move
+// the same bytes in a quarter of the accesses); most of the gain on small tensors is launches.
+#include "lpmm_half.hpp"
+#include "lpmm_search.hpp"
+
+namespace lpmm {
+
+constexpr int kAnyElts = kEltsPerLane;
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t any_dpp(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
+
+// largest of the DPP row's bit patterns, in every lane
+__device__ __forceinline__ uint32_t row16_umax(uint32_t v)
+{
+    v = max(v, any_dpp<0xB1>(v));   // quad_perm:[1,0,3,2]
+    v = max(v, any_dpp<0x4E>(v));   // quad_perm:[2,3,0,1]
+    v = max(v, any_dpp<0x141>(v));  // row_half_mirror
+    v = max(v, any_dpp<0x140>(v));  // row_mirror
+    return v;
+}
+
+__device__ __forceinline__ uint32_t magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// A DPP row's piece of one tensor row: `count` values (1 .. 128) from flattened index `base` on; the values
+// from `split` on belong to the next group of the first moment.
+struct Piece {
+    int64_t base, group;
+    int count, split;
+};
+
+__device__ __forceinline__ Piece piece_of(int64_t cols, uint32_t cg, int64_t r, int lg_group)
+{
+    Piece w;
+    const int64_t c0 = (int64_t)cg * kGroup;
+    w.base = r * cols + c0;
+    w.count = (int)(cols - c0 < kGroup ? cols - c0 : kGroup);
+    w.group = w.base >> lg_group;
+    const int64_t to_next = ((w.group + 1) << lg_group) - w.base;
+    w.split = to_next < kGroup ? (int)to_next : kGroup;
+    return w;
+}
+
+__device__ __forceinline__ int piece_at(const Piece &w, int lane16, int k)
+{
+    const int off = 16 * k + lane16;
+    return off < w.count ? off : w.count - 1;
+}
+
+// codes of the lane's eight values: element k in bits 4 k (two codes a byte) or in byte k (one a byte)
+template <bool BITS>
+__device__ __forceinline__ uint64_t load_codes(const uint8_t *codes, const Piece &w, int lane16)
+{
+    uint64_t out = 0;
+    if (BITS) {
+        const uint8_t *c = codes + w.base;
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            out |= (uint64_t)c[piece_at(w, lane16, k)] << (8 * k);
+    } else {
+        const uint8_t *c = codes + (w.base >> 1);
+        const int odd = (int)(w.base & 1);
+        uint32_t low = 0;
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k) {
+            const int at = piece_at(w, lane16, k) + odd;
+            low |= (((uint32_t)c[at >> 1] >> (4 * (at & 1))) & 15u) << (4 * k);
+        }
+        out = low;
+    }
+    return out;
+}
+
+// sets one half of a cleared byte; the array is 4-byte aligned and whole words long up to the byte
+__device__ __forceinline__ void set_nibble(uint8_t *at, uint32_t shift, uint32_t code)
+{
+    const uintptr_t a = reinterpret_cast<uintptr_t>(at);
+    atomicOr(reinterpret_cast<uint32_t *>(a & ~(uintptr_t)3), code << (8 * (uint32_t)(a & 3) + shift));
+}
+
+// the bytes that a piece shares with its neighbours
+__device__ __forceinline__ void clear_shared(uint8_t *codes, const Piece &w)
+{
+    const int64_t end = w.base + w.count;
+    if (w.base & 1)
+        codes[w.base >> 1] = 0;
+    if (end & 1)
+        codes[end >> 1] = 0;
+}
+
+__device__ __forceinline__ void store_nibbles(uint8_t *codes, const Piece &w, int lane16, uint32_t now)
+{
+    uint8_t *c = codes + (w.base >> 1);
+    const int odd = (int)(w.base & 1);
+    const bool low = ((lane16 + odd) & 1) == 0;  // the lane's codes are low halves of their bytes
+    // the codes one column on: lane 15's are lane 0's of the next sixteen columns
+    const int lane = threadIdx.x & (kWave - 1);
+    uint32_t next = (uint32_t)__shfl((int)now, (lane & ~15) | ((lane + 1) & 15), kWave);
+    if (lane16 == 15)
+        next >>= 4;
+#pragma unroll
+    for (int k = 0; k < kAnyElts; ++k) {
+        const int off = 16 * k + lane16;
+        if (off >= w.count)
+            continue;
+        const uint32_t a = (now >> (4 * k)) & 15u;
+        uint8_t *at = c + ((off + odd) >> 1);
+        if (low) {
+            if (off + 1 < w.count)
+                *at = (uint8_t)(a | (((next >> (4 * k)) & 15u) << 4));
+            else
+                set_nibble(at, 0, a);  // the other half belongs to the next block, row or the padding
+        } else if (off == 0) {
+            set_nibble(at, 4, a);
+        }
+    }
+}
+
+__device__ __forceinline__ void store_bytes(uint8_t *codes, const Piece &w, int lane16, const uint32_t (&now)[kAnyElts])
+{
+    uint8_t *c = codes + w.base;
+#pragma unroll
+    for (int k = 0; k < kAnyElts; ++k) {
+        const int off = 16 * k + lane16;
+        if (off < w.count)
+            c[off] = (uint8_t)now[k];
+    }
+}
+
+// The codes behind the tensor's n values: `last` up to n_group (the zeros that complete a group are divided by
+// its scale like its other values), `zero` up to whole pack groups, 0 in the extra byte.  One workgroup.
+template <bool BITS>
+__device__ __forceinline__ void any_padding(uint8_t *codes, int64_t n, int64_t n_group, uint32_t last, uint32_t zero)
+{
+    const int64_t n_all = (n_group + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP;
+    if (BITS) {
+        for (int64_t i = n + threadIdx.x; i < n_all; i += kThreads)
+            codes[i] = (uint8_t)(i < n_group ? last : zero);
+        if (threadIdx.x == 0)
+            codes[n_all] = 0;
+        return;
+    }
+    if ((n & 1) != 0 && threadIdx.x == 0)
+        set_nibble(codes + (n >> 1), 4, n < n_group ? last : zero);
+    for (int64_t i = (n + 1) / 2 + threadIdx.x; i < n_all / 2; i += kThreads)
+        codes[i] = (uint8_t)((2 * i < n_group ? last : zero) * 0x11u);
+    if (threadIdx.x == 0)
+        codes[n_all / 2] = 0;
+}
+
+// a code array's map: 2^bits floats
+template <bool BITS>
+__device__ __forceinline__ float any_decode(const float *map, uint64_t codes, int k, uint32_t mask)
+{
+    return map[BITS ? (uint32_t)(codes >> (8 * k)) & mask : (uint32_t)(codes >> (4 * k)) & 15u];
+}
+
+__device__ __forceinline__ float rank1_scale(float co, float ro) { return co < ro ? co : ro; }
+
+// REAL: the parameters' type (h16: the chain of half ops, half scales and statistics, float work arrays for the
+// maxima); M32: fp32 first moment; BITS: one code of bits_m / bits_v bits per byte
+template <typename REAL, bool M32, bool BITS>
+__global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const MultiR1 args, const NewCodes out,
+                                                                       const float *__restrict__ qmap_m,
+                                                                       const float *__restrict__ qmap_v, int bits_m, int bits_v)
+{
+    constexpr bool HALF = sizeof(REAL) == 2;
+    constexpr int kMap = BITS ? 256 : 16;
+    __shared__ float map_m[kMap], map_v[kMap];
+    __shared__ uint32_t colred[kMaxWide * kGroup], rowred[kRowSlots];
+    const int lo = find_tensor(args);
+    const TensorR1 &t = args.t[lo];
+    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
+    const Geometry q = geometry(t, tl, drow);
+    const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
+    fill_map(map_m, qmap_m, BITS ? bits_m : 4);
+    fill_map(map_v, qmap_v, BITS ? bits_v : 4);
+    for (int j = threadIdx.x; j < kMaxWide * kGroup; j += kThreads)
+        colred[j] = 0u;
+    if (threadIdx.x < kRowSlots)
+        rowred[threadIdx.x] = 0u;
+    NfHyper h;
+    h.decay = args.decay;
+    h.w1 = args.w1;
+    h.b2 = args.b2;
+    h.w2 = args.w2;
+    h.eps = args.eps;
+    h.neg_step_size = t.neg_step_size;
+    h.bc2_sqrt = t.bc2_sqrt;
+    h.rbc2_sqrt = t.rbc2_sqrt;
+    __syncthreads();
+
+    const uint32_t mask_m = (1u << bits_m) - 1u, mask_v = (1u << bits_v) - 1u;
+    const int lg_group = 7 + (int)t.m_lg;
+    if (q.cg < t.col_blocks && q.row0 < t.rows) {
+        const REAL *row_old = reinterpret_cast<const REAL *>(t.row_old);
+        const REAL *col_old = reinterpret_cast<const REAL *>(t.col_old) + (int64_t)q.cg * kGroup;
+        const REAL *ms = reinterpret_cast<const REAL *>(t.ms);
+        const Piece first = piece_of(cols, q.cg, q.row0, lg_group);
+        REAL co[kAnyElts];
+        uint32_t vtop[kAnyElts];  // the lane's columns: current statistics, maxima over its passes
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k) {
+            co[k] = col_old[piece_at(first, lane16, k)];
+            vtop[k] = 0u;
+        }
+#pragma unroll 1
+        for (int it = 0; it < q.passes; ++it) {
+            const int64_t r = q.row0 + (int64_t)it * q.step;
+            if (r >= t.rows)
+                break;
+            const Piece w = piece_of(cols, q.cg, r, lg_group);
+            REAL *pp = reinterpret_cast<REAL *>(t.p) + w.base;
+            const REAL *gp = reinterpret_cast<const REAL *>(t.g) + w.base;
+            float *mp = reinterpret_cast<float *>(t.mc) + w.base;
+            REAL p[kAnyElts], g[kAnyElts];
+            float m[kAnyElts], v[kAnyElts];
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k) {
+                p[k] = pp[piece_at(w, lane16, k)];
+                g[k] = gp[piece_at(w, lane16, k)];
+            }
+            const uint64_t vc = load_codes<BITS>(t.vc, w, lane16);
+            const REAL ro = row_old[r];
+            if (M32) {
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k)
+                    m[k] = mp[piece_at(w, lane16, k)];
+            } else {
+                const uint64_t mc = load_codes<BITS>(t.mc, w, lane16);
+                const float s0 = (float)ms[w.group], s1 = w.split < w.count ? (float)ms[w.group + 1] : 0.0f;
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k)
+                    m[k] = any_decode<BITS>(map_m, mc, k, mask_m) * (piece_at(w, lane16, k) < w.split ? s0 : s1);
+            }
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k)
+                v[k] = any_decode<BITS>(map_v, vc, k, mask_v) * rank1_scale((float)co[k], (float)ro);
+            if constexpr (HALF) {
+                const MixConst c = mix_const();
+                v2h p2[kPairs], g2[kPairs], m2[kPairs], v2[kPairs];
+#pragma unroll
+                for (int j = 0; j < kPairs; ++j) {
+                    p2[j] = v2h{p[2 * j], p[2 * j + 1]};
+                    g2[j] = v2h{g[2 * j], g[2 * j + 1]};
+                    m2[j] = round2(m[2 * j], m[2 * j + 1]);
+                    v2[j] = round2(v[2 * j], v[2 * j + 1]);
+                }
+                half_elts8<true>(p2, g2, m2, v2, h, c);
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k) {
+                    p[k] = p2[k >> 1][k & 1];
+                    m[k] = (float)m2[k >> 1][k & 1];
+                    v[k] = (float)v2[k >> 1][k & 1];
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k)
+                    nonfused_elt(p[k], g[k], m[k], v[k], h);
+            }
+            uint32_t vmax = 0u;
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k) {
+                vtop[k] = max(vtop[k], magnitude(v[k]));
+                vmax = max(vmax, magnitude(v[k]));
+            }
+            vmax = row16_umax(vmax);
+            if (!M32) {
+                // float: a NaN is left out, as by the block-wise quantiser; half: it is the maximum, as in torch's
+                float m0 = 0.0f, m1 = 0.0f;
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k) {
+                    const bool here = piece_at(w, lane16, k) < w.split;
+                    if (HALF) {
+                        m0 = __uint_as_float(max(__float_as_uint(m0), here ? magnitude(m[k]) : 0u));
+                        m1 = __uint_as_float(max(__float_as_uint(m1), here ? 0u : magnitude(m[k])));
+                    } else {
+                        m0 = fmaxf(m0, here ? fabsf(m[k]) : 0.0f);
+                        m1 = fmaxf(m1, here ? 0.0f : fabsf(m[k]));
+                    }
+                }
+                m0 = __uint_as_float(row16_umax(__float_as_uint(m0)));
+                m1 = __uint_as_float(row16_umax(__float_as_uint(m1)));
+                if (lane16 == 0) {
+                    // zero changes nothing: the next scales start there
+                    if (__float_as_uint(m0) != 0u)
+                        atomic_max_nonneg(t.ms_new + w.group, m0);
+                    if (__float_as_uint(m1) != 0u)
+                        atomic_max_nonneg(t.ms_new + w.group + 1, m1);
+                }
+            }
+            if (lane16 == 0) {
+                atomicMax(rowred + row_slot(t.tile, it, drow), vmax);
+                if (!BITS) {
+                    clear_shared(out.v[lo], w);
+                    if (!M32)
+                        clear_shared(out.m[lo], w);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k) {
+                const int off = 16 * k + lane16;
+                if (off < w.count) {
+                    pp[off] = p[k];
+                    if (M32)
+                        mp[off] = m[k];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            atomicMax(colred + (drow & (q.wide - 1)) * kGroup + piece_at(first, lane16, k), vtop[k]);
+    }
+    __syncthreads();
+    flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
+    const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
+    for (int j = threadIdx.x; j < q.wide * kGroup; j += kThreads)
+        if (tile_c0 + j < cols)
+            atomic_max_nonneg(t.col_new + tile_c0 + j, __uint_as_float(colred[j]));
+}
+
+template <bool BITS>
+struct AnyCoder;
+
+// 4-bit codes: both maps and the encode table in one LDS array
+template <>
+struct AnyCoder<false> {
+    struct Lds {
+        __align__(16) uint32_t w[kLdsBytes / 4];
+    };
+    Lds &l;
+    int kind[2];
+
+    __device__ __forceinline__ AnyCoder(Lds &lds, const float *qm, const float *qv, int, int, const uint32_t *, const uint32_t *) : l(lds)
+    {
+        lds_fill(l.w, qm, qv);
+        kind[0] = classify_map(qm);
+        kind[1] = classify_map(qv);
+    }
+    __device__ __forceinline__ void ready() {}
+    __device__ __forceinline__ const float *map(int which) const { return reinterpret_cast<const float *>(l.w) + 16 * which; }
+    __device__ __forceinline__ uint32_t one(int which, float x) const
+    {
+        const float xs[kAnyElts] = {x, x, x, x, x, x, x, x};
+        return encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], xs) & 15u;
+    }
+    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16) const
+    {
+        store_nibbles(codes, w, lane16, encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], x));
+    }
+};
+
+template <>
+struct AnyCoder<true> {
+    struct Lds {
+        float map[2][256];
+        SearchLds search[2];
+        BucketLds bucket[2];
+    };
+    Lds &l;
+    int bits[2];
+    uint32_t mode[2];
+    bool even[2];
+
+    __device__ __forceinline__ AnyCoder(Lds &lds, const float *qm, const float *qv, int bm, int bv, const uint32_t *tm, const uint32_t *tv) : l(lds)
+    {
+        const float *q[2] = {qm, qv};
+        const uint32_t *table[2] = {tm, tv};
+        bits[0] = bm;
+        bits[1] = bv;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            mode[i] = code_table_mode(code_table_tag(table[i]), bits[i]);
+            fill_map(l.map[i], q[i], bits[i]);
+            if (mode[i] == kCodeTable)
+                code_table_store(l.bucket[i], code_table_load(table[i]));
+            else if (mode[i] == kCodeSearch)
+                fill_search(l.search[i], q[i], bits[i]);
+        }
+    }
+    // after the barrier that follows the constructor
+    __device__ __forceinline__ void ready()
+    {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            even[i] = mode[i] == kCodeEven || (mode[i] == kCodeSearch && map_is_even(l.search[i]));
+    }
+    __device__ __forceinline__ const float *map(int which) const { return l.map[which]; }
+    __device__ __forceinline__ uint32_t one(int which, float x) const
+    {
+        return code1_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], x);
+    }
+    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16) const
+    {
+        uint32_t c[kAnyElts];
+        codes8_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], even[which], x, c);
+        store_bytes(codes, w, lane16, c);
+    }
+};
+
+// x[k] / s[k], rounded to half where the chain is one of half ops.  Every scale is a maximum over the values it
+// divides, so where all of a wave's scales lie in the range in which the reciprocal is exact, one product and two
+// fmas are the correctly rounded quotient.
+template <bool HALF>
+__device__ __forceinline__ void any_quotients(float (&x)[kAnyElts], const float (&s)[kAnyElts])
+{
+    bool safe = true;
+#pragma unroll
+    for (int k = 0; k < kAnyElts; ++k)
+        safe = safe && rc_safe(s[k]);
+    if (__all(safe)) {
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            x[k] = div_by_rc(x[k], s[k], rcp_exact(s[k]));
+    } else {
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            x[k] = x[k] / s[k];
+    }
+    if (HALF)
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            x[k] = rh(x[k]);
+}
+
+template <typename REAL, bool M32, bool BITS>
+__global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const MultiR1 args, const NewCodes out,
+                                                                        const float *__restrict__ qmap_m,
+                                                                        const float *__restrict__ qmap_v, int bits_m, int bits_v,
+                                                                        const uint32_t *__restrict__ table_m,
+                                                                        const uint32_t *__restrict__ table_v)
+{
+    constexpr bool HALF = sizeof(REAL) == 2;
+    __shared__ typename AnyCoder<BITS>::Lds lds;
+    AnyCoder<BITS> coder(lds, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v);
+    const int lo = find_tensor(args);
+    const TensorR1 &t = args.t[lo];
+    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
+    const Geometry q = geometry(t, tl, drow);
+    const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
+    NfHyper h;
+    h.b2 = args.b2;
+    h.w2 = args.w2;
+    h.w1 = args.w1;
+    __syncthreads();
+    coder.ready();
+
+    const uint32_t mask_m = (1u << bits_m) - 1u, mask_v = (1u << bits_v) - 1u;
+    const int lg_group = 7 + (int)t.m_lg;
+    if (tl == 0) {
+        const int64_t n = t.rows * cols;
+        const uint32_t zero_v = coder.one(1, 0.0f);
+        any_padding<BITS>(out.v[lo], n, n, zero_v, zero_v);
+        if (!M32) {
+            const int64_t group = (int64_t)1 << lg_group, n_group = (n + group - 1) / group * group;
+            const float last = 0.0f / t.ms_new[(n - 1) >> lg_group];
+            any_padding<BITS>(out.m[lo], n, n_group, coder.one(0, last), coder.one(0, 0.0f));
+        }
+    }
+    if (q.cg >= t.col_blocks || q.row0 >= t.rows)
+        return;
+    const REAL *row_old = reinterpret_cast<const REAL *>(t.row_old);
+    const REAL *col_old = reinterpret_cast<const REAL *>(t.col_old) + (int64_t)q.cg * kGroup;
+    const float *col_new = t.col_new + (int64_t)q.cg * kGroup;
+    const REAL *ms = reinterpret_cast<const REAL *>(t.ms);
+    const Piece first = piece_of(cols, q.cg, q.row0, lg_group);
+    REAL co[kAnyElts];
+    float cn[kAnyElts];
+#pragma unroll
+    for (int k = 0; k < kAnyElts; ++k) {
+        co[k] = col_old[piece_at(first, lane16, k)];
+        cn[k] = col_new[piece_at(first, lane16, k)];
+    }
+    const MixConst c = mix_const();
+#pragma unroll 1
+    for (int it = 0; it < q.passes; ++it) {
+        const int64_t r = q.row0 + (int64_t)it * q.step;
+        if (r >= t.rows)
+            break;
+        const Piece w = piece_of(cols, q.cg, r, lg_group);
+        const REAL *gp = reinterpret_cast<const REAL *>(t.g) + w.base;
+        REAL g[kAnyElts];
+        float x[kAnyElts], s[kAnyElts];
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            g[k] = gp[piece_at(w, lane16, k)];
+        const uint64_t vc = load_codes<BITS>(t.vc, w, lane16);
+        const uint64_t mc = M32 ? 0 : load_codes<BITS>(t.mc, w, lane16);
+        const REAL ro = row_old[r];
+        const float rn = t.row_new[r];
+        if (!M32) {
+            const bool two = w.split < w.count;
+            const float s0 = (float)ms[w.group], s1 = two ? (float)ms[w.group + 1] : 0.0f;
+            const float n0 = t.ms_new[w.group], n1 = two ? t.ms_new[w.group + 1] : n0;
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k) {
+                const bool here = piece_at(w, lane16, k) < w.split;
+                x[k] = any_decode<BITS>(coder.map(0), mc, k, mask_m) * (here ? s0 : s1);
+                s[k] = here ? n0 : n1;
+            }
+            if constexpr (HALF) {
+#pragma unroll
+                for (int j = 0; j < kPairs; ++j) {
+                    const v2h a = round2(x[2 * j], x[2 * j + 1]);
+                    v2h b;
+                    if (fabsf(h.w1) < 0.5f)
+                        b = round2(half_lerp<true>(a.x, g[2 * j], h.w1, c), half_lerp<true>(a.y, g[2 * j + 1], h.w1, c));
+                    else
+                        b = round2(half_lerp<false>(a.x, g[2 * j], h.w1, c), half_lerp<false>(a.y, g[2 * j + 1], h.w1, c));
+                    x[2 * j] = (float)b.x;
+                    x[2 * j + 1] = (float)b.y;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < kAnyElts; ++k)
+                    x[k] = lerp_w(x[k], g[k], h.w1);
+            }
+            any_quotients<HALF>(x, s);
+            coder.store(0, x, out.m[lo], w, lane16);
+        }
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k) {
+            x[k] = any_decode<BITS>(coder.map(1), vc, k, mask_v) * rank1_scale((float)co[k], (float)ro);
+            s[k] = rank1_scale(cn[k], rn);
+        }
+        if constexpr (HALF) {
+#pragma unroll
+            for (int j = 0; j < kPairs; ++j) {
+                const v2h b = half_second_moment(round2(x[2 * j], x[2 * j + 1]), v2h{g[2 * j], g[2 * j + 1]}, h, c);
+                x[2 * j] = (float)b.x;
+                x[2 * j + 1] = (float)b.y;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kAnyElts; ++k)
+                nonfused_second_moment(x[k], g[k], h);
+        }
+        any_quotients<HALF>(x, s);
+        coder.store(1, x, out.v[lo], w, lane16);
+    }
+}
+
+template <typename REAL, bool M32, bool BITS>
+static void launch(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v, int bits_m, int bits_v,
+                   const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
+{
+    if (passes & 1)
+        hipLaunchKernelGGL((rank1_update_any_kernel<REAL, M32, BITS>), dim3(tiles), dim3(kThreads), 0, stream, args, out, qmap_m,
+                           qmap_v, bits_m, bits_v);
+    if (passes & 2)
+        hipLaunchKernelGGL((rank1_requant_any_kernel<REAL, M32, BITS>), dim3(tiles), dim3(kThreads), 0, stream, args, out, qmap_m,
+                           qmap_v, bits_m, bits_v, table_m, table_v);
+}
+
+void launch_rank1_any(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v, AnyKind kind, int bits_m,
+                      int bits_v, const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
+{
+    switch (kind) {
+    case kAnyCodes4:
+        launch<float, false, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        break;
+    case kAnyFloatM:
+        launch<float, true, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        break;
+    case kAnyBits:
+        launch<float, false, true>(args, out, tiles, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
+        break;
+    case kAnyHalf:
+        launch<h16, false, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        break;
+    }
+}
+
+}  // namespace lpmm

@@ -216,9 +216,29 @@ void launch_rank1_bits(const MultiR1 &args, uint32_t tiles, const float *qmap_m,
                        int bits_v, const uint32_t *table_m, const uint32_t *table_v, hipStream_t stream);
 void launch_rank1_ragged(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v,
                          hipStream_t stream);
+// any column count and alignment (nonfused_rank1_any.hip)
+enum AnyKind : int {
+    kAnyCodes4 = LPMM_RANK1_CODES4,
+    kAnyFloatM = LPMM_RANK1_FLOAT_M,
+    kAnyBits = LPMM_RANK1_CODES8,
+    kAnyHalf = LPMM_RANK1_HALF
+};
+struct NewCodes {  // where the second pass puts a tensor's codes
+    uint8_t *m[kR1Max], *v[kR1Max];
+};
+// passes: 1 the first, 2 the second, 3 both
+void launch_rank1_any(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v,
+                      AnyKind kind, int bits_m, int bits_v, const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream);
 // float16 parameters (nonfused_half.hip): p, g, the first moment's scales and the current statistics
 // of the records point at halfs, the next statistics at float work arrays
 void launch_rank1_half(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v, hipStream_t stream);
+// the records of lpmm_nonfused_adamw_rank1_any_step_multi; float16: the next statistics and scales of the records are
+// float work arrays (rank1_any_half sets them up and writes the halfs out)
+int rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg, const float *qmap_m,
+                         int bits_m, const void *table_m, const float *qmap_v, int bits_v, const void *table_v, double beta1,
+                         double beta2, double lr, double weight_decay, double eps, int passes, void *stream);
+int rank1_any_half(const lpmm_rank1_any_tensor *tensors, int64_t count, const float *qmap_m, const float *qmap_v, double beta1,
+                   double beta2, double lr, double weight_decay, double eps, void *stream);
 int rank1_step_multi_half(const lpmm_nonfused_rank1_tensor *tensors, int64_t count, const float *qmap_m,
                           const float *qmap_v, double beta1, double beta2, double lr, double weight_decay, double eps,
                           void *stream);

@@ -55,6 +55,7 @@ PROTOTYPES = {
     "lpmm_dequant_rank1_bits": (_int, [_vp, _vp, _vp, _vp, _int, _i64, _i64, _vp, _vp]),
     "lpmm_nonfused_update": (_int, [_vp] * 4 + [_i64] + [_d] * 6 + [_vp]),
     "lpmm_nonfused_update_multi": (_int, [_vp, _i64] + [_d] * 5 + [_vp]),
+    "lpmm_nonfused_update_f16_multi": (_int, [_vp, _i64] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw4bit_step_multi": (_int, [_vp, _i64, _vp, _vp] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw4bit_rank1_step_multi": (_int, [_vp, _i64, _vp, _vp] + [_d] * 5 + [_vp]),
     "lpmm_rank1_small_fold_scale_multi": (_int, [_vp, _i64, _vp]),
@@ -66,6 +67,8 @@ PROTOTYPES = {
     "lpmm_nonfused_adamw4bit_rank1_mgroup_step_multi": (_int, [_vp, _i64, _vp, _vp, _i64] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw_bits_rank1_step_multi": (_int, [_vp, _i64, _vp, _int, _vp, _int] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw_bits_rank1_step_multi_table": (_int, [_vp, _i64, _vp, _int, _vp, _vp, _int, _vp] + [_d] * 5 + [_vp]),
+    "lpmm_nonfused_adamw_rank1_any_step_multi": (_int, [_vp, _i64, _int, _i64, _vp, _int, _vp, _vp, _int, _vp] + [_d] * 5
+                                                 + [_int, _vp]),
     "lpmm_factored_workspace_bytes": (_i64, [_i64, _i64]),
     "lpmm_factored_stats": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _d, _vp, _vp]),
     "lpmm_factored_stats_static": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _d, _vp]),
@@ -73,10 +76,10 @@ PROTOTYPES = {
     "lpmm_factored_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
     "lpmm_factored_update_fp32m": (_int, [_vp] * 6 + [_i64, _i64] + [_d] * 6 + [_vp]),
     "lpmm_sgd4bit_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 4 + [_int, _int, _vp]),
+    "lpmm_sgd_fp32_step_multi": (_int, [_vp, _i64] + [_d] * 4 + [_int, _int, _vp]),
     "lpmm_stream_probe": (_int, [_int] + [_vp] * 6 + [_i64, _i64, _vp]),
     "lpmm_selftest_encoders": (_int, [_vp, _vp]),
     "lpmm_selftest_bucket_encoder": (_int, [_vp, _int, _vp, _vp]),
-    "lpmm_sgd_fp32_step_multi": (_int, [_vp, _i64] + [_d] * 4 + [_int, _int, _vp]),
     "lpmm_selftest_arithmetic": (_int, [_vp, ctypes.c_uint32, ctypes.c_uint64, ctypes.c_uint32, _vp]),
 }
 
@@ -104,11 +107,19 @@ RANK1_MGROUP_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("m_codes", "<u8"), 
                                 ("m_max1_next", "<u8"), ("v_codes", "<u8"), ("v_rowmax", "<u8"), ("v_colmax", "<u8"),
                                 ("v_rowmax_next", "<u8"), ("v_colmax_next", "<u8"), ("rows", "<i8"), ("cols", "<i8"),
                                 ("step", "<f4"), ("reserved", "<f4")])
+# tensors of any column count and alignment; kinds: LPMM_RANK1_* of include/lpmm_hip.h
+RANK1_ANY_TENSOR = np.dtype([(k, "<u8") for k in ("p", "g", "m", "m_codes_next", "m_max1", "m_max1_next", "v_codes",
+                                                  "v_codes_next", "v_rowmax", "v_colmax", "v_rowmax_next",
+                                                  "v_colmax_next", "work")]
+                            + [("rows", "<i8"), ("cols", "<i8"), ("step", "<f4"), ("reserved", "<f4")])
+RANK1_CODES4, RANK1_FLOAT_M, RANK1_CODES8, RANK1_HALF = range(4)
 FACTORED_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("m_codes", "<u8"), ("m_max1", "<u8"), ("row", "<u8"),
                             ("col", "<u8"), ("workspace", "<u8"), ("rows", "<i8"), ("cols", "<i8"), ("step", "<f4"),
                             ("first_step", "<i4")])
 SGD4BIT_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("m_codes", "<u8"), ("m_max1", "<u8"), ("n", "<i8"),
                            ("first_step", "<i4"), ("reserved", "<i4")])
+SGD_FP32_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("buf", "<u8"), ("n", "<i8"), ("first_step", "<i4"),
+                            ("reserved", "<i4")])
 ADAMW_FP32_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("m", "<u8"), ("v", "<u8"), ("n", "<i8"),
                               ("step", "<f4"), ("reserved", "<f4")])
 
@@ -118,8 +129,6 @@ _lib = None
 def lib():
     """The loaded library; raises RuntimeError when it has not been built."""
     global _lib
-SGD_FP32_TENSOR = np.dtype([("p", "<u8"), ("g", "<u8"), ("buf", "<u8"), ("n", "<i8"), ("first_step", "<i4"),
-                            ("reserved", "<i4")])
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(

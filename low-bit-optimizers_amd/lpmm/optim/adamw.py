@@ -35,6 +35,13 @@ def _two_pass_columns(rows, cols):
     return cols % 128 == 0 or (cols % 128 == 64 and rows % 2 == 0)
 
 
+def _any_columns(rows, cols):
+    """Matrices that the two passes for any column count take (50000 x 34: 54 us a step, staged 122; 8192 x 6: 52,
+    staged 112-118).  A row costs them a block of 128 columns, so long matrices of a few columns stay with the
+    staged path (200000 x 20 takes 128 us there; the passes would work on 26 million values)."""
+    return rows > 0 and (cols >= 32 or (cols > 0 and rows <= 32768))
+
+
 def _two_pass_nd(shape):
     """Tensors of more than two dimensions that take the two passes on their shape[0] x rest view.  The
     kernels' tiles are 64 rows tall: a large tensor with a handful of rows (a stack of a few matrices)
@@ -44,7 +51,7 @@ def _two_pass_nd(shape):
     rows, numel = shape[0], 1
     for d in shape:
         numel *= d
-    if rows == 0 or not _two_pass_columns(rows, numel // rows):
+    if rows == 0 or not _any_columns(rows, numel // rows):
         return False
     return rows >= 16 or numel <= (1 << 20)
 
@@ -407,7 +414,8 @@ class AdamW(LowBitOptimizer):
             _native.check(st, "non-fused 4-bit AdamW step (rank-1 second moment)")
             records.launched()
 
-        half_flat, half_rank1 = {}, {}  # float16 parameters
+        half_flat, half_rank1, half_plain = {}, {}, {}  # float16 parameters
+        any_rank1 = {}  # matrices of any column count: (kind, device, maps) -> records
 
         def launch_half_flat(key, records):
             dev, qm_ptr, qv_ptr = key
@@ -425,6 +433,17 @@ class AdamW(LowBitOptimizer):
                                                                       beta1, beta2, lr, wd, eps,
                                                                       _native.current_stream(dev))
             _native.check(st, "non-fused 4-bit AdamW step on float16 parameters (rank-1 second moment)")
+            records.launched()
+
+        def launch_any(key, records):
+            kind, dev, qm_ptr, qv_ptr, tm_ptr, tv_ptr = key[:6]
+            table = np.array(records, dtype=_native.RANK1_ANY_TENSOR)
+            bits = (md_m["b"], md_v["b"]) if kind == _native.RANK1_CODES8 else (4, 4)
+            with torch.cuda.device(dev):
+                st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(
+                    table.ctypes.data, len(records), kind, md_m["gp_sz"] if kind == _native.RANK1_CODES4 else 128, qm_ptr, bits[0],
+                    tm_ptr, qv_ptr, bits[1], tv_ptr, beta1, beta2, lr, wd, eps, 3, _native.current_stream(dev))
+            _native.check(st, "non-fused AdamW step (rank-1 second moment, any column count)")
             records.launched()
 
         def launch_group_m32(key, records):
@@ -477,7 +496,24 @@ class AdamW(LowBitOptimizer):
                     continue
                 key = (p.device, state["exp_avg_qstate"]["qmap"].data_ptr(),
                        state["exp_avg_sq_qstate"]["qmap"].data_ptr())
-                if kind == "flat":
+                if kind == "plain":
+                    for name in ("exp_avg", "exp_avg_sq"):
+                        if _is_placeholder(state[name]):
+                            state[name] = torch.zeros_like(p, memory_format=torch.contiguous_format)
+                    half_plain.setdefault(p.device, []).append(
+                        (p.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), state["exp_avg_sq"].data_ptr(),
+                         p.numel(), step, 0.0))
+                elif kind == "any":
+                    pending = any_rank1.setdefault((_native.RANK1_HALF,) + key + (None, None), _Batch())
+                    mc, ms, ms_next = self._group_state_pair(p, state, pending)
+                    vc, *stats = self._rank1_state_f16(p, state, pending, with_groups=True)
+                    pending.append((p.data_ptr(), grad.data_ptr(), mc, self._next_codes(state, "exp_avg", pending), ms, ms_next,
+                                    vc, self._next_codes(state, "exp_avg_sq", pending)) + tuple(stats)
+                                   + (p.shape[0], p.shape[1], step, 0.0))
+                    if len(pending) == _native.RANK1_MULTI_MAX:
+                        launch_any((_native.RANK1_HALF,) + key + (None, None), pending)
+                        pending.clear()
+                elif kind == "flat":
                     pending = half_flat.setdefault(key, [])
                     pending.append(self._nonfused_record(p, p, grad, state, step, v_rank1))
                     if len(pending) == _native.MULTI_MAX:
@@ -539,25 +575,40 @@ class AdamW(LowBitOptimizer):
                 key = (p.device, state["exp_avg_qstate"]["qmap"].data_ptr(),
                        state["exp_avg_sq_qstate"]["qmap"].data_ptr(), ragged)
                 pending = batched_rank1_mgroup.setdefault(key, _Batch())
-                mc, _ = self._group_state(p, state, "exp_avg", md_m["gp_sz"])
-                # the scales trade places with a second buffer, like the second moment's statistics
-                oh = state["exp_avg_qstate"]["overhead"]
-                cur = oh["max1"]
-                nxt = self._spare_scales.get(p)
-                if nxt is None or nxt.device != cur.device or nxt.shape != cur.shape:
-                    nxt = torch.empty_like(cur)
-
-                def commit(p=p, oh=oh, cur=cur, nxt=nxt):
-                    self._spare_scales[p] = cur
-                    oh["max1"] = nxt
-
-                pending.commits.append(commit)
-                pending.append((dense.data_ptr(), grad.data_ptr(), mc, cur.data_ptr(), nxt.data_ptr())
+                pending.append((dense.data_ptr(), grad.data_ptr())
+                               + self._group_state_pair(p, state, pending, md_m["gp_sz"])
                                + self._rank1_state(p, state, pending) + (p.shape[0], p.shape[1], step, 0.0))
                 if len(pending) == _native.RANK1_MULTI_MAX:
                     launch_rank1_mgroup(key, pending)
                     pending.clear()
                 continue
+            # every other matrix under a rank-1 second moment: any column count
+            if en_v and p.dim() == 2 and _any_columns(p.shape[0], p.shape[1]):
+                kind, qm = None, state["exp_avg_qstate"]["qmap"]
+                qv, tables = state["exp_avg_sq_qstate"]["qmap"], (None, None)
+                if en_m and v_rank1 and (m_group128 or m_group_wide):
+                    kind = _native.RANK1_CODES4
+                elif en_m and bits_rank1:
+                    kind = _native.RANK1_CODES8
+                    tables = (code_table(qm, md_m["b"]).data_ptr(), code_table(qv, md_v["b"]).data_ptr())
+                elif not en_m and v_rank1 and (p.shape[1] % 128 != 0 or dense.data_ptr() % 16 or grad.data_ptr() % 16):
+                    kind = _native.RANK1_FLOAT_M
+                if kind is not None:
+                    key = (kind, p.device, qm.data_ptr(), qv.data_ptr()) + tables
+                    pending = any_rank1.setdefault(key, _Batch())
+                    if kind == _native.RANK1_FLOAT_M:
+                        first = (self._materialise(p, state, "exp_avg", False, md_m).data_ptr(), 0, 0, 0)
+                    else:
+                        mc, ms, ms_next = self._group_state_pair(p, state, pending, md_m["gp_sz"], md_m["b"])
+                        first = (mc, self._next_codes(state, "exp_avg", pending), ms, ms_next)
+                    vc, *stats = self._rank1_state(p, state, pending, b=md_v["b"])
+                    pending.append((dense.data_ptr(), grad.data_ptr()) + first
+                                   + (vc, self._next_codes(state, "exp_avg_sq", pending)) + tuple(stats)
+                                   + (0, p.shape[0], p.shape[1], step, 0.0))
+                    if len(pending) == _native.RANK1_MULTI_MAX:
+                        launch_any(key, pending)
+                        pending.clear()
+                    continue
             m = self._materialise(p, state, "exp_avg", en_m, md_m)
             if not en_m and en_v:
                 # only the second moment is quantised: the first is read and written as floats
@@ -614,6 +665,15 @@ class AdamW(LowBitOptimizer):
         for key, records in half_rank1.items():
             if records:
                 launch_half_rank1(key, records)
+        for key, records in any_rank1.items():
+            if records:
+                launch_any(key, records)
+        for dev, records in half_plain.items():
+            table = np.array(records, dtype=_native.ADAMW_FP32_TENSOR)
+            with torch.cuda.device(dev):
+                st = lib.lpmm_nonfused_update_f16_multi(table.ctypes.data, len(records), beta1, beta2, lr, wd, eps,
+                                                        _native.current_stream(dev))
+            _native.check(st, "non-fused AdamW update on float16 states")
         for key, records in batched_rank1_mgroup.items():
             if records:
                 launch_rank1_mgroup(key, records)
@@ -631,13 +691,22 @@ class AdamW(LowBitOptimizer):
     def _half_kernel_kind(self, p, grad, state, m_group128, v_group128, v_rank1):
         """Which HIP step takes a float16 parameter on the non-fused path: "flat" (one pass: both moments
         block-wise over 128 values, a vector under 'rank1' included), "rank1" (two passes: a matrix with
-        a multiple of 128 columns), or None for the chain of PyTorch ops (float64, strided operands,
-        unquantised or differently scaled states, states whose scales are not halfs)."""
+        a multiple of 128 columns), "any" (the passes for any other matrix), "plain" (states that are not
+        quantised), or None for the chain of PyTorch ops (float64, strided operands, differently scaled states,
+        states whose scales are not halfs)."""
         if p.dtype is not torch.float16 or grad.dtype is not torch.float16 or not (p.is_cuda and grad.is_cuda):
             return None
-        if not (p.is_contiguous() and grad.is_contiguous() and m_group128):
+        if not (p.is_contiguous() and grad.is_contiguous()):
             return None
-        if not (self._enabled(p, state, "exp_avg") and self._enabled(p, state, "exp_avg_sq")):
+        en_m, en_v = self._enabled(p, state, "exp_avg"), self._enabled(p, state, "exp_avg_sq")
+        if not en_m and not en_v:
+            for name in ("exp_avg", "exp_avg_sq"):
+                t = state[name]
+                if not _is_placeholder(t) and not (t.dtype is torch.float16 and t.is_cuda and t.is_contiguous()
+                                                   and t.shape == p.shape):
+                    return None
+            return "plain"
+        if not (en_m and en_v and m_group128):
             return None
         for name in ("exp_avg", "exp_avg_sq"):
             if state[f"{name}_qstate"]["qmap"].dtype is not torch.float32:
@@ -652,11 +721,14 @@ class AdamW(LowBitOptimizer):
         if (v_rank1 and p.dim() == 2 and p.shape[1] % 128 == 0 and p.shape[0] > 0
                 and p.data_ptr() % 16 == 0 and grad.data_ptr() % 16 == 0):
             return "rank1"
+        if v_rank1 and p.dim() == 2 and _any_columns(p.shape[0], p.shape[1]):
+            return "any"
         return None
 
-    def _rank1_state_f16(self, p, state, batch):
+    def _rank1_state_f16(self, p, state, batch, with_groups=False):
         """_rank1_state for float16 parameters: half statistics, and a float work array in which the
-        kernels take the maxima of the new second moment (kept until the launch is enqueued)."""
+        kernels take the maxima of the new second moment (with_groups: and of the first moment's groups; kept
+        until the launch is enqueued)."""
         rows, cols = p.shape
         dev = p.device
         qs_v = state["exp_avg_sq_qstate"]
@@ -673,7 +745,8 @@ class AdamW(LowBitOptimizer):
         nxt = self._spare_stats.get(p)
         if nxt is None or nxt[0].device != dev or nxt[0].dtype is not torch.float16:
             nxt = [torch.empty_like(cur[0]), torch.empty_like(cur[1])]
-        work = torch.empty(((rows + 3) // 4 * 4 + cols,), dtype=torch.float32, device=dev)
+        work = torch.empty(((rows + 3) // 4 * 4 + cols + ((rows * cols + 127) // 128 if with_groups else 0),),
+                           dtype=torch.float32, device=dev)
 
         def commit(work=work):  # holds the work array until the kernels are on the stream
             self._spare_stats[p] = cur
@@ -749,6 +822,35 @@ class AdamW(LowBitOptimizer):
                 oh["dim"] = 1
         return state[name].data_ptr(), qstate["overhead"]["max1"].data_ptr()
 
+    def _group_state_pair(self, p, state, batch, gp_sz=128, b=4):
+        """Pointers to the first moment's codes and scales and to the buffer that receives its next scales; the two
+        trade places once the launch is enqueued, like the second moment's statistics."""
+        codes, _ = self._group_state(p, state, "exp_avg", gp_sz, b)
+        oh = state["exp_avg_qstate"]["overhead"]
+        cur = oh["max1"]
+        nxt = self._spare_scales.get(p)
+        if nxt is None or nxt.device != cur.device or nxt.shape != cur.shape:
+            nxt = torch.empty_like(cur)
+
+        def commit():
+            self._spare_scales[p] = cur
+            oh["max1"] = nxt
+
+        batch.commits.append(commit)
+        return codes, cur.data_ptr(), nxt.data_ptr()
+
+    @staticmethod
+    def _next_codes(state, name, batch):
+        """Pointer to the array that receives a state's new codes; it becomes the state once the launch is
+        enqueued.  (The kernels for any column count do not write codes in place.)"""
+        nxt = torch.empty_like(state[name])
+
+        def commit():
+            state[name] = nxt
+
+        batch.commits.append(commit)
+        return nxt.data_ptr()
+
     def _rank1_state(self, p, state, batch, b=4):
         """Pointers to the codes of a rank-1 scaled second moment, the statistics they are scaled
         by and the pair of buffers that receives the next statistics; creates the state on first
@@ -808,13 +910,18 @@ class AdamW(LowBitOptimizer):
         beta1, beta2 = group["betas"]
         lr, wd, eps = group["lr"], group["weight_decay"], group["eps"]
         batch = _Batch()
-        first, second, between = [], [], []
+        # per kind of launch -- whole 128-column blocks, any other column count -- the records of each pass
+        passes, between = [([], []), ([], [])], []
         with torch.cuda.device(dev):
             stream = _native.current_stream(dev)
             for p, dense, grad, state, step in items:
                 rows, cols = p.shape[0], p.numel() // p.shape[0]
                 trailing = tuple(p.shape[1:]) + (1,)  # lpmm_rank1_row_scale_nd leaves the last dimension out
-                mc, ms = self._group_state(p, state, "exp_avg")
+                whole = _two_pass_columns(rows, cols)
+                if whole:
+                    mc, ms = self._group_state(p, state, "exp_avg")
+                else:
+                    mc, ms, ms_next = self._group_state_pair(p, state, batch)
                 vc, cur, nxt = self._rank1_nd_state(p, state, batch)
                 scratch = self._nd_scratch.get(p)
                 if scratch is None or scratch["work"].device != p.device:
@@ -832,42 +939,56 @@ class AdamW(LowBitOptimizer):
                                                      _shape_array(trailing), work[0].data_ptr(), stream)
                     _native.check(st, "rank1_row_scale_nd")
                 raw_row, new_row = [r for r in range(3) if r != old_row]
-                head = (dense.data_ptr(), grad.data_ptr(), mc, ms, vc, cur[0].data_ptr(), work[old_row].data_ptr(),
-                        nxt[0].data_ptr())
-                tail = (rows, cols, step, 0.0)
-                first.append(head + (work[raw_row].data_ptr(),) + tail)
-                second.append(head + (work[new_row].data_ptr(),) + tail)
-                between.append((p, nxt, work[raw_row], work[new_row], trailing))
+                row_ptr = [work.data_ptr() + 4 * cols * r for r in range(3)]
+                if whole:
+                    head, tail = (dense.data_ptr(), grad.data_ptr(), mc, ms, vc), (rows, cols, step, 0.0)
+                else:
+                    head = (dense.data_ptr(), grad.data_ptr(), mc, self._next_codes(state, "exp_avg", batch), ms, ms_next, vc,
+                            self._next_codes(state, "exp_avg_sq", batch))
+                    tail = (0, rows, cols, step, 0.0)
+                head += (cur[0].data_ptr(), row_ptr[old_row], nxt[0].data_ptr())
+                first, second = passes[0 if whole else 1]
+                first.append(head + (row_ptr[raw_row],) + tail)
+                second.append(head + (row_ptr[new_row],) + tail)
+                between.append((p, nxt, cols, row_ptr[raw_row], row_ptr[new_row], trailing))
 
                 def remember(scratch=scratch, nxt=nxt, new_row=new_row):
                     scratch["scale_of"], scratch["row"] = nxt, new_row
 
                 batch.commits.append(remember)
-            for pass_no, records in ((1, first), (2, second)):
-                for i in range(0, len(records), _native.RANK1_MULTI_MAX):
-                    chunk = np.array(records[i:i + _native.RANK1_MULTI_MAX], dtype=_native.NONFUSED_RANK1_TENSOR)
-                    st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(chunk.ctypes.data, len(chunk), qm_ptr, qv_ptr, beta1,
-                                                                      beta2, lr, wd, eps, pass_no, stream)
-                    _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
+            for pass_no in (1, 2):
+                for kind, lists in enumerate(passes):
+                    records = lists[pass_no - 1]
+                    for i in range(0, len(records), _native.RANK1_MULTI_MAX):
+                        chunk = np.array(records[i:i + _native.RANK1_MULTI_MAX],
+                                         dtype=_native.NONFUSED_RANK1_TENSOR if kind == 0 else _native.RANK1_ANY_TENSOR)
+                        if kind == 0:
+                            st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(
+                                chunk.ctypes.data, len(chunk), qm_ptr, qv_ptr, beta1, beta2, lr, wd, eps, pass_no, stream)
+                        else:
+                            st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(
+                                chunk.ctypes.data, len(chunk), _native.RANK1_CODES4, 128, qm_ptr, 4, None, qv_ptr, 4, None,
+                                beta1, beta2, lr, wd, eps, pass_no, stream)
+                        _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
                 if pass_no == 1:
                     # the column maxima of the new second moment -> next statistics of the trailing dimensions
                     # -> their column scale: one launch for all tensors whose statistics fit a workgroup's LDS
                     # (every convolution weight), two calls per tensor otherwise
                     small = []
-                    for p, nxt, raw, scale, trailing in between:
+                    for p, nxt, cols, raw, scale, trailing in between:
                         dims = tuple(p.shape[1:])
                         # one workgroup per vector: for the few thousand values of a convolution weight's
                         # trailing dimensions, not for the millions of a stack of matrices
-                        if sum(dims) <= _native.RANK1_SMALL_SLOTS and raw.numel() <= _native.RANK1_SMALL_VALUES:
+                        if sum(dims) <= _native.RANK1_SMALL_SLOTS and cols <= _native.RANK1_SMALL_VALUES:
                             pad = 7 - len(dims)
-                            small.append((raw.data_ptr(), scale.data_ptr(), tuple(t.data_ptr() for t in nxt[1:]) + (0,) * pad,
+                            small.append((raw, scale, tuple(t.data_ptr() for t in nxt[1:]) + (0,) * pad,
                                           dims + (1,) * pad, len(dims), 0))
                             continue
-                        st = lib.lpmm_rank1_stats_nd(raw.data_ptr(), p.dim() - 1, _shape_array(dims),
+                        st = lib.lpmm_rank1_stats_nd(raw, p.dim() - 1, _shape_array(dims),
                                                      _ptr_array(nxt[1:]), None, stream)
                         _native.check(st, "rank1_stats_nd")
                         st = lib.lpmm_rank1_row_scale_nd(_ptr_array(nxt[1:] + [nxt[0]]), len(trailing),
-                                                         _shape_array(trailing), scale.data_ptr(), stream)
+                                                         _shape_array(trailing), scale, stream)
                         _native.check(st, "rank1_row_scale_nd")
                     if small:
                         vectors = np.array(small, dtype=_native.RANK1_SMALL_VECTOR)

@@ -1,0 +1,197 @@
+"""GPU parity of the two passes for any column count (lpmm_nonfused_adamw_rank1_any_step_multi) and of the float16
+step on states that are not quantised, through lpmm.optim.AdamW against the CPU oracle: codes with their padding,
+scales and statistics bit for bit, parameters bit for bit in float16 and within 1e-6 in float32."""
+import os
+
+import numpy as np
+import pytest
+import torch
+
+from util import assert_rel, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+H = dict(lr=1e-2, betas=(0.9, 0.999), eps=1e-3, weight_decay=0.01)
+# column counts around the 128-column blocks and 16-column strides, odd and even: rows that start inside a code byte;
+# fewer rows than a tile and more; one long row; one column; a row of several tiles; 34 tensors (two launches)
+SHAPES = [(70, 61), (61, 70), (33, 127), (33, 129), (20, 255), (300, 257), (9, 1003), (131, 130), (65, 322), (64, 66),
+          (1, 5001), (4099, 1), (130, 33), (40, 200), (25, 172)] + [(47, 90), (47, 91)] * 10
+KINDS = {
+    "codes4": ("default.yml", 4, np.float32),
+    "float_m": ("2nd_moment_only_default.yml", 4, np.float32),
+    "codes5": ("default_5b.yml", 5, np.float32),
+    "codes8": ("default_8b.yml", 8, np.float32),
+    "half": ("default.yml", 4, np.float16),
+}
+
+
+def _same(got, want, what):
+    got, want = np.ascontiguousarray(got).reshape(-1), np.ascontiguousarray(want).reshape(-1)
+    assert got.dtype == want.dtype, what
+    ok = (got == want) | (np.isnan(got) & np.isnan(want))
+    assert ok.all(), (what, int((~ok).sum()), np.flatnonzero(~ok)[:5], got[~ok][:5], want[~ok][:5])
+
+
+def _setup(kind, shapes, rng):
+    import lpmm
+
+    config, bits, dtype = KINDS[kind]
+    host = [(rng.standard_normal(s) * 0.5).astype(dtype) for s in shapes]
+    # every third parameter starts one value off the allocation
+    stores = [to_dev(np.concatenate([np.zeros(int(i % 3 == 2), dtype), h.reshape(-1)])) for i, h in enumerate(host)]
+    params = [torch.nn.Parameter(s[int(i % 3 == 2):].view(h.shape)) for i, (s, h) in enumerate(zip(stores, host))]
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    return host, params, lpmm.optim.AdamW(params, fused=False, qconfig=path, **H)
+
+
+def _oracle_step(oracle, kind, h, g, state, qm, qv):
+    if kind == "half":
+        oracle.nonfused_step_f16(h, g, state, qm, qv, H["lr"], 0.9, 0.999, H["eps"], H["weight_decay"])
+    elif kind == "float_m":
+        state.step += 1
+        r, c = h.shape
+        if state.m is None:
+            state.m = np.zeros(h.size, np.float32)
+        v = (np.zeros(h.size, np.float32) if state.v is None
+             else np.ascontiguousarray(oracle.dequant_rank1(*state.v, qv, r, c)).reshape(-1))
+        oracle.nonfused_update(h.reshape(-1), g.reshape(-1), state.m, v, 0.9, 0.999, H["lr"], H["weight_decay"], H["eps"],
+                               float(state.step))
+        rowmax, colmax = oracle.rank1_stats(v.reshape(r, c))
+        state.v = (oracle.quant_rank1(v.reshape(r, c), rowmax, colmax, qv), rowmax, colmax)
+    else:
+        oracle.nonfused_step(h, g, state, qm, qv, H["lr"], 0.9, 0.999, H["eps"], H["weight_decay"])
+
+
+def _check(kind, opt, p, h, before, state, what):
+    s = opt.state[p]
+    if kind == "float_m":
+        _same(to_np(s["exp_avg"]).reshape(-1), state.m, what + ": m")
+    else:
+        _same(to_np(s["exp_avg_qstate"]["overhead"]["max1"]), state.m[1], what + ": m scales")
+        _same(to_np(s["exp_avg"]).view(np.uint8), state.m[0], what + ": m codes")
+    oh = s["exp_avg_sq_qstate"]["overhead"]
+    _same(to_np(oh["max_dims"][0]), state.v[1], what + ": row statistics")
+    _same(to_np(oh["max_dims"][1]), state.v[2], what + ": column statistics")
+    _same(to_np(s["exp_avg_sq"]).view(np.uint8), state.v[0], what + ": v codes")
+    if kind == "half":
+        _same(to_np(p.detach()), h, what + ": p")
+    else:
+        assert_rel(to_np(p.detach()), h, what + ": p", scale=before)
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_every_column_count(oracle, kind):
+    bits = KINDS[kind][1]
+    from lpmm.functional import create_general_qmap
+
+    qm, qv = (create_general_qmap(*k).numpy() for k in (("nonlinear", bits, True), ("power-1", bits, False)))
+    rng = np.random.default_rng(90)
+    host, params, opt = _setup(kind, SHAPES, rng)
+    states = [oracle.NonFusedState(s, "rank1", bits=bits) for s in SHAPES]
+    for step in range(1, 4):
+        grads = [(rng.standard_normal(s) * 0.3 * 10.0 ** (1 - step) * np.exp(rng.standard_normal((s[0], 1)))).astype(h.dtype)
+                 for s, h in zip(SHAPES, host)]
+        grads[3][5:12] = 0     # rows, a column and whole groups that never see a gradient: zero scales, NaN codes
+        grads[3][:, 17] = 0
+        grads[4][10:] = 0
+        for p, g in zip(params, grads):
+            p.grad = to_dev(g)
+        opt.step()
+        torch.cuda.synchronize()
+        for i, (p, h, g, st) in enumerate(zip(params, host, grads, states)):
+            before = h.copy()
+            _oracle_step(oracle, kind, h, g, st, qm, qv)
+            _check(kind, opt, p, h, before, st, f"step {step} tensor {i} {SHAPES[i]}")
+
+
+def test_half_infinities_and_nans(oracle, qmaps):
+    """Gradients whose squares overflow a half, an infinite one and a NaN: statistics, scales and codes as the chain of
+    half ops leaves them (a NaN is the maximum of its row, its column and its group)."""
+    qm, qv = qmaps
+    rng = np.random.default_rng(91)
+    shapes = [(70, 61), (40, 200)]
+    host, params, opt = _setup("half", shapes, rng)
+    states = [oracle.NonFusedState(s, "rank1") for s in shapes]
+    for step in range(1, 4):
+        grads = [(rng.standard_normal(s) * 0.1).astype(np.float16) for s in shapes]
+        grads[0][3, 4] = 20000.0
+        grads[1][7, 150] = 20000.0
+        if step == 2:
+            grads[0][20, 60] = np.inf
+            grads[1][30, 5] = np.nan
+        for p, g in zip(params, grads):
+            p.grad = to_dev(g)
+        opt.step()
+        torch.cuda.synchronize()
+        for i, (p, h, g, st) in enumerate(zip(params, host, grads, states)):
+            with np.errstate(all="ignore"):
+                _oracle_step(oracle, "half", h, g, st, qm, qv)
+            _check("half", opt, p, h, None, st, f"step {step} tensor {i}")
+
+
+@pytest.mark.parametrize("eps", [1e-3, 1e-8])
+def test_half_states_that_are_not_quantised(oracle, eps):
+    """lpmm_nonfused_update_f16_multi: sizes around the 2048-value tiles, odd offsets, more tensors than one launch; a
+    gradient of zero under an eps that is zero as a half, one whose square overflows."""
+    import lpmm
+
+    rng = np.random.default_rng(92)
+    sizes = [1, 2, 3, 255, 257, 2047, 2048, 2049, 4095, 4096] + [int(n) for n in rng.integers(2, 4097, 60)]
+    host = [(rng.standard_normal(n) * 0.5).astype(np.float16) for n in sizes]
+    stores = [to_dev(np.concatenate([np.zeros(i % 2, np.float16), h])) for i, h in enumerate(host)]
+    params = [torch.nn.Parameter(s[i % 2:]) for i, s in enumerate(stores)]
+    hyper = dict(H, eps=eps)
+    opt = lpmm.optim.AdamW(params, fused=False, **hyper)
+    ms, vs = [np.zeros_like(h) for h in host], [np.zeros_like(h) for h in host]
+    for step in range(1, 4):
+        grads = [(rng.standard_normal(n) * 0.1).astype(np.float16) for n in sizes]
+        grads[4][7] = 0
+        grads[5][9] = 20000.0
+        for p, g in zip(params, grads):
+            p.grad = to_dev(g)
+        opt.step()
+        torch.cuda.synchronize()
+        for i, (p, h, g, m, v) in enumerate(zip(params, host, grads, ms, vs)):
+            if h.size == 1:  # a one-element state counts as not created yet, on every step
+                m[:], v[:] = 0, 0
+            with np.errstate(all="ignore"):
+                oracle.nonfused_update_f16(h, g, m, v, 0.9, 0.999, hyper["lr"], hyper["weight_decay"], eps, float(step))
+            _same(to_np(p.detach()), h, f"step {step} tensor {i}: p")
+            _same(to_np(opt.state[p]["exp_avg"]), m, f"step {step} tensor {i}: m")
+            _same(to_np(opt.state[p]["exp_avg_sq"]), v, f"step {step} tensor {i}: v")
+
+
+def test_tensors_of_more_dimensions(oracle, qmaps):
+    """The same passes on the shape[0] x rest view, one at a time: trailing products that are odd, a multiple of 8, and
+    neither."""
+    import lpmm
+
+    qm, qv = qmaps
+    rng = np.random.default_rng(93)
+    shapes = [(64, 3, 7, 7), (40, 40, 3, 3), (24, 10, 5, 5), (600, 1, 3, 3), (33, 5, 27)] + [(32, 24, 3, 3)] * 33
+    host = [(rng.standard_normal(s) * 0.5).astype(np.float32) for s in shapes]
+    params = [torch.nn.Parameter(to_dev(h.copy())) for h in host]
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    opt = lpmm.optim.AdamW(params, fused=False, qconfig=path, **H)
+    states = [oracle.NonFusedState(s, "rank1") for s in shapes]
+    for step in range(1, 4):
+        grads = []
+        for s in shapes:
+            g = rng.standard_normal(s) * 1e-1
+            for d in range(len(s)):
+                g = g * np.exp(0.7 * rng.standard_normal([n if i == d else 1 for i, n in enumerate(s)]))
+            grads.append(g.astype(np.float32))
+        for p, g in zip(params, grads):
+            p.grad = to_dev(g)
+        opt.step()
+        torch.cuda.synchronize()
+        for i, (p, h, g, st) in enumerate(zip(params, host, grads, states)):
+            before = h.copy()
+            oracle.nonfused_step(h, g, st, qm, qv, H["lr"], 0.9, 0.999, H["eps"], H["weight_decay"])
+            s, what, n = opt.state[p], f"step {step} tensor {i} {shapes[i]}", h.size
+            for got, want in zip(s["exp_avg_sq_qstate"]["overhead"]["max_dims"], st.v[1]):
+                _same(to_np(got), want, what + ": statistics")
+            _same(to_np(s["exp_avg_qstate"]["overhead"]["max1"]), st.m[1], what + ": m scales")
+            _same(to_np(s["exp_avg"]).view(np.uint8)[: (n + 1) // 2], st.m[0][: (n + 1) // 2], what + ": m codes")
+            _same(to_np(s["exp_avg_sq"]).view(np.uint8)[: (n + 1) // 2], st.v[0][: (n + 1) // 2], what + ": v codes")
+            assert_rel(to_np(p.detach()), h, what + ": p", scale=before)
