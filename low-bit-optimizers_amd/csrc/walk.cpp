@@ -1,0 +1,731 @@
+// The host side of a step on a model whose optimizer states exist: one walk over a parameter group's tensors
+// that writes the records of the multi-tensor launches.  In Python the same walk is dozens of attribute and
+// dictionary reads a tensor -- 3 to 15 us a tensor, against 0.4 here, while the kernels take 1 us for a tensor of a
+// million values -- and bound every model of small tensors: fifty tensors of a few thousand to a million values
+// 186 -> 43 us a step, the 254 of a wide ResNet-152 1634 -> 1054, GPT-2-XL's 580 1.8 -> 0.23 ms of host time.
+// lpmm/optim/adamw.py and sgd.py keep that walk for what is not served here: first steps, other data types,
+// strided operands, other routes; and for every error.
+//
+// collect() decides for each tensor, from the tensor and its state alone and anew on every step, whether it is
+// served, and reads its pointers; no state changes.  Plan.start() advances the step counts and completes the
+// records; after a launch is on the stream, Plan.commit() lets the states point to their new statistics (and, on
+// the kernels for any column count, codes).  A Plan lives for one step.
+#include <Python.h>
+
+#include <ATen/ops/empty.h>
+#include <ATen/ops/empty_like.h>
+#include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstring>
+#include <memory>
+#include <vector>
+
+#include "lpmm_hip.h"
+
+namespace {
+
+enum Kind : int { kFused4, kPlain, kFlat, kRank1, kNd, kFlatM32, kRank1M32, kRank1Bits, kRank1Wide, kSgd4, kSgdPlain,
+                  kAny, kNdAny, kHalfPlain, kHalfFlat, kHalfRank1, kKinds };
+
+constexpr size_t kRecordBytes[kKinds] = {
+    sizeof(lpmm_adamw4bit_tensor),     sizeof(lpmm_adamw_fp32_tensor),     sizeof(lpmm_adamw4bit_tensor),
+    sizeof(lpmm_nonfused_rank1_tensor), sizeof(lpmm_nonfused_rank1_tensor), sizeof(lpmm_adamw_v4bit_tensor),
+    sizeof(lpmm_rank1_v4bit_tensor),   sizeof(lpmm_nonfused_rank1_tensor), sizeof(lpmm_rank1_mgroup_tensor),
+    sizeof(lpmm_sgd4bit_tensor),       sizeof(lpmm_sgd_fp32_tensor),       sizeof(lpmm_rank1_any_tensor),
+    sizeof(lpmm_rank1_any_tensor),     sizeof(lpmm_adamw_fp32_tensor),     sizeof(lpmm_adamw4bit_f16_tensor),
+    sizeof(lpmm_nonfused_rank1_f16_tensor)};
+
+struct Names {
+    PyObject *step, *exp_avg, *exp_avg_sq, *exp_avg_qstate, *exp_avg_sq_qstate, *exp_avg_sq_row, *enable, *overhead, *qmap, *max1,
+        *max_dims, *work, *scale_of, *row, *momentum_buffer, *momentum_buffer_qstate, *dtype;
+} N;
+
+// dict[key] = value, once the launch is on the stream; strong references
+struct Swap {
+    PyObject *dict, *key, *value;
+};
+
+struct Item {
+    float *step = nullptr;
+    Swap swap[8];
+    int swaps = 0;
+};
+
+struct Batch {
+    Kind kind;
+    int device, flag;  // flag: kRank1Wide: ragged rows; kAny: the kind of its entry point
+    PyObject *qm, *qv;  // the maps' tensors (borrowed from held references)
+    std::vector<uint8_t> records, second;
+    std::vector<lpmm_rank1_small_vector> fold;
+    std::vector<Item> items;
+};
+
+struct Plan {
+    PyObject_HEAD
+    std::vector<Batch> *batches;
+    std::vector<at::Tensor> *scratch;
+    std::vector<PyObject *> *held;  // what the records point into: kept until the step is over
+    PyObject *rest;
+};
+
+const at::Tensor *tensor_of(PyObject *o)
+{
+    return o != nullptr && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+}
+
+PyObject *get(PyObject *dict, PyObject *key)  // borrowed; null where absent (a Python error stays set)
+{
+    return dict != nullptr && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, key) : nullptr;
+}
+
+bool on_gpu(const at::Tensor &t)
+{
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided &&
+           !t.unsafeGetTensorImpl()->key_set().has(c10::DispatchKey::Python) && t.is_contiguous();
+}
+
+bool floats(const at::Tensor &t) { return on_gpu(t) && t.scalar_type() == at::kFloat; }
+bool halfs(const at::Tensor &t) { return on_gpu(t) && t.scalar_type() == at::kHalf; }
+
+template <typename T = void>
+T *ptr(const at::Tensor &t)
+{
+    return static_cast<T *>(t.unsafeGetTensorImpl()->mutable_data());
+}
+
+bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+struct Settings {
+    int fused, m_group128, v_group128, v_rank1, m_wide, bits_rank1;
+    int64_t m_group;
+};
+
+struct Walk {
+    Plan *plan;
+    PyObject *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
+    Settings s;
+
+    // a dense tensor of n values beside p and of its type (parameters on the kernels are float or half)
+    static const at::Tensor *reals_of(PyObject *o, const at::Tensor &p, int64_t n)
+    {
+        const at::Tensor *t = tensor_of(o);
+        return t != nullptr && on_gpu(*t) && t->scalar_type() == p.scalar_type() && t->numel() == n && t->get_device() == p.get_device() ? t : nullptr;
+    }
+    // a state of p's values; a single value: not created yet
+    static const at::Tensor *reals_like(PyObject *o, const at::Tensor &p) { return p.numel() > 1 ? reals_of(o, p, p.numel()) : nullptr; }
+    // a state's codes, at least `bytes` of them
+    static const at::Tensor *codes(PyObject *o, const at::Tensor &p, int64_t bytes)
+    {
+        const at::Tensor *t = tensor_of(o);
+        return t != nullptr && t->numel() > 1 && t->numel() >= bytes && on_gpu(*t) && t->scalar_type() == at::kChar &&
+                       t->get_device() == p.get_device()
+                   ? t
+                   : nullptr;
+    }
+    // the scales of `groups` groups
+    static const at::Tensor *scales(PyObject *qstate, PyObject **overhead, const at::Tensor &p, int64_t groups)
+    {
+        *overhead = get(qstate, N.overhead);
+        return reals_of(get(*overhead, N.max1), p, groups);
+    }
+    // one tensor per dimension
+    template <typename T>
+    static bool statistics(PyObject *list, const at::Tensor &p, T **out)
+    {
+        if (list == nullptr || !PyList_Check(list) || PyList_GET_SIZE(list) != p.dim())
+            return false;
+        for (Py_ssize_t i = 0; i < p.dim(); ++i) {
+            const at::Tensor *t = reals_of(PyList_GET_ITEM(list, i), p, p.size(i));
+            if (t == nullptr)
+                return false;
+            out[i] = ptr<T>(*t);
+        }
+        return true;
+    }
+
+    Batch &batch(Kind kind, const at::Tensor &p, PyObject *qm, PyObject *qv, int flag = 0)
+    {
+        const int device = p.get_device();
+        for (Batch &b : *plan->batches)
+            if (b.kind == kind && b.device == device && b.qm == qm && b.qv == qv && b.flag == flag)
+                return b;
+        plan->batches->push_back(Batch{kind, device, flag, qm, qv, {}, {}, {}, {}});
+        keep(qm);
+        keep(qv);
+        return plan->batches->back();
+    }
+    void keep(PyObject *o)
+    {
+        if (o != nullptr) {
+            Py_INCREF(o);
+            plan->held->push_back(o);
+        }
+    }
+    template <typename R>
+    static void append(std::vector<uint8_t> &to, const R &record)
+    {
+        const uint8_t *r = reinterpret_cast<const uint8_t *>(&record);
+        to.insert(to.end(), r, r + sizeof(R));
+    }
+    template <typename R>
+    void add(Batch &b, const R &record, const Item &item)
+    {
+        append(b.records, record);
+        b.items.push_back(item);
+        for (int i = 0; i < item.swaps; ++i) {
+            Py_INCREF(item.swap[i].dict);
+            Py_INCREF(item.swap[i].key);
+            Py_INCREF(item.swap[i].value);
+        }
+    }
+
+    int enabled(PyObject *p, PyObject *qstate)  // -1: not decided here
+    {
+        if (override_ != nullptr && PyDict_GET_SIZE(override_) != 0) {
+            PyObject *id = PyLong_FromVoidPtr(p);
+            if (id == nullptr)
+                return -1;
+            PyObject *o = PyDict_GetItemWithError(override_, id);
+            Py_DECREF(id);
+            if (o != nullptr)
+                return PyObject_IsTrue(o);
+        }
+        PyObject *e = get(qstate, N.enable);
+        return e != nullptr ? PyObject_IsTrue(e) : -1;
+    }
+
+    // where a state's new codes go: a tensor that becomes the state (st[name])
+    uint8_t *next_codes(Item &item, PyObject *st, PyObject *name, const at::Tensor &codes)
+    {
+        const at::Tensor next = at::empty_like(codes);
+        PyObject *o = THPVariable_Wrap(next);
+        if (o == nullptr)
+            throw std::runtime_error("no tensor object");
+        plan->held->push_back(o);
+        item.swap[item.swaps++] = Swap{st, name, o};
+        return ptr<uint8_t>(next);
+    }
+    float *scratch(const at::Tensor &p, int64_t n)
+    {
+        plan->scratch->push_back(at::empty({n}, p.options().dtype(at::kFloat)));
+        return ptr<float>(plan->scratch->back());
+    }
+
+    bool adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+    bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
+    bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const at::Tensor *mc,
+             const at::Tensor *ms, const at::Tensor &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
+    bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const at::Tensor *any_mc,
+            PyObject *oh_m, const at::Tensor &vc, PyObject *oh_v, PyObject *qm, PyObject *qv);
+    bool sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+};
+
+void swap_later(Item &item, PyObject *dict, PyObject *key, PyObject *value) { item.swap[item.swaps++] = Swap{dict, key, value}; }
+
+// true: a record was added.  Every return before that leaves the plan as it was.
+bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
+{
+    if (!g.defined() || !on_gpu(p) || !on_gpu(g) || p.device() != g.device() || p.numel() != g.numel() ||
+        g.scalar_type() != p.scalar_type() || get(st, N.exp_avg_sq_row) != nullptr)
+        return false;
+    const at::Tensor *step = tensor_of(get(st, N.step));
+    if (step == nullptr || !step->is_cpu() || step->scalar_type() != at::kFloat || step->dim() != 0)
+        return false;
+    if (!floats(p))
+        return halfs(p) && !s.fused && half(po, p, g, st, *step);
+    PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
+    PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
+    const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
+    if (en_m < 0 || en_v < 0)
+        return false;
+    Item item;
+    item.step = ptr<float>(*step);
+    const int64_t n = p.numel();
+    if (!en_m && !en_v) {
+        const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
+        if (m == nullptr || v == nullptr)
+            return false;
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<float>(*v), n, 0.0f, 0.0f};
+        add(batch(kPlain, p, nullptr, nullptr), r, item);
+        return true;
+    }
+    PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap);
+    const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
+    const at::Tensor *vc = codes(vo, p, s.bits_rank1 ? n : (n + 1) / 2);
+    if (map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) || vc == nullptr || !en_v)
+        return false;
+    PyObject *oh_m = nullptr, *oh_v = nullptr;
+    if (s.fused || s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
+        const at::Tensor *vs = scales(qs_v, &oh_v, p, (n + 127) / 128);
+        if (vs == nullptr)
+            return false;
+        if (!en_m) {
+            const at::Tensor *m = reals_like(mo, p);
+            if (s.fused || m == nullptr)
+                return false;
+            lpmm_adamw_v4bit_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<uint8_t>(*vc), ptr<float>(*vs), n, 0.0f, 0.0f};
+            add(batch(kFlatM32, p, nullptr, qv), r, item);
+            return true;
+        }
+        const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
+        if (!(s.fused ? n % 2 == 0 : s.m_group128 != 0) || mc == nullptr || ms == nullptr)
+            return false;
+        lpmm_adamw4bit_tensor r;
+        memset(&r, 0, sizeof r);
+        r.p = ptr<float>(p);
+        r.g = ptr<float>(g);
+        r.m_codes = ptr<uint8_t>(*mc);
+        r.v_codes = ptr<uint8_t>(*vc);
+        r.m_scale = ptr<float>(*ms);
+        r.v_scale = ptr<float>(*vs);
+        r.n = n;
+        add(batch(s.fused ? kFused4 : kFlat, p, qm, qv), r, item);
+        return true;
+    }
+    oh_v = get(qs_v, N.overhead);
+    PyObject *cur = get(oh_v, N.max_dims);
+    if (!(s.v_rank1 || s.bits_rank1) || cur == nullptr || p.dim() < 2 || p.size(0) == 0)
+        return false;
+    lpmm_nonfused_rank1_tensor r;
+    memset(&r, 0, sizeof r);
+    r.p = ptr<float>(p);
+    r.g = ptr<float>(g);
+    r.v_codes = ptr<uint8_t>(*vc);
+    r.rows = p.size(0);
+    r.cols = n / r.rows;
+    const at::Tensor *mc = nullptr, *ms = nullptr;
+    if (en_m) {
+        mc = codes(mo, p, s.bits_rank1 ? n : (n + 1) / 2);
+        ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
+        if (mc == nullptr || ms == nullptr)
+            return false;
+        r.m_codes = ptr<uint8_t>(*mc);
+        r.m_max1 = ptr<float>(*ms);
+    }
+    const bool whole = r.cols % 128 == 0, folds = r.cols % 128 == 64 && r.rows % 2 == 0;
+    const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
+    if (p.dim() > 2)
+        return en_m && s.m_group128 && s.v_rank1 && served &&
+               nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, *vc, oh_v, qm, qv);
+    PyObject *nxt = get(spare_stats, po);
+    float *now[2], *next[2];
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
+        return false;
+    r.v_rowmax = now[0];
+    r.v_colmax = now[1];
+    r.v_rowmax_next = next[0];
+    r.v_colmax_next = next[1];
+    swap_later(item, spare_stats, po, cur);
+    swap_later(item, oh_v, N.max_dims, nxt);
+    if (!en_m) {
+        const at::Tensor *m = reals_like(mo, p);
+        if (!s.v_rank1 || m == nullptr)
+            return false;
+        if (!whole || !aligned16(r.p) || !aligned16(r.g)) {
+            item.swaps = 0;
+            return served && any(po, p, g, st, item, LPMM_RANK1_FLOAT_M, m, nullptr, *vc, nullptr, oh_v, qm, qv);
+        }
+        if (!aligned16(ptr(*m)))
+            return false;
+        lpmm_rank1_v4bit_tensor f = {r.p, r.g, ptr<float>(*m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
+                                     r.rows, r.cols, 0.0f, 0.0f};
+        add(batch(kRank1M32, p, nullptr, qv), f, item);
+        return true;
+    }
+    if (s.bits_rank1) {
+        if (!whole) {
+            item.swaps = 0;
+            return served && any(po, p, g, st, item, LPMM_RANK1_CODES8, mc, ms, *vc, oh_m, oh_v, qm, qv);
+        }
+        add(batch(kRank1Bits, p, qm, qv), r, item);
+        return true;
+    }
+    if (s.m_group128 && (whole || folds)) {
+        add(batch(kRank1, p, qm, qv), r, item);
+        return true;
+    }
+    const bool ragged = !whole && r.cols % 8 == 0;
+    if (!whole && !ragged) {
+        item.swaps = 0;
+        return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, *vc, oh_m, oh_v, qm, qv);
+    }
+    PyObject *spare = get(spare_scales, po);
+    const at::Tensor *ms_next = reals_of(spare, p, ms->numel());
+    if (!((s.m_wide && whole) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
+        return false;
+    lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        ptr<float>(*ms_next), r.v_codes, r.v_rowmax,
+                                  r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
+    swap_later(item, spare_scales, po, get(oh_m, N.max1));
+    swap_later(item, oh_m, N.max1, spare);
+    add(batch(kRank1Wide, p, qm, qv, ragged), w, item);
+    return true;
+}
+
+// a matrix of any column count (lpmm_nonfused_adamw_rank1_any_step_multi); mc: the first moment's codes or values
+bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const at::Tensor *mc,
+               const at::Tensor *ms, const at::Tensor &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv)
+{
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *spare = get(spare_scales, po);
+    void *now[2], *next[2];
+    const at::Tensor *ms_next = ms != nullptr ? reals_of(spare, p, ms->numel()) : nullptr;
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || (ms != nullptr && ms_next == nullptr))
+        return false;
+    lpmm_rank1_any_tensor r;
+    memset(&r, 0, sizeof r);
+    r.p = ptr(p);
+    r.g = ptr(g);
+    r.m = ptr(*mc);
+    r.v_codes = ptr<uint8_t>(vc);
+    r.v_rowmax = now[0];
+    r.v_colmax = now[1];
+    r.v_rowmax_next = next[0];
+    r.v_colmax_next = next[1];
+    r.rows = p.size(0);
+    r.cols = p.size(1);
+    if (kind == LPMM_RANK1_HALF)
+        r.work = scratch(p, r.rows + r.cols + (p.numel() + 127) / 128);
+    swap_later(item, spare_stats, po, cur);
+    swap_later(item, oh_v, N.max_dims, nxt);
+    r.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
+    if (ms != nullptr) {
+        r.m_max1 = ptr(*ms);
+        r.m_max1_next = ptr(*ms_next);
+        r.m_codes_next = next_codes(item, st, N.exp_avg, *mc);
+        swap_later(item, spare_scales, po, get(oh_m, N.max1));
+        swap_later(item, oh_m, N.max1, spare);
+    }
+    add(batch(kAny, p, qm, qv, kind), r, item);
+    return true;
+}
+
+// float16 parameters on the non-fused path (lpmm/optim/adamw.py: _half_kernel_kind)
+bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step)
+{
+    PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
+    PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
+    const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
+    const int64_t n = p.numel(), groups = (n + 127) / 128;
+    Item item;
+    item.step = ptr<float>(step);
+    if (en_m == 0 && en_v == 0) {
+        const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
+        if (m == nullptr || v == nullptr || m->sizes() != p.sizes() || v->sizes() != p.sizes())
+            return false;
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<float>(*v), n, 0.0f, 0.0f};
+        add(batch(kHalfPlain, p, nullptr, nullptr), r, item);
+        return true;
+    }
+    PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap), *oh_m = nullptr, *oh_v = get(qs_v, N.overhead);
+    const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
+    const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *vc = codes(vo, p, (n + 1) / 2), *ms = scales(qs_m, &oh_m, p, groups);
+    PyObject *const half_type = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
+    if (en_m != 1 || en_v != 1 || !s.m_group128 || map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) ||
+        mc == nullptr || vc == nullptr || ms == nullptr || get(oh_m, N.dtype) != half_type || get(oh_v, N.dtype) != half_type)
+        return false;
+    if (s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
+        const at::Tensor *vs = scales(qs_v, &oh_v, p, groups);
+        if (vs == nullptr)
+            return false;
+        lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), ptr<uint8_t>(*mc), ptr<uint8_t>(*vc), ptr(*ms), ptr(*vs), n, 0.0f, 0.0f};
+        add(batch(kHalfFlat, p, qm, qv), r, item);
+        return true;
+    }
+    if (!s.v_rank1 || p.dim() != 2 || p.size(0) == 0)
+        return false;
+    const int64_t rows = p.size(0), cols = p.size(1);
+    if (cols % 128 != 0 || !aligned16(ptr(p)) || !aligned16(ptr(g)))
+        return (cols >= 32 || rows <= 32768) && any(po, p, g, st, item, LPMM_RANK1_HALF, mc, ms, *vc, oh_m, oh_v, qm, qv);
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po);
+    void *now[2], *next[2];
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
+        return false;
+    swap_later(item, spare_stats, po, cur);
+    swap_later(item, oh_v, N.max_dims, nxt);
+    lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), ptr<uint8_t>(*mc), ptr(*ms), ptr<uint8_t>(*vc), now[0], now[1], next[0], next[1],
+                                        scratch(p, (rows + 3) / 4 * 4 + cols), rows, cols, 0.0f, 0.0f};
+    add(batch(kHalfRank1, p, qm, qv), r, item);
+    return true;
+}
+
+// a tensor of 3 to 8 dimensions on its shape[0] x rest view, where the fold between the passes takes one workgroup
+// and the column scale the last step left still holds (lpmm/optim/adamw.py: _rank1_nd_steps)
+bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const at::Tensor *any_mc,
+              PyObject *oh_m, const at::Tensor &vc, PyObject *oh_v, PyObject *qm, PyObject *qv)
+{
+    const int dims = (int)p.dim();
+    if (dims > LPMM_RANK1_ND_MAX || (r.rows < 16 && p.numel() > (1 << 20)) || r.cols > (1 << 16))
+        return false;
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *scratch = get(nd_scratch, po);
+    PyObject *row = get(scratch, N.row);
+    const at::Tensor *work = reals_of(get(scratch, N.work), p, 3 * r.cols);
+    float *now[LPMM_RANK1_ND_MAX], *next[LPMM_RANK1_ND_MAX];
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
+        return false;
+    const long old_row = PyLong_AsLong(row);
+    if (old_row < 0 || old_row > 2)
+        return false;
+    const int raw_row = old_row == 0 ? 1 : 0, new_row = old_row == 2 ? 1 : 2;
+    lpmm_rank1_small_vector fold;
+    memset(&fold, 0, sizeof fold);
+    int64_t slots = 0;
+    for (int i = 0; i < LPMM_RANK1_ND_MAX - 1; ++i) {
+        fold.shape[i] = i + 1 < dims ? p.size(i + 1) : 1;
+        fold.stats[i] = i + 1 < dims ? next[i + 1] : nullptr;
+        slots += i + 1 < dims ? fold.shape[i] : 0;
+    }
+    if (slots > 8192)
+        return false;
+    float *const rows = ptr<float>(*work);
+    fold.ndim = dims - 1;
+    fold.x = rows + raw_row * r.cols;
+    fold.scale = rows + new_row * r.cols;
+    r.v_rowmax = now[0];
+    r.v_rowmax_next = next[0];
+    r.v_colmax = rows + old_row * r.cols;
+    r.v_colmax_next = rows + raw_row * r.cols;
+    // any_mc: a column count for the general kernels, which also need the next scales
+    PyObject *spare = get(spare_scales, po);
+    const at::Tensor *ms_next = any_mc != nullptr ? reals_of(spare, p, (p.numel() + 127) / 128) : nullptr;
+    if (any_mc != nullptr && ms_next == nullptr)
+        return false;
+    PyObject *row_obj = PyLong_FromLong(new_row);
+    if (row_obj == nullptr)
+        return false;
+    plan->held->push_back(row_obj);
+    swap_later(item, spare_stats, po, cur);
+    swap_later(item, oh_v, N.max_dims, nxt);
+    swap_later(item, scratch, N.scale_of, nxt);
+    swap_later(item, scratch, N.row, row_obj);
+    if (any_mc == nullptr) {
+        Batch &b = batch(kNd, p, qm, qv);
+        add(b, r, item);
+        r.v_colmax_next = rows + new_row * r.cols;
+        append(b.second, r);
+        b.fold.push_back(fold);
+        return true;
+    }
+    lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, ptr(*ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
+                               r.v_rowmax_next, r.v_colmax_next, nullptr, r.rows, r.cols, 0.0f, 0.0f};
+    w.m_codes_next = next_codes(item, st, N.exp_avg, *any_mc);
+    w.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
+    swap_later(item, spare_scales, po, get(oh_m, N.max1));
+    swap_later(item, oh_m, N.max1, spare);
+    Batch &b = batch(kNdAny, p, qm, qv);
+    add(b, w, item);
+    w.v_colmax_next = rows + new_row * r.cols;
+    append(b.second, w);
+    b.fold.push_back(fold);
+    return true;
+}
+
+bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
+{
+    if (!g.defined() || !floats(p) || !floats(g) || p.device() != g.device() || p.numel() != g.numel())
+        return false;
+    PyObject *qs = get(st, N.momentum_buffer_qstate), *bo = get(st, N.momentum_buffer);
+    const int en = enabled(po, qs);
+    if (en < 0)
+        return false;
+    if (!en) {
+        const at::Tensor *buf = reals_like(bo, p);
+        if (buf == nullptr || buf->sizes() != p.sizes())
+            return false;
+        lpmm_sgd_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*buf), p.numel(), 0, 0};
+        add(batch(kSgdPlain, p, nullptr, nullptr), r, Item());
+        return true;
+    }
+    PyObject *oh = nullptr, *qm = get(qs, N.qmap);
+    const at::Tensor *map = tensor_of(qm), *mc = codes(bo, p, (p.numel() + 1) / 2), *ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
+    if (!s.m_group128 || map == nullptr || !floats(*map) || mc == nullptr || ms == nullptr)
+        return false;
+    lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), ptr<uint8_t>(*mc), ptr<float>(*ms), p.numel(), 0, 0};
+    add(batch(kSgd4, p, qm, nullptr), r, Item());
+    return true;
+}
+
+// ---- the Plan object ---------------------------------------------------------------------------
+void plan_dealloc(PyObject *self)
+{
+    Plan *plan = reinterpret_cast<Plan *>(self);
+    if (plan->batches != nullptr)
+        for (Batch &b : *plan->batches)
+            for (Item &item : b.items)
+                for (int i = 0; i < item.swaps; ++i) {
+                    Py_DECREF(item.swap[i].dict);
+                    Py_DECREF(item.swap[i].key);
+                    Py_DECREF(item.swap[i].value);
+                }
+    if (plan->held != nullptr)
+        for (PyObject *o : *plan->held)
+            Py_DECREF(o);
+    delete plan->batches;
+    delete plan->held;
+    delete plan->scratch;
+    Py_XDECREF(plan->rest);
+    Py_TYPE(self)->tp_free(self);
+}
+
+PyObject *plan_rest(PyObject *self, void *)
+{
+    PyObject *rest = reinterpret_cast<Plan *>(self)->rest;
+    Py_INCREF(rest);
+    return rest;
+}
+
+// advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
+// address of the records, address of the second pass's records or 0, address of the fold records or 0)
+PyObject *plan_start(PyObject *self, PyObject *)
+{
+    Plan *plan = reinterpret_cast<Plan *>(self);
+    PyObject *out = PyList_New(0);
+    if (out == nullptr)
+        return nullptr;
+    for (Batch &b : *plan->batches) {
+        const size_t bytes = kRecordBytes[b.kind];
+        const bool has_step = b.kind != kSgd4 && b.kind != kSgdPlain;
+        for (size_t i = 0; i < b.items.size() && has_step; ++i) {
+            const float step = *b.items[i].step += 1.0f;
+            // every record ends in  float step, reserved
+            memcpy(&b.records[(i + 1) * bytes - 8], &step, 4);
+            if (!b.second.empty())
+                memcpy(&b.second[(i + 1) * bytes - 8], &step, 4);
+        }
+        PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,
+                                    b.qv != nullptr ? b.qv : Py_None, b.flag, (Py_ssize_t)b.items.size(),
+                                    (unsigned long long)(uintptr_t)b.records.data(), (unsigned long long)(uintptr_t)b.second.data(),
+                                    (unsigned long long)(uintptr_t)b.fold.data());
+        if (t == nullptr || PyList_Append(out, t) != 0) {
+            Py_XDECREF(t);
+            Py_DECREF(out);
+            return nullptr;
+        }
+        Py_DECREF(t);
+    }
+    return out;
+}
+
+// commit(batch, first, count): the launch of these records is on the stream
+PyObject *plan_commit(PyObject *self, PyObject *args)
+{
+    Plan *plan = reinterpret_cast<Plan *>(self);
+    Py_ssize_t k, first, count;
+    if (!PyArg_ParseTuple(args, "nnn", &k, &first, &count))
+        return nullptr;
+    if (k < 0 || (size_t)k >= plan->batches->size() || first < 0 || count < 0 ||
+        (size_t)(first + count) > (*plan->batches)[k].items.size()) {
+        PyErr_SetString(PyExc_IndexError, "no such records");
+        return nullptr;
+    }
+    for (Py_ssize_t i = first; i < first + count; ++i) {
+        const Item &item = (*plan->batches)[k].items[i];
+        for (int j = 0; j < item.swaps; ++j)
+            if (PyDict_SetItem(item.swap[j].dict, item.swap[j].key, item.swap[j].value) != 0)
+                return nullptr;
+    }
+    Py_RETURN_NONE;
+}
+
+PyMethodDef plan_methods[] = {{"start", plan_start, METH_NOARGS, "advance the step counts and return the batches"},
+                              {"commit", plan_commit, METH_VARARGS, "records [first, first + count) of a batch are on the stream"},
+                              {nullptr, nullptr, 0, nullptr}};
+PyObject *plan_served(PyObject *self, void *) { return PyBool_FromLong(!reinterpret_cast<Plan *>(self)->batches->empty()); }
+
+PyGetSetDef plan_getset[] = {{"served", plan_served, nullptr, "are there records", nullptr},
+                             {"rest", plan_rest, nullptr, "parameters with a gradient that are not served here", nullptr},
+                             {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+// collect(sgd, params, state, override, spare_stats, spare_scales, nd_scratch, serve, settings)
+PyObject *collect(PyObject *, PyObject *args)
+{
+    int is_sgd, serve;
+    PyObject *params, *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
+    Walk w;
+    int m_group;
+    if (!PyArg_ParseTuple(args, "iO!O!O!O!O!O!p(iiiiiii)", &is_sgd, &PyList_Type, &params, &PyDict_Type, &state, &PyDict_Type,
+                          &override_, &PyDict_Type, &spare_stats, &PyDict_Type, &spare_scales, &PyDict_Type, &nd_scratch, &serve,
+                          &w.s.fused, &w.s.m_group128, &w.s.v_group128, &w.s.v_rank1, &w.s.m_wide, &w.s.bits_rank1, &m_group))
+        return nullptr;
+    w.s.m_group = m_group;
+    Plan *plan = reinterpret_cast<Plan *>(PlanType.tp_alloc(&PlanType, 0));
+    if (plan == nullptr)
+        return nullptr;
+    std::unique_ptr<PyObject, void (*)(PyObject *)> owner(reinterpret_cast<PyObject *>(plan), [](PyObject *o) { Py_DECREF(o); });
+    try {
+        plan->batches = new std::vector<Batch>();
+        plan->held = new std::vector<PyObject *>();
+        plan->scratch = new std::vector<at::Tensor>();
+        plan->rest = PyList_New(0);
+        if (plan->rest == nullptr)
+            return nullptr;
+        plan->batches->reserve(16);
+        w.plan = plan;
+        w.state = state;
+        w.override_ = override_;
+        w.spare_stats = spare_stats;
+        w.spare_scales = spare_scales;
+        w.nd_scratch = nd_scratch;
+        for (Py_ssize_t i = 0; i < PyList_GET_SIZE(params); ++i) {
+            PyObject *po = PyList_GET_ITEM(params, i);
+            bool served = false;
+            if (THPVariable_Check(po)) {
+                const at::Tensor &p = THPVariable_Unpack(po);
+                const at::Tensor &g = p.grad();
+                const bool own = THPVariable_CheckExact(po);  // a Tensor or a Parameter, no subclass of either
+                if (!g.defined() && own)
+                    continue;
+                if (serve && own) {
+                    PyObject *st = PyDict_GetItemWithError(state, po);
+                    if (st != nullptr && PyDict_Check(st) && PyDict_GET_SIZE(st) != 0)
+                        served = is_sgd ? w.sgd(po, p, g, st) : w.adamw(po, p, g, st);
+                }
+            }
+            if (PyErr_Occurred())
+                return nullptr;
+            if (!served && PyList_Append(plan->rest, po) != 0)
+                return nullptr;
+        }
+    } catch (const std::exception &e) {
+        PyErr_SetString(PyExc_RuntimeError, e.what());
+        return nullptr;
+    }
+    return owner.release();
+}
+
+PyMethodDef methods[] = {{"collect", collect, METH_VARARGS, "walk a parameter group"}, {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_walk", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__walk()
+{
+    PlanType.tp_name = "lpmm._walk.Plan";
+    PlanType.tp_basicsize = sizeof(Plan);
+    PlanType.tp_dealloc = plan_dealloc;
+    PlanType.tp_flags = Py_TPFLAGS_DEFAULT;
+    PlanType.tp_methods = plan_methods;
+    PlanType.tp_getset = plan_getset;
+    if (PyType_Ready(&PlanType) < 0)
+        return nullptr;
+#define LPMM_NAME(n) N.n = PyUnicode_InternFromString(#n)
+    LPMM_NAME(step);
+    LPMM_NAME(exp_avg);
+    LPMM_NAME(exp_avg_sq);
+    LPMM_NAME(exp_avg_qstate);
+    LPMM_NAME(exp_avg_sq_qstate);
+    LPMM_NAME(exp_avg_sq_row);
+    LPMM_NAME(enable);
+    LPMM_NAME(overhead);
+    LPMM_NAME(qmap);
+    LPMM_NAME(max1);
+    LPMM_NAME(max_dims);
+    LPMM_NAME(work);
+    LPMM_NAME(scale_of);
+    LPMM_NAME(row);
+    LPMM_NAME(dtype);
+    LPMM_NAME(momentum_buffer);
+    LPMM_NAME(momentum_buffer_qstate);
+#undef LPMM_NAME
+    return PyModule_Create(&module);
+}

@@ -146,6 +146,27 @@ def lib():
     return _lib
 
 
+_walk = None
+
+
+def walk():
+    """The host walk (csrc/walk.cpp, an extension module); raises RuntimeError when it has not been built."""
+    global _walk
+    if _walk is None:
+        try:
+            from . import _walk as module
+        except ImportError as e:
+            raise RuntimeError("lpmm: the extension module lpmm/_walk.so is missing or does not load. Build it with "
+                               "`make -C low-bit-optimizers_amd/csrc`.") from e
+        _walk = module
+    return _walk
+
+
+# kinds of records a walk makes (enum Kind of csrc/walk.cpp)
+(WALK_FUSED4, WALK_PLAIN, WALK_FLAT, WALK_RANK1, WALK_ND, WALK_FLAT_M32, WALK_RANK1_M32, WALK_RANK1_BITS, WALK_RANK1_WIDE, WALK_SGD4,
+ WALK_SGD_PLAIN, WALK_ANY, WALK_ND_ANY, WALK_HALF_PLAIN, WALK_HALF_FLAT, WALK_HALF_RANK1) = range(16)
+
+
 def check(status, what):
     if status != 0:
         msg = lib().lpmm_status_string(status).decode()

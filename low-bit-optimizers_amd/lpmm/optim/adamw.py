@@ -79,6 +79,30 @@ def _zero_byte(qmap):
     return hit[1]
 
 
+class _Routes:
+    """What the quantisation settings of the two moments allow."""
+
+    def __init__(self, md_m, md_v):
+        def fits(md):
+            return md["b"] == 4 and md["round_type"] == "real-nearest"
+
+        # 5 to 8 bits (configs/default_{5,6,7,8}b.yml): one code per byte, the same two passes
+        def wide_codes(md):
+            return md["b"] in (5, 6, 7, 8) and md["round_type"] == "real-nearest"
+
+        m_group, v_group = md_m["scale_type"] == "group", md_v["scale_type"] == "group"
+        self.m, self.v = md_m, md_v
+        self.m_group128 = fits(md_m) and m_group and md_m["gp_sz"] == 128
+        self.v_group128 = fits(md_v) and v_group and md_v["gp_sz"] == 128
+        self.v_rank1 = fits(md_v) and md_v["scale_type"] == "rank1"
+        # first-moment groups of 256 .. 4096 values (configs/1st_moment_group_*.yml)
+        self.m_group_wide = fits(md_m) and m_group and md_m["gp_sz"] in (256, 512, 1024, 2048, 4096)
+        self.bits_rank1 = (wide_codes(md_m) and m_group and md_m["gp_sz"] == 128
+                           and wide_codes(md_v) and md_v["scale_type"] == "rank1")
+        # the fused operator: 4-bit states; other settings go on with a warning or an error
+        self.fused4 = md_m["b"] == 4 and md_v["b"] == 4 and m_group and v_group
+
+
 class _Batch(list):
     """Records of one pending launch, plus what becomes true once that launch has been enqueued: states
     whose statistics trade places with a second buffer point to the new buffer only after the kernels
@@ -193,29 +217,128 @@ class AdamW(LowBitOptimizer):
             with torch.enable_grad():
                 loss = closure()
 
+        routes = _Routes(self.get_qmetadata_by_state_name("exp_avg"), self.get_qmetadata_by_state_name("exp_avg_sq"))
         for group in self.param_groups:
+            # tensors in their steady state; the loop below has the others, and every error
+            plan = self._walk(group, routes)
             work = []
-            for p in group["params"]:
+            for p in plan.rest:
                 if p.grad is None:
                     continue
                 if p.grad.is_sparse:
                     raise RuntimeError("AdamW does not support sparse gradients")
                 state, factored = self._state_of(group, p)
                 work.append((p, p.grad, state, factored))
-            if not work:
-                continue
-            if group["fused"]:
-                self._step_fused(group, work)
-            else:
-                self._step_single(group, work)
+            if work:
+                if group["fused"]:
+                    self._step_fused(group, work, routes)
+                else:
+                    self._step_single(group, work, routes)
+            if plan.served:
+                self._launch_walk(group, plan, routes)
         return loss
 
+    def _walk(self, group, routes):
+        fused = bool(group["fused"])
+        return _native.walk().collect(
+            0, group["params"], self.state, self.override_q_enable, self._spare_stats, self._spare_scales, self._nd_scratch,
+            routes.fused4 if fused else True,
+            (fused, routes.m_group128, routes.v_group128, routes.v_rank1, routes.m_group_wide, routes.bits_rank1, routes.m["gp_sz"]))
+
+    def _launch_walk(self, group, plan, routes):
+        """The launches of the walk's records: those that _step_fused and _step_single make."""
+        beta1, beta2 = group["betas"]
+        hyper = (beta1, beta2, group["lr"], group["weight_decay"], group["eps"])
+        lib = _native.lib()
+        for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(plan.start()):
+            with torch.cuda.device(index):
+                stream = _native.current_stream(index)
+                qm_ptr, qv_ptr = (None if q is None else q.data_ptr() for q in (qm, qv))
+                if kind == _native.WALK_FUSED4:
+                    st = lib.lpmm_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
+                elif kind == _native.WALK_PLAIN:
+                    run = lib.lpmm_adamw_fp32_step_multi if group["fused"] else lib.lpmm_nonfused_update_multi
+                    st = run(records, count, *hyper, stream)
+                elif kind == _native.WALK_FLAT:
+                    st = lib.lpmm_nonfused_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
+                elif kind == _native.WALK_FLAT_M32:
+                    st = lib.lpmm_nonfused_adamw_v4bit_step_multi(records, count, qv_ptr, *hyper, stream)
+                elif kind == _native.WALK_HALF_PLAIN:
+                    st = lib.lpmm_nonfused_update_f16_multi(records, count, *hyper, stream)
+                elif kind == _native.WALK_HALF_FLAT:
+                    st = lib.lpmm_nonfused_adamw4bit_f16_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
+                else:
+                    self._launch_walk_rank1(plan, k, kind, qm, qv, flag, count, records, second, fold, hyper, routes, stream)
+                    continue
+            _native.check(st, "AdamW step")
+
+    @staticmethod
+    def _launch_walk_rank1(plan, k, kind, qm, qv, flag, count, records, second, fold, hyper, routes, stream):
+        """Two passes: a state's statistics (and wide scales) are the new ones once its launch is on the stream."""
+        lib, most = _native.lib(), _native.RANK1_MULTI_MAX
+        qv_ptr = qv.data_ptr()
+
+        def code_tables():
+            return [code_table(q, md["b"]).data_ptr() for q, md in ((qm, routes.m), (qv, routes.v))]
+
+        if kind in (_native.WALK_ND, _native.WALK_ND_ANY):
+            for pass_no, table in ((1, records), (2, second)):
+                if kind == _native.WALK_ND:
+                    st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(table, count, qm.data_ptr(), qv_ptr, *hyper, pass_no, stream)
+                else:
+                    st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, count, _native.RANK1_CODES4, 128, qm.data_ptr(), 4, None,
+                                                                      qv_ptr, 4, None, *hyper, pass_no, stream)
+                _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
+                if pass_no == 1:
+                    st = lib.lpmm_rank1_small_fold_scale_multi(fold, count, stream)
+                    _native.check(st, "rank1_small_fold_scale_multi")
+            plan.commit(k, 0, count)
+            return
+        if kind == _native.WALK_RANK1:
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw4bit_rank1_step_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, stream)
+            size = _native.NONFUSED_RANK1_TENSOR.itemsize
+        elif kind == _native.WALK_RANK1_M32:
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw_v4bit_rank1_step_multi(table, n, qv_ptr, *hyper, stream)
+            size = _native.RANK1_V4BIT_TENSOR.itemsize
+        elif kind == _native.WALK_ANY:
+            bits, tables, group = (4, 4), (None, None), 128
+            if flag == _native.RANK1_CODES8:
+                bits, tables = (routes.m["b"], routes.v["b"]), code_tables()
+            elif flag == _native.RANK1_CODES4:
+                group = routes.m["gp_sz"]
+
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, flag, group, qm.data_ptr(), bits[0], tables[0], qv_ptr,
+                                                                    bits[1], tables[1], *hyper, 3, stream)
+            size = _native.RANK1_ANY_TENSOR.itemsize
+        elif kind == _native.WALK_HALF_RANK1:
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw4bit_rank1_f16_step_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, stream)
+            size = _native.NONFUSED_RANK1_F16_TENSOR.itemsize
+        elif kind == _native.WALK_RANK1_BITS:
+            tables = code_tables()
+
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw_bits_rank1_step_multi_table(
+                    table, n, qm.data_ptr(), routes.m["b"], tables[0], qv_ptr, routes.v["b"], tables[1], *hyper, stream)
+            size = _native.NONFUSED_RANK1_TENSOR.itemsize
+        else:
+            def run(table, n):
+                return lib.lpmm_nonfused_adamw4bit_rank1_mgroup_step_multi(table, n, qm.data_ptr(), qv_ptr, routes.m["gp_sz"],
+                                                                           *hyper, stream)
+            size = _native.RANK1_MGROUP_TENSOR.itemsize
+        for i in range(0, count, most):
+            n = min(most, count - i)
+            _native.check(run(records + i * size, n), "non-fused AdamW step (rank-1 second moment)")
+            plan.commit(k, i, n)
+
     # ---- fused path (lpmm/optim/adamw.py:439-561) ---------------------------------------
-    def _step_fused(self, group, work):
+    def _step_fused(self, group, work, routes):
         beta1, beta2 = group["betas"]
         lr, wd, eps = group["lr"], group["weight_decay"], group["eps"]
-        md_m = self.get_qmetadata_by_state_name("exp_avg")
-        md_v = self.get_qmetadata_by_state_name("exp_avg_sq")
+        md_m, md_v = routes.m, routes.v
         quant, plain, plain16 = {}, {}, {}  # device -> list of records
         factored_work = []
         lib = _native.lib()
@@ -365,32 +488,19 @@ class AdamW(LowBitOptimizer):
         return torch.empty_like(p, device="meta", memory_format=torch.preserve_format).stride()
 
     # ---- non-fused path (lpmm/optim/adamw.py:332-436) -----------------------------------
-    def _step_single(self, group, work):
+    def _step_single(self, group, work, routes):
         beta1, beta2 = group["betas"]
         lr, wd, eps = group["lr"], group["weight_decay"], group["eps"]
-        md_m = self.get_qmetadata_by_state_name("exp_avg")
-        md_v = self.get_qmetadata_by_state_name("exp_avg_sq")
+        md_m, md_v = routes.m, routes.v
         lib = _native.lib()
         # both moments 4-bit, first moment block-wise over 128 values, second moment either the
         # same or rank-1 on a 2-D tensor with a multiple of 128 columns: dequantise, update and
         # re-quantise in one kernel (two for rank-1), all such tensors of the group per launch
-        def fits(md):
-            return md["b"] == 4 and md["round_type"] == "real-nearest"
-
-        m_group128 = fits(md_m) and md_m["scale_type"] == "group" and md_m["gp_sz"] == 128
-        v_group128 = fits(md_v) and md_v["scale_type"] == "group" and md_v["gp_sz"] == 128
-        v_rank1 = fits(md_v) and md_v["scale_type"] == "rank1"
-        # first-moment groups of 256 .. 4096 values (configs/1st_moment_group_*.yml)
-        m_group_wide = fits(md_m) and md_m["scale_type"] == "group" and md_m["gp_sz"] in (256, 512, 1024, 2048, 4096)
+        m_group128, v_group128, v_rank1 = routes.m_group128, routes.v_group128, routes.v_rank1
+        m_group_wide, bits_rank1 = routes.m_group_wide, routes.bits_rank1
         batched, batched_rank1, plain = {}, {}, {}
         batched_m32, batched_rank1_m32 = {}, {}  # fp32 first moment, quantised second moment
         batched_rank1_mgroup = {}
-        # 5 to 8 bits (configs/default_{5,6,7,8}b.yml): one code per byte, the same two passes
-        def wide_codes(md):
-            return md["b"] in (5, 6, 7, 8) and md["round_type"] == "real-nearest"
-
-        bits_rank1 = (wide_codes(md_m) and md_m["scale_type"] == "group" and md_m["gp_sz"] == 128
-                      and wide_codes(md_v) and md_v["scale_type"] == "rank1")
         batched_rank1_bits = {}
         factored_work = []
         nd_work = {}  # tensors of more than two dimensions that take the two passes (per device and maps)

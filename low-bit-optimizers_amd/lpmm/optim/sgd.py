@@ -69,7 +69,10 @@ class SGD(LowBitOptimizer):
             momentum, dampening = group["momentum"], group["dampening"]
             batched = {}  # (device, map address) -> records of the one-pass kernel
             plain = {}  # device -> records of the kernel on float buffers
-            for p in group["params"]:
+            # tensors whose buffers exist; the loop below has the others, and every error
+            plan = _native.walk().collect(1, group["params"], self.state, self.override_q_enable, {}, {}, {}, momentum != 0,
+                                          (False, one_pass_config, False, False, False, False, 128))
+            for p in plan.rest:
                 if p.grad is None:
                     continue
                 if p.grad.is_sparse:
@@ -150,4 +153,15 @@ class SGD(LowBitOptimizer):
                         table.ctypes.data, len(records), momentum, dampening, group["lr"], group["weight_decay"],
                         int(bool(group["nesterov"])), int(bool(group["maximize"])), _native.current_stream(dev))
                 _native.check(st, "SGD step on float buffers")
+            if plan.served:
+                hyper = (momentum, dampening, group["lr"], group["weight_decay"], int(bool(group["nesterov"])),
+                         int(bool(group["maximize"])))
+                for kind, index, qmap, _, _, count, records, _, _ in plan.start():
+                    with torch.cuda.device(index):
+                        stream = _native.current_stream(index)
+                        if kind == _native.WALK_SGD4:
+                            st = _native.lib().lpmm_sgd4bit_step_multi(records, count, qmap.data_ptr(), *hyper, stream)
+                        else:
+                            st = _native.lib().lpmm_sgd_fp32_step_multi(records, count, *hyper, stream)
+                    _native.check(st, "SGD step")
         return loss

@@ -1,0 +1,157 @@
+"""The host walk (csrc/walk.cpp) against the Python loops it stands in for: the same steps with and without it leave
+the same bits everywhere, whatever the route, across missing gradients, strided tensors, a checkpoint load, an
+overridden state and states the caller has moved."""
+import copy
+import os
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+MATRICES = [(64, 256), (48, 192), (33, 200), (33, 130), (5000,), (70,), (17, 16, 8), (32, 24, 3, 3), (40, 5, 7, 5), (90, 128)]
+CASES = {
+    "fused": dict(fused=True),
+    "fused_factored": dict(fused=True, factor_second_moment=True),
+    "default": dict(qconfig="default.yml"),
+    "group": dict(qconfig="2nd_moment_group_128.yml"),
+    "float_m": dict(qconfig="2nd_moment_only_default.yml"),
+    "float_m_group": dict(qconfig="2nd_moment_only_group_128.yml"),
+    "wide": dict(qconfig="1st_moment_group_512.yml"),
+    "bits": dict(qconfig="default_6b.yml"),
+    "half": dict(qconfig="default.yml", dtype=torch.float16),
+    "half_group": dict(qconfig="2nd_moment_group_128.yml", dtype=torch.float16),
+    "sgd": dict(sgd=True),
+}
+
+
+class _Native:
+    """lpmm._native with a walk that serves nothing, or counts what it serves."""
+
+    def __init__(self, native, serve):
+        self._native, self._serve, self.served, self.rest = native, serve, 0, 0
+
+    def __getattr__(self, name):
+        return getattr(self._native, name)
+
+    def walk(self):
+        return self
+
+    def collect(self, *args):
+        args = list(args)
+        args[7] = args[7] and self._serve
+        plan = self._native.walk().collect(*args)
+        self.served += plan.served
+        self.rest += len(plan.rest)
+        return plan
+
+
+def _build(case, rng):
+    import lpmm
+
+    kw = dict(CASES[case])
+    dtype, sgd = kw.pop("dtype", torch.float32), kw.pop("sgd", False)
+    if "qconfig" in kw:
+        kw["qconfig"] = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", kw["qconfig"])
+    shapes = [s for s in MATRICES if dtype is torch.float32 or len(s) < 3]
+    params = [torch.nn.Parameter(torch.from_numpy(rng.standard_normal(s) * 0.1).to(dtype).cuda()) for s in shapes]
+    if not kw.get("fused"):  # the fused operators refuse strided parameters
+        params.append(torch.nn.Parameter(torch.from_numpy(rng.standard_normal((96, 80))).float().cuda().t().to(dtype)))
+    if sgd:
+        return params, lpmm.optim.SGD(params, lr=1e-2, momentum=0.9, weight_decay=1e-3, nesterov=True)
+    return params, lpmm.optim.AdamW(params, lr=1e-2, eps=1e-3, **kw)
+
+
+def _state(opt, p):
+    out = {}
+    for k, v in opt.state[p].items():
+        if torch.is_tensor(v):
+            out[k] = v
+        else:
+            for name, o in v["overhead"].items():
+                for i, t in enumerate(o if isinstance(o, list) else [o]):
+                    if torch.is_tensor(t):
+                        out[k, name, i] = t
+    return out
+
+
+@pytest.mark.parametrize("case", list(CASES))
+def test_walk_equals_the_loops(case, monkeypatch):
+    import lpmm.optim.adamw as adamw
+    import lpmm.optim.sgd as sgd
+    from lpmm import _native
+
+    sides = [_build(case, np.random.default_rng(5)) for _ in range(2)]
+    rng = np.random.default_rng(6)
+    natives = [_Native(_native, True), _Native(_native, False)]
+    for step in range(6):
+        grads = [rng.standard_normal(p.shape) * 0.1 for p in sides[0][0]]
+        for side, ((params, opt), native) in enumerate(zip(sides, natives)):
+            monkeypatch.setattr(adamw, "_native", native)
+            monkeypatch.setattr(sgd, "_native", native)
+            for i, (p, g) in enumerate(zip(params, grads)):
+                p.grad = None if (step + i) % 5 == 4 else torch.from_numpy(g).to(p.dtype).cuda()
+            if step == 3:  # a checkpoint round trip in the middle
+                opt.load_state_dict(copy.deepcopy(opt.state_dict()))
+            if step == 4:  # a state in other memory
+                for s in opt.state.values():
+                    for k, v in s.items():
+                        if torch.is_tensor(v) and v.dtype is torch.int8:
+                            s[k] = v.clone()
+            opt.step()
+        torch.cuda.synchronize()
+        for i, (p, q) in enumerate(zip(sides[0][0], sides[1][0])):
+            assert torch.equal(p.detach(), q.detach()), (step, i)
+            a, b = _state(sides[0][1], p), _state(sides[1][1], q)
+            assert a.keys() == b.keys()
+            for k in a:
+                assert a[k].shape == b[k].shape and a[k].dtype == b[k].dtype, (step, i, k)
+                assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), \
+                    (step, i, k)
+    assert natives[0].served > 0 and natives[1].served == 0
+    # the steady state: everything but the strided tensor (and factored ones) is served
+    native = natives[0]
+    monkeypatch.setattr(adamw, "_native", native)
+    monkeypatch.setattr(sgd, "_native", native)
+    params, opt = sides[0]
+    for _ in range(2):
+        native.rest = 0
+        for p, g in zip(params, grads):
+            p.grad = torch.from_numpy(g).to(p.dtype).cuda()
+        opt.step()
+    matrices = sum(p.dim() > 1 for p in params)
+    # other N-D routes than the default configuration's are the staged path's
+    staged = 2 if case in ("float_m", "wide", "bits") else 0
+    staged += {"wide": 1, "bits": 1}.get(case, 0)  # the 5000-long vector
+    assert native.rest == (matrices if case == "fused_factored" else 0 if case == "fused" else staged + 1), native.rest
+
+
+def test_walk_leaves_overridden_and_subclassed_parameters_to_the_loops():
+    """An override is looked up by the parameter; a subclass of Parameter may define its own .grad."""
+    import lpmm
+    from lpmm import _native
+
+    class Own(torch.nn.Parameter):
+        pass
+
+    class Module(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.a = torch.nn.Parameter(torch.randn(64, 128, device="cuda"))
+            self.b = torch.nn.Parameter(torch.randn(64, 128, device="cuda"))
+            self.c = Own(torch.randn(64, 128, device="cuda"))
+
+    m = Module()
+    opt = lpmm.optim.AdamW(list(m.parameters()), fused=True)
+    opt.override_quantize_enable(m, "b", False)
+    for _ in range(2):
+        for p in m.parameters():
+            p.grad = torch.randn_like(p)
+        opt.step()
+    assert opt.state[m.a]["exp_avg"].dtype is torch.int8 and opt.state[m.b]["exp_avg"].dtype is torch.float32
+    plan = opt._walk(opt.param_groups[0], lpmm.optim.adamw._Routes(opt.get_qmetadata_by_state_name("exp_avg"),
+                                                                    dict(opt.get_qmetadata_by_state_name("exp_avg_sq"), scale_type="group")))
+    assert [p is m.c for p in plan.rest] == [True]
+    kinds = {batch[0]: batch[5] for batch in plan.start()}
+    assert kinds == {_native.WALK_FUSED4: 1, _native.WALK_PLAIN: 1}
