@@ -627,6 +627,14 @@ int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int64_t count,
                              double beta1, double beta2, double lr, double weight_decay, double eps,
                              void *stream);
 
+/* The same for any column count and natural alignment, and for fp32 first moments: a record whose m_max1 is NULL
+ * has m_codes pointing to float[rows * cols], updated in place (first_step is not read).  What
+ * lpmm_factored_stats, lpmm_factored_update and lpmm_factored_update_fp32m compute, in four launches for up to
+ * 24 tensors. */
+int lpmm_factored_any_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
+                                 double beta1, double beta2, double lr, double weight_decay, double eps,
+                                 void *stream);
+
 /* The same pass with an fp32 first moment (m read and written as floats): tensors at or
  * under the quantisation threshold, or first-moment quantisation disabled
  * (the `else: exp_avg = q_exp_avg` branch, lpmm/optim/adamw.py:603-604). */

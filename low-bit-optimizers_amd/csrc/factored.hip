@@ -216,17 +216,16 @@ __global__ void factored_mean_kernel(const double *__restrict__ rowblock, int ro
 // (row, column).
 // ---------------------------------------------------------------------------------------
 template <bool ROWS>
-__global__ __launch_bounds__(kFThreads) void factored_update_kernel(
-    float *__restrict__ p, const float *__restrict__ g, uint8_t *__restrict__ m_codes,
+__device__ __forceinline__ void update_flat_body(
+    uint32_t *lds, float *__restrict__ p, const float *__restrict__ g, uint8_t *__restrict__ m_codes,
     float *__restrict__ m_max1, const float *__restrict__ qmap_m, const float *__restrict__ row,
     const float *__restrict__ col, const float *__restrict__ row_mean_all, int64_t n, int64_t C,
-    int64_t n_groups, int64_t n_padded, NfHyper h, bool first_step, bool vec)
+    int64_t n_groups, int64_t n_padded, const NfHyper &h, bool first_step, bool vec, uint32_t tile)
 {
-    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
     lds_fill(lds, qmap_m, nullptr);
     const int kind = classify_map(qmap_m);
     __syncthreads();
-    const int64_t base = ((int64_t)blockIdx.x * kFThreads + threadIdx.x) * kFElts;
+    const int64_t base = ((int64_t)tile * kFThreads + threadIdx.x) * kFElts;
     if (base == 0)
         m_codes[n_padded / 2] = 0;
     const int64_t grp = base / kGroup;
@@ -306,6 +305,18 @@ __global__ __launch_bounds__(kFThreads) void factored_update_kernel(
             if (base + k < n)
                 p[base + k] = pv[k];
     }
+}
+
+template <bool ROWS>
+__global__ __launch_bounds__(kFThreads) void factored_update_kernel(
+    float *__restrict__ p, const float *__restrict__ g, uint8_t *__restrict__ m_codes,
+    float *__restrict__ m_max1, const float *__restrict__ qmap_m, const float *__restrict__ row,
+    const float *__restrict__ col, const float *__restrict__ row_mean_all, int64_t n, int64_t C,
+    int64_t n_groups, int64_t n_padded, NfHyper h, bool first_step, bool vec)
+{
+    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    update_flat_body<ROWS>(lds, p, g, m_codes, m_max1, qmap_m, row, col, row_mean_all, n, C, n_groups, n_padded, h,
+                           first_step, vec, blockIdx.x);
 }
 
 // The same pass when the column count is a multiple of 128: every 128-element group of the
@@ -433,13 +444,13 @@ __global__ __launch_bounds__(kFThreads) void factored_update_rows128_kernel(
 
 // The same update with an fp32 first moment (tensors at or under the quantisation threshold,
 // or first-moment quantisation disabled): m is read and written as floats.
-__global__ __launch_bounds__(kFThreads) void factored_update_fp32m_kernel(
+__device__ __forceinline__ void update_fp32m_body(
     float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m, const float *__restrict__ row,
-    const float *__restrict__ col, const float *__restrict__ row_mean_all, int64_t n, int64_t C, NfHyper h)
+    const float *__restrict__ col, const float *__restrict__ row_mean_all, int64_t n, int64_t C, const NfHyper &h,
+    int64_t begin, int64_t stride)
 {
     const float mean_all = *row_mean_all;
-    const int64_t stride = (int64_t)gridDim.x * kFThreads;
-    for (int64_t i = (int64_t)blockIdx.x * kFThreads + threadIdx.x; i < n; i += stride) {
+    for (int64_t i = begin + threadIdx.x; i < n; i += stride) {
         const int64_t r = i / C, c = i - r * C;
         const float pi = p[i] * h.decay;
         const float mi = lerp_w(m[i], g[i], h.w1);
@@ -448,6 +459,14 @@ __global__ __launch_bounds__(kFThreads) void factored_update_fp32m_kernel(
         p[i] = pi + div_fast(h.neg_step_size * mi, denom);
         m[i] = mi;
     }
+}
+
+__global__ __launch_bounds__(kFThreads) void factored_update_fp32m_kernel(
+    float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m, const float *__restrict__ row,
+    const float *__restrict__ col, const float *__restrict__ row_mean_all, int64_t n, int64_t C, NfHyper h)
+{
+    update_fp32m_body(p, g, m, row, col, row_mean_all, n, C, h, (int64_t)blockIdx.x * kFThreads,
+                      (int64_t)gridDim.x * kFThreads);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -474,9 +493,14 @@ struct TensorFa {
     uint32_t tiles_x, tiles_y;  // statistics tiles
     uint32_t row_blocks;        // finalize: workgroups that take rows; the rest take 64 columns each
     uint32_t upd_x;             // update: 2048-element tiles of the tensor
-    uint32_t first_step;
+    uint32_t first_step : 1;
+    // general launch groups: g allows 16-byte loads in the statistics pass, p and g in the update; the update's kind
+    uint32_t vec_g : 1, vec : 1, kind : 2;
     float neg_step_size, bc2_sqrt, rbc2_sqrt;
 };
+
+// updates of a general launch group: fp32 first moment, a multiple of 8 columns, any other column count
+enum FlatKind : uint32_t { kFlatFloat = 0, kFlatRows = 1, kFlatAny = 2 };
 
 // Launch groups are bounded by the tensor count alone.  Both passes stream the gradient from HBM
 // (nontemporal loads): batches small enough for the statistics pass to leave the gradient in the
@@ -548,6 +572,48 @@ __global__ __launch_bounds__(kFThreads) void factored_update_multi_kernel(const 
     h.rbc2_sqrt = t.rbc2_sqrt;
     update_rows128_body(t.p, t.g, t.mc, t.ms, qmap_m, t.row, t.col, t.mean, t.R, t.C, t.n_padded, h,
                         t.first_step != 0, local);
+}
+
+// General launch groups: any column count and alignment, fp32 first moments.  One launch each for up to 24 tensors
+// in place of four per tensor, whose gaps and host time took most of a step on small matrices (three layers of
+// width 248: 295 -> 51 us a step; 48 layers of width 64, half of whose matrices keep fp32 first moments: 3110 -> 326).
+// The bodies are those of the single-tensor kernels: same results.
+__global__ __launch_bounds__(kFThreads) void factored_partial_any_multi_kernel(const MultiFa args)
+{
+    const int i = find_slot(args.start_stats, blockIdx.x);
+    const TensorFa &t = args.t[i];
+    const uint32_t local = blockIdx.x - args.start_stats[i];
+    const uint32_t by = local / t.tiles_x, bx = local - by * t.tiles_x;
+    partial_body(t.g, t.R, t.C, t.colpart, t.rowpart, t.vec_g != 0, bx, by);
+}
+
+__global__ __launch_bounds__(kFThreads) void factored_update_any_multi_kernel(const MultiFa args,
+                                                                              const float *__restrict__ qmap_m)
+{
+    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    const int i = find_slot(args.start_upd, blockIdx.x);
+    const TensorFa &t = args.t[i];
+    const uint32_t tile = blockIdx.x - args.start_upd[i];
+    NfHyper h;
+    h.decay = args.decay;
+    h.w1 = args.w1;
+    h.b2 = args.b2;
+    h.w2 = args.w2;
+    h.eps = args.eps;
+    h.neg_step_size = t.neg_step_size;
+    h.bc2_sqrt = t.bc2_sqrt;
+    h.rbc2_sqrt = t.rbc2_sqrt;
+    const int64_t n = t.R * t.C, n_groups = (n + kGroup - 1) / kGroup;
+    if (t.kind == kFlatFloat) {
+        const int64_t begin = (int64_t)tile * kFTile, end = begin + kFTile < n ? begin + kFTile : n;
+        update_fp32m_body(t.p, t.g, reinterpret_cast<float *>(t.mc), t.row, t.col, t.mean, end, t.C, h, begin, kFThreads);
+    } else if (t.kind == kFlatRows) {
+        update_flat_body<true>(lds, t.p, t.g, t.mc, t.ms, qmap_m, t.row, t.col, t.mean, n, t.C, n_groups, t.n_padded, h,
+                               t.first_step != 0, t.vec != 0, tile);
+    } else {
+        update_flat_body<false>(lds, t.p, t.g, t.mc, t.ms, qmap_m, t.row, t.col, t.mean, n, t.C, n_groups, t.n_padded, h,
+                                t.first_step != 0, t.vec != 0, tile);
+    }
 }
 
 inline int64_t round_up(int64_t a, int64_t b) { return (a + b - 1) / b * b; }
@@ -782,10 +848,11 @@ extern "C" int lpmm_factored_update_fp32m(float *p, const float *g, float *m, co
     return launch_status();
 }
 
-extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
-                                        double beta1, double beta2, double lr, double weight_decay, double eps,
-                                        void *stream)
+// general: any column count and natural alignment; a tensor without m_max1 has an fp32 first moment
+static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m, double beta1,
+                          double beta2, double lr, double weight_decay, double eps, bool general, void *stream)
 {
+    const uintptr_t align = general ? 4 : 16;
     if (count < 0)
         return LPMM_ERR_SIZE;
     if (count == 0)
@@ -795,26 +862,27 @@ extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int
     LPMM_REQUIRE_ALIGN(qmap_m, 4);
     for (int64_t i = 0; i < count; ++i) {
         const lpmm_factored_tensor &t = tensors[i];
-        if (t.rows <= 0 || t.cols <= 0 || t.cols % kGroup != 0 || t.rows > INT64_MAX / t.cols)
+        if (t.rows <= 0 || t.cols <= 0 || (!general && t.cols % kGroup != 0) || t.rows > INT64_MAX / t.cols)
             return LPMM_ERR_SIZE;
         const int64_t ty = (t.rows + kSRows - 1) / kSRows, tx = (t.cols + kSCols - 1) / kSCols;
         const int64_t ux = (t.cols + kFTile - 1) / kFTile + 1;  // per row: an upper bound for any tile shape
-        if (tx > 0x7fffffffLL / ty || ux > 0x7fffffffLL / t.rows ||
+        if ((general && ty > 65535) || tx > 0x7fffffffLL / ty || ux > 0x7fffffffLL / t.rows ||
             (t.rows + kFThreads - 1) / kFThreads + (t.cols + 63) / 64 > 0x7fffffffLL)
             return LPMM_ERR_SIZE;
         LPMM_REQUIRE_PTR(t.p);
         LPMM_REQUIRE_PTR(t.g);
         LPMM_REQUIRE_PTR(t.m_codes);
-        LPMM_REQUIRE_PTR(t.m_max1);
+        if (!general)
+            LPMM_REQUIRE_PTR(t.m_max1);
         LPMM_REQUIRE_PTR(t.row);
         LPMM_REQUIRE_PTR(t.col);
         LPMM_REQUIRE_PTR(t.workspace);
-        LPMM_REQUIRE_ALIGN(t.p, 16);
-        LPMM_REQUIRE_ALIGN(t.g, 16);
+        LPMM_REQUIRE_ALIGN(t.p, align);
+        LPMM_REQUIRE_ALIGN(t.g, align);
         LPMM_REQUIRE_ALIGN(t.m_codes, 4);
         LPMM_REQUIRE_ALIGN(t.m_max1, 4);
         LPMM_REQUIRE_ALIGN(t.row, 4);
-        LPMM_REQUIRE_ALIGN(t.col, 16);
+        LPMM_REQUIRE_ALIGN(t.col, align);
         LPMM_REQUIRE_ALIGN(t.workspace, 8);
     }
 
@@ -835,7 +903,7 @@ extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int
             const uint64_t ty = (uint64_t)((t.rows + kSRows - 1) / kSRows), tx = (uint64_t)((t.cols + kSCols - 1) / kSCols);
             const uint64_t row_blocks = (uint64_t)((t.rows + kFThreads - 1) / kFThreads);
             const uint64_t fin = row_blocks + (uint64_t)((t.cols + 63) / 64);
-            const uint64_t ux = update_tiles(t.rows, t.cols);
+            const uint64_t ux = general ? (uint64_t)((t.rows * t.cols + kFTile - 1) / kFTile) : update_tiles(t.rows, t.cols);
             if (n_stats + tx * ty > 0x7fffffffULL || n_fin + fin > 0x7fffffffULL ||
                 n_upd + ux > 0x7fffffffULL) {
                 if (k == 0)
@@ -861,6 +929,9 @@ extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int
             d.row_blocks = (uint32_t)row_blocks;
             d.upd_x = (uint32_t)ux;
             d.first_step = t.first_step != 0;
+            d.vec_g = aligned_to(t.g, 16) && t.cols % 4 == 0;
+            d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16);
+            d.kind = t.m_max1 == nullptr ? kFlatFloat : t.cols % 8 == 0 && aligned_to(t.col, 16) ? kFlatRows : kFlatAny;
             const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
@@ -881,13 +952,33 @@ extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int
             args.start_upd[j] = (uint32_t)n_upd;
         }
         hipStream_t s = (hipStream_t)stream;
-        hipLaunchKernelGGL(factored_partial_multi_kernel, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
+        if (general)
+            hipLaunchKernelGGL(factored_partial_any_multi_kernel, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
+        else
+            hipLaunchKernelGGL(factored_partial_multi_kernel, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
         hipLaunchKernelGGL(factored_finalize_multi_kernel, dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
         hipLaunchKernelGGL(factored_mean_multi_kernel, dim3((uint32_t)k), dim3(kWave), 0, s, args);
-        hipLaunchKernelGGL(factored_update_multi_kernel, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
+        if (general)
+            hipLaunchKernelGGL(factored_update_any_multi_kernel, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
+        else
+            hipLaunchKernelGGL(factored_update_multi_kernel, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;
     }
     return LPMM_OK;
+}
+
+extern "C" int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
+                                        double beta1, double beta2, double lr, double weight_decay, double eps,
+                                        void *stream)
+{
+    return factored_multi(tensors, count, qmap_m, beta1, beta2, lr, weight_decay, eps, false, stream);
+}
+
+extern "C" int lpmm_factored_any_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
+                                            double beta1, double beta2, double lr, double weight_decay, double eps,
+                                            void *stream)
+{
+    return factored_multi(tensors, count, qmap_m, beta1, beta2, lr, weight_decay, eps, true, stream);
 }

@@ -26,7 +26,7 @@
 namespace {
 
 enum Kind : int { kFused4, kPlain, kFlat, kRank1, kNd, kFlatM32, kRank1M32, kRank1Bits, kRank1Wide, kSgd4, kSgdPlain,
-                  kAny, kNdAny, kHalfPlain, kHalfFlat, kHalfRank1, kKinds };
+                  kAny, kNdAny, kHalfPlain, kHalfFlat, kHalfRank1, kFactored, kFactoredAny, kKinds };
 
 constexpr size_t kRecordBytes[kKinds] = {
     sizeof(lpmm_adamw4bit_tensor),     sizeof(lpmm_adamw_fp32_tensor),     sizeof(lpmm_adamw4bit_tensor),
@@ -34,10 +34,10 @@ constexpr size_t kRecordBytes[kKinds] = {
     sizeof(lpmm_rank1_v4bit_tensor),   sizeof(lpmm_nonfused_rank1_tensor), sizeof(lpmm_rank1_mgroup_tensor),
     sizeof(lpmm_sgd4bit_tensor),       sizeof(lpmm_sgd_fp32_tensor),       sizeof(lpmm_rank1_any_tensor),
     sizeof(lpmm_rank1_any_tensor),     sizeof(lpmm_adamw_fp32_tensor),     sizeof(lpmm_adamw4bit_f16_tensor),
-    sizeof(lpmm_nonfused_rank1_f16_tensor)};
+    sizeof(lpmm_nonfused_rank1_f16_tensor), sizeof(lpmm_factored_tensor), sizeof(lpmm_factored_tensor)};
 
 struct Names {
-    PyObject *step, *exp_avg, *exp_avg_sq, *exp_avg_qstate, *exp_avg_sq_qstate, *exp_avg_sq_row, *enable, *overhead, *qmap, *max1,
+    PyObject *step, *exp_avg, *exp_avg_sq, *exp_avg_qstate, *exp_avg_sq_qstate, *exp_avg_sq_row, *exp_avg_sq_col, *enable, *overhead, *qmap, *max1,
         *max_dims, *work, *scale_of, *row, *momentum_buffer, *momentum_buffer_qstate, *dtype;
 } N;
 
@@ -97,7 +97,8 @@ T *ptr(const at::Tensor &t)
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 struct Settings {
-    int fused, m_group128, v_group128, v_rank1, m_wide, bits_rank1;
+    int fused;  // 0: the non-fused path, 1: the fused operators, 2: settings the fused operators warn about or refuse
+    int m_group128, v_group128, v_rank1, m_wide, bits_rank1;
     int64_t m_group;
 };
 
@@ -105,6 +106,7 @@ struct Walk {
     Plan *plan;
     PyObject *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
     Settings s;
+    int64_t (*workspace_bytes)(int64_t, int64_t);  // lpmm_factored_workspace_bytes
 
     // a dense tensor of n values beside p and of its type (parameters on the kernels are float or half)
     static const at::Tensor *reals_of(PyObject *o, const at::Tensor &p, int64_t n)
@@ -213,6 +215,7 @@ struct Walk {
     }
 
     bool adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+    bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
     bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
     bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const at::Tensor *mc,
              const at::Tensor *ms, const at::Tensor &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
@@ -227,13 +230,18 @@ void swap_later(Item &item, PyObject *dict, PyObject *key, PyObject *value) { it
 bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
 {
     if (!g.defined() || !on_gpu(p) || !on_gpu(g) || p.device() != g.device() || p.numel() != g.numel() ||
-        g.scalar_type() != p.scalar_type() || get(st, N.exp_avg_sq_row) != nullptr)
+        g.scalar_type() != p.scalar_type())
         return false;
     const at::Tensor *step = tensor_of(get(st, N.step));
     if (step == nullptr || !step->is_cpu() || step->scalar_type() != at::kFloat || step->dim() != 0)
         return false;
+    const bool is_factored = get(st, N.exp_avg_sq_row) != nullptr;
     if (!floats(p))
-        return halfs(p) && !s.fused && half(po, p, g, st, *step);
+        return halfs(p) && !s.fused && !is_factored && half(po, p, g, st, *step);
+    if (is_factored)
+        return factored(po, p, g, st, *step);
+    if (s.fused == 2)
+        return false;
     PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
     PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
     const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
@@ -396,6 +404,45 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
         swap_later(item, oh_m, N.max1, spare);
     }
     add(batch(kAny, p, qm, qv, kind), r, item);
+    return true;
+}
+
+// a matrix with a factored second moment, its first moment 4-bit in groups of 128 values or not quantised
+bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step)
+{
+    if (p.dim() != 2 || p.numel() == 0 || workspace_bytes == nullptr)
+        return false;
+    const int64_t rows = p.size(0), cols = p.size(1), n = p.numel();
+    PyObject *qs = get(st, N.exp_avg_qstate), *mo = get(st, N.exp_avg), *qm = get(qs, N.qmap), *oh = nullptr;
+    const at::Tensor *row = reals_of(get(st, N.exp_avg_sq_row), p, rows), *col = reals_of(get(st, N.exp_avg_sq_col), p, cols);
+    const at::Tensor *map = tensor_of(qm);
+    const int en = enabled(po, qs);
+    if (en < 0 || row == nullptr || col == nullptr || map == nullptr || !floats(*map))
+        return false;
+    Item item;
+    item.step = ptr<float>(step);
+    lpmm_factored_tensor r;
+    memset(&r, 0, sizeof r);
+    r.p = ptr<float>(p);
+    r.g = ptr<float>(g);
+    r.row = ptr<float>(*row);
+    r.col = ptr<float>(*col);
+    r.rows = rows;
+    r.cols = cols;
+    if (en) {
+        const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *ms = scales(qs, &oh, p, (n + 127) / 128);
+        if (!s.m_group128 || mc == nullptr || ms == nullptr)
+            return false;
+        r.m_codes = ptr<uint8_t>(*mc);
+        r.m_max1 = ptr<float>(*ms);
+    } else {
+        const at::Tensor *m = reals_like(mo, p);
+        if (m == nullptr)
+            return false;
+        r.m_codes = ptr<uint8_t>(*m);
+    }
+    r.workspace = scratch(p, (workspace_bytes(rows, cols) + 3) / 4);
+    add(batch(en && cols % 128 == 0 ? kFactored : kFactoredAny, p, qm, nullptr), r, item);
     return true;
 }
 
@@ -586,7 +633,7 @@ PyObject *plan_start(PyObject *self, PyObject *)
         const bool has_step = b.kind != kSgd4 && b.kind != kSgdPlain;
         for (size_t i = 0; i < b.items.size() && has_step; ++i) {
             const float step = *b.items[i].step += 1.0f;
-            // every record ends in  float step, reserved
+            // every record ends in  float step  and four more bytes
             memcpy(&b.records[(i + 1) * bytes - 8], &step, 4);
             if (!b.second.empty())
                 memcpy(&b.second[(i + 1) * bytes - 8], &step, 4);
@@ -636,18 +683,21 @@ PyGetSetDef plan_getset[] = {{"served", plan_served, nullptr, "are there records
                              {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
-// collect(sgd, params, state, override, spare_stats, spare_scales, nd_scratch, serve, settings)
+// collect(sgd, params, state, override, spare_stats, spare_scales, nd_scratch, serve, settings,
+// address of lpmm_factored_workspace_bytes or 0)
 PyObject *collect(PyObject *, PyObject *args)
 {
     int is_sgd, serve;
     PyObject *params, *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
     Walk w;
     int m_group;
-    if (!PyArg_ParseTuple(args, "iO!O!O!O!O!O!p(iiiiiii)", &is_sgd, &PyList_Type, &params, &PyDict_Type, &state, &PyDict_Type,
+    unsigned long long workspace;
+    if (!PyArg_ParseTuple(args, "iO!O!O!O!O!O!p(iiiiiii)K", &is_sgd, &PyList_Type, &params, &PyDict_Type, &state, &PyDict_Type,
                           &override_, &PyDict_Type, &spare_stats, &PyDict_Type, &spare_scales, &PyDict_Type, &nd_scratch, &serve,
-                          &w.s.fused, &w.s.m_group128, &w.s.v_group128, &w.s.v_rank1, &w.s.m_wide, &w.s.bits_rank1, &m_group))
+                          &w.s.fused, &w.s.m_group128, &w.s.v_group128, &w.s.v_rank1, &w.s.m_wide, &w.s.bits_rank1, &m_group, &workspace))
         return nullptr;
     w.s.m_group = m_group;
+    w.workspace_bytes = reinterpret_cast<int64_t (*)(int64_t, int64_t)>((uintptr_t)workspace);
     Plan *plan = reinterpret_cast<Plan *>(PlanType.tp_alloc(&PlanType, 0));
     if (plan == nullptr)
         return nullptr;
@@ -715,6 +765,7 @@ PyMODINIT_FUNC PyInit__walk()
     LPMM_NAME(exp_avg_qstate);
     LPMM_NAME(exp_avg_sq_qstate);
     LPMM_NAME(exp_avg_sq_row);
+    LPMM_NAME(exp_avg_sq_col);
     LPMM_NAME(enable);
     LPMM_NAME(overhead);
     LPMM_NAME(qmap);

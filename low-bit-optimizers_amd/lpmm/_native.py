@@ -74,6 +74,7 @@ PROTOTYPES = {
     "lpmm_factored_stats_static": (_int, [_vp, _i64, _i64, _vp, _vp, _vp, _d, _vp]),
     "lpmm_factored_update": (_int, [_vp] * 8 + [_i64, _i64] + [_d] * 6 + [_int, _vp]),
     "lpmm_factored_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
+    "lpmm_factored_any_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
     "lpmm_factored_update_fp32m": (_int, [_vp] * 6 + [_i64, _i64] + [_d] * 6 + [_vp]),
     "lpmm_sgd4bit_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 4 + [_int, _int, _vp]),
     "lpmm_sgd_fp32_step_multi": (_int, [_vp, _i64] + [_d] * 4 + [_int, _int, _vp]),
@@ -162,9 +163,15 @@ def walk():
     return _walk
 
 
+def factored_workspace():
+    """Address of lpmm_factored_workspace_bytes, which the walk calls."""
+    return ctypes.cast(lib().lpmm_factored_workspace_bytes, ctypes.c_void_p).value
+
+
 # kinds of records a walk makes (enum Kind of csrc/walk.cpp)
 (WALK_FUSED4, WALK_PLAIN, WALK_FLAT, WALK_RANK1, WALK_ND, WALK_FLAT_M32, WALK_RANK1_M32, WALK_RANK1_BITS, WALK_RANK1_WIDE, WALK_SGD4,
- WALK_SGD_PLAIN, WALK_ANY, WALK_ND_ANY, WALK_HALF_PLAIN, WALK_HALF_FLAT, WALK_HALF_RANK1) = range(16)
+ WALK_SGD_PLAIN, WALK_ANY, WALK_ND_ANY, WALK_HALF_PLAIN, WALK_HALF_FLAT, WALK_HALF_RANK1, WALK_FACTORED,
+ WALK_FACTORED_ANY) = range(18)
 
 
 def check(status, what):

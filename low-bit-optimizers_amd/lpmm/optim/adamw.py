@@ -240,10 +240,12 @@ class AdamW(LowBitOptimizer):
 
     def _walk(self, group, routes):
         fused = bool(group["fused"])
+        # a factored tensor takes the same kernels whatever the group's flag and the second moment's settings
         return _native.walk().collect(
             0, group["params"], self.state, self.override_q_enable, self._spare_stats, self._spare_scales, self._nd_scratch,
-            routes.fused4 if fused else True,
-            (fused, routes.m_group128, routes.v_group128, routes.v_rank1, routes.m_group_wide, routes.bits_rank1, routes.m["gp_sz"]))
+            True,
+            (0 if not fused else 1 if routes.fused4 else 2, routes.m_group128, routes.v_group128, routes.v_rank1, routes.m_group_wide, routes.bits_rank1, routes.m["gp_sz"]),
+            _native.factored_workspace())
 
     def _launch_walk(self, group, plan, routes):
         """The launches of the walk's records: those that _step_fused and _step_single make."""
@@ -263,6 +265,9 @@ class AdamW(LowBitOptimizer):
                     st = lib.lpmm_nonfused_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
                 elif kind == _native.WALK_FLAT_M32:
                     st = lib.lpmm_nonfused_adamw_v4bit_step_multi(records, count, qv_ptr, *hyper, stream)
+                elif kind in (_native.WALK_FACTORED, _native.WALK_FACTORED_ANY):
+                    run = lib.lpmm_factored_step_multi if kind == _native.WALK_FACTORED else lib.lpmm_factored_any_step_multi
+                    st = run(records, count, qm_ptr, *hyper, stream)
                 elif kind == _native.WALK_HALF_PLAIN:
                     st = lib.lpmm_nonfused_update_f16_multi(records, count, *hyper, stream)
                 elif kind == _native.WALK_HALF_FLAT:
@@ -1192,9 +1197,9 @@ class AdamW(LowBitOptimizer):
 
     # ---- factored second moment (lpmm/optim/adamw.py:579-627) ---------------------------
     def _factored_steps(self, group, items):
-        """Factored tensors of a parameter group: 2-D tensors with a multiple of 128 columns and a
-        4-bit block-wise first moment go to the multi-tensor kernels together, the others one
-        by one."""
+        """Factored tensors of a parameter group: matrices with a 4-bit block-wise or an unquantised first moment
+        go to the multi-tensor kernels together (those with a multiple of 128 columns and a quantised one to the
+        tuned launch), the others one by one."""
         if not items:
             return
         beta1, beta2 = group["betas"]
@@ -1203,39 +1208,47 @@ class AdamW(LowBitOptimizer):
         m_fits = (md_m["scale_type"] == "group" and md_m["gp_sz"] == 128 and md_m["b"] == 4
                   and md_m["round_type"] == "real-nearest")
         lib = _native.lib()
-        batched = {}
+        batched, general = {}, {}
         held = []  # contiguous copies of strided operands
+        kept = []
         for p, grad, state, step in items:
             dense, grad = self._dense_operands(p, grad, held)
-            if not (m_fits and p.dim() == 2 and p.shape[1] % 128 == 0 and self._enabled(p, state, "exp_avg")):
+            enabled = self._enabled(p, state, "exp_avg")
+            if p.dim() != 2 or p.numel() == 0 or (enabled and not m_fits):
                 self._factored_step(group, p, dense, grad, state, step)
                 continue
             rows, cols = p.shape
             qstate = state["exp_avg_qstate"]
-            first = _is_placeholder(state["exp_avg"])
-            if first:
-                groups = p.numel() // 128
-                state["exp_avg"] = torch.empty((packed_nbytes(p.numel()),), dtype=torch.int8, device=p.device)
-                qstate["overhead"].clear()
-                qstate["overhead"].update({"dtype": p.dtype, "stride": self._state_stride(p),
-                                           "max1": torch.empty((groups, 1), dtype=torch.float32, device=p.device),
-                                           "scaled_shape": torch.Size((groups, 128))})
+            tuned = enabled and cols % 128 == 0
+            first = False
+            if enabled:
+                first = _is_placeholder(state["exp_avg"])
+                if first:
+                    groups = (p.numel() + 127) // 128
+                    state["exp_avg"] = torch.empty((packed_nbytes(groups * 128),), dtype=torch.int8, device=p.device)
+                    qstate["overhead"].clear()
+                    qstate["overhead"].update({"dtype": p.dtype, "stride": self._state_stride(p),
+                                               "max1": torch.empty((groups, 1), dtype=torch.float32, device=p.device),
+                                               "scaled_shape": torch.Size((groups, 128))})
+                m, ms = state["exp_avg"].data_ptr(), qstate["overhead"]["max1"].data_ptr()
+            else:
+                kept.append(self._materialise(p, state, "exp_avg", False, md_m))
+                m, ms = kept[-1].data_ptr(), 0
             key = (p.device, qstate["qmap"].data_ptr())
             ws = (lib.lpmm_factored_workspace_bytes(rows, cols) + 255) // 256 * 256
-            batched.setdefault(key, []).append(
-                [dense.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(), qstate["overhead"]["max1"].data_ptr(),
-                 state["exp_avg_sq_row"].data_ptr(), state["exp_avg_sq_col"].data_ptr(), ws, rows, cols, step,
-                 1 if first else 0])
-        for (dev, qm_ptr), records in batched.items():
-            with torch.cuda.device(dev):
-                work = torch.empty((sum(r[6] for r in records),), dtype=torch.uint8, device=dev)
-                offset = work.data_ptr()
-                for r in records:
-                    r[6], offset = offset, offset + r[6]
-                table = np.array([tuple(r) for r in records], dtype=_native.FACTORED_TENSOR)
-                st = lib.lpmm_factored_step_multi(table.ctypes.data, len(records), qm_ptr, beta1, beta2, lr, wd, eps,
-                                                  _native.current_stream(dev))
-            _native.check(st, "factored step")
+            (batched if tuned else general).setdefault(key, []).append(
+                [dense.data_ptr(), grad.data_ptr(), m, ms, state["exp_avg_sq_row"].data_ptr(),
+                 state["exp_avg_sq_col"].data_ptr(), ws, rows, cols, step, 1 if first else 0])
+        for run, tables in ((lib.lpmm_factored_step_multi, batched), (lib.lpmm_factored_any_step_multi, general)):
+            for (dev, qm_ptr), records in tables.items():
+                with torch.cuda.device(dev):
+                    work = torch.empty((sum(r[6] for r in records),), dtype=torch.uint8, device=dev)
+                    offset = work.data_ptr()
+                    for r in records:
+                        r[6], offset = offset, offset + r[6]
+                    table = np.array([tuple(r) for r in records], dtype=_native.FACTORED_TENSOR)
+                    st = run(table.ctypes.data, len(records), qm_ptr, beta1, beta2, lr, wd, eps, _native.current_stream(dev))
+                _native.check(st, "factored step")
         self._write_back(held)
 
     def _factored_step(self, group, p, dense, grad, state, step):

@@ -250,3 +250,60 @@ def test_factored_step_multi_large_batches_equal_single_tensor_calls(qmaps):
     for x, y in zip(a, b):
         for k in ("p", "row", "col", "codes", "max1"):
             assert torch.equal(x[k], y[k]), f'{k} of {x["r"]}x{x["c"]}'
+
+
+def test_factored_any_step_multi_equals_single_tensor_calls(qmaps):
+    """lpmm_factored_any_step_multi on column counts of every kind (whole groups, a multiple of 8, of 4, of 2, odd), one
+    column, one row, unaligned operands, fp32 first moments and first steps, 26 tensors (two launch groups): bit for bit
+    what the single-tensor calls leave."""
+    from lpmm import _native
+
+    lib = _lib()
+    dqm = to_dev(qmaps[0])
+    gen = torch.Generator(device="cuda").manual_seed(78)
+    shapes = [(64, 128), (300, 190), (70, 1000), (65, 764), (33, 257), (1, 9000), (9000, 1), (257, 66)] * 3 + [(50, 60), (700, 520)]
+
+    def fresh(i, r, c):
+        n, off = r * c, int(i % 4 == 3)
+        groups = (n + 127) // 128
+        dense = lambda scale: (torch.randn(n + off, device="cuda", generator=gen) * scale)[off:]
+        t = dict(r=r, c=c, fp32=i % 5 == 4, first=int(i % 5 == 2), p=dense(0.02), g=dense(1e-3), m=dense(1e-3),
+                 row=torch.rand(r, device="cuda", generator=gen) * 1e-6, col=torch.rand(c + off, device="cuda", generator=gen)[off:] * 1e-6,
+                 codes=torch.randint(0, 256, ((n + 2047) // 2048 * 1024 + 1,), dtype=torch.uint8, device="cuda", generator=gen),
+                 max1=torch.rand(groups, device="cuda", generator=gen) * 1e-3,
+                 work=torch.empty(lib.lpmm_factored_workspace_bytes(r, c), dtype=torch.uint8, device="cuda"))
+        return t
+
+    def copied(v):  # at the same offset within its 16 bytes
+        off = v.data_ptr() % 16 // v.element_size()
+        return torch.cat([v.new_zeros(off), v])[off:]
+
+    a = [fresh(i, r, c) for i, (r, c) in enumerate(shapes)]
+    b = [{k: (copied(v) if torch.is_tensor(v) and v.is_floating_point() else v.clone() if torch.is_tensor(v) else v)
+          for k, v in t.items()} for t in a]
+    recs = [(t["p"].data_ptr(), t["g"].data_ptr(), t["m"].data_ptr() if t["fp32"] else t["codes"].data_ptr(),
+             0 if t["fp32"] else t["max1"].data_ptr(), t["row"].data_ptr(), t["col"].data_ptr(), t["work"].data_ptr(), t["r"], t["c"],
+             7.0, t["first"]) for t in a]
+    table = np.array(recs, dtype=_native.FACTORED_TENSOR)
+    hyper = (H["beta1"], H["beta2"], H["lr"], H["wd"], H["eps"])
+    assert lib.lpmm_factored_any_step_multi(table.ctypes.data, len(recs), dqm.data_ptr(), *hyper, _stream()) == 0
+    mean_all = torch.zeros(1, dtype=torch.float32, device="cuda")
+    for t in b:
+        r, c = t["r"], t["c"]
+        assert lib.lpmm_factored_stats(t["g"].data_ptr(), r, c, t["row"].data_ptr(), t["col"].data_ptr(), mean_all.data_ptr(),
+                                       H["beta2"], t["work"].data_ptr(), _stream()) == 0
+        if t["fp32"]:
+            assert lib.lpmm_factored_update_fp32m(t["p"].data_ptr(), t["g"].data_ptr(), t["m"].data_ptr(), t["row"].data_ptr(),
+                                                  t["col"].data_ptr(), mean_all.data_ptr(), r, c, *hyper, 7.0, _stream()) == 0
+        else:
+            assert lib.lpmm_factored_update(t["p"].data_ptr(), t["g"].data_ptr(), t["codes"].data_ptr(), t["max1"].data_ptr(),
+                                            dqm.data_ptr(), t["row"].data_ptr(), t["col"].data_ptr(), mean_all.data_ptr(), r, c,
+                                            *hyper, 7.0, t["first"], _stream()) == 0
+    torch.cuda.synchronize()
+    for i, (x, y) in enumerate(zip(a, b)):
+        for k in ("p", "m", "row", "col", "codes", "max1"):
+            assert torch.equal(x[k], y[k]), f'{k} of tensor {i}, {x["r"]}x{x["c"]}'
+    bad = list(recs[1])
+    bad[1] = 0
+    table = np.array([tuple(bad)], dtype=_native.FACTORED_TENSOR)
+    assert lib.lpmm_factored_any_step_multi(table.ctypes.data, 1, dqm.data_ptr(), *hyper, _stream()) != 0
