@@ -47,6 +47,9 @@ __device__ __forceinline__ MixConst mix_const()
 __device__ __forceinline__ float mix_mul(h16 a, float b, const MixConst &c) { return __builtin_fmaf((float)a, b, c.neg_zero); }
 __device__ __forceinline__ float mix_add(h16 a, float b, const MixConst &c) { return __builtin_fmaf((float)a, c.one, b); }
 
+// a * b + c rounded to half once, from the exact result (v_fma_mixlo_f16: nothing pins the float result here)
+__device__ __forceinline__ h16 round_once_fma(float a, float b, h16 c) { return (h16)__builtin_fmaf(a, b, (float)c); }
+
 // rh of two values; see rh for the pins
 __device__ __forceinline__ v2h round2(float a, float b)
 {
@@ -104,12 +107,37 @@ __device__ __forceinline__ void store_pairs(h16 *p, const v2h (&x)[kPairs])
     __builtin_nontemporal_store(hi, reinterpret_cast<v2w *>(p + 64));
 }
 
-// v.mul_(beta2).addcmul_(g, g, value=1 - beta2) on half tensors
+// v.mul_(beta2).addcmul_(g, g, value=1 - beta2) on half tensors, as PyTorch's CPU kernel: v + (value * g) * g
 __device__ __forceinline__ v2h half_second_moment(v2h v, v2h g, const NfHyper &h, const MixConst &c)
 {
     v = round2(mix_mul(v.x, h.b2, c), mix_mul(v.y, h.b2, c));
     const float ax = mix_mul(g.x, mix_mul(g.x, h.w2, c), c), ay = mix_mul(g.y, mix_mul(g.y, h.w2, c), c);
     return round2(mix_add(v.x, ax, c), mix_add(v.y, ay, c));
+}
+
+// The same as PyTorch's GPU kernel leaves it, for the kernels that stand for the chain of device ops (any column
+// count, states that are not quantised): v + value * (g * g), the square exact in float.  With beta2 = 0.999 one gradient
+// in a few hundred puts that sum half way between two halfs, where it shows how it is rounded, as the product before it does: twice (to float, then to
+// half) in whole blocks of 2048 values of operands on 16-byte boundaries, and once (a mixed-precision fma) behind
+// them and everywhere on other boundaries.  once: bit 0 for the first value, bit 1 for the second.
+constexpr int64_t kOpsBlock = 2048;
+
+__device__ __forceinline__ int64_t ops_twice(const void *a, const void *b, int64_t n)
+{
+    return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 ? n / kOpsBlock * kOpsBlock : 0;
+}
+
+__device__ __forceinline__ v2h half_second_moment_ops(v2h v, v2h g, const NfHyper &h, const MixConst &c, uint32_t once)
+{
+    const v2h d = round2(mix_mul(v.x, h.b2, c), mix_mul(v.y, h.b2, c));
+    const float gx = mix_mul(g.x, (float)g.x, c), gy = mix_mul(g.y, (float)g.y, c);
+    v2h r = round2(mix_add(d.x, h.w2 * gx, c), mix_add(d.y, h.w2 * gy, c));
+    const h16 none = (h16)c.neg_zero;
+    if (once & 1u)
+        r.x = round_once_fma(h.w2, gx, round_once_fma((float)v.x, h.b2, none));
+    if (once & 2u)
+        r.y = round_once_fma(h.w2, gy, round_once_fma((float)v.y, h.b2, none));
+    return r;
 }
 
 // m.lerp_(g, 1 - beta1); NEAR: the weight lies below 0.5 (lerp_w)
@@ -163,9 +191,10 @@ __device__ __forceinline__ v2h half_param(v2h p, v2h m, v2h v, const NfHyper &h,
 }
 
 // A lane's eight elements through the chain; p, m and v are updated in place.  Both branches are uniform.
-template <bool IEEE = false>
+// OPS: the second moment as the device ops leave it, once: a bit per value (half_second_moment_ops)
+template <bool IEEE = false, bool OPS = false>
 __device__ __forceinline__ void half_elts8(v2h (&p)[kPairs], const v2h (&g)[kPairs], v2h (&m)[kPairs], v2h (&v)[kPairs],
-                                           const NfHyper &h, const MixConst &c)
+                                           const NfHyper &h, const MixConst &c, uint32_t once = 0)
 {
     if (fabsf(h.w1) < 0.5f) {
 #pragma unroll
@@ -178,7 +207,7 @@ __device__ __forceinline__ void half_elts8(v2h (&p)[kPairs], const v2h (&g)[kPai
     }
 #pragma unroll
     for (int j = 0; j < kPairs; ++j)
-        v[j] = half_second_moment(v[j], g[j], h, c);
+        v[j] = OPS ? half_second_moment_ops(v[j], g[j], h, c, once >> (2 * j)) : half_second_moment(v[j], g[j], h, c);
     // an eps that is positive as a half keeps every denominator positive: rounding is monotonic
     if (IEEE || h.eps > 0x1p-25f) {
 #pragma unroll

@@ -247,6 +247,8 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
 // ---------------------------------------------------------------------------------------
 constexpr int kHPlainMax = 64;
 
+static_assert(kHTile == kOpsBlock, "a tile is rounded one way");
+
 struct TensorHPlain {
     h16 *p;
     const h16 *g;
@@ -288,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void nonfused_half_plain_kernel(const Mul
         m[k >> 1][k & 1] = in ? t.m[i] : (h16)0.0f;
         v[k >> 1][k & 1] = in ? t.v[i] : (h16)0.0f;
     }
-    half_elts8<true>(p, g, m, v, h, mix_const());
+    half_elts8<true, true>(p, g, m, v, h, mix_const(), i0 - threadIdx.x + kHTile <= ops_twice(t.g, t.v, t.n) ? 0u : 0xffu);
 #pragma unroll
     for (int k = 0; k < kEltsPerLane; ++k) {
         const int64_t i = i0 + k * kThreads;

@@ -581,9 +581,22 @@ void lpmm_oracle_f32_to_f16(const float *f, uint16_t *h, int64_t n)
 
 static inline float rh(float x) { return h2f(f2h(x)); }
 
+/* rounds to half once: to an odd float first, which lies on its side of every tie between halfs */
+static inline float rh_once(double s)
+{
+    float f = (float)s;
+    uint32_t u;
+    if ((double)f == s || !isfinite(f))
+        return rh(f);
+    memcpy(&u, &f, 4);
+    u = (u - (fabs((double)f) > fabs(s) ? 1u : 0u)) | 1u;
+    memcpy(&f, &u, 4);
+    return rh(f);
+}
+
 void lpmm_oracle_nonfused_update_f16(uint16_t *p, const uint16_t *g, uint16_t *m, uint16_t *v, int64_t n,
                                      double beta1, double beta2, double lr, double weight_decay,
-                                     double eps, double step)
+                                     double eps, double step, int64_t twice)
 {
     const float decay = (float)(1.0 - lr * weight_decay);
     const float w1 = (float)(1.0 - beta1);
@@ -600,7 +613,14 @@ void lpmm_oracle_nonfused_update_f16(uint16_t *p, const uint16_t *g, uint16_t *m
         const float pi = rh(h2f(p[i]) * decay);            /* param.mul_(1 - lr * weight_decay) */
         const float mi = rh(lerp_small_w(h2f(m[i]), gi, w1)); /* exp_avg.lerp_(grad, 1 - beta1) */
         float vi = rh(h2f(v[i]) * b2);                      /* exp_avg_sq.mul_(beta2) */
-        vi = rh(vi + (w2 * gi) * gi);                       /* .addcmul_(grad, grad, value=1 - beta2) */
+        /* .addcmul_(grad, grad, value=1 - beta2); twice >= 0: v + value * (g * g) of PyTorch's GPU kernel, both ops
+         * rounded to float and to half in the first `twice` values, once to half behind them */
+        if (twice < 0)
+            vi = rh(vi + (w2 * gi) * gi);
+        else if (i < twice)
+            vi = rh(vi + w2 * (gi * gi));
+        else
+            vi = rh_once((double)rh_once((double)h2f(v[i]) * b2) + (double)w2 * ((double)gi * gi));
         float denom = rh(sqrtf(vi));                        /* exp_avg_sq.sqrt() */
         denom = rh(denom / bc2_sqrt);                       /* / bias_correction2_sqrt */
         denom = rh(denom + epsf);                           /* .add_(eps) */

@@ -87,7 +87,7 @@ _nonfused_update = _sig("lpmm_oracle_nonfused_update", None, _f32p, _f32p, _f32p
                         _d, _d, _d, _d, _d, _d)
 _u16p = np.ctypeslib.ndpointer(dtype=np.uint16, flags="C_CONTIGUOUS")
 _nonfused_update_f16 = _sig("lpmm_oracle_nonfused_update_f16", None, _u16p, _u16p, _u16p, _u16p, _i64,
-                            _d, _d, _d, _d, _d, _d)
+                            _d, _d, _d, _d, _d, _d, _i64)
 _adamw4bit_f16 = _sig("lpmm_oracle_adamw4bit_step_f16", None, _u16p, _u16p, _u8p, _u8p, _u16p, _u16p,
                       _f32p, _f32p, _i64, _f, _f, _f, _f, _f, _f)
 _f16_to_f32 = _sig("lpmm_oracle_f16_to_f32", None, _u16p, _f32p, _i64)
@@ -582,12 +582,15 @@ def f32_to_f16(x):
     return out.view(np.float16)
 
 
-def nonfused_update_f16(p, g, m, v, beta1, beta2, lr, wd, eps, step):
-    """Elementwise part of the step on float16 arrays, in place."""
+def nonfused_update_f16(p, g, m, v, beta1, beta2, lr, wd, eps, step, device_ops=False):
+    """Elementwise part of the step on float16 arrays, in place.  device_ops: addcmul_ as PyTorch's GPU kernel
+    rounds v + value * (g * g) for operands on 16-byte boundaries: to float and to half in whole blocks of 2048 values, to
+    half at once behind them."""
     for a in (p, g, m, v):
         assert a.dtype == np.float16 and a.flags.c_contiguous
     _nonfused_update_f16(p.reshape(-1).view(np.uint16), g.reshape(-1).view(np.uint16), m.reshape(-1).view(np.uint16),
-                         v.reshape(-1).view(np.uint16), p.size, beta1, beta2, lr, wd, eps, step)
+                         v.reshape(-1).view(np.uint16), p.size, beta1, beta2, lr, wd, eps, step,
+                         p.size // 2048 * 2048 if device_ops else -1)
 
 
 def _pack_padded(normed16, qmap):
@@ -634,7 +637,7 @@ def dequant_rank1_f16(codes, rowmax, colmax, qmap, r, c):
     return (vals * _rank1_scale_f16(rowmax, colmax)).astype(np.float16)
 
 
-def nonfused_step_f16(p, g, state, qm, qv, lr, beta1, beta2, eps, wd):
+def nonfused_step_f16(p, g, state, qm, qv, lr, beta1, beta2, eps, wd, device_ops=False):
     """One step of _single_tensor_adamw4bit on one quantised float16 tensor (4-bit states, first
     moment 'group' 128, second 'group' 128 or 'rank1' on a matrix).  p (float16) is updated in place;
     state is a NonFusedState whose scales and statistics are float16 arrays."""
@@ -653,7 +656,7 @@ def nonfused_step_f16(p, g, state, qm, qv, lr, beta1, beta2, eps, wd):
         v = dequant_group_f16(state.v[0], state.v[1], qv, n)
     m, v = np.ascontiguousarray(m), np.ascontiguousarray(v)
     nonfused_update_f16(p.reshape(-1), np.ascontiguousarray(g).reshape(-1), m, v, beta1, beta2, lr, wd, eps,
-                        float(state.step))
+                        float(state.step), device_ops)
     state.m = quant_group_f16(m, qm)
     if rank1:
         v2 = v.reshape(state.shape)

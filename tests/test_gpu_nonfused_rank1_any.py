@@ -46,7 +46,7 @@ def _setup(kind, shapes, rng):
 
 def _oracle_step(oracle, kind, h, g, state, qm, qv):
     if kind == "half":
-        oracle.nonfused_step_f16(h, g, state, qm, qv, H["lr"], 0.9, 0.999, H["eps"], H["weight_decay"])
+        oracle.nonfused_step_f16(h, g, state, qm, qv, H["lr"], 0.9, 0.999, H["eps"], H["weight_decay"], device_ops=True)
     elif kind == "float_m":
         state.step += 1
         r, c = h.shape
@@ -155,10 +155,37 @@ def test_half_states_that_are_not_quantised(oracle, eps):
             if h.size == 1:  # a one-element state counts as not created yet, on every step
                 m[:], v[:] = 0, 0
             with np.errstate(all="ignore"):
-                oracle.nonfused_update_f16(h, g, m, v, 0.9, 0.999, hyper["lr"], hyper["weight_decay"], eps, float(step))
+                oracle.nonfused_update_f16(h, g, m, v, 0.9, 0.999, hyper["lr"], hyper["weight_decay"], eps, float(step), device_ops=True)
             _same(to_np(p.detach()), h, f"step {step} tensor {i}: p")
             _same(to_np(opt.state[p]["exp_avg"]), m, f"step {step} tensor {i}: m")
             _same(to_np(opt.state[p]["exp_avg_sq"]), v, f"step {step} tensor {i}: v")
+
+
+@pytest.mark.parametrize("offset", [0, 1, 8])
+@pytest.mark.parametrize("shape", [(300,), (2048,), (4095,), (70, 61), (64, 66), (33, 1000)])
+def test_half_second_moment_at_ties(shape, offset):
+    """Gradients whose square times 1 - beta2 lies half way between two halfs (odd multiples of 200 * 2^-14): the kernels
+    round as the PyTorch ops on the device do, in whole blocks of 2048 values, behind them and off 16-byte boundaries."""
+    import lpmm
+
+    n = int(np.prod(shape))
+    p = torch.nn.Parameter(to_dev(np.zeros(shape, np.float16)))
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    opt = lpmm.optim.AdamW([p], fused=False, qconfig=path, **H)
+    v = torch.zeros(shape, dtype=torch.float16, device="cuda")
+    for step in range(3):
+        g = np.zeros(offset + n, np.float16)
+        g[offset:] = 200.0 * (1 + (np.arange(n) + 3 * step) % 10) * 2.0 ** -14
+        p.grad = to_dev(g)[offset:].view(shape)
+        opt.step()
+        v.mul_(0.999).addcmul_(p.grad, p.grad, value=1 - 0.999)
+        if len(shape) == 1:
+            _same(to_np(opt.state[p]["exp_avg_sq"]), to_np(v), f"step {step}: second moment")
+        else:
+            rows, cols = opt.state[p]["exp_avg_sq_qstate"]["overhead"]["max_dims"]
+            _same(to_np(rows), to_np(v.amax(1)), "row statistics")
+            _same(to_np(cols), to_np(v.amax(0)), "column statistics")
+            break  # the next second moment starts from the codes
 
 
 def test_tensors_of_more_dimensions(oracle, qmaps):
