@@ -47,6 +47,14 @@ __device__ __forceinline__ uint32_t row16_umax(uint32_t v)
 
 __device__ __forceinline__ uint32_t magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 
+// Larger of a maximum so far and |x|, as a bit pattern.  float: a NaN is left out, as by the quantisers' statistics
+// (one NaN gradient costs its own parameter and not its row); HALF: it is the maximum, as in the chain of half ops.
+template <bool HALF>
+__device__ __forceinline__ uint32_t larger(uint32_t top, float x)
+{
+    return HALF ? max(top, magnitude(x)) : __float_as_uint(fmaxf(__uint_as_float(top), fabsf(x)));
+}
+
 // A DPP row's piece of one tensor row: `count` values (1 .. 128) from flattened index `base` on; the values
 // from `split` on belong to the next group of the first moment.
 struct Piece {
@@ -300,32 +308,26 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             uint32_t vmax = 0u;
 #pragma unroll
             for (int k = 0; k < kAnyElts; ++k) {
-                vtop[k] = max(vtop[k], magnitude(v[k]));
-                vmax = max(vmax, magnitude(v[k]));
+                vtop[k] = larger<HALF>(vtop[k], v[k]);
+                vmax = larger<HALF>(vmax, v[k]);
             }
             vmax = row16_umax(vmax);
             if (!M32) {
-                // float: a NaN is left out, as by the block-wise quantiser; half: it is the maximum, as in torch's
-                float m0 = 0.0f, m1 = 0.0f;
+                uint32_t m0 = 0u, m1 = 0u;
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k) {
                     const bool here = piece_at(w, lane16, k) < w.split;
-                    if (HALF) {
-                        m0 = __uint_as_float(max(__float_as_uint(m0), here ? magnitude(m[k]) : 0u));
-                        m1 = __uint_as_float(max(__float_as_uint(m1), here ? 0u : magnitude(m[k])));
-                    } else {
-                        m0 = fmaxf(m0, here ? fabsf(m[k]) : 0.0f);
-                        m1 = fmaxf(m1, here ? 0.0f : fabsf(m[k]));
-                    }
+                    m0 = larger<HALF>(m0, here ? m[k] : 0.0f);
+                    m1 = larger<HALF>(m1, here ? 0.0f : m[k]);
                 }
-                m0 = __uint_as_float(row16_umax(__float_as_uint(m0)));
-                m1 = __uint_as_float(row16_umax(__float_as_uint(m1)));
+                m0 = row16_umax(m0);
+                m1 = row16_umax(m1);
                 if (lane16 == 0) {
                     // zero changes nothing: the next scales start there
-                    if (__float_as_uint(m0) != 0u)
-                        atomic_max_nonneg(t.ms_new + w.group, m0);
-                    if (__float_as_uint(m1) != 0u)
-                        atomic_max_nonneg(t.ms_new + w.group + 1, m1);
+                    if (m0 != 0u)
+                        atomic_max_nonneg(t.ms_new + w.group, __uint_as_float(m0));
+                    if (m1 != 0u)
+                        atomic_max_nonneg(t.ms_new + w.group + 1, __uint_as_float(m1));
                 }
             }
             if (lane16 == 0) {

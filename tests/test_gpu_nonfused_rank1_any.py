@@ -129,6 +129,63 @@ def test_half_infinities_and_nans(oracle, qmaps):
             _check("half", opt, p, h, None, st, f"step {step} tensor {i}")
 
 
+class _NoWalk:
+    """lpmm._native with a walk that serves nothing."""
+
+    def __init__(self, native):
+        self._native = native
+
+    def __getattr__(self, name):
+        return getattr(self._native, name)
+
+    def walk(self):
+        return self
+
+    def collect(self, *args):
+        return self._native.walk().collect(*args[:7], False, *args[8:])
+
+
+def _tensors(opt, p):
+    out = [p.detach()]
+    for name in ("exp_avg", "exp_avg_sq"):
+        out.append(opt.state[p][name])
+        oh = opt.state[p][name + "_qstate"]["overhead"]
+        out += ([oh["max1"]] if oh.get("max1") is not None else []) + list(oh.get("max_dims", ()))
+    return [to_np(t) for t in out]
+
+
+@pytest.mark.parametrize("kind", ["codes4", "float_m", "codes5", "codes8"])
+def test_a_nan_gradient_costs_its_own_parameter(kind, monkeypatch):
+    """One NaN gradient: parameters, statistics, scales and codes of the step after it and of two more are those of the
+    staged route (dequantise, update, quantise), and every other parameter stays finite.  (Of more than two dimensions only
+    the latter: the staged route's statistics keep a NaN there, and lose whole slices to it.)"""
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    shapes = [(70, 61), (33, 129), (40, 257)] + [(24, 10, 5, 5)] * (kind == "codes4")
+    (_, params, opt), (_, staged_params, staged) = (_setup(kind, shapes, np.random.default_rng(94)) for _ in range(2))
+    rng = np.random.default_rng(95)
+    for step in range(4):
+        grads = [(rng.standard_normal(s) * 0.1).astype(np.float32) for s in shapes]
+        if step == 1:
+            for g, at in zip(grads, (1250, 773, 0, 3001)):
+                g.reshape(-1)[at] = np.nan
+        for p, q, g in zip(params, staged_params, grads):
+            p.grad, q.grad = to_dev(g), to_dev(g)
+        opt.step()
+        with monkeypatch.context() as patch:
+            patch.setattr(adamw, "_any_columns", lambda rows, cols: False)
+            patch.setattr(adamw, "_native", _NoWalk(_native))
+            staged.step()
+        torch.cuda.synchronize()
+        for i, (p, q) in enumerate(zip(params, staged_params)):
+            assert int(p.isnan().sum()) == (step > 0), f"step {step} tensor {i}"
+            if p.dim() > 2:
+                continue
+            for j, (got, want) in enumerate(zip(_tensors(opt, p), _tensors(staged, q))):
+                _same(got, want, f"step {step} tensor {i}, {j}")
+
+
 @pytest.mark.parametrize("eps", [1e-3, 1e-8])
 def test_half_states_that_are_not_quantised(oracle, eps):
     """lpmm_nonfused_update_f16_multi: sizes around the 2048-value tiles, odd offsets, more tensors than one launch; a
