@@ -50,6 +50,16 @@ struct Item {
     float *step = nullptr;
     Swap swap[8];
     int swaps = 0;
+    // what the record points into: between collect() and the launch runs the loop over the other tensors, and with it
+    // code of the caller's (a gradient that is a property), which may drop gradients or states
+    std::vector<at::Tensor> kept;
+
+    template <typename T = void>
+    T *use(const at::Tensor &t)
+    {
+        kept.push_back(t);
+        return static_cast<T *>(t.unsafeGetTensorImpl()->mutable_data());
+    }
 };
 
 struct Batch {
@@ -65,7 +75,7 @@ struct Plan {
     PyObject_HEAD
     std::vector<Batch> *batches;
     std::vector<at::Tensor> *scratch;
-    std::vector<PyObject *> *held;  // what the records point into: kept until the step is over
+    std::vector<PyObject *> *held;  // the maps and the new objects of the swaps: kept until the step is over
     PyObject *rest;
 };
 
@@ -133,7 +143,7 @@ struct Walk {
     }
     // one tensor per dimension
     template <typename T>
-    static bool statistics(PyObject *list, const at::Tensor &p, T **out)
+    static bool statistics(Item &item, PyObject *list, const at::Tensor &p, T **out)
     {
         if (list == nullptr || !PyList_Check(list) || PyList_GET_SIZE(list) != p.dim())
             return false;
@@ -141,7 +151,7 @@ struct Walk {
             const at::Tensor *t = reals_of(PyList_GET_ITEM(list, i), p, p.size(i));
             if (t == nullptr)
                 return false;
-            out[i] = ptr<T>(*t);
+            out[i] = item.use<T>(*t);
         }
         return true;
     }
@@ -171,15 +181,27 @@ struct Walk {
         to.insert(to.end(), r, r + sizeof(R));
     }
     template <typename R>
-    void add(Batch &b, const R &record, const Item &item)
+    void add(Batch &b, const R &record, Item &item)
     {
         append(b.records, record);
-        b.items.push_back(item);
-        for (int i = 0; i < item.swaps; ++i) {
-            Py_INCREF(item.swap[i].dict);
-            Py_INCREF(item.swap[i].key);
-            Py_INCREF(item.swap[i].value);
+        b.items.push_back(std::move(item));
+        const Item &own = b.items.back();
+        for (int i = 0; i < own.swaps; ++i) {
+            Py_INCREF(own.swap[i].dict);
+            Py_INCREF(own.swap[i].key);
+            Py_INCREF(own.swap[i].value);
         }
+    }
+    // an item for a parameter with its gradient
+    static Item item_of(const at::Tensor &p, const at::Tensor &g, const at::Tensor *step)
+    {
+        Item item;
+        item.kept.reserve(12);
+        item.kept.push_back(p);
+        item.kept.push_back(g);
+        if (step != nullptr)
+            item.step = item.use<float>(*step);
+        return item;
     }
 
     int enabled(PyObject *p, PyObject *qstate)  // -1: not decided here
@@ -247,14 +269,13 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
     if (en_m < 0 || en_v < 0)
         return false;
-    Item item;
-    item.step = ptr<float>(*step);
+    Item item = item_of(p, g, step);
     const int64_t n = p.numel();
     if (!en_m && !en_v) {
         const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
         if (m == nullptr || v == nullptr)
             return false;
-        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<float>(*v), n, 0.0f, 0.0f};
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<float>(*v), n, 0.0f, 0.0f};
         add(batch(kPlain, p, nullptr, nullptr), r, item);
         return true;
     }
@@ -272,7 +293,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
             const at::Tensor *m = reals_like(mo, p);
             if (s.fused || m == nullptr)
                 return false;
-            lpmm_adamw_v4bit_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<uint8_t>(*vc), ptr<float>(*vs), n, 0.0f, 0.0f};
+            lpmm_adamw_v4bit_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<uint8_t>(*vc), item.use<float>(*vs), n, 0.0f, 0.0f};
             add(batch(kFlatM32, p, nullptr, qv), r, item);
             return true;
         }
@@ -283,10 +304,10 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         memset(&r, 0, sizeof r);
         r.p = ptr<float>(p);
         r.g = ptr<float>(g);
-        r.m_codes = ptr<uint8_t>(*mc);
-        r.v_codes = ptr<uint8_t>(*vc);
-        r.m_scale = ptr<float>(*ms);
-        r.v_scale = ptr<float>(*vs);
+        r.m_codes = item.use<uint8_t>(*mc);
+        r.v_codes = item.use<uint8_t>(*vc);
+        r.m_scale = item.use<float>(*ms);
+        r.v_scale = item.use<float>(*vs);
         r.n = n;
         add(batch(s.fused ? kFused4 : kFlat, p, qm, qv), r, item);
         return true;
@@ -299,7 +320,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     memset(&r, 0, sizeof r);
     r.p = ptr<float>(p);
     r.g = ptr<float>(g);
-    r.v_codes = ptr<uint8_t>(*vc);
+    r.v_codes = item.use<uint8_t>(*vc);
     r.rows = p.size(0);
     r.cols = n / r.rows;
     const at::Tensor *mc = nullptr, *ms = nullptr;
@@ -308,8 +329,8 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
         if (mc == nullptr || ms == nullptr)
             return false;
-        r.m_codes = ptr<uint8_t>(*mc);
-        r.m_max1 = ptr<float>(*ms);
+        r.m_codes = item.use<uint8_t>(*mc);
+        r.m_max1 = item.use<float>(*ms);
     }
     const bool whole = r.cols % 128 == 0, folds = r.cols % 128 == 64 && r.rows % 2 == 0;
     const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
@@ -318,7 +339,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
                nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, *vc, oh_v, qm, qv);
     PyObject *nxt = get(spare_stats, po);
     float *now[2], *next[2];
-    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
+    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next))
         return false;
     r.v_rowmax = now[0];
     r.v_colmax = now[1];
@@ -336,7 +357,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         }
         if (!aligned16(ptr(*m)))
             return false;
-        lpmm_rank1_v4bit_tensor f = {r.p, r.g, ptr<float>(*m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
+        lpmm_rank1_v4bit_tensor f = {r.p, r.g, item.use<float>(*m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
                                      r.rows, r.cols, 0.0f, 0.0f};
         add(batch(kRank1M32, p, nullptr, qv), f, item);
         return true;
@@ -362,7 +383,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const at::Tensor *ms_next = reals_of(spare, p, ms->numel());
     if (!((s.m_wide && whole) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
         return false;
-    lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        ptr<float>(*ms_next), r.v_codes, r.v_rowmax,
+    lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        item.use<float>(*ms_next), r.v_codes, r.v_rowmax,
                                   r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
     swap_later(item, spare_scales, po, get(oh_m, N.max1));
     swap_later(item, oh_m, N.max1, spare);
@@ -377,14 +398,14 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *spare = get(spare_scales, po);
     void *now[2], *next[2];
     const at::Tensor *ms_next = ms != nullptr ? reals_of(spare, p, ms->numel()) : nullptr;
-    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || (ms != nullptr && ms_next == nullptr))
+    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next) || (ms != nullptr && ms_next == nullptr))
         return false;
     lpmm_rank1_any_tensor r;
     memset(&r, 0, sizeof r);
     r.p = ptr(p);
     r.g = ptr(g);
-    r.m = ptr(*mc);
-    r.v_codes = ptr<uint8_t>(vc);
+    r.m = item.use(*mc);
+    r.v_codes = item.use<uint8_t>(vc);
     r.v_rowmax = now[0];
     r.v_colmax = now[1];
     r.v_rowmax_next = next[0];
@@ -397,8 +418,8 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     swap_later(item, oh_v, N.max_dims, nxt);
     r.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
     if (ms != nullptr) {
-        r.m_max1 = ptr(*ms);
-        r.m_max1_next = ptr(*ms_next);
+        r.m_max1 = item.use(*ms);
+        r.m_max1_next = item.use(*ms_next);
         r.m_codes_next = next_codes(item, st, N.exp_avg, *mc);
         swap_later(item, spare_scales, po, get(oh_m, N.max1));
         swap_later(item, oh_m, N.max1, spare);
@@ -419,27 +440,26 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
     const int en = enabled(po, qs);
     if (en < 0 || row == nullptr || col == nullptr || map == nullptr || !floats(*map))
         return false;
-    Item item;
-    item.step = ptr<float>(step);
+    Item item = item_of(p, g, &step);
     lpmm_factored_tensor r;
     memset(&r, 0, sizeof r);
     r.p = ptr<float>(p);
     r.g = ptr<float>(g);
-    r.row = ptr<float>(*row);
-    r.col = ptr<float>(*col);
+    r.row = item.use<float>(*row);
+    r.col = item.use<float>(*col);
     r.rows = rows;
     r.cols = cols;
     if (en) {
         const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *ms = scales(qs, &oh, p, (n + 127) / 128);
         if (!s.m_group128 || mc == nullptr || ms == nullptr)
             return false;
-        r.m_codes = ptr<uint8_t>(*mc);
-        r.m_max1 = ptr<float>(*ms);
+        r.m_codes = item.use<uint8_t>(*mc);
+        r.m_max1 = item.use<float>(*ms);
     } else {
         const at::Tensor *m = reals_like(mo, p);
         if (m == nullptr)
             return false;
-        r.m_codes = ptr<uint8_t>(*m);
+        r.m_codes = item.use<uint8_t>(*m);
     }
     r.workspace = scratch(p, (workspace_bytes(rows, cols) + 3) / 4);
     add(batch(en && cols % 128 == 0 ? kFactored : kFactoredAny, p, qm, nullptr), r, item);
@@ -453,13 +473,12 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
     PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
     const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
     const int64_t n = p.numel(), groups = (n + 127) / 128;
-    Item item;
-    item.step = ptr<float>(step);
+    Item item = item_of(p, g, &step);
     if (en_m == 0 && en_v == 0) {
         const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
         if (m == nullptr || v == nullptr || m->sizes() != p.sizes() || v->sizes() != p.sizes())
             return false;
-        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*m), ptr<float>(*v), n, 0.0f, 0.0f};
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<float>(*v), n, 0.0f, 0.0f};
         add(batch(kHalfPlain, p, nullptr, nullptr), r, item);
         return true;
     }
@@ -474,7 +493,7 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
         const at::Tensor *vs = scales(qs_v, &oh_v, p, groups);
         if (vs == nullptr)
             return false;
-        lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), ptr<uint8_t>(*mc), ptr<uint8_t>(*vc), ptr(*ms), ptr(*vs), n, 0.0f, 0.0f};
+        lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), item.use<uint8_t>(*mc), item.use<uint8_t>(*vc), item.use(*ms), item.use(*vs), n, 0.0f, 0.0f};
         add(batch(kHalfFlat, p, qm, qv), r, item);
         return true;
     }
@@ -485,11 +504,11 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
         return (cols >= 32 || rows <= 32768) && any(po, p, g, st, item, LPMM_RANK1_HALF, mc, ms, *vc, oh_m, oh_v, qm, qv);
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po);
     void *now[2], *next[2];
-    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
+    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next))
         return false;
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
-    lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), ptr<uint8_t>(*mc), ptr(*ms), ptr<uint8_t>(*vc), now[0], now[1], next[0], next[1],
+    lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), item.use<uint8_t>(*mc), item.use(*ms), item.use<uint8_t>(*vc), now[0], now[1], next[0], next[1],
                                         scratch(p, (rows + 3) / 4 * 4 + cols), rows, cols, 0.0f, 0.0f};
     add(batch(kHalfRank1, p, qm, qv), r, item);
     return true;
@@ -507,7 +526,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     PyObject *row = get(scratch, N.row);
     const at::Tensor *work = reals_of(get(scratch, N.work), p, 3 * r.cols);
     float *now[LPMM_RANK1_ND_MAX], *next[LPMM_RANK1_ND_MAX];
-    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
+    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
         return false;
     const long old_row = PyLong_AsLong(row);
     if (old_row < 0 || old_row > 2)
@@ -523,7 +542,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     }
     if (slots > 8192)
         return false;
-    float *const rows = ptr<float>(*work);
+    float *const rows = item.use<float>(*work);
     fold.ndim = dims - 1;
     fold.x = rows + raw_row * r.cols;
     fold.scale = rows + new_row * r.cols;
@@ -552,7 +571,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         b.fold.push_back(fold);
         return true;
     }
-    lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, ptr(*ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
+    lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, item.use(*ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
                                r.v_rowmax_next, r.v_colmax_next, nullptr, r.rows, r.cols, 0.0f, 0.0f};
     w.m_codes_next = next_codes(item, st, N.exp_avg, *any_mc);
     w.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
@@ -571,6 +590,7 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     if (!g.defined() || !floats(p) || !floats(g) || p.device() != g.device() || p.numel() != g.numel())
         return false;
     PyObject *qs = get(st, N.momentum_buffer_qstate), *bo = get(st, N.momentum_buffer);
+    Item item = item_of(p, g, nullptr);
     const int en = enabled(po, qs);
     if (en < 0)
         return false;
@@ -578,16 +598,16 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
         const at::Tensor *buf = reals_like(bo, p);
         if (buf == nullptr || buf->sizes() != p.sizes())
             return false;
-        lpmm_sgd_fp32_tensor r = {ptr<float>(p), ptr<float>(g), ptr<float>(*buf), p.numel(), 0, 0};
-        add(batch(kSgdPlain, p, nullptr, nullptr), r, Item());
+        lpmm_sgd_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*buf), p.numel(), 0, 0};
+        add(batch(kSgdPlain, p, nullptr, nullptr), r, item);
         return true;
     }
     PyObject *oh = nullptr, *qm = get(qs, N.qmap);
     const at::Tensor *map = tensor_of(qm), *mc = codes(bo, p, (p.numel() + 1) / 2), *ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
     if (!s.m_group128 || map == nullptr || !floats(*map) || mc == nullptr || ms == nullptr)
         return false;
-    lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), ptr<uint8_t>(*mc), ptr<float>(*ms), p.numel(), 0, 0};
-    add(batch(kSgd4, p, qm, nullptr), r, Item());
+    lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), item.use<uint8_t>(*mc), item.use<float>(*ms), p.numel(), 0, 0};
+    add(batch(kSgd4, p, qm, nullptr), r, item);
     return true;
 }
 

@@ -155,3 +155,50 @@ def test_walk_leaves_overridden_and_subclassed_parameters_to_the_loops():
     assert [p is m.c for p in plan.rest] == [True]
     kinds = {batch[0]: batch[5] for batch in plan.start()}
     assert kinds == {_native.WALK_FUSED4: 1, _native.WALK_PLAIN: 1}
+
+
+@pytest.mark.parametrize("case", ["fused", "default", "half", "sgd"])
+def test_tensors_dropped_during_the_step_outlive_it(case):
+    """The .grad of a Parameter's subclass is the caller's code and runs after the walk: it may drop gradients and states
+    that the walk's records point into, and allocate over them."""
+    import lpmm
+
+    rng = np.random.default_rng(8)
+    drop = []
+
+    class Own(torch.nn.Parameter):
+        @property
+        def grad(self):
+            for p, state in drop:
+                shapes = [t.shape for t in (p.grad, *state.values()) if torch.is_tensor(t) and t.is_cuda]
+                p.grad = None
+                state.clear()
+                junk.extend(torch.full(s, 3.0, device="cuda", dtype=p.dtype) for s in shapes for _ in range(3))
+            drop.clear()
+            return None
+
+    kw = dict(CASES[case])
+    dtype, sgd = kw.pop("dtype", torch.float32), kw.pop("sgd", False)
+    if "qconfig" in kw:
+        kw["qconfig"] = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", kw["qconfig"])
+    shapes = [(64, 128), (48, 192), (33, 130), (70,)]
+    host = [rng.standard_normal(s) for s in shapes]
+    results = []
+    for dropping in (False, True):
+        junk = []
+        params = [torch.nn.Parameter(torch.from_numpy(h).to(dtype).cuda()) for h in host]
+        own = Own(torch.zeros(4, device="cuda"))
+        opt = (lpmm.optim.SGD(params + [own], lr=1e-2, momentum=0.9) if sgd
+               else lpmm.optim.AdamW(params + [own], lr=1e-2, eps=1e-3, **kw))
+        grads = np.random.default_rng(9)
+        for step in range(3):
+            for p in params:
+                p.grad = torch.from_numpy(grads.standard_normal(p.shape)).to(dtype).cuda()
+            if dropping and step == 2:
+                drop.extend((p, opt.state[p]) for p in params)
+            opt.step()
+        torch.cuda.synchronize()
+        results.append([p.detach().clone() for p in params])
+    assert junk and not opt.state[params[0]].get("exp_avg_qstate")
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
