@@ -104,6 +104,15 @@ T *ptr(const at::Tensor &t)
     return static_cast<T *>(t.unsafeGetTensorImpl()->mutable_data());
 }
 
+// Bytes of a state's codes as the kernels write them: whole groups, rounded up to pack groups, and one more
+// (lpmm/functional.py: packed_nbytes).  The fused operators alone ask for no more than the values.
+int64_t packed(int64_t n, int64_t group, bool bytes)
+{
+    const int64_t scaled = (n + group - 1) / group * group;
+    const int64_t all = (scaled + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP;
+    return (bytes ? all : all / 2) + 1;
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 struct Settings {
@@ -281,7 +290,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     }
     PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap);
     const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
-    const at::Tensor *vc = codes(vo, p, s.bits_rank1 ? n : (n + 1) / 2);
+    const at::Tensor *vc = codes(vo, p, s.fused ? (n + 1) / 2 : packed(n, 128, s.bits_rank1));
     if (map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) || vc == nullptr || !en_v)
         return false;
     PyObject *oh_m = nullptr, *oh_v = nullptr;
@@ -297,7 +306,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
             add(batch(kFlatM32, p, nullptr, qv), r, item);
             return true;
         }
-        const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
+        const at::Tensor *mc = codes(mo, p, s.fused ? (n + 1) / 2 : packed(n, 128, false)), *ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
         if (!(s.fused ? n % 2 == 0 : s.m_group128 != 0) || mc == nullptr || ms == nullptr)
             return false;
         lpmm_adamw4bit_tensor r;
@@ -325,7 +334,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     r.cols = n / r.rows;
     const at::Tensor *mc = nullptr, *ms = nullptr;
     if (en_m) {
-        mc = codes(mo, p, s.bits_rank1 ? n : (n + 1) / 2);
+        mc = codes(mo, p, packed(n, s.m_group, s.bits_rank1));
         ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
         if (mc == nullptr || ms == nullptr)
             return false;
@@ -450,7 +459,7 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
     r.rows = rows;
     r.cols = cols;
     if (en) {
-        const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *ms = scales(qs, &oh, p, (n + 127) / 128);
+        const at::Tensor *mc = codes(mo, p, packed(n, 128, false)), *ms = scales(qs, &oh, p, (n + 127) / 128);
         if (!s.m_group128 || mc == nullptr || ms == nullptr)
             return false;
         r.m_codes = item.use<uint8_t>(*mc);
@@ -484,7 +493,7 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
     }
     PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap), *oh_m = nullptr, *oh_v = get(qs_v, N.overhead);
     const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
-    const at::Tensor *mc = codes(mo, p, (n + 1) / 2), *vc = codes(vo, p, (n + 1) / 2), *ms = scales(qs_m, &oh_m, p, groups);
+    const at::Tensor *mc = codes(mo, p, packed(n, 128, false)), *vc = codes(vo, p, packed(n, 128, false)), *ms = scales(qs_m, &oh_m, p, groups);
     PyObject *const half_type = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
     if (en_m != 1 || en_v != 1 || !s.m_group128 || map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) ||
         mc == nullptr || vc == nullptr || ms == nullptr || get(oh_m, N.dtype) != half_type || get(oh_v, N.dtype) != half_type)
@@ -603,7 +612,7 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
         return true;
     }
     PyObject *oh = nullptr, *qm = get(qs, N.qmap);
-    const at::Tensor *map = tensor_of(qm), *mc = codes(bo, p, (p.numel() + 1) / 2), *ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
+    const at::Tensor *map = tensor_of(qm), *mc = codes(bo, p, packed(p.numel(), 128, false)), *ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
     if (!s.m_group128 || map == nullptr || !floats(*map) || mc == nullptr || ms == nullptr)
         return false;
     lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), item.use<uint8_t>(*mc), item.use<float>(*ms), p.numel(), 0, 0};

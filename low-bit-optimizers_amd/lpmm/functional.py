@@ -246,6 +246,17 @@ def packed_nbytes(numel_scaled, b=4):
     return (numel_scaled + PACK_GROUP - 1) // PACK_GROUP * (PACK_GROUP * storage_bits(b) // 8) + 1
 
 
+def whole_codes(codes, nbytes):
+    """Codes in the layout the step kernels read and write in full.  A state may come without the padding: the fused
+    operators' layout is (numel + 1) // 2 bytes (lpmm/optim/adamw.py:508-523), and a step on it has to give what
+    it gives on the padded array."""
+    if codes.numel() >= nbytes:
+        return codes
+    out = codes.new_zeros(nbytes)
+    out[: codes.numel()] = codes.reshape(-1)
+    return out
+
+
 _CODE_TABLES = {}
 _CODE_TABLES_MAX = 64
 

@@ -23,7 +23,7 @@ import numpy as np
 import torch
 
 from .. import _native
-from ..functional import RANK1_ND_MAX, _ptr_array, _shape_array, code_table, packed_nbytes, vectorwise_dequant, vectorwise_quant
+from ..functional import RANK1_ND_MAX, _ptr_array, _shape_array, code_table, packed_nbytes, vectorwise_dequant, vectorwise_quant, whole_codes
 from .optimizer import LowBitOptimizer
 
 __all__ = ["AdamW"]
@@ -855,6 +855,7 @@ class AdamW(LowBitOptimizer):
                                      "max_dims": [torch.zeros((rows, 1), dtype=torch.float16, device=dev),
                                                   torch.zeros((1, cols), dtype=torch.float16, device=dev)],
                                      "scaled_shape": p.shape})
+        state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), 4))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
         nxt = self._spare_stats.get(p)
@@ -935,6 +936,7 @@ class AdamW(LowBitOptimizer):
                        "scaled_shape": torch.Size((groups, gp_sz))})
             if rank1_vector:  # the 'rank1' branch records the dimension count (lpmm/functional.py:191)
                 oh["dim"] = 1
+        state[name] = whole_codes(state[name], packed_nbytes(groups * gp_sz, b))
         return state[name].data_ptr(), qstate["overhead"]["max1"].data_ptr()
 
     def _group_state_pair(self, p, state, batch, gp_sz=128, b=4):
@@ -983,6 +985,7 @@ class AdamW(LowBitOptimizer):
                                      "max_dims": [torch.zeros((rows, 1), dtype=torch.float32, device=dev),
                                                   torch.zeros((1, cols), dtype=torch.float32, device=dev)],
                                      "scaled_shape": p.shape})
+        state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), b))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
         nxt = self._spare_stats.get(p)
@@ -1127,6 +1130,7 @@ class AdamW(LowBitOptimizer):
             qs_v["overhead"].clear()
             qs_v["overhead"].update({"dtype": p.dtype, "stride": self._state_stride(p), "dim": p.dim(), "max1": None,
                                      "max_dims": stats, "scaled_shape": p.shape})
+        state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), 4))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
         nxt = self._spare_stats.get(p)
@@ -1230,6 +1234,7 @@ class AdamW(LowBitOptimizer):
                     qstate["overhead"].update({"dtype": p.dtype, "stride": self._state_stride(p),
                                                "max1": torch.empty((groups, 1), dtype=torch.float32, device=p.device),
                                                "scaled_shape": torch.Size((groups, 128))})
+                state["exp_avg"] = whole_codes(state["exp_avg"], packed_nbytes(p.numel()))
                 m, ms = state["exp_avg"].data_ptr(), qstate["overhead"]["max1"].data_ptr()
             else:
                 kept.append(self._materialise(p, state, "exp_avg", False, md_m))
@@ -1281,6 +1286,7 @@ class AdamW(LowBitOptimizer):
                     state["exp_avg"] = torch.empty((packed_nbytes(groups * 128),), dtype=torch.int8, device=dev)
                     max1 = torch.empty((groups, 1), dtype=torch.float32, device=dev)
                 else:
+                    state["exp_avg"] = whole_codes(state["exp_avg"], packed_nbytes(p.numel()))
                     max1 = qstate["overhead"]["max1"]
                 st = lib.lpmm_factored_update(dense.data_ptr(), grad.data_ptr(), state["exp_avg"].data_ptr(),
                                               max1.data_ptr(), qstate["qmap"].data_ptr(), row.data_ptr(),

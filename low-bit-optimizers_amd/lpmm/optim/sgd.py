@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from .. import _native
-from ..functional import packed_nbytes, vectorwise_dequant, vectorwise_quant
+from ..functional import packed_nbytes, vectorwise_dequant, vectorwise_quant, whole_codes
 from .optimizer import LowBitOptimizer
 
 __all__ = ["SGD"]
@@ -107,6 +107,7 @@ class SGD(LowBitOptimizer):
                         qstate["overhead"].update({"dtype": p.dtype, "stride": p.stride(),
                                                    "max1": torch.empty((groups, 1), dtype=torch.float32, device=p.device),
                                                    "scaled_shape": torch.Size((groups, 128))})
+                    state["momentum_buffer"] = whole_codes(state["momentum_buffer"], packed_nbytes(p.numel()))
                     batched.setdefault((p.device, qstate["qmap"].data_ptr()), []).append(
                         (p.data_ptr(), p.grad.data_ptr(), state["momentum_buffer"].data_ptr(),
                          qstate["overhead"]["max1"].data_ptr(), p.numel(), 1 if first else 0, 0))

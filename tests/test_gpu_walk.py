@@ -202,3 +202,45 @@ def test_tensors_dropped_during_the_step_outlive_it(case):
     assert junk and not opt.state[params[0]].get("exp_avg_qstate")
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if not c.startswith("fused")] + ["factored"])
+def test_codes_without_their_padding(case, monkeypatch):
+    """States whose code arrays end with the values (the fused operators' layout): the walk leaves them to the loops, the
+    step completes them, and leaves what it leaves on the padded arrays."""
+    import lpmm.optim.adamw as adamw
+    import lpmm.optim.sgd as sgd
+    from lpmm import _native
+
+    monkeypatch.setitem(CASES, "factored", dict(factor_second_moment=True))
+    sides = [_build(case, np.random.default_rng(5)) for _ in range(2)]
+    rng = np.random.default_rng(7)
+    for step in range(4):
+        grads = [rng.standard_normal(p.shape) * 0.1 for p in sides[0][0]]
+        for side, (params, opt) in enumerate(sides):
+            for p, g in zip(params, grads):
+                p.grad = torch.from_numpy(g).to(p.dtype).cuda()
+            cut = 0
+            if step == 2 and side == 1:
+                for p in params:
+                    if p.dtype is torch.float16 and not p.is_contiguous():
+                        continue  # the chain of torch ops refuses short codes
+                    for k, v in opt.state[p].items():
+                        if torch.is_tensor(v) and v.dtype is torch.int8:
+                            bytes_ = p.numel() if case == "bits" else (p.numel() + 1) // 2
+                            opt.state[p][k], cut = v[:bytes_].clone(), cut + 1
+                native = _Native(_native, True)
+                with monkeypatch.context() as patch:
+                    patch.setattr(adamw, "_native", native)
+                    patch.setattr(sgd, "_native", native)
+                    opt.step()
+                assert 0 < cut <= 2 * native.rest
+            else:
+                opt.step()
+        torch.cuda.synchronize()
+        for i, (p, q) in enumerate(zip(sides[0][0], sides[1][0])):
+            assert torch.equal(p.detach(), q.detach()), (step, i)
+            a, b = _state(sides[0][1], p), _state(sides[1][1], q)
+            for k in a:
+                assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), \
+                    (step, i, k)
