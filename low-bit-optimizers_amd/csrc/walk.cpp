@@ -118,7 +118,7 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 struct Settings {
     int fused;  // 0: the non-fused path, 1: the fused operators, 2: settings the fused operators warn about or refuse
     int m_group128, v_group128, v_rank1, m_wide, bits_rank1;
-    int64_t m_group;
+    int64_t m_group;  // values per group of the first moment's scales; 0: scaled in a way that is not served here
 };
 
 struct Walk {
@@ -334,6 +334,8 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     r.cols = n / r.rows;
     const at::Tensor *mc = nullptr, *ms = nullptr;
     if (en_m) {
+        if (s.m_group <= 0)
+            return false;
         mc = codes(mo, p, packed(n, s.m_group, s.bits_rank1));
         ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
         if (mc == nullptr || ms == nullptr)

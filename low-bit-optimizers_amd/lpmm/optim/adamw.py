@@ -99,6 +99,8 @@ class _Routes:
         self.m_group_wide = fits(md_m) and m_group and md_m["gp_sz"] in (256, 512, 1024, 2048, 4096)
         self.bits_rank1 = (wide_codes(md_m) and m_group and md_m["gp_sz"] == 128
                            and wide_codes(md_v) and md_v["scale_type"] == "rank1")
+        # the group size as a number the walk may divide by; other scalings of the first moment may state any, or none
+        self.m_group = md_m["gp_sz"] if self.m_group128 or self.m_group_wide or self.bits_rank1 else 0
         # the fused operator: 4-bit states; other settings go on with a warning or an error
         self.fused4 = md_m["b"] == 4 and md_v["b"] == 4 and m_group and v_group
 
@@ -244,7 +246,8 @@ class AdamW(LowBitOptimizer):
         return _native.walk().collect(
             0, group["params"], self.state, self.override_q_enable, self._spare_stats, self._spare_scales, self._nd_scratch,
             True,
-            (0 if not fused else 1 if routes.fused4 else 2, routes.m_group128, routes.v_group128, routes.v_rank1, routes.m_group_wide, routes.bits_rank1, routes.m["gp_sz"]),
+            (0 if not fused else 1 if routes.fused4 else 2, routes.m_group128, routes.v_group128, routes.v_rank1,
+             routes.m_group_wide, routes.bits_rank1, routes.m_group),
             _native.factored_workspace())
 
     def _launch_walk(self, group, plan, routes):

@@ -244,3 +244,18 @@ def test_codes_without_their_padding(case, monkeypatch):
             for k in a:
                 assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), \
                     (step, i, k)
+
+
+def test_rank1_scales_without_a_group_size():
+    """Rank-1 scales for both moments and a group size of zero: the staged route, on every step."""
+    import lpmm
+
+    p = torch.nn.Parameter(torch.ones(70, 61, device="cuda"))
+    opt = lpmm.optim.AdamW([p], lr=1e-2, qconfig=dict(QUANT=dict(M=dict(SCALE_TYPE=dict(DEFAULT="rank1"), GROUP_SIZE=0),
+                                                                SQM=dict(SCALE_TYPE=dict(DEFAULT="rank1")))))
+    for _ in range(3):
+        p.grad = torch.ones_like(p)
+        opt.step()
+    # a constant gradient moves every value by lr a step, weight decay by lr * 0.01 at most
+    assert torch.allclose(p, torch.full_like(p, 1 - 3e-2), atol=4e-4)
+    assert len(opt.state[p]["exp_avg_qstate"]["overhead"]["max_dims"]) == 2

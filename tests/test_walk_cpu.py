@@ -1,6 +1,10 @@
 """The host walk (csrc/walk.cpp) where no GPU is needed."""
 import struct
 
+import pytest
+import torch
+
+import lpmm
 from lpmm import _native
 
 
@@ -20,3 +24,13 @@ def test_the_module_has_no_thread_local_storage():
     process, torch's own among them."""
     types = _program_header_types(_native.walk().__file__)
     assert 1 in types and 7 not in types  # PT_LOAD, PT_TLS
+
+
+@pytest.mark.parametrize("group_size", [None, 0, 1 << 40])
+def test_a_group_size_that_nothing_reads(group_size):
+    """Rank-1 scales for both moments: the group size is not read, and may be anything."""
+    p = torch.nn.Parameter(torch.zeros(70, 61))
+    opt = lpmm.optim.AdamW([p], qconfig=dict(QUANT=dict(M=dict(SCALE_TYPE=dict(DEFAULT="rank1"), GROUP_SIZE=group_size),
+                                                        SQM=dict(SCALE_TYPE=dict(DEFAULT="rank1")))))
+    assert opt.step() is None
+    assert lpmm.optim.adamw._Routes(*map(opt.get_qmetadata_by_state_name, ("exp_avg", "exp_avg_sq"))).m_group == 0
