@@ -15,11 +15,12 @@
 //     second), as in the ragged kernels;
 //   * the new codes go to arrays of their own, as on the staged path (the state's tensors are replaced); two codes
 //     that share a byte may belong to neighbouring lanes (they meet by a lane exchange) or, where the column
-//     count is odd, to different rows: the first pass clears such a byte, the second sets its halves by atomic or.
+//     count is odd, to different rows: the first pass clears the word around such a byte, the second sets the word's codes
+//     by atomic or (store_nibbles).
 // Before, these tensors took the staged path (dequantise, update, statistics, normalise: six to eight
 // launches a tensor and 50 bytes a value; float16: about thirty PyTorch ops a tensor).  One step on one tensor,
 // staged -> here: 4096 x 4100 default 224 -> 107 us, fp32 first moment 183 -> 104, 8 bits 221 -> 102, float16
-// 539 -> 151; 4095 x 4099 271 -> 159; 50000 x 34 122 -> 55 (4096 x 4096 on the tuned kernels: 74-84, float16 67).
+// 539 -> 151; 4095 x 4099 271 -> 142; 50000 x 34 122 -> 55 (4096 x 4096 on the tuned kernels: 74-84, float16 67).
 // What bounds them: instructions, the code bytes' extraction and one access per value (the tuned kernels move
 // the same bytes in a quarter of the accesses); most of the gain on small tensors is launches.
 #include "lpmm_half.hpp"
@@ -33,6 +34,15 @@ template <int CTRL>
 __device__ __forceinline__ uint32_t any_dpp(uint32_t v)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
+
+__device__ __forceinline__ uint32_t row16_or(uint32_t v)
+{
+    v |= any_dpp<0xB1>(v);
+    v |= any_dpp<0x4E>(v);
+    v |= any_dpp<0x141>(v);
+    v |= any_dpp<0x140>(v);
+    return v;
 }
 
 // largest of the DPP row's bit patterns, in every lane
@@ -115,48 +125,59 @@ __device__ __forceinline__ uint64_t load_codes(const uint8_t *codes, const Piece
     return out;
 }
 
-// sets one half of a cleared byte; the array is 4-byte aligned and whole words long up to the byte
-__device__ __forceinline__ void set_nibble(uint8_t *at, uint32_t shift, uint32_t code)
-{
-    const uintptr_t a = reinterpret_cast<uintptr_t>(at);
-    atomicOr(reinterpret_cast<uint32_t *>(a & ~(uintptr_t)3), code << (8 * (uint32_t)(a & 3) + shift));
-}
+// Two codes share a byte, and where the column count is odd the two may belong to different rows, which different
+// workgroups write.  An atomic or covers four bytes, so it is the whole word around such a byte that is put together
+// this way: in an odd matrix the first pass clears every word that a piece does not fill by itself, the second sets
+// the piece's codes of either such word with one atomic, and plain byte stores go only to words that lie wholly
+// inside one piece.  No byte is written both ways, and no word by stores of one size while another workgroup
+// writes it with the other.  (An atomic per shared byte beside plain stores into the same words took 155 us for
+// 4095 x 4099, this 142.)
+__device__ __forceinline__ uint32_t *word_of(uint8_t *codes, int64_t flat) { return reinterpret_cast<uint32_t *>(codes) + (flat >> 3); }
 
-// the bytes that a piece shares with its neighbours
+// the words that a piece of an odd matrix shares with its neighbours
 __device__ __forceinline__ void clear_shared(uint8_t *codes, const Piece &w)
 {
     const int64_t end = w.base + w.count;
-    if (w.base & 1)
-        codes[w.base >> 1] = 0;
-    if (end & 1)
-        codes[end >> 1] = 0;
+    if (w.base & 7)
+        *word_of(codes, w.base) = 0u;
+    if (end & 7)
+        *word_of(codes, end) = 0u;
 }
 
-__device__ __forceinline__ void store_nibbles(uint8_t *codes, const Piece &w, int lane16, uint32_t now)
+__device__ __forceinline__ void store_nibbles(uint8_t *codes, const Piece &w, int lane16, uint32_t now, bool odd_cols)
 {
     uint8_t *c = codes + (w.base >> 1);
     const int odd = (int)(w.base & 1);
     const bool low = ((lane16 + odd) & 1) == 0;  // the lane's codes are low halves of their bytes
+    // the piece's values in words of its own; an even matrix has no shared bytes
+    const int first = odd_cols ? (int)(-w.base & 7) : 0, end = odd_cols ? w.count - (int)((w.base + w.count) & 7) : w.count;
     // the codes one column on: lane 15's are lane 0's of the next sixteen columns
     const int lane = threadIdx.x & (kWave - 1);
     uint32_t next = (uint32_t)__shfl((int)now, (lane & ~15) | ((lane + 1) & 15), kWave);
     if (lane16 == 15)
         next >>= 4;
+    if (low) {
+        uint8_t *at = c + ((lane16 + odd) >> 1);
 #pragma unroll
-    for (int k = 0; k < kAnyElts; ++k) {
-        const int off = 16 * k + lane16;
-        if (off >= w.count)
-            continue;
-        const uint32_t a = (now >> (4 * k)) & 15u;
-        uint8_t *at = c + ((off + odd) >> 1);
-        if (low) {
-            if (off + 1 < w.count)
-                *at = (uint8_t)(a | (((next >> (4 * k)) & 15u) << 4));
-            else
-                set_nibble(at, 0, a);  // the other half belongs to the next block, row or the padding
-        } else if (off == 0) {
-            set_nibble(at, 4, a);
+        for (int k = 0; k < kAnyElts; ++k) {
+            const int off = 16 * k + lane16;
+            if (off >= first && off < end)
+                at[8 * k] = (uint8_t)(((now >> (4 * k)) & 15u) | (((next >> (4 * k)) & 15u) << 4));
         }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (!odd_cols)
+        return;
+    // at most seven values at either end: a lane has at most its first one there and its last one here
+    const int k = (w.count - 1 - lane16) >> 4, off = 16 * k + lane16;
+    const uint32_t head = lane16 < first && lane16 < w.count ? (now & 15u) << (4 * ((int)(w.base + lane16) & 7)) : 0u;
+    const uint32_t tail = off >= end && off >= first ? ((now >> (4 * (k & 7))) & 15u) << (4 * ((int)(w.base + off) & 7)) : 0u;
+    const uint32_t heads = row16_or(head), tails = row16_or(tail);
+    if (lane16 == 0) {
+        if (heads != 0u)
+            atomicOr(word_of(codes, w.base), heads);
+        if (tails != 0u)
+            atomicOr(word_of(codes, w.base + w.count - 1), tails);
     }
 }
 
@@ -174,7 +195,7 @@ __device__ __forceinline__ void store_bytes(uint8_t *codes, const Piece &w, int 
 // The codes behind the tensor's n values: `last` up to n_group (the zeros that complete a group are divided by
 // its scale like its other values), `zero` up to whole pack groups, 0 in the extra byte.  One workgroup.
 template <bool BITS>
-__device__ __forceinline__ void any_padding(uint8_t *codes, int64_t n, int64_t n_group, uint32_t last, uint32_t zero)
+__device__ __forceinline__ void any_padding(uint8_t *codes, int64_t n, int64_t n_group, uint32_t last, uint32_t zero, bool odd_cols)
 {
     const int64_t n_all = (n_group + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP;
     if (BITS) {
@@ -184,9 +205,11 @@ __device__ __forceinline__ void any_padding(uint8_t *codes, int64_t n, int64_t n
             codes[n_all] = 0;
         return;
     }
-    if ((n & 1) != 0 && threadIdx.x == 0)
-        set_nibble(codes + (n >> 1), 4, n < n_group ? last : zero);
-    for (int64_t i = (n + 1) / 2 + threadIdx.x; i < n_all / 2; i += kThreads)
+    // the rest of the last value's word goes the word's way
+    const int64_t from = odd_cols ? (n + 7) & ~(int64_t)7 : n;
+    if (n + threadIdx.x < from)
+        atomicOr(word_of(codes, n), (n + threadIdx.x < n_group ? last : zero) << (4 * ((int)(n + threadIdx.x) & 7)));
+    for (int64_t i = from / 2 + threadIdx.x; i < n_all / 2; i += kThreads)
         codes[i] = (uint8_t)((2 * i < n_group ? last : zero) * 0x11u);
     if (threadIdx.x == 0)
         codes[n_all / 2] = 0;
@@ -332,7 +355,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             }
             if (lane16 == 0) {
                 atomicMax(rowred + row_slot(t.tile, it, drow), vmax);
-                if (!BITS) {
+                if (!BITS && (cols & 1) != 0) {
                     clear_shared(out.v[lo], w);
                     if (!M32)
                         clear_shared(out.m[lo], w);
@@ -385,9 +408,9 @@ struct AnyCoder<false> {
         const float xs[kAnyElts] = {x, x, x, x, x, x, x, x};
         return encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], xs) & 15u;
     }
-    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16) const
+    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16, bool odd_cols) const
     {
-        store_nibbles(codes, w, lane16, encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], x));
+        store_nibbles(codes, w, lane16, encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], x), odd_cols);
     }
 };
 
@@ -431,7 +454,7 @@ struct AnyCoder<true> {
     {
         return code1_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], x);
     }
-    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16) const
+    __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16, bool) const
     {
         uint32_t c[kAnyElts];
         codes8_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], even[which], x, c);
@@ -480,6 +503,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
+    const bool odd_cols = (cols & 1) != 0;
     NfHyper h;
     h.b2 = args.b2;
     h.w2 = args.w2;
@@ -494,11 +518,11 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
     if (tl == 0) {
         const int64_t n = t.rows * cols;
         const uint32_t zero_v = coder.one(1, 0.0f);
-        any_padding<BITS>(out.v[lo], n, n, zero_v, zero_v);
+        any_padding<BITS>(out.v[lo], n, n, zero_v, zero_v, odd_cols);
         if (!M32) {
             const int64_t group = (int64_t)1 << lg_group, n_group = (n + group - 1) / group * group;
             const float last = 0.0f / t.ms_new[(n - 1) >> lg_group];
-            any_padding<BITS>(out.m[lo], n, n_group, coder.one(0, last), coder.one(0, 0.0f));
+            any_padding<BITS>(out.m[lo], n, n_group, coder.one(0, last), coder.one(0, 0.0f), odd_cols);
         }
     }
     if (q.cg >= t.col_blocks || q.row0 >= t.rows)
@@ -560,7 +584,9 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
                     x[k] = lerp_w(x[k], g[k], h.w1);
             }
             any_quotients<HALF>(x, s);
-            coder.store(0, x, out.m[lo], w, lane16);
+            coder.store(0, x, out.m[lo], w, lane16, odd_cols);
+            // the second moment's loads stay behind the stores: 12 instead of 100 bytes of spilled registers a lane
+            __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k) {
@@ -581,7 +607,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
                 nonfused_second_moment(x[k], g[k], h);
         }
         any_quotients<HALF>(x, s);
-        coder.store(1, x, out.v[lo], w, lane16);
+        coder.store(1, x, out.v[lo], w, lane16, odd_cols);
     }
 }
 
