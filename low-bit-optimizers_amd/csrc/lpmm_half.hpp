@@ -115,28 +115,39 @@ __device__ __forceinline__ v2h half_second_moment(v2h v, v2h g, const NfHyper &h
     return round2(mix_add(v.x, ax, c), mix_add(v.y, ay, c));
 }
 
-// The same as PyTorch's GPU kernel leaves it, for the kernels that stand for the chain of device ops (any column
-// count, states that are not quantised): v + value * (g * g), the square exact in float.  With beta2 = 0.999 one gradient
-// in a few hundred puts that sum half way between two halfs, where it shows how it is rounded, as the product before it does: twice (to float, then to
-// half) in whole blocks of 2048 values of operands on 16-byte boundaries, and once (a mixed-precision fma) behind
-// them and everywhere on other boundaries.  once: bit 0 for the first value, bit 1 for the second.
+// The same as PyTorch's GPU kernels leave it, for the kernels that stand for the chain of device ops (any column
+// count, states that are not quantised): v + value * (g * g), the square exact in float.  Each of the two ops, the product by
+// beta2 and this sum, rounds twice (to float, then to half) in whole blocks of 2048 values if all its operands lie on 16-byte
+// boundaries, and once (a mixed-precision fma) behind them and everywhere on other boundaries.  With beta2 = 0.999 one
+// gradient in a few hundred puts the sum half way between two halfs, where that shows; a product does in ten thousand.
 constexpr int64_t kOpsBlock = 2048;
 
+// how many values of the flattened tensor are rounded twice by an op on these operands
 __device__ __forceinline__ int64_t ops_twice(const void *a, const void *b, int64_t n)
 {
     return ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0 ? n / kOpsBlock * kOpsBlock : 0;
 }
 
-__device__ __forceinline__ v2h half_second_moment_ops(v2h v, v2h g, const NfHyper &h, const MixConst &c, uint32_t once)
+// which of a lane's values the product and the sum round once, a bit per value
+struct RoundOnce {
+    uint32_t product, sum;
+};
+
+// pair j of the lane's
+__device__ __forceinline__ v2h half_second_moment_ops(v2h v, v2h g, const NfHyper &h, const MixConst &c, const RoundOnce &once, int j)
 {
-    const v2h d = round2(mix_mul(v.x, h.b2, c), mix_mul(v.y, h.b2, c));
+    const h16 none = (h16)c.neg_zero;
+    v2h d = round2(mix_mul(v.x, h.b2, c), mix_mul(v.y, h.b2, c));
+    if (once.product & (1u << (2 * j)))
+        d.x = round_once_fma((float)v.x, h.b2, none);
+    if (once.product & (2u << (2 * j)))
+        d.y = round_once_fma((float)v.y, h.b2, none);
     const float gx = mix_mul(g.x, (float)g.x, c), gy = mix_mul(g.y, (float)g.y, c);
     v2h r = round2(mix_add(d.x, h.w2 * gx, c), mix_add(d.y, h.w2 * gy, c));
-    const h16 none = (h16)c.neg_zero;
-    if (once & 1u)
-        r.x = round_once_fma(h.w2, gx, round_once_fma((float)v.x, h.b2, none));
-    if (once & 2u)
-        r.y = round_once_fma(h.w2, gy, round_once_fma((float)v.y, h.b2, none));
+    if (once.sum & (1u << (2 * j)))
+        r.x = round_once_fma(h.w2, gx, d.x);
+    if (once.sum & (2u << (2 * j)))
+        r.y = round_once_fma(h.w2, gy, d.y);
     return r;
 }
 
@@ -191,10 +202,10 @@ __device__ __forceinline__ v2h half_param(v2h p, v2h m, v2h v, const NfHyper &h,
 }
 
 // A lane's eight elements through the chain; p, m and v are updated in place.  Both branches are uniform.
-// OPS: the second moment as the device ops leave it, once: a bit per value (half_second_moment_ops)
+// OPS: the second moment as the device ops leave it (half_second_moment_ops)
 template <bool IEEE = false, bool OPS = false>
 __device__ __forceinline__ void half_elts8(v2h (&p)[kPairs], const v2h (&g)[kPairs], v2h (&m)[kPairs], v2h (&v)[kPairs],
-                                           const NfHyper &h, const MixConst &c, uint32_t once = 0)
+                                           const NfHyper &h, const MixConst &c, const RoundOnce &once = {})
 {
     if (fabsf(h.w1) < 0.5f) {
 #pragma unroll
@@ -207,7 +218,7 @@ __device__ __forceinline__ void half_elts8(v2h (&p)[kPairs], const v2h (&g)[kPai
     }
 #pragma unroll
     for (int j = 0; j < kPairs; ++j)
-        v[j] = OPS ? half_second_moment_ops(v[j], g[j], h, c, once >> (2 * j)) : half_second_moment(v[j], g[j], h, c);
+        v[j] = OPS ? half_second_moment_ops(v[j], g[j], h, c, once, j) : half_second_moment(v[j], g[j], h, c);
     // an eps that is positive as a half keeps every denominator positive: rounding is monotonic
     if (IEEE || h.eps > 0x1p-25f) {
 #pragma unroll

@@ -290,7 +290,9 @@ __global__ __launch_bounds__(kThreads) void nonfused_half_plain_kernel(const Mul
         m[k >> 1][k & 1] = in ? t.m[i] : (h16)0.0f;
         v[k >> 1][k & 1] = in ? t.v[i] : (h16)0.0f;
     }
-    half_elts8<true, true>(p, g, m, v, h, mix_const(), i0 - threadIdx.x + kHTile <= ops_twice(t.g, t.v, t.n) ? 0u : 0xffu);
+    const int64_t tile_end = i0 - threadIdx.x + kHTile;
+    const RoundOnce once = {tile_end <= ops_twice(t.v, nullptr, t.n) ? 0u : 0xffu, tile_end <= ops_twice(t.g, t.v, t.n) ? 0u : 0xffu};
+    half_elts8<true, true>(p, g, m, v, h, mix_const(), once);
 #pragma unroll
     for (int k = 0; k < kEltsPerLane; ++k) {
         const int64_t i = i0 + k * kThreads;

@@ -90,15 +90,16 @@ __device__ __forceinline__ int piece_at(const Piece &w, int lane16, int k)
     return off < w.count ? off : w.count - 1;
 }
 
-// bit k: the lane's value k lies behind the first `twice` of the flattened tensor (half_second_moment_ops)
-__device__ __forceinline__ uint32_t rounded_once(const Piece &w, int lane16, int64_t twice)
+// The chain of ops has its second moment in a tensor of its own, on a 16-byte boundary; the gradient may lie anywhere.
+__device__ __forceinline__ RoundOnce rounded_once(const Piece &w, int lane16, int64_t n, const void *g)
 {
-    uint32_t bits = 0;
+    const int64_t twice = ops_twice(nullptr, nullptr, n);
+    uint32_t behind = 0;
     if (w.base + w.count > twice)
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
-            bits |= (w.base + piece_at(w, lane16, k) >= twice ? 1u : 0u) << k;
-    return bits;
+            behind |= (w.base + piece_at(w, lane16, k) >= twice ? 1u : 0u) << k;
+    return RoundOnce{behind, ops_twice(g, nullptr, n) == twice ? behind : 0xffu};
 }
 
 // codes of the lane's eight values: element k in bits 4 k (two codes a byte) or in byte k (one a byte)
@@ -260,8 +261,6 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
 
     const uint32_t mask_m = (1u << bits_m) - 1u, mask_v = (1u << bits_v) - 1u;
     const int lg_group = 7 + (int)t.m_lg;
-    // the chain of ops has its second moment in a tensor of its own, on such a boundary
-    const int64_t twice = HALF ? ops_twice(t.g, nullptr, t.rows * cols) : 0;
     if (q.cg < t.col_blocks && q.row0 < t.rows) {
         const REAL *row_old = reinterpret_cast<const REAL *>(t.row_old);
         const REAL *col_old = reinterpret_cast<const REAL *>(t.col_old) + (int64_t)q.cg * kGroup;
@@ -316,7 +315,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                     m2[j] = round2(m[2 * j], m[2 * j + 1]);
                     v2[j] = round2(v[2 * j], v[2 * j + 1]);
                 }
-                half_elts8<true, true>(p2, g2, m2, v2, h, c, rounded_once(w, lane16, twice));
+                half_elts8<true, true>(p2, g2, m2, v2, h, c, rounded_once(w, lane16, t.rows * cols, t.g));
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k) {
                     p[k] = p2[k >> 1][k & 1];
@@ -513,8 +512,6 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
 
     const uint32_t mask_m = (1u << bits_m) - 1u, mask_v = (1u << bits_v) - 1u;
     const int lg_group = 7 + (int)t.m_lg;
-    // the chain of ops has its second moment in a tensor of its own, on such a boundary
-    const int64_t twice = HALF ? ops_twice(t.g, nullptr, t.rows * cols) : 0;
     if (tl == 0) {
         const int64_t n = t.rows * cols;
         const uint32_t zero_v = coder.one(1, 0.0f);
@@ -594,10 +591,10 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
             s[k] = rank1_scale(cn[k], rn);
         }
         if constexpr (HALF) {
-            const uint32_t once = rounded_once(w, lane16, twice);
+            const RoundOnce once = rounded_once(w, lane16, t.rows * cols, t.g);
 #pragma unroll
             for (int j = 0; j < kPairs; ++j) {
-                const v2h b = half_second_moment_ops(round2(x[2 * j], x[2 * j + 1]), v2h{g[2 * j], g[2 * j + 1]}, h, c, once >> (2 * j));
+                const v2h b = half_second_moment_ops(round2(x[2 * j], x[2 * j + 1]), v2h{g[2 * j], g[2 * j + 1]}, h, c, once, j);
                 x[2 * j] = (float)b.x;
                 x[2 * j + 1] = (float)b.y;
             }

@@ -313,3 +313,43 @@ def test_large_odd_matrices_equal_the_staged_route(kind, shape, monkeypatch):
                 params[1].data.copy_(params[0])
                 continue
             _same(got, want, f"step {step}, {j}")
+
+
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_half_second_moment_with_gradients_off_a_boundary(offset, monkeypatch):
+    """The product by beta2 is an op on the second moment alone, whose rounding the gradient's address does not change: a
+    hundred thousand random values a step (one in ten thousand tells), in 64 tensors whose states are not quantised and, as the
+    maxima of short rows, in a matrix; against torch's own ops and the chain of them."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    gen = torch.Generator(device="cuda").manual_seed(97)
+
+    def gradient(shape):
+        n = int(np.prod(shape))
+        return (torch.randn(offset + n, device="cuda", generator=gen) * 0.1).half()[offset:].view(shape)
+
+    plain = [torch.nn.Parameter(torch.zeros(4096 - i % 3, device="cuda", dtype=torch.float16)) for i in range(64)]
+    moments = [torch.zeros_like(p) for p in plain]
+    opt = lpmm.optim.AdamW(plain, fused=False, **H)
+    for step in range(4):
+        for p, v in zip(plain, moments):
+            p.grad = gradient(p.shape)
+            v.mul_(0.999).addcmul_(p.grad, p.grad, value=1 - 0.999)
+        opt.step()
+        for i, (p, v) in enumerate(zip(plain, moments)):
+            _same(to_np(opt.state[p]["exp_avg_sq"]), to_np(v), f"step {step} tensor {i}: second moment")
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    params = [torch.nn.Parameter(torch.zeros(32768, 35, device="cuda", dtype=torch.float16)) for _ in range(2)]
+    opts = [lpmm.optim.AdamW([p], qconfig=path, **H) for p in params]
+    for step in range(4):
+        params[0].grad = params[1].grad = gradient(params[0].shape)
+        opts[0].step()
+        with monkeypatch.context() as patch:
+            patch.setattr(adamw, "_any_columns", lambda rows, cols: False)
+            patch.setattr(adamw, "_native", _NoWalk(_native))
+            opts[1].step()
+        for j, (got, want) in enumerate(zip(_tensors(opts[0], params[0])[1:], _tensors(opts[1], params[1])[1:])):
+            _same(got, want, f"step {step}, {j}")
