@@ -343,7 +343,9 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         r.m_codes = item.use<uint8_t>(*mc);
         r.m_max1 = item.use<float>(*ms);
     }
-    const bool whole = r.cols % 128 == 0, folds = r.cols % 128 == 64 && r.rows % 2 == 0;
+    // the kernels that take 16 bytes an access; other operands go to the kernels for any column count
+    const bool aligned = aligned16(r.p) && aligned16(r.g);
+    const bool whole = aligned && r.cols % 128 == 0, folds = aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
     const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
     if (p.dim() > 2)
         return en_m && s.m_group128 && s.v_rank1 && served &&
@@ -362,7 +364,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         const at::Tensor *m = reals_like(mo, p);
         if (!s.v_rank1 || m == nullptr)
             return false;
-        if (!whole || !aligned16(r.p) || !aligned16(r.g)) {
+        if (!whole) {
             item.swaps = 0;
             return served && any(po, p, g, st, item, LPMM_RANK1_FLOAT_M, m, nullptr, *vc, nullptr, oh_v, qm, qv);
         }
@@ -385,7 +387,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         add(batch(kRank1, p, qm, qv), r, item);
         return true;
     }
-    const bool ragged = !whole && r.cols % 8 == 0;
+    const bool ragged = aligned && !whole && r.cols % 8 == 0;
     if (!whole && !ragged) {
         item.swaps = 0;
         return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, *vc, oh_m, oh_v, qm, qv);
@@ -473,7 +475,8 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
         r.m_codes = item.use<uint8_t>(*m);
     }
     r.workspace = scratch(p, (workspace_bytes(rows, cols) + 3) / 4);
-    add(batch(en && cols % 128 == 0 ? kFactored : kFactoredAny, p, qm, nullptr), r, item);
+    const bool tuned = en && cols % 128 == 0 && aligned16(r.p) && aligned16(r.g) && aligned16(r.col);
+    add(batch(tuned ? kFactored : kFactoredAny, p, qm, nullptr), r, item);
     return true;
 }
 

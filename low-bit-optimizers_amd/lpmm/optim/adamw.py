@@ -35,6 +35,12 @@ def _two_pass_columns(rows, cols):
     return cols % 128 == 0 or (cols % 128 == 64 and rows % 2 == 0)
 
 
+def _aligned(*tensors):
+    """Do the kernels that take 16 bytes an access take these operands?  Others (views at an odd offset of a flat buffer) go
+    to the kernels for any column count."""
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def _any_columns(rows, cols):
     """Matrices that the two passes for any column count take (50000 x 34: 54 us a step, staged 122; 8192 x 6: 52,
     staged 112-118).  A row costs them a block of 128 columns, so long matrices of a few columns stay with the
@@ -665,15 +671,14 @@ class AdamW(LowBitOptimizer):
                     continue
                 # whole 128-column blocks, or half a block left over with an even row count (taken
                 # as double rows: GPT-2-XL's 1600 and 4800 columns)
-                if v_rank1 and p.dim() == 2 and (p.shape[1] % 128 == 0
-                                                 or (p.shape[1] % 128 == 64 and p.shape[0] % 2 == 0)):
+                if v_rank1 and p.dim() == 2 and _two_pass_columns(*p.shape) and _aligned(dense, grad):
                     pending = batched_rank1.setdefault(key, _Batch())
                     pending.append(self._nonfused_rank1_record(p, dense, grad, state, step, pending))
                     if len(pending) == _native.RANK1_MULTI_MAX:
                         launch_rank1(key, pending)
                         pending.clear()
                     continue
-            if bits_rank1 and en_m and en_v and p.dim() == 2 and p.shape[1] % 128 == 0:
+            if bits_rank1 and en_m and en_v and p.dim() == 2 and p.shape[1] % 128 == 0 and _aligned(dense, grad):
                 qm, qv = state["exp_avg_qstate"]["qmap"], state["exp_avg_sq_qstate"]["qmap"]
                 key = (p.device, qm.data_ptr(), qv.data_ptr(), code_table(qm, md_m["b"]).data_ptr(),
                        code_table(qv, md_v["b"]).data_ptr())
@@ -688,7 +693,7 @@ class AdamW(LowBitOptimizer):
             # wide first-moment groups, or rows that are no whole number of 128-value groups (a multiple
             # of 8 columns; the two kinds go to different launches: the second takes more general kernels)
             ragged = p.dim() == 2 and p.shape[1] % 128 != 0 and p.shape[1] % 8 == 0
-            if (en_m and en_v and v_rank1 and p.dim() == 2
+            if (en_m and en_v and v_rank1 and p.dim() == 2 and _aligned(dense, grad)
                     and ((m_group_wide and p.shape[1] % 128 == 0) or ((m_group_wide or m_group128) and ragged))):
                 key = (p.device, state["exp_avg_qstate"]["qmap"].data_ptr(),
                        state["exp_avg_sq_qstate"]["qmap"].data_ptr(), ragged)
@@ -709,7 +714,7 @@ class AdamW(LowBitOptimizer):
                 elif en_m and bits_rank1:
                     kind = _native.RANK1_CODES8
                     tables = (code_table(qm, md_m["b"]).data_ptr(), code_table(qv, md_v["b"]).data_ptr())
-                elif not en_m and v_rank1 and (p.shape[1] % 128 != 0 or dense.data_ptr() % 16 or grad.data_ptr() % 16):
+                elif not en_m and v_rank1 and (p.shape[1] % 128 != 0 or not _aligned(dense, grad)):
                     kind = _native.RANK1_FLOAT_M
                 if kind is not None:
                     key = (kind, p.device, qm.data_ptr(), qv.data_ptr()) + tables
@@ -837,7 +842,7 @@ class AdamW(LowBitOptimizer):
         if v_group128 or (v_rank1 and p.dim() == 1):
             return "flat"
         if (v_rank1 and p.dim() == 2 and p.shape[1] % 128 == 0 and p.shape[0] > 0
-                and p.data_ptr() % 16 == 0 and grad.data_ptr() % 16 == 0):
+                and _aligned(p, grad)):
             return "rank1"
         if v_rank1 and p.dim() == 2 and _any_columns(p.shape[0], p.shape[1]):
             return "any"
@@ -1038,7 +1043,7 @@ class AdamW(LowBitOptimizer):
             for p, dense, grad, state, step in items:
                 rows, cols = p.shape[0], p.numel() // p.shape[0]
                 trailing = tuple(p.shape[1:]) + (1,)  # lpmm_rank1_row_scale_nd leaves the last dimension out
-                whole = _two_pass_columns(rows, cols)
+                whole = _two_pass_columns(rows, cols) and _aligned(dense, grad)
                 if whole:
                     mc, ms = self._group_state(p, state, "exp_avg")
                 else:
@@ -1226,7 +1231,7 @@ class AdamW(LowBitOptimizer):
                 continue
             rows, cols = p.shape
             qstate = state["exp_avg_qstate"]
-            tuned = enabled and cols % 128 == 0
+            tuned = enabled and cols % 128 == 0 and _aligned(dense, grad, state["exp_avg_sq_col"])
             first = False
             if enabled:
                 first = _is_placeholder(state["exp_avg"])

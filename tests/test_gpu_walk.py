@@ -259,3 +259,49 @@ def test_rank1_scales_without_a_group_size():
     # a constant gradient moves every value by lr a step, weight decay by lr * 0.01 at most
     assert torch.allclose(p, torch.full_like(p, 1 - 3e-2), atol=4e-4)
     assert len(opt.state[p]["exp_avg_qstate"]["overhead"]["max_dims"]) == 2
+
+
+@pytest.mark.parametrize("case", [c for c in CASES if c != "sgd" and not c.startswith("half")])
+def test_operands_off_a_16_byte_boundary(case, monkeypatch):
+    """Parameters and gradients that are views at an odd offset of a flat buffer, one or both, on every route and column
+    count: the step leaves what it leaves on aligned twins, through the walk and through the loops.  (float16 rounds by
+    the addresses, as torch's ops: test_gpu_nonfused_rank1_any.py.)"""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    kw = dict(CASES[case])
+    if "qconfig" in kw:
+        kw["qconfig"] = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", kw["qconfig"])
+    shapes = MATRICES + [(17, 8, 24), (40, 1024)]
+    rng = np.random.default_rng(12)
+    host = [rng.standard_normal(s) * 0.1 for s in shapes]
+
+    def at(a, off):
+        flat = torch.zeros(a.size + off, device="cuda")
+        flat[off:] = torch.from_numpy(a.reshape(-1)).float()
+        return flat[off:].view(a.shape)
+
+    def build(off):
+        params = [torch.nn.Parameter(at(h, off)) for h in host]
+        return params, lpmm.optim.AdamW(params, lr=1e-2, eps=1e-3, **kw)
+
+    sides = [build(0), build(1), build(0), build(3)]  # aligned; parameters, gradients, both off; the last without the walk
+    for step in range(4):
+        grads = [rng.standard_normal(s) * 0.1 for s in shapes]
+        for k, (params, opt) in enumerate(sides):
+            for p, g in zip(params, grads):
+                p.grad = at(g, (0, 0, 2, 1)[k])
+            with monkeypatch.context() as patch:
+                patch.setattr(adamw, "_native", _Native(_native, k != 3))
+                opt.step()
+        torch.cuda.synchronize()
+        for i, p in enumerate(sides[0][0]):
+            a = _state(sides[0][1], p)
+            for params, opt in sides[1:]:
+                b = _state(opt, params[i])
+                assert a.keys() == b.keys()
+                for k in a:
+                    assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), \
+                        (step, i, shapes[i], k)
+                assert torch.allclose(p, params[i], rtol=1e-6, atol=1e-7), (step, i, shapes[i])
