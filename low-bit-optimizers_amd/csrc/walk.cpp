@@ -7,16 +7,18 @@
 // strided operands, other routes; and for every error.
 //
 // collect() decides for each tensor, from the tensor and its state alone and anew on every step, whether it is
-// served, and reads its pointers; no state changes.  Plan.start() advances the step counts and completes the
-// records; after a launch is on the stream, Plan.commit() lets the states point to their new statistics (and, on
-// the kernels for any column count, codes).  A Plan lives for one step.
+// served, and reads its pointers; no state changes.  Plan.start() advances the step counts, Plan.prepare()
+// allocates what a launch's records need; after it is on the stream, Plan.commit() lets the states point to their new
+// statistics (and, on the kernels for any column count, codes).  A Plan lives for one step.
 #include <Python.h>
 
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <torch/csrc/DynamicTypes.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <cstddef>
 #include <cstring>
 #include <memory>
 #include <vector>
@@ -46,11 +48,21 @@ struct Swap {
     PyObject *dict, *key, *value;
 };
 
+// memory of a record, allocated when its launch is next (prepare): n floats of this step's scratch, or the array that
+// becomes the state which swap number `swap` replaces
+struct Need {
+    size_t at;  // of the pointer in the record
+    int64_t n;
+    int swap;
+    at::Tensor like;
+};
+
 struct Item {
     float *step = nullptr;
     Swap swap[8];
     int swaps = 0;
-    // what the record points into: between collect() and the launch runs the loop over the other tensors, and with it
+    std::vector<Need> needs;
+    // what the record points into, until its launch is on the stream: between collect() and then runs the loop over the other tensors, and with it
     // code of the caller's (a gradient that is a property), which may drop gradients or states
     std::vector<at::Tensor> kept;
 
@@ -74,8 +86,7 @@ struct Batch {
 struct Plan {
     PyObject_HEAD
     std::vector<Batch> *batches;
-    std::vector<at::Tensor> *scratch;
-    std::vector<PyObject *> *held;  // the maps and the new objects of the swaps: kept until the step is over
+    std::vector<PyObject *> *held;  // the maps and some of the swaps' objects: kept until the step is over
     PyObject *rest;
 };
 
@@ -198,7 +209,7 @@ struct Walk {
         for (int i = 0; i < own.swaps; ++i) {
             Py_INCREF(own.swap[i].dict);
             Py_INCREF(own.swap[i].key);
-            Py_INCREF(own.swap[i].value);
+            Py_XINCREF(own.swap[i].value);
         }
     }
     // an item for a parameter with its gradient
@@ -229,21 +240,12 @@ struct Walk {
     }
 
     // where a state's new codes go: a tensor that becomes the state (st[name])
-    uint8_t *next_codes(Item &item, PyObject *st, PyObject *name, const at::Tensor &codes)
+    static void next_codes(Item &item, size_t at, PyObject *st, PyObject *name, const at::Tensor &codes)
     {
-        const at::Tensor next = at::empty_like(codes);
-        PyObject *o = THPVariable_Wrap(next);
-        if (o == nullptr)
-            throw std::runtime_error("no tensor object");
-        plan->held->push_back(o);
-        item.swap[item.swaps++] = Swap{st, name, o};
-        return ptr<uint8_t>(next);
+        item.needs.push_back(Need{at, 0, item.swaps, codes});
+        item.swap[item.swaps++] = Swap{st, name, nullptr};
     }
-    float *scratch(const at::Tensor &p, int64_t n)
-    {
-        plan->scratch->push_back(at::empty({n}, p.options().dtype(at::kFloat)));
-        return ptr<float>(plan->scratch->back());
-    }
+    static void scratch(Item &item, size_t at, int64_t n) { item.needs.push_back(Need{at, n, -1, at::Tensor()}); }
 
     bool adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
     bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
@@ -426,14 +428,14 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     r.rows = p.size(0);
     r.cols = p.size(1);
     if (kind == LPMM_RANK1_HALF)
-        r.work = scratch(p, r.rows + r.cols + (p.numel() + 127) / 128);
+        scratch(item, offsetof(lpmm_rank1_any_tensor, work), r.rows + r.cols + (p.numel() + 127) / 128);
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
-    r.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
+    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, vc);
     if (ms != nullptr) {
         r.m_max1 = item.use(*ms);
         r.m_max1_next = item.use(*ms_next);
-        r.m_codes_next = next_codes(item, st, N.exp_avg, *mc);
+        next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *mc);
         swap_later(item, spare_scales, po, get(oh_m, N.max1));
         swap_later(item, oh_m, N.max1, spare);
     }
@@ -474,7 +476,7 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
             return false;
         r.m_codes = item.use<uint8_t>(*m);
     }
-    r.workspace = scratch(p, (workspace_bytes(rows, cols) + 3) / 4);
+    scratch(item, offsetof(lpmm_factored_tensor, workspace), (workspace_bytes(rows, cols) + 3) / 4);
     const bool tuned = en && cols % 128 == 0 && aligned16(r.p) && aligned16(r.g) && aligned16(r.col);
     add(batch(tuned ? kFactored : kFactoredAny, p, qm, nullptr), r, item);
     return true;
@@ -523,7 +525,8 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
     lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), item.use<uint8_t>(*mc), item.use(*ms), item.use<uint8_t>(*vc), now[0], now[1], next[0], next[1],
-                                        scratch(p, (rows + 3) / 4 * 4 + cols), rows, cols, 0.0f, 0.0f};
+                                        nullptr, rows, cols, 0.0f, 0.0f};
+    scratch(item, offsetof(lpmm_nonfused_rank1_f16_tensor, work), (rows + 3) / 4 * 4 + cols);
     add(batch(kHalfRank1, p, qm, qv), r, item);
     return true;
 }
@@ -587,8 +590,8 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     }
     lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, item.use(*ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
                                r.v_rowmax_next, r.v_colmax_next, nullptr, r.rows, r.cols, 0.0f, 0.0f};
-    w.m_codes_next = next_codes(item, st, N.exp_avg, *any_mc);
-    w.v_codes_next = next_codes(item, st, N.exp_avg_sq, vc);
+    next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *any_mc);
+    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, vc);
     swap_later(item, spare_scales, po, get(oh_m, N.max1));
     swap_later(item, oh_m, N.max1, spare);
     Batch &b = batch(kNdAny, p, qm, qv);
@@ -635,14 +638,13 @@ void plan_dealloc(PyObject *self)
                 for (int i = 0; i < item.swaps; ++i) {
                     Py_DECREF(item.swap[i].dict);
                     Py_DECREF(item.swap[i].key);
-                    Py_DECREF(item.swap[i].value);
+                    Py_XDECREF(item.swap[i].value);
                 }
     if (plan->held != nullptr)
         for (PyObject *o : *plan->held)
             Py_DECREF(o);
     delete plan->batches;
     delete plan->held;
-    delete plan->scratch;
     Py_XDECREF(plan->rest);
     Py_TYPE(self)->tp_free(self);
 }
@@ -686,28 +688,81 @@ PyObject *plan_start(PyObject *self, PyObject *)
     return out;
 }
 
-// commit(batch, first, count): the launch of these records is on the stream
-PyObject *plan_commit(PyObject *self, PyObject *args)
+// the arguments (batch, first, count) of the two methods below
+Batch *batch_of(PyObject *self, PyObject *args, Py_ssize_t *first, Py_ssize_t *end)
 {
     Plan *plan = reinterpret_cast<Plan *>(self);
-    Py_ssize_t k, first, count;
-    if (!PyArg_ParseTuple(args, "nnn", &k, &first, &count))
+    Py_ssize_t k, count;
+    if (!PyArg_ParseTuple(args, "nnn", &k, first, &count))
         return nullptr;
-    if (k < 0 || (size_t)k >= plan->batches->size() || first < 0 || count < 0 ||
-        (size_t)(first + count) > (*plan->batches)[k].items.size()) {
+    if (k < 0 || (size_t)k >= plan->batches->size() || *first < 0 || count < 0 ||
+        (size_t)(*first + count) > (*plan->batches)[k].items.size()) {
         PyErr_SetString(PyExc_IndexError, "no such records");
         return nullptr;
     }
-    for (Py_ssize_t i = first; i < first + count; ++i) {
-        const Item &item = (*plan->batches)[k].items[i];
+    *end = *first + count;
+    return &(*plan->batches)[k];
+}
+
+// prepare(batch, first, count): these records are launched next.  Their memory is allocated now and not in collect():
+// what the launches before them have released, old codes and scratch, is used again, so that a step holds
+// one launch's arrays beside the states and not a second set of them.
+PyObject *plan_prepare(PyObject *self, PyObject *args)
+{
+    HANDLE_TH_ERRORS
+    Py_ssize_t first, end;
+    Batch *b = batch_of(self, args, &first, &end);
+    if (b == nullptr)
+        return nullptr;
+    const size_t bytes = kRecordBytes[b->kind];
+    const auto floats = at::TensorOptions().dtype(at::kFloat).device(at::Device(at::kCUDA, (at::DeviceIndex)b->device));
+    for (Py_ssize_t i = first; i < end; ++i) {
+        Item &item = b->items[i];
+        for (Need &need : item.needs) {
+            const at::Tensor t = need.like.defined() ? at::empty_like(need.like) : at::empty({need.n}, floats);
+            if (need.like.defined()) {
+                PyObject *o = THPVariable_Wrap(t);
+                if (o == nullptr)
+                    return nullptr;
+                Py_XDECREF(item.swap[need.swap].value);
+                item.swap[need.swap].value = o;
+            } else {
+                item.kept.push_back(t);
+            }
+            const void *const p = ptr(t);
+            memcpy(&b->records[i * bytes + need.at], &p, sizeof p);
+            if (!b->second.empty())
+                memcpy(&b->second[i * bytes + need.at], &p, sizeof p);
+        }
+        item.needs.clear();
+    }
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
+
+// commit(batch, first, count): the launch of these records is on the stream
+PyObject *plan_commit(PyObject *self, PyObject *args)
+{
+    Py_ssize_t first, end;
+    Batch *b = batch_of(self, args, &first, &end);
+    if (b == nullptr)
+        return nullptr;
+    for (Py_ssize_t i = first; i < end; ++i) {
+        Item &item = b->items[i];
+        item.kept.clear();
         for (int j = 0; j < item.swaps; ++j)
-            if (PyDict_SetItem(item.swap[j].dict, item.swap[j].key, item.swap[j].value) != 0)
+            if (item.swap[j].value == nullptr) {
+                PyErr_SetString(PyExc_RuntimeError, "records that were not prepared");
                 return nullptr;
+            } else if (PyDict_SetItem(item.swap[j].dict, item.swap[j].key, item.swap[j].value) != 0) {
+                return nullptr;
+            }
     }
     Py_RETURN_NONE;
 }
 
 PyMethodDef plan_methods[] = {{"start", plan_start, METH_NOARGS, "advance the step counts and return the batches"},
+                              {"prepare", plan_prepare, METH_VARARGS, "allocate for records [first, first + count) of a batch"},
                               {"commit", plan_commit, METH_VARARGS, "records [first, first + count) of a batch are on the stream"},
                               {nullptr, nullptr, 0, nullptr}};
 PyObject *plan_served(PyObject *self, void *) { return PyBool_FromLong(!reinterpret_cast<Plan *>(self)->batches->empty()); }
@@ -739,7 +794,6 @@ PyObject *collect(PyObject *, PyObject *args)
     try {
         plan->batches = new std::vector<Batch>();
         plan->held = new std::vector<PyObject *>();
-        plan->scratch = new std::vector<at::Tensor>();
         plan->rest = PyList_New(0);
         if (plan->rest == nullptr)
             return nullptr;

@@ -14,6 +14,7 @@ RANK1_SMALL_SLOTS = 8192  # statistics entries of a vector lpmm_rank1_small_fold
 RANK1_SMALL_VALUES = 1 << 16  # longest vector worth the single workgroup that call gives it
 RANK1_MULTI_MAX = 32  # tensors per launch of the two-pass rank-1 step (kR1Max in csrc/nonfused_rank1.hip)
 SGD_MULTI_MAX = 64  # tensors per launch of the one-pass SGD step (kSgdMax in csrc/sgd.hip)
+FACTORED_MULTI_MAX = 24  # tensors per launch group of the factored step (kFaMax in csrc/factored.hip)
 V4BIT_MULTI_MAX = 48  # tensors per launch of the one-pass step with an fp32 first moment (kV4Max in csrc/nonfused_m32.hip)
 ABI_VERSION = 2
 CODE_TABLE_BYTES = 12288  # LPMM_CODE_TABLE_BYTES

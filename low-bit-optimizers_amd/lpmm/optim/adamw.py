@@ -276,7 +276,13 @@ class AdamW(LowBitOptimizer):
                     st = lib.lpmm_nonfused_adamw_v4bit_step_multi(records, count, qv_ptr, *hyper, stream)
                 elif kind in (_native.WALK_FACTORED, _native.WALK_FACTORED_ANY):
                     run = lib.lpmm_factored_step_multi if kind == _native.WALK_FACTORED else lib.lpmm_factored_any_step_multi
-                    st = run(records, count, qm_ptr, *hyper, stream)
+                    size, most = _native.FACTORED_TENSOR.itemsize, _native.FACTORED_MULTI_MAX
+                    for i in range(0, count, most):
+                        n = min(most, count - i)
+                        plan.prepare(k, i, n)
+                        _native.check(run(records + i * size, n, qm_ptr, *hyper, stream), "factored step")
+                        plan.commit(k, i, n)
+                    continue
                 elif kind == _native.WALK_HALF_PLAIN:
                     st = lib.lpmm_nonfused_update_f16_multi(records, count, *hyper, stream)
                 elif kind == _native.WALK_HALF_FLAT:
@@ -296,17 +302,23 @@ class AdamW(LowBitOptimizer):
             return [code_table(q, md["b"]).data_ptr() for q, md in ((qm, routes.m), (qv, routes.v))]
 
         if kind in (_native.WALK_ND, _native.WALK_ND_ANY):
-            for pass_no, table in ((1, records), (2, second)):
-                if kind == _native.WALK_ND:
-                    st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(table, count, qm.data_ptr(), qv_ptr, *hyper, pass_no, stream)
-                else:
-                    st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, count, _native.RANK1_CODES4, 128, qm.data_ptr(), 4, None,
-                                                                      qv_ptr, 4, None, *hyper, pass_no, stream)
-                _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
-                if pass_no == 1:
-                    st = lib.lpmm_rank1_small_fold_scale_multi(fold, count, stream)
-                    _native.check(st, "rank1_small_fold_scale_multi")
-            plan.commit(k, 0, count)
+            # the kernels for any column count write their codes to new arrays: one launch's worth of them at a time
+            whole = kind == _native.WALK_ND
+            size, chunk = (_native.NONFUSED_RANK1_TENSOR.itemsize, count) if whole else (_native.RANK1_ANY_TENSOR.itemsize, most)
+            for i in range(0, count, chunk):
+                n = min(chunk, count - i)
+                plan.prepare(k, i, n)
+                for pass_no, table in ((1, records + i * size), (2, second + i * size)):
+                    if whole:
+                        st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, pass_no, stream)
+                    else:
+                        st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, _native.RANK1_CODES4, 128, qm.data_ptr(), 4, None,
+                                                                          qv_ptr, 4, None, *hyper, pass_no, stream)
+                    _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
+                    if pass_no == 1:
+                        st = lib.lpmm_rank1_small_fold_scale_multi(fold + i * _native.RANK1_SMALL_VECTOR.itemsize, n, stream)
+                        _native.check(st, "rank1_small_fold_scale_multi")
+                plan.commit(k, i, n)
             return
         if kind == _native.WALK_RANK1:
             def run(table, n):
@@ -345,6 +357,7 @@ class AdamW(LowBitOptimizer):
             size = _native.RANK1_MGROUP_TENSOR.itemsize
         for i in range(0, count, most):
             n = min(most, count - i)
+            plan.prepare(k, i, n)
             _native.check(run(records + i * size, n), "non-fused AdamW step (rank-1 second moment)")
             plan.commit(k, i, n)
 
@@ -769,7 +782,14 @@ class AdamW(LowBitOptimizer):
                 self._requantise(p, state, "exp_avg_sq", v, md_v)
         self._factored_steps(group, factored_work)
         for key, items in nd_work.items():
-            self._rank1_nd_steps(group, key, items)
+            # the kernels for any column count write their codes to new arrays: one launch's worth of them at a time
+            whole, others = [], []
+            for item in items:
+                whole.append(item) if self._two_pass_whole(*item[:3]) else others.append(item)
+            if whole:
+                self._rank1_nd_steps(group, key, whole)
+            for i in range(0, len(others), _native.RANK1_MULTI_MAX):
+                self._rank1_nd_steps(group, key, others[i:i + _native.RANK1_MULTI_MAX])
         for dev, records in plain.items():
             table = np.array(records, dtype=_native.ADAMW_FP32_TENSOR)
             with torch.cuda.device(dev):
@@ -1020,6 +1040,11 @@ class AdamW(LowBitOptimizer):
         return (dense.data_ptr(), grad.data_ptr(), mc, ms) + self._rank1_state(p, state, batch) + (
             p.shape[0], p.shape[1], step, 0.0)
 
+    @staticmethod
+    def _two_pass_whole(p, dense, grad):
+        """Do the tuned two passes take this tensor of more than two dimensions?"""
+        return _two_pass_columns(p.shape[0], p.numel() // p.shape[0]) and _aligned(dense, grad)
+
     def _rank1_nd_steps(self, group, key, items):
         """The two-pass step on tensors of 3 to 8 dimensions (default configuration: first moment in
         groups of 128 values, rank-1 second moment).  The reference's scale of such a tensor is the
@@ -1043,7 +1068,7 @@ class AdamW(LowBitOptimizer):
             for p, dense, grad, state, step in items:
                 rows, cols = p.shape[0], p.numel() // p.shape[0]
                 trailing = tuple(p.shape[1:]) + (1,)  # lpmm_rank1_row_scale_nd leaves the last dimension out
-                whole = _two_pass_columns(rows, cols) and _aligned(dense, grad)
+                whole = self._two_pass_whole(p, dense, grad)
                 if whole:
                     mc, ms = self._group_state(p, state, "exp_avg")
                 else:
@@ -1253,15 +1278,17 @@ class AdamW(LowBitOptimizer):
                 [dense.data_ptr(), grad.data_ptr(), m, ms, state["exp_avg_sq_row"].data_ptr(),
                  state["exp_avg_sq_col"].data_ptr(), ws, rows, cols, step, 1 if first else 0])
         for run, tables in ((lib.lpmm_factored_step_multi, batched), (lib.lpmm_factored_any_step_multi, general)):
-            for (dev, qm_ptr), records in tables.items():
-                with torch.cuda.device(dev):
-                    work = torch.empty((sum(r[6] for r in records),), dtype=torch.uint8, device=dev)
-                    offset = work.data_ptr()
-                    for r in records:
-                        r[6], offset = offset, offset + r[6]
-                    table = np.array([tuple(r) for r in records], dtype=_native.FACTORED_TENSOR)
-                    st = run(table.ctypes.data, len(records), qm_ptr, beta1, beta2, lr, wd, eps, _native.current_stream(dev))
-                _native.check(st, "factored step")
+            for (dev, qm_ptr), pending in tables.items():
+                for first in range(0, len(pending), _native.FACTORED_MULTI_MAX):
+                    records = pending[first:first + _native.FACTORED_MULTI_MAX]
+                    with torch.cuda.device(dev):
+                        work = torch.empty((sum(r[6] for r in records),), dtype=torch.uint8, device=dev)
+                        offset = work.data_ptr()
+                        for r in records:
+                            r[6], offset = offset, offset + r[6]
+                        table = np.array([tuple(r) for r in records], dtype=_native.FACTORED_TENSOR)
+                        st = run(table.ctypes.data, len(records), qm_ptr, beta1, beta2, lr, wd, eps, _native.current_stream(dev))
+                    _native.check(st, "factored step")
         self._write_back(held)
 
     def _factored_step(self, group, p, dense, grad, state, step):

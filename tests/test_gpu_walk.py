@@ -305,3 +305,36 @@ def test_operands_off_a_16_byte_boundary(case, monkeypatch):
                     assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), \
                         (step, i, shapes[i], k)
                 assert torch.allclose(p, params[i], rtol=1e-6, atol=1e-7), (step, i, shapes[i])
+
+
+@pytest.mark.parametrize("case,shape", [("default", (300, 501)), ("half", (300, 501)), ("bits", (300, 501)), ("default", (100, 61, 5, 5)),
+                                        ("fused_factored", (300, 501))])
+@pytest.mark.parametrize("walk", [True, False])
+def test_a_step_holds_one_launch_of_new_arrays(case, shape, walk, monkeypatch):
+    """160 matrices of odd width, whose codes go to new arrays on every step: beside the states a step holds the
+    arrays of one launch (at most 32 tensors), not a second set of all states.  The bound is a quarter of the codes
+    (a launch's are a fifth; a factored step's workspaces are less still)."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    kw = dict(CASES[case])
+    dtype = kw.pop("dtype", torch.float32)
+    if "qconfig" in kw:
+        kw["qconfig"] = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", kw["qconfig"])
+    params = [torch.nn.Parameter(torch.full(shape, 0.1, device="cuda", dtype=dtype)) for _ in range(160)]
+    opt = lpmm.optim.AdamW(params, lr=1e-3, eps=1e-3, **kw)
+    for p in params:
+        p.grad = torch.full_like(p, 0.01)
+    with monkeypatch.context() as patch:
+        patch.setattr(adamw, "_native", _Native(_native, walk))
+        for _ in range(2):  # the states and the second buffers of their statistics exist
+            opt.step()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        opt.step()
+    grown = torch.cuda.max_memory_allocated() - before
+    codes = sum(t.numel() for p in params for t in opt.state[p].values() if torch.is_tensor(t) and t.dtype is torch.int8)
+    assert codes > 10 << 20 and grown <= codes // 4, (grown, codes)
+    assert torch.cuda.memory_allocated() <= before
