@@ -57,21 +57,21 @@ struct Need {
     at::Tensor like;
 };
 
+// a record in the making
 struct Item {
-    float *step = nullptr;
+    PyObject *step = nullptr;
+    const at::Tensor *grad = nullptr;
+    size_t held = 0;  // its objects in the plan's begin here
     Swap swap[8];
-    int swaps = 0;
-    std::vector<Need> needs;
-    // what the record points into, until its launch is on the stream: between collect() and then runs the loop over the other tensors, and with it
-    // code of the caller's (a gradient that is a property), which may drop gradients or states
-    std::vector<at::Tensor> kept;
+    int swaps = 0, needs = 0;
+    Need need[3];
+};
 
-    template <typename T = void>
-    T *use(const at::Tensor &t)
-    {
-        kept.push_back(t);
-        return static_cast<T *>(t.unsafeGetTensorImpl()->mutable_data());
-    }
+// what belongs to a record: ranges of the plan's and the batch's lists
+struct Record {
+    float *step;
+    at::Tensor grad, scratch;
+    uint32_t held, held_end, swaps, swaps_end, needs, needs_end;
 };
 
 struct Batch {
@@ -80,20 +80,37 @@ struct Batch {
     PyObject *qm, *qv;  // the maps' tensors (borrowed from held references)
     std::vector<uint8_t> records, second;
     std::vector<lpmm_rank1_small_vector> fold;
-    std::vector<Item> items;
+    std::vector<Record> items;
+    std::vector<Swap> swaps;
+    std::vector<Need> needs;
 };
 
 struct Plan {
     PyObject_HEAD
     std::vector<Batch> *batches;
-    std::vector<PyObject *> *held;  // the maps and some of the swaps' objects: kept until the step is over
+    // what the records point into (parameters, step counts, states), until their launch is on the stream:
+    // between collect() and then runs the loop over the other tensors, and with it code of the caller's (a gradient that is a
+    // property), which may drop gradients or states.  References of the Python objects: with copies of the tensors instead,
+    // counted atomically, 580 tensors took 60 us more a step.
+    std::vector<PyObject *> *held;
+    std::vector<PyObject *> *others;  // the maps, and objects made for the swaps: until the step is over
     PyObject *rest;
 };
 
-const at::Tensor *tensor_of(PyObject *o)
-{
-    return o != nullptr && THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
-}
+// a Python object that is a tensor (borrowed), or none
+struct Ref {
+    PyObject *o = nullptr;
+
+    Ref() = default;
+    Ref(std::nullptr_t) {}
+    explicit Ref(PyObject *tensor) : o(tensor) {}
+    const at::Tensor &operator*() const { return THPVariable_Unpack(o); }
+    const at::Tensor *operator->() const { return &THPVariable_Unpack(o); }
+    bool operator==(std::nullptr_t) const { return o == nullptr; }
+    bool operator!=(std::nullptr_t) const { return o != nullptr; }
+};
+
+Ref tensor_of(PyObject *o) { return o != nullptr && THPVariable_Check(o) ? Ref(o) : Ref(); }
 
 PyObject *get(PyObject *dict, PyObject *key)  // borrowed; null where absent (a Python error stays set)
 {
@@ -139,39 +156,39 @@ struct Walk {
     int64_t (*workspace_bytes)(int64_t, int64_t);  // lpmm_factored_workspace_bytes
 
     // a dense tensor of n values beside p and of its type (parameters on the kernels are float or half)
-    static const at::Tensor *reals_of(PyObject *o, const at::Tensor &p, int64_t n)
+    static Ref reals_of(PyObject *o, const at::Tensor &p, int64_t n)
     {
-        const at::Tensor *t = tensor_of(o);
+        const Ref t = tensor_of(o);
         return t != nullptr && on_gpu(*t) && t->scalar_type() == p.scalar_type() && t->numel() == n && t->get_device() == p.get_device() ? t : nullptr;
     }
     // a state of p's values; a single value: not created yet
-    static const at::Tensor *reals_like(PyObject *o, const at::Tensor &p) { return p.numel() > 1 ? reals_of(o, p, p.numel()) : nullptr; }
+    static Ref reals_like(PyObject *o, const at::Tensor &p) { return p.numel() > 1 ? reals_of(o, p, p.numel()) : nullptr; }
     // a state's codes, at least `bytes` of them
-    static const at::Tensor *codes(PyObject *o, const at::Tensor &p, int64_t bytes)
+    static Ref codes(PyObject *o, const at::Tensor &p, int64_t bytes)
     {
-        const at::Tensor *t = tensor_of(o);
+        const Ref t = tensor_of(o);
         return t != nullptr && t->numel() > 1 && t->numel() >= bytes && on_gpu(*t) && t->scalar_type() == at::kChar &&
                        t->get_device() == p.get_device()
                    ? t
                    : nullptr;
     }
     // the scales of `groups` groups
-    static const at::Tensor *scales(PyObject *qstate, PyObject **overhead, const at::Tensor &p, int64_t groups)
+    static Ref scales(PyObject *qstate, PyObject **overhead, const at::Tensor &p, int64_t groups)
     {
         *overhead = get(qstate, N.overhead);
         return reals_of(get(*overhead, N.max1), p, groups);
     }
     // one tensor per dimension
     template <typename T>
-    static bool statistics(Item &item, PyObject *list, const at::Tensor &p, T **out)
+    bool statistics(PyObject *list, const at::Tensor &p, T **out)
     {
         if (list == nullptr || !PyList_Check(list) || PyList_GET_SIZE(list) != p.dim())
             return false;
         for (Py_ssize_t i = 0; i < p.dim(); ++i) {
-            const at::Tensor *t = reals_of(PyList_GET_ITEM(list, i), p, p.size(i));
+            const Ref t = reals_of(PyList_GET_ITEM(list, i), p, p.size(i));
             if (t == nullptr)
                 return false;
-            out[i] = item.use<T>(*t);
+            out[i] = use<T>(t);
         }
         return true;
     }
@@ -182,17 +199,18 @@ struct Walk {
         for (Batch &b : *plan->batches)
             if (b.kind == kind && b.device == device && b.qm == qm && b.qv == qv && b.flag == flag)
                 return b;
-        plan->batches->push_back(Batch{kind, device, flag, qm, qv, {}, {}, {}, {}});
-        keep(qm);
-        keep(qv);
+        plan->batches->push_back(Batch{kind, device, flag, qm, qv, {}, {}, {}, {}, {}, {}});
+        for (PyObject *map : {qm, qv})
+            if (map != nullptr) {
+                Py_INCREF(map);
+                plan->others->push_back(map);
+            }
         return plan->batches->back();
     }
     void keep(PyObject *o)
     {
-        if (o != nullptr) {
-            Py_INCREF(o);
-            plan->held->push_back(o);
-        }
+        Py_INCREF(o);
+        plan->held->push_back(o);
     }
     template <typename R>
     static void append(std::vector<uint8_t> &to, const R &record)
@@ -204,23 +222,37 @@ struct Walk {
     void add(Batch &b, const R &record, Item &item)
     {
         append(b.records, record);
-        b.items.push_back(std::move(item));
-        const Item &own = b.items.back();
-        for (int i = 0; i < own.swaps; ++i) {
-            Py_INCREF(own.swap[i].dict);
-            Py_INCREF(own.swap[i].key);
-            Py_XINCREF(own.swap[i].value);
+        const uint32_t swaps = (uint32_t)b.swaps.size(), needs = (uint32_t)b.needs.size();
+        for (int i = 0; i < item.needs; ++i) {
+            item.need[i].swap += item.need[i].swap >= 0 ? (int)swaps : 0;
+            b.needs.push_back(std::move(item.need[i]));
         }
+        for (int i = 0; i < item.swaps; ++i) {
+            Py_INCREF(item.swap[i].dict);
+            Py_INCREF(item.swap[i].key);
+            Py_XINCREF(item.swap[i].value);
+            b.swaps.push_back(item.swap[i]);
+        }
+        b.items.push_back(Record{item.step != nullptr ? ptr<float>(THPVariable_Unpack(item.step)) : nullptr, *item.grad, at::Tensor(),
+                                 (uint32_t)item.held, (uint32_t)plan->held->size(), swaps, (uint32_t)b.swaps.size(), needs,
+                                 (uint32_t)b.needs.size()});
     }
-    // an item for a parameter with its gradient
-    static Item item_of(const at::Tensor &p, const at::Tensor &g, const at::Tensor *step)
+    // the data of a tensor that the plan holds from here on
+    template <typename T = void>
+    T *use(const Ref &t)
+    {
+        keep(t.o);
+        return ptr<T>(*t);
+    }
+    // an item for a parameter with its gradient; step: its count, or null
+    Item item_of(PyObject *po, const at::Tensor &g, const Ref &step)
     {
         Item item;
-        item.kept.reserve(12);
-        item.kept.push_back(p);
-        item.kept.push_back(g);
+        item.held = plan->held->size();
+        item.grad = &g;
+        keep(po);
         if (step != nullptr)
-            item.step = item.use<float>(*step);
+            keep(item.step = step.o);
         return item;
     }
 
@@ -242,18 +274,18 @@ struct Walk {
     // where a state's new codes go: a tensor that becomes the state (st[name])
     static void next_codes(Item &item, size_t at, PyObject *st, PyObject *name, const at::Tensor &codes)
     {
-        item.needs.push_back(Need{at, 0, item.swaps, codes});
+        item.need[item.needs++] = Need{at, 0, item.swaps, codes};
         item.swap[item.swaps++] = Swap{st, name, nullptr};
     }
-    static void scratch(Item &item, size_t at, int64_t n) { item.needs.push_back(Need{at, n, -1, at::Tensor()}); }
+    static void scratch(Item &item, size_t at, int64_t n) { item.need[item.needs++] = Need{at, n, -1, at::Tensor()}; }
 
     bool adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
-    bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
-    bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step);
-    bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const at::Tensor *mc,
-             const at::Tensor *ms, const at::Tensor &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
-    bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const at::Tensor *any_mc,
-            PyObject *oh_m, const at::Tensor &vc, PyObject *oh_v, PyObject *qm, PyObject *qv);
+    bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+    bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+    bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const Ref &mc,
+             const Ref &ms, const Ref &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
+    bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const Ref &any_mc,
+            PyObject *oh_m, const Ref &vc, PyObject *oh_v, PyObject *qm, PyObject *qv);
     bool sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
 };
 
@@ -265,14 +297,14 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     if (!g.defined() || !on_gpu(p) || !on_gpu(g) || p.device() != g.device() || p.numel() != g.numel() ||
         g.scalar_type() != p.scalar_type())
         return false;
-    const at::Tensor *step = tensor_of(get(st, N.step));
+    const Ref step = tensor_of(get(st, N.step));
     if (step == nullptr || !step->is_cpu() || step->scalar_type() != at::kFloat || step->dim() != 0)
         return false;
     const bool is_factored = get(st, N.exp_avg_sq_row) != nullptr;
     if (!floats(p))
-        return halfs(p) && !s.fused && !is_factored && half(po, p, g, st, *step);
+        return halfs(p) && !s.fused && !is_factored && half(po, p, g, st);
     if (is_factored)
-        return factored(po, p, g, st, *step);
+        return factored(po, p, g, st);
     if (s.fused == 2)
         return false;
     PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
@@ -280,45 +312,45 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
     if (en_m < 0 || en_v < 0)
         return false;
-    Item item = item_of(p, g, step);
+    Item item = item_of(po, g, tensor_of(get(st, N.step)));
     const int64_t n = p.numel();
     if (!en_m && !en_v) {
-        const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
+        const Ref m = reals_like(mo, p), v = reals_like(vo, p);
         if (m == nullptr || v == nullptr)
             return false;
-        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<float>(*v), n, 0.0f, 0.0f};
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), use<float>(m), use<float>(v), n, 0.0f, 0.0f};
         add(batch(kPlain, p, nullptr, nullptr), r, item);
         return true;
     }
     PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap);
-    const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
-    const at::Tensor *vc = codes(vo, p, s.fused ? (n + 1) / 2 : packed(n, 128, s.bits_rank1));
+    const Ref map_m = tensor_of(qm), map_v = tensor_of(qv);
+    const Ref vc = codes(vo, p, s.fused ? (n + 1) / 2 : packed(n, 128, s.bits_rank1));
     if (map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) || vc == nullptr || !en_v)
         return false;
     PyObject *oh_m = nullptr, *oh_v = nullptr;
     if (s.fused || s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
-        const at::Tensor *vs = scales(qs_v, &oh_v, p, (n + 127) / 128);
+        const Ref vs = scales(qs_v, &oh_v, p, (n + 127) / 128);
         if (vs == nullptr)
             return false;
         if (!en_m) {
-            const at::Tensor *m = reals_like(mo, p);
+            const Ref m = reals_like(mo, p);
             if (s.fused || m == nullptr)
                 return false;
-            lpmm_adamw_v4bit_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<uint8_t>(*vc), item.use<float>(*vs), n, 0.0f, 0.0f};
+            lpmm_adamw_v4bit_tensor r = {ptr<float>(p), ptr<float>(g), use<float>(m), use<uint8_t>(vc), use<float>(vs), n, 0.0f, 0.0f};
             add(batch(kFlatM32, p, nullptr, qv), r, item);
             return true;
         }
-        const at::Tensor *mc = codes(mo, p, s.fused ? (n + 1) / 2 : packed(n, 128, false)), *ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
+        const Ref mc = codes(mo, p, s.fused ? (n + 1) / 2 : packed(n, 128, false)), ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
         if (!(s.fused ? n % 2 == 0 : s.m_group128 != 0) || mc == nullptr || ms == nullptr)
             return false;
         lpmm_adamw4bit_tensor r;
         memset(&r, 0, sizeof r);
         r.p = ptr<float>(p);
         r.g = ptr<float>(g);
-        r.m_codes = item.use<uint8_t>(*mc);
-        r.v_codes = item.use<uint8_t>(*vc);
-        r.m_scale = item.use<float>(*ms);
-        r.v_scale = item.use<float>(*vs);
+        r.m_codes = use<uint8_t>(mc);
+        r.v_codes = use<uint8_t>(vc);
+        r.m_scale = use<float>(ms);
+        r.v_scale = use<float>(vs);
         r.n = n;
         add(batch(s.fused ? kFused4 : kFlat, p, qm, qv), r, item);
         return true;
@@ -331,10 +363,10 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     memset(&r, 0, sizeof r);
     r.p = ptr<float>(p);
     r.g = ptr<float>(g);
-    r.v_codes = item.use<uint8_t>(*vc);
+    r.v_codes = use<uint8_t>(vc);
     r.rows = p.size(0);
     r.cols = n / r.rows;
-    const at::Tensor *mc = nullptr, *ms = nullptr;
+    Ref mc, ms;
     if (en_m) {
         if (s.m_group <= 0)
             return false;
@@ -342,8 +374,8 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
         if (mc == nullptr || ms == nullptr)
             return false;
-        r.m_codes = item.use<uint8_t>(*mc);
-        r.m_max1 = item.use<float>(*ms);
+        r.m_codes = use<uint8_t>(mc);
+        r.m_max1 = use<float>(ms);
     }
     // the kernels that take 16 bytes an access; other operands go to the kernels for any column count
     const bool aligned = aligned16(r.p) && aligned16(r.g);
@@ -351,10 +383,10 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
     if (p.dim() > 2)
         return en_m && s.m_group128 && s.v_rank1 && served &&
-               nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, *vc, oh_v, qm, qv);
+               nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, vc, oh_v, qm, qv);
     PyObject *nxt = get(spare_stats, po);
     float *now[2], *next[2];
-    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next))
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
         return false;
     r.v_rowmax = now[0];
     r.v_colmax = now[1];
@@ -363,16 +395,16 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
     if (!en_m) {
-        const at::Tensor *m = reals_like(mo, p);
+        const Ref m = reals_like(mo, p);
         if (!s.v_rank1 || m == nullptr)
             return false;
         if (!whole) {
             item.swaps = 0;
-            return served && any(po, p, g, st, item, LPMM_RANK1_FLOAT_M, m, nullptr, *vc, nullptr, oh_v, qm, qv);
+            return served && any(po, p, g, st, item, LPMM_RANK1_FLOAT_M, m, nullptr, vc, nullptr, oh_v, qm, qv);
         }
         if (!aligned16(ptr(*m)))
             return false;
-        lpmm_rank1_v4bit_tensor f = {r.p, r.g, item.use<float>(*m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
+        lpmm_rank1_v4bit_tensor f = {r.p, r.g, use<float>(m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
                                      r.rows, r.cols, 0.0f, 0.0f};
         add(batch(kRank1M32, p, nullptr, qv), f, item);
         return true;
@@ -380,7 +412,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     if (s.bits_rank1) {
         if (!whole) {
             item.swaps = 0;
-            return served && any(po, p, g, st, item, LPMM_RANK1_CODES8, mc, ms, *vc, oh_m, oh_v, qm, qv);
+            return served && any(po, p, g, st, item, LPMM_RANK1_CODES8, mc, ms, vc, oh_m, oh_v, qm, qv);
         }
         add(batch(kRank1Bits, p, qm, qv), r, item);
         return true;
@@ -392,13 +424,13 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const bool ragged = aligned && !whole && r.cols % 8 == 0;
     if (!whole && !ragged) {
         item.swaps = 0;
-        return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, *vc, oh_m, oh_v, qm, qv);
+        return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, vc, oh_m, oh_v, qm, qv);
     }
     PyObject *spare = get(spare_scales, po);
-    const at::Tensor *ms_next = reals_of(spare, p, ms->numel());
+    const Ref ms_next = reals_of(spare, p, ms->numel());
     if (!((s.m_wide && whole) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
         return false;
-    lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        item.use<float>(*ms_next), r.v_codes, r.v_rowmax,
+    lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        use<float>(ms_next), r.v_codes, r.v_rowmax,
                                   r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
     swap_later(item, spare_scales, po, get(oh_m, N.max1));
     swap_later(item, oh_m, N.max1, spare);
@@ -407,20 +439,20 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
 }
 
 // a matrix of any column count (lpmm_nonfused_adamw_rank1_any_step_multi); mc: the first moment's codes or values
-bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const at::Tensor *mc,
-               const at::Tensor *ms, const at::Tensor &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv)
+bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const Ref &mc,
+               const Ref &ms, const Ref &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv)
 {
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *spare = get(spare_scales, po);
     void *now[2], *next[2];
-    const at::Tensor *ms_next = ms != nullptr ? reals_of(spare, p, ms->numel()) : nullptr;
-    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next) || (ms != nullptr && ms_next == nullptr))
+    const Ref ms_next = ms != nullptr ? reals_of(spare, p, ms->numel()) : nullptr;
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || (ms != nullptr && ms_next == nullptr))
         return false;
     lpmm_rank1_any_tensor r;
     memset(&r, 0, sizeof r);
     r.p = ptr(p);
     r.g = ptr(g);
-    r.m = item.use(*mc);
-    r.v_codes = item.use<uint8_t>(vc);
+    r.m = use<>(mc);
+    r.v_codes = use<uint8_t>(vc);
     r.v_rowmax = now[0];
     r.v_colmax = now[1];
     r.v_rowmax_next = next[0];
@@ -431,10 +463,10 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
         scratch(item, offsetof(lpmm_rank1_any_tensor, work), r.rows + r.cols + (p.numel() + 127) / 128);
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
-    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, vc);
+    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, *vc);
     if (ms != nullptr) {
-        r.m_max1 = item.use(*ms);
-        r.m_max1_next = item.use(*ms_next);
+        r.m_max1 = use<>(ms);
+        r.m_max1_next = use<>(ms_next);
         next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *mc);
         swap_later(item, spare_scales, po, get(oh_m, N.max1));
         swap_later(item, oh_m, N.max1, spare);
@@ -444,37 +476,37 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
 }
 
 // a matrix with a factored second moment, its first moment 4-bit in groups of 128 values or not quantised
-bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step)
+bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
 {
     if (p.dim() != 2 || p.numel() == 0 || workspace_bytes == nullptr)
         return false;
     const int64_t rows = p.size(0), cols = p.size(1), n = p.numel();
     PyObject *qs = get(st, N.exp_avg_qstate), *mo = get(st, N.exp_avg), *qm = get(qs, N.qmap), *oh = nullptr;
-    const at::Tensor *row = reals_of(get(st, N.exp_avg_sq_row), p, rows), *col = reals_of(get(st, N.exp_avg_sq_col), p, cols);
-    const at::Tensor *map = tensor_of(qm);
+    const Ref row = reals_of(get(st, N.exp_avg_sq_row), p, rows), col = reals_of(get(st, N.exp_avg_sq_col), p, cols);
+    const Ref map = tensor_of(qm);
     const int en = enabled(po, qs);
     if (en < 0 || row == nullptr || col == nullptr || map == nullptr || !floats(*map))
         return false;
-    Item item = item_of(p, g, &step);
+    Item item = item_of(po, g, tensor_of(get(st, N.step)));
     lpmm_factored_tensor r;
     memset(&r, 0, sizeof r);
     r.p = ptr<float>(p);
     r.g = ptr<float>(g);
-    r.row = item.use<float>(*row);
-    r.col = item.use<float>(*col);
+    r.row = use<float>(row);
+    r.col = use<float>(col);
     r.rows = rows;
     r.cols = cols;
     if (en) {
-        const at::Tensor *mc = codes(mo, p, packed(n, 128, false)), *ms = scales(qs, &oh, p, (n + 127) / 128);
+        const Ref mc = codes(mo, p, packed(n, 128, false)), ms = scales(qs, &oh, p, (n + 127) / 128);
         if (!s.m_group128 || mc == nullptr || ms == nullptr)
             return false;
-        r.m_codes = item.use<uint8_t>(*mc);
-        r.m_max1 = item.use<float>(*ms);
+        r.m_codes = use<uint8_t>(mc);
+        r.m_max1 = use<float>(ms);
     } else {
-        const at::Tensor *m = reals_like(mo, p);
+        const Ref m = reals_like(mo, p);
         if (m == nullptr)
             return false;
-        r.m_codes = item.use<uint8_t>(*m);
+        r.m_codes = use<uint8_t>(m);
     }
     scratch(item, offsetof(lpmm_factored_tensor, workspace), (workspace_bytes(rows, cols) + 3) / 4);
     const bool tuned = en && cols % 128 == 0 && aligned16(r.p) && aligned16(r.g) && aligned16(r.col);
@@ -483,33 +515,33 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
 }
 
 // float16 parameters on the non-fused path (lpmm/optim/adamw.py: _half_kernel_kind)
-bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const at::Tensor &step)
+bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
 {
     PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
     PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
     const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
     const int64_t n = p.numel(), groups = (n + 127) / 128;
-    Item item = item_of(p, g, &step);
+    Item item = item_of(po, g, tensor_of(get(st, N.step)));
     if (en_m == 0 && en_v == 0) {
-        const at::Tensor *m = reals_like(mo, p), *v = reals_like(vo, p);
+        const Ref m = reals_like(mo, p), v = reals_like(vo, p);
         if (m == nullptr || v == nullptr || m->sizes() != p.sizes() || v->sizes() != p.sizes())
             return false;
-        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*m), item.use<float>(*v), n, 0.0f, 0.0f};
+        lpmm_adamw_fp32_tensor r = {ptr<float>(p), ptr<float>(g), use<float>(m), use<float>(v), n, 0.0f, 0.0f};
         add(batch(kHalfPlain, p, nullptr, nullptr), r, item);
         return true;
     }
     PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap), *oh_m = nullptr, *oh_v = get(qs_v, N.overhead);
-    const at::Tensor *map_m = tensor_of(qm), *map_v = tensor_of(qv);
-    const at::Tensor *mc = codes(mo, p, packed(n, 128, false)), *vc = codes(vo, p, packed(n, 128, false)), *ms = scales(qs_m, &oh_m, p, groups);
+    const Ref map_m = tensor_of(qm), map_v = tensor_of(qv);
+    const Ref mc = codes(mo, p, packed(n, 128, false)), vc = codes(vo, p, packed(n, 128, false)), ms = scales(qs_m, &oh_m, p, groups);
     PyObject *const half_type = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
     if (en_m != 1 || en_v != 1 || !s.m_group128 || map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) ||
         mc == nullptr || vc == nullptr || ms == nullptr || get(oh_m, N.dtype) != half_type || get(oh_v, N.dtype) != half_type)
         return false;
     if (s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
-        const at::Tensor *vs = scales(qs_v, &oh_v, p, groups);
+        const Ref vs = scales(qs_v, &oh_v, p, groups);
         if (vs == nullptr)
             return false;
-        lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), item.use<uint8_t>(*mc), item.use<uint8_t>(*vc), item.use(*ms), item.use(*vs), n, 0.0f, 0.0f};
+        lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), use<uint8_t>(mc), use<uint8_t>(vc), use<>(ms), use<>(vs), n, 0.0f, 0.0f};
         add(batch(kHalfFlat, p, qm, qv), r, item);
         return true;
     }
@@ -517,14 +549,14 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
         return false;
     const int64_t rows = p.size(0), cols = p.size(1);
     if (cols % 128 != 0 || !aligned16(ptr(p)) || !aligned16(ptr(g)))
-        return (cols >= 32 || rows <= 32768) && any(po, p, g, st, item, LPMM_RANK1_HALF, mc, ms, *vc, oh_m, oh_v, qm, qv);
+        return (cols >= 32 || rows <= 32768) && any(po, p, g, st, item, LPMM_RANK1_HALF, mc, ms, vc, oh_m, oh_v, qm, qv);
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po);
     void *now[2], *next[2];
-    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next))
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next))
         return false;
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
-    lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), item.use<uint8_t>(*mc), item.use(*ms), item.use<uint8_t>(*vc), now[0], now[1], next[0], next[1],
+    lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), use<uint8_t>(mc), use<>(ms), use<uint8_t>(vc), now[0], now[1], next[0], next[1],
                                         nullptr, rows, cols, 0.0f, 0.0f};
     scratch(item, offsetof(lpmm_nonfused_rank1_f16_tensor, work), (rows + 3) / 4 * 4 + cols);
     add(batch(kHalfRank1, p, qm, qv), r, item);
@@ -533,17 +565,17 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
 
 // a tensor of 3 to 8 dimensions on its shape[0] x rest view, where the fold between the passes takes one workgroup
 // and the column scale the last step left still holds (lpmm/optim/adamw.py: _rank1_nd_steps)
-bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const at::Tensor *any_mc,
-              PyObject *oh_m, const at::Tensor &vc, PyObject *oh_v, PyObject *qm, PyObject *qv)
+bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const Ref &any_mc,
+              PyObject *oh_m, const Ref &vc, PyObject *oh_v, PyObject *qm, PyObject *qv)
 {
     const int dims = (int)p.dim();
     if (dims > LPMM_RANK1_ND_MAX || (r.rows < 16 && p.numel() > (1 << 20)) || r.cols > (1 << 16))
         return false;
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *scratch = get(nd_scratch, po);
     PyObject *row = get(scratch, N.row);
-    const at::Tensor *work = reals_of(get(scratch, N.work), p, 3 * r.cols);
+    const Ref work = reals_of(get(scratch, N.work), p, 3 * r.cols);
     float *now[LPMM_RANK1_ND_MAX], *next[LPMM_RANK1_ND_MAX];
-    if (!statistics(item, cur, p, now) || !statistics(item, nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
+    if (!statistics(cur, p, now) || !statistics(nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
         return false;
     const long old_row = PyLong_AsLong(row);
     if (old_row < 0 || old_row > 2)
@@ -559,7 +591,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     }
     if (slots > 8192)
         return false;
-    float *const rows = item.use<float>(*work);
+    float *const rows = use<float>(work);
     fold.ndim = dims - 1;
     fold.x = rows + raw_row * r.cols;
     fold.scale = rows + new_row * r.cols;
@@ -569,13 +601,13 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     r.v_colmax_next = rows + raw_row * r.cols;
     // any_mc: a column count for the general kernels, which also need the next scales
     PyObject *spare = get(spare_scales, po);
-    const at::Tensor *ms_next = any_mc != nullptr ? reals_of(spare, p, (p.numel() + 127) / 128) : nullptr;
+    const Ref ms_next = any_mc != nullptr ? reals_of(spare, p, (p.numel() + 127) / 128) : nullptr;
     if (any_mc != nullptr && ms_next == nullptr)
         return false;
     PyObject *row_obj = PyLong_FromLong(new_row);
     if (row_obj == nullptr)
         return false;
-    plan->held->push_back(row_obj);
+    plan->others->push_back(row_obj);
     swap_later(item, spare_stats, po, cur);
     swap_later(item, oh_v, N.max_dims, nxt);
     swap_later(item, scratch, N.scale_of, nxt);
@@ -588,10 +620,10 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         b.fold.push_back(fold);
         return true;
     }
-    lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, item.use(*ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
+    lpmm_rank1_any_tensor w = {r.p, r.g, r.m_codes, nullptr, r.m_max1, use<>(ms_next), r.v_codes, nullptr, r.v_rowmax, r.v_colmax,
                                r.v_rowmax_next, r.v_colmax_next, nullptr, r.rows, r.cols, 0.0f, 0.0f};
     next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *any_mc);
-    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, vc);
+    next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, *vc);
     swap_later(item, spare_scales, po, get(oh_m, N.max1));
     swap_later(item, oh_m, N.max1, spare);
     Batch &b = batch(kNdAny, p, qm, qv);
@@ -607,23 +639,23 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     if (!g.defined() || !floats(p) || !floats(g) || p.device() != g.device() || p.numel() != g.numel())
         return false;
     PyObject *qs = get(st, N.momentum_buffer_qstate), *bo = get(st, N.momentum_buffer);
-    Item item = item_of(p, g, nullptr);
+    Item item = item_of(po, g, nullptr);
     const int en = enabled(po, qs);
     if (en < 0)
         return false;
     if (!en) {
-        const at::Tensor *buf = reals_like(bo, p);
+        const Ref buf = reals_like(bo, p);
         if (buf == nullptr || buf->sizes() != p.sizes())
             return false;
-        lpmm_sgd_fp32_tensor r = {ptr<float>(p), ptr<float>(g), item.use<float>(*buf), p.numel(), 0, 0};
+        lpmm_sgd_fp32_tensor r = {ptr<float>(p), ptr<float>(g), use<float>(buf), p.numel(), 0, 0};
         add(batch(kSgdPlain, p, nullptr, nullptr), r, item);
         return true;
     }
     PyObject *oh = nullptr, *qm = get(qs, N.qmap);
-    const at::Tensor *map = tensor_of(qm), *mc = codes(bo, p, packed(p.numel(), 128, false)), *ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
+    const Ref map = tensor_of(qm), mc = codes(bo, p, packed(p.numel(), 128, false)), ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
     if (!s.m_group128 || map == nullptr || !floats(*map) || mc == nullptr || ms == nullptr)
         return false;
-    lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), item.use<uint8_t>(*mc), item.use<float>(*ms), p.numel(), 0, 0};
+    lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), use<uint8_t>(mc), use<float>(ms), p.numel(), 0, 0};
     add(batch(kSgd4, p, qm, nullptr), r, item);
     return true;
 }
@@ -634,17 +666,18 @@ void plan_dealloc(PyObject *self)
     Plan *plan = reinterpret_cast<Plan *>(self);
     if (plan->batches != nullptr)
         for (Batch &b : *plan->batches)
-            for (Item &item : b.items)
-                for (int i = 0; i < item.swaps; ++i) {
-                    Py_DECREF(item.swap[i].dict);
-                    Py_DECREF(item.swap[i].key);
-                    Py_XDECREF(item.swap[i].value);
-                }
-    if (plan->held != nullptr)
-        for (PyObject *o : *plan->held)
-            Py_DECREF(o);
+            for (Swap &swap : b.swaps) {
+                Py_DECREF(swap.dict);
+                Py_DECREF(swap.key);
+                Py_XDECREF(swap.value);
+            }
+    for (std::vector<PyObject *> *list : {plan->held, plan->others})
+        if (list != nullptr)
+            for (PyObject *o : *list)
+                Py_XDECREF(o);
     delete plan->batches;
     delete plan->held;
+    delete plan->others;
     Py_XDECREF(plan->rest);
     Py_TYPE(self)->tp_free(self);
 }
@@ -717,24 +750,26 @@ PyObject *plan_prepare(PyObject *self, PyObject *args)
     const size_t bytes = kRecordBytes[b->kind];
     const auto floats = at::TensorOptions().dtype(at::kFloat).device(at::Device(at::kCUDA, (at::DeviceIndex)b->device));
     for (Py_ssize_t i = first; i < end; ++i) {
-        Item &item = b->items[i];
-        for (Need &need : item.needs) {
+        Record &item = b->items[i];
+        for (uint32_t j = item.needs; j < item.needs_end; ++j) {
+            Need &need = b->needs[j];
             const at::Tensor t = need.like.defined() ? at::empty_like(need.like) : at::empty({need.n}, floats);
             if (need.like.defined()) {
                 PyObject *o = THPVariable_Wrap(t);
                 if (o == nullptr)
                     return nullptr;
-                Py_XDECREF(item.swap[need.swap].value);
-                item.swap[need.swap].value = o;
+                Py_XDECREF(b->swaps[need.swap].value);
+                b->swaps[need.swap].value = o;
             } else {
-                item.kept.push_back(t);
+                item.scratch = t;
             }
+            need.like.reset();
             const void *const p = ptr(t);
             memcpy(&b->records[i * bytes + need.at], &p, sizeof p);
             if (!b->second.empty())
                 memcpy(&b->second[i * bytes + need.at], &p, sizeof p);
         }
-        item.needs.clear();
+        item.needs = item.needs_end;
     }
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS
@@ -744,17 +779,21 @@ PyObject *plan_prepare(PyObject *self, PyObject *args)
 PyObject *plan_commit(PyObject *self, PyObject *args)
 {
     Py_ssize_t first, end;
+    Plan *plan = reinterpret_cast<Plan *>(self);
     Batch *b = batch_of(self, args, &first, &end);
     if (b == nullptr)
         return nullptr;
     for (Py_ssize_t i = first; i < end; ++i) {
-        Item &item = b->items[i];
-        item.kept.clear();
-        for (int j = 0; j < item.swaps; ++j)
-            if (item.swap[j].value == nullptr) {
+        Record &item = b->items[i];
+        item.grad.reset();
+        item.scratch.reset();
+        for (uint32_t j = item.held; j < item.held_end; ++j)
+            Py_CLEAR((*plan->held)[j]);
+        for (uint32_t j = item.swaps; j < item.swaps_end; ++j)
+            if (b->swaps[j].value == nullptr) {
                 PyErr_SetString(PyExc_RuntimeError, "records that were not prepared");
                 return nullptr;
-            } else if (PyDict_SetItem(item.swap[j].dict, item.swap[j].key, item.swap[j].value) != 0) {
+            } else if (PyDict_SetItem(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value) != 0) {
                 return nullptr;
             }
     }
@@ -794,6 +833,8 @@ PyObject *collect(PyObject *, PyObject *args)
     try {
         plan->batches = new std::vector<Batch>();
         plan->held = new std::vector<PyObject *>();
+        plan->others = new std::vector<PyObject *>();
+        plan->held->reserve(8 * PyList_GET_SIZE(params));
         plan->rest = PyList_New(0);
         if (plan->rest == nullptr)
             return nullptr;
