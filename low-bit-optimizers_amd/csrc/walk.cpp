@@ -700,6 +700,13 @@ PyObject *plan_start(PyObject *self, PyObject *)
     for (Batch &b : *plan->batches) {
         const size_t bytes = kRecordBytes[b.kind];
         const bool has_step = b.kind != kSgd4 && b.kind != kSgdPlain;
+        // steps that stand for in-place operations of torch count as one for autograd's check of saved tensors
+        if (b.kind == kSgdPlain || b.kind == kHalfPlain || (b.kind == kAny && b.flag == LPMM_RANK1_HALF))
+            for (const Record &item : b.items) {
+                const at::Tensor &p = THPVariable_Unpack((*plan->held)[item.held]);
+                if (!p.is_inference())
+                    p.unsafeGetTensorImpl()->bump_version();
+            }
         for (size_t i = 0; i < b.items.size() && has_step; ++i) {
             const float step = *b.items[i].step += 1.0f;
             // every record ends in  float step  and four more bytes

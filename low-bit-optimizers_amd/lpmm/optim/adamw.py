@@ -24,7 +24,7 @@ import torch
 
 from .. import _native
 from ..functional import RANK1_ND_MAX, _ptr_array, _shape_array, code_table, packed_nbytes, vectorwise_dequant, vectorwise_quant, whole_codes
-from .optimizer import LowBitOptimizer
+from .optimizer import LowBitOptimizer, count_as_modified
 
 __all__ = ["AdamW"]
 
@@ -633,6 +633,8 @@ class AdamW(LowBitOptimizer):
                     continue
                 key = (p.device, state["exp_avg_qstate"]["qmap"].data_ptr(),
                        state["exp_avg_sq_qstate"]["qmap"].data_ptr())
+                if kind in ("plain", "any"):
+                    count_as_modified(p)
                 if kind == "plain":
                     for name in ("exp_avg", "exp_avg_sq"):
                         if _is_placeholder(state[name]):

@@ -23,6 +23,13 @@ def _quantize_enabled(p, prior_enable, threshold):
     return True
 
 
+def count_as_modified(p):
+    """Autograd's count of a parameter's in-place modifications, for steps that stand for torch's operations and write
+    through a pointer: a backward pass over what was saved before the step has to fail, as it does behind those."""
+    if not p.is_inference():
+        torch.autograd.graph.increment_version(p)
+
+
 class LowBitOptimizer(torch.optim.Optimizer):
     def __init__(self, params, defaults, config):
         super().__init__(params, defaults)

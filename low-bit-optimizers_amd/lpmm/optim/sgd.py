@@ -18,7 +18,7 @@ import torch
 
 from .. import _native
 from ..functional import packed_nbytes, vectorwise_dequant, vectorwise_quant, whole_codes
-from .optimizer import LowBitOptimizer
+from .optimizer import LowBitOptimizer, count_as_modified
 
 __all__ = ["SGD"]
 
@@ -93,6 +93,7 @@ class SGD(LowBitOptimizer):
                         buf = torch.empty_like(p, memory_format=torch.contiguous_format)
                     if buf.dtype is torch.float32 and buf.is_contiguous() and buf.shape == p.shape and buf.device == p.device:
                         state["momentum_buffer"] = buf
+                        count_as_modified(p)
                         plain.setdefault(p.device, []).append(
                             (p.data_ptr(), p.grad.data_ptr(), buf.data_ptr(), p.numel(), 1 if first else 0, 0))
                         continue

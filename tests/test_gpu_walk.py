@@ -338,3 +338,23 @@ def test_a_step_holds_one_launch_of_new_arrays(case, shape, walk, monkeypatch):
     codes = sum(t.numel() for p in params for t in opt.state[p].values() if torch.is_tensor(t) and t.dtype is torch.int8)
     assert codes > 10 << 20 and grown <= codes // 4, (grown, codes)
     assert torch.cuda.memory_allocated() <= before
+
+
+@pytest.mark.parametrize("kind", ["sgd", "half vector", "half matrix"])
+def test_backward_over_tensors_saved_before_a_step_fails(kind):
+    """Steps that stand for a chain of torch's in-place operations count as a modification of the parameter: on the first step
+    and on later ones."""
+    import lpmm
+
+    dtype = torch.float32 if kind == "sgd" else torch.float16
+    p = torch.nn.Parameter(torch.full((70, 61) if kind == "half matrix" else (70,), 0.5, device="cuda", dtype=dtype))
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    opt = (lpmm.optim.SGD([p], lr=1e-2, momentum=0.9) if kind == "sgd" else lpmm.optim.AdamW([p], lr=1e-2, eps=1e-3, qconfig=path))
+    for _ in range(3):
+        before = p._version
+        loss = (p * p).sum()
+        p.grad = torch.full_like(p, 0.1)
+        opt.step()
+        assert p._version > before
+        with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+            loss.backward()
