@@ -4,6 +4,7 @@ There is no fallback: if the library is missing or a call fails, a RuntimeError 
 """
 import ctypes
 import os
+import warnings
 
 import numpy as np
 
@@ -151,15 +152,30 @@ def lib():
 _walk = None
 
 
+class _NoWalk:
+    """What stands for the host walk where its module does not load: it serves no tensor, and the optimizers' Python loops
+    take them all, to the same kernels."""
+
+    served = False
+
+    def __init__(self, rest=()):
+        self.rest = rest
+
+    def collect(self, is_sgd, params, *_):
+        return _NoWalk(params)
+
+
 def walk():
-    """The host walk (csrc/walk.cpp, an extension module); raises RuntimeError when it has not been built."""
+    """The host walk (csrc/walk.cpp): an extension module, built against one version of torch and of Python.  Without it, or
+    under another version, steps take the Python loops, with a warning."""
     global _walk
     if _walk is None:
         try:
             from . import _walk as module
         except ImportError as e:
-            raise RuntimeError("lpmm: the extension module lpmm/_walk.so is missing or does not load. Build it with "
-                               "`make -C low-bit-optimizers_amd/csrc`.") from e
+            warnings.warn(f"lpmm: the extension module lpmm/_walk.so does not load ({e}); optimizer steps walk their tensors in "
+                          "Python, 3 to 15 us a tensor. Build it with `make -C low-bit-optimizers_amd/csrc`.", RuntimeWarning)
+            module = _NoWalk()
         _walk = module
     return _walk
 

@@ -1,5 +1,6 @@
 """The host walk (csrc/walk.cpp) where no GPU is needed."""
 import struct
+import sys
 
 import pytest
 import torch
@@ -34,3 +35,21 @@ def test_a_group_size_that_nothing_reads(group_size):
                                                         SQM=dict(SCALE_TYPE=dict(DEFAULT="rank1")))))
     assert opt.step() is None
     assert lpmm.optim.adamw._Routes(*map(opt.get_qmetadata_by_state_name, ("exp_avg", "exp_avg_sq"))).m_group == 0
+
+
+def test_steps_without_the_module(monkeypatch):
+    """Where the module does not load (another version of torch or Python), one warning is given and the Python loops take
+    every tensor: SGD on tensors in host memory, which needs no library at all."""
+    monkeypatch.setattr(_native, "_walk", None)
+    monkeypatch.setattr(lpmm, "_walk", None, raising=False)
+    monkeypatch.delattr(lpmm, "_walk")
+    monkeypatch.setitem(sys.modules, "lpmm._walk", None)
+    p, q = (torch.nn.Parameter(torch.arange(1.0, 8.0)) for _ in range(2))
+    ours, torchs = lpmm.optim.SGD([p], lr=0.1, momentum=0.9), torch.optim.SGD([q], lr=0.1, momentum=0.9)
+    with pytest.warns(RuntimeWarning, match="_walk.so does not load") as warned:
+        for step in range(3):
+            p.grad, q.grad = torch.full((7,), 1.0 + step), torch.full((7,), 1.0 + step)
+            ours.step()
+            torchs.step()
+    assert len(warned) == 1 and torch.allclose(p, q)
+    assert lpmm.optim.AdamW([torch.nn.Parameter(torch.zeros(3))]).step() is None
