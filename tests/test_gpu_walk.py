@@ -358,3 +358,45 @@ def test_backward_over_tensors_saved_before_a_step_fails(kind):
         assert p._version > before
         with pytest.raises(RuntimeError, match="modified by an inplace operation"):
             loss.backward()
+
+
+# (shape, configuration): both sides of every limit that the walk and the loops' routes share
+LIMITS = [((32768, 31), "default.yml"), ((32769, 31), "default.yml"), ((32769, 32), "default.yml"), ((32769, 33), "default.yml"),
+          ((32768, 31), "2nd_moment_only_default.yml"), ((32769, 31), "2nd_moment_only_default.yml"),
+          ((32768, 31), "default_8b.yml"), ((32769, 31), "default_8b.yml"), ((32769, 24), "1st_moment_group_256.yml"),
+          ((15, 64, 1093), "default.yml"), ((15, 64, 1092), "default.yml"), ((16, 64, 1093), "default.yml"),  # 2^20 values, 16 rows
+          ((16, 8, 8184), "default.yml"), ((16, 8, 8185), "default.yml"),  # 8192 statistics of the trailing dimensions
+          ((16, 256, 256), "default.yml"), ((16, 256, 257), "default.yml"), ((32, 255, 257), "default.yml"),  # 2^16 trailing values
+          ((2,) * 13, "default.yml"), ((3, 3, 3, 3, 3, 3, 3, 3), "default.yml"), ((3, 3, 3, 3, 3, 3, 3, 3, 3), "default.yml"),
+          ((64, 192), "default.yml"), ((63, 192), "default.yml"), ((4097,), "default.yml"), ((4096,), "default.yml")]
+
+
+@pytest.mark.parametrize("shape,config", LIMITS)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_walk_and_loops_choose_one_route_at_the_limits(shape, config, dtype, monkeypatch):
+    """A step by the walk leaves what a step by the loops leaves, in the same arrays' shapes, on either side of each limit."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    gen = torch.Generator(device="cuda").manual_seed(31)
+    start = (torch.randn(shape, device="cuda", generator=gen) * 0.1).to(dtype)
+    sides = []
+    for _ in range(2):
+        p = torch.nn.Parameter(start.clone())
+        sides.append((p, lpmm.optim.AdamW([p], lr=1e-2, eps=1e-3, qconfig=path)))
+    for step in range(4):
+        g = (torch.randn(shape, device="cuda", generator=gen) * 0.1).to(dtype)
+        for serve, (p, opt) in zip((True, False), sides):
+            p.grad = g
+            with monkeypatch.context() as patch:
+                patch.setattr(adamw, "_native", _Native(_native, serve))
+                opt.step()
+    (p, a), (q, b) = sides
+    assert torch.equal(p, q)
+    x, y = _state(a, p), _state(b, q)
+    assert x.keys() == y.keys()
+    for k in x:
+        assert x[k].shape == y[k].shape and x[k].dtype == y[k].dtype, k
+        assert torch.equal(x[k].nan_to_num(), y[k].nan_to_num()) if x[k].is_floating_point() else torch.equal(x[k], y[k]), k
