@@ -176,8 +176,8 @@ __device__ __forceinline__ float half_quotient(float x, h16 dh)
 // The parameter of two elements from their updated moments.  The root of a half rounded to half lies at
 // least 0.5 ulp of a float away from a tie, and the hardware's float root (1 ulp) rounds to the same half as
 // the correctly rounded one for every half (all of them are compared by the tests).  IEEE: divisions as the
-// compiler writes them, for kernels that arithmetic does not bound: infinite second moments (a gradient above 255
-// squares to one) divide as in the chain too.
+// compiler writes them, for kernels that arithmetic does not bound: infinite second moments (with beta2 = 0.999
+// gradients above 8090, where (1 - beta2) g^2 passes 65504) divide as in the chain too.
 template <bool ZERO, bool IEEE>
 __device__ __forceinline__ v2h half_param(v2h p, v2h m, v2h v, const NfHyper &h, const MixConst &c)
 {

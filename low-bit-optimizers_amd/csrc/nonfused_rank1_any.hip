@@ -1,7 +1,7 @@
 // The two passes of the non-fused AdamW step with a rank-1 second moment for any column count and any
 // alignment, for every kind of state and parameter the tuned kernels serve: 4-bit states (what
 // nonfused_rank1_ragged.hip leaves: columns that are no multiple of 8), an fp32 first moment, 5-8-bit
-// codes and float16 parameters on columns that are no multiple of 128.  Tiles, records and statistics
+// codes and float16 parameters on columns that are no multiple of 128, operands off a 16-byte boundary.  Tiles, records and statistics
 // as in nonfused_rank1.hip.
 //
 // What the tuned kernels rely on and these do not: rows that start on a 16-byte boundary and on a whole

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(kSgdThreads) void sgd4bit_kernel(const MultiSgd arg
 // ---------------------------------------------------------------------------------------
 // The same chain on a float buffer: tensors whose buffer is not quantised (4096 values or fewer
 // by default: biases, norm weights).  As three or four torch operations each they took most of a
-// small model's step -- host time and launches, not bytes (the 51 vectors of a wide ResNet-152 among its 254
+// small model's step -- host time and launches, not bytes (the 51 vectors of a wide ResNet-152 among its 203
 // tensors: 150 launches and 0.25 ms of GPU time one after another; in one launch the whole step goes from
 // 1110-1120 to 466-470 us).  One tile
 // of 1024 values per workgroup: the tensors are short, and four values a thread are one 16-byte

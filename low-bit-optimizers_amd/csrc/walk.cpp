@@ -2,7 +2,7 @@
 // that writes the records of the multi-tensor launches.  In Python the same walk is dozens of attribute and
 // dictionary reads a tensor -- 3 to 15 us a tensor, against 0.4 here, while the kernels take 1 us for a tensor of a
 // million values -- and bound every model of small tensors: fifty tensors of a few thousand to a million values
-// 186 -> 43 us a step, the 254 of a wide ResNet-152 1634 -> 1054, GPT-2-XL's 580 1.8 -> 0.23 ms of host time.
+// 186 -> 43 us a step, the 203 of a wide ResNet-152 1634 -> 1054, GPT-2-XL's 580 1.8 -> 0.23 ms of host time.
 // lpmm/optim/adamw.py and sgd.py keep that walk for what is not served here: first steps, other data types,
 // strided operands, other routes; and for every error.
 //
