@@ -560,10 +560,10 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
     }
 }
 
-void launch_rank1_half(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v, hipStream_t stream)
+void launch_rank1_half(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream)
 {
-    hipLaunchKernelGGL(rank1_update_half_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_m, qmap_v);
-    hipLaunchKernelGGL(rank1_requant_half_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_m, qmap_v);
+    hipLaunchKernelGGL(rank1_update_half_kernel, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
+    hipLaunchKernelGGL(rank1_requant_half_kernel, dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, qmap_m, qmap_v);
 }
 
 // The maxima in the float work arrays, written out as the half statistics of the state.

@@ -25,33 +25,34 @@
 // LLaMA-7B shapes: a workgroup that walks through many passes is slower than the same accesses
 // made by short-lived workgroups in dispatch order (tiles of 1 or 2 passes run at the rate of
 // the one-shot fused step, 8 passes over 16 rows by 1024 columns 13 % below it), but short
-// tiles mean more column atomics and more tile set-up.  Tiles of 64 rows by 256 columns
-// (8 passes of 8 rows) are the best compromise for both kernels.  The row blocks that are
+// tiles mean more column atomics and more tile set-up.  Tiles are 256 columns wide and 16 to 64 rows tall, by pass and
+// by the size of the launch (pass_rows_policy).  The row blocks that are
 // resident together interleave their passes (block k of a group of `comb` blocks takes the rows
 // of pass i at (i * comb + k) * pass_rows), so that at any time a group works on one contiguous
 // band of the tensor instead of on `comb` bands a tile apart.  Together 2130 -> 1990 us (first
 // pass) and 770 -> 705 us (second pass) per launch of 8.4e8 elements.
 #include "rank1_tiles.hpp"
 
+#include <cstring>
+
 namespace lpmm {
 
-__global__ __launch_bounds__(kThreads) void rank1_clear_kernel(const MultiR1 args)
+// Zeroes the arrays that the first pass merges maxima into: the next statistics, and the next scales of first-moment
+// groups that are wider than 128 values or straddle rows.  Ranges of all tensors of a call in one launch (5 us each on an
+// otherwise idle stream), neighbours in memory joined.
+constexpr int kClearMax = 240;
+struct ClearRanges {
+    float *at[kClearMax];
+    int64_t n[kClearMax];
+};
+static_assert(sizeof(ClearRanges) <= 4096, "kernel arguments exceed 4 KB");
+
+__global__ __launch_bounds__(kThreads) void rank1_clear_kernel(const ClearRanges ranges)
 {
-    const TensorR1 &t = args.t[blockIdx.y];
-    const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
-    // first-moment groups that are wider than 128 values or straddle rows: their next scales are
-    // merged with atomic maxima as well
-    const int64_t group = (int64_t)kGroup << t.m_lg;
-    const int64_t m_groups = t.ms_new != nullptr ? (t.rows * cols + group - 1) / group : 0;
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < t.rows + cols + m_groups;
-         i += (int64_t)gridDim.x * kThreads) {
-        if (i < t.rows)
-            t.row_new[i] = 0.0f;
-        else if (i < t.rows + cols)
-            t.col_new[i - t.rows] = 0.0f;
-        else
-            t.ms_new[i - t.rows - cols] = 0.0f;
-    }
+    float *const at = ranges.at[blockIdx.y];
+    const int64_t n = ranges.n[blockIdx.y];
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+        at[i] = 0.0f;
 }
 
 // operands of one pass of a DPP row, as loaded
@@ -468,11 +469,44 @@ static uint64_t shape_tiles(int64_t rows, uint32_t col_blocks, TileShape &ts, ui
     const uint64_t row_blocks = (uint64_t)((rows + tile_rows - 1) / tile_rows);
     uint64_t comb = kPolicyResident / col_tiles;
     comb = comb < 1 ? 1 : comb;
-    comb = comb > row_blocks ? row_blocks : comb;
+    // groups of equal size, so that the last one holds few empty blocks (13 row blocks in groups of 5, not 6)
+    const uint64_t groups = (row_blocks + comb - 1) / comb;
+    comb = (row_blocks + groups - 1) / groups;
     ts.lg_wide = lg_wide;
     ts.tile_rows = tile_rows;
     ts.comb = (uint32_t)comb;
-    return (row_blocks + comb - 1) / comb * comb * col_tiles;  // whole groups: the last may hold empty blocks
+    return groups * comb * col_tiles;
+}
+
+// What a launch is, as far as its tile shapes depend on it.
+struct LaunchKind {
+    bool half_io, m32, bits;
+    double values;  // of all its tensors
+};
+
+// Rows of a pass's tiles on a matrix of `rows` rows.  A tile of fewer rows means more column atomics and more set-up, one of
+// more rows a longer walk, fewer workgroups and a longer end of the launch.  Measured (us; update pass, then second pass):
+//   * few values leave the chip idle with tall tiles.  2048 x 2048 alone: 64 rows 22.3 / 10.0, 32 rows 15.9 / 7.9, 16 rows
+//     14.2 / 7.3; 32 weights of 256 x 2304: 59 / 21, 52 / 22, 50 / 24; of 512 x 2048: 90 / 37, 87 / 35, 84 / 43; 24 of
+//     1600 x 6400 (246M values): 571 / 209, 560 / 218, 578 / 274.  So the second pass goes below 64 rows only under
+//     14M values, the update pass under 64M;
+//   * no more than 256 row blocks of 16 rows on a column: their atomics on one address queue up (8192 x 256 among 5.5M
+//     values: 16 rows 27.2, 32 rows 20.9);
+//   * larger launches: the update pass does best with 32 rows where a DPP row is a whole column block (LLaMA-7B decoder
+//     layers 1853 -> 1818), with 16 where the first moment is fp32 (a pass moves 20.5 instead of 13.5 bytes a value; a step of
+//     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold or codes are bytes
+//     (GPT-2-XL's set 5590 -> 5549 a step; 8 bits 2925 -> 2916).
+// The float16 passes are bound by their arithmetic: tall tiles spread a tile's set-up (four decoder layers of width 4096:
+// 32 rows 1821, 64 rows 1751, 128 rows 1729 a step).
+static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows)
+{
+    if (l.half_io)
+        return kPolicyRowsHalf;
+    if (requant)
+        return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 ? kPolicyRows / 2 : kPolicyRows;
+    if (l.values < 64e6)
+        return rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : kPolicyRows / 2;
+    return l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
 }
 
 // The first moment of a record: its codes and scales, or the fp32 moment itself.
@@ -489,7 +523,27 @@ static float *next_scales(const lpmm_rank1_mgroup_tensor &t) { return t.m_max1_n
 // a tensor that the kernels take as double rows
 static bool folds(int64_t rows, int64_t cols) { return cols % kGroup == 64 && rows % 2 == 0; }
 
-// Validation, batching into launches of at most kR1Max tensors, and the three launches.
+template <int MODE, bool FOLD>
+static void launch_rank1_passes(const R1Launch &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
+{
+    if (passes & 1)
+        hipLaunchKernelGGL((rank1_update_kernel<MODE, FOLD>), dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m,
+                           qmap_v);
+    if (passes & 2)
+        hipLaunchKernelGGL((rank1_requant_kernel<MODE == kMCodesWide, FOLD>), dim3(l.requant_tiles), dim3(kThreads), 0, stream,
+                           l.requant, qmap_m, qmap_v);
+}
+
+template <int MODE>
+static void launch_rank1(const R1Launch &l, bool folded, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
+{
+    if constexpr (MODE == kMCodes128)
+        if (folded)
+            return launch_rank1_passes<MODE, true>(l, qmap_m, qmap_v, passes, stream);
+    launch_rank1_passes<MODE, false>(l, qmap_m, qmap_v, passes, stream);
+}
+
+// Validation, batching into launches of at most kR1Max tensors, and the launches.
 // m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
 template <int MODE, class Record>
 static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
@@ -508,11 +562,6 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
     // served as double rows (rank1_tiles.hpp)
     const bool can_fold = MODE == kMCodes128 && bits_m == 4 && !half_io;
-    // rows per tile: with an fp32 first moment a pass moves 24.5 instead of 13.5 bytes per element, and
-    // tiles of half the rows do better (LLaMA-7B-shaped set 29.3 -> 28.6 ms per step); the passes on float16
-    // parameters are bound by their arithmetic, and taller tiles spread a tile's set-up over more rows (update
-    // and second pass of four decoder layers of width 4096: 1254 + 519 -> 1244 + 498 us)
-    const uint32_t policy_rows = M32 ? kPolicyRowsM32 : half_io ? kPolicyRowsHalf : kPolicyRows;
     // column counts that are no multiple of 128 (wide-group records only): every tensor of the call
     // then takes the kernels for ragged rows
     bool ragged = false;
@@ -569,8 +618,49 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             return LPMM_ERR_ARG;
     }
 
+    hipStream_t s = (hipStream_t)stream;
+    if (passes & 1) {
+        ClearRanges ranges;
+        int n = 0;
+        int64_t longest = 0;
+        const auto launch_clear = [&] {
+            const int64_t blocks = (longest + kThreads - 1) / kThreads;
+            if (n != 0)
+                hipLaunchKernelGGL(rank1_clear_kernel, dim3((uint32_t)(blocks > 64 ? 64 : blocks), (uint32_t)n), dim3(kThreads), 0,
+                                   s, ranges);
+            n = 0;
+            longest = 0;
+        };
+        const auto clear = [&](float *at, int64_t count_of) {
+            if (n != 0 && ranges.at[n - 1] + ranges.n[n - 1] == at) {
+                ranges.n[n - 1] += count_of;
+            } else {
+                if (n == kClearMax)
+                    launch_clear();
+                ranges.at[n] = at;
+                ranges.n[n++] = count_of;
+            }
+            longest = ranges.n[n - 1] > longest ? ranges.n[n - 1] : longest;
+        };
+        const int64_t group = (int64_t)kGroup << m_lg;
+        for (int64_t i = 0; i < count; ++i) {
+            const Record &t = tensors[i];
+            if (t.rows == 0 || t.cols == 0)
+                continue;
+            clear(t.v_rowmax_next, t.rows);
+            clear(t.v_colmax_next, t.cols);
+            if (next_scales(t) != nullptr)
+                clear(next_scales(t), (t.rows * t.cols + group - 1) / group);
+        }
+        launch_clear();
+        const int st = launch_status();
+        if (st != LPMM_OK)
+            return st;
+    }
+
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
-    MultiR1 args;
+    R1Launch l;
+    MultiR1 &args = l.update;
     args.decay = c.decay;
     args.w1 = c.w1;
     args.b2 = c.b2;
@@ -579,8 +669,17 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     int64_t i = 0;
     while (i < count) {
         int k = 0;
-        uint64_t tiles = 0;
-        int64_t longest = 0;
+        // what this launch will hold decides its tiles' rows
+        LaunchKind kind = {half_io, M32, bits_m != 4, 0};
+        for (int64_t j = i; j < count && k < kR1Max; ++j)
+            if (tensors[j].rows != 0 && tensors[j].cols != 0) {
+                kind.values += (double)tensors[j].rows * (double)tensors[j].cols;
+                ++k;
+            }
+        k = 0;
+        uint64_t tiles = 0, tiles2 = 0;
+        uint32_t start2[kR1Max + 1] = {0};
+        TileShape shape2[kR1Max];
         bool folded = false;  // does a tensor of this launch have folded rows
         args.tile_start[0] = 0;
         while (i < count && k < kR1Max) {
@@ -592,9 +691,11 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             const uint32_t col_blocks = (uint32_t)((t.cols + kGroup - 1) / kGroup);
             TensorR1 &d = args.t[k];
             const bool fold = t.cols % kGroup != 0 && can_fold;  // validated above: 64 modulo 128, even rows
-            const uint64_t nt = fold ? shape_tiles(t.rows / 2, 2 * col_blocks - 1, d.tile, policy_rows)
-                                     : shape_tiles(t.rows, col_blocks, d.tile, policy_rows);
-            if (tiles + nt > 0x7fffffffULL)
+            const int64_t rows = fold ? t.rows / 2 : t.rows;
+            const uint32_t blocks = fold ? 2 * col_blocks - 1 : col_blocks;
+            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows));
+            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows));
+            if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
             d.p = t.p;
             d.g = t.g;
@@ -614,10 +715,11 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             d.rbc2_sqrt = h.rbc2_sqrt;
-            longest = t.rows + t.cols > longest ? t.rows + t.cols : longest;
             tiles += nt;
+            tiles2 += nt2;
             folded = folded || fold;
             args.tile_start[++k] = (uint32_t)tiles;
+            start2[k] = (uint32_t)tiles2;
             ++i;
         }
         if (k == 0) {
@@ -626,40 +728,29 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             continue;
         }
         args.count = k;
-        for (int j = k + 1; j <= kR1Max; ++j)
+        for (int j = k + 1; j <= kR1Max; ++j) {
             args.tile_start[j] = (uint32_t)tiles;
-        hipStream_t s = (hipStream_t)stream;
-        int64_t clear_blocks = (longest + kThreads - 1) / kThreads;
-        clear_blocks = clear_blocks > 64 ? 64 : clear_blocks;
-        if (passes & 1)
-            hipLaunchKernelGGL(rank1_clear_kernel, dim3((uint32_t)clear_blocks, (uint32_t)k), dim3(kThreads), 0,
-                               s, args);
+            start2[j] = (uint32_t)tiles2;
+        }
+        l.requant = args;
+        for (int j = 0; j < k; ++j)
+            l.requant.t[j].tile = shape2[j];
+        memcpy(l.requant.tile_start, start2, sizeof start2);
+        l.update_tiles = (uint32_t)tiles;
+        l.requant_tiles = (uint32_t)tiles2;
         if (general) {
-            const AnyKind kind = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
-            launch_rank1_any(args, *out, (uint32_t)tiles, qmap_m, qmap_v, kind, bits_m, bits_v,
-                             static_cast<const uint32_t *>(table_m), static_cast<const uint32_t *>(table_v), passes, s);
+            const AnyKind any = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
+            launch_rank1_any(l, *out, qmap_m, qmap_v, any, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
+                             static_cast<const uint32_t *>(table_v), passes, s);
         } else if (half_io) {
-            launch_rank1_half(args, (uint32_t)tiles, qmap_m, qmap_v, s);
+            launch_rank1_half(l, qmap_m, qmap_v, s);
         } else if (ragged || (MODE == kMCodesWide && m_lg == 0)) {
-            launch_rank1_ragged(args, (uint32_t)tiles, qmap_m, qmap_v, s);
+            launch_rank1_ragged(l, qmap_m, qmap_v, s);
         } else if (bits_m != 4) {
-            launch_rank1_bits(args, (uint32_t)tiles, qmap_m, qmap_v, bits_m, bits_v,
-                              static_cast<const uint32_t *>(table_m), static_cast<const uint32_t *>(table_v),
-                              s);
-        } else if (MODE == kMCodes128 && folded) {
-            if (passes & 1)
-                hipLaunchKernelGGL((rank1_update_kernel<kMCodes128, true>), dim3((uint32_t)tiles), dim3(kThreads), 0,
-                                   s, args, qmap_m, qmap_v);
-            if (passes & 2)
-                hipLaunchKernelGGL((rank1_requant_kernel<false, true>), dim3((uint32_t)tiles), dim3(kThreads), 0,
-                                   s, args, qmap_m, qmap_v);
+            launch_rank1_bits(l, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
+                              static_cast<const uint32_t *>(table_v), s);
         } else {
-            if (passes & 1)
-                hipLaunchKernelGGL((rank1_update_kernel<MODE, false>), dim3((uint32_t)tiles), dim3(kThreads), 0,
-                                   s, args, qmap_m, qmap_v);
-            if (passes & 2)
-                hipLaunchKernelGGL((rank1_requant_kernel<MODE == kMCodesWide, false>), dim3((uint32_t)tiles),
-                                   dim3(kThreads), 0, s, args, qmap_m, qmap_v);
+            launch_rank1<MODE>(l, MODE == kMCodes128 && folded, qmap_m, qmap_v, passes, s);
         }
         const int st = launch_status();
         if (st != LPMM_OK)

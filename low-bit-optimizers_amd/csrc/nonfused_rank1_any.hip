@@ -609,32 +609,32 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
 }
 
 template <typename REAL, bool M32, bool BITS>
-static void launch(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v, int bits_m, int bits_v,
+static void launch(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v, int bits_m, int bits_v,
                    const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
 {
     if (passes & 1)
-        hipLaunchKernelGGL((rank1_update_any_kernel<REAL, M32, BITS>), dim3(tiles), dim3(kThreads), 0, stream, args, out, qmap_m,
-                           qmap_v, bits_m, bits_v);
+        hipLaunchKernelGGL((rank1_update_any_kernel<REAL, M32, BITS>), dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, out,
+                           qmap_m, qmap_v, bits_m, bits_v);
     if (passes & 2)
-        hipLaunchKernelGGL((rank1_requant_any_kernel<REAL, M32, BITS>), dim3(tiles), dim3(kThreads), 0, stream, args, out, qmap_m,
-                           qmap_v, bits_m, bits_v, table_m, table_v);
+        hipLaunchKernelGGL((rank1_requant_any_kernel<REAL, M32, BITS>), dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, out,
+                           qmap_m, qmap_v, bits_m, bits_v, table_m, table_v);
 }
 
-void launch_rank1_any(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v, AnyKind kind, int bits_m,
-                      int bits_v, const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
+void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v, AnyKind kind, int bits_m, int bits_v,
+                      const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
 {
     switch (kind) {
     case kAnyCodes4:
-        launch<float, false, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<float, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
         break;
     case kAnyFloatM:
-        launch<float, true, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<float, true, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
         break;
     case kAnyBits:
-        launch<float, false, true>(args, out, tiles, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
+        launch<float, false, true>(l, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
         break;
     case kAnyHalf:
-        launch<h16, false, false>(args, out, tiles, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<h16, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
         break;
     }
 }

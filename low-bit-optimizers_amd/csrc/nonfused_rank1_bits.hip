@@ -280,12 +280,12 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_bits_kernel(const Mult
     }
 }
 
-void launch_rank1_bits(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v, int bits_m,
+void launch_rank1_bits(const R1Launch &l, const float *qmap_m, const float *qmap_v, int bits_m,
                        int bits_v, const uint32_t *table_m, const uint32_t *table_v, hipStream_t stream)
 {
-    hipLaunchKernelGGL(rank1_update_bits_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_m, qmap_v, bits_m,
+    hipLaunchKernelGGL(rank1_update_bits_kernel, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v, bits_m,
                        bits_v, table_m);
-    hipLaunchKernelGGL(rank1_requant_bits_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_v, bits_v, table_v);
+    hipLaunchKernelGGL(rank1_requant_bits_kernel, dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, qmap_v, bits_v, table_v);
 }
 
 }  // namespace lpmm

@@ -286,11 +286,10 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_ragged_kernel(const Mu
     }
 }
 
-void launch_rank1_ragged(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v,
-                         hipStream_t stream)
+void launch_rank1_ragged(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream)
 {
-    hipLaunchKernelGGL(rank1_update_ragged_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_m, qmap_v);
-    hipLaunchKernelGGL(rank1_requant_ragged_kernel, dim3(tiles), dim3(kThreads), 0, stream, args, qmap_m, qmap_v);
+    hipLaunchKernelGGL(rank1_update_ragged_kernel, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
+    hipLaunchKernelGGL(rank1_requant_ragged_kernel, dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, qmap_m, qmap_v);
 }
 
 }  // namespace lpmm

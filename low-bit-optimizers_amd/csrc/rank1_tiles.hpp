@@ -23,7 +23,6 @@ constexpr int kR1Max = 32;               // tensors per launch
 #endif
 constexpr int kPolicyLgWide = LPMM_R1_LG;
 constexpr uint32_t kPolicyRows = LPMM_R1_ROWS, kPolicyResident = LPMM_R1_RESIDENT;
-constexpr uint32_t kPolicyRowsM32 = LPMM_R1_ROWS / 2;  // fp32 first moment
 constexpr uint32_t kPolicyRowsHalf = LPMM_R1_ROWS * 2;  // float16 parameters
 constexpr uint32_t kPolicyRowsMost = kPolicyRowsHalf;
 static_assert(LPMM_R1_LG >= 1 && LPMM_R1_LG <= 3, "a tile is 256 to 1024 columns wide at most");
@@ -179,7 +178,7 @@ __device__ __forceinline__ void fold_rows(const Fold &f, int64_t r, uint32_t cg,
 // set 21.23 -> 20.85 ms per step, GPT-2-XL-shaped set 6.30 -> 5.71 ms).
 constexpr int kRowSlots = 2 * (int)kPolicyRowsMost;
 static_assert(kRowSlots <= kThreads, "one thread per row slot");
-static_assert(kPolicyRows >= (uint32_t)kDppRows, "a tile holds the policy's rows: one slot pair per row");
+static_assert(kPolicyRows / 4 >= (uint32_t)kDppRows, "a tile holds the policy's rows: one slot pair per row");
 
 __device__ __forceinline__ int row_slot(const TileShape &ts, int pass, int drow)
 {
@@ -211,11 +210,16 @@ __device__ __forceinline__ void write_padding(uint8_t *codes, int64_t n, int64_t
         codes[n_padded / 2] = 0;
 }
 
-// The launches of the other kernel families (defined next to their kernels); tiles = workgroups.
-void launch_rank1_bits(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v, int bits_m,
+// One launch's tensors with the tile shapes of either pass (they differ: pass_rows_policy), and its workgroups.
+struct R1Launch {
+    MultiR1 update, requant;
+    uint32_t update_tiles, requant_tiles;
+};
+
+// The launches of the other kernel families (defined next to their kernels).
+void launch_rank1_bits(const R1Launch &l, const float *qmap_m, const float *qmap_v, int bits_m,
                        int bits_v, const uint32_t *table_m, const uint32_t *table_v, hipStream_t stream);
-void launch_rank1_ragged(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v,
-                         hipStream_t stream);
+void launch_rank1_ragged(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream);
 // any column count and alignment (nonfused_rank1_any.hip)
 enum AnyKind : int {
     kAnyCodes4 = LPMM_RANK1_CODES4,
@@ -227,11 +231,11 @@ struct NewCodes {  // where the second pass puts a tensor's codes
     uint8_t *m[kR1Max], *v[kR1Max];
 };
 // passes: 1 the first, 2 the second, 3 both
-void launch_rank1_any(const MultiR1 &args, const NewCodes &out, uint32_t tiles, const float *qmap_m, const float *qmap_v,
+void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v,
                       AnyKind kind, int bits_m, int bits_v, const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream);
 // float16 parameters (nonfused_half.hip): p, g, the first moment's scales and the current statistics
 // of the records point at halfs, the next statistics at float work arrays
-void launch_rank1_half(const MultiR1 &args, uint32_t tiles, const float *qmap_m, const float *qmap_v, hipStream_t stream);
+void launch_rank1_half(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream);
 // the records of lpmm_nonfused_adamw_rank1_any_step_multi; float16: the next statistics and scales of the records are
 // float work arrays (rank1_any_half sets them up and writes the halfs out)
 int rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg, const float *qmap_m,
