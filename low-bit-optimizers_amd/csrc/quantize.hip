@@ -8,7 +8,7 @@
 // 16 lanes) and, for larger groups, 16 floats of LDS per workgroup.  Code assignment uses
 // the table / closed-form encoders of lpmm_codec.hpp when the map is one of the two
 // standard ones and the count-of-midpoints search otherwise.
-#include "lpmm_codec.hpp"
+#include "rank1_rows.hpp"
 
 namespace lpmm {
 
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(kQThreads) void dequant_group_kernel(const uint8_t 
 
 // Row layout (as in the fused step): 16 lanes own one 128-value group, lane l owns values
 // [4l, 4l+4) and [64+4l, 64+4l+4), so that every 16-byte store of a row covers whole cache
-// lines.  Handles the groups that lie fully inside the tensor; n must be >= 128.
+// lines; the values behind the last whole group go element by element.  n must be >= 128.
 #ifndef LPMM_DQ_LDS_KB
 #define LPMM_DQ_LDS_KB 0
 #endif
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(kQThreads) void dequant_group_rows_kernel(const uin
                                                                        const float *__restrict__ max1,
                                                                        const float *__restrict__ qmap,
                                                                        int64_t full_groups, int rows_per_group,
-                                                                       float *__restrict__ out)
+                                                                       int64_t n, float *__restrict__ out)
 {
     __shared__ __align__(16) uint32_t lds[kDequantLdsWords];
     const int lane16 = threadIdx.x & 15;
@@ -307,6 +307,18 @@ __global__ __launch_bounds__(kQThreads) void dequant_group_rows_kernel(const uin
         store4(o, make_float4(v[0], v[1], v[2], v[3]));
         store4(o + 64, make_float4(v[4], v[5], v[6], v[7]));
     }
+    // the values behind the last whole group: in the last workgroup instead of a launch of their own (80 million values and
+    // 64: 62 + 5 -> 62 us)
+    const int64_t base = full_groups * kGroup + threadIdx.x * kQElts;
+    if (blockIdx.x == gridDim.x - 1 && base < n) {
+        const Nibbles nb = split_nibbles(load_codes8(codes, base, n, false));
+        const float scale = max1[full_groups / rows_per_group];
+        float v[kQElts];
+#pragma unroll
+        for (int k = 0; k < kQElts; ++k)
+            v[k] = decode_nibble(lds, kLdsQ0, nb, k) * scale;
+        store8(out, base, n, false, v);
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -321,115 +333,108 @@ __global__ void fill_zero_kernel(float *__restrict__ a, int64_t na, float *__res
         b[i] = 0.0f;
 }
 
-constexpr int kStatRows = 64;
-constexpr int kStatCols = 1024;  // 256 threads x 4 columns
-constexpr int kStatUnroll = 8;   // rows in flight per lane
+// One workgroup takes batches of 32 rows (more where a row needs fewer than 64 lanes) of a tile of up to 256 columns; a wave issues
+// eight rows' loads at once, keeps its lanes' column maxima over the batches, and the waves' column maxima meet in LDS: one
+// atomic per column and tile (a maximum is exact and order-free).  Atomics on one address are served one after the other, about
+// 18 ns each, so a column may have one tile per 40000 values of the tensor at most: half the time that reading them takes.  One
+// batch a tile where that allows it: the many small workgroups then keep the memory system busy the way a plain streaming read does.
+// Measured, against one batch a tile of 256 columns and (40000 x 1601) a kernel of 1024 columns with one load a value:
+// 524288 x 128 311.6 -> 56.0 us, 1000000 x 20 361.4 -> 25.2, 40000 x 1601 173.7 -> 58.3; 50257 x 1600 54.5 -> 55.0, 16384 x 4096
+// 46.6 -> 45.2.
+constexpr int kStatBatch = 8;                                    // loads of a lane in flight
+constexpr int kStatTileRows = (kQThreads / kWave) * kStatBatch;  // rows of a batch with one row a load
 
-// Tile of kStatRows x kStatCols; a lane keeps 4 column maxima in registers, row maxima are
-// reduced over the wave and merged with atomics (max is exact and order-independent).
-__global__ __launch_bounds__(kQThreads) void rank1_stats_kernel(const float *__restrict__ x, int64_t R,
-                                                                int64_t C, float *__restrict__ rowmax,
-                                                                float *__restrict__ colmax, bool vec)
+struct StatShape {
+    uint32_t tiles_x;  // column tiles
+    uint32_t lg_lanes; // lanes that share a row: a tile is 4 << lg_lanes columns wide
+    uint32_t batches;
+};
+
+template <bool VEC>
+__global__ __launch_bounds__(kQThreads) void rank1_stats_tile_kernel(const float *__restrict__ x, int64_t R, int64_t C,
+                                                                     const StatShape sh, float *__restrict__ rowmax,
+                                                                     float *__restrict__ colmax)
 {
-    const int64_t c0 = (int64_t)blockIdx.x * kStatCols + (int64_t)threadIdx.x * 4;
-    const int64_t r0 = (int64_t)blockIdx.y * kStatRows;
-    const int64_t r1 = (r0 + kStatRows < R) ? r0 + kStatRows : R;
-    const bool lane_vec = vec && c0 + 4 <= C;
+    __shared__ uint32_t s_col[4 * kWave];
+    const uint32_t ty = blockIdx.x / sh.tiles_x, tx = blockIdx.x - ty * sh.tiles_x;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const int lanes = 1 << sh.lg_lanes, sub = kWave >> sh.lg_lanes;
+    const int sl = lane & (lanes - 1), sr = lane >> sh.lg_lanes;
+    const int64_t tile_c0 = (int64_t)tx * (4 * lanes);
+    // VEC: four neighbouring columns a lane; otherwise four that lie `lanes` apart
+    const int64_t c0 = tile_c0 + (VEC ? sl * 4 : sl), c_step = VEC ? 1 : lanes;
+    const bool cols_in = c0 + 3 * c_step < C;
+    s_col[threadIdx.x] = 0u;
     float cm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int64_t rb = r0; rb < r1; rb += kStatUnroll) {
-        float a[kStatUnroll][4];
-        if (lane_vec && rb + kStatUnroll <= r1) {
-            // straight-line: all loads of the batch are in flight before the first use
-            float4 t[kStatUnroll];
+    for (uint32_t it = 0; it < sh.batches; ++it) {
+        const int64_t first = ((int64_t)ty * sh.batches + it) * (kStatTileRows * sub) + (int64_t)wave * (kStatBatch * sub);
+        if (first >= R)
+            break;
+        float a[kStatBatch][4];
+        if (cols_in && first + kStatBatch * sub <= R) {
+            const float *base = x + (first + sr) * C + c0;
+            const int64_t step = (int64_t)sub * C;
 #pragma unroll
-            for (int u = 0; u < kStatUnroll; ++u)
-                t[u] = load4(x + (rb + u) * C + c0);
+            for (int u = 0; u < kStatBatch; ++u) {
+                if (VEC) {
+                    const float4 t = load4(base + u * step);
+                    a[u][0] = t.x; a[u][1] = t.y; a[u][2] = t.z; a[u][3] = t.w;
+                } else {
 #pragma unroll
-            for (int u = 0; u < kStatUnroll; ++u) {
-                a[u][0] = fabsf(t[u].x); a[u][1] = fabsf(t[u].y); a[u][2] = fabsf(t[u].z); a[u][3] = fabsf(t[u].w);
+                    for (int k = 0; k < 4; ++k)
+                        a[u][k] = __builtin_nontemporal_load(base + u * step + k * c_step);
+                }
             }
         } else {
 #pragma unroll
-            for (int u = 0; u < kStatUnroll; ++u) {
-                const int64_t r = rb + u;
+            for (int u = 0; u < kStatBatch; ++u) {
+                const int64_t r = first + u * sub + sr;
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    a[u][k] = (r < r1 && c0 + k < C) ? fabsf(x[r * C + c0 + k]) : 0.0f;
+                    a[u][k] = (r < R && c0 + k * c_step < C) ? x[r * C + c0 + k * c_step] : 0.0f;
             }
         }
-        float rm[kStatUnroll];
+        float rm[kStatBatch];
 #pragma unroll
-        for (int u = 0; u < kStatUnroll; ++u) {
-            rm[u] = fmaxf(fmaxf(a[u][0], a[u][1]), fmaxf(a[u][2], a[u][3]));
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                cm[k] = fmaxf(cm[k], a[u][k]);
+        for (int u = 0; u < kStatBatch; ++u) {
+            const float a0 = fabsf(a[u][0]), a1 = fabsf(a[u][1]), a2 = fabsf(a[u][2]), a3 = fabsf(a[u][3]);
+            rm[u] = fmaxf(fmaxf(a0, a1), fmaxf(a2, a3));
+            cm[0] = fmaxf(cm[0], a0);
+            cm[1] = fmaxf(cm[1], a1);
+            cm[2] = fmaxf(cm[2], a2);
+            cm[3] = fmaxf(cm[3], a3);
         }
-        // the wave's 8 row maxima at once: lane 8u holds the maximum of row rb + u
-        static_assert(kStatUnroll == 8, "wave_max8 reduces eight rows");
-        const int lane = threadIdx.x & 63;
-        const float m = wave_max8(rm, lane);
-        if ((lane & 7) == 0 && rb + (lane >> 3) < r1)
-            atomic_max_nonneg(rowmax + rb + (lane >> 3), m);
+        if (lanes == kWave) {
+            const float m = wave_max8(rm, lane);  // lane 8u: maximum of row first + u over the tile's columns
+            const int64_t r = first + (lane >> 3);
+            if ((lane & 7) == 0 && r < R) {
+                if (sh.tiles_x == 1)
+                    rowmax[r] = m;
+                else
+                    atomic_max_nonneg(rowmax + r, m);
+            }
+        } else {
+            // a tile this narrow is the whole row
+            for (int o = lanes >> 1; o > 0; o >>= 1) {
+#pragma unroll
+                for (int u = 0; u < kStatBatch; ++u)
+                    rm[u] = fmaxf(rm[u], __shfl_xor(rm[u], o, kWave));
+            }
+#pragma unroll
+            for (int u = 0; u < kStatBatch; ++u) {
+                const int64_t r = first + u * sub + sr;
+                if (sl == (u & (lanes - 1)) && r < R)
+                    rowmax[r] = rm[u];
+            }
+        }
     }
+    lds_barrier();
 #pragma unroll
     for (int k = 0; k < 4; ++k)
-        if (c0 + k < C)
-            atomic_max_nonneg(colmax + c0 + k, cm[k]);
-}
-
-// The same statistics, one-shot: a workgroup takes a tile of 32 rows x 256 columns, a wave 8 of
-// those rows (a lane: 4 columns of each), and issues all its loads at once -- no loop, so the
-// grid's many small workgroups keep the memory system busy the way a plain streaming read does.
-// Column maxima of the four waves meet in LDS: one atomic per column and tile.  Requires whole
-// tiles' worth of vector access: 16-byte aligned x, columns a multiple of 4.
-constexpr int kStat2Rows = 32, kStat2Cols = 256;
-#ifndef LPMM_STAT2_LDS_KB
-#define LPMM_STAT2_LDS_KB 4
-#endif
-
-__global__ __launch_bounds__(kQThreads) void rank1_stats_tile_kernel(const float *__restrict__ x, int64_t R, int64_t C,
-                                                                     uint32_t tiles_x, float *__restrict__ rowmax,
-                                                                     float *__restrict__ colmax)
-{
-    __shared__ float s_col[LPMM_STAT2_LDS_KB * 256];  // [4 waves][256 columns] used; the rest caps residency
-    const uint32_t ty = blockIdx.x / tiles_x, tx = blockIdx.x - ty * tiles_x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t c0 = (int64_t)tx * kStat2Cols + lane * 4;
-    const int64_t r0 = (int64_t)ty * kStat2Rows + wave * 8;
-    const bool cols_in = c0 + 4 <= C;
-    float4 t[8];
-    if (cols_in && r0 + 8 <= R) {
-        const float *base = x + r0 * C + c0;
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            t[u] = load4(base + (int64_t)u * C);
-    } else {
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            t[u] = (cols_in && r0 + u < R) ? load4(x + (r0 + u) * C + c0) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    }
-    float rm[8], cm[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const float a0 = fabsf(t[u].x), a1 = fabsf(t[u].y), a2 = fabsf(t[u].z), a3 = fabsf(t[u].w);
-        rm[u] = fmaxf(fmaxf(a0, a1), fmaxf(a2, a3));
-        cm[0] = fmaxf(cm[0], a0);
-        cm[1] = fmaxf(cm[1], a1);
-        cm[2] = fmaxf(cm[2], a2);
-        cm[3] = fmaxf(cm[3], a3);
-    }
-    const float m = wave_max8(rm, lane);  // lane 8u: maximum of row r0 + u over the wave's 256 columns
-    if ((lane & 7) == 0 && r0 + (lane >> 3) < R)
-        atomic_max_nonneg(rowmax + r0 + (lane >> 3), m);
-    *reinterpret_cast<float4 *>(s_col + wave * kStat2Cols + lane * 4) = make_float4(cm[0], cm[1], cm[2], cm[3]);
-    __syncthreads();
-    const int64_t c = (int64_t)tx * kStat2Cols + threadIdx.x;
-    if (c < C) {
-        const float v = fmaxf(fmaxf(s_col[threadIdx.x], s_col[kStat2Cols + threadIdx.x]),
-                              fmaxf(s_col[2 * kStat2Cols + threadIdx.x], s_col[3 * kStat2Cols + threadIdx.x]));
-        atomic_max_nonneg(colmax + c, v);
-    }
+        atomicMax(s_col + (VEC ? sl * 4 + k : sl + k * lanes), __float_as_uint(cm[k]));
+    lds_barrier();
+    if (threadIdx.x < 4u * lanes && tile_c0 + threadIdx.x < C)
+        atomic_max_nonneg(colmax + tile_c0 + threadIdx.x, __uint_as_float(s_col[threadIdx.x]));
 }
 
 // Normalise by min(rowmax[r], colmax[c]), search, pack.  Flattened indexing: a lane's 8
@@ -513,18 +518,9 @@ __device__ __forceinline__ uint32_t encode8_rank1(const uint32_t *lds, int kind,
     return encode8_plain(lds, kLdsQ0, kind, xs);
 }
 
-// The same when C is a multiple of 8: a lane's 8 values lie in one row, the grid is
-// (column chunks, rows) and no index division is needed.  Workgroup (0,0) also writes the
-// pad codes past the tensor.
-constexpr int kR1Cols = kQThreads * kQElts;  // columns per workgroup
-
-#ifndef LPMM_R1_ROWS_PER_WG
-#define LPMM_R1_ROWS_PER_WG 4
-#endif
-constexpr int kR1RowsPerWg = LPMM_R1_ROWS_PER_WG;  // rows of one column chunk per workgroup: the column maxima are loaded once
-
-__global__ __launch_bounds__(kQThreads) void quant_rank1_rows_kernel(const float *__restrict__ x, int64_t R,
-                                                                     int64_t C, const float *__restrict__ rowmax,
+template <bool ONE>
+__global__ __launch_bounds__(kQThreads) void quant_rank1_rows_kernel(const float *__restrict__ x, int64_t R, int64_t C,
+                                                                     const RowShape sh, const float *__restrict__ rowmax,
                                                                      const float *__restrict__ colmax,
                                                                      const float *__restrict__ qmap,
                                                                      uint8_t *__restrict__ codes, int64_t n_padded)
@@ -532,83 +528,19 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_rows_kernel(const float
     constexpr int T = kR1RowsPerWg;
     __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
     const int64_t n = R * C;
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c = (int64_t)blockIdx.x * kR1Cols + (int64_t)threadIdx.x * kQElts;
-    const bool live = c < C;
-    // the lane's loads first, the LDS tables afterwards
-    float4 a[T], b[T], ca, cb;
-    float rm[T];
-    if (live) {
-        ca = *reinterpret_cast<const float4 *>(colmax + c);
-        cb = *reinterpret_cast<const float4 *>(colmax + c + 4);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                const float *p = x + (r0 + t) * C + c;
-                a[t] = load4(p);
-                b[t] = load4(p + 4);
-                rm[t] = rowmax[r0 + t];
-            }
-        }
-    }
-    lds_fill(lds, qmap, nullptr);
-    const int kind = classify_map(qmap);
-    lds_barrier();
-    if (blockIdx.x == 0 && blockIdx.y == 0) {
-        const float z[kQElts] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        const uint32_t wz = encode8_plain(lds, kLdsQ0, kind, z);
-        for (int64_t i = n + (int64_t)threadIdx.x * kQElts; i < n_padded; i += kR1Cols)
-            *reinterpret_cast<uint32_t *>(codes + (i >> 1)) = wz;
-        if (threadIdx.x == 0)
-            codes[n_padded / 2] = 0;
-    }
-    if (!live)
-        return;
-    const float cmx[kQElts] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
-    const ColRcp cr = col_rcp(cmx);
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
-            break;
-        const float v[kQElts] = {a[t].x, a[t].y, a[t].z, a[t].w, b[t].x, b[t].y, b[t].z, b[t].w};
-        store_u32(reinterpret_cast<uint32_t *>(codes + (((r0 + t) * C + c) >> 1)),
-                  encode8_rank1(lds, kind, v, cmx, cr, rm[t]));
-    }
-}
-
-// The same in the row layout of the fused step for column counts that are a multiple of 128:
-// 16 lanes own 128 consecutive columns of one row, lane l the columns [4l, 4l+4) and
-// [64+4l, 64+4l+4), so that every 16-byte load covers whole cache lines.
-__global__ __launch_bounds__(kQThreads) void quant_rank1_rows128_kernel(const float *__restrict__ x, int64_t R,
-                                                                        int64_t C, const float *__restrict__ rowmax,
-                                                                        const float *__restrict__ colmax,
-                                                                        const float *__restrict__ qmap,
-                                                                        uint8_t *__restrict__ codes, int64_t n_padded)
-{
-    constexpr int T = kR1RowsPerWg;
-    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
-    const int64_t n = R * C;
-    const int lane16 = threadIdx.x & 15;
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c0 = (int64_t)blockIdx.x * kR1Cols + (int64_t)(threadIdx.x >> 4) * kGroup;
-    const bool live = c0 < C;  // uniform over the 16 lanes of a group
+    const RowLane q = row_lane<ONE>(sh, C);
     // the small loads that feed LDS first (they return first), then the rows' loads
     const LdsFill fill = lds_fill_load(qmap, qmap);
     float4 a[T], b[T], ca, cb;
     float rm[T];
-    if (live) {
-        const float *cmp = colmax + c0 + lane16 * 4;
-        ca = *reinterpret_cast<const float4 *>(cmp);
-        cb = *reinterpret_cast<const float4 *>(cmp + 64);
+    ca = *reinterpret_cast<const float4 *>(colmax + q.c);
+    cb = *reinterpret_cast<const float4 *>(colmax + q.c2);
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                const float *p = x + (r0 + t) * C + c0 + lane16 * 4;
-                a[t] = load4(p);
-                b[t] = load4(p + 64);
-                rm[t] = rowmax[r0 + t];
-            }
-        }
+    for (int t = 0; t < T; ++t) {
+        const int64_t r_in = row_of<ONE>(q, sh, t), r = r_in < R ? r_in : R - 1;
+        a[t] = load4(x + r * C + q.c);
+        b[t] = load4(x + r * C + q.c2);
+        rm[t] = rowmax[r];
     }
     lds_fill_store(lds, fill);
     const int kind = classify_map(qmap);
@@ -616,24 +548,29 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_rows128_kernel(const fl
     if (blockIdx.x == 0 && blockIdx.y == 0) {
         const float z[kQElts] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         const uint32_t wz = encode8_plain(lds, kLdsQ0, kind, z);
-        for (int64_t i = n + (int64_t)threadIdx.x * kQElts; i < n_padded; i += kR1Cols)
+        // n is a multiple of 4 here: its first run of padding is half a word
+        if (threadIdx.x == 0 && n < n_padded && (n & 4) != 0)
+            *reinterpret_cast<uint16_t *>(codes + (n >> 1)) = (uint16_t)wz;
+        for (int64_t i = (n + 7) / 8 * 8 + (int64_t)threadIdx.x * kQElts; i < n_padded; i += kR1Cols)
             *reinterpret_cast<uint32_t *>(codes + (i >> 1)) = wz;
         if (threadIdx.x == 0)
             codes[n_padded / 2] = 0;
     }
-    if (!live)
+    if (!q.live)
         return;
     const float cmx[kQElts] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
     const ColRcp cr = col_rcp(cmx);
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
+        const int64_t r = row_of<ONE>(q, sh, t);
+        if (r >= R)
             break;
         const float v[kQElts] = {a[t].x, a[t].y, a[t].z, a[t].w, b[t].x, b[t].y, b[t].z, b[t].w};
         const uint32_t w = encode8_rank1(lds, kind, v, cmx, cr, rm[t]);
-        uint16_t *cp = reinterpret_cast<uint16_t *>(codes + (((r0 + t) * C + c0) >> 1)) + lane16;
+        uint16_t *cp = reinterpret_cast<uint16_t *>(codes + ((r * C + q.c) >> 1));
         store_u16(cp, w & 0xFFFFu);
-        store_u16(cp + 16, w >> 16);
+        if (q.second)
+            store_u16(cp + kRowHalf / 4, w >> 16);
     }
 }
 
@@ -672,102 +609,139 @@ __global__ __launch_bounds__(kQThreads) void dequant_rank1_kernel(const uint8_t 
     store8(out, base, n, vec, v);
 }
 
+// columns a multiple of 128: every lane that works has its second run
+template <bool ONE>
 __global__ __launch_bounds__(kQThreads) void dequant_rank1_rows_kernel(const uint8_t *__restrict__ codes,
                                                                        const float *__restrict__ rowmax,
                                                                        const float *__restrict__ colmax,
                                                                        const float *__restrict__ qmap, int64_t R,
-                                                                       int64_t C, float *__restrict__ out)
+                                                                       int64_t C, const RowShape sh, float *__restrict__ out)
 {
     constexpr int T = kR1RowsPerWg;
     __shared__ __align__(16) uint32_t lds[32];
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c = (int64_t)blockIdx.x * kR1Cols + (int64_t)threadIdx.x * kQElts;
-    const bool live = c < C;
-    uint32_t w[T];
-    float rm[T];
-    float4 ca, cb;
-    if (live) {
-        ca = *reinterpret_cast<const float4 *>(colmax + c);
-        cb = *reinterpret_cast<const float4 *>(colmax + c + 4);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                w[t] = load_u32(reinterpret_cast<const uint32_t *>(codes + (((r0 + t) * C + c) >> 1)));
-                rm[t] = rowmax[r0 + t];
-            }
-        }
-    }
-    if (threadIdx.x < 16)
-        lds[threadIdx.x] = __float_as_uint(qmap[threadIdx.x]);
-    lds_barrier();
-    if (!live)
-        return;
-    const float cmx[kQElts] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
-#pragma unroll
-    for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
-            break;
-        const Nibbles nb = split_nibbles(w[t]);
-        float v[kQElts];
-#pragma unroll
-        for (int k = 0; k < kQElts; ++k)
-            v[k] = decode_nibble(lds, kLdsQ0, nb, k) * ((cmx[k] < rm[t]) ? cmx[k] : rm[t]);
-        float *o = out + (r0 + t) * C + c;
-        store4(o, make_float4(v[0], v[1], v[2], v[3]));
-        store4(o + 4, make_float4(v[4], v[5], v[6], v[7]));
-    }
-}
-
-// Row layout variant for column counts that are a multiple of 128: 16 lanes own 128
-// consecutive columns of one row, lane l the columns [4l, 4l+4) and [64+4l, 64+4l+4), so that
-// every 16-byte store covers whole cache lines.
-__global__ __launch_bounds__(kQThreads) void dequant_rank1_rows128_kernel(const uint8_t *__restrict__ codes,
-                                                                          const float *__restrict__ rowmax,
-                                                                          const float *__restrict__ colmax,
-                                                                          const float *__restrict__ qmap, int64_t R,
-                                                                          int64_t C, float *__restrict__ out)
-{
-    constexpr int T = kR1RowsPerWg;
-    __shared__ __align__(16) uint32_t lds[kDequantLdsWords];
-    const int lane16 = threadIdx.x & 15;
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c0 = (int64_t)blockIdx.x * kR1Cols + (int64_t)(threadIdx.x >> 4) * kGroup;
-    const bool live = c0 < C;
+    const RowLane q = row_lane<ONE>(sh, C);
     uint32_t w0[T], w1[T];
     float rm[T];
     float4 ca, cb;
-    if (live) {
-        const float *cmp = colmax + c0 + lane16 * 4;
-        ca = *reinterpret_cast<const float4 *>(cmp);
-        cb = *reinterpret_cast<const float4 *>(cmp + 64);
+    ca = *reinterpret_cast<const float4 *>(colmax + q.c);
+    cb = *reinterpret_cast<const float4 *>(colmax + q.c2);
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                const uint16_t *cp = reinterpret_cast<const uint16_t *>(codes + (((r0 + t) * C + c0) >> 1)) + lane16;
-                w0[t] = load_u16(cp);
-                w1[t] = load_u16(cp + 16);
-                rm[t] = rowmax[r0 + t];
-            }
-        }
+    for (int t = 0; t < T; ++t) {
+        const int64_t r_in = row_of<ONE>(q, sh, t), r = r_in < R ? r_in : R - 1;
+        w0[t] = load_u16(reinterpret_cast<const uint16_t *>(codes + ((r * C + q.c) >> 1)));
+        w1[t] = load_u16(reinterpret_cast<const uint16_t *>(codes + ((r * C + q.c) >> 1)) + kRowHalf / 4);
+        rm[t] = rowmax[r];
     }
     if (threadIdx.x < 16)
         lds[threadIdx.x] = __float_as_uint(qmap[threadIdx.x]);
     lds_barrier();
-    if (!live)
+    if (!q.live)
         return;
     const float cmx[kQElts] = {ca.x, ca.y, ca.z, ca.w, cb.x, cb.y, cb.z, cb.w};
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
+        const int64_t r = row_of<ONE>(q, sh, t);
+        if (r >= R)
             break;
         const Nibbles nb = split_nibbles(w0[t] | (w1[t] << 16));
         float v[kQElts];
 #pragma unroll
         for (int k = 0; k < kQElts; ++k)
             v[k] = decode_nibble(lds, kLdsQ0, nb, k) * ((cmx[k] < rm[t]) ? cmx[k] : rm[t]);
-        float *o = out + (r0 + t) * C + c0 + lane16 * 4;
+        float *o = out + r * C + q.c;
         store4(o, make_float4(v[0], v[1], v[2], v[3]));
-        store4(o + 64, make_float4(v[4], v[5], v[6], v[7]));
+        store4(o + kRowHalf, make_float4(v[4], v[5], v[6], v[7]));
+    }
+}
+
+template <bool RUNS>
+__global__ __launch_bounds__(kQThreads) void quant_rank1_flat_kernel(const float *__restrict__ x, int64_t n, const FlatCols f,
+                                                                     const float *__restrict__ rowmax,
+                                                                     const float *__restrict__ colmax,
+                                                                     const float *__restrict__ qmap,
+                                                                     uint8_t *__restrict__ codes, int64_t n_padded)
+{
+    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    const int64_t b0 = (int64_t)flat_tile(x) * kFlatTile;
+    const bool whole = b0 + kFlatTile <= n;
+    const LdsFill fill = lds_fill_load(qmap, qmap);
+    float4 a[kFlatT];
+    FlatStats<RUNS> st[kFlatT];
+    flat_load<RUNS>(x, b0, n, whole, a);
+    flat_stats_of_tile<RUNS>(rowmax, colmax, b0, n, whole, f, st);
+    lds_fill_store(lds, fill);
+    const int kind = classify_map(qmap);
+    lds_barrier();
+    if (b0 == 0 && threadIdx.x == 0)
+        codes[n_padded / 2] = 0;
+#pragma unroll
+    for (int t = 0; t < kFlatT; t += 2) {
+        const int64_t i0 = b0 + t * kFlatPass + threadIdx.x * 4, i1 = i0 + kFlatPass;
+        const float v[kQElts] = {a[t].x, a[t].y, a[t].z, a[t].w, a[t + 1].x, a[t + 1].y, a[t + 1].z, a[t + 1].w};
+        float s[kQElts], xs[kQElts];
+        flat_scales<RUNS>(st[t], s);
+        flat_scales<RUNS>(st[t + 1], s + 4);
+        bool safe = kind != kMapGeneric;
+#pragma unroll
+        for (int k = 0; k < kQElts; ++k)
+            safe = safe && rc_safe(s[k]);
+        uint32_t w;
+        if (__all(safe)) {
+#pragma unroll
+            for (int k = 0; k < kQElts; ++k)
+                xs[k] = div_by_rc(v[k], s[k], rcp_exact(s[k]));
+            w = kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
+        } else {
+            // the values that pad the tensor are plain zeros
+#pragma unroll
+            for (int k = 0; k < kQElts; ++k) {
+                const int64_t i = (k < 4 ? i0 : i1) + (k & 3);
+                xs[k] = i < n ? v[k] / s[k] : 0.0f;
+            }
+            w = encode8_plain(lds, kLdsQ0, kind, xs);
+        }
+        if (whole || i0 < n_padded)
+            store_u16(reinterpret_cast<uint16_t *>(codes + (i0 >> 1)), w & 0xFFFFu);
+        if (whole || i1 < n_padded)
+            store_u16(reinterpret_cast<uint16_t *>(codes + (i1 >> 1)), w >> 16);
+    }
+}
+
+template <bool RUNS>
+__global__ __launch_bounds__(kQThreads) void dequant_rank1_flat_kernel(const uint8_t *__restrict__ codes, int64_t n,
+                                                                       const FlatCols f, const float *__restrict__ rowmax,
+                                                                       const float *__restrict__ colmax,
+                                                                       const float *__restrict__ qmap, float *__restrict__ out)
+{
+    __shared__ __align__(16) uint32_t lds[32];
+    const int64_t b0 = (int64_t)flat_tile(out) * kFlatTile;
+    const bool whole = b0 + kFlatTile <= n;
+    uint32_t w[kFlatT];
+    FlatStats<RUNS> st[kFlatT];
+#pragma unroll
+    for (int t = 0; t < kFlatT; ++t) {
+        const int64_t idx = b0 + t * kFlatPass + threadIdx.x * 4;
+        w[t] = 0;
+        if (whole || idx + 4 <= n)
+            w[t] = load_u16(reinterpret_cast<const uint16_t *>(codes + (idx >> 1)));
+        else if (!RUNS && idx < n)
+            w[t] = codes[idx >> 1] | (idx + 2 < n ? (uint32_t)codes[(idx >> 1) + 1] << 8 : 0u);
+    }
+    flat_stats_of_tile<RUNS>(rowmax, colmax, b0, n, whole, f, st);
+    if (threadIdx.x < 16)
+        lds[threadIdx.x] = __float_as_uint(qmap[threadIdx.x]);
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < kFlatT; t += 2) {
+        const Nibbles nb = split_nibbles(w[t] | (w[t + 1] << 16));
+        float s[kQElts], v[kQElts];
+        flat_scales<RUNS>(st[t], s);
+        flat_scales<RUNS>(st[t + 1], s + 4);
+#pragma unroll
+        for (int k = 0; k < kQElts; ++k)
+            v[k] = decode_nibble(lds, kLdsQ0, nb, k) * s[k];
+        flat_store<RUNS>(out, b0 + t * kFlatPass + threadIdx.x * 4, n, whole, v);
+        flat_store<RUNS>(out, b0 + (t + 1) * kFlatPass + threadIdx.x * 4, n, whole, v + 4);
     }
 }
 
@@ -879,18 +853,13 @@ extern "C" int lpmm_dequant_group(const uint8_t *codes, const float *max1, const
     const bool vec = aligned_to(out, 16) && aligned_to(codes, 4);
     const int64_t full_groups = n / kGroup;
     if (vec && full_groups > 0 && full_groups <= 0x7fffffffLL * 16) {
-        // whole 128-value rows in the row layout, the ragged tail (< 128 values) element-wise
 #ifndef LPMM_DQ_T
 #define LPMM_DQ_T 2
 #endif
         constexpr int kT = LPMM_DQ_T;  // passes of 16 rows per workgroup
         hipLaunchKernelGGL(dequant_group_rows_kernel<kT>, dim3((uint32_t)((full_groups + 16 * kT - 1) / (16 * kT))),
                            dim3(kQThreads), 0, (hipStream_t)stream, codes, max1, qmap, full_groups,
-                           (int)(gp_sz / kGroup), out);
-        const int64_t done = full_groups * kGroup;
-        if (done < n)
-            hipLaunchKernelGGL(dequant_group_kernel, dim3(1), dim3(kQThreads), 0, (hipStream_t)stream,
-                               codes + done / 2, max1 + done / gp_sz, qmap, n - done, gp_sz, out + done, false);
+                           (int)(gp_sz / kGroup), n, out);
         return launch_status();
     }
     hipLaunchKernelGGL(dequant_group_kernel, dim3(tiles), dim3(kQThreads), 0, (hipStream_t)stream, codes,
@@ -909,27 +878,31 @@ extern "C" int lpmm_rank1_stats(const float *x, int64_t rows, int64_t cols, floa
     LPMM_REQUIRE_ALIGN(x, 4);
     LPMM_REQUIRE_ALIGN(rowmax, 4);
     LPMM_REQUIRE_ALIGN(colmax, 4);
-    const int64_t gx = (cols + kStatCols - 1) / kStatCols, gy = (rows + kStatRows - 1) / kStatRows;
-    if (gx > 0x7fffffffLL || gy > 65535)
+    if ((cols + 1023) / 1024 > 0x7fffffffLL || (rows + 63) / 64 > 65535)
         return LPMM_ERR_SIZE;
     const int64_t mx = rows > cols ? rows : cols;
     hipLaunchKernelGGL(fill_zero_kernel, dim3((uint32_t)((mx + 255) / 256)), dim3(256), 0,
                        (hipStream_t)stream, rowmax, rows, colmax, cols);
-    const bool vec = aligned_to(x, 16) && (cols % 4) == 0;
-    const int64_t tx = (cols + kStat2Cols - 1) / kStat2Cols, ty = (rows + kStat2Rows - 1) / kStat2Rows;
-    if (vec && tx * ty <= 0x7fffffffLL)
-        hipLaunchKernelGGL(rank1_stats_tile_kernel, dim3((uint32_t)(tx * ty)), dim3(kQThreads), 0, (hipStream_t)stream,
-                           x, rows, cols, (uint32_t)tx, rowmax, colmax);
+    StatShape sh;
+    sh.lg_lanes = 6;
+    while (sh.lg_lanes > 0 && (4LL << (sh.lg_lanes - 1)) >= cols)
+        --sh.lg_lanes;
+    const int64_t tx = (cols + (4LL << sh.lg_lanes) - 1) / (4LL << sh.lg_lanes);
+    const int64_t batch_rows = (int64_t)kStatTileRows * (kWave >> sh.lg_lanes), row_batches = (rows + batch_rows - 1) / batch_rows;
+    // tiles on a column: see rank1_stats_tile_kernel
+    const int64_t most = rows * cols / 40000 > 256 ? rows * cols / 40000 : 256;
+    sh.tiles_x = (uint32_t)tx;
+    sh.batches = (uint32_t)((row_batches + most - 1) / most);
+    const int64_t tiles = tx * ((row_batches + sh.batches - 1) / sh.batches);
+    if (tiles > 0x7fffffffLL)
+        return LPMM_ERR_SIZE;
+    if (aligned_to(x, 16) && (cols % 4) == 0)
+        hipLaunchKernelGGL(rank1_stats_tile_kernel<true>, dim3((uint32_t)tiles), dim3(kQThreads), 0, (hipStream_t)stream, x, rows,
+                           cols, sh, rowmax, colmax);
     else
-        hipLaunchKernelGGL(rank1_stats_kernel, dim3((uint32_t)gx, (uint32_t)gy), dim3(kQThreads), 0,
-                           (hipStream_t)stream, x, rows, cols, rowmax, colmax, vec);
+        hipLaunchKernelGGL(rank1_stats_tile_kernel<false>, dim3((uint32_t)tiles), dim3(kQThreads), 0, (hipStream_t)stream, x, rows,
+                           cols, sh, rowmax, colmax);
     return launch_status();
-}
-
-// row-wise kernels: columns a multiple of 8, 16-byte aligned operands, rows fit grid.y
-static bool rank1_rows_ok(const void *x, const void *colmax, const void *codes, int64_t rows, int64_t cols)
-{
-    return (cols % 8) == 0 && rows <= 65535LL * kR1RowsPerWg && aligned_to(x, 16) && aligned_to(colmax, 16) && aligned_to(codes, 4);
 }
 
 extern "C" int lpmm_quant_rank1(const float *x, int64_t rows, int64_t cols, const float *rowmax,
@@ -952,15 +925,20 @@ extern "C" int lpmm_quant_rank1(const float *x, int64_t rows, int64_t cols, cons
     if (!tiles_ok(n, kQTile, &tiles))
         return LPMM_ERR_SIZE;
     const int64_t n_padded = (int64_t)tiles * kQTile;
-    if (rank1_rows_ok(x, colmax, codes, rows, cols)) {
-        const uint32_t gx = (uint32_t)((cols + kR1Cols - 1) / kR1Cols);
-        const uint32_t gy = (uint32_t)((rows + kR1RowsPerWg - 1) / kR1RowsPerWg);
-        if ((cols % kGroup) == 0)
-            hipLaunchKernelGGL(quant_rank1_rows128_kernel, dim3(gx, gy), dim3(kQThreads), 0,
-                               (hipStream_t)stream, x, rows, cols, rowmax, colmax, qmap, codes, n_padded);
+    RowShape sh;
+    dim3 rows_grid;
+    if (rank1_rows(x, colmax, codes, rows, cols, true, sh, rows_grid)) {
+        const auto kernel = sh.groups == 1 ? quant_rank1_rows_kernel<true> : quant_rank1_rows_kernel<false>;
+        hipLaunchKernelGGL(kernel, rows_grid, dim3(kQThreads), 0, (hipStream_t)stream, x, rows, cols, sh, rowmax,
+                           colmax, qmap, codes, n_padded);
+    } else if (rank1_flat_ok(x, colmax, codes, cols)) {
+        const dim3 grid((uint32_t)((n_padded + kFlatTile - 1) / kFlatTile));
+        if (cols % 4 == 0)
+            hipLaunchKernelGGL(quant_rank1_flat_kernel<true>, grid, dim3(kQThreads), 0, (hipStream_t)stream, x, n, flat_cols(cols),
+                               rowmax, colmax, qmap, codes, n_padded);
         else
-            hipLaunchKernelGGL(quant_rank1_rows_kernel, dim3(gx, gy), dim3(kQThreads), 0,
-                               (hipStream_t)stream, x, rows, cols, rowmax, colmax, qmap, codes, n_padded);
+            hipLaunchKernelGGL(quant_rank1_flat_kernel<false>, grid, dim3(kQThreads), 0, (hipStream_t)stream, x, n, flat_cols(cols),
+                               rowmax, colmax, qmap, codes, n_padded);
     } else {
         hipLaunchKernelGGL(quant_rank1_kernel, dim3(tiles), dim3(kQThreads), 0, (hipStream_t)stream, x, n, cols,
                            rowmax, colmax, qmap, codes, n_padded, aligned_to(x, 16));
@@ -986,16 +964,20 @@ extern "C" int lpmm_dequant_rank1(const uint8_t *codes, const float *rowmax, con
     uint32_t tiles;
     if (!tiles_ok(n, kQTile, &tiles))
         return LPMM_ERR_SIZE;
-    if (rank1_rows_ok(out, colmax, codes, rows, cols) && (cols % kGroup) == 0) {
-        const uint32_t gx = (uint32_t)((cols + kR1Cols - 1) / kR1Cols);
-        const uint32_t gy = (uint32_t)((rows + kR1RowsPerWg - 1) / kR1RowsPerWg);
-        hipLaunchKernelGGL(dequant_rank1_rows128_kernel, dim3(gx, gy), dim3(kQThreads), 0,
-                           (hipStream_t)stream, codes, rowmax, colmax, qmap, rows, cols, out);
-    } else if (rank1_rows_ok(out, colmax, codes, rows, cols)) {
-        const uint32_t gx = (uint32_t)((cols + kR1Cols - 1) / kR1Cols);
-        const uint32_t gy = (uint32_t)((rows + kR1RowsPerWg - 1) / kR1RowsPerWg);
-        hipLaunchKernelGGL(dequant_rank1_rows_kernel, dim3(gx, gy), dim3(kQThreads), 0,
-                           (hipStream_t)stream, codes, rowmax, colmax, qmap, rows, cols, out);
+    RowShape sh;
+    dim3 rows_grid;
+    if (rank1_rows(out, colmax, codes, rows, cols, false, sh, rows_grid)) {
+        const auto kernel = sh.groups == 1 ? dequant_rank1_rows_kernel<true> : dequant_rank1_rows_kernel<false>;
+        hipLaunchKernelGGL(kernel, rows_grid, dim3(kQThreads), 0, (hipStream_t)stream, codes, rowmax, colmax, qmap,
+                           rows, cols, sh, out);
+    } else if (rank1_flat_ok(out, colmax, codes, cols)) {
+        const dim3 grid((uint32_t)((n + kFlatTile - 1) / kFlatTile));
+        if (cols % 4 == 0)
+            hipLaunchKernelGGL(dequant_rank1_flat_kernel<true>, grid, dim3(kQThreads), 0, (hipStream_t)stream, codes, n,
+                               flat_cols(cols), rowmax, colmax, qmap, out);
+        else
+            hipLaunchKernelGGL(dequant_rank1_flat_kernel<false>, grid, dim3(kQThreads), 0, (hipStream_t)stream, codes, n,
+                               flat_cols(cols), rowmax, colmax, qmap, out);
     } else {
         const bool vec = aligned_to(out, 16) && aligned_to(codes, 4);
         hipLaunchKernelGGL(dequant_rank1_kernel, dim3(tiles), dim3(kQThreads), 0, (hipStream_t)stream, codes,

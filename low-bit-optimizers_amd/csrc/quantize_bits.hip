@@ -13,6 +13,7 @@
 // found by the reference's own search (upper bound, then the midpoint test, :397-427), so maps
 // with repeated entries behave as there.
 #include "lpmm_search.hpp"
+#include "rank1_rows.hpp"
 
 namespace lpmm {
 
@@ -419,7 +420,6 @@ __global__ __launch_bounds__(kBThreads) void dequant_rank1_bits_kernel(const uin
 #define LPMM_BROWS_T 2
 #endif
 constexpr int kBRowsT = LPMM_BROWS_T;       // tiles (passes of 16 groups) per workgroup: loads first, map afterwards
-constexpr int kBRank1Rows = 4;   // rows of one 2048-column chunk per workgroup of the rank-1 kernels
 
 __device__ __forceinline__ uint32_t bytes4(uint32_t a, uint32_t b, uint32_t c, uint32_t d)
 {
@@ -594,48 +594,36 @@ __global__ __launch_bounds__(kBThreads) void dequant_group_bits_rows_kernel(cons
     }
 }
 
-// 'rank1' scaling, columns a multiple of 128: grid (2048-column chunks, groups of kBRank1Rows
-// rows).  A lane keeps the maxima of its 8 columns, and their correctly rounded reciprocals,
-// over the rows of its workgroup; x / min(rowmax, colmax) is then one multiply and two fmas that
-// give the correctly rounded quotient (|x| <= scale by construction) wherever all the scales of
-// the wave lie in the range in which the reciprocal is exact, and the plain division otherwise.
-__global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows128_kernel(const float *__restrict__ x, int64_t R,
-                                                                             int64_t C,
-                                                                             const float *__restrict__ rowmax,
-                                                                             const float *__restrict__ colmax,
-                                                                             const float *__restrict__ qmap, int bits,
-                                                                             const uint32_t *__restrict__ table,
-                                                                             uint8_t *__restrict__ codes,
-                                                                             int64_t n_padded)
+// 'rank1' scaling, one code per byte, in the splits of rank1_rows.hpp (rows; flat).  x / min(rowmax, colmax) is one multiply and
+// two fmas that give the correctly rounded quotient (|x| <= scale by construction) wherever all the scales of the wave lie in
+// the range in which the reciprocal is exact, and the plain division otherwise.
+template <bool ONE>
+__global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows_kernel(const float *__restrict__ x, int64_t R, int64_t C,
+                                                                          const RowShape sh, const float *__restrict__ rowmax,
+                                                                          const float *__restrict__ colmax,
+                                                                          const float *__restrict__ qmap, int bits,
+                                                                          const uint32_t *__restrict__ table,
+                                                                          uint8_t *__restrict__ codes, int64_t n_padded)
 {
-    constexpr int T = kBRank1Rows;
+    constexpr int T = kR1RowsPerWg;
     __shared__ SearchLds lds_map;
     __shared__ BucketLds lds_bucket;
     const uint32_t tag = code_table_tag(table);
     const int64_t n = R * C;
-    const int lane16 = threadIdx.x & 15;
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c0 = (int64_t)blockIdx.x * kBTile + (int64_t)(threadIdx.x >> 4) * kGroup;
-    const bool live = c0 < C;  // uniform over the 16 lanes of a group
+    const RowLane q = row_lane<ONE>(sh, C);
     // the small loads that feed LDS first (they return first), then the rows' loads
     SearchFill fill;
     if (table == nullptr)
         fill = fill_search_load(qmap, bits);
-    float4 a[T], b[T], ca, cb;
+    float4 a[T], b[T];
     float rm[T];
-    if (live) {
-        const float *cmp = colmax + c0 + lane16 * 4;
-        ca = *reinterpret_cast<const float4 *>(cmp);
-        cb = *reinterpret_cast<const float4 *>(cmp + 64);
+    const float4 ca = *reinterpret_cast<const float4 *>(colmax + q.c), cb = *reinterpret_cast<const float4 *>(colmax + q.c2);
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                const float *p = x + (r0 + t) * C + c0 + lane16 * 4;
-                a[t] = load4(p);
-                b[t] = load4(p + 64);
-                rm[t] = rowmax[r0 + t];
-            }
-        }
+    for (int t = 0; t < T; ++t) {
+        const int64_t r_in = row_of<ONE>(q, sh, t), r = r_in < R ? r_in : R - 1;
+        a[t] = load4(x + r * C + q.c);
+        b[t] = load4(x + r * C + q.c2);
+        rm[t] = rowmax[r];
     }
     const uint32_t mode = code_table_mode(tag, bits);
     if (mode == kCodeTable) {
@@ -656,7 +644,7 @@ __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows128_kernel(con
         if (threadIdx.x == 0)
             codes[n_padded] = 0;
     }
-    if (!live)
+    if (!q.live)
         return;
     float cmx[kBElts], crc[kBElts];
     unpack8(ca, cb, cmx);
@@ -668,7 +656,8 @@ __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows128_kernel(con
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
+        const int64_t r = row_of<ONE>(q, sh, t);
+        if (r >= R)
             break;
         float v[kBElts], xs[kBElts];
         unpack8(a[t], b[t], v);
@@ -686,71 +675,158 @@ __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows128_kernel(con
         }
         uint32_t c[kBElts];
         codes8_by_mode(mode, lds_map, lds_bucket, bits, map_even, xs, c);
-        uint32_t *cp = reinterpret_cast<uint32_t *>(codes + (r0 + t) * C + c0) + lane16;
-        store_u32(cp, bytes4(c[0], c[1], c[2], c[3]));
-        store_u32(cp + 16, bytes4(c[4], c[5], c[6], c[7]));
+        store_u32(reinterpret_cast<uint32_t *>(codes + r * C + q.c), bytes4(c[0], c[1], c[2], c[3]));
+        if (q.second)
+            store_u32(reinterpret_cast<uint32_t *>(codes + r * C + q.c2), bytes4(c[4], c[5], c[6], c[7]));
     }
 }
 
-__global__ __launch_bounds__(kBThreads) void dequant_rank1_bits_rows128_kernel(const uint8_t *__restrict__ codes,
-                                                                               const float *__restrict__ rowmax,
-                                                                               const float *__restrict__ colmax,
-                                                                               const float *__restrict__ qmap, int bits,
-                                                                               int64_t R, int64_t C,
-                                                                               float *__restrict__ out)
+// columns a multiple of 128: every lane that works has its second run
+template <bool ONE>
+__global__ __launch_bounds__(kBThreads) void dequant_rank1_bits_rows_kernel(const uint8_t *__restrict__ codes,
+                                                                            const float *__restrict__ rowmax,
+                                                                            const float *__restrict__ colmax,
+                                                                            const float *__restrict__ qmap, int bits,
+                                                                            int64_t R, int64_t C, const RowShape sh,
+                                                                            float *__restrict__ out)
 {
-    constexpr int T = kBRank1Rows;
+    constexpr int T = kR1RowsPerWg;
     __shared__ float lds_map[256];
-    const int lane16 = threadIdx.x & 15;
-    const int64_t r0 = (int64_t)blockIdx.y * T;
-    const int64_t c0 = (int64_t)blockIdx.x * kBTile + (int64_t)(threadIdx.x >> 4) * kGroup;
-    const bool live = c0 < C;
+    const RowLane q = row_lane<ONE>(sh, C);
     uint32_t w0[T], w1[T];
     float rm[T];
-    float4 ca, cb;
-    if (live) {
-        const float *cmp = colmax + c0 + lane16 * 4;
-        ca = *reinterpret_cast<const float4 *>(cmp);
-        cb = *reinterpret_cast<const float4 *>(cmp + 64);
+    const float4 ca = *reinterpret_cast<const float4 *>(colmax + q.c), cb = *reinterpret_cast<const float4 *>(colmax + q.c2);
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            if (r0 + t < R) {
-                const uint32_t *cp = reinterpret_cast<const uint32_t *>(codes + (r0 + t) * C + c0) + lane16;
-                w0[t] = load_u32(cp);
-                w1[t] = load_u32(cp + 16);
-                rm[t] = rowmax[r0 + t];
-            }
-        }
+    for (int t = 0; t < T; ++t) {
+        const int64_t r_in = row_of<ONE>(q, sh, t), r = r_in < R ? r_in : R - 1;
+        w0[t] = load_u32(reinterpret_cast<const uint32_t *>(codes + r * C + q.c));
+        w1[t] = load_u32(reinterpret_cast<const uint32_t *>(codes + r * C + q.c + kRowHalf));
+        rm[t] = rowmax[r];
     }
     fill_map(lds_map, qmap, bits);
     lds_barrier();
-    if (!live)
+    if (!q.live)
         return;
     float cmx[kBElts];
     unpack8(ca, cb, cmx);
     const uint32_t mask = (1u << bits) - 1u;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-        if (r0 + t >= R)
+        const int64_t r = row_of<ONE>(q, sh, t);
+        if (r >= R)
             break;
         float v[kBElts];
         decode_bytes(w0[t], w1[t], mask, lds_map, v);
 #pragma unroll
         for (int k = 0; k < kBElts; ++k)
             v[k] *= (cmx[k] < rm[t]) ? cmx[k] : rm[t];
-        float *o = out + (r0 + t) * C + c0 + lane16 * 4;
+        float *o = out + r * C + q.c;
         store4(o, make_float4(v[0], v[1], v[2], v[3]));
-        store4(o + 64, make_float4(v[4], v[5], v[6], v[7]));
+        store4(o + kRowHalf, make_float4(v[4], v[5], v[6], v[7]));
     }
 }
 
-// rank-1 row kernels: one code per byte, columns a multiple of 128, aligned operands, rows fit grid.y
-inline bool rank1_bits_rows_ok(int bits, const void *x, const void *colmax, const void *codes, int64_t rows,
-                               int64_t cols)
+template <bool RUNS>
+__global__ __launch_bounds__(kBThreads) void quant_rank1_bits_flat_kernel(const float *__restrict__ x, int64_t n, const FlatCols f,
+                                                                          const float *__restrict__ rowmax,
+                                                                          const float *__restrict__ colmax,
+                                                                          const float *__restrict__ qmap, int bits,
+                                                                          const uint32_t *__restrict__ table,
+                                                                          uint8_t *__restrict__ codes, int64_t n_padded)
 {
-    return codes_per_byte(bits) == 1 && (cols % kGroup) == 0 && rows <= 65535LL * kBRank1Rows &&
-           (cols + kBTile - 1) / kBTile <= 0x7fffffffLL && aligned_to(x, 16) && aligned_to(colmax, 16) &&
-           aligned_to(codes, 4);
+    __shared__ SearchLds lds_map;
+    __shared__ BucketLds lds_bucket;
+    const uint32_t tag = code_table_tag(table);
+    const int64_t b0 = (int64_t)flat_tile(x) * kFlatTile;
+    const bool whole = b0 + kFlatTile <= n;
+    SearchFill fill;
+    if (table == nullptr)
+        fill = fill_search_load(qmap, bits);
+    float4 a[kFlatT];
+    FlatStats<RUNS> st[kFlatT];
+    flat_load<RUNS>(x, b0, n, whole, a);
+    flat_stats_of_tile<RUNS>(rowmax, colmax, b0, n, whole, f, st);
+    const uint32_t mode = code_table_mode(tag, bits);
+    if (mode == kCodeTable) {
+        code_table_store(lds_bucket, code_table_load(table));
+    } else if (mode == kCodeSearch) {
+        if (table != nullptr)  // a table that says "search"
+            fill = fill_search_load(qmap, bits);
+        fill_search_store(lds_map, fill, bits);
+    }
+    lds_barrier();
+    const bool map_even = mode == kCodeEven || (mode == kCodeSearch && map_is_even(lds_map));
+    if (b0 == 0 && threadIdx.x == 0)
+        codes[n_padded] = 0;
+#pragma unroll
+    for (int t = 0; t < kFlatT; t += 2) {
+        const int64_t i0 = b0 + t * kFlatPass + threadIdx.x * 4, i1 = i0 + kFlatPass;
+        float v[kBElts], s[kBElts], xs[kBElts];
+        unpack8(a[t], a[t + 1], v);
+        flat_scales<RUNS>(st[t], s);
+        flat_scales<RUNS>(st[t + 1], s + 4);
+        bool safe = true;
+#pragma unroll
+        for (int k = 0; k < kBElts; ++k)
+            safe = safe && rc_safe(s[k]);
+        if (__all(safe)) {
+#pragma unroll
+            for (int k = 0; k < kBElts; ++k)
+                xs[k] = div_by_rc(v[k], s[k], rcp_exact(s[k]));
+        } else {
+            // the values that pad the tensor are plain zeros
+#pragma unroll
+            for (int k = 0; k < kBElts; ++k)
+                xs[k] = (k < 4 ? i0 : i1) + (k & 3) < n ? v[k] / s[k] : 0.0f;
+        }
+        uint32_t c[kBElts];
+        codes8_by_mode(mode, lds_map, lds_bucket, bits, map_even, xs, c);
+        if (whole || i0 < n_padded)
+            store_u32(reinterpret_cast<uint32_t *>(codes + i0), bytes4(c[0], c[1], c[2], c[3]));
+        if (whole || i1 < n_padded)
+            store_u32(reinterpret_cast<uint32_t *>(codes + i1), bytes4(c[4], c[5], c[6], c[7]));
+    }
+}
+
+template <bool RUNS>
+__global__ __launch_bounds__(kBThreads) void dequant_rank1_bits_flat_kernel(const uint8_t *__restrict__ codes, int64_t n,
+                                                                            const FlatCols f, const float *__restrict__ rowmax,
+                                                                            const float *__restrict__ colmax,
+                                                                            const float *__restrict__ qmap, int bits,
+                                                                            float *__restrict__ out)
+{
+    __shared__ float lds_map[256];
+    const int64_t b0 = (int64_t)flat_tile(out) * kFlatTile;
+    const bool whole = b0 + kFlatTile <= n;
+    uint32_t w[kFlatT];
+    FlatStats<RUNS> st[kFlatT];
+#pragma unroll
+    for (int t = 0; t < kFlatT; ++t) {
+        const int64_t idx = b0 + t * kFlatPass + threadIdx.x * 4;
+        w[t] = 0;
+        if (whole || idx + 4 <= n) {
+            w[t] = load_u32(reinterpret_cast<const uint32_t *>(codes + idx));
+        } else if (!RUNS) {
+            for (int k = 0; k < 3; ++k)
+                w[t] |= idx + k < n ? (uint32_t)codes[idx + k] << (8 * k) : 0u;
+        }
+    }
+    flat_stats_of_tile<RUNS>(rowmax, colmax, b0, n, whole, f, st);
+    fill_map(lds_map, qmap, bits);
+    lds_barrier();
+    const uint32_t mask = (1u << bits) - 1u;
+#pragma unroll
+    for (int t = 0; t < kFlatT; t += 2) {
+        float s[kBElts], v[kBElts];
+        decode_bytes(w[t], w[t + 1], mask, lds_map, v);
+        flat_scales<RUNS>(st[t], s);
+        flat_scales<RUNS>(st[t + 1], s + 4);
+#pragma unroll
+        for (int k = 0; k < kBElts; ++k)
+            v[k] *= s[k];
+        flat_store<RUNS>(out, b0 + t * kFlatPass + threadIdx.x * 4, n, whole, v);
+        flat_store<RUNS>(out, b0 + (t + 1) * kFlatPass + threadIdx.x * 4, n, whole, v + 4);
+    }
 }
 
 inline bool bits_ok(int bits) { return bits >= 1 && bits <= 8; }
@@ -956,15 +1032,24 @@ extern "C" int lpmm_quant_rank1_bits_table(const float *x, int64_t rows, int64_t
     uint32_t tiles;
     if (!tiles_for(n, &tiles))
         return LPMM_ERR_SIZE;
-    if (rank1_bits_rows_ok(bits, x, colmax, codes, rows, cols)) {
-        const dim3 grid((uint32_t)((cols + kBTile - 1) / kBTile), (uint32_t)((rows + kBRank1Rows - 1) / kBRank1Rows));
-        hipLaunchKernelGGL(quant_rank1_bits_rows128_kernel, grid, dim3(kBThreads), 0, (hipStream_t)stream, x, rows, cols,
-                           rowmax, colmax, qmap, bits, static_cast<const uint32_t *>(table), codes,
-                           (int64_t)tiles * kBTile);
+    const int64_t n_padded = (int64_t)tiles * kBTile;
+    RowShape sh;
+    dim3 grid;
+    if (codes_per_byte(bits) == 1 && rank1_rows(x, colmax, codes, rows, cols, true, sh, grid)) {
+        const auto kernel = sh.groups == 1 ? quant_rank1_bits_rows_kernel<true> : quant_rank1_bits_rows_kernel<false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kBThreads), 0, (hipStream_t)stream, x, rows, cols, sh, rowmax, colmax,
+                           qmap, bits, static_cast<const uint32_t *>(table), codes, n_padded);
+        return launch_status();
+    }
+    if (codes_per_byte(bits) == 1 && rank1_flat_ok(x, colmax, codes, cols)) {
+        const auto kernel = cols % 4 == 0 ? quant_rank1_bits_flat_kernel<true> : quant_rank1_bits_flat_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((n_padded + kFlatTile - 1) / kFlatTile)), dim3(kBThreads), 0,
+                           (hipStream_t)stream, x, n, flat_cols(cols), rowmax, colmax, qmap, bits,
+                           static_cast<const uint32_t *>(table), codes, n_padded);
         return launch_status();
     }
     hipLaunchKernelGGL(quant_rank1_bits_kernel, dim3(tiles), dim3(kBThreads), 0, (hipStream_t)stream, x, n, cols,
-                       rowmax, colmax, qmap, bits, codes, (int64_t)tiles * kBTile, aligned_to(x, 16));
+                       rowmax, colmax, qmap, bits, codes, n_padded, aligned_to(x, 16));
     return launch_status();
 }
 
@@ -988,10 +1073,18 @@ extern "C" int lpmm_dequant_rank1_bits(const uint8_t *codes, const float *rowmax
     uint32_t tiles;
     if (!tiles_for(n, &tiles))
         return LPMM_ERR_SIZE;
-    if (rank1_bits_rows_ok(bits, out, colmax, codes, rows, cols)) {
-        const dim3 grid((uint32_t)((cols + kBTile - 1) / kBTile), (uint32_t)((rows + kBRank1Rows - 1) / kBRank1Rows));
-        hipLaunchKernelGGL(dequant_rank1_bits_rows128_kernel, grid, dim3(kBThreads), 0, (hipStream_t)stream, codes,
-                           rowmax, colmax, qmap, bits, rows, cols, out);
+    RowShape sh;
+    dim3 grid;
+    if (codes_per_byte(bits) == 1 && rank1_rows(out, colmax, codes, rows, cols, false, sh, grid)) {
+        const auto kernel = sh.groups == 1 ? dequant_rank1_bits_rows_kernel<true> : dequant_rank1_bits_rows_kernel<false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(kBThreads), 0, (hipStream_t)stream, codes, rowmax, colmax, qmap, bits,
+                           rows, cols, sh, out);
+        return launch_status();
+    }
+    if (codes_per_byte(bits) == 1 && rank1_flat_ok(out, colmax, codes, cols)) {
+        const auto kernel = cols % 4 == 0 ? dequant_rank1_bits_flat_kernel<true> : dequant_rank1_bits_flat_kernel<false>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)((n + kFlatTile - 1) / kFlatTile)), dim3(kBThreads), 0, (hipStream_t)stream,
+                           codes, n, flat_cols(cols), rowmax, colmax, qmap, bits, out);
         return launch_status();
     }
     hipLaunchKernelGGL(dequant_rank1_bits_kernel, dim3(tiles), dim3(kBThreads), 0, (hipStream_t)stream, codes, rowmax,

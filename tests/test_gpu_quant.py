@@ -356,3 +356,43 @@ def test_quant_group_extreme_scales(oracle, qmaps):
             torch.cuda.synchronize()
             np.testing.assert_array_equal(to_np(codes), want_codes)
             np.testing.assert_array_equal(to_np(max1), want_max1)
+
+
+# columns on either side of every limit of the rank-1 kernels' dispatch (rows of a chunk at a time for whole runs of four and at
+# least 16 columns, flattened otherwise, one lane a run of eight below 4 columns or off a 16-byte boundary; the statistics by
+# lanes a row), with rows that fill a workgroup's tile, leave one over and are fewer than its groups
+RANK1_EDGES = [(1, 4), (9, 1), (7, 3), (1030, 5), (4099, 6), (1, 16), (341, 20), (2049, 12), (700, 52), (129, 100), (513, 130),
+               (130, 256), (67, 257), (33, 300), (21, 516), (17, 1601), (9, 2048), (5, 2056), (3, 4100), (70001, 8), (3, 11009)]
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("shape", RANK1_EDGES)
+def test_rank1_dispatch_edges(oracle, qmaps, shape, shift):
+    lib = _lib()
+    r, c = shape
+    n = r * c
+    rng = np.random.default_rng(n + shift)
+    for qmap, x in ((qmaps[1], _unsigned(rng, n).reshape(r, c)), (qmaps[0], _signed(rng, n).reshape(r, c))):
+        x[0, :] = 0.0
+        x[:, c - 1] = 0.0
+        x[r - 1, c // 2] = np.inf  # a row and a column whose scale is not finite
+        want_row, want_col = oracle.rank1_stats(x)
+        want_codes = oracle.quant_rank1(x, want_row, want_col, qmap)
+        want = oracle.dequant_rank1(want_codes, want_row, want_col, qmap, r, c)
+        dx = torch.empty(n + 4, device="cuda")[shift: shift + n]  # shift: operands off a 16-byte boundary
+        dx.copy_(to_dev(x).view(-1))
+        dq, codes = to_dev(qmap), torch.full((want_codes.size + 16,), 0x55, dtype=torch.uint8, device="cuda")
+        rowmax, colmax = torch.full((r + 1,), -1.0, device="cuda"), torch.full((c + 1,), -1.0, device="cuda")
+        out = torch.full((n + 8,), -1.0, device="cuda")
+        assert lib.lpmm_rank1_stats(dx.data_ptr(), r, c, rowmax.data_ptr(), colmax.data_ptr(), _stream()) == 0
+        assert lib.lpmm_quant_rank1(dx.data_ptr(), r, c, rowmax.data_ptr(), colmax.data_ptr(), dq.data_ptr(), codes.data_ptr(),
+                                    _stream()) == 0
+        assert lib.lpmm_dequant_rank1(codes.data_ptr(), rowmax.data_ptr(), colmax.data_ptr(), dq.data_ptr(), r, c,
+                                      out[shift:].data_ptr(), _stream()) == 0
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(to_np(rowmax), np.append(want_row, np.float32(-1)))
+        np.testing.assert_array_equal(to_np(colmax), np.append(want_col, np.float32(-1)))
+        np.testing.assert_array_equal(to_np(codes)[: want_codes.size], want_codes)
+        assert (to_np(codes)[want_codes.size:] == 0x55).all()
+        np.testing.assert_array_equal(to_np(out)[shift: shift + n], want.reshape(-1))
+        assert (to_np(out)[:shift] == -1).all() and (to_np(out)[shift + n:] == -1).all()
