@@ -17,6 +17,10 @@
 //     that share a byte may belong to neighbouring lanes (they meet by a lane exchange) or, where the column
 //     count is odd, to different rows: the first pass clears the word around such a byte, the second sets the word's codes
 //     by atomic or (store_nibbles).
+// Two forms (rank1_any_runs): runs of four neighbouring values a lane where every tensor of a launch allows it, single values 16 apart
+// otherwise.  A step on six tensors, single values -> runs (with the order of xcd_neighbours and quotients by reciprocals kept over
+// a lane's rows): 4096 x 4100 595 -> 510 us, fp32 first moment 600 -> 505, 8 bits 609 -> 555, float16 696 -> 580; 4096 x 1600
+// 246 -> 200 (fp32), 262 -> 210 (8 bits), 345 -> 270 (float16).
 // Before, these tensors took the staged path (dequantise, update, statistics, normalise: six to eight
 // launches a tensor and 50 bytes a value; float16: about thirty PyTorch ops a tensor).  One step on one tensor,
 // staged -> here: 4096 x 4100 default 224 -> 107 us, fp32 first moment 183 -> 104, 8 bits 221 -> 102, float16
@@ -84,13 +88,75 @@ __device__ __forceinline__ Piece piece_of(int64_t cols, uint32_t cg, int64_t r, 
     return w;
 }
 
+// Which of a piece's values a lane has.  VEC: two runs of four neighbours, 64 apart, as in the tuned kernels (rows of a multiple of four
+// values, operands on the boundaries that whole runs need); otherwise values 16 apart.  A lane beyond the piece's end has
+// the last run or value once more.
+template <bool VEC>
+__device__ __forceinline__ bool piece_has(const Piece &w, int lane16, int k)
+{
+    return (VEC ? 4 * lane16 + 64 * (k >> 2) : 16 * k + lane16) < w.count;
+}
+
+template <bool VEC>
 __device__ __forceinline__ int piece_at(const Piece &w, int lane16, int k)
 {
-    const int off = 16 * k + lane16;
-    return off < w.count ? off : w.count - 1;
+    const int off = VEC ? 4 * lane16 + 64 * (k >> 2) : 16 * k + lane16;
+    return VEC ? (off < w.count ? off : w.count - 4) + (k & 3) : off < w.count ? off : w.count - 1;
+}
+
+// KEEP: without the nontemporal hint.  Where rows do not start on cache lines, a line at the edge of a piece is read by two workgroups, and
+// the update pass finds it in the L2 the second time (neighbouring tiles are on one XCD: xcd_neighbours).  Six tensors of 4096 x 4100, update
+// pass with and without the hint: 294 and 261 us, fp32 first moment 445 and 367, 8 bits 331 and 286; of 4096 x 1600, where rows start on
+// lines, fp32 first moment 137 and 139-158.  The second pass reads g for the last time: 125 with the hint, 156 without (fp32).
+template <bool KEEP>
+__device__ __forceinline__ void load_run(const float *at, float *o)
+{
+    const float4 a = KEEP ? *reinterpret_cast<const float4 *>(at) : load4(at);
+    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
+}
+template <bool KEEP>
+__device__ __forceinline__ void load_run(const h16 *at, h16 *o)
+{
+    const v4h a = KEEP ? *reinterpret_cast<const v4h *>(at) : load_h4(at);
+    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
+}
+__device__ __forceinline__ void store_run(float *at, const float *x) { store4(at, make_float4(x[0], x[1], x[2], x[3])); }
+__device__ __forceinline__ void store_run(h16 *at, const h16 *x)
+{
+    __builtin_nontemporal_store(v4h{x[0], x[1], x[2], x[3]}, reinterpret_cast<v4h *>(at));
+}
+
+template <bool VEC, bool KEEP, typename T>
+__device__ __forceinline__ void load_values(const T *at, const Piece &w, int lane16, T (&o)[kAnyElts])
+{
+    if constexpr (VEC) {
+        load_run<KEEP>(at + piece_at<true>(w, lane16, 0), o);
+        load_run<KEEP>(at + piece_at<true>(w, lane16, 4), o + 4);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            o[k] = at[piece_at<false>(w, lane16, k)];
+    }
+}
+
+template <bool VEC, typename T>
+__device__ __forceinline__ void store_values(T *at, const Piece &w, int lane16, const T (&x)[kAnyElts])
+{
+    if constexpr (VEC) {
+        if (piece_has<true>(w, lane16, 0))
+            store_run(at + 4 * lane16, x);
+        if (piece_has<true>(w, lane16, 4))
+            store_run(at + 4 * lane16 + 64, x + 4);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kAnyElts; ++k)
+            if (piece_has<false>(w, lane16, k))
+                at[16 * k + lane16] = x[k];
+    }
 }
 
 // The chain of ops has its second moment in a tensor of its own, on a 16-byte boundary; the gradient may lie anywhere.
+template <bool VEC>
 __device__ __forceinline__ RoundOnce rounded_once(const Piece &w, int lane16, int64_t n, const void *g)
 {
     const int64_t twice = ops_twice(nullptr, nullptr, n);
@@ -98,27 +164,35 @@ __device__ __forceinline__ RoundOnce rounded_once(const Piece &w, int lane16, in
     if (w.base + w.count > twice)
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
-            behind |= (w.base + piece_at(w, lane16, k) >= twice ? 1u : 0u) << k;
+            behind |= (w.base + piece_at<VEC>(w, lane16, k) >= twice ? 1u : 0u) << k;
     return RoundOnce{behind, ops_twice(g, nullptr, n) == twice ? behind : 0xffu};
 }
 
 // codes of the lane's eight values: element k in bits 4 k (two codes a byte) or in byte k (one a byte)
-template <bool BITS>
+template <bool BITS, bool VEC>
 __device__ __forceinline__ uint64_t load_codes(const uint8_t *codes, const Piece &w, int lane16)
 {
     uint64_t out = 0;
+    if (VEC) {
+        const int64_t a = w.base + piece_at<true>(w, lane16, 0), b = w.base + piece_at<true>(w, lane16, 4);
+        if (BITS)
+            return load_u32(reinterpret_cast<const uint32_t *>(codes + a)) |
+                   (uint64_t)load_u32(reinterpret_cast<const uint32_t *>(codes + b)) << 32;
+        return load_u16(reinterpret_cast<const uint16_t *>(codes + (a >> 1))) |
+               load_u16(reinterpret_cast<const uint16_t *>(codes + (b >> 1))) << 16;
+    }
     if (BITS) {
         const uint8_t *c = codes + w.base;
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
-            out |= (uint64_t)c[piece_at(w, lane16, k)] << (8 * k);
+            out |= (uint64_t)c[piece_at<false>(w, lane16, k)] << (8 * k);
     } else {
         const uint8_t *c = codes + (w.base >> 1);
         const int odd = (int)(w.base & 1);
         uint32_t low = 0;
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k) {
-            const int at = piece_at(w, lane16, k) + odd;
+            const int at = piece_at<false>(w, lane16, k) + odd;
             low |= (((uint32_t)c[at >> 1] >> (4 * (at & 1))) & 15u) << (4 * k);
         }
         out = low;
@@ -182,9 +256,28 @@ __device__ __forceinline__ void store_nibbles(uint8_t *codes, const Piece &w, in
     }
 }
 
+// VEC: no two rows share a byte
+__device__ __forceinline__ void store_nibble_runs(uint8_t *codes, const Piece &w, int lane16, uint32_t now)
+{
+    uint16_t *c = reinterpret_cast<uint16_t *>(codes + (w.base >> 1)) + lane16;
+    if (piece_has<true>(w, lane16, 0))
+        store_u16(c, now & 0xFFFFu);
+    if (piece_has<true>(w, lane16, 4))
+        store_u16(c + 16, now >> 16);
+}
+
+template <bool VEC>
 __device__ __forceinline__ void store_bytes(uint8_t *codes, const Piece &w, int lane16, const uint32_t (&now)[kAnyElts])
 {
     uint8_t *c = codes + w.base;
+    if (VEC) {
+        uint32_t *at = reinterpret_cast<uint32_t *>(c) + lane16;
+        if (piece_has<true>(w, lane16, 0))
+            store_u32(at, now[0] | (now[1] << 8) | (now[2] << 16) | (now[3] << 24));
+        if (piece_has<true>(w, lane16, 4))
+            store_u32(at + 16, now[4] | (now[5] << 8) | (now[6] << 16) | (now[7] << 24));
+        return;
+    }
 #pragma unroll
     for (int k = 0; k < kAnyElts; ++k) {
         const int off = 16 * k + lane16;
@@ -227,7 +320,7 @@ __device__ __forceinline__ float rank1_scale(float co, float ro) { return co < r
 
 // REAL: the parameters' type (h16: the chain of half ops, half scales and statistics, float work arrays for the
 // maxima); M32: fp32 first moment; BITS: one code of bits_m / bits_v bits per byte
-template <typename REAL, bool M32, bool BITS>
+template <typename REAL, bool M32, bool BITS, bool VEC>
 __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const MultiR1 args, const NewCodes out,
                                                                        const float *__restrict__ qmap_m,
                                                                        const float *__restrict__ qmap_v, int bits_m, int bits_v)
@@ -238,7 +331,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
     __shared__ uint32_t colred[kMaxWide * kGroup], rowred[kRowSlots];
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const uint32_t tl = xcd_neighbours(blockIdx.x - args.tile_start[lo], args.tile_start[lo + 1] - args.tile_start[lo]);
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
@@ -261,6 +354,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
 
     const uint32_t mask_m = (1u << bits_m) - 1u, mask_v = (1u << bits_v) - 1u;
     const int lg_group = 7 + (int)t.m_lg;
+    const bool keep = cols % (128 / (int)sizeof(REAL)) != 0;
     if (q.cg < t.col_blocks && q.row0 < t.rows) {
         const REAL *row_old = reinterpret_cast<const REAL *>(t.row_old);
         const REAL *col_old = reinterpret_cast<const REAL *>(t.col_old) + (int64_t)q.cg * kGroup;
@@ -270,7 +364,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
         uint32_t vtop[kAnyElts];  // the lane's columns: current statistics, maxima over its passes
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k) {
-            co[k] = col_old[piece_at(first, lane16, k)];
+            co[k] = col_old[piece_at<VEC>(first, lane16, k)];
             vtop[k] = 0u;
         }
 #pragma unroll 1
@@ -284,23 +378,25 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             float *mp = reinterpret_cast<float *>(t.mc) + w.base;
             REAL p[kAnyElts], g[kAnyElts];
             float m[kAnyElts], v[kAnyElts];
-#pragma unroll
-            for (int k = 0; k < kAnyElts; ++k) {
-                p[k] = pp[piece_at(w, lane16, k)];
-                g[k] = gp[piece_at(w, lane16, k)];
-            }
-            const uint64_t vc = load_codes<BITS>(t.vc, w, lane16);
-            const REAL ro = row_old[r];
-            if (M32) {
-#pragma unroll
-                for (int k = 0; k < kAnyElts; ++k)
-                    m[k] = mp[piece_at(w, lane16, k)];
+            if (keep) {
+                load_values<VEC, true>(pp, w, lane16, p);
+                load_values<VEC, true>(gp, w, lane16, g);
+                if (M32)
+                    load_values<VEC, true>(mp, w, lane16, m);
             } else {
-                const uint64_t mc = load_codes<BITS>(t.mc, w, lane16);
+                load_values<VEC, false>(pp, w, lane16, p);
+                load_values<VEC, false>(gp, w, lane16, g);
+                if (M32)
+                    load_values<VEC, false>(mp, w, lane16, m);
+            }
+            const uint64_t vc = load_codes<BITS, VEC>(t.vc, w, lane16);
+            const REAL ro = row_old[r];
+            if (!M32) {
+                const uint64_t mc = load_codes<BITS, VEC>(t.mc, w, lane16);
                 const float s0 = (float)ms[w.group], s1 = w.split < w.count ? (float)ms[w.group + 1] : 0.0f;
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k)
-                    m[k] = any_decode<BITS>(map_m, mc, k, mask_m) * (piece_at(w, lane16, k) < w.split ? s0 : s1);
+                    m[k] = any_decode<BITS>(map_m, mc, k, mask_m) * (piece_at<VEC>(w, lane16, k) < w.split ? s0 : s1);
             }
 #pragma unroll
             for (int k = 0; k < kAnyElts; ++k)
@@ -315,7 +411,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                     m2[j] = round2(m[2 * j], m[2 * j + 1]);
                     v2[j] = round2(v[2 * j], v[2 * j + 1]);
                 }
-                half_elts8<true, true>(p2, g2, m2, v2, h, c, rounded_once(w, lane16, t.rows * cols, t.g));
+                half_elts8<true, true>(p2, g2, m2, v2, h, c, rounded_once<VEC>(w, lane16, t.rows * cols, t.g));
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k) {
                     p[k] = p2[k >> 1][k & 1];
@@ -338,7 +434,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                 uint32_t m0 = 0u, m1 = 0u;
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k) {
-                    const bool here = piece_at(w, lane16, k) < w.split;
+                    const bool here = piece_at<VEC>(w, lane16, k) < w.split;
                     m0 = larger<HALF>(m0, here ? m[k] : 0.0f);
                     m1 = larger<HALF>(m1, here ? 0.0f : m[k]);
                 }
@@ -360,19 +456,13 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                         clear_shared(out.m[lo], w);
                 }
             }
-#pragma unroll
-            for (int k = 0; k < kAnyElts; ++k) {
-                const int off = 16 * k + lane16;
-                if (off < w.count) {
-                    pp[off] = p[k];
-                    if (M32)
-                        mp[off] = m[k];
-                }
-            }
+            store_values<VEC>(pp, w, lane16, p);
+            if (M32)
+                store_values<VEC>(mp, w, lane16, m);
         }
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
-            atomicMax(colred + (drow & (q.wide - 1)) * kGroup + piece_at(first, lane16, k), vtop[k]);
+            atomicMax(colred + (drow & (q.wide - 1)) * kGroup + piece_at<VEC>(first, lane16, k), vtop[k]);
     }
     __syncthreads();
     flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
@@ -407,9 +497,14 @@ struct AnyCoder<false> {
         const float xs[kAnyElts] = {x, x, x, x, x, x, x, x};
         return encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], xs) & 15u;
     }
+    template <bool VEC>
     __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16, bool odd_cols) const
     {
-        store_nibbles(codes, w, lane16, encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], x), odd_cols);
+        const uint32_t now = encode8_plain(l.w, which ? kLdsQ1 : kLdsQ0, kind[which], x);
+        if (VEC)
+            store_nibble_runs(codes, w, lane16, now);
+        else
+            store_nibbles(codes, w, lane16, now, odd_cols);
     }
 };
 
@@ -453,28 +548,42 @@ struct AnyCoder<true> {
     {
         return code1_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], x);
     }
+    template <bool VEC>
     __device__ __forceinline__ void store(int which, const float (&x)[kAnyElts], uint8_t *codes, const Piece &w, int lane16, bool) const
     {
         uint32_t c[kAnyElts];
         codes8_by_mode(mode[which], l.search[which], l.bucket[which], bits[which], even[which], x, c);
-        store_bytes(codes, w, lane16, c);
+        store_bytes<VEC>(codes, w, lane16, c);
     }
 };
 
-// x[k] / s[k], rounded to half where the chain is one of half ops.  Every scale is a maximum over the values it
-// divides, so where all of a wave's scales lie in the range in which the reciprocal is exact, one product and two
-// fmas are the correctly rounded quotient.
-template <bool HALF>
-__device__ __forceinline__ void any_quotients(float (&x)[kAnyElts], const float (&s)[kAnyElts])
+// A wave's reciprocals of the scales s[k], and whether they may be used (any_quotients).  KEPT: the caller has them already, from
+// statistics that stay over a lane's rows; where a lane takes single values the registers for that are not there (float16, 4095 x 4099:
+// 795 -> 982 us a step on six tensors).
+template <bool KEPT>
+__device__ __forceinline__ bool any_reciprocals(const float (&s)[kAnyElts], float (&rc)[kAnyElts], bool safe)
 {
-    bool safe = true;
+    if (!KEPT) {
+        safe = true;
 #pragma unroll
-    for (int k = 0; k < kAnyElts; ++k)
-        safe = safe && rc_safe(s[k]);
-    if (__all(safe)) {
+        for (int k = 0; k < kAnyElts; ++k) {
+            safe = safe && rc_safe(s[k]);
+            rc[k] = rcp_exact(s[k]);
+        }
+    }
+    return __all(safe);
+}
+
+// x[k] / s[k] with rc[k] = 1 / s[k], rounded to half where the chain is one of half ops.  Every scale is a maximum over the
+// values it divides, so where all of a wave's scales lie in the range in which the reciprocal is exact (fast), one product and
+// two fmas are the correctly rounded quotient.
+template <bool HALF>
+__device__ __forceinline__ void any_quotients(float (&x)[kAnyElts], const float (&s)[kAnyElts], const float (&rc)[kAnyElts], bool fast)
+{
+    if (fast) {
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
-            x[k] = div_by_rc(x[k], s[k], rcp_exact(s[k]));
+            x[k] = div_by_rc(x[k], s[k], rc[k]);
     } else {
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k)
@@ -486,7 +595,7 @@ __device__ __forceinline__ void any_quotients(float (&x)[kAnyElts], const float 
             x[k] = rh(x[k]);
 }
 
-template <typename REAL, bool M32, bool BITS>
+template <typename REAL, bool M32, bool BITS, bool VEC>
 __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const MultiR1 args, const NewCodes out,
                                                                         const float *__restrict__ qmap_m,
                                                                         const float *__restrict__ qmap_v, int bits_m, int bits_v,
@@ -498,7 +607,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
     AnyCoder<BITS> coder(lds, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v);
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const uint32_t tl = xcd_neighbours(blockIdx.x - args.tile_start[lo], args.tile_start[lo + 1] - args.tile_start[lo]);
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
@@ -530,11 +639,14 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
     const REAL *ms = reinterpret_cast<const REAL *>(t.ms);
     const Piece first = piece_of(cols, q.cg, q.row0, lg_group);
     REAL co[kAnyElts];
-    float cn[kAnyElts];
+    float cn[kAnyElts], rcn[kAnyElts];
+    bool cols_safe = true;
 #pragma unroll
     for (int k = 0; k < kAnyElts; ++k) {
-        co[k] = col_old[piece_at(first, lane16, k)];
-        cn[k] = col_new[piece_at(first, lane16, k)];
+        co[k] = col_old[piece_at<VEC>(first, lane16, k)];
+        cn[k] = col_new[piece_at<VEC>(first, lane16, k)];
+        rcn[k] = VEC ? rcp_exact(cn[k]) : 0.0f;
+        cols_safe = VEC && cols_safe && rc_safe(cn[k]);
     }
     const MixConst c = mix_const();
 #pragma unroll 1
@@ -545,23 +657,23 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
         const Piece w = piece_of(cols, q.cg, r, lg_group);
         const REAL *gp = reinterpret_cast<const REAL *>(t.g) + w.base;
         REAL g[kAnyElts];
-        float x[kAnyElts], s[kAnyElts];
-#pragma unroll
-        for (int k = 0; k < kAnyElts; ++k)
-            g[k] = gp[piece_at(w, lane16, k)];
-        const uint64_t vc = load_codes<BITS>(t.vc, w, lane16);
-        const uint64_t mc = M32 ? 0 : load_codes<BITS>(t.mc, w, lane16);
+        float x[kAnyElts], s[kAnyElts], rc[kAnyElts];
+        load_values<VEC, false>(gp, w, lane16, g);
+        const uint64_t vc = load_codes<BITS, VEC>(t.vc, w, lane16);
+        const uint64_t mc = M32 ? 0 : load_codes<BITS, VEC>(t.mc, w, lane16);
         const REAL ro = row_old[r];
         const float rn = t.row_new[r];
         if (!M32) {
             const bool two = w.split < w.count;
             const float s0 = (float)ms[w.group], s1 = two ? (float)ms[w.group + 1] : 0.0f;
             const float n0 = t.ms_new[w.group], n1 = two ? t.ms_new[w.group + 1] : n0;
+            const float rc0 = VEC ? rcp_exact(n0) : 0.0f, rc1 = VEC ? rcp_exact(n1) : 0.0f;
 #pragma unroll
             for (int k = 0; k < kAnyElts; ++k) {
-                const bool here = piece_at(w, lane16, k) < w.split;
+                const bool here = piece_at<VEC>(w, lane16, k) < w.split;
                 x[k] = any_decode<BITS>(coder.map(0), mc, k, mask_m) * (here ? s0 : s1);
                 s[k] = here ? n0 : n1;
+                rc[k] = here ? rc0 : rc1;
             }
             if constexpr (HALF) {
 #pragma unroll
@@ -580,18 +692,21 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
                 for (int k = 0; k < kAnyElts; ++k)
                     x[k] = lerp_w(x[k], g[k], h.w1);
             }
-            any_quotients<HALF>(x, s);
-            coder.store(0, x, out.m[lo], w, lane16, odd_cols);
+            any_quotients<HALF>(x, s, rc, any_reciprocals<VEC>(s, rc, rc_safe(n0) && rc_safe(n1)));
+            coder.template store<VEC>(0, x, out.m[lo], w, lane16, odd_cols);
             // the second moment's loads stay behind the stores: 12 instead of 100 bytes of spilled registers a lane
             __builtin_amdgcn_sched_barrier(0);
         }
+        const float rcr = VEC ? rcp_exact(rn) : 0.0f;
 #pragma unroll
         for (int k = 0; k < kAnyElts; ++k) {
             x[k] = any_decode<BITS>(coder.map(1), vc, k, mask_v) * rank1_scale((float)co[k], (float)ro);
-            s[k] = rank1_scale(cn[k], rn);
+            const bool by_col = cn[k] < rn;
+            s[k] = by_col ? cn[k] : rn;
+            rc[k] = by_col ? rcn[k] : rcr;
         }
         if constexpr (HALF) {
-            const RoundOnce once = rounded_once(w, lane16, t.rows * cols, t.g);
+            const RoundOnce once = rounded_once<VEC>(w, lane16, t.rows * cols, t.g);
 #pragma unroll
             for (int j = 0; j < kPairs; ++j) {
                 const v2h b = half_second_moment_ops(round2(x[2 * j], x[2 * j + 1]), v2h{g[2 * j], g[2 * j + 1]}, h, c, once, j);
@@ -603,21 +718,39 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
             for (int k = 0; k < kAnyElts; ++k)
                 nonfused_second_moment(x[k], g[k], h);
         }
-        any_quotients<HALF>(x, s);
-        coder.store(1, x, out.v[lo], w, lane16, odd_cols);
+        any_quotients<HALF>(x, s, rc, any_reciprocals<VEC>(s, rc, cols_safe && rc_safe(rn)));
+        coder.template store<VEC>(1, x, out.v[lo], w, lane16, odd_cols);
     }
+}
+
+template <typename REAL, bool M32, bool BITS, bool VEC>
+static void launch_passes(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v, int bits_m, int bits_v,
+                          const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
+{
+    if (passes & 1)
+        hipLaunchKernelGGL((rank1_update_any_kernel<REAL, M32, BITS, VEC>), dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update,
+                           out, qmap_m, qmap_v, bits_m, bits_v);
+    if (passes & 2)
+        hipLaunchKernelGGL((rank1_requant_any_kernel<REAL, M32, BITS, VEC>), dim3(l.requant_tiles), dim3(kThreads), 0, stream,
+                           l.requant, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v);
 }
 
 template <typename REAL, bool M32, bool BITS>
 static void launch(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v, int bits_m, int bits_v,
-                   const uint32_t *table_m, const uint32_t *table_v, int passes, hipStream_t stream)
+                   const uint32_t *table_m, const uint32_t *table_v, bool runs, int passes, hipStream_t stream)
 {
-    if (passes & 1)
-        hipLaunchKernelGGL((rank1_update_any_kernel<REAL, M32, BITS>), dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, out,
-                           qmap_m, qmap_v, bits_m, bits_v);
-    if (passes & 2)
-        hipLaunchKernelGGL((rank1_requant_any_kernel<REAL, M32, BITS>), dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, out,
-                           qmap_m, qmap_v, bits_m, bits_v, table_m, table_v);
+    if (runs)
+        launch_passes<REAL, M32, BITS, true>(l, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
+    else
+        launch_passes<REAL, M32, BITS, false>(l, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
+}
+
+// Runs of four where every access of a run is whole: columns a multiple of 4, parameters, gradients and an fp32 first moment on
+// boundaries of four values (code arrays lie on 4-byte boundaries in any case).
+bool rank1_any_runs(const lpmm_rank1_any_tensor &t, AnyKind kind)
+{
+    const uintptr_t run = kind == kAnyHalf ? 8 : 16;
+    return t.cols % 4 == 0 && aligned_to(t.p, run) && aligned_to(t.g, run) && (kind != kAnyFloatM || aligned_to(t.m, run));
 }
 
 void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v, AnyKind kind, int bits_m, int bits_v,
@@ -625,16 +758,16 @@ void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_
 {
     switch (kind) {
     case kAnyCodes4:
-        launch<float, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<float, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, out.runs, passes, stream);
         break;
     case kAnyFloatM:
-        launch<float, true, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<float, true, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, out.runs, passes, stream);
         break;
     case kAnyBits:
-        launch<float, false, true>(l, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, passes, stream);
+        launch<float, false, true>(l, out, qmap_m, qmap_v, bits_m, bits_v, table_m, table_v, out.runs, passes, stream);
         break;
     case kAnyHalf:
-        launch<h16, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, passes, stream);
+        launch<h16, false, false>(l, out, qmap_m, qmap_v, 4, 4, nullptr, nullptr, out.runs, passes, stream);
         break;
     }
 }

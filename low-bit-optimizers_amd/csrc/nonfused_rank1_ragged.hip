@@ -12,13 +12,15 @@ namespace lpmm {
 // takes the route of the wide groups above: the update pass merges the maxima of the new first
 // moment into the next scales (one masked row maximum per group a DPP row touches) and the second
 // pass recomputes it and writes its codes; any group size from 128 to 4096 is served.  The last
-// 128-column block of a row is cut: its lanes beyond the row load nothing, store nothing and
-// contribute zeros to every maximum.  A lane's two runs of four values stay whole (the column
+// 128-column block of a row is cut: its lanes beyond the row work on the row's last run (or their own first one) once more, with a
+// column statistic of zero, and store nothing.  That changes no maximum -- the first moment is the same, the second at most what it is
+// in its own column -- and no load has a branch around it.  A lane's two runs of four values stay whole (the column
 // count is a multiple of 4), their codes are one 16-bit access each.
 // ---------------------------------------------------------------------------------------
 struct RaggedRow {
-    int64_t flat;  // index of the DPP row's first value in the flattened tensor
-    bool in0, in1;  // does the lane's first / second run of four lie inside the tensor row
+    int64_t flat;    // index of the DPP row's first value in the flattened tensor
+    int64_t f0, f1;  // of the lane's first / second run of four
+    bool in0, in1;   // does that run lie inside the tensor row
 };
 
 __device__ __forceinline__ RaggedRow ragged_row(const TensorR1 &t, int64_t cols, uint32_t cg, int lane16, int64_t r)
@@ -28,6 +30,8 @@ __device__ __forceinline__ RaggedRow ragged_row(const TensorR1 &t, int64_t cols,
     w.flat = r * cols + c0;
     w.in0 = c0 + lane16 * 4 < cols;
     w.in1 = c0 + 64 + lane16 * 4 < cols;
+    w.f0 = w.in0 ? w.flat + lane16 * 4 : (r + 1) * cols - 4;
+    w.f1 = w.in1 ? w.flat + lane16 * 4 + 64 : w.f0;
     return w;
 }
 
@@ -39,7 +43,7 @@ __global__ __launch_bounds__(kThreads) void rank1_update_ragged_kernel(const Mul
     uint32_t *rowred = colred + kMaxWide * kRedSlotWords;
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const uint32_t tl = xcd_neighbours(blockIdx.x - args.tile_start[lo], args.tile_start[lo + 1] - args.tile_start[lo]);
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
@@ -75,23 +79,18 @@ __global__ __launch_bounds__(kThreads) void rank1_update_ragged_kernel(const Mul
             if (r >= t.rows)
                 break;
             const RaggedRow w = ragged_row(t, cols, q.cg, lane16, r);
-            const int64_t f0 = w.flat + lane16 * 4, f1 = f0 + 64;
-            const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const float4 a0 = w.in0 ? load4(t.p + f0) : zero4, a1 = w.in1 ? load4(t.p + f1) : zero4;
-            const float4 b0 = w.in0 ? load4(t.g + f0) : zero4, b1 = w.in1 ? load4(t.g + f1) : zero4;
+            const int64_t f0 = w.f0, f1 = w.f1;
+            // without the nontemporal hint: the lines at a piece's ends are read by two workgroups (the tiles beside it are on the same
+            // XCD).  Six tensors of 4096 x 4104, update pass: 290 -> 255-267 us, thirty of 1000 x 1000 83 -> 70.  In the second
+            // pass, the last to read g, the hint is better where the gradients are more than the cache holds (201 against 210).
+            const float4 a0 = *reinterpret_cast<const float4 *>(t.p + f0), a1 = *reinterpret_cast<const float4 *>(t.p + f1);
+            const float4 b0 = *reinterpret_cast<const float4 *>(t.g + f0), b1 = *reinterpret_cast<const float4 *>(t.g + f1);
             const int64_t g0 = f0 >> lg_group, g1 = f1 >> lg_group;
-            uint32_t wm = 0, wv = 0;
-            float sm0 = 0.0f, sm1 = 0.0f;
-            if (w.in0) {
-                wm = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (f0 >> 1)));
-                wv = load_u16(reinterpret_cast<const uint16_t *>(t.vc + (f0 >> 1)));
-                sm0 = t.ms[g0];
-            }
-            if (w.in1) {
-                wm |= (uint32_t)load_u16(reinterpret_cast<const uint16_t *>(t.mc + (f1 >> 1))) << 16;
-                wv |= (uint32_t)load_u16(reinterpret_cast<const uint16_t *>(t.vc + (f1 >> 1))) << 16;
-                sm1 = t.ms[g1];
-            }
+            const uint32_t wm = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (f0 >> 1))) |
+                                load_u16(reinterpret_cast<const uint16_t *>(t.mc + (f1 >> 1))) << 16;
+            const uint32_t wv = load_u16(reinterpret_cast<const uint16_t *>(t.vc + (f0 >> 1))) |
+                                load_u16(reinterpret_cast<const uint16_t *>(t.vc + (f1 >> 1))) << 16;
+            const float sm0 = t.ms[g0], sm1 = t.ms[g1];
             const float ro = t.row_old[r];
             float pv[kEltsPerLane], gv[kEltsPerLane], m[kEltsPerLane], v[kEltsPerLane];
             unpack8(a0, a1, pv);
@@ -100,10 +99,9 @@ __global__ __launch_bounds__(kThreads) void rank1_update_ragged_kernel(const Mul
             float max0 = 0.0f, max1 = 0.0f, vmax = 0.0f;
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
-                // outside the row: p = g = 0 and zero scales, so m = v = 0 and nothing below sees them
                 m[k] = decode_nibble(lds, kLdsQ0, nm, k) * (k < 4 ? sm0 : sm1);
                 const float sc = (co[k] < ro) ? co[k] : ro;
-                v[k] = decode_nibble(lds, kLdsQ1, nv, k) * ((k < 4 ? w.in0 : w.in1) ? sc : 0.0f);
+                v[k] = decode_nibble(lds, kLdsQ1, nv, k) * sc;
                 nonfused_elt(pv[k], gv[k], m[k], v[k], h);
                 if (k < 4)
                     max0 = fmaxf(max0, fabsf(m[k]));
@@ -153,7 +151,7 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_ragged_kernel(const Mu
     const int kind_m = classify_map(qmap_m), kind_v = classify_map(qmap_v);
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
-    const uint32_t tl = blockIdx.x - args.tile_start[lo];
+    const uint32_t tl = xcd_neighbours(blockIdx.x - args.tile_start[lo], args.tile_start[lo + 1] - args.tile_start[lo]);
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)(t.col_blocks - 1) * kGroup + t.col_tail;
@@ -216,25 +214,13 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_ragged_kernel(const Mu
         if (r >= t.rows)
             break;
         const RaggedRow w = ragged_row(t, cols, q.cg, lane16, r);
-        const int64_t f0 = w.flat + lane16 * 4, f1 = f0 + 64;
-        const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        const float4 b0 = w.in0 ? load4(t.g + f0) : zero4, b1 = w.in1 ? load4(t.g + f1) : zero4;
+        const int64_t f0 = w.f0, f1 = w.f1;
+        const float4 b0 = load4(t.g + f0), b1 = load4(t.g + f1);
         uint16_t *mc0 = reinterpret_cast<uint16_t *>(t.mc + (f0 >> 1)), *mc1 = reinterpret_cast<uint16_t *>(t.mc + (f1 >> 1));
         uint16_t *vc0 = reinterpret_cast<uint16_t *>(t.vc + (f0 >> 1)), *vc1 = reinterpret_cast<uint16_t *>(t.vc + (f1 >> 1));
-        uint32_t wm = 0, wv = 0;
-        float so0 = 0.0f, so1 = 0.0f, sn0 = 1.0f, sn1 = 1.0f;  // outside the row: 0 / 1
-        if (w.in0) {
-            wm = load_u16(mc0);
-            wv = load_u16(vc0);
-            so0 = t.ms[f0 >> lg_group];
-            sn0 = t.ms_new[f0 >> lg_group];
-        }
-        if (w.in1) {
-            wm |= (uint32_t)load_u16(mc1) << 16;
-            wv |= (uint32_t)load_u16(vc1) << 16;
-            so1 = t.ms[f1 >> lg_group];
-            sn1 = t.ms_new[f1 >> lg_group];
-        }
+        const uint32_t wm = load_u16(mc0) | load_u16(mc1) << 16, wv = load_u16(vc0) | load_u16(vc1) << 16;
+        const float so0 = t.ms[f0 >> lg_group], so1 = t.ms[f1 >> lg_group];
+        const float sn0 = t.ms_new[f0 >> lg_group], sn1 = t.ms_new[f1 >> lg_group];
         const float ro = t.row_old[r], rn = t.row_new[r];
         float gv[kEltsPerLane], v[kEltsPerLane], m[kEltsPerLane], x[kEltsPerLane];
         unpack8(b0, b1, gv);

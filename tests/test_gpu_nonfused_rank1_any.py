@@ -104,6 +104,17 @@ def test_every_column_count(oracle, kind):
             _check(kind, opt, p, h, before, st, f"step {step} tensor {i} {SHAPES[i]}")
 
 
+# columns that are a multiple of 4 (runs of four a lane), on either side of a whole column block, with one run in the last block and one
+# missing
+RUN_SHAPES = [(70, 60), (61, 68), (33, 132), (20, 252), (300, 260), (9, 1004), (131, 196), (40, 132), (65, 388), (1030, 36)]
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+def test_columns_in_runs_of_four(oracle, kind, monkeypatch):
+    monkeypatch.setitem(globals(), "SHAPES", RUN_SHAPES)
+    test_every_column_count(oracle, kind)
+
+
 def test_half_infinities_and_nans(oracle, qmaps):
     """Gradients whose squares overflow a half, an infinite one and a NaN: statistics, scales and codes as the chain of
     half ops leaves them (a NaN is the maximum of its row, its column and its group)."""
@@ -159,10 +170,18 @@ def test_a_nan_gradient_costs_its_own_parameter(kind, monkeypatch):
     """One NaN gradient: parameters, statistics, scales and codes of the step after it and of two more are those of the
     staged route (dequantise, update, quantise), and every other parameter stays finite.  (Of more than two dimensions only
     the latter: the staged route's statistics keep a NaN there, and lose whole slices to it.)"""
+    _nan_case(kind, [(70, 61), (33, 129), (40, 257)] + [(24, 10, 5, 5)] * (kind == "codes4"), monkeypatch)
+
+
+@pytest.mark.parametrize("kind", ["codes4", "float_m", "codes5", "codes8"])
+def test_a_nan_gradient_in_runs_of_four(kind, monkeypatch):
+    _nan_case(kind, [(70, 60), (33, 132), (40, 260)], monkeypatch)
+
+
+def _nan_case(kind, shapes, monkeypatch):
     import lpmm.optim.adamw as adamw
     from lpmm import _native
 
-    shapes = [(70, 61), (33, 129), (40, 257)] + [(24, 10, 5, 5)] * (kind == "codes4")
     (_, params, opt), (_, staged_params, staged) = (_setup(kind, shapes, np.random.default_rng(94)) for _ in range(2))
     rng = np.random.default_rng(95)
     for step in range(4):
