@@ -63,7 +63,7 @@ struct PassRegs {
     float sm, ro, ro1;  // ro1: the second half's row statistic (folded rows; otherwise ro)
 };
 
-template <int MODE, bool FOLD>
+template <int MODE, bool FOLD, bool KEEP>
 __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uint32_t cg, int lane16, int64_t r, PassRegs &x)
 {
     const int64_t grp = r * f.col_blocks + cg;
@@ -72,8 +72,8 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
     const float *gp = t.g + gbase + lane16 * 4;
     x.a0 = load4(pp);
     x.a1 = load4(pp + 64);
-    x.b0 = load4(gp);
-    x.b1 = load4(gp + 64);
+    x.b0 = load4_for<KEEP>(gp);
+    x.b1 = load4_for<KEEP>(gp + 64);
     const uint16_t *vcp = reinterpret_cast<const uint16_t *>(t.vc + (gbase >> 1)) + lane16;
     if (MODE == kMFloat) {
         const float *mp = reinterpret_cast<const float *>(t.mc) + gbase + lane16 * 4;
@@ -85,8 +85,8 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
         x.m1 = load_u16(mcp + 16);
         x.sm = t.ms[MODE == kMCodesWide ? grp >> t.m_lg : grp];
     }
-    x.v0 = load_u16(vcp);
-    x.v1 = load_u16(vcp + 16);
+    x.v0 = load_u16_for<KEEP>(vcp);
+    x.v1 = load_u16_for<KEEP>(vcp + 16);
     if (FOLD) {
         int64_t r0, r1;
         fold_rows(f, r, cg, r0, r1);
@@ -102,7 +102,7 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
 #endif
 // 4 waves per SIMD, up to 128 registers: the first pass's operands stay live across the prologue and
 // the lane's column statistics across the passes (with 5 or 6 the compiler spills or re-reads)
-template <int MODE, bool FOLD>
+template <int MODE, bool FOLD, bool KEEP>
 __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                 const float *__restrict__ qmap_v)
 {
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
     const bool row_live = q.cg < f.col_blocks;  // the whole DPP row
     PassRegs x;
     if (row_live && q.row0 < f.rows)
-        pass_fetch<MODE, FOLD>(t, f, q.cg, lane16, q.row0, x);
+        pass_fetch<MODE, FOLD, KEEP>(t, f, q.cg, lane16, q.row0, x);
     lds_fill_store(lds, fill);
     for (int j = threadIdx.x; j < kMaxWide * (int)kRedSlotWords; j += kThreads)
         colred[j] = 0u;
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
             if (r >= f.rows)
                 break;
             if (it > 0)
-                pass_fetch<MODE, FOLD>(t, f, q.cg, lane16, r, x);
+                pass_fetch<MODE, FOLD, KEEP>(t, f, q.cg, lane16, r, x);
             const int64_t grp = r * f.col_blocks + q.cg;
             const int64_t gbase = grp * kGroup;
             float *pp = t.p + gbase + lane16 * 4;
@@ -509,6 +509,13 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     return l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
 }
 
+// Launches of at most this many values leave the gradient and the second moment's codes in the cache (R1Launch::keep).  The memory-side
+// cache holds 256 MB, the gradients of 64M values; the tail of a larger launch still finds its part there.  Steps (us; hint on all loads, then
+// without it on these): one to three tensors of 4096 x 4096 65.1 -> 63.0, 122.5 -> 116.8, 174.9 -> 166.4, eight 434.5 -> 427.3;
+// 8 bits 78.7 -> 75.7 ... 212.8 -> 199.1; 30 of 512 x 2048 120.9 -> 116.2; GPT-2-XL's set (launches of 210M) 5605 -> 5470; but four
+// decoder layers of width 4096 (809M) 2451 -> 2507.
+constexpr double kKeepValues = 256e6;
+
 // The first moment of a record: its codes and scales, or the fp32 moment itself.
 static uint8_t *first_moment(const lpmm_nonfused_rank1_tensor &t) { return t.m_codes; }
 static float *first_moment_scales(const lpmm_nonfused_rank1_tensor &t) { return t.m_max1; }
@@ -526,9 +533,10 @@ static bool folds(int64_t rows, int64_t cols) { return cols % kGroup == 64 && ro
 template <int MODE, bool FOLD>
 static void launch_rank1_passes(const R1Launch &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
 {
-    if (passes & 1)
-        hipLaunchKernelGGL((rank1_update_kernel<MODE, FOLD>), dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m,
-                           qmap_v);
+    if (passes & 1) {
+        const auto update = l.keep ? rank1_update_kernel<MODE, FOLD, true> : rank1_update_kernel<MODE, FOLD, false>;
+        hipLaunchKernelGGL(update, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
+    }
     if (passes & 2)
         hipLaunchKernelGGL((rank1_requant_kernel<MODE == kMCodesWide, FOLD>), dim3(l.requant_tiles), dim3(kThreads), 0, stream,
                            l.requant, qmap_m, qmap_v);
@@ -738,6 +746,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         memcpy(l.requant.tile_start, start2, sizeof start2);
         l.update_tiles = (uint32_t)tiles;
         l.requant_tiles = (uint32_t)tiles2;
+        l.keep = kind.values <= kKeepValues;
         if (general) {
             const AnyKind any = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
             launch_rank1_any(l, *out, qmap_m, qmap_v, any, bits_m, bits_v, static_cast<const uint32_t *>(table_m),

@@ -38,6 +38,7 @@ __device__ __forceinline__ void write_padding_bytes(uint8_t *codes, int64_t n, i
         codes[n_padded] = 0;
 }
 
+template <bool KEEP>
 __global__ __launch_bounds__(kThreads) void rank1_update_bits_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                     const float *__restrict__ qmap_v, int bits_m,
                                                                     int bits_v, const uint32_t *__restrict__ table_m)
@@ -110,12 +111,12 @@ __global__ __launch_bounds__(kThreads) void rank1_update_bits_kernel(const Multi
             const uint32_t *vcp = reinterpret_cast<const uint32_t *>(t.vc + gbase) + lane16;
             x.a0 = load4(pp);
             x.a1 = load4(pp + 64);
-            x.b0 = load4(gp);
-            x.b1 = load4(gp + 64);
+            x.b0 = load4_for<KEEP>(gp);
+            x.b1 = load4_for<KEEP>(gp + 64);
             x.wm0 = load_u32(mcp);
             x.wm1 = load_u32(mcp + 16);
-            x.wv0 = load_u32(vcp);
-            x.wv1 = load_u32(vcp + 16);
+            x.wv0 = load_u32_for<KEEP>(vcp);
+            x.wv1 = load_u32_for<KEEP>(vcp + 16);
             x.sm = t.ms[grp];
             x.ro = t.row_old[r];
             return x;
@@ -283,8 +284,8 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_bits_kernel(const Mult
 void launch_rank1_bits(const R1Launch &l, const float *qmap_m, const float *qmap_v, int bits_m,
                        int bits_v, const uint32_t *table_m, const uint32_t *table_v, hipStream_t stream)
 {
-    hipLaunchKernelGGL(rank1_update_bits_kernel, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v, bits_m,
-                       bits_v, table_m);
+    const auto update = l.keep ? rank1_update_bits_kernel<true> : rank1_update_bits_kernel<false>;
+    hipLaunchKernelGGL(update, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v, bits_m, bits_v, table_m);
     hipLaunchKernelGGL(rank1_requant_bits_kernel, dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, qmap_v, bits_v, table_v);
 }
 

@@ -222,10 +222,23 @@ __device__ __forceinline__ void write_padding(uint8_t *codes, int64_t n, int64_t
         codes[n_padded / 2] = 0;
 }
 
+// Loads of what the second pass reads again (the gradient, the second moment's codes): without the nontemporal hint (KEEP) where a launch's
+// gradients fit the memory-side cache, which then serves the second pass.
+template <bool KEEP>
+__device__ __forceinline__ float4 load4_for(const float *p)
+{
+    return KEEP ? *reinterpret_cast<const float4 *>(p) : load4(p);
+}
+template <bool KEEP>
+__device__ __forceinline__ uint32_t load_u16_for(const uint16_t *p) { return KEEP ? *p : load_u16(p); }
+template <bool KEEP>
+__device__ __forceinline__ uint32_t load_u32_for(const uint32_t *p) { return KEEP ? *p : load_u32(p); }
+
 // One launch's tensors with the tile shapes of either pass (they differ: pass_rows_policy), and its workgroups.
 struct R1Launch {
     MultiR1 update, requant;
     uint32_t update_tiles, requant_tiles;
+    bool keep;  // the update pass leaves what the second pass reads again in the cache
 };
 
 // The launches of the other kernel families (defined next to their kernels).
