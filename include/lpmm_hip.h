@@ -120,6 +120,18 @@ int lpmm_adamw_fp32_step_multi(const lpmm_adamw_fp32_tensor *tensors, int64_t co
                                float beta1, float beta2, float lr, float weight_decay,
                                float eps, void *stream);
 
+/* Both kinds of tensors of a parameter group, the quantised ones (lpmm_adamw4bit_step_multi) and those with fp32 states
+ * (lpmm_adamw_fp32_step_multi): in one launch where at most 48 of the former and 64 of the latter are given, which is what the step of a small
+ * model costs; otherwise as the two calls.  Either array may be empty. */
+int lpmm_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain,
+                                   int64_t plain_count, const float *qmap_m, const float *qmap_v, float beta1, float beta2, float lr,
+                                   float weight_decay, float eps, void *stream);
+
+/* The same for lpmm_nonfused_adamw4bit_step_multi and lpmm_nonfused_update_multi. */
+int lpmm_nonfused_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain,
+                                            int64_t plain_count, const float *qmap_m, const float *qmap_v, double beta1, double beta2,
+                                            double lr, double weight_decay, double eps, void *stream);
+
 /* The same step for IEEE half-precision tensors: the p, g, m and v of every record point to
  * fp16[n] (2-byte aligned); all arithmetic is float.  Replaces fused_adamw.adamw_single_tensor
  * for at::Half tensors (the kernel template instantiated by AT_DISPATCH_FLOATING_TYPES_AND_HALF,

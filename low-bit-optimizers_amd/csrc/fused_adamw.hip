@@ -345,11 +345,9 @@ __device__ __forceinline__ void group_step(const Tensor4 &t, const TileView &w, 
 // launch is a whole number of tiles, so no access needs a guard and the loads are straight-line
 // code.
 template <bool ALIGNED, bool ALLFULL, class Arith>
-__global__ __launch_bounds__(kThreads) void adamw4bit_kernel(const Multi4 args,
-                                                             const float *__restrict__ qmap_m,
-                                                             const float *__restrict__ qmap_v)
+__device__ __forceinline__ void tile4(const Multi4 &args, const float *__restrict__ qmap_m, const float *__restrict__ qmap_v,
+                                      uint32_t *lds)
 {
-    __shared__ __align__(16) uint32_t lds[fused_lds_bytes<ALLFULL>() / 4];
     // a short pause before the first load: see kStartDelay
     if (ALLFULL && !Arith::kPadded && kStartDelay > 0)
         __builtin_amdgcn_s_sleep(kStartDelay);
@@ -422,6 +420,14 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_kernel(const Multi4 args,
         group_step<false>(t, view, h, lds, std_maps, grp, lane16, regs);
 }
 
+template <bool ALIGNED, bool ALLFULL, class Arith>
+__global__ __launch_bounds__(kThreads) void adamw4bit_kernel(const Multi4 args, const float *__restrict__ qmap_m,
+                                                             const float *__restrict__ qmap_v)
+{
+    __shared__ __align__(16) uint32_t lds[fused_lds_bytes<ALLFULL>() / 4];
+    tile4<ALIGNED, ALLFULL, Arith>(args, qmap_m, qmap_v, lds);
+}
+
 // ---------------------------------------------------------------------------------------
 // fp32-state step (lpmm/cpp_extension/fused_adamw_kernel.cu:52-78).
 // ---------------------------------------------------------------------------------------
@@ -449,19 +455,19 @@ static_assert(sizeof(MultiF) <= 4096, "kernel arguments exceed 4 KB");
 // fp32 states, either arithmetic (the FusedArith / NonFusedArith constructors only read the
 // scalars, which Multi4 and MultiF name alike)
 template <class Arith>
-__global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
+__device__ __forceinline__ void tile_fp32(const MultiF &args, uint32_t tile)
 {
     int lo = 0, hi = args.count;
     while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
-        if (args.tile_start[mid] <= blockIdx.x)
+        if (args.tile_start[mid] <= tile)
             lo = mid;
         else
             hi = mid;
     }
     const TensorF &t = args.t[lo];
     const Arith h(args, t);
-    const int64_t tile0 = (int64_t)(blockIdx.x - args.tile_start[lo]) * kTileF;
+    const int64_t tile0 = (int64_t)(tile - args.tile_start[lo]) * kTileF;
 #pragma unroll
     for (int k = 0; k < kTileF / kThreads; ++k) {
         const int64_t i = tile0 + k * kThreads + threadIdx.x;
@@ -473,6 +479,26 @@ __global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
             t.v[i] = v;
         }
     }
+}
+
+template <class Arith>
+__global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
+{
+    tile_fp32<Arith>(args, blockIdx.x);
+}
+
+// Both kinds of tensors of a small model in one launch: the tiles of the quantised tensors, then those of the ones with fp32 states.
+// A step of such a model is bound by the host, which a launch costs about 7 us (the call, its kernel arguments, the device and stream around it):
+// fifty tensors of 7.5M values 39.5 -> 33.2 us a step.
+template <bool ALIGNED, bool ALLFULL, class Arith, class ArithF>
+__global__ __launch_bounds__(kThreads) void adamw_joined_kernel(const Multi4 args, const MultiF plain, const float *__restrict__ qmap_m,
+                                                                const float *__restrict__ qmap_v, uint32_t tiles)
+{
+    __shared__ __align__(16) uint32_t lds[fused_lds_bytes<ALLFULL>() / 4];
+    if (blockIdx.x < tiles)
+        tile4<ALIGNED, ALLFULL, Arith>(args, qmap_m, qmap_v, lds);
+    else
+        tile_fp32<ArithF>(plain, blockIdx.x - tiles);
 }
 
 // The fp32-state step on half-precision tensors: p, g, m and v are stored as IEEE half, every
@@ -516,16 +542,8 @@ __global__ __launch_bounds__(kThreads) void adamw_fp16_kernel(const MultiF args)
 
 using namespace lpmm;
 
-// Validation, batching into launches of at most LPMM_MULTI_MAX tensors, and launch, shared
-// by the arithmetics.  per_tensor(step, k) fills the per-tensor scalars.
-template <class Arith, class PerTensor>
-static int step_multi4(const lpmm_adamw4bit_tensor *tensors, int64_t count, const float *qmap_m,
-                       const float *qmap_v, const float (&scalars)[7], PerTensor per_tensor, void *stream)
+static int check4(const lpmm_adamw4bit_tensor *tensors, int64_t count, const float *qmap_m, const float *qmap_v)
 {
-    if (count < 0)
-        return LPMM_ERR_SIZE;
-    if (count == 0)
-        return LPMM_OK;
     LPMM_REQUIRE_PTR(tensors);
     LPMM_REQUIRE_PTR(qmap_m);
     LPMM_REQUIRE_PTR(qmap_v);
@@ -550,59 +568,79 @@ static int step_multi4(const lpmm_adamw4bit_tensor *tensors, int64_t count, cons
         if ((t.n + kTile - 1) / kTile > 0x7fffffffLL)
             return LPMM_ERR_SIZE;
     }
+    return LPMM_OK;
+}
 
+// One launch's records from tensors[i] on, at most LPMM_MULTI_MAX that are not empty; its tiles (0: none left).
+struct Launch4 {
+    bool aligned, allfull;  // do all pointers allow vector access, is every tensor a whole number of tiles
+    uint32_t tiles;
+};
+
+template <class PerTensor>
+static Launch4 fill4(Multi4 &args, const lpmm_adamw4bit_tensor *tensors, int64_t count, int64_t &i, PerTensor per_tensor)
+{
+    int k = 0;
+    uint64_t tiles = 0;
+    bool aligned = true, allfull = true;
+    args.tile_start[0] = 0;
+    while (i < count && k < LPMM_MULTI_MAX) {
+        const lpmm_adamw4bit_tensor &t = tensors[i];
+        if (t.n == 0) {
+            ++i;
+            continue;
+        }
+        const uint64_t nt = (uint64_t)((t.n + kTile - 1) / kTile);
+        if (tiles + nt > 0x7fffffffULL)
+            break;
+        allfull = allfull && (t.n % kTile) == 0;
+        aligned = aligned && aligned_to(t.p, 16) && aligned_to(t.g, 16) && aligned_to(t.m_codes, 2) &&
+                  aligned_to(t.v_codes, 2);
+        Tensor4 &d = args.t[k];
+        d.p = t.p;
+        d.g = t.g;
+        d.mc = t.m_codes;
+        d.vc = t.v_codes;
+        d.ms = t.m_scale;
+        d.vs = t.v_scale;
+        d.n = t.n;
+        per_tensor(t.step, d.k);
+        tiles += nt;
+        args.tile_start[++k] = (uint32_t)tiles;
+        ++i;
+    }
+    args.count = k;
+    for (int j = k + 1; j < kStartSlots; ++j)
+        args.tile_start[j] = (uint32_t)tiles;
+    for (int j = 0; j < kCoarseSlots; ++j)
+        args.coarse[j] = args.tile_start[8 * (j + 1)];
+    return {aligned, allfull, (uint32_t)tiles};
+}
+
+// Validation, batching into launches of at most LPMM_MULTI_MAX tensors, and launch, shared
+// by the arithmetics.  per_tensor(step, k) fills the per-tensor scalars.
+template <class Arith, class PerTensor>
+static int step_multi4(const lpmm_adamw4bit_tensor *tensors, int64_t count, const float *qmap_m,
+                       const float *qmap_v, const float (&scalars)[7], PerTensor per_tensor, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    const int bad = check4(tensors, count, qmap_m, qmap_v);
+    if (bad != LPMM_OK)
+        return bad;
     Multi4 args;
     for (int j = 0; j < 7; ++j)
         args.s[j] = scalars[j];
-    int64_t i = 0;
-    while (i < count) {
-        int k = 0;
-        uint64_t tiles = 0;
-        // per launch: do all pointers allow vector access, is every tensor a whole number of tiles
-        bool aligned = true, allfull = true;
-        args.tile_start[0] = 0;
-        while (i < count && k < LPMM_MULTI_MAX) {
-            const lpmm_adamw4bit_tensor &t = tensors[i];
-            if (t.n == 0) {
-                ++i;
-                continue;
-            }
-            const uint64_t nt = (uint64_t)((t.n + kTile - 1) / kTile);
-            if (tiles + nt > 0x7fffffffULL)
-                break;
-            allfull = allfull && (t.n % kTile) == 0;
-            aligned = aligned && aligned_to(t.p, 16) && aligned_to(t.g, 16) && aligned_to(t.m_codes, 2) &&
-                      aligned_to(t.v_codes, 2);
-            Tensor4 &d = args.t[k];
-            d.p = t.p;
-            d.g = t.g;
-            d.mc = t.m_codes;
-            d.vc = t.v_codes;
-            d.ms = t.m_scale;
-            d.vs = t.v_scale;
-            d.n = t.n;
-            per_tensor(t.step, d.k);
-            tiles += nt;
-            args.tile_start[++k] = (uint32_t)tiles;
-            ++i;
-        }
-        if (k == 0)
+    for (int64_t i = 0; i < count;) {
+        const Launch4 l = fill4(args, tensors, count, i, per_tensor);
+        if (l.tiles == 0)
             continue;
-        args.count = k;
-        for (int j = k + 1; j < kStartSlots; ++j)
-            args.tile_start[j] = (uint32_t)tiles;
-        for (int j = 0; j < kCoarseSlots; ++j)
-            args.coarse[j] = args.tile_start[8 * (j + 1)];
-        const dim3 grid((uint32_t)tiles), block(kThreads);
-        if (aligned && allfull)
-            hipLaunchKernelGGL((adamw4bit_kernel<true, true, Arith>), grid, block, 0, (hipStream_t)stream, args,
-                               qmap_m, qmap_v);
-        else if (aligned)
-            hipLaunchKernelGGL((adamw4bit_kernel<true, false, Arith>), grid, block, 0, (hipStream_t)stream, args,
-                               qmap_m, qmap_v);
-        else
-            hipLaunchKernelGGL((adamw4bit_kernel<false, false, Arith>), grid, block, 0, (hipStream_t)stream, args,
-                               qmap_m, qmap_v);
+        const auto kernel = l.aligned && l.allfull ? adamw4bit_kernel<true, true, Arith>
+                            : l.aligned            ? adamw4bit_kernel<true, false, Arith>
+                                                   : adamw4bit_kernel<false, false, Arith>;
+        hipLaunchKernelGGL(kernel, dim3(l.tiles), dim3(kThreads), 0, (hipStream_t)stream, args, qmap_m, qmap_v);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;
@@ -658,15 +696,8 @@ extern "C" int lpmm_adamw4bit_step(float *p, const float *g, uint8_t *m_codes, u
     return lpmm_adamw4bit_step_multi(&t, 1, qmap_m, qmap_v, beta1, beta2, lr, weight_decay, eps, stream);
 }
 
-template <class Arith, bool HALF = false, class PerTensor>
-static int step_multi_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count, const float (&scalars)[7],
-                           PerTensor per_tensor, void *stream)
+static int check_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count, uintptr_t elt_align)
 {
-    constexpr uintptr_t kEltAlign = HALF ? 2 : 4;
-    if (count < 0)
-        return LPMM_ERR_SIZE;
-    if (count == 0)
-        return LPMM_OK;
     LPMM_REQUIRE_PTR(tensors);
     for (int64_t i = 0; i < count; ++i) {
         const lpmm_adamw_fp32_tensor &t = tensors[i];
@@ -678,54 +709,135 @@ static int step_multi_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count,
         LPMM_REQUIRE_PTR(t.g);
         LPMM_REQUIRE_PTR(t.m);
         LPMM_REQUIRE_PTR(t.v);
-        LPMM_REQUIRE_ALIGN(t.p, kEltAlign);
-        LPMM_REQUIRE_ALIGN(t.g, kEltAlign);
-        LPMM_REQUIRE_ALIGN(t.m, kEltAlign);
-        LPMM_REQUIRE_ALIGN(t.v, kEltAlign);
+        LPMM_REQUIRE_ALIGN(t.p, elt_align);
+        LPMM_REQUIRE_ALIGN(t.g, elt_align);
+        LPMM_REQUIRE_ALIGN(t.m, elt_align);
+        LPMM_REQUIRE_ALIGN(t.v, elt_align);
     }
+    return LPMM_OK;
+}
+
+// As fill4: the launch's tiles.
+template <class PerTensor>
+static uint32_t fill_fp32(MultiF &args, const lpmm_adamw_fp32_tensor *tensors, int64_t count, int64_t &i, PerTensor per_tensor)
+{
+    int k = 0;
+    uint64_t tiles = 0;
+    args.tile_start[0] = 0;
+    while (i < count && k < kMultiFMax) {
+        const lpmm_adamw_fp32_tensor &t = tensors[i];
+        if (t.n == 0) {
+            ++i;
+            continue;
+        }
+        const uint64_t nt = (uint64_t)((t.n + kTileF - 1) / kTileF);
+        if (tiles + nt > 0x7fffffffULL)
+            break;
+        TensorF &d = args.t[k];
+        d.p = t.p;
+        d.g = t.g;
+        d.m = t.m;
+        d.v = t.v;
+        d.n = t.n;
+        per_tensor(t.step, d.k);
+        tiles += nt;
+        args.tile_start[++k] = (uint32_t)tiles;
+        ++i;
+    }
+    args.count = k;
+    for (int j = k + 1; j <= kMultiFMax; ++j)
+        args.tile_start[j] = (uint32_t)tiles;
+    return (uint32_t)tiles;
+}
+
+template <class Arith, bool HALF = false, class PerTensor>
+static int step_multi_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count, const float (&scalars)[7],
+                           PerTensor per_tensor, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    const int bad = check_fp32(tensors, count, HALF ? 2 : 4);
+    if (bad != LPMM_OK)
+        return bad;
     MultiF args;
     for (int j = 0; j < 7; ++j)
         args.s[j] = scalars[j];
-    int64_t i = 0;
-    while (i < count) {
-        int k = 0;
-        uint64_t tiles = 0;
-        args.tile_start[0] = 0;
-        while (i < count && k < kMultiFMax) {
-            const lpmm_adamw_fp32_tensor &t = tensors[i];
-            if (t.n == 0) {
-                ++i;
-                continue;
-            }
-            const uint64_t nt = (uint64_t)((t.n + kTileF - 1) / kTileF);
-            if (tiles + nt > 0x7fffffffULL)
-                break;
-            TensorF &d = args.t[k];
-            d.p = t.p;
-            d.g = t.g;
-            d.m = t.m;
-            d.v = t.v;
-            d.n = t.n;
-            per_tensor(t.step, d.k);
-            tiles += nt;
-            args.tile_start[++k] = (uint32_t)tiles;
-            ++i;
-        }
-        if (k == 0)
+    for (int64_t i = 0; i < count;) {
+        const uint32_t tiles = fill_fp32(args, tensors, count, i, per_tensor);
+        if (tiles == 0)
             continue;
-        args.count = k;
-        for (int j = k + 1; j <= kMultiFMax; ++j)
-            args.tile_start[j] = (uint32_t)tiles;
-        if (HALF)
-            hipLaunchKernelGGL(adamw_fp16_kernel, dim3((uint32_t)tiles), dim3(kThreads), 0, (hipStream_t)stream, args);
-        else
-            hipLaunchKernelGGL(adamw_fp32_kernel<Arith>, dim3((uint32_t)tiles), dim3(kThreads), 0,
-                               (hipStream_t)stream, args);
+        hipLaunchKernelGGL(HALF ? adamw_fp16_kernel : adamw_fp32_kernel<Arith>, dim3(tiles), dim3(kThreads), 0, (hipStream_t)stream,
+                           args);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;
     }
     return LPMM_OK;
+}
+
+// Quantised tensors and tensors with fp32 states of one parameter group: one launch where both fit one, else two kinds of launches.
+template <class Arith, class ArithF, class PerTensor, class PerTensorF>
+static int step_joined(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain, int64_t plain_count,
+                       const float *qmap_m, const float *qmap_v, const float (&scalars)[7], PerTensor per_tensor,
+                       PerTensorF per_tensor_f, void *stream)
+{
+    if (count < 0 || plain_count < 0)
+        return LPMM_ERR_SIZE;
+    int bad = count == 0 ? LPMM_OK : check4(tensors, count, qmap_m, qmap_v);
+    if (bad == LPMM_OK && plain_count != 0)
+        bad = check_fp32(plain, plain_count, 4);
+    if (bad != LPMM_OK)
+        return bad;
+    if (count != 0 && plain_count != 0 && count <= LPMM_MULTI_MAX && plain_count <= kMultiFMax) {
+        Multi4 args;
+        MultiF args_f;
+        for (int j = 0; j < 7; ++j)
+            args.s[j] = args_f.s[j] = scalars[j];
+        int64_t i = 0, i_f = 0;
+        const Launch4 l = fill4(args, tensors, count, i, per_tensor);
+        const uint32_t tiles_f = fill_fp32(args_f, plain, plain_count, i_f, per_tensor_f);
+        if (l.tiles != 0 && tiles_f != 0 && i == count && i_f == plain_count && (uint64_t)l.tiles + tiles_f <= 0x7fffffffULL) {
+            const auto kernel = l.aligned && l.allfull ? adamw_joined_kernel<true, true, Arith, ArithF>
+                                : l.aligned            ? adamw_joined_kernel<true, false, Arith, ArithF>
+                                                       : adamw_joined_kernel<false, false, Arith, ArithF>;
+            hipLaunchKernelGGL(kernel, dim3(l.tiles + tiles_f), dim3(kThreads), 0, (hipStream_t)stream, args, args_f, qmap_m, qmap_v,
+                               l.tiles);
+            return launch_status();
+        }
+    }
+    bad = step_multi4<Arith>(tensors, count, qmap_m, qmap_v, scalars, per_tensor, stream);
+    return bad != LPMM_OK ? bad : step_multi_fp32<ArithF>(plain, plain_count, scalars, per_tensor_f, stream);
+}
+
+extern "C" int lpmm_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain,
+                                              int64_t plain_count, const float *qmap_m, const float *qmap_v, float beta1, float beta2,
+                                              float lr, float weight_decay, float eps, void *stream)
+{
+    const float scalars[7] = {beta1, beta2, 1 - beta1, 1 - beta2, lr, weight_decay, eps};
+    return step_joined<FusedStep4, FusedArith>(
+        tensors, count, plain, plain_count, qmap_m, qmap_v, scalars,
+        [=](float step, float (&k)[4]) { FusedStep4::per_tensor(beta1, beta2, eps, step, k); },
+        [=](float step, float (&k)[4]) { FusedArith::per_tensor(beta1, beta2, eps, step, k); }, stream);
+}
+
+extern "C" int lpmm_nonfused_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count,
+                                                       const lpmm_adamw_fp32_tensor *plain, int64_t plain_count, const float *qmap_m,
+                                                       const float *qmap_v, double beta1, double beta2, double lr, double weight_decay,
+                                                       double eps, void *stream)
+{
+    const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
+    const float scalars[7] = {c.decay, c.w1, c.b2, c.w2, c.eps, 0.0f, 0.0f};
+    const auto per_tensor = [=](float step, float (&k)[4]) {
+        const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, step);
+        k[0] = h.neg_step_size;
+        k[1] = h.bc2_sqrt;
+        k[2] = h.rbc2_sqrt;
+        k[3] = 0.0f;
+    };
+    return step_joined<NonFusedArith, NonFusedArith>(tensors, count, plain, plain_count, qmap_m, qmap_v, scalars, per_tensor, per_tensor,
+                                                     stream);
 }
 
 extern "C" int lpmm_adamw_fp32_step_multi(const lpmm_adamw_fp32_tensor *tensors, int64_t count,

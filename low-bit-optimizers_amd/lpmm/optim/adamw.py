@@ -256,16 +256,37 @@ class AdamW(LowBitOptimizer):
              routes.m_group_wide, routes.bits_rank1, routes.m_group),
             _native.factored_workspace())
 
+    @staticmethod
+    def _joined(batches, fused):
+        """Where the quantised tensors and those with fp32 states stand that share one launch, or two Nones: a small model's."""
+        quantised, four, plain = _native.WALK_FUSED4 if fused else _native.WALK_FLAT, None, None
+        for k, batch in enumerate(batches):
+            if batch[0] == _native.WALK_PLAIN and batch[5] <= _native.PLAIN_MULTI_MAX:
+                plain = k
+            elif batch[0] == quantised and batch[5] <= _native.MULTI_MAX:
+                four = k
+        if four is None or plain is None or batches[four][1] != batches[plain][1]:
+            return None, None
+        return four, plain
+
     def _launch_walk(self, group, plan, routes):
         """The launches of the walk's records: those that _step_fused and _step_single make."""
         beta1, beta2 = group["betas"]
         hyper = (beta1, beta2, group["lr"], group["weight_decay"], group["eps"])
         lib = _native.lib()
-        for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(plan.start()):
+        batches = plan.start()
+        four, plain = self._joined(batches, group["fused"])
+        for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(batches):
+            if k == plain:
+                continue  # goes with the quantised tensors
             with torch.cuda.device(index):
                 stream = _native.current_stream(index)
                 qm_ptr, qv_ptr = (None if q is None else q.data_ptr() for q in (qm, qv))
-                if kind == _native.WALK_FUSED4:
+                if k == four:
+                    run = lib.lpmm_adamw4bit_fp32_step_multi if group["fused"] else lib.lpmm_nonfused_adamw4bit_fp32_step_multi
+                    plain_count, plain_records = batches[plain][5:7]
+                    st = run(records, count, plain_records, plain_count, qm_ptr, qv_ptr, *hyper, stream)
+                elif kind == _native.WALK_FUSED4:
                     st = lib.lpmm_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
                 elif kind == _native.WALK_PLAIN:
                     run = lib.lpmm_adamw_fp32_step_multi if group["fused"] else lib.lpmm_nonfused_update_multi

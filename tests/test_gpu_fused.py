@@ -406,3 +406,50 @@ def test_fused_multi_step_under_graph_capture(qmaps):
             c["g"].copy_(torch.randn(c["n"], device="cuda", generator=gen) * 1e-3)
         for c, e in zip(captured, eager):
             e["g"].copy_(c["g"])
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("sizes", ["whole", "ragged", "shifted"])
+@pytest.mark.parametrize("counts", [(0, 3), (3, 0), (1, 1), (48, 64), (49, 64), (48, 65), (5, 130)])
+def test_joined_launch_equals_two(qmaps, counts, sizes, fused):
+    """Quantised tensors and tensors with fp32 states in one call (one launch up to 48 and 64 of them): the bytes of the two calls."""
+    nat = _native()
+    lib = nat.lib()
+    dqm, dqv = (to_dev(q) for q in qmaps)
+    rng = np.random.default_rng(7)
+    n4 = [2048 * int(k) if sizes == "whole" else int(k) * 1000 + 130 for k in rng.integers(2, 6, counts[0])]
+    nf = [int(k) for k in rng.integers(1, 4097, counts[1])]
+    shift = 1 if sizes == "shifted" else 0
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def tensors():
+        gen = np.random.default_rng(8)
+        four, plain = [], []
+        for n in n4:
+            pad = -(-n // 2048) * 2048
+            four.append([to_dev(gen.standard_normal(n + shift).astype(np.float32)) for _ in range(2)]
+                        + [to_dev(gen.integers(0, 256, pad // 2 + 1, dtype=np.uint8)) for _ in range(2)]
+                        + [to_dev(np.abs(gen.standard_normal(pad // 128)).astype(np.float32)) for _ in range(2)])
+        for n in nf:
+            plain.append([to_dev(np.abs(gen.standard_normal(n)).astype(np.float32)) for _ in range(4)])
+        table = np.array([tuple(t.data_ptr() + 4 * shift * (i < 2) for i, t in enumerate(ts)) + (n, 1.0 + j, 0.0)
+                          for j, (ts, n) in enumerate(zip(four, n4))], dtype=nat.ADAMW4BIT_TENSOR)
+        table_f = np.array([tuple(t.data_ptr() for t in ts) + (n, 1.0 + j, 0.0) for j, (ts, n) in enumerate(zip(plain, nf))],
+                           dtype=nat.ADAMW_FP32_TENSOR)
+        return four + plain, table, table_f
+
+    hyper = (0.9, 0.999, 1e-3, 0.01, 1e-8)
+    joined, table, table_f = tensors()
+    both = lib.lpmm_adamw4bit_fp32_step_multi if fused else lib.lpmm_nonfused_adamw4bit_fp32_step_multi
+    assert both(table.ctypes.data, len(n4), table_f.ctypes.data, len(nf), dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) == 0
+    apart, table, table_f = tensors()
+    one, other = ((lib.lpmm_adamw4bit_step_multi, lib.lpmm_adamw_fp32_step_multi) if fused else
+                  (lib.lpmm_nonfused_adamw4bit_step_multi, lib.lpmm_nonfused_update_multi))
+    assert one(table.ctypes.data, len(n4), dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) == 0
+    assert other(table_f.ctypes.data, len(nf), *hyper, stream) == 0
+    torch.cuda.synchronize()
+    for i, (a, b) in enumerate(zip(joined, apart)):
+        for x, y in zip(a, b):
+            assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), i
+    assert both(None, 1, table_f.ctypes.data, len(nf), dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) != 0
+    assert both(table.ctypes.data, -1, table_f.ctypes.data, 1, dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) != 0
