@@ -133,9 +133,10 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                        : 0u;
     }
     const bool row_live = q.cg < f.col_blocks;  // the whole DPP row
+    // No branch around the first pass's loads: behind one the compiler waits for all of them before the LDS writes, as the path without
+    // them has nothing else to count.  A DPP row without work loads what is there.
     PassRegs x;
-    if (row_live && q.row0 < f.rows)
-        pass_fetch<MODE, FOLD, KEEP>(t, f, q.cg, lane16, q.row0, x);
+    pass_fetch<MODE, FOLD, KEEP>(t, f, row_live ? q.cg : f.col_blocks - 1u, lane16, q.row0 < f.rows ? q.row0 : f.rows - 1, x);
     lds_fill_store(lds, fill);
     for (int j = threadIdx.x; j < kMaxWide * (int)kRedSlotWords; j += kThreads)
         colred[j] = 0u;
@@ -349,24 +350,26 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1 a
             break;
         const int64_t gbase = (r * f.col_blocks + q.cg) * kGroup;
         const float *gp = t.g + gbase + lane16 * 4;
+        int64_t r0 = r, r1 = r;  // the tensor rows of the DPP row's two halves
+        if (FOLD)
+            fold_rows(f, r, q.cg, r0, r1);
         const float4 b0 = load4(gp), b1 = load4(gp + 64);
         uint32_t *vcp = reinterpret_cast<uint32_t *>(t.vc + (gbase >> 1)) + code_dword;
-        const uint32_t wv = swap_code_halves(load_u32(vcp), code_sel);
+        const uint32_t in_v = load_u32(vcp);
+        const float ro = t.row_old[r0], rn = t.row_new[r0];
+        const float ro1 = FOLD ? t.row_old[r1] : ro, rn1 = FOLD ? t.row_new[r1] : rn;
         uint32_t *mcp = nullptr;
         uint32_t wm = 0;
         float ms_old = 0.0f, ms_new = 0.0f;
         if (MWIDE) {
             mcp = reinterpret_cast<uint32_t *>(t.mc + (gbase >> 1)) + code_dword;
-            wm = swap_code_halves(load_u32(mcp), code_sel);
+            const uint32_t in_m = load_u32(mcp);
             const int64_t mg = gbase >> (7 + t.m_lg);
             ms_old = t.ms[mg];
             ms_new = t.ms_new[mg];
+            wm = swap_code_halves(in_m, code_sel);
         }
-        int64_t r0 = r, r1 = r;  // the tensor rows of the DPP row's two halves
-        if (FOLD)
-            fold_rows(f, r, q.cg, r0, r1);
-        const float ro = t.row_old[r0], rn = t.row_new[r0];
-        const float ro1 = FOLD ? t.row_old[r1] : ro, rn1 = FOLD ? t.row_new[r1] : rn;
+        const uint32_t wv = swap_code_halves(in_v, code_sel);
         float gv[kEltsPerLane], v[kEltsPerLane], x[kEltsPerLane];
         unpack8(b0, b1, gv);
         const Nibbles nv = split_nibbles(wv);

@@ -378,6 +378,16 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             float *mp = reinterpret_cast<float *>(t.mc) + w.base;
             REAL p[kAnyElts], g[kAnyElts];
             float m[kAnyElts], v[kAnyElts];
+            // the small loads ahead of the branch between the values' loads
+            const uint64_t vc = load_codes<BITS, VEC>(t.vc, w, lane16);
+            const REAL ro = row_old[r];
+            uint64_t mc = 0;
+            float s0 = 0.0f, s1 = 0.0f;
+            if (!M32) {
+                mc = load_codes<BITS, VEC>(t.mc, w, lane16);
+                s0 = (float)ms[w.group];
+                s1 = (float)ms[w.group + (w.split < w.count ? 1 : 0)];
+            }
             if (keep) {
                 load_values<VEC, true>(pp, w, lane16, p);
                 load_values<VEC, true>(gp, w, lane16, g);
@@ -389,11 +399,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                 if (M32)
                     load_values<VEC, false>(mp, w, lane16, m);
             }
-            const uint64_t vc = load_codes<BITS, VEC>(t.vc, w, lane16);
-            const REAL ro = row_old[r];
             if (!M32) {
-                const uint64_t mc = load_codes<BITS, VEC>(t.mc, w, lane16);
-                const float s0 = (float)ms[w.group], s1 = w.split < w.count ? (float)ms[w.group + 1] : 0.0f;
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k)
                     m[k] = any_decode<BITS>(map_m, mc, k, mask_m) * (piece_at<VEC>(w, lane16, k) < w.split ? s0 : s1);
@@ -664,9 +670,10 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
         const REAL ro = row_old[r];
         const float rn = t.row_new[r];
         if (!M32) {
-            const bool two = w.split < w.count;
-            const float s0 = (float)ms[w.group], s1 = two ? (float)ms[w.group + 1] : 0.0f;
-            const float n0 = t.ms_new[w.group], n1 = two ? t.ms_new[w.group + 1] : n0;
+            // a piece in one group takes that group's scales twice: no load waits for another behind a branch
+            const int64_t next = w.group + (w.split < w.count ? 1 : 0);
+            const float s0 = (float)ms[w.group], s1 = (float)ms[next];
+            const float n0 = t.ms_new[w.group], n1 = t.ms_new[next];
             const float rc0 = VEC ? rcp_exact(n0) : 0.0f, rc1 = VEC ? rcp_exact(n1) : 0.0f;
 #pragma unroll
             for (int k = 0; k < kAnyElts; ++k) {

@@ -170,15 +170,13 @@ __device__ __forceinline__ Fold fold_of(const TensorR1 &t)
 // column of the tensor for column c of the matrix (c < 2 C)
 __device__ __forceinline__ uint32_t fold_col(const Fold &f, uint32_t c) { return c >= f.real_cols ? c - f.real_cols : c; }
 
-// tensor rows of the two halves of column block cg in row r of the matrix
+// Tensor rows of the two halves of column block cg in row r of the matrix.  No branch: a pass's loads of the row statistics stay among
+// its other loads, ahead of the first wait.
 __device__ __forceinline__ void fold_rows(const Fold &f, int64_t r, uint32_t cg, int64_t &r0, int64_t &r1)
 {
-    if (f.on) {
-        r0 = 2 * r + (cg * kGroup >= f.real_cols ? 1 : 0);
-        r1 = 2 * r + (cg * kGroup + 64 >= f.real_cols ? 1 : 0);
-    } else {
-        r0 = r1 = r;
-    }
+    const int on = f.on ? 1 : 0;
+    r0 = (r << on) + (on & (cg * kGroup >= f.real_cols ? 1 : 0));
+    r1 = (r << on) + (on & (cg * kGroup + 64 >= f.real_cols ? 1 : 0));
 }
 
 // Row maxima of a tile.  An atomic maximum on global memory goes out to the fabric (the L2s of
