@@ -652,22 +652,24 @@ def main():
     n_quant_tensors = sum(1 for p in params if p.numel() > 4096)
     launches_per_step = math.ceil(n_quant_tensors / MULTI_MAX)
 
-    # events around the dominant kernel's launches (same stream as the launches)
+    # events around the dominant kernel's launches (same stream as the launches): the call with both kinds of tensors
     events = []
-    real_call = lib.lpmm_adamw4bit_step_multi
     recording = {"on": False}
 
-    def timed_call(*a):
-        if not recording["on"]:
-            return real_call(*a)
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record()
-        st = real_call(*a)
-        e1.record()
-        events.append((e0, e1))
-        return st
+    def timed(real_call):
+        def call(*a):
+            if not recording["on"]:
+                return real_call(*a)
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            st = real_call(*a)
+            e1.record()
+            events.append((e0, e1))
+            return st
+        return call
 
-    lib.lpmm_adamw4bit_step_multi = timed_call
+    for name in ("lpmm_adamw4bit_step_multi", "lpmm_adamw4bit_fp32_step_multi"):
+        setattr(lib, name, timed(getattr(lib, name)))
 
     marks = [torch.cuda.Event(enable_timing=True) for _ in range(args.steps + 1)]
     with _gc_paused():
@@ -716,7 +718,7 @@ def main():
         "verified_on": verified_on,
         "config": {"workload": desc, "tensors": len(params), "params": n_total, "quantized_params": n_quant,
                    # the 4-bit kernel's launches plus the fp32-state kernel's (tensors of <= 4096 elements, 64 per launch)
-                   "launches_per_step": launches_per_step + math.ceil((len(params) - n_quant_tensors) / 64)},
+                   "launches_per_step": max(launches_per_step, math.ceil((len(params) - n_quant_tensors) / 64))},
         "effective_gbs": (n_quant * BYTES_PER_PARAM_4BIT + (n_total - n_quant) * BYTES_PER_PARAM_FP32)
         / (elapsed / args.steps) / 1e9,
         "roofline": {

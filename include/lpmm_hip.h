@@ -121,8 +121,7 @@ int lpmm_adamw_fp32_step_multi(const lpmm_adamw_fp32_tensor *tensors, int64_t co
                                float eps, void *stream);
 
 /* Both kinds of tensors of a parameter group, the quantised ones (lpmm_adamw4bit_step_multi) and those with fp32 states
- * (lpmm_adamw_fp32_step_multi): in one launch where at most 48 of the former and 64 of the latter are given, which is what the step of a small
- * model costs; otherwise as the two calls.  Either array may be empty. */
+ * (lpmm_adamw_fp32_step_multi): up to 64 of the latter go with each launch of up to 48 of the former.  Either array may be empty. */
 int lpmm_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain,
                                    int64_t plain_count, const float *qmap_m, const float *qmap_v, float beta1, float beta2, float lr,
                                    float weight_decay, float eps, void *stream);

@@ -487,8 +487,9 @@ __global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
     tile_fp32<Arith>(args, blockIdx.x);
 }
 
-// Both kinds of tensors of a small model in one launch: the tiles of the quantised tensors, then those of the ones with fp32 states.
-// A step of such a model is bound by the host, which a launch costs about 7 us (the call, its kernel arguments, the device and stream around it):
+// Both kinds of tensors in one launch: the tiles of the quantised tensors, then those of the ones with fp32 states, whose own launches
+// are latency (6 us each; GPT-2-XL's set has five).
+// A small model's step is bound by the host, which a launch costs about 7 us (the call, its kernel arguments, the device and stream around it):
 // fifty tensors of 7.5M values 39.5 -> 33.2 us a step.
 template <bool ALIGNED, bool ALLFULL, class Arith, class ArithF>
 __global__ __launch_bounds__(kThreads) void adamw_joined_kernel(const Multi4 args, const MultiF plain, const float *__restrict__ qmap_m,
@@ -777,7 +778,8 @@ static int step_multi_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count,
     return LPMM_OK;
 }
 
-// Quantised tensors and tensors with fp32 states of one parameter group: one launch where both fit one, else two kinds of launches.
+// Quantised tensors and tensors with fp32 states of one parameter group: as many of the latter as fit one launch go with each launch of
+// the former, what is left of either kind in launches of its own.
 template <class Arith, class ArithF, class PerTensor, class PerTensorF>
 static int step_joined(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain, int64_t plain_count,
                        const float *qmap_m, const float *qmap_v, const float (&scalars)[7], PerTensor per_tensor,
@@ -785,30 +787,36 @@ static int step_joined(const lpmm_adamw4bit_tensor *tensors, int64_t count, cons
 {
     if (count < 0 || plain_count < 0)
         return LPMM_ERR_SIZE;
-    int bad = count == 0 ? LPMM_OK : check4(tensors, count, qmap_m, qmap_v);
-    if (bad == LPMM_OK && plain_count != 0)
-        bad = check_fp32(plain, plain_count, 4);
-    if (bad != LPMM_OK)
-        return bad;
-    if (count != 0 && plain_count != 0 && count <= LPMM_MULTI_MAX && plain_count <= kMultiFMax) {
-        Multi4 args;
-        MultiF args_f;
-        for (int j = 0; j < 7; ++j)
-            args.s[j] = args_f.s[j] = scalars[j];
-        int64_t i = 0, i_f = 0;
+    int st = count == 0 ? LPMM_OK : check4(tensors, count, qmap_m, qmap_v);
+    if (st == LPMM_OK && plain_count != 0)
+        st = check_fp32(plain, plain_count, 4);
+    if (st != LPMM_OK)
+        return st;
+    Multi4 args;
+    MultiF args_f;
+    for (int j = 0; j < 7; ++j)
+        args.s[j] = args_f.s[j] = scalars[j];
+    int64_t i = 0, i_f = 0;
+    while (i < count && i_f < plain_count) {
+        const int64_t from = i, from_f = i_f;
         const Launch4 l = fill4(args, tensors, count, i, per_tensor);
         const uint32_t tiles_f = fill_fp32(args_f, plain, plain_count, i_f, per_tensor_f);
-        if (l.tiles != 0 && tiles_f != 0 && i == count && i_f == plain_count && (uint64_t)l.tiles + tiles_f <= 0x7fffffffULL) {
-            const auto kernel = l.aligned && l.allfull ? adamw_joined_kernel<true, true, Arith, ArithF>
-                                : l.aligned            ? adamw_joined_kernel<true, false, Arith, ArithF>
-                                                       : adamw_joined_kernel<false, false, Arith, ArithF>;
-            hipLaunchKernelGGL(kernel, dim3(l.tiles + tiles_f), dim3(kThreads), 0, (hipStream_t)stream, args, args_f, qmap_m, qmap_v,
-                               l.tiles);
-            return launch_status();
+        if (l.tiles == 0 || tiles_f == 0 || (uint64_t)l.tiles + tiles_f > 0x7fffffffULL) {
+            i = from;
+            i_f = from_f;
+            break;
         }
+        const auto kernel = l.aligned && l.allfull ? adamw_joined_kernel<true, true, Arith, ArithF>
+                            : l.aligned            ? adamw_joined_kernel<true, false, Arith, ArithF>
+                                                   : adamw_joined_kernel<false, false, Arith, ArithF>;
+        hipLaunchKernelGGL(kernel, dim3(l.tiles + tiles_f), dim3(kThreads), 0, (hipStream_t)stream, args, args_f, qmap_m, qmap_v,
+                           l.tiles);
+        st = launch_status();
+        if (st != LPMM_OK)
+            return st;
     }
-    bad = step_multi4<Arith>(tensors, count, qmap_m, qmap_v, scalars, per_tensor, stream);
-    return bad != LPMM_OK ? bad : step_multi_fp32<ArithF>(plain, plain_count, scalars, per_tensor_f, stream);
+    st = step_multi4<Arith>(tensors + i, count - i, qmap_m, qmap_v, scalars, per_tensor, stream);
+    return st != LPMM_OK ? st : step_multi_fp32<ArithF>(plain + i_f, plain_count - i_f, scalars, per_tensor_f, stream);
 }
 
 extern "C" int lpmm_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tensor *tensors, int64_t count, const lpmm_adamw_fp32_tensor *plain,

@@ -258,12 +258,12 @@ class AdamW(LowBitOptimizer):
 
     @staticmethod
     def _joined(batches, fused):
-        """Where the quantised tensors and those with fp32 states stand that share one launch, or two Nones: a small model's."""
+        """Where the quantised tensors and those with fp32 states stand that share launches, or two Nones."""
         quantised, four, plain = _native.WALK_FUSED4 if fused else _native.WALK_FLAT, None, None
         for k, batch in enumerate(batches):
-            if batch[0] == _native.WALK_PLAIN and batch[5] <= _native.PLAIN_MULTI_MAX:
+            if batch[0] == _native.WALK_PLAIN:
                 plain = k
-            elif batch[0] == quantised and batch[5] <= _native.MULTI_MAX:
+            elif batch[0] == quantised:
                 four = k
         if four is None or plain is None or batches[four][1] != batches[plain][1]:
             return None, None

@@ -410,9 +410,9 @@ def test_fused_multi_step_under_graph_capture(qmaps):
 
 @pytest.mark.parametrize("fused", [True, False])
 @pytest.mark.parametrize("sizes", ["whole", "ragged", "shifted"])
-@pytest.mark.parametrize("counts", [(0, 3), (3, 0), (1, 1), (48, 64), (49, 64), (48, 65), (5, 130)])
+@pytest.mark.parametrize("counts", [(0, 3), (3, 0), (1, 1), (48, 64), (49, 64), (48, 65), (5, 130), (100, 70)])
 def test_joined_launch_equals_two(qmaps, counts, sizes, fused):
-    """Quantised tensors and tensors with fp32 states in one call (one launch up to 48 and 64 of them): the bytes of the two calls."""
+    """Quantised tensors and tensors with fp32 states in one call (launches of up to 48 and 64 of them): the bytes of the two calls."""
     nat = _native()
     lib = nat.lib()
     dqm, dqv = (to_dev(q) for q in qmaps)
