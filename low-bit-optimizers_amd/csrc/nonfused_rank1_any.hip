@@ -18,9 +18,9 @@
 //     count is odd, to different rows: the first pass clears the word around such a byte, the second sets the word's codes
 //     by atomic or (store_nibbles).
 // Two forms (rank1_any_runs): runs of four neighbouring values a lane where every tensor of a launch allows it, single values 16 apart
-// otherwise.  A step on six tensors, single values -> runs (with the order of xcd_neighbours and quotients by reciprocals kept over
-// a lane's rows): 4096 x 4100 595 -> 510 us, fp32 first moment 600 -> 505, 8 bits 609 -> 555, float16 696 -> 580; 4096 x 1600
-// 246 -> 200 (fp32), 262 -> 210 (8 bits), 345 -> 270 (float16).
+// otherwise.  A step on six tensors, single values -> runs (with the order of xcd_neighbours, quotients by reciprocals kept over
+// a lane's rows and no load behind a branch): 4096 x 4100 600 -> 486 us, fp32 first moment 620 -> 518, 8 bits 618 -> 540,
+// float16 724 -> 528; 4096 x 1600 258 -> 201 (fp32), 264 -> 214 (8 bits), 350 -> 257 (float16).
 // Before, these tensors took the staged path (dequantise, update, statistics, normalise: six to eight
 // launches a tensor and 50 bytes a value; float16: about thirty PyTorch ops a tensor).  One step on one tensor,
 // staged -> here: 4096 x 4100 default 224 -> 107 us, fp32 first moment 183 -> 104, 8 bits 221 -> 102, float16
@@ -378,16 +378,27 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             float *mp = reinterpret_cast<float *>(t.mc) + w.base;
             REAL p[kAnyElts], g[kAnyElts];
             float m[kAnyElts], v[kAnyElts];
-            // the small loads ahead of the branch between the values' loads
-            const uint64_t vc = load_codes<BITS, VEC>(t.vc, w, lane16);
-            const REAL ro = row_old[r];
-            uint64_t mc = 0;
+            // The small loads: ahead of the branch between the values' loads where a lane takes runs (behind it the compiler
+            // waits for values before it issues them), behind single values' loads, where ahead they cost more than they
+            // save (72M values in rows of 1682, 4 bits: update 227 -> 206 us with them behind, and the requantisation
+            // with the conditional second scale 243 -> 213 us).
+            uint64_t vc = 0, mc = 0;
+            REAL ro;
             float s0 = 0.0f, s1 = 0.0f;
-            if (!M32) {
-                mc = load_codes<BITS, VEC>(t.mc, w, lane16);
-                s0 = (float)ms[w.group];
-                s1 = (float)ms[w.group + (w.split < w.count ? 1 : 0)];
-            }
+            const auto small_loads = [&] {
+                vc = load_codes<BITS, VEC>(t.vc, w, lane16);
+                ro = row_old[r];
+                if (!M32) {
+                    mc = load_codes<BITS, VEC>(t.mc, w, lane16);
+                    s0 = (float)ms[w.group];
+                    if (VEC)
+                        s1 = (float)ms[w.group + (w.split < w.count ? 1 : 0)];
+                    else
+                        s1 = w.split < w.count ? (float)ms[w.group + 1] : 0.0f;
+                }
+            };
+            if (VEC)
+                small_loads();
             if (keep) {
                 load_values<VEC, true>(pp, w, lane16, p);
                 load_values<VEC, true>(gp, w, lane16, g);
@@ -399,6 +410,8 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
                 if (M32)
                     load_values<VEC, false>(mp, w, lane16, m);
             }
+            if (!VEC)
+                small_loads();
             if (!M32) {
 #pragma unroll
                 for (int k = 0; k < kAnyElts; ++k)
@@ -670,10 +683,11 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
         const REAL ro = row_old[r];
         const float rn = t.row_new[r];
         if (!M32) {
-            // a piece in one group takes that group's scales twice: no load waits for another behind a branch
-            const int64_t next = w.group + (w.split < w.count ? 1 : 0);
-            const float s0 = (float)ms[w.group], s1 = (float)ms[next];
-            const float n0 = t.ms_new[w.group], n1 = t.ms_new[next];
+            // runs: a piece in one group takes that group's scales twice, so that no load waits for another behind a branch
+            const bool two = w.split < w.count;
+            const int64_t next = w.group + (two ? 1 : 0);
+            const float s0 = (float)ms[w.group], s1 = VEC ? (float)ms[next] : two ? (float)ms[w.group + 1] : 0.0f;
+            const float n0 = t.ms_new[w.group], n1 = VEC ? t.ms_new[next] : two ? t.ms_new[w.group + 1] : n0;
             const float rc0 = VEC ? rcp_exact(n0) : 0.0f, rc1 = VEC ? rcp_exact(n1) : 0.0f;
 #pragma unroll
             for (int k = 0; k < kAnyElts; ++k) {
