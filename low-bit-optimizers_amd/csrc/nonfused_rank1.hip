@@ -499,14 +499,16 @@ struct LaunchKind {
 //     layers 1853 -> 1818), with 16 where the first moment is fp32 (a pass moves 20.5 instead of 13.5 bytes a value; a step of
 //     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold or codes are bytes
 //     (GPT-2-XL's set 5590 -> 5549 a step; 8 bits 2925 -> 2916).
+//   * rows of an odd column count: the second pass sets the 4-bit codes of shared bytes by atomics, which shorter tiles spread (six
+//     tensors of 4095 x 4099, a step: 64 rows 986, 32 rows 965; fp32 first moment 851, 834).
 // The float16 passes are bound by their arithmetic: tall tiles spread a tile's set-up (four decoder layers of width 4096:
 // 32 rows 1821, 64 rows 1751, 128 rows 1729 a step).
-static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows)
+static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, bool odd_cols)
 {
     if (l.half_io)
         return kPolicyRowsHalf;
     if (requant)
-        return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 ? kPolicyRows / 2 : kPolicyRows;
+        return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
     if (l.values < 64e6)
         return rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : kPolicyRows / 2;
     return l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
@@ -704,8 +706,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             const bool fold = t.cols % kGroup != 0 && can_fold;  // validated above: 64 modulo 128, even rows
             const int64_t rows = fold ? t.rows / 2 : t.rows;
             const uint32_t blocks = fold ? 2 * col_blocks - 1 : col_blocks;
-            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows));
-            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows));
+            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, t.cols & 1));
+            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, t.cols & 1));
             if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
             d.p = t.p;
