@@ -494,7 +494,7 @@ struct LaunchKind {
 //     1600 x 6400 (246M values): 571 / 209, 560 / 218, 578 / 274.  So the second pass goes below 64 rows only under
 //     14M values, the update pass under 64M;
 //   * no more than 256 row blocks of 16 rows on a column: their atomics on one address queue up (8192 x 256 among 5.5M
-//     values: 16 rows 27.2, 32 rows 20.9);
+//     values: 16 rows 27.2, 32 rows 20.9), nor many more than 256 of 32 rows (21788 x 256: 32 rows 42.5, 64 rows 36.0 to 38.8);
 //   * larger launches: the update pass does best with 32 rows where a DPP row is a whole column block (LLaMA-7B decoder
 //     layers 1853 -> 1818), with 16 where the first moment is fp32 (a pass moves 20.5 instead of 13.5 bytes a value; a step of
 //     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold or codes are bytes
@@ -510,7 +510,7 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     if (requant)
         return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
     if (l.values < 64e6)
-        return rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : kPolicyRows / 2;
+        return rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
     return l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
 }
 
