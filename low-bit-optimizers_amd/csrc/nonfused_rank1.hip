@@ -556,32 +556,13 @@ static void launch_rank1(const R1Launch &l, bool folded, const float *qmap_m, co
     launch_rank1_passes<MODE, false>(l, qmap_m, qmap_v, passes, stream);
 }
 
-// Validation, batching into launches of at most kR1Max tensors, and the launches.
-// m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
+// The checks of a call's records.  general: they are for any column count and alignment; can_fold: see rank1_step_multi.
 template <int MODE, class Record>
-static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
-                            uint32_t m_lg, double beta1, double beta2, double lr, double weight_decay, double eps,
-                            void *stream, int bits_m = 4, int bits_v = 4, const void *table_m = nullptr,
-                            const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr)
+static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v, bool general, bool half_io,
+                       bool can_fold)
 {
-    // passes: 1 = the first pass alone (with the clearing of the next statistics), 2 = the second alone,
-    // 3 = both; one at a time only where the launches below are this file's own, or general ones: any column count,
-    // any alignment (nonfused_rank1_any.hip; wide-group and fp32 records, at most one launch's worth, none empty).
-    const bool general = out != nullptr;
-    if (passes < 1 || passes > 3 || (passes != 3 && !general && (MODE != kMCodes128 || bits_m != 4 || half_io)))
-        return LPMM_ERR_ARG;
     const int64_t real_bytes = general && half_io ? 2 : 4, vec_bytes = general ? real_bytes : 16;
     constexpr bool M32 = MODE == kMFloat;
-    // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
-    // served as double rows (rank1_tiles.hpp)
-    const bool can_fold = MODE == kMCodes128 && bits_m == 4 && !half_io;
-    // column counts that are no multiple of 128 (wide-group records only): every tensor of the call
-    // then takes the kernels for ragged rows
-    bool ragged = false;
-    if (count < 0)
-        return LPMM_ERR_SIZE;
-    if (count == 0)
-        return LPMM_OK;
     LPMM_REQUIRE_PTR(tensors);
     LPMM_REQUIRE_PTR(qmap_m);
     LPMM_REQUIRE_PTR(qmap_v);
@@ -593,7 +574,6 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             return LPMM_ERR_SIZE;
         if (!general && t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && folds(t.rows, t.cols)))
             return LPMM_ERR_SIZE;
-        ragged = ragged || (MODE == kMCodesWide && t.cols % kGroup != 0);
         if (t.rows == 0 || t.cols == 0)
             continue;
         const int64_t col_blocks = (t.cols + kGroup - 1) / kGroup;
@@ -630,6 +610,41 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         if (t.v_rowmax == t.v_rowmax_next || t.v_colmax == t.v_colmax_next)
             return LPMM_ERR_ARG;
     }
+    return LPMM_OK;
+}
+
+// Validation, batching into launches of at most kR1Max tensors, and the launches.
+// m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
+template <int MODE, class Record>
+static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
+                            uint32_t m_lg, double beta1, double beta2, double lr, double weight_decay, double eps,
+                            void *stream, int bits_m = 4, int bits_v = 4, const void *table_m = nullptr,
+                            const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr)
+{
+    // passes: 1 = the first pass alone (with the clearing of the next statistics), 2 = the second alone,
+    // 3 = both; one at a time only where the launches below are this file's own, or general ones: any column count,
+    // any alignment (nonfused_rank1_any.hip; wide-group and fp32 records, at most one launch's worth, none empty, checked by the caller).
+    const bool general = out != nullptr;
+    if (passes < 1 || passes > 3 || (passes != 3 && !general && (MODE != kMCodes128 || bits_m != 4 || half_io)))
+        return LPMM_ERR_ARG;
+    constexpr bool M32 = MODE == kMFloat;
+    // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
+    // served as double rows (rank1_tiles.hpp)
+    const bool can_fold = MODE == kMCodes128 && bits_m == 4 && !half_io;
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    if (!general) {
+        const int bad = check_rank1<MODE>(tensors, count, qmap_m, qmap_v, false, half_io, can_fold);
+        if (bad != LPMM_OK)
+            return bad;
+    }
+    // column counts that are no multiple of 128 (wide-group records only): every tensor of the call
+    // then takes the kernels for ragged rows
+    bool ragged = false;
+    for (int64_t i = 0; i < count; ++i)
+        ragged = ragged || (MODE == kMCodesWide && tensors[i].cols % kGroup != 0);
 
     hipStream_t s = (hipStream_t)stream;
     if (passes & 1) {
@@ -849,13 +864,74 @@ extern "C" int lpmm_nonfused_adamw_bits_rank1_step_multi_table(const lpmm_nonfus
                                         bits_m, bits_v, table_m, table_v);
 }
 
+// A launch's worth of records for any column count in the two forms that rank1_step_multi takes.
+struct AnyRecords {
+    lpmm_rank1_mgroup_tensor wide[kR1Max];
+    lpmm_rank1_v4bit_tensor plain[kR1Max];  // fp32 first moment
+
+    void set(int k, const lpmm_rank1_any_tensor &t)
+    {
+        lpmm_rank1_mgroup_tensor &w = wide[k];
+        lpmm_rank1_v4bit_tensor &f = plain[k];
+        f.p = w.p = static_cast<float *>(t.p);
+        f.g = w.g = static_cast<const float *>(t.g);
+        f.m = static_cast<float *>(t.m);
+        w.m_codes = static_cast<uint8_t *>(t.m);
+        w.m_max1 = static_cast<const float *>(t.m_max1);
+        w.m_max1_next = static_cast<float *>(t.m_max1_next);
+        f.v_codes = w.v_codes = const_cast<uint8_t *>(t.v_codes);
+        f.v_rowmax = w.v_rowmax = static_cast<const float *>(t.v_rowmax);
+        f.v_colmax = w.v_colmax = static_cast<const float *>(t.v_colmax);
+        f.v_rowmax_next = w.v_rowmax_next = static_cast<float *>(t.v_rowmax_next);
+        f.v_colmax_next = w.v_colmax_next = static_cast<float *>(t.v_colmax_next);
+        f.rows = w.rows = t.rows;
+        f.cols = w.cols = t.cols;
+        f.step = w.step = t.step;
+        f.reserved = w.reserved = 0.0f;
+    }
+};
+
+// All records of a call, before the first launch: a call with an invalid one changes nothing.
+static int check_any(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, const float *qmap_m, const float *qmap_v)
+{
+    for (int64_t i = 0; i < count; ++i) {
+        const lpmm_rank1_any_tensor &t = tensors[i];
+        if (t.rows == 0 || t.cols == 0)
+            continue;
+        LPMM_REQUIRE_PTR(t.v_codes_next);
+        LPMM_REQUIRE_ALIGN(t.v_codes_next, 4);
+        if (t.v_codes_next == t.v_codes)
+            return LPMM_ERR_ARG;
+        if (kind != kAnyFloatM) {
+            LPMM_REQUIRE_PTR(t.m_codes_next);
+            LPMM_REQUIRE_ALIGN(t.m_codes_next, 4);
+            if (t.m_codes_next == t.m)
+                return LPMM_ERR_ARG;
+        }
+    }
+    AnyRecords one;
+    for (int64_t i = 0; i < count; ++i) {
+        if (tensors[i].rows == 0 || tensors[i].cols == 0)
+            continue;
+        one.set(0, tensors[i]);
+        const int bad = kind == kAnyFloatM
+                            ? check_rank1<kMFloat>(one.plain, 1, qmap_v, qmap_v, true, false, false)
+                            : check_rank1<kMCodesWide>(one.wide, 1, qmap_m, qmap_v, true, kind == kAnyHalf, false);
+        if (bad != LPMM_OK)
+            return bad;
+    }
+    return LPMM_OK;
+}
+
 int lpmm::rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg,
                                const float *qmap_m, int bits_m, const void *table_m, const float *qmap_v, int bits_v,
                                const void *table_v, double beta1, double beta2, double lr, double weight_decay, double eps,
                                int passes, void *stream)
 {
-    lpmm_rank1_mgroup_tensor wide[kR1Max];
-    lpmm_rank1_v4bit_tensor plain[kR1Max];
+    const int bad = check_any(tensors, count, kind, qmap_m, qmap_v);
+    if (bad != LPMM_OK)
+        return bad;
+    AnyRecords rec;
     NewCodes out;
     // First the tensors that go in runs of four values, then the others: a launch holds one kind.  Where a call has both, the second
     // set of launches (about 30 us: three layers of width 64 and 218 in float16 90 -> 124 us a step) has to be worth it: runs save about
@@ -877,40 +953,14 @@ int lpmm::rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t cou
                 const lpmm_rank1_any_tensor &t = tensors[i];
                 if (t.rows == 0 || t.cols == 0 || (use_runs && rank1_any_runs(t, kind)) != out.runs)
                     continue;
-                lpmm_rank1_mgroup_tensor &w = wide[k];
-                lpmm_rank1_v4bit_tensor &f = plain[k];
-                f.p = w.p = static_cast<float *>(t.p);
-                f.g = w.g = static_cast<const float *>(t.g);
-                f.m = static_cast<float *>(t.m);
-                w.m_codes = static_cast<uint8_t *>(t.m);
-                w.m_max1 = static_cast<const float *>(t.m_max1);
-                w.m_max1_next = static_cast<float *>(t.m_max1_next);
-                f.v_codes = w.v_codes = const_cast<uint8_t *>(t.v_codes);
-                f.v_rowmax = w.v_rowmax = static_cast<const float *>(t.v_rowmax);
-                f.v_colmax = w.v_colmax = static_cast<const float *>(t.v_colmax);
-                f.v_rowmax_next = w.v_rowmax_next = static_cast<float *>(t.v_rowmax_next);
-                f.v_colmax_next = w.v_colmax_next = static_cast<float *>(t.v_colmax_next);
-                f.rows = w.rows = t.rows;
-                f.cols = w.cols = t.cols;
-                f.step = w.step = t.step;
-                f.reserved = w.reserved = 0.0f;
-                LPMM_REQUIRE_PTR(t.v_codes_next);
-                LPMM_REQUIRE_ALIGN(t.v_codes_next, 4);
-                if (t.v_codes_next == t.v_codes)
-                    return LPMM_ERR_ARG;
-                if (kind != kAnyFloatM) {
-                    LPMM_REQUIRE_PTR(t.m_codes_next);
-                    LPMM_REQUIRE_ALIGN(t.m_codes_next, 4);
-                    if (t.m_codes_next == t.m)
-                        return LPMM_ERR_ARG;
-                }
+                rec.set(k, t);
                 out.v[k] = t.v_codes_next;
                 out.m[k++] = t.m_codes_next;
             }
             const int st = kind == kAnyFloatM
-                               ? rank1_step_multi<kMFloat>(plain, k, qmap_v, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, 4,
+                               ? rank1_step_multi<kMFloat>(rec.plain, k, qmap_v, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, 4,
                                                            4, nullptr, nullptr, passes, false, &out)
-                               : rank1_step_multi<kMCodesWide>(wide, k, qmap_m, qmap_v, m_lg, beta1, beta2, lr, weight_decay, eps,
+                               : rank1_step_multi<kMCodesWide>(rec.wide, k, qmap_m, qmap_v, m_lg, beta1, beta2, lr, weight_decay, eps,
                                                                stream, bits_m, bits_v, table_m, table_v, passes, kind == kAnyHalf, &out);
             if (st != LPMM_OK)
                 return st;

@@ -83,6 +83,31 @@ def test_argument_errors_without_gpu():
         _native.check(SIZE, "probe")
 
 
+@pytest.mark.parametrize("kind", ["RANK1_CODES4", "RANK1_FLOAT_M", "RANK1_CODES8", "RANK1_HALF"])
+@pytest.mark.parametrize("field, change, status", [("v_codes_next", "null", 1), ("v_codes_next", "shift", 2),
+                                                   ("v_codes_next", "v_codes", 5), ("p", "null", 1), ("g", "shift", 2),
+                                                   ("v_rowmax_next", "v_rowmax", 5), ("rows", "negative", 3)])
+def test_a_call_for_any_column_count_checks_every_record_first(kind, field, change, status):
+    """A record that is taken in runs of four values, large enough for launches of its own beside the other kind, and an
+    invalid one of the other kind: its status comes back, and not that of the first one's launch (there is no device here)."""
+    from lpmm import _native
+
+    lib, k = _native.lib(), getattr(_native, kind)
+    memory = np.zeros(4096, np.uint8)  # never read: only the addresses count
+    base = (memory.ctypes.data + 63) // 64 * 64
+    records = np.zeros(2, _native.RANK1_ANY_TENSOR)
+    for i, (rows, cols) in enumerate([(12000, 2004), (70, 61)]):
+        for j, name in enumerate(_native.RANK1_ANY_TENSOR.names[:13]):
+            records[i][name] = base + 1024 * i + 64 * j
+        records[i]["rows"], records[i]["cols"], records[i]["step"] = rows, cols, 1.0
+    bad = records[1]
+    bad[field] = 0 if change == "null" else bad[field] + 1 if change == "shift" else -1 if change == "negative" else bad[change]
+    bits = 8 if kind == "RANK1_CODES8" else 4
+    for table in (records, records[::-1].copy()):
+        assert lib.lpmm_nonfused_adamw_rank1_any_step_multi(table.ctypes.data, 2, k, 128, base, bits, None, base, bits, None, 0.9, 0.999,
+                                                            1e-3, 0.01, 1e-8, 3, None) == status
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
