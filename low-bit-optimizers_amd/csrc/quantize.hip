@@ -344,6 +344,9 @@ __global__ void fill_zero_kernel(float *__restrict__ a, int64_t na, float *__res
 constexpr int kStatBatch = 8;                                    // loads of a lane in flight
 constexpr int kStatTileRows = (kQThreads / kWave) * kStatBatch;  // rows of a batch with one row a load
 
+// More rows are refused, as they always were: callers may count on the status.
+constexpr int64_t kStatMaxRows = 65535LL * 64;
+
 struct StatShape {
     uint32_t tiles_x;  // column tiles
     uint32_t lg_lanes; // lanes that share a row: a tile is 4 << lg_lanes columns wide
@@ -878,24 +881,23 @@ extern "C" int lpmm_rank1_stats(const float *x, int64_t rows, int64_t cols, floa
     LPMM_REQUIRE_ALIGN(x, 4);
     LPMM_REQUIRE_ALIGN(rowmax, 4);
     LPMM_REQUIRE_ALIGN(colmax, 4);
-    if ((cols + 1023) / 1024 > 0x7fffffffLL || (rows + 63) / 64 > 65535)
-        return LPMM_ERR_SIZE;
-    const int64_t mx = rows > cols ? rows : cols;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((uint32_t)((mx + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, rowmax, rows, colmax, cols);
     StatShape sh;
     sh.lg_lanes = 6;
     while (sh.lg_lanes > 0 && (4LL << (sh.lg_lanes - 1)) >= cols)
         --sh.lg_lanes;
-    const int64_t tx = (cols + (4LL << sh.lg_lanes) - 1) / (4LL << sh.lg_lanes);
+    const int64_t tx = (cols - 1) / (4LL << sh.lg_lanes) + 1;
+    if (tx > 0x7fffffffLL || rows > kStatMaxRows)
+        return LPMM_ERR_SIZE;
     const int64_t batch_rows = (int64_t)kStatTileRows * (kWave >> sh.lg_lanes), row_batches = (rows + batch_rows - 1) / batch_rows;
-    // tiles on a column: see rank1_stats_tile_kernel
-    const int64_t most = rows * cols / 40000 > 256 ? rows * cols / 40000 : 256;
+    // tiles on a column: see rank1_stats_tile_kernel; and no more than a grid holds
+    int64_t most = rows * cols / 40000 > 256 ? rows * cols / 40000 : 256;
+    most = most < 0x7fffffffLL / tx ? most : 0x7fffffffLL / tx;
     sh.tiles_x = (uint32_t)tx;
     sh.batches = (uint32_t)((row_batches + most - 1) / most);
     const int64_t tiles = tx * ((row_batches + sh.batches - 1) / sh.batches);
-    if (tiles > 0x7fffffffLL)
-        return LPMM_ERR_SIZE;
+    const int64_t mx = rows > cols ? rows : cols;
+    hipLaunchKernelGGL(fill_zero_kernel, dim3((uint32_t)((mx + 255) / 256)), dim3(256), 0,
+                       (hipStream_t)stream, rowmax, rows, colmax, cols);
     if (aligned_to(x, 16) && (cols % 4) == 0)
         hipLaunchKernelGGL(rank1_stats_tile_kernel<true>, dim3((uint32_t)tiles), dim3(kQThreads), 0, (hipStream_t)stream, x, rows,
                            cols, sh, rowmax, colmax);

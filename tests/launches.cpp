@@ -1,0 +1,109 @@
+// Prints what the library would launch, on a machine without a GPU: this program's own launch functions stand before the HIP
+// runtime's and record the grids.  The arguments' addresses are made up and never read.  One line of standard input is one call,
+//   stats ROWS COLS                     lpmm_rank1_stats
+//   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment) or codes8
+// and one line of output its status and the grids, "x,y" each.
+// Build: g++ -O1 -rdynamic -D__HIP_PLATFORM_AMD__ -I<rocm>/include -I<include> launches.cpp -llpmm_hip
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstring>
+#include <iostream>
+#include <sstream>
+#include <string>
+#include <vector>
+
+#include "lpmm_hip.h"
+
+static std::vector<dim3> launches;
+static dim3 next_grid, next_block;
+
+extern "C" hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t)
+{
+    next_grid = grid;
+    next_block = block;
+    return hipSuccess;
+}
+
+extern "C" hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hipStream_t *stream)
+{
+    *grid = next_grid;
+    *block = next_block;
+    *shared = 0;
+    *stream = nullptr;
+    return hipSuccess;
+}
+
+extern "C" hipError_t hipLaunchKernel(const void *, dim3 grid, dim3, void **, size_t, hipStream_t)
+{
+    launches.push_back(grid);
+    return hipSuccess;
+}
+
+extern "C" hipError_t hipGetLastError() { return hipSuccess; }
+
+// distinct addresses on a 256-byte boundary
+static char *made_up()
+{
+    static uintptr_t at = 1u << 20;
+    return reinterpret_cast<char *>(at += uintptr_t(1) << 30);
+}
+
+static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, int64_t>> &shapes)
+{
+    std::vector<lpmm_nonfused_rank1_tensor> coded;
+    std::vector<lpmm_rank1_v4bit_tensor> plain;
+    for (const auto &[rows, cols] : shapes) {
+        lpmm_nonfused_rank1_tensor t;
+        lpmm_rank1_v4bit_tensor f;
+        memset(&t, 0, sizeof t);
+        memset(&f, 0, sizeof f);
+        f.p = t.p = (float *)made_up();
+        f.g = t.g = (const float *)made_up();
+        t.m_codes = (uint8_t *)made_up();
+        f.m = (float *)made_up();
+        t.m_max1 = (float *)made_up();
+        f.v_codes = t.v_codes = (uint8_t *)made_up();
+        f.v_rowmax = t.v_rowmax = (const float *)made_up();
+        f.v_colmax = t.v_colmax = (const float *)made_up();
+        f.v_rowmax_next = t.v_rowmax_next = (float *)made_up();
+        f.v_colmax_next = t.v_colmax_next = (float *)made_up();
+        f.rows = t.rows = rows;
+        f.cols = t.cols = cols;
+        f.step = t.step = 1.0f;
+        coded.push_back(t);
+        plain.push_back(f);
+    }
+    const float *map = (const float *)made_up();
+    const int64_t n = (int64_t)shapes.size();
+    if (mode == "float_m")
+        return lpmm_nonfused_adamw_v4bit_rank1_step_multi(plain.data(), n, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
+    if (mode == "codes8")
+        return lpmm_nonfused_adamw_bits_rank1_step_multi(coded.data(), n, map, 8, map, 8, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
+    return lpmm_nonfused_adamw4bit_rank1_step_multi(coded.data(), n, map, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
+}
+
+int main()
+{
+    std::string line;
+    while (std::getline(std::cin, line)) {
+        std::istringstream in(line);
+        std::string call, mode;
+        std::vector<std::pair<int64_t, int64_t>> shapes;
+        int64_t rows, cols;
+        in >> call;
+        if (call == "rank1")
+            in >> mode;
+        while (in >> rows >> cols)
+            shapes.push_back({rows, cols});
+        launches.clear();
+        const int status = call == "stats" ? lpmm_rank1_stats((const float *)made_up(), shapes[0].first, shapes[0].second,
+                                                              (float *)made_up(), (float *)made_up(), nullptr)
+                                           : rank1(mode, shapes);
+        printf("%d", status);
+        for (const dim3 &grid : launches)
+            printf(" %u,%u", grid.x, grid.y);
+        printf("\n");
+    }
+    return 0;
+}

@@ -108,6 +108,34 @@ def test_a_call_for_any_column_count_checks_every_record_first(kind, field, chan
                                                             1e-3, 0.01, 1e-8, 3, None) == status
 
 
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    """launches(line, ...): per line (a call as tests/launches.cpp describes it) its status and the grids it launches, in order."""
+    from lpmm import _native
+
+    exe, libs, rocm = str(tmp_path_factory.mktemp("launches") / "launches"), os.path.dirname(_native.LIB_PATH), "/opt/rocm"
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-Wall", "-rdynamic", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include",
+                           "-I" + os.path.join(ROOT, "include"), os.path.join(HERE, "launches.cpp"), "-L" + libs, "-llpmm_hip",
+                           f"-L{rocm}/lib", "-lamdhip64", f"-Wl,-rpath,{libs}", f"-Wl,-rpath,{rocm}/lib", "-o", exe])
+
+    def run(*lines):
+        out = subprocess.run([exe], input="\n".join(lines), capture_output=True, text=True, check=True).stdout.splitlines()
+        assert len(out) == len(lines)
+        return [(int(words[0]), [tuple(map(int, w.split(","))) for w in words[1:]]) for words in map(str.split, out)]
+
+    return run
+
+
+def test_rank1_statistics_of_extreme_sizes(launches):
+    """What lpmm_rank1_stats refuses it refuses before the launch that clears the caller's arrays, and a matrix of more tiles
+    than a grid holds is taken in taller ones."""
+    rows, limit = 65535 * 64, 0x7fffffff
+    for status, grids in launches(f"stats {rows + 1} 1", f"stats 1 {limit * 256 + 1}", "stats 0 8", "stats 8 0", "stats -1 8"):
+        assert (status, grids) == (3, [])
+    for status, grids in launches(f"stats {rows} 1", f"stats {rows} {1 << 24}", f"stats 40 {1 << 36}", "stats 40 100"):
+        assert status == 0 and len(grids) == 2 and all(0 < x <= limit and y == 1 for x, y in grids)
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
