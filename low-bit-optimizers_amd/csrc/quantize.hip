@@ -417,7 +417,11 @@ __global__ __launch_bounds__(kQThreads) void rank1_stats_tile_kernel(const float
                     atomic_max_nonneg(rowmax + r, m);
             }
         } else {
-            // a tile this narrow is the whole row
+            // a tile this narrow is the whole row; no maximum is below zero, so that a row of NaNs alone has zero, as it has
+            // where lanes without columns take part
+#pragma unroll
+            for (int u = 0; u < kStatBatch; ++u)
+                rm[u] = fmaxf(rm[u], 0.0f);
             for (int o = lanes >> 1; o > 0; o >>= 1) {
 #pragma unroll
                 for (int u = 0; u < kStatBatch; ++u)

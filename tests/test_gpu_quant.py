@@ -396,3 +396,22 @@ def test_rank1_dispatch_edges(oracle, qmaps, shape, shift):
         assert (to_np(codes)[want_codes.size:] == 0x55).all()
         np.testing.assert_array_equal(to_np(out)[shift: shift + n], want.reshape(-1))
         assert (to_np(out)[:shift] == -1).all() and (to_np(out)[shift + n:] == -1).all()
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("shape", [(70, 4), (70, 8), (9, 16), (33, 64), (40, 100), (33, 128), (5, 200)])
+def test_rank1_statistics_of_a_row_of_nans(oracle, shape, shift):
+    """A NaN is no maximum, also where a row holds nothing else: its statistic is zero whatever columns fill a tile's lanes."""
+    r, c = shape
+    x = _signed(np.random.default_rng(r * c), r * c).reshape(r, c)
+    x[1, :] = np.nan
+    x[3, c // 2] = np.nan
+    want_row, want_col = oracle.rank1_stats(x)
+    assert want_row[1] == 0
+    dx = torch.empty(r * c + 4, device="cuda")[shift: shift + r * c]
+    dx.copy_(to_dev(x).view(-1))
+    rowmax, colmax = torch.empty(r, device="cuda"), torch.empty(c, device="cuda")
+    assert _lib().lpmm_rank1_stats(dx.data_ptr(), r, c, rowmax.data_ptr(), colmax.data_ptr(), _stream()) == 0
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(to_np(rowmax), want_row)
+    np.testing.assert_array_equal(to_np(colmax), want_col)
