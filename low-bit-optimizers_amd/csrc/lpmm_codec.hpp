@@ -60,8 +60,8 @@ __device__ __forceinline__ float div_fast(float x, float d)
 }
 
 // x / y given rc = RN(1/y): one multiply and two fmas give the correctly rounded quotient
-// when y lies in [2^-60, 2^60] and |x| <= y (no intermediate underflow where a code depends
-// on it).
+// when y lies in [2^-60, 2^60] (no intermediate underflow where a code depends on it), or a NaN
+// where the quotient leaves the range of a float or x is infinite, which |x| <= y excludes.
 __device__ __forceinline__ float div_by_rc(float x, float y, float rc)
 {
     const float q = x * rc;
@@ -70,6 +70,13 @@ __device__ __forceinline__ float div_by_rc(float x, float y, float rc)
 }
 
 __device__ __forceinline__ bool rc_safe(float y) { return y >= 0x1p-60f && y <= 0x1p60f; }
+
+// Is there a NaN among the eight values?  Two a comparison.
+__device__ __forceinline__ bool any_nan(const float (&x)[8])
+{
+    return __builtin_isunordered(x[0], x[1]) || __builtin_isunordered(x[2], x[3]) || __builtin_isunordered(x[4], x[5]) ||
+           __builtin_isunordered(x[6], x[7]);
+}
 
 // 1 / y for y in [2^-60, 2^60]: the hardware approximation and one Newton step.  Equal to the
 // correctly rounded reciprocal for every float of that range on gfx950 (all 1 006 632 961 of

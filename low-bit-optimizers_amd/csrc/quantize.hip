@@ -485,9 +485,9 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_kernel(const float *__r
 // Codes of v[k] / min(cmx[k], rm) for a lane's 8 values of one row.  The column maxima stay the
 // same for every row a lane handles, so their correctly rounded reciprocals are formed once
 // (col_rcp); with the row's reciprocal that turns every division into one multiply and two fmas
-// that give the correctly rounded quotient (|v| <= scale by construction).  Scales outside the
-// range in which the reciprocal is exact, and maps other than the two standard ones, take the
-// plain division and the generic search.
+// that give the correctly rounded quotient.  Scales outside the range in which the reciprocal is
+// exact, maps other than the two standard ones and NaN quotients (statistics that do not cover the
+// values: div_by_rc) take the plain division.
 struct ColRcp {
     float rc[kQElts];
     bool safe;
@@ -516,8 +516,9 @@ __device__ __forceinline__ uint32_t encode8_rank1(const uint32_t *lds, int kind,
             const bool by_col = cmx[k] < rm;
             xs[k] = div_by_rc(v[k], by_col ? cmx[k] : rm, by_col ? cr.rc[k] : rr);
         }
-        // the closed form of the second-moment code needs 0 <= x <= 1; values below 0 are legal here
-        return kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
+        // the closed form of the second-moment code needs 0 <= x <= 1; other values are legal here
+        if (!__any(any_nan(xs)))
+            return kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
     }
 #pragma unroll
     for (int k = 0; k < kQElts; ++k)
@@ -692,21 +693,22 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_flat_kernel(const float
 #pragma unroll
         for (int k = 0; k < kQElts; ++k)
             safe = safe && rc_safe(s[k]);
-        uint32_t w;
-        if (__all(safe)) {
+        bool fast = __all(safe);
+        if (fast) {
 #pragma unroll
             for (int k = 0; k < kQElts; ++k)
                 xs[k] = div_by_rc(v[k], s[k], rcp_exact(s[k]));
-            w = kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
-        } else {
+            fast = !__any(any_nan(xs));  // as in encode8_rank1
+        }
+        if (!fast) {
             // the values that pad the tensor are plain zeros
 #pragma unroll
             for (int k = 0; k < kQElts; ++k) {
                 const int64_t i = (k < 4 ? i0 : i1) + (k & 3);
                 xs[k] = i < n ? v[k] / s[k] : 0.0f;
             }
-            w = encode8_plain(lds, kLdsQ0, kind, xs);
         }
+        const uint32_t w = fast && kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
         if (whole || i0 < n_padded)
             store_u16(reinterpret_cast<uint16_t *>(codes + (i0 >> 1)), w & 0xFFFFu);
         if (whole || i1 < n_padded)

@@ -361,3 +361,38 @@ def test_nonfused_optimizer_other_widths(oracle, bits):
         bad = lpmm.optim.AdamW([torch.nn.Parameter(to_dev(host[1]))], fused=True, qconfig=cfg, **H)
         bad.param_groups[0]["params"][0].grad = to_dev(host[1])
         bad.step()
+
+
+@pytest.mark.parametrize("with_table", [False, True])
+@pytest.mark.parametrize("bits", [4, 5, 8])
+@pytest.mark.parametrize("shape", [(33, 300), (67, 257), (70, 256), (700, 52), (40, 1600), (9, 2049), (130, 24)])
+def test_rank1_statistics_that_do_not_cover_the_values(oracle, bits, shape, with_table):
+    """The code is that of x / min(rowmax, colmax) whatever the statistics are: quotients beyond one, beyond the range of a float
+    and of infinities, of either sign, on every split of the work."""
+    lib = _lib()
+    r, c = shape
+    rng = np.random.default_rng(r + bits)
+    qmap = oracle.create_dynamic_map(True, bits - 1, bits)
+    x = (rng.standard_normal(shape) * np.exp(rng.standard_normal((r, 1)))).astype(np.float32)
+    rowmax, colmax = (s * np.float32(0.3) for s in oracle.rank1_stats(x))
+    rowmax[5] = 2.0 ** -50
+    x[5, 1], x[5, 2] = -1e30, 1e30
+    for row, value in ((7, -np.inf), (8, np.inf), (9 % r, -np.nan), (11 % r, -3e38), (12 % r, 3e38)):
+        if row < r:
+            x[row, row % c] = value
+    x[6, 1::2] *= 1e3
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = oracle.quant_rank1_bits(x, rowmax, colmax, qmap, bits)
+    dx, dq, dr, dc = to_dev(x), to_dev(qmap), to_dev(rowmax), to_dev(colmax)
+    codes = torch.full((want.size,), 0x5A, dtype=torch.uint8, device="cuda")
+    args = (dx.data_ptr(), r, c, dr.data_ptr(), dc.data_ptr(), dq.data_ptr())
+    if bits == 4:
+        st = lib.lpmm_quant_rank1(*args, codes.data_ptr(), _stream())
+    elif with_table:
+        table = _code_table(dq, bits)
+        st = lib.lpmm_quant_rank1_bits_table(*args, bits, table.data_ptr(), codes.data_ptr(), _stream())
+    else:
+        st = lib.lpmm_quant_rank1_bits(*args, bits, codes.data_ptr(), _stream())
+    assert st == 0
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(to_np(codes), want)
