@@ -260,7 +260,7 @@ def test_tile_shapes_do_not_show_in_the_result(config, half):
         pytest.skip("float16 parameters take the two passes under the default configuration")
     path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
     dtype = torch.float16 if half else torch.float32
-    shapes = [(272, 384), (17, 256), (130, 192), (200, 136), (96, 45), (48, 32, 3, 3), (40, 7, 5, 5)]
+    shapes = [(272, 384), (17, 256), (130, 192), (200, 136), (96, 45), (48, 32, 3, 3), (40, 7, 5, 5), (9000, 128), (21788, 256)]
     want = None
     for beside in (None, (1024, 4608), (4096, 4224), (8200, 8064)):
         gen = torch.Generator(device="cuda").manual_seed(5)

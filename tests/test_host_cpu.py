@@ -136,6 +136,20 @@ def test_rank1_statistics_of_extreme_sizes(launches):
         assert status == 0 and len(grids) == 2 and all(0 < x <= limit and y == 1 for x, y in grids)
 
 
+# matrices of one column of tiles, so that a pass's grid is its row blocks
+NARROW = [(mode, rows, cols) for mode in ("codes4", "float_m", "codes8")
+          for rows, cols in [(20000, 128), (21788, 256), (50257, 128), (70001, 256), (100000, 128)]]
+
+
+def test_interleaved_groups_of_narrow_matrices(launches):
+    """Groups of row blocks that work on neighbouring rows are of a multiple of 32 blocks where they are large: neighbours share
+    cache lines of statistics and scales."""
+    for case, (status, grids) in zip(NARROW, launches(*("rank1 %s %d %d" % case for case in NARROW))):
+        assert status == 0 and len(grids) == 3, case
+        for x, y in grids[1:]:
+            assert y == 1 and x % 32 == 0 and x * 128 >= case[1], (case, grids)
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
