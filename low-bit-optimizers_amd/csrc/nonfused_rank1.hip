@@ -462,6 +462,7 @@ static uint32_t choose_lg_wide(uint32_t col_blocks)
     return best;
 }
 
+constexpr double kValuesPerRowBlock = 12000;  // pass_rows_policy
 constexpr uint64_t kCombMultiple = 32;
 static_assert(kPolicyResident % kCombMultiple == 0, "a rounded group is no larger than the resident set");
 
@@ -507,19 +508,30 @@ struct LaunchKind {
 //     layers 1853 -> 1818), with 16 where the first moment is fp32 (a pass moves 20.5 instead of 13.5 bytes a value; a step of
 //     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold or codes are bytes
 //     (GPT-2-XL's set 5590 -> 5549 a step; 8 bits 2925 -> 2916).
+//   * whatever the launch holds, a column takes no more row blocks than one per 12000 values of its matrix, or 512: 18 ns an atomic on
+//     one address are then less than the time of its values (13.5 to 20.5 bytes each at 6 TB/s).  Steps with tiles of 16, 32, 64, 128
+//     rows: 1048576 x 128 1377, 777, 498, 450 (fp32 first moment 1379, 805, 628, 621; 8 bits 1406, 822, 508, 504), 524288 x 256
+//     769, 492, 448, 443, 262144 x 512 492, 426, 430, 438, 131072 x 1024 419, 421, 428, 437 (fp32 573, 584, 596, 605);
 //   * rows of an odd column count: the second pass sets the 4-bit codes of shared bytes by atomics, which shorter tiles spread (six
 //     tensors of 4095 x 4099, a step: 64 rows 986, 32 rows 965; fp32 first moment 851, 834).
 // The float16 passes are bound by their arithmetic: tall tiles spread a tile's set-up (four decoder layers of width 4096:
 // 32 rows 1821, 64 rows 1751, 128 rows 1729 a step).
-static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, bool odd_cols)
+static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, uint32_t col_blocks, bool odd_cols)
 {
     if (l.half_io)
         return kPolicyRowsHalf;
     if (requant)
         return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
+    uint32_t tile_rows;
     if (l.values < 64e6)
-        return rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
-    return l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
+        tile_rows = rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
+    else
+        tile_rows = l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
+    const double values = (double)rows * (double)col_blocks * kGroup;
+    const double most = values / kValuesPerRowBlock > 512 ? values / kValuesPerRowBlock : 512;
+    while (tile_rows < kPolicyRowsMost && (double)rows > most * tile_rows)
+        tile_rows *= 2;
+    return tile_rows;
 }
 
 // Launches of at most this many values leave the gradient and the second moment's codes in the cache (R1Launch::keep).  The memory-side
@@ -729,8 +741,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             const bool fold = t.cols % kGroup != 0 && can_fold;  // validated above: 64 modulo 128, even rows
             const int64_t rows = fold ? t.rows / 2 : t.rows;
             const uint32_t blocks = fold ? 2 * col_blocks - 1 : col_blocks;
-            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, t.cols & 1));
-            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, t.cols & 1));
+            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, blocks, t.cols & 1));
+            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, blocks, t.cols & 1));
             if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
             d.p = t.p;

@@ -150,6 +150,21 @@ def test_interleaved_groups_of_narrow_matrices(launches):
             assert y == 1 and x % 32 == 0 and x * 128 >= case[1], (case, grids)
 
 
+def test_row_blocks_of_a_column(launches):
+    """Atomics of a column's row blocks queue up on one address: the update pass of a tall narrow matrix keeps them few, alone
+    and beside large matrices, below and above the sizes at which its tiles change."""
+    cases = [(mode, rows, cols, beside) for mode in ("codes4", "float_m", "codes8") for cols in (128, 256, 512, 1024)
+             for values in (6e6, 60e6, 70e6, 300e6) for rows in [int(values) // cols] for beside in ("", " 8192 8192")]
+    for (mode, rows, cols, beside), (status, grids) in zip(cases, launches(*("rank1 %s %d %d%s" % case for case in cases))):
+        assert status == 0 and len(grids) == 3
+        tiles = grids[1][0]
+        if beside:
+            tiles -= 8192 * 8192 // 256 // 16  # at most: tiles of 16 rows by 256 columns
+        col_tiles = (cols + 255) // 256
+        # the rule, the tallest tiles, and the empty blocks of a group
+        assert tiles // col_tiles <= max(512, rows * cols / 12000, rows / 128) + 256, (mode, rows, cols, beside, grids)
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
