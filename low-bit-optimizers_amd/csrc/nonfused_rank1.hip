@@ -501,7 +501,8 @@ struct LaunchKind {
 //   * few values leave the chip idle with tall tiles.  2048 x 2048 alone: 64 rows 22.3 / 10.0, 32 rows 15.9 / 7.9, 16 rows
 //     14.2 / 7.3; 32 weights of 256 x 2304: 59 / 21, 52 / 22, 50 / 24; of 512 x 2048: 90 / 37, 87 / 35, 84 / 43; 24 of
 //     1600 x 6400 (246M values): 571 / 209, 560 / 218, 578 / 274.  So the second pass goes below 64 rows only under
-//     14M values, the update pass under 64M;
+//     14M values, the update pass under 64M.  Tiles of one column group hold half as many values: second pass on 5000 x 640
+//     with 32 and 16 rows 6.7, 8.2 (fp32 first moment 6.5, 8.0), on 4000 x 640 6.8, 6.3 (6.4, 5.8);
 //   * no more than 256 row blocks of 16 rows on a column: their atomics on one address queue up (8192 x 256 among 5.5M
 //     values: 16 rows 27.2, 32 rows 20.9), nor many more than 256 of 32 rows (21788 x 256: 32 rows 42.5, 64 rows 36.0 to 38.8);
 //   * larger launches: the update pass does best with 32 rows where a DPP row is a whole column block (LLaMA-7B decoder
@@ -521,7 +522,7 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     if (l.half_io)
         return kPolicyRowsHalf;
     if (requant)
-        return l.values < 4e6 ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
+        return l.values < (choose_lg_wide(col_blocks) == 0 ? 3e6 : 4e6) ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
     uint32_t tile_rows;
     if (l.values < 64e6)
         tile_rows = rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;

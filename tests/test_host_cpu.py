@@ -165,6 +165,18 @@ def test_row_blocks_of_a_column(launches):
         assert tiles // col_tiles <= max(512, rows * cols / 12000, rows / 128) + 256, (mode, rows, cols, beside, grids)
 
 
+def test_second_pass_of_tiles_of_one_column_group(launches):
+    """Five column groups go one to a tile; above 3M values such tiles have 32 rows in the second pass, as many values as the
+    16-row tiles of two groups that matrices of up to 4M values take."""
+    calls = ["rank1 %s %d %d" % (mode, rows, cols) for mode in ("codes4", "float_m", "codes8")
+             for rows, cols in [(5000, 640), (4000, 640), (2500, 1280)]]
+    for call, (status, grids) in zip(calls, launches(*calls)):
+        rows = call.split()[2]
+        tile_rows = 32 if rows == "5000" else 16
+        blocks, tiles = -(-int(rows) // tile_rows), 5
+        assert status == 0 and blocks * tiles <= grids[2][0] < (blocks + 64) * tiles, (call, grids)
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
