@@ -76,7 +76,7 @@ struct Record {
 
 struct Batch {
     Kind kind;
-    int device, flag;  // flag: kRank1Wide: ragged rows; kAny: the kind of its entry point
+    int device, flag;  // flag: kRank1Wide: ragged rows; kAny: the kind of its entry point; plan_start: kPlain
     PyObject *qm, *qv;  // the maps' tensors (borrowed from held references)
     std::vector<uint8_t> records, second;
     std::vector<lpmm_rank1_small_vector> fold;
@@ -689,8 +689,28 @@ PyObject *plan_rest(PyObject *self, void *)
     return rest;
 }
 
+// The tensors with fp32 states that share the launches of the quantised tensors b (lpmm_adamw4bit_fp32_step_multi and its
+// non-fused form), or null.  Decided here: a loop over the batches in Python cost every step 1.0 us, of 34 on three layers of width 128.
+const Batch *joined(const std::vector<Batch> &batches, const Batch &b)
+{
+    if (b.kind != kFused4 && b.kind != kFlat)
+        return nullptr;
+    const Batch *plain = nullptr;
+    for (const Batch &other : batches) {
+        if (other.device != b.device)
+            continue;
+        if (other.kind == b.kind && &other < &b)
+            return nullptr;  // they go with the first of several
+        if (other.kind == kPlain)
+            plain = &other;
+    }
+    return plain;
+}
+
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
-// address of the records, address of the second pass's records or 0, address of the fold records or 0)
+// address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
+// that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's, and
+// flag 1 in the latter's own batch.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
     Plan *plan = reinterpret_cast<Plan *>(self);
@@ -714,10 +734,17 @@ PyObject *plan_start(PyObject *self, PyObject *)
             if (!b.second.empty())
                 memcpy(&b.second[(i + 1) * bytes - 8], &step, 4);
         }
+        const Batch *const plain = joined(*plan->batches, b);
+        bool elsewhere = false;
+        if (b.kind == kPlain)
+            for (const Batch &other : *plan->batches)
+                elsewhere = elsewhere || joined(*plan->batches, other) == &b;
         PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,
-                                    b.qv != nullptr ? b.qv : Py_None, b.flag, (Py_ssize_t)b.items.size(),
-                                    (unsigned long long)(uintptr_t)b.records.data(), (unsigned long long)(uintptr_t)b.second.data(),
-                                    (unsigned long long)(uintptr_t)b.fold.data());
+                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : b.flag, (Py_ssize_t)b.items.size(),
+                                    (unsigned long long)(uintptr_t)b.records.data(),
+                                    (unsigned long long)(uintptr_t)(plain != nullptr ? plain->records.data() : b.second.data()),
+                                    plain != nullptr ? (unsigned long long)plain->items.size()
+                                                     : (unsigned long long)(uintptr_t)b.fold.data());
         if (t == nullptr || PyList_Append(out, t) != 0) {
             Py_XDECREF(t);
             Py_DECREF(out);

@@ -256,43 +256,30 @@ class AdamW(LowBitOptimizer):
              routes.m_group_wide, routes.bits_rank1, routes.m_group),
             _native.factored_workspace())
 
-    @staticmethod
-    def _joined(batches, fused):
-        """Where the quantised tensors and those with fp32 states stand that share launches, or two Nones."""
-        quantised, four, plain = _native.WALK_FUSED4 if fused else _native.WALK_FLAT, None, None
-        for k, batch in enumerate(batches):
-            if batch[0] == _native.WALK_PLAIN:
-                plain = k
-            elif batch[0] == quantised:
-                four = k
-        if four is None or plain is None or batches[four][1] != batches[plain][1]:
-            return None, None
-        return four, plain
-
     def _launch_walk(self, group, plan, routes):
         """The launches of the walk's records: those that _step_fused and _step_single make."""
         beta1, beta2 = group["betas"]
         hyper = (beta1, beta2, group["lr"], group["weight_decay"], group["eps"])
         lib = _native.lib()
-        batches = plan.start()
-        four, plain = self._joined(batches, group["fused"])
-        for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(batches):
-            if k == plain:
-                continue  # goes with the quantised tensors
+        for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(plan.start()):
+            if flag and kind == _native.WALK_PLAIN:
+                continue  # these go with the quantised tensors
             with torch.cuda.device(index):
                 stream = _native.current_stream(index)
                 qm_ptr, qv_ptr = (None if q is None else q.data_ptr() for q in (qm, qv))
-                if k == four:
-                    run = lib.lpmm_adamw4bit_fp32_step_multi if group["fused"] else lib.lpmm_nonfused_adamw4bit_fp32_step_multi
-                    plain_count, plain_records = batches[plain][5:7]
-                    st = run(records, count, plain_records, plain_count, qm_ptr, qv_ptr, *hyper, stream)
-                elif kind == _native.WALK_FUSED4:
-                    st = lib.lpmm_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
+                if kind == _native.WALK_FUSED4:
+                    if fold:
+                        st = lib.lpmm_adamw4bit_fp32_step_multi(records, count, second, fold, qm_ptr, qv_ptr, *hyper, stream)
+                    else:
+                        st = lib.lpmm_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
                 elif kind == _native.WALK_PLAIN:
                     run = lib.lpmm_adamw_fp32_step_multi if group["fused"] else lib.lpmm_nonfused_update_multi
                     st = run(records, count, *hyper, stream)
                 elif kind == _native.WALK_FLAT:
-                    st = lib.lpmm_nonfused_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
+                    if fold:
+                        st = lib.lpmm_nonfused_adamw4bit_fp32_step_multi(records, count, second, fold, qm_ptr, qv_ptr, *hyper, stream)
+                    else:
+                        st = lib.lpmm_nonfused_adamw4bit_step_multi(records, count, qm_ptr, qv_ptr, *hyper, stream)
                 elif kind == _native.WALK_FLAT_M32:
                     st = lib.lpmm_nonfused_adamw_v4bit_step_multi(records, count, qv_ptr, *hyper, stream)
                 elif kind in (_native.WALK_FACTORED, _native.WALK_FACTORED_ANY):

@@ -400,3 +400,62 @@ def test_walk_and_loops_choose_one_route_at_the_limits(shape, config, dtype, mon
     for k in x:
         assert x[k].shape == y[k].shape and x[k].dtype == y[k].dtype, k
         assert torch.equal(x[k].nan_to_num(), y[k].nan_to_num()) if x[k].is_floating_point() else torch.equal(x[k], y[k]), k
+
+
+@pytest.mark.parametrize("case", ["fused", "group", "default", "half_group"])
+def test_which_tensors_share_launches(case, monkeypatch):
+    """Quantised tensors and tensors with fp32 states go to the library in one call, as the walk's batches say; float16 tensors
+    have no such call, and their batches stay apart."""
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    params, opt = _build(case, np.random.default_rng(7))
+    batches, calls = [], []
+
+    class Plan:
+        def __init__(self, plan):
+            self._plan = plan
+
+        def __getattr__(self, name):
+            return getattr(self._plan, name)
+
+        def start(self):
+            batches.append(self._plan.start())
+            return batches[-1]
+
+    class Lib:
+        def __getattr__(self, name):
+            calls.append(name)
+            return getattr(_native.lib(), name)
+
+    class Native:
+        def __getattr__(self, name):
+            return getattr(_native, name)
+
+        def walk(self):
+            return self
+
+        def lib(self):
+            return Lib()
+
+        def collect(self, *args):
+            return Plan(_native.walk().collect(*args))
+
+    for p in params:
+        p.grad = torch.ones_like(p) if p.is_contiguous() else None  # a strided one goes by the loops
+    for _ in range(2):
+        opt.step()
+    monkeypatch.setattr(adamw, "_native", Native())
+    opt.step()
+    (kinds,) = [{b[0]: b for b in batch} for batch in batches]
+    quantised = kinds[{"fused": _native.WALK_FUSED4, "half_group": _native.WALK_HALF_FLAT}.get(case, _native.WALK_FLAT)]
+    plain = kinds[_native.WALK_HALF_PLAIN if case == "half_group" else _native.WALK_PLAIN]
+    if case == "half_group":
+        assert quantised[5] > 0 and plain[5] > 0 and quantised[7:] == (0, 0) and plain[4] == 0
+        assert {"lpmm_nonfused_adamw4bit_f16_step_multi", "lpmm_nonfused_update_f16_multi"} <= set(calls)
+    else:
+        assert quantised[5] > 0 and plain[5] > 0 and quantised[7:] == (plain[6], plain[5]) and plain[4] == 1
+        one = "lpmm_adamw4bit_fp32_step_multi" if case == "fused" else "lpmm_nonfused_adamw4bit_fp32_step_multi"
+        assert calls.count(one) == 1
+        assert not {"lpmm_adamw4bit_step_multi", "lpmm_adamw_fp32_step_multi", "lpmm_nonfused_adamw4bit_step_multi",
+                    "lpmm_nonfused_update_multi"} & set(calls)
