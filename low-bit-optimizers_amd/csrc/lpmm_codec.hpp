@@ -71,11 +71,12 @@ __device__ __forceinline__ float div_by_rc(float x, float y, float rc)
 
 __device__ __forceinline__ bool rc_safe(float y) { return y >= 0x1p-60f && y <= 0x1p60f; }
 
-// Is there a NaN among the eight values?  Two a comparison.
-__device__ __forceinline__ bool any_nan(const float (&x)[8])
+// Are the quotients of x[k] by scales that rc_safe accepts those of div_by_rc?  Not where a value is infinite or so large that
+// the product could overflow; a NaN has its NaN either way.
+__device__ __forceinline__ bool rc_covers(const float (&x)[8])
 {
-    return __builtin_isunordered(x[0], x[1]) || __builtin_isunordered(x[2], x[3]) || __builtin_isunordered(x[4], x[5]) ||
-           __builtin_isunordered(x[6], x[7]);
+    const float a = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fabsf(x[2])), b = fmaxf(fmaxf(fabsf(x[3]), fabsf(x[4])), fabsf(x[5]));
+    return fmaxf(fmaxf(fmaxf(a, b), fabsf(x[6])), fabsf(x[7])) < 0x1p66f;
 }
 
 // 1 / y for y in [2^-60, 2^60]: the hardware approximation and one Newton step.  Equal to the

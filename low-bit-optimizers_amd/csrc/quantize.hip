@@ -486,8 +486,8 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_kernel(const float *__r
 // same for every row a lane handles, so their correctly rounded reciprocals are formed once
 // (col_rcp); with the row's reciprocal that turns every division into one multiply and two fmas
 // that give the correctly rounded quotient.  Scales outside the range in which the reciprocal is
-// exact, maps other than the two standard ones and NaN quotients (statistics that do not cover the
-// values: div_by_rc) take the plain division.
+// exact, maps other than the two standard ones and values far beyond their statistics (rc_covers)
+// take the plain division.
 struct ColRcp {
     float rc[kQElts];
     bool safe;
@@ -509,7 +509,7 @@ __device__ __forceinline__ uint32_t encode8_rank1(const uint32_t *lds, int kind,
                                                   const float (&cmx)[kQElts], const ColRcp &cr, float rm)
 {
     float xs[kQElts];
-    if (kind != kMapGeneric && __all(cr.safe && rc_safe(rm))) {
+    if (kind != kMapGeneric && __all(cr.safe & rc_safe(rm) & rc_covers(v))) {
         const float rr = rcp_exact(rm);
 #pragma unroll
         for (int k = 0; k < kQElts; ++k) {
@@ -517,8 +517,7 @@ __device__ __forceinline__ uint32_t encode8_rank1(const uint32_t *lds, int kind,
             xs[k] = div_by_rc(v[k], by_col ? cmx[k] : rm, by_col ? cr.rc[k] : rr);
         }
         // the closed form of the second-moment code needs 0 <= x <= 1; other values are legal here
-        if (!__any(any_nan(xs)))
-            return kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
+        return kind == kMapStdM ? encode8_std_m(lds, xs) : encode8_plain(lds, kLdsQ0, kind, xs);
     }
 #pragma unroll
     for (int k = 0; k < kQElts; ++k)
@@ -693,14 +692,12 @@ __global__ __launch_bounds__(kQThreads) void quant_rank1_flat_kernel(const float
 #pragma unroll
         for (int k = 0; k < kQElts; ++k)
             safe = safe && rc_safe(s[k]);
-        bool fast = __all(safe);
+        const bool fast = __all(safe) && __all(rc_covers(v));
         if (fast) {
 #pragma unroll
             for (int k = 0; k < kQElts; ++k)
                 xs[k] = div_by_rc(v[k], s[k], rcp_exact(s[k]));
-            fast = !__any(any_nan(xs));  // as in encode8_rank1
-        }
-        if (!fast) {
+        } else {
             // the values that pad the tensor are plain zeros
 #pragma unroll
             for (int k = 0; k < kQElts; ++k) {

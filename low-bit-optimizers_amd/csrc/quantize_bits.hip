@@ -596,7 +596,7 @@ __global__ __launch_bounds__(kBThreads) void dequant_group_bits_rows_kernel(cons
 
 // 'rank1' scaling, one code per byte, in the splits of rank1_rows.hpp (rows; flat).  x / min(rowmax, colmax) is one multiply and
 // two fmas that give the correctly rounded quotient wherever all the scales of the wave lie in the range in which the reciprocal is
-// exact, and the plain division otherwise and where a quotient is a NaN (statistics that do not cover the values: div_by_rc).
+// exact, and the plain division otherwise and for values far beyond their statistics (rc_covers).
 template <bool ONE>
 __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows_kernel(const float *__restrict__ x, int64_t R, int64_t C,
                                                                           const RowShape sh, const float *__restrict__ rowmax,
@@ -661,17 +661,14 @@ __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_rows_kernel(const 
             break;
         float v[kBElts], xs[kBElts];
         unpack8(a[t], b[t], v);
-        bool fast = __all(cols_safe && rc_safe(rm[t]));
-        if (fast) {
+        if (__all(cols_safe & rc_safe(rm[t]) & rc_covers(v))) {
             const float rr = rcp_exact(rm[t]);
 #pragma unroll
             for (int k = 0; k < kBElts; ++k) {
                 const bool by_col = cmx[k] < rm[t];
                 xs[k] = div_by_rc(v[k], by_col ? cmx[k] : rm[t], by_col ? crc[k] : rr);
             }
-            fast = !__any(any_nan(xs));
-        }
-        if (!fast) {
+        } else {
 #pragma unroll
             for (int k = 0; k < kBElts; ++k)
                 xs[k] = v[k] / ((cmx[k] < rm[t]) ? cmx[k] : rm[t]);
@@ -768,18 +765,15 @@ __global__ __launch_bounds__(kBThreads) void quant_rank1_bits_flat_kernel(const 
         unpack8(a[t], a[t + 1], v);
         flat_scales<RUNS>(st[t], s);
         flat_scales<RUNS>(st[t + 1], s + 4);
-        bool safe = true;
+        bool safe = rc_covers(v);
 #pragma unroll
         for (int k = 0; k < kBElts; ++k)
             safe = safe && rc_safe(s[k]);
-        bool fast = __all(safe);
-        if (fast) {
+        if (__all(safe)) {
 #pragma unroll
             for (int k = 0; k < kBElts; ++k)
                 xs[k] = div_by_rc(v[k], s[k], rcp_exact(s[k]));
-            fast = !__any(any_nan(xs));
-        }
-        if (!fast) {
+        } else {
             // the values that pad the tensor are plain zeros
 #pragma unroll
             for (int k = 0; k < kBElts; ++k)
