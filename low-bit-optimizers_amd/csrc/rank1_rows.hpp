@@ -211,8 +211,45 @@ __device__ __forceinline__ void flat_store(float *__restrict__ out, int64_t idx,
 }
 
 // ---- host: which split, and its shape ----------------------------------------------------
-// The rows split where it is the faster one (the table above).  The chunk is the widest that leaves at most a tenth of the lanes
-// idle, else the one that leaves fewest.
+// The rows split where it is the faster one (the table above), and the column groups of its chunks.  Chunks of 16 or 8 groups, whose
+// workgroups take runs of 8 or 4 KB, where at most 3 % of them lie beyond the row's end; else narrow ones from 4096 columns on, several
+// rows side by side, if rows start on cache lines.  Otherwise a quantiser takes the widest chunk that leaves at most a tenth of the lanes idle, else the one
+// that leaves fewest; a dequantiser, which has nothing to keep over the rows but cuts lines at a chunk's end, whole rows of 1, 2 or 4 groups,
+// pairs of groups from 12 groups on, and for the rest the flat split.  Dequantisers (us, 4 / 8 bits; "lanes": with the quantiser's
+// rule for every column count that is a multiple of 128; "before" as above):
+//                  lanes         here          before
+//   70000 x 1152   82.1 / 74.8   70.7 / 70.6   73.1 / 75.0
+//   50000 x 1664   77.1 / 75.0   74.4 / 75.0   73.9 / 76.6
+//   36000 x 2176   86.1 / 80.7   72.0 / 74.2   105.9 / 115.8
+//   36000 x 2304   77.4 / 75.6   71.5 / 72.4   103.9 / 117.0
+//   20000 x 4224   93.4 / 90.0   81.4 / 74.7   81.6 / 81.7
+//   15000 x 5504   82.5 / 78.1   79.0 / 75.0   79.3 / 78.4
+//   7200 x 11008   72.4 / 72.1   72.4 / 72.2   80.3 / 83.9
+// Quantisers: 20000 x 4224 63.0 / 71.5, 59.9 / 68.3, 64.0 / 70.3; 15000 x 5504 60.4 / 67.4, 59.1 / 66.7, 59.3 / 66.4.
+inline int64_t row_chunk_groups(int64_t cols, bool quantise)
+{
+    const int64_t groups = (cols + kGroup - 1) / kGroup;
+    for (int64_t wide = 16; wide >= 8; wide /= 2)
+        if ((double)cols >= 0.97 * (double)((groups + wide - 1) / wide * wide * kGroup))
+            return wide;
+    if (cols >= 4096 && cols % kGroup == 0)
+        return quantise ? 4 : 2;
+    if (!quantise)
+        return groups == 1 || groups == 2 || groups == 4 ? groups : groups >= 12 && groups % 2 == 0 ? 2 : 0;
+    const int64_t least = (cols + kR1Cols - 1) / kR1Cols;
+    double best = 0.0;
+    int64_t found = 0;
+    for (int64_t k = least; k <= 2 * least + 2 && best < 0.9; ++k) {
+        const int64_t wide = (groups + k - 1) / k, lanes = 16 * wide;
+        const double use = (double)(kRank1Threads / lanes * lanes) / kRank1Threads * (double)cols / (double)(kGroup * wide * k);
+        if (use > best + 0.02) {
+            best = use;
+            found = wide;
+        }
+    }
+    return found;
+}
+
 inline bool rank1_rows(const void *x, const void *colmax, const void *codes, int64_t rows, int64_t cols, bool quantise, RowShape &sh,
                        dim3 &grid)
 {
@@ -220,18 +257,11 @@ inline bool rank1_rows(const void *x, const void *colmax, const void *codes, int
         return false;
     if (cols % 4 != 0 || !aligned_to(x, 16) || !aligned_to(colmax, 16) || !aligned_to(codes, 4))
         return false;
-    const int64_t blocks = (cols + kGroup - 1) / kGroup, least = (cols + kR1Cols - 1) / kR1Cols;
-    double best = 0.0;
-    int64_t chunks = 0;
-    for (int64_t k = least; k <= 2 * least + 2 && best < 0.9; ++k) {
-        const int64_t wide = (blocks + k - 1) / k, lanes = 16 * wide;
-        const double use = (double)(kRank1Threads / lanes * lanes) / kRank1Threads * (double)cols / (double)(kGroup * wide * k);
-        if (use > best + 0.02) {
-            best = use;
-            chunks = k;
-            sh.lanes = (uint32_t)lanes;
-        }
-    }
+    const int64_t wide = row_chunk_groups(cols, quantise);
+    if (wide == 0)
+        return false;
+    const int64_t chunks = (cols + wide * kGroup - 1) / (wide * kGroup);
+    sh.lanes = (uint32_t)(16 * wide);
     sh.width = 8 * sh.lanes;
     sh.magic = (uint32_t)((1ULL << 32) / sh.lanes) + 1u;
     sh.groups = kRank1Threads / sh.lanes;

@@ -1,6 +1,8 @@
 // Prints what the library would launch, on a machine without a GPU: this program's own launch functions stand before the HIP
 // runtime's and record the grids.  The arguments' addresses are made up and never read.  One line of standard input is one call,
 //   stats ROWS COLS                     lpmm_rank1_stats
+//   quant BITS ROWS COLS                lpmm_quant_rank1 (4 bits) or lpmm_quant_rank1_bits
+//   dequant BITS ROWS COLS              the way back
 //   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment) or codes8
 // and one line of output its status and the grids, "x,y" each.
 // Build: g++ -O1 -rdynamic -D__HIP_PLATFORM_AMD__ -I<rocm>/include -I<include> launches.cpp -llpmm_hip
@@ -83,6 +85,18 @@ static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, i
     return lpmm_nonfused_adamw4bit_rank1_step_multi(coded.data(), n, map, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
 }
 
+static int quantiser(bool back, int bits, int64_t rows, int64_t cols)
+{
+    const float *x = (const float *)made_up(), *rowmax = (const float *)made_up(), *colmax = (const float *)made_up();
+    const float *map = (const float *)made_up();
+    uint8_t *codes = (uint8_t *)made_up();
+    if (back)
+        return bits == 4 ? lpmm_dequant_rank1(codes, rowmax, colmax, map, rows, cols, const_cast<float *>(x), nullptr)
+                         : lpmm_dequant_rank1_bits(codes, rowmax, colmax, map, bits, rows, cols, const_cast<float *>(x), nullptr);
+    return bits == 4 ? lpmm_quant_rank1(x, rows, cols, rowmax, colmax, map, codes, nullptr)
+                     : lpmm_quant_rank1_bits(x, rows, cols, rowmax, colmax, map, bits, codes, nullptr);
+}
+
 int main()
 {
     std::string line;
@@ -92,14 +106,16 @@ int main()
         std::vector<std::pair<int64_t, int64_t>> shapes;
         int64_t rows, cols;
         in >> call;
-        if (call == "rank1")
+        if (call != "stats")
             in >> mode;
         while (in >> rows >> cols)
             shapes.push_back({rows, cols});
         launches.clear();
-        const int status = call == "stats" ? lpmm_rank1_stats((const float *)made_up(), shapes[0].first, shapes[0].second,
-                                                              (float *)made_up(), (float *)made_up(), nullptr)
-                                           : rank1(mode, shapes);
+        const auto &[r, c] = shapes.at(0);
+        const int status = call == "stats"   ? lpmm_rank1_stats((const float *)made_up(), r, c, (float *)made_up(), (float *)made_up(),
+                                                                nullptr)
+                           : call == "rank1" ? rank1(mode, shapes)
+                                             : quantiser(call == "dequant", std::stoi(mode), r, c);
         printf("%d", status);
         for (const dim3 &grid : launches)
             printf(" %u,%u", grid.x, grid.y);

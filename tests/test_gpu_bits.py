@@ -297,7 +297,7 @@ def _rank1_bits_case(oracle, bits, shape, qmap, with_table, signed=False):
 
 @pytest.mark.parametrize("bits", [3, 5, 8])
 @pytest.mark.parametrize("shape", [(341, 20), (700, 52), (1030, 9), (2049, 12), (513, 130), (67, 257), (33, 300), (21, 516), (17, 1601),
-                                   (9, 2048), (7, 11009)])
+                                   (9, 2048), (7, 11009), (131, 256), (40, 640), (65, 1536), (6, 1664), (31, 2304), (63, 4224), (34, 5504)])
 def test_rank1_bits_dispatch_edges(oracle, bits, shape):
     """Columns on either side of the limits between the splits of rank1_rows.hpp, rows that leave a tile partly filled."""
     _rank1_bits_case(oracle, bits, shape, oracle.create_pow_map(bits, False, 1), False)

@@ -358,15 +358,20 @@ def test_quant_group_extreme_scales(oracle, qmaps):
             np.testing.assert_array_equal(to_np(max1), want_max1)
 
 
-# columns on either side of every limit of the rank-1 kernels' dispatch (rows of a chunk at a time for whole runs of four and at
-# least 16 columns, flattened otherwise, one lane a run of eight below 4 columns or off a 16-byte boundary; the statistics by
-# lanes a row), with rows that fill a workgroup's tile, leave one over and are fewer than its groups
+# columns on either side of every limit of the rank-1 kernels' dispatch (rows of a chunk at a time where the quantiser has runs of four
+# and 256 columns or whole groups of 128, the dequantiser whole groups; flattened otherwise, one lane a run of eight below 4 columns or
+# off a 16-byte boundary; the statistics by lanes a row), with rows that fill a workgroup's tile, leave one over and are fewer than its groups
 RANK1_EDGES = [(1, 4), (9, 1), (7, 3), (1030, 5), (4099, 6), (1, 16), (341, 20), (2049, 12), (700, 52), (129, 100), (513, 130),
                (130, 256), (67, 257), (33, 300), (21, 516), (17, 1601), (9, 2048), (5, 2056), (3, 4100), (70001, 8), (3, 11009)]
 
 
+# whole column groups: chunks of 16, 8, 4 and 2, single rows of 1, 2 and 4, and those that only a quantiser takes by rows
+RANK1_CHUNKS = [(65, 128), (131, 256), (9, 384), (33, 512), (40, 640), (35, 896), (17, 1024), (6, 1152), (65, 1536), (5, 1664), (31, 2304),
+                (3, 3200), (63, 4224), (34, 5504), (9, 6144), (10, 11008)]
+
+
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("shape", RANK1_EDGES)
+@pytest.mark.parametrize("shape", RANK1_EDGES + RANK1_CHUNKS)
 def test_rank1_dispatch_edges(oracle, qmaps, shape, shift):
     lib = _lib()
     r, c = shape

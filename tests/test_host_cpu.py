@@ -136,6 +136,26 @@ def test_rank1_statistics_of_extreme_sizes(launches):
         assert status == 0 and len(grids) == 2 and all(0 < x <= limit and y == 1 for x, y in grids)
 
 
+def test_rank1_quantisers_of_more_rows_than_a_grid_holds(launches):
+    """Rows go along the grid's second dimension, which ends at 65535; a matrix with more takes the flat split, in one dimension."""
+    limit = 65535 * 64  # rows of 128 columns: 16 side by side, four of each
+    calls = [f"{way} {bits} {rows} 128" for way in ("quant", "dequant") for bits in (4, 8) for rows in (limit, limit + 1)]
+    for call, (status, grids) in zip(calls, launches(*calls)):
+        values = 128 * int(call.split()[2])
+        rows_split, flat = (1, 65535), (-(-values // 4096), 1)
+        assert status == 0 and grids == [rows_split if values == 128 * limit else flat], call
+
+
+def test_chunks_of_the_rank1_dequantisers(launches):
+    """Whole column groups: chunks that leave few lanes idle or cut few lines, and the flat split (0) for the others."""
+    rows = 1000
+    chunks = {1: 1, 2: 2, 4: 4, 3: 0, 5: 0, 6: 0, 9: 0, 12: 2, 13: 0, 18: 2, 33: 2, 43: 2, 8: 8, 16: 16, 40: 8, 64: 16, 86: 8, 250: 16}
+    calls = {f"dequant {bits} {rows} {128 * groups}": (groups, wide) for groups, wide in chunks.items() for bits in (4, 8)}
+    for (call, (groups, wide)), (status, grids) in zip(calls.items(), launches(*calls)):
+        want = (-(-groups // wide), -(-rows // (4 * (16 // wide)))) if wide else (-(-rows * 128 * groups // 4096), 1)
+        assert (status, grids) == (0, [want]), call
+
+
 # matrices of one column of tiles, so that a pass's grid is its row blocks
 NARROW = [(mode, rows, cols) for mode in ("codes4", "float_m", "codes8")
           for rows, cols in [(20000, 128), (21788, 256), (50257, 128), (70001, 256), (100000, 128)]]
