@@ -466,35 +466,63 @@ constexpr double kValuesPerRowBlock = 12000;  // pass_rows_policy
 constexpr uint64_t kCombMultiple = 32;
 static_assert(kPolicyResident % kCombMultiple == 0, "a rounded group is no larger than the resident set");
 
-// Tile shape of a rows x (128 * col_blocks) tensor, and its tile count.
-static uint64_t shape_tiles(int64_t rows, uint32_t col_blocks, TileShape &ts, uint32_t policy_rows)
+// Row blocks of a matrix, and its tiles side by side.
+struct Blocks {
+    uint32_t lg_wide, tile_rows;
+    uint64_t rows, col_tiles;
+};
+
+static Blocks blocks_of(int64_t rows, uint32_t col_blocks, uint32_t policy_rows)
 {
-    const uint32_t lg_wide = choose_lg_wide(col_blocks);
-    const uint32_t col_tiles = (col_blocks + (1u << lg_wide) - 1) >> lg_wide;
-    const uint32_t pass_rows = (uint32_t)kDppRows >> lg_wide;
-    const uint32_t tile_rows = pass_rows > policy_rows ? pass_rows : policy_rows;
-    const uint64_t row_blocks = (uint64_t)((rows + tile_rows - 1) / tile_rows);
-    uint64_t comb = kPolicyResident / col_tiles;
+    Blocks b;
+    b.lg_wide = choose_lg_wide(col_blocks);
+    b.col_tiles = (col_blocks + (1u << b.lg_wide) - 1) >> b.lg_wide;
+    const uint32_t pass_rows = (uint32_t)kDppRows >> b.lg_wide;
+    b.tile_rows = pass_rows > policy_rows ? pass_rows : policy_rows;
+    b.rows = (uint64_t)((rows + b.tile_rows - 1) / b.tile_rows);
+    return b;
+}
+
+// Tile shape of a rows x (128 * col_blocks) tensor, and its tile count.  Row blocks interleave in groups of as many as are resident
+// together.
+// spread: what is left for the last group goes to as many blocks, each with fewer passes.  In launches of few workgroups these
+// short ones even out what the CUs have to do (LaunchKind::spread).
+static uint64_t shape_tiles(int64_t rows, uint32_t col_blocks, TileShape &ts, uint32_t policy_rows, bool spread)
+{
+    const Blocks b = blocks_of(rows, col_blocks, policy_rows);
+    uint64_t comb = kPolicyResident / b.col_tiles;
     comb = comb < 1 ? 1 : comb;
-    // groups of equal size, so that the last one holds few empty blocks (13 row blocks in groups of 5, not 6)
-    const uint64_t groups = (row_blocks + comb - 1) / comb;
-    comb = (row_blocks + groups - 1) / groups;
-    // Large groups (narrow matrices) hold a multiple of 32 blocks: neighbours share cache lines of row statistics and scales, and with
-    // an odd number the sharing blocks, and the XCDs they are on, change from pass to pass.  Update and second pass, equal groups ->
-    // multiples of 32: 50257 x 128 31.6 / 10.9 -> 28.6 / 9.1 us, 21788 x 256 25.4 / 9.1 -> 23.0 / 7.3.
-    if (comb >= 2 * kCombMultiple)
-        comb = (comb + kCombMultiple - 1) / kCombMultiple * kCombMultiple;
-    ts.lg_wide = lg_wide;
-    ts.tile_rows = tile_rows;
+    if (spread) {
+        comb = comb > b.rows ? b.rows : comb;
+    } else {
+        // groups of equal size, so that the last one holds few empty blocks (13 row blocks in groups of 5, not 6)
+        const uint64_t groups = (b.rows + comb - 1) / comb;
+        comb = (b.rows + groups - 1) / groups;
+        // Large groups (narrow matrices) hold a multiple of 32 blocks: neighbours share cache lines of row statistics and scales, and with
+        // an odd number the sharing blocks, and the XCDs they are on, change from pass to pass.  Update and second pass, equal groups ->
+        // multiples of 32: 50257 x 128 31.6 / 10.9 -> 28.6 / 9.1 us, 21788 x 256 25.4 / 9.1 -> 23.0 / 7.3.
+        if (comb >= 2 * kCombMultiple)
+            comb = (comb + kCombMultiple - 1) / kCombMultiple * kCombMultiple;
+    }
+    ts.lg_wide = b.lg_wide;
+    ts.tile_rows = b.tile_rows;
     ts.comb = (uint32_t)comb;
-    return (row_blocks + comb - 1) / comb * comb * col_tiles;
+    return (b.rows + comb - 1) / comb * comb * b.col_tiles;
 }
 
 // What a launch is, as far as its tile shapes depend on it.
 struct LaunchKind {
     bool half_io, m32, bits;
     double values;  // of all its tensors
+    bool spread[2];  // update pass, second pass: see shape_tiles
 };
+
+// Launches of fewer workgroups than this have their remainders spread: the float16 kernels and those for any column count, whose tiles take
+// longest.  Update and second pass (us; equal groups -> spread): float16 6974 x 3840 59.6 / 24.8 -> 53.2 / 23.5, 1962 x 6831 61.8 / 89.3
+// -> 54.7 / 84.2, 39877 x 128 27.7 / 10.7 -> 24.1 / 9.2, but 11008 x 4096 (1376 workgroups) 84.1 / 34.1 -> 86.0 / 35.6 and eight of
+// 962 x 9856 (2496) 141.5 / 60.0 -> 155.6 / 63.5; second pass on 1071 x 7515 51.4 -> 45.9, at 8 bits 28.8 -> 24.0, two of 5000 x 2000 at
+// 8 bits 52.7 -> 47.9, but 24 of 2196 x 1956 (6720) 202.8 -> 214.9.
+constexpr uint64_t kSpreadBelow = 1280;
 
 // Rows of a pass's tiles on a matrix of `rows` rows.  A tile of fewer rows means more column atomics and more set-up, one of
 // more rows a longer walk, fewer workgroups and a longer end of the launch.  Measured (us; update pass, then second pass):
@@ -719,13 +747,28 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     while (i < count) {
         int k = 0;
         // what this launch will hold decides its tiles' rows
-        LaunchKind kind = {half_io, M32, bits_m != 4, 0};
-        for (int64_t j = i; j < count && k < kR1Max; ++j)
-            if (tensors[j].rows != 0 && tensors[j].cols != 0) {
-                kind.values += (double)tensors[j].rows * (double)tensors[j].cols;
-                ++k;
-            }
-        k = 0;
+        LaunchKind kind = {half_io, M32, bits_m != 4, 0, {false, false}};
+        const auto each = [&](auto &&f) {
+            int k = 0;
+            for (int64_t j = i; j < count && k < kR1Max; ++j)
+                if (tensors[j].rows != 0 && tensors[j].cols != 0) {
+                    f(tensors[j]);
+                    ++k;
+                }
+        };
+        each([&](const Record &t) { kind.values += (double)t.rows * (double)t.cols; });
+        if (general || half_io) {
+            uint64_t blocks[2] = {0, 0};
+            each([&](const Record &t) {
+                const uint32_t col_blocks = (uint32_t)((t.cols + kGroup - 1) / kGroup);
+                for (int pass = 0; pass < 2; ++pass) {
+                    const Blocks b = blocks_of(t.rows, col_blocks, pass_rows_policy(kind, pass == 1, false, t.rows, col_blocks, t.cols & 1));
+                    blocks[pass] += b.rows * b.col_tiles;
+                }
+            });
+            kind.spread[0] = blocks[0] < kSpreadBelow;
+            kind.spread[1] = blocks[1] < kSpreadBelow;
+        }
         uint64_t tiles = 0, tiles2 = 0;
         uint32_t start2[kR1Max + 1] = {0};
         TileShape shape2[kR1Max];
@@ -742,8 +785,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             const bool fold = t.cols % kGroup != 0 && can_fold;  // validated above: 64 modulo 128, even rows
             const int64_t rows = fold ? t.rows / 2 : t.rows;
             const uint32_t blocks = fold ? 2 * col_blocks - 1 : col_blocks;
-            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, blocks, t.cols & 1));
-            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, blocks, t.cols & 1));
+            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, blocks, t.cols & 1), kind.spread[0]);
+            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, blocks, t.cols & 1), kind.spread[1]);
             if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
             d.p = t.p;

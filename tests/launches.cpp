@@ -3,7 +3,8 @@
 //   stats ROWS COLS                     lpmm_rank1_stats
 //   quant BITS ROWS COLS                lpmm_quant_rank1 (4 bits) or lpmm_quant_rank1_bits
 //   dequant BITS ROWS COLS              the way back
-//   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment) or codes8
+//   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment), codes8 or
+//                                       half (float16)
 // and one line of output its status and the grids, "x,y" each.
 // Build: g++ -O1 -rdynamic -D__HIP_PLATFORM_AMD__ -I<rocm>/include -I<include> launches.cpp -llpmm_hip
 #include <hip/hip_runtime_api.h>
@@ -55,6 +56,7 @@ static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, i
 {
     std::vector<lpmm_nonfused_rank1_tensor> coded;
     std::vector<lpmm_rank1_v4bit_tensor> plain;
+    std::vector<lpmm_nonfused_rank1_f16_tensor> halfs;
     for (const auto &[rows, cols] : shapes) {
         lpmm_nonfused_rank1_tensor t;
         lpmm_rank1_v4bit_tensor f;
@@ -75,11 +77,15 @@ static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, i
         f.step = t.step = 1.0f;
         coded.push_back(t);
         plain.push_back(f);
+        halfs.push_back({t.p, t.g, t.m_codes, t.m_max1, t.v_codes, t.v_rowmax, t.v_colmax, t.v_rowmax_next, t.v_colmax_next,
+                         (float *)made_up(), rows, cols, 1.0f, 0.0f});
     }
     const float *map = (const float *)made_up();
     const int64_t n = (int64_t)shapes.size();
     if (mode == "float_m")
         return lpmm_nonfused_adamw_v4bit_rank1_step_multi(plain.data(), n, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
+    if (mode == "half")
+        return lpmm_nonfused_adamw4bit_rank1_f16_step_multi(halfs.data(), n, map, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
     if (mode == "codes8")
         return lpmm_nonfused_adamw_bits_rank1_step_multi(coded.data(), n, map, 8, map, 8, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
     return lpmm_nonfused_adamw4bit_rank1_step_multi(coded.data(), n, map, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);

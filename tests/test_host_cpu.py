@@ -197,6 +197,14 @@ def test_second_pass_of_tiles_of_one_column_group(launches):
         assert status == 0 and blocks * tiles <= grids[2][0] < (blocks + 64) * tiles, (call, grids)
 
 
+def test_remainders_of_small_float16_launches(launches):
+    """55 row blocks of 128 rows, 17 resident beside 15 column tiles: launches of few workgroups take four groups of 17, the last one's
+    rows spread over all of its blocks; others take groups of equal size."""
+    few, many = launches("rank1 half 6974 3840", "rank1 half" + 2 * " 6974 3840")
+    assert few[0] == 0 and [x for x, y in few[1][1:3]] == [4 * 17 * 15] * 2
+    assert many[0] == 0 and [x for x, y in many[1][1:3]] == [2 * 4 * 14 * 15] * 2
+
+
 def test_config_defaults_and_yaml():
     from lpmm.config import CONFIG_DIR, get_config
 
