@@ -529,8 +529,13 @@ constexpr uint64_t kSpreadBelow = 1280;
 //   * few values leave the chip idle with tall tiles.  2048 x 2048 alone: 64 rows 22.3 / 10.0, 32 rows 15.9 / 7.9, 16 rows
 //     14.2 / 7.3; 32 weights of 256 x 2304: 59 / 21, 52 / 22, 50 / 24; of 512 x 2048: 90 / 37, 87 / 35, 84 / 43; 24 of
 //     1600 x 6400 (246M values): 571 / 209, 560 / 218, 578 / 274.  So the second pass goes below 64 rows only under
-//     14M values, the update pass under 64M.  Tiles of one column group hold half as many values: second pass on 5000 x 640
-//     with 32 and 16 rows 6.7, 8.2 (fp32 first moment 6.5, 8.0), on 4000 x 640 6.8, 6.3 (6.4, 5.8);
+//     14M values, the update pass under 64M;
+//   * tiles of one column group (narrow matrices, odd numbers of groups) hold half as many values, so their limits lie at fewer.
+//     24 of 3760 x 128: 16 rows 40.7 / 18.4, 32 rows 32.3 / 14.7, 64 rows 31.6 / 12.5; 8 of 4000 x 384: 43.3 / 21.5, 34.4 / 15.8, 34.8 /
+//     12.4; 8 of 9000 x 128: 44.5 / 14.8, 31.0 / 12.1, 27.0 / 9.9; second pass on 5000 x 640 8.2, 6.7, 7.5, on 4000 x 640 16 rows 6.3,
+//     32 rows 6.8; but 24 of 600 x 128 8.2 / 5.7, 8.7 / 6.0, 12.4 / 6.8;
+//   * byte codes gain less from short tiles: update of 4096 x 4096 56 with 16 rows, 51.6 with 32, 50.4 with 64, of 24 of 4000 x 256 85.0,
+//     74.3, 79.2, of 8 of 626 x 2304 (11.5M values) 39.3, 40.3, 39.8, of 6 of 2000 x 640 31.5, 28.2, 26.6;
 //   * no more than 256 row blocks of 16 rows on a column: their atomics on one address queue up (8192 x 256 among 5.5M
 //     values: 16 rows 27.2, 32 rows 20.9), nor many more than 256 of 32 rows (21788 x 256: 32 rows 42.5, 64 rows 36.0 to 38.8);
 //   * larger launches: the update pass does best with 32 rows where a DPP row is a whole column block (LLaMA-7B decoder
@@ -549,13 +554,19 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
 {
     if (l.half_io)
         return kPolicyRowsHalf;
+    const bool single = choose_lg_wide(col_blocks) == 0;  // tiles of one column group
     if (requant)
-        return l.values < (choose_lg_wide(col_blocks) == 0 ? 3e6 : 4e6) ? kPolicyRows / 4 : l.values < 14e6 || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
+        return l.values < (single ? 3e6 : 4e6) ? kPolicyRows / 4
+               : l.values < (single ? 6e6 : 14e6) || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
     uint32_t tile_rows;
-    if (l.values < 64e6)
-        tile_rows = rows <= 256 * (int64_t)(kPolicyRows / 4) ? kPolicyRows / 4 : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
-    else
+    if (l.values >= 64e6)
         tile_rows = l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
+    else if (single)
+        tile_rows = l.values < 3e6 && rows <= 2048 ? kPolicyRows / 4
+                    : rows <= 8192 && !(l.bits && l.values >= 6e6) ? kPolicyRows / 2 : kPolicyRows;
+    else
+        tile_rows = rows <= 256 * (int64_t)(kPolicyRows / 4) && !(l.bits && l.values >= 14e6) ? kPolicyRows / 4
+                    : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
     const double values = (double)rows * (double)col_blocks * kGroup;
     const double most = values / kValuesPerRowBlock > 512 ? values / kValuesPerRowBlock : 512;
     while (tile_rows < kPolicyRowsMost && (double)rows > most * tile_rows)

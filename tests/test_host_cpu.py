@@ -197,6 +197,16 @@ def test_second_pass_of_tiles_of_one_column_group(launches):
         assert status == 0 and blocks * tiles <= grids[2][0] < (blocks + 64) * tiles, (call, grids)
 
 
+def test_update_tiles_of_small_launches(launches):
+    """Workgroups of the update pass (row blocks times column tiles; full groups, so that none is empty): tiles of one column group have 16
+    rows only in the smallest launches, byte codes 32 rows at least from 14M values on."""
+    want = {"rank1 codes4 2048 128": 2048 // 16, "rank1 codes4" + 24 * " 4096 128": 24 * 4096 // 32, "rank1 float_m" + 24 * " 4096 128": 24 * 4096 // 32,
+            "rank1 codes8" + 24 * " 4096 128": 24 * 4096 // 64, "rank1 codes8 4096 4096": 4096 // 32 * 16, "rank1 codes4 4096 4096": 4096 // 16 * 16,
+            "rank1 codes8 2048 2048": 2048 // 16 * 8}
+    for (call, tiles), (status, grids) in zip(want.items(), launches(*want)):
+        assert status == 0 and grids[1] == (tiles, 1), (call, grids)
+
+
 def test_remainders_of_small_float16_launches(launches):
     """55 row blocks of 128 rows, 17 resident beside 15 column tiles: launches of few workgroups take four groups of 17, the last one's
     rows spread over all of its blocks; others take groups of equal size."""
