@@ -573,7 +573,8 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         return false;
     PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *scratch = get(nd_scratch, po);
     PyObject *row = get(scratch, N.row);
-    const Ref work = reals_of(get(scratch, N.work), p, 3 * r.cols);
+    const int64_t pitch = (r.cols + 31) / 32 * 32;  // _nd_pitch
+    const Ref work = reals_of(get(scratch, N.work), p, 3 * pitch);
     float *now[LPMM_RANK1_ND_MAX], *next[LPMM_RANK1_ND_MAX];
     if (!statistics(cur, p, now) || !statistics(nxt, p, next) || work == nullptr || get(scratch, N.scale_of) != cur || row == nullptr || !PyLong_Check(row))
         return false;
@@ -593,12 +594,12 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         return false;
     float *const rows = use<float>(work);
     fold.ndim = dims - 1;
-    fold.x = rows + raw_row * r.cols;
-    fold.scale = rows + new_row * r.cols;
+    fold.x = rows + raw_row * pitch;
+    fold.scale = rows + new_row * pitch;
     r.v_rowmax = now[0];
     r.v_rowmax_next = next[0];
-    r.v_colmax = rows + old_row * r.cols;
-    r.v_colmax_next = rows + raw_row * r.cols;
+    r.v_colmax = rows + old_row * pitch;
+    r.v_colmax_next = rows + raw_row * pitch;
     // any_mc: a column count for the general kernels, which also need the next scales
     PyObject *spare = get(spare_scales, po);
     const Ref ms_next = any_mc != nullptr ? reals_of(spare, p, (p.numel() + 127) / 128) : nullptr;
@@ -615,7 +616,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     if (any_mc == nullptr) {
         Batch &b = batch(kNd, p, qm, qv);
         add(b, r, item);
-        r.v_colmax_next = rows + new_row * r.cols;
+        r.v_colmax_next = rows + new_row * pitch;
         append(b.second, r);
         b.fold.push_back(fold);
         return true;
@@ -628,7 +629,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     swap_later(item, oh_m, N.max1, spare);
     Batch &b = batch(kNdAny, p, qm, qv);
     add(b, w, item);
-    w.v_colmax_next = rows + new_row * r.cols;
+    w.v_colmax_next = rows + new_row * pitch;
     append(b.second, w);
     b.fold.push_back(fold);
     return true;

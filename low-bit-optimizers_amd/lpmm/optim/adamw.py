@@ -85,6 +85,13 @@ def _zero_byte(qmap):
     return hit[1]
 
 
+def _nd_pitch(cols):
+    """Floats from one vector of AdamW._nd_scratch to the next, so that no two share a cache line: every workgroup of the first pass
+    reads the scale, and a line of it that also holds column maxima goes back and forth between the XCDs with their atomics
+    (281283 x 48 x 3 x 3, tiles of 32 rows: first pass 683 -> 334 us).  csrc/walk.cpp has the same."""
+    return -(-cols // 32) * 32
+
+
 class _Routes:
     """What the quantisation settings of the two moments allow."""
 
@@ -1087,7 +1094,7 @@ class AdamW(LowBitOptimizer):
                 scratch = self._nd_scratch.get(p)
                 if scratch is None or scratch["work"].device != p.device:
                     scratch = self._nd_scratch[p] = {
-                        "work": torch.empty((3, cols), dtype=torch.float32, device=p.device), "scale_of": None, "row": 0}
+                        "work": torch.empty((3, _nd_pitch(cols)), dtype=torch.float32, device=p.device), "scale_of": None, "row": 0}
                 work = scratch["work"]
                 # rows of `work`: the column scale of the current statistics, the column maxima of the new
                 # second moment, the column scale of the next statistics.  The last step's third row is this
@@ -1100,7 +1107,7 @@ class AdamW(LowBitOptimizer):
                                                      _shape_array(trailing), work[0].data_ptr(), stream)
                     _native.check(st, "rank1_row_scale_nd")
                 raw_row, new_row = [r for r in range(3) if r != old_row]
-                row_ptr = [work.data_ptr() + 4 * cols * r for r in range(3)]
+                row_ptr = [work[r].data_ptr() for r in range(3)]
                 if whole:
                     head, tail = (dense.data_ptr(), grad.data_ptr(), mc, ms, vc), (rows, cols, step, 0.0)
                 else:
@@ -1189,7 +1196,7 @@ class AdamW(LowBitOptimizer):
 
     @property
     def _nd_scratch(self):
-        # three vectors of numel / shape[0] floats per tensor of more than two dimensions (the column
+        # three vectors of numel / shape[0] floats (_nd_pitch apart) per tensor of more than two dimensions (the column
         # scale of the current statistics, the column maxima of the new second moment, the column
         # scale of the next statistics) and which statistics the kept scale belongs to; not part of
         # the optimizer state

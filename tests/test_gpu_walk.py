@@ -459,3 +459,24 @@ def test_which_tensors_share_launches(case, monkeypatch):
         assert calls.count(one) == 1
         assert not {"lpmm_adamw4bit_step_multi", "lpmm_adamw_fp32_step_multi", "lpmm_nonfused_adamw4bit_step_multi",
                     "lpmm_nonfused_update_multi"} & set(calls)
+
+
+@pytest.mark.parametrize("serve", [True, False])
+def test_scratch_vectors_share_no_cache_line(serve, monkeypatch):
+    """Tensors of more than two dimensions: the column scale and the column maxima of the passes, whatever the columns."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    params = [torch.nn.Parameter(torch.randn(s, device="cuda")) for s in [(300, 12, 6, 6), (90, 7, 7, 9), (40, 64, 3, 3), (64, 128, 1, 1)]]
+    opt = lpmm.optim.AdamW(params, lr=1e-2, qconfig=path)
+    monkeypatch.setattr(adamw, "_native", _Native(_native, serve))
+    for step in range(3):
+        for p in params:
+            p.grad = torch.randn_like(p)
+        opt.step()
+    for p in params:
+        work, cols = opt._nd_scratch[p]["work"], p.numel() // p.shape[0]
+        assert work.dtype is torch.float32 and work.shape[0] == 3 and work.shape[1] >= cols
+        assert all(work[r].data_ptr() % 128 == 0 for r in range(3))
