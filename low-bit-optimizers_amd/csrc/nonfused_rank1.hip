@@ -546,8 +546,9 @@ constexpr uint64_t kSpreadBelow = 1280;
 //     one address are then less than the time of its values (13.5 to 20.5 bytes each at 6 TB/s).  Steps with tiles of 16, 32, 64, 128
 //     rows: 1048576 x 128 1377, 777, 498, 450 (fp32 first moment 1379, 805, 628, 621; 8 bits 1406, 822, 508, 504), 524288 x 256
 //     769, 492, 448, 443, 262144 x 512 492, 426, 430, 438, 131072 x 1024 419, 421, 428, 437 (fp32 573, 584, 596, 605);
-//   * rows of an odd column count: the second pass sets the 4-bit codes of shared bytes by atomics, which shorter tiles spread (six
-//     tensors of 4095 x 4099, a step: 64 rows 986, 32 rows 965; fp32 first moment 851, 834).
+//   * rows of an odd column count: the second pass sets the 4-bit codes of shared bytes by atomics, which shorter tiles spread.  Six
+//     tensors of 4095 x 4099: 64 rows 657, 32 rows 630, 16 rows 614 (fp32 first moment 414, 396, 376); 5000 x 5001 128, 127, 123; 2072 x 4615
+//     50, 59 (1235 workgroups, a fifth more than are resident together), 52; ten of 1001 x 1003 54, 58, 51; but 2001 x 3001 40, 34, 36.
 // The float16 passes are bound by their arithmetic: tall tiles spread a tile's set-up (four decoder layers of width 4096:
 // 32 rows 1821, 64 rows 1751, 128 rows 1729 a step).
 static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, uint32_t col_blocks, bool odd_cols)
@@ -555,9 +556,10 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     if (l.half_io)
         return kPolicyRowsHalf;
     const bool single = choose_lg_wide(col_blocks) == 0;  // tiles of one column group
+    if (requant && odd_cols && !l.bits)
+        return l.values >= (single ? 3e6 : 4e6) && l.values < 9e6 ? kPolicyRows / 2 : kPolicyRows / 4;
     if (requant)
-        return l.values < (single ? 3e6 : 4e6) ? kPolicyRows / 4
-               : l.values < (single ? 6e6 : 14e6) || (odd_cols && !l.bits) ? kPolicyRows / 2 : kPolicyRows;
+        return l.values < (single ? 3e6 : 4e6) ? kPolicyRows / 4 : l.values < (single ? 6e6 : 14e6) ? kPolicyRows / 2 : kPolicyRows;
     uint32_t tile_rows;
     if (l.values >= 64e6)
         tile_rows = l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;

@@ -5,6 +5,7 @@
 //   dequant BITS ROWS COLS              the way back
 //   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment), codes8 or
 //                                       half (float16)
+//   any ROWS COLS [ROWS COLS]...        one step with 4-bit codes by the kernels for any column count
 // and one line of output its status and the grids, "x,y" each.
 // Build: g++ -O1 -rdynamic -D__HIP_PLATFORM_AMD__ -I<rocm>/include -I<include> launches.cpp -llpmm_hip
 #include <hip/hip_runtime_api.h>
@@ -91,6 +92,34 @@ static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, i
     return lpmm_nonfused_adamw4bit_rank1_step_multi(coded.data(), n, map, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
 }
 
+static int any_columns(const std::vector<std::pair<int64_t, int64_t>> &shapes)
+{
+    std::vector<lpmm_rank1_any_tensor> records;
+    for (const auto &[rows, cols] : shapes) {
+        lpmm_rank1_any_tensor t;
+        memset(&t, 0, sizeof t);
+        t.p = made_up();
+        t.g = made_up();
+        t.m = made_up();
+        t.m_codes_next = (uint8_t *)made_up();
+        t.m_max1 = made_up();
+        t.m_max1_next = made_up();
+        t.v_codes = (const uint8_t *)made_up();
+        t.v_codes_next = (uint8_t *)made_up();
+        t.v_rowmax = made_up();
+        t.v_colmax = made_up();
+        t.v_rowmax_next = made_up();
+        t.v_colmax_next = made_up();
+        t.rows = rows;
+        t.cols = cols;
+        t.step = 1.0f;
+        records.push_back(t);
+    }
+    const float *map = (const float *)made_up();
+    return lpmm_nonfused_adamw_rank1_any_step_multi(records.data(), (int64_t)records.size(), LPMM_RANK1_CODES4, 128, map, 4, nullptr, map, 4,
+                                                    nullptr, 0.9, 0.999, 1e-3, 0.01, 1e-8, 3, nullptr);
+}
+
 static int quantiser(bool back, int bits, int64_t rows, int64_t cols)
 {
     const float *x = (const float *)made_up(), *rowmax = (const float *)made_up(), *colmax = (const float *)made_up();
@@ -112,7 +141,7 @@ int main()
         std::vector<std::pair<int64_t, int64_t>> shapes;
         int64_t rows, cols;
         in >> call;
-        if (call != "stats")
+        if (call != "stats" && call != "any")
             in >> mode;
         while (in >> rows >> cols)
             shapes.push_back({rows, cols});
@@ -121,6 +150,7 @@ int main()
         const int status = call == "stats"   ? lpmm_rank1_stats((const float *)made_up(), r, c, (float *)made_up(), (float *)made_up(),
                                                                 nullptr)
                            : call == "rank1" ? rank1(mode, shapes)
+                           : call == "any"   ? any_columns(shapes)
                                              : quantiser(call == "dequant", std::stoi(mode), r, c);
         printf("%d", status);
         for (const dim3 &grid : launches)

@@ -207,6 +207,15 @@ def test_update_tiles_of_small_launches(launches):
         assert status == 0 and grids[1] == (tiles, 1), (call, grids)
 
 
+def test_second_pass_tiles_of_odd_columns(launches):
+    """Rows of an odd column count share code bytes: tiles of 16 rows, of 32 in between.  (The call takes any column count.)"""
+    for values_of, tile_rows in (((1000, 2001), 16), ((2001, 3001), 32), ((2072, 4615), 16), ((5000, 5001), 16)):
+        rows, cols = values_of
+        (status, grids), = launches(f"any {rows} {cols}")
+        blocks, tiles = -(-rows // tile_rows), -(-(-(-cols // 128)) // 2)
+        assert status == 0 and blocks * tiles <= grids[2][0] < (blocks + 256 // tiles) * tiles, (values_of, grids)
+
+
 def test_remainders_of_small_float16_launches(launches):
     """55 row blocks of 128 rows, 17 resident beside 15 column tiles: launches of few workgroups take four groups of 17, the last one's
     rows spread over all of its blocks; others take groups of equal size."""
