@@ -463,7 +463,7 @@ static uint32_t choose_lg_wide(uint32_t col_blocks)
 }
 
 constexpr double kValuesPerRowBlock = 12000;  // pass_rows_policy
-constexpr uint64_t kCombMultiple = 32;
+constexpr uint64_t kCombMultiple = 8;
 static_assert(kPolicyResident % kCombMultiple == 0, "a rounded group is no larger than the resident set");
 
 // Row blocks of a matrix, and its tiles side by side.
@@ -498,10 +498,11 @@ static uint64_t shape_tiles(int64_t rows, uint32_t col_blocks, TileShape &ts, ui
         // groups of equal size, so that the last one holds few empty blocks (13 row blocks in groups of 5, not 6)
         const uint64_t groups = (b.rows + comb - 1) / comb;
         comb = (b.rows + groups - 1) / groups;
-        // Large groups (narrow matrices) hold a multiple of 32 blocks: neighbours share cache lines of row statistics and scales, and with
+        // Large groups (narrow matrices) hold a multiple of 8 blocks: neighbours share cache lines of row statistics and scales, and with
         // an odd number the sharing blocks, and the XCDs they are on, change from pass to pass.  Update and second pass, equal groups ->
-        // multiples of 32: 50257 x 128 31.6 / 10.9 -> 28.6 / 9.1 us, 21788 x 256 25.4 / 9.1 -> 23.0 / 7.3.
-        if (comb >= 2 * kCombMultiple)
+        // multiples of 8: 50257 x 128 31.7 / 10.9 -> 29.1 / 9.1 us, 100000 x 128 49.2 / 16.0 -> 49.3 / 14.9.  (Multiples of 32 leave more
+        // blocks empty: a step on 24 of 12592 x 278 632 -> 660.)
+        if (comb >= 64)
             comb = (comb + kCombMultiple - 1) / kCombMultiple * kCombMultiple;
     }
     ts.lg_wide = b.lg_wide;
@@ -517,12 +518,13 @@ struct LaunchKind {
     bool spread[2];  // update pass, second pass: see shape_tiles
 };
 
-// Launches of fewer workgroups than this have their remainders spread: the float16 kernels and those for any column count, whose tiles take
-// longest.  Update and second pass (us; equal groups -> spread): float16 6974 x 3840 59.6 / 24.8 -> 53.2 / 23.5, 1962 x 6831 61.8 / 89.3
-// -> 54.7 / 84.2, 39877 x 128 27.7 / 10.7 -> 24.1 / 9.2, but 11008 x 4096 (1376 workgroups) 84.1 / 34.1 -> 86.0 / 35.6 and eight of
-// 962 x 9856 (2496) 141.5 / 60.0 -> 155.6 / 63.5; second pass on 1071 x 7515 51.4 -> 45.9, at 8 bits 28.8 -> 24.0, two of 5000 x 2000 at
-// 8 bits 52.7 -> 47.9, but 24 of 2196 x 1956 (6720) 202.8 -> 214.9.
-constexpr uint64_t kSpreadBelow = 1280;
+// Launches of fewer workgroups than are resident together have their remainders spread: those of the float16 kernels and of the ones for any
+// column count, whose tiles take longest, and those of one tensor.  Update and second pass (us; equal groups -> spread): float16
+// 6974 x 3840 59.6 / 24.8 -> 53.2 / 23.5, 1962 x 6831 61.8 / 89.3 -> 54.7 / 84.2, 39877 x 128 27.7 / 10.7 -> 24.1 / 9.2, but a step on four of
+// 39394 x 128 (1232 workgroups) 74 -> 78, 11008 x 4096 (1376) 84.1 / 34.1 -> 86.0 / 35.6, eight of 962 x 9856 (2496) 141.5 / 60.0 -> 155.6 /
+// 63.5; second pass on 1071 x 7515 51.4 -> 45.9, at 8 bits 28.8 -> 24.0; float32 21788 x 256 24.9 / 7.9 -> 23.4 / 7.3, 20000 x 128 15.8 /
+// 5.4 -> 15.0 / 5.5, but four of 482 x 4608 26 / 10.4 -> 26 / 12.2.
+constexpr uint64_t kSpreadBelow = 1024;
 
 // Rows of a pass's tiles on a matrix of `rows` rows.  A tile of fewer rows means more column atomics and more set-up, one of
 // more rows a longer walk, fewer workgroups and a longer end of the launch.  Measured (us; update pass, then second pass):
@@ -596,6 +598,20 @@ static float *next_scales(const lpmm_rank1_mgroup_tensor &t) { return t.m_max1_n
 
 // a tensor that the kernels take as double rows
 static bool folds(int64_t rows, int64_t cols) { return cols % kGroup == 64 && rows % 2 == 0; }
+
+// The matrix that a pass's tiles cover; can_fold: column counts that are no multiple of 128 are folded (and satisfy folds).
+struct Matrix {
+    int64_t rows;
+    uint32_t col_blocks;
+    bool fold;
+};
+
+static Matrix matrix_of(int64_t rows, int64_t cols, bool can_fold)
+{
+    const uint32_t blocks = (uint32_t)((cols + kGroup - 1) / kGroup);
+    const bool fold = can_fold && cols % kGroup != 0;
+    return fold ? Matrix{rows / 2, 2 * blocks - 1, true} : Matrix{rows, blocks, false};
+}
 
 template <int MODE, bool FOLD>
 static void launch_rank1_passes(const R1Launch &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
@@ -769,13 +785,17 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
                     ++k;
                 }
         };
-        each([&](const Record &t) { kind.values += (double)t.rows * (double)t.cols; });
-        if (general || half_io) {
+        int held = 0;
+        each([&](const Record &t) {
+            kind.values += (double)t.rows * (double)t.cols;
+            ++held;
+        });
+        if (general || half_io || held == 1) {
             uint64_t blocks[2] = {0, 0};
             each([&](const Record &t) {
-                const uint32_t col_blocks = (uint32_t)((t.cols + kGroup - 1) / kGroup);
+                const Matrix m = matrix_of(t.rows, t.cols, can_fold);
                 for (int pass = 0; pass < 2; ++pass) {
-                    const Blocks b = blocks_of(t.rows, col_blocks, pass_rows_policy(kind, pass == 1, false, t.rows, col_blocks, t.cols & 1));
+                    const Blocks b = blocks_of(m.rows, m.col_blocks, pass_rows_policy(kind, pass == 1, m.fold, m.rows, m.col_blocks, t.cols & 1));
                     blocks[pass] += b.rows * b.col_tiles;
                 }
             });
@@ -795,11 +815,12 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             }
             const uint32_t col_blocks = (uint32_t)((t.cols + kGroup - 1) / kGroup);
             TensorR1 &d = args.t[k];
-            const bool fold = t.cols % kGroup != 0 && can_fold;  // validated above: 64 modulo 128, even rows
-            const int64_t rows = fold ? t.rows / 2 : t.rows;
-            const uint32_t blocks = fold ? 2 * col_blocks - 1 : col_blocks;
-            const uint64_t nt = shape_tiles(rows, blocks, d.tile, pass_rows_policy(kind, false, fold, rows, blocks, t.cols & 1), kind.spread[0]);
-            const uint64_t nt2 = shape_tiles(rows, blocks, shape2[k], pass_rows_policy(kind, true, fold, rows, blocks, t.cols & 1), kind.spread[1]);
+            const Matrix m = matrix_of(t.rows, t.cols, can_fold);
+            const bool odd = t.cols & 1;
+            const uint64_t nt = shape_tiles(m.rows, m.col_blocks, d.tile, pass_rows_policy(kind, false, m.fold, m.rows, m.col_blocks, odd),
+                                            kind.spread[0]);
+            const uint64_t nt2 = shape_tiles(m.rows, m.col_blocks, shape2[k], pass_rows_policy(kind, true, m.fold, m.rows, m.col_blocks, odd),
+                                             kind.spread[1]);
             if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
             d.p = t.p;
@@ -822,7 +843,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             d.rbc2_sqrt = h.rbc2_sqrt;
             tiles += nt;
             tiles2 += nt2;
-            folded = folded || fold;
+            folded = folded || m.fold;
             args.tile_start[++k] = (uint32_t)tiles;
             start2[k] = (uint32_t)tiles2;
             ++i;

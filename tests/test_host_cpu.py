@@ -162,12 +162,12 @@ NARROW = [(mode, rows, cols) for mode in ("codes4", "float_m", "codes8")
 
 
 def test_interleaved_groups_of_narrow_matrices(launches):
-    """Groups of row blocks that work on neighbouring rows are of a multiple of 32 blocks where they are large: neighbours share
+    """Groups of row blocks that work on neighbouring rows are of a multiple of 8 blocks where they are large: neighbours share
     cache lines of statistics and scales."""
     for case, (status, grids) in zip(NARROW, launches(*("rank1 %s %d %d" % case for case in NARROW))):
         assert status == 0 and len(grids) == 3, case
         for x, y in grids[1:]:
-            assert y == 1 and x % 32 == 0 and x * 128 >= case[1], (case, grids)
+            assert y == 1 and x % 8 == 0 and x * 128 >= case[1], (case, grids)
 
 
 def test_row_blocks_of_a_column(launches):
