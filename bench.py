@@ -41,6 +41,7 @@ HBM_PEAK_GBS = 8000.0          # MI355X HBM3E, published
 BYTES_PER_PARAM_4BIT = 14.125  # p r/w 8 + g 4 + m codes 1 + v codes 1 + scales 16/128
 BYTES_PER_PARAM_FP32 = 28.0    # p, m, v r/w + g r
 MULTI_MAX = 48                 # tensors per launch record (LPMM_MULTI_MAX)
+PLAIN_MAX = 64                 # tensors with fp32 states per launch
 # HBM bytes per launch of the dominant kernel are not measured by this script: they come from
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this same command (each counter scaled by what it
 # reads for a plain 1 GiB copy, --copy-probe), whose summary is kept in this file; the line
@@ -650,9 +651,13 @@ def main():
     n_total = sum(p.numel() for p in params)
     n_quant = sum(p.numel() for p in params if p.numel() > 4096)
     n_quant_tensors = sum(1 for p in params if p.numel() > 4096)
-    launches_per_step = math.ceil(n_quant_tensors / MULTI_MAX)
+    quant_launches = math.ceil(n_quant_tensors / MULTI_MAX)
+    plain_launches = math.ceil((len(params) - n_quant_tensors) / PLAIN_MAX)
+    # tensors of <= 4096 elements, whose states are fp32, go with the quantised ones' launches, one of theirs with each
+    joined_launches = min(quant_launches, plain_launches)
+    launches_per_step = max(quant_launches, plain_launches)
 
-    # events around the dominant kernel's launches (same stream as the launches): the call with both kinds of tensors
+    # events around the step's launches (same stream), as one call makes them for both kinds of tensors
     events = []
     recording = {"on": False}
 
@@ -694,8 +699,15 @@ def main():
     value = n_total / (elapsed / args.steps)
     kernel_ms_per_step = sum(e0.elapsed_time(e1) for e0, e1 in events) / args.steps
     launch_ms = kernel_ms_per_step / launches_per_step
-    bytes_per_launch = n_quant * BYTES_PER_PARAM_4BIT / launches_per_step
+    bytes_per_launch = (n_quant * BYTES_PER_PARAM_4BIT + (n_total - n_quant) * BYTES_PER_PARAM_FP32) / launches_per_step
     achieved = bytes_per_launch / (launch_ms * 1e-3) / 1e9
+
+    # second template argument, chosen per launch: every quantised tensor of the launch is a whole number of 2048-element tiles
+    full = "true" if all(p.numel() % 2048 == 0 for p in params if p.numel() > 4096) else "true|false"
+    kernels = ", ".join(f"{n} x {name}" for n, name in (
+        (quant_launches - joined_launches, f"lpmm::adamw4bit_kernel<true, {full}, lpmm::FusedArith4>"),
+        (joined_launches, f"lpmm::adamw_joined_kernel<true, {full}, lpmm::FusedArith4, lpmm::FusedArith>"),
+        (plain_launches - joined_launches, "lpmm::adamw_fp32_kernel<lpmm::FusedArith>")) if n)
 
     out = {
         "metric": "fused 4-bit AdamW step: params/sec and % HBM roofline, 1 MI355X",
@@ -717,16 +729,12 @@ def main():
         "verified": verified,
         "verified_on": verified_on,
         "config": {"workload": desc, "tensors": len(params), "params": n_total, "quantized_params": n_quant,
-                   # the 4-bit kernel's launches plus the fp32-state kernel's (tensors of <= 4096 elements, 64 per launch)
-                   "launches_per_step": max(launches_per_step, math.ceil((len(params) - n_quant_tensors) / 64))},
+                   "launches_per_step": launches_per_step},
         "effective_gbs": (n_quant * BYTES_PER_PARAM_4BIT + (n_total - n_quant) * BYTES_PER_PARAM_FP32)
         / (elapsed / args.steps) / 1e9,
         "roofline": {
             "bound": "hbm",
-            # second template argument, chosen per launch: every tensor of the launch is a whole
-            # number of 2048-element tiles
-            "kernel": "lpmm::adamw4bit_kernel<true, %s, lpmm::FusedArith4>" % (
-                "true" if all(p.numel() % 2048 == 0 for p in params if p.numel() > 4096) else "true|false"),
+            "kernel": kernels,
             "achieved": achieved,
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
