@@ -453,3 +453,57 @@ def test_joined_launch_equals_two(qmaps, counts, sizes, fused):
             assert torch.equal(x.view(torch.uint8), y.view(torch.uint8)), i
     assert both(None, 1, table_f.ctypes.data, len(nf), dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) != 0
     assert both(table.ctypes.data, -1, table_f.ctypes.data, 1, dqm.data_ptr(), dqv.data_ptr(), *hyper, stream) != 0
+
+
+@pytest.mark.parametrize("config", [None, "2nd_moment_group_128.yml"])
+def test_joined_launch_under_graph_capture(config):
+    """A whole step whose quantised tensors and tensors with fp32 states share launches, recorded into a HIP graph: each of four replays,
+    with eager work between them, leaves what the same step leaves on an optimizer beside it.  (A step's count is an argument of its
+    launches and stays as recorded: the other optimizer's are set back.)"""
+    import os
+
+    import lpmm
+
+    path = None if config is None else os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    sizes = [4098, 70, 2048 * 9, 4096, 1, 130 * 64, 640]
+    start = [torch.randn(n, device="cuda", generator=gen) for n in sizes]
+    sides = []
+    for _ in range(2):
+        params = [torch.nn.Parameter(p.clone()) for p in start]
+        opt = lpmm.optim.AdamW(params, lr=1e-3, weight_decay=0.01, fused=config is None, qconfig=path)
+        for p in params:
+            p.grad = torch.zeros_like(p)
+        sides.append((params, opt))
+    (params, captured), (others, eager) = sides
+
+    def gradients():
+        for p, q in zip(params, others):
+            p.grad.copy_(torch.randn(p.shape, device="cuda", generator=gen) * 1e-3)
+            q.grad.copy_(p.grad)
+
+    for _ in range(2):
+        gradients()
+        captured.step()
+        eager.step()
+    counts = [float(eager.state[q]["step"]) for q in others]
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            captured.step()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    for replay in range(4):
+        gradients()
+        graph.replay()
+        for q, count in zip(others, counts):
+            eager.state[q]["step"].fill_(count)
+        eager.step()
+        scratch = torch.randn(1 << 16, device="cuda", generator=gen).sum()
+        torch.cuda.synchronize()
+        assert torch.isfinite(scratch)
+        for p, q in zip(params, others):
+            assert torch.equal(p, q), (replay, p.numel())
+            for name in ("exp_avg", "exp_avg_sq"):
+                assert torch.equal(captured.state[p][name], eager.state[q][name]), (replay, p.numel(), name)

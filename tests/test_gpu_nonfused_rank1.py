@@ -262,7 +262,8 @@ def test_tile_shapes_do_not_show_in_the_result(config, half):
     dtype = torch.float16 if half else torch.float32
     shapes = [(272, 384), (17, 256), (130, 192), (200, 136), (96, 45), (48, 32, 3, 3), (40, 7, 5, 5), (9000, 128), (21788, 256)]
     want = None
-    for beside in (None, (1024, 4608), (4096, 4224), (8200, 8064)):
+    # the last two put launches above the values up to which loads stay in the cache, whole blocks and folded rows
+    for beside in (None, (1024, 4608), (4096, 4224), (8200, 8064), (16400, 16640), (16402, 16704)):
         gen = torch.Generator(device="cuda").manual_seed(5)
         params = [torch.nn.Parameter(torch.randn(s, device="cuda", generator=gen).to(dtype)) for s in shapes]
         grads = [[torch.randn(s, device="cuda", generator=gen).mul_(0.1).to(dtype) for s in shapes] for _ in range(3)]

@@ -372,3 +372,43 @@ def test_half_second_moment_with_gradients_off_a_boundary(offset, monkeypatch):
             opts[1].step()
         for j, (got, want) in enumerate(zip(_tensors(opts[0], params[0])[1:], _tensors(opts[1], params[1])[1:])):
             _same(got, want, f"step {step}, {j}")
+
+
+@pytest.mark.parametrize("config, dtype", [("default.yml", torch.float32), ("2nd_moment_only_default.yml", torch.float32),
+                                           ("default_8b.yml", torch.float32), ("1st_moment_group_256.yml", torch.float32),
+                                           ("default.yml", torch.float16)])
+def test_runs_and_single_values_in_one_call(config, dtype):
+    """More tensors than a launch holds, in turn with columns that go in runs of four and columns that do not: alone they go together, one
+    value at a time, and beside a tensor of 24M values that is worth it in launches of either kind.  The same bits."""
+    import lpmm
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    shapes = [(70 + k, 60 + 4 * k) if k % 2 else (64 + k, 65 + 2 * k) for k in range(40)] + [(40, 7, 5, 5), (48, 4, 3, 3)]
+    if dtype is torch.float16:
+        shapes = [s for s in shapes if len(s) == 2]
+    want = None
+    for beside in ([], [(6004, 4004)]):
+        gen = torch.Generator(device="cuda").manual_seed(6)
+        params = [torch.nn.Parameter(torch.randn(s, device="cuda", generator=gen).to(dtype)) for s in shapes]
+        grads = [[torch.randn(s, device="cuda", generator=gen).mul_(0.1).to(dtype) for s in shapes] for _ in range(3)]
+        others = [torch.nn.Parameter(torch.zeros(s, dtype=dtype, device="cuda")) for s in beside]
+        for p in others:
+            p.grad = torch.ones_like(p)
+        opt = lpmm.optim.AdamW(params[:7] + others + params[7:], lr=1e-3, eps=1e-3, weight_decay=0.01, fused=False, qconfig=path)
+        for step in grads:
+            for p, g in zip(params, step):
+                p.grad = g
+            opt.step()
+        got = []
+        for p in params:
+            state = opt.state[p]
+            got += [p.detach(), state["exp_avg"], state["exp_avg_sq"]]
+            for name in ("exp_avg_qstate", "exp_avg_sq_qstate"):
+                overhead = state[name]["overhead"]
+                got += [t for t in [overhead.get("max1")] + list(overhead.get("max_dims") or ()) if t is not None]
+        for p in others:
+            assert torch.isfinite(p).all() and (p.detach() == p.detach().view(-1)[0]).all()
+        want = want or got
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b), (beside, tuple(a.shape))
