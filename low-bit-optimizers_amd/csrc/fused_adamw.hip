@@ -491,6 +491,8 @@ __global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
 // are latency (6 us each; GPT-2-XL's set has five).
 // A small model's step is bound by the host, which a launch costs about 7 us (the call, its kernel arguments, the device and stream around it):
 // fifty tensors of 7.5M values 39.5 -> 33.2 us a step.
+static_assert(sizeof(Multi4) + sizeof(MultiF) + 3 * sizeof(void *) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
+
 template <bool ALIGNED, bool ALLFULL, class Arith, class ArithF>
 __global__ __launch_bounds__(kThreads) void adamw_joined_kernel(const Multi4 args, const MultiF plain, const float *__restrict__ qmap_m,
                                                                 const float *__restrict__ qmap_v, uint32_t tiles)

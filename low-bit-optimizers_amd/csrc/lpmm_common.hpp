@@ -33,6 +33,11 @@ inline int launch_status()
     return hipGetLastError() == hipSuccess ? LPMM_OK : LPMM_ERR_LAUNCH;
 }
 
+// Bytes of a kernel's arguments.  Every launch copies them, so one array of records takes 4 KB at most ("kernel arguments exceed 4 KB" at
+// each); a launch that takes two (quantised tensors with others, records with the arrays for their new codes) 8 KB.  HIP states no limit
+// of its own; the tests launch the largest.
+constexpr size_t kMostKernargBytes = 8192;
+
 // ---------------------------------------------------------------------------------------
 // Tile order of the one-shot streaming kernels.  The hardware hands consecutive workgroup indices to
 // the 8 XCDs of an MI355X in turn, so with "workgroup i takes tile i" every XCD touches every

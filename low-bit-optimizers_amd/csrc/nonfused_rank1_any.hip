@@ -25,8 +25,8 @@
 // launches a tensor and 50 bytes a value; float16: about thirty PyTorch ops a tensor).  One step on one tensor,
 // staged -> here: 4096 x 4100 default 224 -> 107 us, fp32 first moment 183 -> 104, 8 bits 221 -> 102, float16
 // 539 -> 151; 4095 x 4099 271 -> 142; 50000 x 34 122 -> 55 (4096 x 4096 on the tuned kernels: 74-84, float16 67).
-// What bounds them: instructions, the code bytes' extraction and one access per value (the tuned kernels move
-// the same bytes in a quarter of the accesses); most of the gain on small tensors is launches.
+// What bounds them: instructions; with single values also the code bytes' extraction and one access per value (runs and the tuned
+// kernels move the same bytes in a quarter of the accesses); most of the gain on small tensors is launches.
 #include "lpmm_half.hpp"
 #include "lpmm_search.hpp"
 

@@ -254,6 +254,7 @@ struct NewCodes {  // where the second pass puts a tensor's codes
     uint8_t *m[kR1Max], *v[kR1Max];
     bool runs;  // every tensor of the launch may be taken in runs of four values (rank1_any_runs)
 };
+static_assert(sizeof(MultiR1) + sizeof(NewCodes) + 6 * sizeof(void *) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
 bool rank1_any_runs(const lpmm_rank1_any_tensor &t, AnyKind kind);
 // passes: 1 the first, 2 the second, 3 both
 void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_m, const float *qmap_v,
