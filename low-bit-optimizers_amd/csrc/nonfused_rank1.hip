@@ -518,12 +518,12 @@ struct LaunchKind {
     bool spread[2];  // update pass, second pass: see shape_tiles
 };
 
-// Launches of fewer workgroups than are resident together have their remainders spread: those of the float16 kernels and of the ones for any
-// column count, whose tiles take longest, and those of one tensor.  Update and second pass (us; equal groups -> spread): float16
-// 6974 x 3840 59.6 / 24.8 -> 53.2 / 23.5, 1962 x 6831 61.8 / 89.3 -> 54.7 / 84.2, 39877 x 128 27.7 / 10.7 -> 24.1 / 9.2, but a step on four of
-// 39394 x 128 (1232 workgroups) 74 -> 78, 11008 x 4096 (1376) 84.1 / 34.1 -> 86.0 / 35.6, eight of 962 x 9856 (2496) 141.5 / 60.0 -> 155.6 /
-// 63.5; second pass on 1071 x 7515 51.4 -> 45.9, at 8 bits 28.8 -> 24.0; float32 21788 x 256 24.9 / 7.9 -> 23.4 / 7.3, 20000 x 128 15.8 /
-// 5.4 -> 15.0 / 5.5, but four of 482 x 4608 26 / 10.4 -> 26 / 12.2.
+// Launches of fewer workgroups than are resident together have their remainders spread: those of the float16 kernels and of the
+// ones for any column count, whose tiles take longest, and those of one tensor.  Update and second pass (us; equal groups ->
+// spread): float16 6974 x 3840 59.6 / 24.8 -> 53.2 / 23.5, 1962 x 6831 61.8 / 89.3 -> 54.7 / 84.2, 39877 x 128 27.7 / 10.7 ->
+// 24.1 / 9.2, but a step on four of 39394 x 128 (1232 workgroups) 74 -> 78, 11008 x 4096 (1376) 84.1 / 34.1 -> 86.0 / 35.6, eight
+// of 962 x 9856 (2496) 141.5 / 60.0 -> 155.6 / 63.5; second pass on 1071 x 7515 51.4 -> 45.9, at 8 bits 28.8 -> 24.0; float32
+// 21788 x 256 24.9 / 7.9 -> 23.4 / 7.3, 20000 x 128 15.8 / 5.4 -> 15.0 / 5.5, but four of 482 x 4608 26 / 10.4 -> 26 / 12.2.
 constexpr uint64_t kSpreadBelow = 1024;
 
 // Rows of a pass's tiles on a matrix of `rows` rows.  A tile of fewer rows means more column atomics and more set-up, one of
@@ -542,8 +542,8 @@ constexpr uint64_t kSpreadBelow = 1024;
 //     values: 16 rows 27.2, 32 rows 20.9), nor many more than 256 of 32 rows (21788 x 256: 32 rows 42.5, 64 rows 36.0 to 38.8);
 //   * larger launches: the update pass does best with 32 rows where a DPP row is a whole column block (LLaMA-7B decoder
 //     layers 1853 -> 1818), with 16 where the first moment is fp32 (a pass moves 20.5 instead of 13.5 bytes a value; a step of
-//     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold or codes are bytes
-//     (GPT-2-XL's set 5590 -> 5549 a step; 8 bits 2925 -> 2916).
+//     these layers with 64, 32, 24, 16 rows: 3515, 3425, 3375, 3333) and with 64 where rows fold (GPT-2-XL's set 5590 ->
+//     5549 a step); for byte codes 32 and 64 rows are the same (2925, 2916 a step, within the spread of one side's runs).
 //   * whatever the launch holds, a column takes no more row blocks than one per 12000 values of its matrix, or 512: 18 ns an atomic on
 //     one address are then less than the time of its values (13.5 to 20.5 bytes each at 6 TB/s).  Steps with tiles of 16, 32, 64, 128
 //     rows: 1048576 x 128 1377, 777, 498, 450 (fp32 first moment 1379, 805, 628, 621; 8 bits 1406, 822, 508, 504), 524288 x 256

@@ -628,8 +628,9 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_requant_any_kernel(const Mu
     const TensorR1 &t = args.t[lo];
     const uint32_t index = blockIdx.x - args.tile_start[lo];
     // Rows of an odd column count share bytes of the new codes: neighbouring tiles meet in atomics on the
-    // words around them, and launch order, which spreads them over the XCDs, is faster (six tensors of 4095 x 4099, a step, neighbours on one XCD -> here: 4 bits 965 -> 948 us,
-    // fp32 first moment 834 -> 823, float16 812 -> 791; byte codes share nothing and lose 606 -> 617).
+    // words around them, and launch order, which spreads them over the XCDs, is faster (six tensors of 4095 x 4099, a step,
+    // neighbours on one XCD -> here: 4 bits 965 -> 948 us, fp32 first moment 834 -> 823, float16 812 -> 791; byte codes share
+    // nothing and lose 606 -> 617).
     const bool shared = !BITS && !VEC && (t.col_tail & 1) != 0;
     const uint32_t tl = shared ? index : xcd_neighbours(index, args.tile_start[lo + 1] - args.tile_start[lo]);
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;

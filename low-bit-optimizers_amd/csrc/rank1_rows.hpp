@@ -11,8 +11,8 @@
 // one division of the index and plain divisions for other columns, 16 lanes to 128 columns for multiples of 128):
 //                     rows          flat          before
 //   50257 x 1600      62.8 / 80.4   78.5 / 72.7   73.8 / 99.2
-//   16384 x 4096      49.4 / 57     70.4 / 68.4   49.9 / 57.6
-//   524288 x 128      47.8 / 57     63.6 / 56.7   154.6 / 153.8
+//   16384 x 4096      47.9 / 55.1   70.4 / 68.4   47.8 / 57.0
+//   524288 x 128      48.2 / 54.5   63.6 / 56.7   157.5 / 152.3
 //   20000 x 1000      18.8 / 22.0   23.3 / 20.2   24.4 / 29.0
 //   40000 x 500       18.4 / 24.2   22.8 / 19.3   49.7 / 46.5
 //   60000 x 300       24.2 / 28.2   21.7 / 17.4   45.1 / 42.7
@@ -212,11 +212,12 @@ __device__ __forceinline__ void flat_store(float *__restrict__ out, int64_t idx,
 
 // ---- host: which split, and its shape ----------------------------------------------------
 // The rows split where it is the faster one (the table above), and the column groups of its chunks.  Chunks of 16 or 8 groups, whose
-// workgroups take runs of 8 or 4 KB, where at most 3 % of them lie beyond the row's end; else narrow ones from 4096 columns on, several
-// rows side by side, if rows start on cache lines.  Otherwise a quantiser takes the widest chunk that leaves at most a tenth of the lanes idle, else the one
-// that leaves fewest; a dequantiser, which has nothing to keep over the rows but cuts lines at a chunk's end, whole rows of 1, 2 or 4 groups,
-// pairs of groups from 12 groups on, and for the rest the flat split.  Dequantisers (us, 4 / 8 bits; "lanes": with the quantiser's
-// rule for every column count that is a multiple of 128; "before" as above):
+// workgroups take runs of 8 or 4 KB, where at most 3 % of them lie beyond the row's end; else narrow ones from 4096 columns on,
+// several rows side by side, if rows start on cache lines.  Otherwise a quantiser takes the widest chunk that leaves at most a
+// tenth of the lanes idle, else the one that leaves fewest; a dequantiser, which has nothing to keep over the rows but cuts lines
+// at a chunk's end, whole rows of 1, 2 or 4 groups, pairs of groups from 12 groups on, and for the rest the flat split.
+// Dequantisers (us, 4 / 8 bits; "lanes": with the quantiser's rule for every column count that is a multiple of 128; "before" as
+// above; 1.5 to 2 % slower than before: 1280, 1536 and 1920 columns at 4 bits):
 //                  lanes         here          before
 //   70000 x 1152   82.1 / 74.8   70.7 / 70.6   73.1 / 75.0
 //   50000 x 1664   77.1 / 75.0   74.4 / 75.0   73.9 / 76.6
