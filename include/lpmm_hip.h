@@ -174,7 +174,7 @@ int lpmm_dequant_group(const uint8_t *codes, const float *max1, const float *qma
 /* Rank-1 statistics of a row-major R x C tensor: rowmax[r] = max_c |x|, colmax[c] = max_r |x|.
  * Replaces get_sm3_statistics / _max_reduce_except_dim (lpmm/functional.py:512-531).
  * colmax is accumulated with atomics on the bit patterns of non-negative floats and is
- * cleared by the call itself. */
+ * cleared by the call itself.  LPMM_ERR_SIZE, with nothing written, for more than 64 * 65535 rows. */
 int lpmm_rank1_stats(const float *x, int64_t rows, int64_t cols, float *rowmax, float *colmax,
                      void *stream);
 
