@@ -131,6 +131,29 @@ def build(q):
     return entries
 
 
+def build_half(q):
+    """256 entries (base, slope) for values that are halfs, indexed by the upper byte of their bits -- sign, exponent and two
+    mantissa bits, the values of a bucket sharing at most two codes: code = (base + slope * bits as a signed 16-bit number) >> 16,
+    whose carry or borrow is the comparison with the midpoint.  For every half but signalling NaNs (quiet ones: 15)."""
+    mids = midpoints(q)
+    entries = []
+    for b in range(256):
+        patterns = np.arange(b << 8, (b + 1) << 8, dtype=np.uint16)
+        values = patterns.view(np.float16).astype(np.float32)
+        codes = [15 if v != v else code_of(mids, v) for v in values]
+        le = codes[0]
+        thr = int(patterns[max(i for i, c in enumerate(codes) if c == le)]) if b != 0xFC else 0xFCFF
+        if b < 0x80:
+            base, slope = (le << 16) + 0xFFFF - thr, 1
+        else:
+            base, slope = (le << 16) + thr - 0x10000, -1
+        for x, c in zip(patterns, codes):
+            signed = int(x) - (0x10000 if x >= 0x8000 else 0)
+            assert (base + slope * signed) >> 16 == c or (b == 0xFC and x > 0xFC00), (hex(x), c)
+        entries.append((base & 0xFFFFFFFF, slope & 0xFFFFFFFF))
+    return entries
+
+
 COMPACT_LO, COMPACT_HI = 24, 63  # magnitude bytes kept in the stored table; the others repeat these two
 
 
@@ -172,6 +195,13 @@ def main():
     out.write("static constexpr uint32_t kEncTableM[%d][4] = {\n" % len(entries))
     for thr, cle, cgt in entries:
         out.write("    {0x%08xu, %du, %du, 0u},\n" % (thr, cle, cgt))
+    out.write("};\n")
+    out.write("// The same for values that are halfs: entry {base, slope} of the upper byte of a half's bits;\n")
+    out.write("// code = (base + slope * bits as a signed 16-bit number) >> 16, for every half but signalling NaNs (quiet ones: 15).\n")
+    entries = build_half(qm)
+    out.write("static constexpr uint32_t kEncHalfM[%d][2] = {\n" % len(entries))
+    for i in range(0, len(entries), 4):
+        out.write("    %s,\n" % ", ".join("{0x%08xu, 0x%08xu}" % e for e in entries[i:i + 4]))
     out.write("};\n")
 
 

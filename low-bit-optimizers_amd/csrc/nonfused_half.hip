@@ -18,12 +18,14 @@
 // float images of the half values in a float work array (a maximum of half values is a half value);
 // a last small kernel writes them out as halfs.
 //
-// Both passes are bound by their arithmetic (eleven roundings per element in the first), so what counts is
-// instructions per element.  Halfs stay in pairs, roundings are packed, products read halfs directly (below),
-// maxima over a lane's columns stay in registers through its passes instead of going to LDS one by one,
-// and addresses advance by one addition each.  Four decoder layers of width 4096 (8.1e8 values), update +
-// second pass: 1603 + 779 us (78 and 38 issue slots per element) -> 1240 + 498 us; 970 + 390 us would be the
-// memory system's.  Six waves per SIMD: with five the update takes 1295 us, with seven it spills.
+// Arithmetic bounds the one pass and the update (eleven roundings per element), so what counts is
+// instructions per element.  Halfs stay in pairs, roundings are packed, products read halfs directly (lpmm_half.hpp), two codes
+// are decoded by one read and the normalised halfs encoded as halfs, maxima over a lane's columns stay in registers through its
+// passes instead of going to LDS one by one, and addresses advance by one addition each.  Kernels of the usual constants (USUAL)
+// have no branch in the chain.  VALU instructions an element, before and after the decoding, encoding and roots of halfs: update 48 -> 37,
+// second pass 19 -> 15.  Four decoder layers of width 4096 (8.1e8 values), a step: 1737 -> 1570 us (the memory system's: 1360);
+// the one pass on a LLaMA-7B-shaped set (6.7e9 values) 13.4 -> 11.3 ms a step.  Six waves per SIMD for the update: within 1 % of four,
+// five and seven.
 #include "lpmm_half.hpp"
 
 namespace lpmm {
@@ -85,12 +87,13 @@ __device__ __forceinline__ void store_codes_guarded(uint8_t *codes, int64_t gbas
 // ops: codes and scales without padding, the map entry rounded to half before it meets the scale
 // ((T)qmap[idx] * scale, a product of halfs), moments and parameter rounded to half where the kernel
 // assigns them to T, everything else in float -- the normalised values included.
-template <bool FUSED>
+// USUAL: half_elts8.
+template <bool FUSED, bool USUAL>
 __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH args, const Hyper fh,
                                                                  const float *__restrict__ qmap_m,
                                                                  const float *__restrict__ qmap_v)
 {
-    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    __shared__ __align__(16) uint32_t lds[(FUSED ? kLdsBytes : kHalfLdsBytes) / 4];
     const int lane = threadIdx.x & (kWave - 1);
     const bool started = lane + 1 < kHMax && args.tile_start[lane + 1] <= blockIdx.x;
     const int lo = __popcll(__ballot(started));
@@ -110,7 +113,12 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
     h16 *pp = t.p + gbase + lane16 * 4;
     uint16_t *mcp = reinterpret_cast<uint16_t *>(t.mc + (gbase >> 1)) + lane16;
     uint16_t *vcp = reinterpret_cast<uint16_t *>(t.vc + (gbase >> 1)) + lane16;
-    const LdsFill fill = lds_fill_load(qmap_m, qmap_v);
+    LdsFill fill;
+    HalfLdsFill half_fill;
+    if constexpr (FUSED)
+        fill = lds_fill_load(qmap_m, qmap_v);
+    else
+        half_fill = half_lds_load(qmap_m, qmap_v);
     v2h p2[kPairs], g2[kPairs];
     uint32_t wm = 0, wv = 0;
     float sm = 0.0f, sv = 0.0f;
@@ -139,7 +147,10 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
         sm = (float)t.ms[grp];
         sv = (float)t.vs[grp];
     }
-    lds_fill_store(lds, fill);
+    if constexpr (FUSED)
+        lds_fill_store(lds, fill);
+    else
+        half_lds_store(lds, half_fill);
     const int kind_m = classify_map(qmap_m), kind_v = classify_map(qmap_v);
     lds_barrier();
 
@@ -151,8 +162,8 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
     if (FUSED && !live)
         return;
     if (!live) {
-        const float z[kEltsPerLane] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        const uint32_t zm = encode8_plain(lds, kLdsQ0, kind_m, z), zv = encode8_plain(lds, kLdsQ1, kind_v, z);
+        const v2h z[kPairs] = {};
+        const uint32_t zm = encode8_half(lds, kLdsQ0, kind_m, z), zv = encode8_half(lds, kLdsQ1, kind_v, z);
         store_u16(mcp, zm & 0xFFFFu);
         store_u16(mcp + 16, zm >> 16);
         store_u16(vcp, zv & 0xFFFFu);
@@ -169,10 +180,10 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
     h.neg_step_size = t.neg_step_size;
     h.bc2_sqrt = t.bc2_sqrt;
     h.rbc2_sqrt = t.rbc2_sqrt;
-    const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
     float amax_m = 0.0f, amax_v = 0.0f;
     uint32_t om, ov;
     if constexpr (FUSED) {
+        const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
         float m[kEltsPerLane], v[kEltsPerLane];
 #pragma unroll
         for (int k = 0; k < kEltsPerLane; ++k) {
@@ -194,13 +205,13 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_half_kernel(const MultiH a
         ov = encode8_scaled(lds, kLdsQ1, kind_v, v, amax_v);
     } else {
         const MixConst c = mix_const();
-        v2h m[kPairs], v[kPairs];
+        v2h m[kPairs], v[kPairs], scale[kPairs];
 #pragma unroll
-        for (int j = 0; j < kPairs; ++j) {
-            m[j] = round2(decode_nibble(lds, kLdsQ0, nm, 2 * j) * sm, decode_nibble(lds, kLdsQ0, nm, 2 * j + 1) * sm);
-            v[j] = round2(decode_nibble(lds, kLdsQ1, nv, 2 * j) * sv, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1) * sv);
-        }
-        half_elts8(p2, g2, m, v, h, c);
+        for (int j = 0; j < kPairs; ++j)
+            scale[j] = v2h{(h16)sv, (h16)sv};
+        half_decode_m(lds, wm, sm, m);
+        half_decode_v(lds, kind_v, wv, scale, v, c);
+        half_elts8<false, false, USUAL>(p2, g2, m, v, h, c);
         if (!full) {
             // elements past the end of the tensor: the zero padding of the chain's quantiser
 #pragma unroll
@@ -348,20 +359,11 @@ __device__ __forceinline__ float max_bits(float a, float b)
     return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
 }
 
-// The second pass's part of lds_fill: the second moment's map, and the first moment's encode table only where
-// the caller's map is that one.
-__device__ __forceinline__ void lds_fill_v(uint32_t *lds, int kind_v, const float *__restrict__ qmap_v)
-{
-    if (kind_v == kMapStdM)
-        lds_fill(lds, qmap_v, qmap_v);
-    else if (threadIdx.x < 16)
-        lds[kLdsQ1 / 4 + threadIdx.x] = __float_as_uint(qmap_v[threadIdx.x]);
-}
-
+template <bool USUAL>
 __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                     const float *__restrict__ qmap_v)
 {
-    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    __shared__ __align__(16) uint32_t lds[kHalfLdsBytes / 4];
     __shared__ __align__(16) h16 col_old[kMaxWide * kGroup];
     __shared__ uint32_t colred[kMaxWide * kRedSlotWords];
     __shared__ uint32_t rowred[kRowSlots];
@@ -373,14 +375,14 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
     const Geometry q = geometry(t, tl, drow);
     const int64_t cols = (int64_t)t.col_blocks * kGroup;
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
-    lds_fill(lds, qmap_m, qmap_v);
+    half_lds_fill(lds, qmap_m, qmap_v);
     for (int j = threadIdx.x; j < kMaxWide * kGroup; j += kThreads)
         col_old[j] = (j < q.wide * kGroup && tile_c0 + j < cols) ? COL_OLD[tile_c0 + j] : (h16)0.0f;
     for (int j = threadIdx.x; j < kMaxWide * (int)kRedSlotWords; j += kThreads)
         colred[j] = 0u;
     if (threadIdx.x < kRowSlots)
         rowred[threadIdx.x] = 0u;
-    const int kind_m = classify_map(qmap_m);
+    const int kind_m = classify_map(qmap_m), kind_v = classify_map(qmap_v);
     NfHyper h;
     h.decay = args.decay;
     h.w1 = args.w1;
@@ -394,10 +396,10 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
     __syncthreads();
 
     if (tl == 0) {
-        const float z[kEltsPerLane] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        const v2h z[kPairs] = {};
         const int64_t n = t.rows * cols;
         write_padding(t.mc, n, (n + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP,
-                      encode8_plain(lds, kLdsQ0, kind_m, z));
+                      encode8_half(lds, kLdsQ0, kind_m, z));
     }
     const int slot = drow & (q.wide - 1);
     if (q.cg < t.col_blocks && q.row0 < t.rows) {
@@ -405,8 +407,10 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
         v2h co[kPairs], vtop[kPairs];  // the lane's columns: current statistics, maxima over its passes
         pairs_of(cop[0], cop[16], co);
 #pragma unroll
-        for (int j = 0; j < kPairs; ++j)
+        for (int j = 0; j < kPairs; ++j) {
+            co[j] = rank1_columns(co[j]);
             vtop[j] = v2h{(h16)0.0f, (h16)0.0f};
+        }
         HalfCursor at(t, q, lane16);
 #pragma unroll 1
         for (int it = 0; it < q.passes && at.row < t.rows; ++it, at.advance()) {
@@ -415,18 +419,15 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
             const uint32_t wv = load_u16(at.vc) | (load_u16(at.vc + 16) << 16);
             const float sm = (float)*at.ms;
             const h16 ro = *at.row_old;
-            v2h p2[kPairs], g2[kPairs], m[kPairs], v[kPairs];
+            v2h p2[kPairs], g2[kPairs], m[kPairs], v[kPairs], s[kPairs];
             pairs_of(a0, a1, p2);
             pairs_of(b0, b1, g2);
-            const Nibbles nm = split_nibbles(wm), nv = split_nibbles(wv);
 #pragma unroll
-            for (int j = 0; j < kPairs; ++j) {
-                m[j] = round2(decode_nibble(lds, kLdsQ0, nm, 2 * j) * sm, decode_nibble(lds, kLdsQ0, nm, 2 * j + 1) * sm);
-                const v2h s = rank1_scales(co[j], ro);
-                v[j] = round2(mix_mul(s.x, decode_nibble(lds, kLdsQ1, nv, 2 * j), c),
-                              mix_mul(s.y, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1), c));
-            }
-            half_elts8(p2, g2, m, v, h, c);
+            for (int j = 0; j < kPairs; ++j)
+                s[j] = rank1_scales(co[j], ro);
+            half_decode_m(lds, wm, sm, m);
+            half_decode_v(lds, kind_v, wv, s, v, c);
+            half_elts8<false, false, USUAL>(p2, g2, m, v, h, c);
 #pragma unroll
             for (int j = 0; j < kPairs; ++j)
                 vtop[j] = max2_bits(vtop[j], v[j]);
@@ -460,7 +461,7 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
 __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
                                                                      const float *__restrict__ qmap_v)
 {
-    __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    __shared__ __align__(16) uint32_t lds[kHalfLdsBytes / 4];
     __shared__ __align__(16) h16 col_old[kMaxWide * kGroup];
     __shared__ __align__(16) float col_new[kMaxWide * kGroup], col_rcp[kMaxWide * kGroup];
     __shared__ uint32_t odd_columns;  // does the tile have a column statistic outside the reciprocal's exact range
@@ -473,7 +474,7 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
     const int64_t cols = (int64_t)t.col_blocks * kGroup;
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
     const int kind_v = classify_map(qmap_v);
-    lds_fill_v(lds, kind_v, qmap_v);
+    half_lds_fill(lds, qmap_m, qmap_v);
     if (threadIdx.x == 0)
         odd_columns = 0u;
     __syncthreads();
@@ -493,10 +494,10 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
     __syncthreads();
 
     if (tl == 0) {
-        const float z[kEltsPerLane] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+        const v2h z[kPairs] = {};
         const int64_t n = t.rows * cols;
         write_padding(t.vc, n, (n + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP,
-                      encode8_plain(lds, kLdsQ1, kind_v, z));
+                      encode8_half(lds, kLdsQ1, kind_v, z));
     }
     if (q.cg >= t.col_blocks)
         return;
@@ -505,6 +506,9 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
     v2h co[kPairs];
     float rcn[kEltsPerLane];
     pairs_of(cop[0], cop[16], co);
+#pragma unroll
+    for (int j = 0; j < kPairs; ++j)
+        co[j] = rank1_columns(co[j]);
     unpack8(*reinterpret_cast<const float4 *>(col_rcp + col_off), *reinterpret_cast<const float4 *>(col_rcp + col_off + 64), rcn);
     const bool even = kind_v == kMapStdV && __builtin_amdgcn_readfirstlane(odd_columns) == 0u;
     const uint32_t code_dword = code_dword_of_lane(lane16), code_sel = code_swap_selector(lane16);
@@ -521,17 +525,15 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
         const uint32_t wv = swap_code_halves(load_u32(vcp), code_sel);
         const h16 ro = *row_old;
         const float rn = *row_new;
-        v2h g2[kPairs], v[kPairs];
+        v2h g2[kPairs], v[kPairs], s[kPairs], x[kPairs];
         pairs_of(b0, b1, g2);
-        const Nibbles nv = split_nibbles(wv);
 #pragma unroll
-        for (int j = 0; j < kPairs; ++j) {
-            const v2h s = rank1_scales(co[j], ro);
-            v[j] = round2(mix_mul(s.x, decode_nibble(lds, kLdsQ1, nv, 2 * j), c),
-                          mix_mul(s.y, decode_nibble(lds, kLdsQ1, nv, 2 * j + 1), c));
+        for (int j = 0; j < kPairs; ++j)
+            s[j] = rank1_scales(co[j], ro);
+        half_decode_v(lds, kind_v, wv, s, v, c);
+#pragma unroll
+        for (int j = 0; j < kPairs; ++j)
             v[j] = half_second_moment(v[j], g2[j], h, c);
-        }
-        float x[kEltsPerLane];
         uint32_t ov;
         // every scale is a maximum over the values it divides: where all of the wave's scales lie in the
         // range in which the reciprocal is exact, one product gives the quotient as a half, and the reciprocal
@@ -539,22 +541,22 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
         if (even && __all(rc_safe(rn))) {
             const float rcr = rcp_exact(rn);
 #pragma unroll
-            for (int j = 0; j < kPairs; ++j) {
-                const v2h qt = half_quotients(v[j], max_bits(rcn[2 * j], rcr), max_bits(rcn[2 * j + 1], rcr), c);
-                // quotients in [0, 1]: the closed form of the standard map (encode8_std_v)
-                x[2 * j] = (float)qt.x;
-                x[2 * j + 1] = (float)qt.y;
-            }
-            ov = encode8_std_v(x);
+            for (int j = 0; j < kPairs; ++j)
+                x[j] = half_quotients(v[j], max_bits(rcn[2 * j], rcr), max_bits(rcn[2 * j + 1], rcr), c);
+            ov = encode8_half_v(x);  // quotients in [0, 1]
         } else {
 #pragma unroll
-            for (int k = 0; k < kEltsPerLane; ++k) {
-                v2h pair = v[k >> 1];
+            for (int j = 0; j < kPairs; ++j) {
+                v2h pair = v[j];
                 asm volatile("" : "+v"(pair));  // what only this branch needs stays in it
-                const float cn = col_new[col_off + (k & 3) + (k >> 2) * 64];
-                x[k] = rh((float)pair[k & 1] / ((cn < rn) ? cn : rn));
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int k = 2 * j + i;
+                    const float cn = col_new[col_off + (k & 3) + (k >> 2) * 64];
+                    x[j][i] = (h16)rh((float)pair[i] / ((cn < rn) ? cn : rn));
+                }
             }
-            ov = encode8_plain(lds, kLdsQ1, kind_v, x);
+            ov = encode8_half(lds, kLdsQ1, kind_v, x);
         }
         store_u32(vcp, swap_code_halves(ov, code_sel));
     }
@@ -562,7 +564,8 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_requant_half_kernel(const M
 
 void launch_rank1_half(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream)
 {
-    hipLaunchKernelGGL(rank1_update_half_kernel, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
+    const auto update = half_near(l.update.w1) && half_eps_positive(l.update.eps) ? rank1_update_half_kernel<true> : rank1_update_half_kernel<false>;
+    hipLaunchKernelGGL(update, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
     hipLaunchKernelGGL(rank1_requant_half_kernel, dim3(l.requant_tiles), dim3(kThreads), 0, stream, l.requant, qmap_m, qmap_v);
 }
 
@@ -678,8 +681,9 @@ static int half_step_multi(const lpmm_adamw4bit_f16_tensor *tensors, int64_t cou
             continue;
         for (int j = k + 1; j <= kHMax; ++j)
             args.tile_start[j] = (uint32_t)tiles;
-        hipLaunchKernelGGL(adamw4bit_half_kernel<FUSED>, dim3((uint32_t)tiles), dim3(kThreads), 0, (hipStream_t)stream,
-                           args, fh, qmap_m, qmap_v);
+        const auto kernel = !FUSED && half_near(c.w1) && half_eps_positive(c.eps) ? adamw4bit_half_kernel<FUSED, !FUSED>
+                                                                                  : adamw4bit_half_kernel<FUSED, false>;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)tiles), dim3(kThreads), 0, (hipStream_t)stream, args, fh, qmap_m, qmap_v);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;

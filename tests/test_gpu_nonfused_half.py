@@ -374,3 +374,41 @@ def test_half_quotient_of_every_pair_of_significands(oracle, qmaps):
     _one_step(nat, t, g, 1, qmaps, 0.0, 0.999, 1e-2, 0.01, 1e-3)
     oracle.nonfused_step_f16(t.host_p, g, t.state, *qmaps, 1e-2, 0.0, 0.999, 1e-3, 0.01)
     t.check("every pair of significands")
+
+
+def _two_pass_step(nat, t, g, step, maps, lr, beta1, beta2, eps, wd):
+    dqm, dqv = (to_dev(q) for q in maps)
+    table = np.array([t.record(g, step)], dtype=nat.NONFUSED_RANK1_F16_TENSOR)
+    st = nat.lib().lpmm_nonfused_adamw4bit_rank1_f16_step_multi(table.ctypes.data, 1, dqm.data_ptr(), dqv.data_ptr(), beta1, beta2,
+                                                                lr, wd, eps, nat.current_stream(torch.device("cuda:0")))
+    assert st == 0
+    torch.cuda.synchronize()
+    t.launched()
+
+
+@pytest.mark.parametrize("maps", ["swapped", "moved"])
+def test_half_steps_with_other_maps(oracle, qmaps, maps):
+    """Maps that the closed forms and tables do not serve, or not in this place, in one and in two passes; with a weight of 0.7 in
+    the first step's lerp, and groups whose scale is zero."""
+    nat = _native()
+    rng = np.random.default_rng(73)
+    qm, qv = qmaps
+    if maps == "swapped":
+        qm, qv = qv, qm
+    else:  # one value of either differs from the standard map's
+        qm, qv = qm.copy(), qv.copy()
+        qm[9] *= np.float32(1.25)
+        qv[3] *= np.float32(1.0625)
+    flat, matrix = _Flat(oracle, 5000, rng), _Matrix(oracle, 150, 384, rng)
+    for step, beta1 in ((1, 0.3), (2, 0.9)):
+        hyper = (beta1, 0.99, 1e-2, 0.01, 1e-3)
+        g = (rng.standard_normal(flat.n) * 0.3).astype(f16)
+        g[128:384] = 0
+        _one_step(nat, flat, g, step, (qm, qv), *hyper)
+        oracle.nonfused_step_f16(flat.host_p, g, flat.state, qm, qv, hyper[2], beta1, hyper[1], hyper[4], hyper[3])
+        flat.check(f"{maps} maps, one pass, step {step}")
+        g = (rng.standard_normal((150, 384)) * 0.3).astype(f16)
+        g[9] = 0
+        _two_pass_step(nat, matrix, g, step, (qm, qv), hyper[2], beta1, hyper[1], hyper[4], hyper[3])
+        oracle.nonfused_step_f16(matrix.host_p, g, matrix.state, qm, qv, hyper[2], beta1, hyper[1], hyper[4], hyper[3])
+        matrix.check(f"{maps} maps, two passes, step {step}")

@@ -6,6 +6,7 @@ maps as obtained from the reference's own construction recipe run with PyTorch o
 (c) brute force around every map point and midpoint."""
 import json
 import os
+import re
 import subprocess
 import sys
 
@@ -116,3 +117,23 @@ def test_fast_encoders_exhaustive(tmp_path):
     out = subprocess.check_output([exe], text=True)
     assert "bad_m 0 bad_v 0" in out, out
     assert "checked 4278190082" in out, out
+
+
+def test_half_encoders_on_every_half(oracle):
+    """The bucket table and the closed form that give the codes of normalised halfs (lpmm_half.hpp: encode8_half_m, encode8_half_v),
+    restated, against the search on every half (the closed form: on those from -1 to 1)."""
+    txt = open(os.path.join(CSRC, "std_tables.inc")).read()
+    body = txt.split("kEncHalfM[256][2]")[1].split("};", 1)[0]
+    words = np.array([int(w, 16) for w in re.findall(r"0x[0-9a-f]{8}", body)], dtype=np.uint32).astype(np.int32).astype(np.int64)
+    entries = words.reshape(256, 2)
+    bits16 = np.arange(1 << 16, dtype=np.uint16)
+    x = bits16.view(np.float16)
+    e = entries[bits16 >> 8]
+    got = (e[:, 0] + e[:, 1] * bits16.view(np.int16).astype(np.int64)) >> 16
+    want = oracle.qmapping(oracle.qmap_m(), x.astype(np.float32))
+    signalling = np.isnan(x) & ((bits16 & 0x200) == 0)  # arithmetic gives none
+    assert np.array_equal(got[~signalling], want[~signalling])
+    x = x[np.abs(x.astype(np.float32)) <= 1]
+    r = np.maximum((x.astype(np.float64) * 15.9921875 + 1023).astype(np.float16), np.float16(1024))  # one rounding: an fma
+    want = oracle.qmapping(oracle.qmap_v(), x.astype(np.float32))
+    assert np.array_equal(r.view(np.uint16) - 0x6400, want)
