@@ -412,3 +412,16 @@ def test_half_steps_with_other_maps(oracle, qmaps, maps):
         _two_pass_step(nat, matrix, g, step, (qm, qv), hyper[2], beta1, hyper[1], hyper[4], hyper[3])
         oracle.nonfused_step_f16(matrix.host_p, g, matrix.state, qm, qv, hyper[2], beta1, hyper[1], hyper[4], hyper[3])
         matrix.check(f"{maps} maps, two passes, step {step}")
+
+
+@pytest.mark.parametrize("rows, cols", [(4097, 128), (6000, 1152), (13001, 1152), (40001, 128)])
+def test_two_pass_half_step_tile_rows(oracle, qmaps, rows, cols):
+    """Tiles of 16, 32, 64 and 128 rows in the first pass (by the launch's values and a column's row blocks), of 16 to 64 in the second."""
+    nat = _native()
+    rng = np.random.default_rng(74)
+    t = _Matrix(oracle, rows, cols, rng)
+    for step in (1, 2):
+        g = (rng.standard_normal((rows, cols)).astype(np.float32) * 0.3).astype(f16)
+        _two_pass_step(nat, t, g, step, qmaps, 1e-2, 0.9, 0.999, 1e-3, 0.01)
+        oracle.nonfused_step_f16(t.host_p, g, t.state, *qmaps, 1e-2, 0.9, 0.999, 1e-3, 0.01)
+    t.check(f"{rows} x {cols}")
