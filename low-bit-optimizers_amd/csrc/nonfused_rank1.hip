@@ -553,7 +553,8 @@ constexpr uint64_t kSpreadBelow = 1024;
 //     50, 59 (1235 workgroups, a fifth more than are resident together), 52; ten of 1001 x 1003 54, 58, 51; but 2001 x 3001 40, 34, 36.
 // The float16 update is bound by its arithmetic, so that large launches take tall tiles, which spread a tile's set-up; small ones
 // leave the chip idle with them.  Update / second pass with tiles of 128, 64, 32, 16 rows: 20 of 4096 x 11008 (902M values) 1323 / 495, 1333 /
-// 518, 1391 / 509, 1507 / 743; 8 of 4096 x 4096 233 / 91, 225 / 90; 4 of them 102 / 47, 97 / 42, 103 / 43; one 35.8 / 18.7, 31.1 / 14.0,
+// 518, 1391 / 509, 1507 / 743; 8 of 4096 x 4096 233 / 91, 225 / 90; 4 of them 102 / 47, 97 / 42, 103 / 43 (128 rows all the same:
+// from 26M values on launches keep the groups of kSpreadBelow); one 35.8 / 18.7, 31.1 / 14.0,
 // 30.2 / 14.6, 32.6 / 16.4; 24 of 512 x 2048 45.8 / 21.9, 41.5 / 18.3, 42.7 / 19.5; 32 of 256 x 2304 43.6 / 20.7, 35.8 / 15.9, 33.6 / 16.2,
 // 36.6 / 18.4; 8 of 1024 x 1024 28.7 / 16.4, 21.0 / 11.0, 19.0 / 8.9, 19.6 / 10.2; 24 of 512 x 512 27.9 / 15.5, 20.5 / 11.0, 16.5 /
 // 8.3, 15.7 / 7.9; update of 39877 x 128 22.6, 29.0 (a column's row blocks).  Any column count likewise: 2001 x 3001 49.5 / 82, 29.7, 30.2, 30.3 / 35.8;
@@ -561,7 +562,7 @@ constexpr uint64_t kSpreadBelow = 1024;
 static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, uint32_t col_blocks, bool odd_cols)
 {
     if (l.half_io && requant)
-        return l.values < 6.5e6 ? kPolicyRows / 4 : l.values < 14e6 ? kPolicyRows / 2 : l.values < 100e6 ? kPolicyRows : kPolicyRowsHalf;
+        return l.values < 6.5e6 ? kPolicyRows / 4 : l.values < 14e6 ? kPolicyRows / 2 : l.values < 26e6 ? kPolicyRows : kPolicyRowsHalf;
     const bool single = choose_lg_wide(col_blocks) == 0;  // tiles of one column group
     if (requant && odd_cols && !l.bits)
         return l.values >= (single ? 3e6 : 4e6) && l.values < 9e6 ? kPolicyRows / 2 : kPolicyRows / 4;
@@ -571,7 +572,7 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     if (l.half_io)
         tile_rows = l.values < 6.5e6 && rows <= 256 * (int64_t)(kPolicyRows / 4)  ? kPolicyRows / 4
                     : l.values < 25e6 && rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2
-                    : l.values < 100e6                                            ? kPolicyRows
+                    : l.values < 26e6                                             ? kPolicyRows
                                                                                   : kPolicyRowsHalf;
     else if (l.values >= 64e6)
         tile_rows = l.m32 ? kPolicyRows / 4 : fold || l.bits ? kPolicyRows : kPolicyRows / 2;
