@@ -365,6 +365,16 @@ int lpmm_nonfused_adamw4bit_rank1_pass_multi(const lpmm_nonfused_rank1_tensor *t
                                              double beta2, double lr, double weight_decay, double eps,
                                              int pass, void *stream);
 
+/* Both passes on tensors of more than two dimensions, and what lies between them, launch by launch: pass 1 on up to 32 tensors,
+ * lpmm_rank1_small_fold_scale_multi on their vectors, pass 2, so that the second pass of a launch finds in the cache what its first
+ * has read.  tensors: the records of pass 1; folds[i]: the vector of tensors[i], x its v_colmax_next (cols values), scale what
+ * pass 2 divides by (16-byte aligned, another array than v_colmax); ndim 0: a matrix, whose column maxima are its statistics. */
+int lpmm_nonfused_adamw4bit_rank1_nd_step_multi(const lpmm_nonfused_rank1_tensor *tensors,
+                                                const lpmm_rank1_small_vector *folds, int64_t count,
+                                                const float *qmap_m, const float *qmap_v, double beta1,
+                                                double beta2, double lr, double weight_decay, double eps,
+                                                void *stream);
+
 /* The non-fused step on float16 parameters (4-bit states, first moment 'group' gp_sz 128).  With
  * fused=False the reference's op sequence runs PyTorch's half kernels: every op computes in float
  * and rounds its result to half once, Python scalars enter as floats

@@ -39,15 +39,17 @@ namespace lpmm {
 
 // Zeroes the arrays that the first pass merges maxima into: the next statistics, and the next scales of first-moment
 // groups that are wider than 128 values or straddle rows.  Ranges of all tensors of a call in one launch (5 us each on an
-// otherwise idle stream), neighbours in memory joined.
-constexpr int kClearMax = 240;
+// otherwise idle stream), neighbours in memory joined.  Two sizes of arguments: the host copies them whole.
+constexpr int kClearMax = 480, kClearFew = 64;
+template <int N>
 struct ClearRanges {
-    float *at[kClearMax];
-    int64_t n[kClearMax];
+    float *at[N];
+    int64_t n[N];
 };
-static_assert(sizeof(ClearRanges) <= 4096, "kernel arguments exceed 4 KB");
+static_assert(sizeof(ClearRanges<kClearMax>) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
 
-__global__ __launch_bounds__(kThreads) void rank1_clear_kernel(const ClearRanges ranges)
+template <int N>
+__global__ __launch_bounds__(kThreads) void rank1_clear_kernel(const ClearRanges<N> ranges)
 {
     float *const at = ranges.at[blockIdx.y];
     const int64_t n = ranges.n[blockIdx.y];
@@ -705,11 +707,13 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
 
 // Validation, batching into launches of at most kR1Max tensors, and the launches.
 // m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
+// folds: a record per tensor, of ndim 0 where the tensor is a matrix (lpmm_nonfused_adamw4bit_rank1_nd_step_multi).
 template <int MODE, class Record>
 static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
                             uint32_t m_lg, double beta1, double beta2, double lr, double weight_decay, double eps,
                             void *stream, int bits_m = 4, int bits_v = 4, const void *table_m = nullptr,
-                            const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr)
+                            const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr,
+                            const lpmm_rank1_small_vector *folds = nullptr)
 {
     // passes: 1 = the first pass alone (with the clearing of the next statistics), 2 = the second alone,
     // 3 = both; one at a time only where the launches below are this file's own, or general ones: any column count,
@@ -738,14 +742,20 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
 
     hipStream_t s = (hipStream_t)stream;
     if (passes & 1) {
-        ClearRanges ranges;
+        ClearRanges<kClearMax> ranges;
         int n = 0;
         int64_t longest = 0;
         const auto launch_clear = [&] {
             const int64_t blocks = (longest + kThreads - 1) / kThreads;
-            if (n != 0)
-                hipLaunchKernelGGL(rank1_clear_kernel, dim3((uint32_t)(blocks > 64 ? 64 : blocks), (uint32_t)n), dim3(kThreads), 0,
-                                   s, ranges);
+            const dim3 grid((uint32_t)(blocks > 64 ? 64 : blocks), (uint32_t)n);
+            if (n > kClearFew) {
+                hipLaunchKernelGGL(rank1_clear_kernel<kClearMax>, grid, dim3(kThreads), 0, s, ranges);
+            } else if (n != 0) {
+                ClearRanges<kClearFew> few;
+                memcpy(few.at, ranges.at, sizeof few.at);
+                memcpy(few.n, ranges.n, sizeof few.n);
+                hipLaunchKernelGGL(rank1_clear_kernel<kClearFew>, grid, dim3(kThreads), 0, s, few);
+            }
             n = 0;
             longest = 0;
         };
@@ -817,6 +827,9 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         uint64_t tiles = 0, tiles2 = 0;
         uint32_t start2[kR1Max + 1] = {0};
         TileShape shape2[kR1Max];
+        float *scale2[kR1Max];  // the column statistics of the second pass
+        const lpmm_rank1_small_vector *between[kR1Max];
+        int betweens = 0;
         bool folded = false;  // does a tensor of this launch have folded rows
         args.tile_start[0] = 0;
         while (i < count && k < kR1Max) {
@@ -856,6 +869,11 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             tiles += nt;
             tiles2 += nt2;
             folded = folded || m.fold;
+            scale2[k] = d.col_new;
+            if (folds != nullptr && folds[i].ndim != 0) {
+                scale2[k] = folds[i].scale;
+                between[betweens++] = folds + i;
+            }
             args.tile_start[++k] = (uint32_t)tiles;
             start2[k] = (uint32_t)tiles2;
             ++i;
@@ -871,8 +889,10 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             start2[j] = (uint32_t)tiles2;
         }
         l.requant = args;
-        for (int j = 0; j < k; ++j)
+        for (int j = 0; j < k; ++j) {
             l.requant.t[j].tile = shape2[j];
+            l.requant.t[j].col_new = scale2[j];
+        }
         memcpy(l.requant.tile_start, start2, sizeof start2);
         l.update_tiles = (uint32_t)tiles;
         l.requant_tiles = (uint32_t)tiles2;
@@ -888,6 +908,12 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         } else if (bits_m != 4) {
             launch_rank1_bits(l, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
                               static_cast<const uint32_t *>(table_v), s);
+        } else if (betweens != 0) {
+            launch_rank1<MODE>(l, folded, qmap_m, qmap_v, 1, s);
+            const int st = launch_small_vectors(between, betweens, s);
+            if (st != LPMM_OK)
+                return st;
+            launch_rank1<MODE>(l, folded, qmap_m, qmap_v, 2, s);
         } else {
             launch_rank1<MODE>(l, MODE == kMCodes128 && folded, qmap_m, qmap_v, passes, s);
         }
@@ -923,6 +949,37 @@ extern "C" int lpmm_nonfused_adamw4bit_rank1_pass_multi(const lpmm_nonfused_rank
         return LPMM_ERR_ARG;
     return rank1_step_multi<kMCodes128>(tensors, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream,
                                         4, 4, nullptr, nullptr, pass);
+}
+
+extern "C" int lpmm_nonfused_adamw4bit_rank1_nd_step_multi(const lpmm_nonfused_rank1_tensor *tensors,
+                                                           const lpmm_rank1_small_vector *folds, int64_t count, const float *qmap_m,
+                                                           const float *qmap_v, double beta1, double beta2, double lr,
+                                                           double weight_decay, double eps, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    LPMM_REQUIRE_PTR(tensors);
+    LPMM_REQUIRE_PTR(folds);
+    for (int64_t i = 0; i < count; ++i) {
+        const lpmm_rank1_small_vector &v = folds[i];
+        if (v.ndim == 0 || tensors[i].rows == 0 || tensors[i].cols == 0)
+            continue;
+        const int bad = check_small_vectors(&v, 1);
+        if (bad != LPMM_OK)
+            return bad;
+        int64_t n = 1;
+        for (int k = 0; k < v.ndim; ++k)
+            n *= v.shape[k];
+        if (n != tensors[i].cols)
+            return LPMM_ERR_SIZE;
+        if (v.x != tensors[i].v_colmax_next || v.scale == v.x || v.scale == tensors[i].v_colmax)
+            return LPMM_ERR_ARG;
+        LPMM_REQUIRE_ALIGN(v.scale, 16);
+    }
+    return rank1_step_multi<kMCodes128>(tensors, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, 4, 4, nullptr,
+                                        nullptr, 3, false, nullptr, folds);
 }
 
 extern "C" int lpmm_nonfused_adamw_v4bit_rank1_step_multi(const lpmm_rank1_v4bit_tensor *tensors, int64_t count,

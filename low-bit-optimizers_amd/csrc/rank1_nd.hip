@@ -22,7 +22,7 @@
 //     leading dimensions' statistics.  With that array as `rowmax` and stat_k as `colmax` the
 //     2-D quantise / dequantise kernels (any code width) serve the N-D tensor unchanged:
 //     min(min(leading statistics), stat_k) is the reference's scale.
-#include "lpmm_common.hpp"
+#include "rank1_tiles.hpp"
 
 namespace lpmm {
 
@@ -227,15 +227,13 @@ static_assert(sizeof(NdSmallArgs) <= 4096, "kernel arguments exceed 4 KB");
 // One workgroup a tensor, so what counts is the chain of a thread: 1024 threads, so that a few thousand entries are a few
 // rounds; the divisions by the dimensions in registers (the loops over them are unrolled, their trip count would put the
 // bases into scratch memory); and the statistics of a dimension of a few entries (the taps of a convolution, a dimension of
-// one) in kNdCopies copies, since the LDS takes atomics on one address one lane at a time.  Up to 32 tensors of a wide
-// ResNet-152 (256 to 4608 entries): 23.5 -> 11.3 us a launch.
+// one) in kNdCopies copies, since the LDS takes atomics on one address one lane at a time.
 constexpr int kNdFoldThreads = 1024;
 constexpr uint32_t kNdFew = 16, kNdCopies = 32;
 
-__global__ __launch_bounds__(kNdFoldThreads) void rank1_small_fold_scale_kernel(const NdSmallArgs args)
+// any dimensions
+__device__ void fold_small(const NdSmall &t, uint32_t *slots)
 {
-    __shared__ uint32_t slots[kNdSmallSlots + (kNdMax - 1) * kNdFew * kNdCopies];
-    const NdSmall &t = args.t[blockIdx.x];
     const int ndim = (int)t.ndim;
     const uint32_t tid = threadIdx.x, copy = tid & (kNdCopies - 1);
     uint32_t base[kNdMax - 1], total = 0;
@@ -296,6 +294,102 @@ __global__ __launch_bounds__(kNdFoldThreads) void rank1_small_fold_scale_kernel(
         t.scale[e] = scale;
     }
 }
+
+// A first dimension of any length over at most TAPS values (convolution weights: channels over the taps of the kernel, or over one):
+// a thread takes whole channels, their maxima need no atomics and no value a division.  TAPS loads are in flight per
+// channel whatever the tensor has; the last is read again instead of a branch.
+template <uint32_t TAPS>
+__device__ __forceinline__ void fold_taps(const NdSmall &t, uint32_t taps, uint32_t *slots)
+{
+    uint32_t *const channel = slots, *const copies = slots + kNdSmallSlots;  // copies: [tap][kNdCopies]
+    uint32_t *const stat = copies + TAPS * kNdCopies;                        // [later dimension][kNdFew]
+    const uint32_t tid = threadIdx.x, copy = tid & (kNdCopies - 1), channels = t.dim[0];
+    const int ndim = (int)t.ndim;
+    for (uint32_t j = tid; j < TAPS * kNdCopies + (kNdMax - 2) * kNdFew; j += kNdFoldThreads)
+        copies[j] = 0u;
+    uint32_t top[TAPS];
+#pragma unroll
+    for (uint32_t k = 0; k < TAPS; ++k)
+        top[k] = 0u;
+    for (uint32_t c = tid; c < channels; c += kNdFoldThreads) {
+        uint32_t v[TAPS], most = 0u;
+#pragma unroll
+        for (uint32_t k = 0; k < TAPS; ++k)
+            v[k] = abs_bits(t.x[c * taps + (k < taps ? k : taps - 1u)]);
+#pragma unroll
+        for (uint32_t k = 0; k < TAPS; ++k) {
+            most = v[k] > most ? v[k] : most;
+            top[k] = v[k] > top[k] ? v[k] : top[k];
+        }
+        channel[c] = most;
+        t.stat[0][c] = __uint_as_float(most);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < TAPS; ++k)
+        atomicMax(copies + k * kNdCopies + copy, top[k]);
+    __syncthreads();
+    // a thread per tap: its maximum, then the later dimensions' statistics it belongs to
+    uint32_t index[kNdMax - 2];
+    if (tid < taps) {
+        uint32_t v = 0u, rem = tid;
+        for (uint32_t c = 0; c < kNdCopies; ++c) {
+            const uint32_t x = copies[tid * kNdCopies + ((c + tid) & (kNdCopies - 1))];
+            v = x > v ? x : v;
+        }
+#pragma unroll
+        for (int i = kNdMax - 2; i >= 1; --i) {
+            if (i >= ndim)
+                continue;
+            const uint32_t q = rem / t.dim[i];
+            index[i - 1] = rem - q * t.dim[i];
+            rem = q;
+            atomicMax(stat + (i - 1) * kNdFew + index[i - 1], v);
+        }
+    }
+    __syncthreads();
+    if (tid < taps) {
+        float scale = 0.0f;
+#pragma unroll
+        for (int i = kNdMax - 2; i >= 1; --i) {
+            if (i >= ndim)
+                continue;
+            const float s = __uint_as_float(stat[(i - 1) * kNdFew + index[i - 1]]);
+            t.stat[i][index[i - 1]] = s;  // taps that share an entry write the same
+            scale = i == ndim - 1 ? s : min_nan(scale, s);
+        }
+        copies[tid] = __float_as_uint(scale);
+    }
+    __syncthreads();
+    float least[TAPS];
+#pragma unroll
+    for (uint32_t k = 0; k < TAPS; ++k)
+        least[k] = __uint_as_float(copies[k < taps ? k : taps - 1u]);
+    for (uint32_t c = tid; c < channels; c += kNdFoldThreads) {
+        const float s = __uint_as_float(channel[c]);
+#pragma unroll
+        for (uint32_t k = 0; k < TAPS; ++k)
+            if (k < taps)
+                t.scale[c * taps + k] = ndim == 1 ? s : min_nan(least[k], s);
+    }
+}
+
+__global__ __launch_bounds__(kNdFoldThreads) void rank1_small_fold_scale_kernel(const NdSmallArgs args)
+{
+    __shared__ uint32_t slots[kNdSmallSlots + (kNdMax - 1) * kNdFew * kNdCopies];
+    const NdSmall &t = args.t[blockIdx.x];
+    uint32_t taps = 1;
+#pragma unroll
+    for (int i = 1; i < kNdMax - 1; ++i)
+        taps *= i < (int)t.ndim ? t.dim[i] : 1u;  // fewer than 2^31: checked on the host
+    if (taps == 1)
+        fold_taps<1>(t, taps, slots);
+    else if (taps <= 9)
+        fold_taps<9>(t, taps, slots);
+    else
+        fold_small(t, slots);
+}
+static_assert(9 * kNdCopies + (kNdMax - 2) * kNdFew <= (kNdMax - 1) * kNdFew * kNdCopies && 9 <= kNdFew, "fold_taps fits the LDS");
 
 // shape -> NdDims for the first `ndim` dimensions; false when a size is not positive, the element
 // count overflows or the tile count does not fit a grid
@@ -408,13 +502,8 @@ extern "C" int lpmm_rank1_row_scale_nd(const float *const *stats, int ndim, cons
     return launch_status();
 }
 
-extern "C" int lpmm_rank1_small_fold_scale_multi(const lpmm_rank1_small_vector *vectors, int64_t count, void *stream)
+int lpmm::check_small_vectors(const lpmm_rank1_small_vector *vectors, int64_t count)
 {
-    if (count < 0)
-        return LPMM_ERR_SIZE;
-    if (count == 0)
-        return LPMM_OK;
-    LPMM_REQUIRE_PTR(vectors);
     for (int64_t i = 0; i < count; ++i) {
         const lpmm_rank1_small_vector &v = vectors[i];
         if (v.ndim < 1 || v.ndim > kNdMax - 1)
@@ -435,11 +524,16 @@ extern "C" int lpmm_rank1_small_fold_scale_multi(const lpmm_rank1_small_vector *
         if (slots > kNdSmallSlots)
             return LPMM_ERR_SIZE;
     }
+    return LPMM_OK;
+}
+
+int lpmm::launch_small_vectors(const lpmm_rank1_small_vector *const *vectors, int64_t count, hipStream_t stream)
+{
     for (int64_t i = 0; i < count; i += kNdSmallMax) {
         NdSmallArgs args;
         const int k = (int)(count - i < kNdSmallMax ? count - i : kNdSmallMax);
         for (int j = 0; j < k; ++j) {
-            const lpmm_rank1_small_vector &v = vectors[i + j];
+            const lpmm_rank1_small_vector &v = *vectors[i + j];
             NdSmall &t = args.t[j];
             t.x = v.x;
             t.scale = v.scale;
@@ -452,8 +546,30 @@ extern "C" int lpmm_rank1_small_fold_scale_multi(const lpmm_rank1_small_vector *
             }
             t.n = n;
         }
-        hipLaunchKernelGGL(rank1_small_fold_scale_kernel, dim3((uint32_t)k), dim3(kNdFoldThreads), 0, (hipStream_t)stream, args);
+        hipLaunchKernelGGL(rank1_small_fold_scale_kernel, dim3((uint32_t)k), dim3(kNdFoldThreads), 0, stream, args);
         const int st = launch_status();
+        if (st != LPMM_OK)
+            return st;
+    }
+    return LPMM_OK;
+}
+
+extern "C" int lpmm_rank1_small_fold_scale_multi(const lpmm_rank1_small_vector *vectors, int64_t count, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    LPMM_REQUIRE_PTR(vectors);
+    const int bad = check_small_vectors(vectors, count);
+    if (bad != LPMM_OK)
+        return bad;
+    for (int64_t i = 0; i < count; i += kNdSmallMax) {
+        const lpmm_rank1_small_vector *list[kNdSmallMax];
+        const int64_t k = count - i < kNdSmallMax ? count - i : kNdSmallMax;
+        for (int64_t j = 0; j < k; ++j)
+            list[j] = vectors + i + j;
+        const int st = launch_small_vectors(list, k, (hipStream_t)stream);
         if (st != LPMM_OK)
             return st;
     }

@@ -262,6 +262,9 @@ void launch_rank1_any(const R1Launch &l, const NewCodes &out, const float *qmap_
 // float16 parameters (nonfused_half.hip): p, g, the first moment's scales and the current statistics
 // of the records point at halfs, the next statistics at float work arrays
 void launch_rank1_half(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream);
+// statistics and scale of short vectors (rank1_nd.hip): the checks and the launches of lpmm_rank1_small_fold_scale_multi
+int check_small_vectors(const lpmm_rank1_small_vector *vectors, int64_t count);
+int launch_small_vectors(const lpmm_rank1_small_vector *const *vectors, int64_t count, hipStream_t stream);
 // the records of lpmm_nonfused_adamw_rank1_any_step_multi; float16: the next statistics and scales of the records are
 // float work arrays (rank1_any_half sets them up and writes the halfs out)
 int rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg, const float *qmap_m,

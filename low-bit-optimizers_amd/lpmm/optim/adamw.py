@@ -316,19 +316,20 @@ class AdamW(LowBitOptimizer):
         def code_tables():
             return [code_table(q, md["b"]).data_ptr() for q, md in ((qm, routes.m), (qv, routes.v))]
 
-        if kind in (_native.WALK_ND, _native.WALK_ND_ANY):
+        if kind == _native.WALK_ND:
+            st = lib.lpmm_nonfused_adamw4bit_rank1_nd_step_multi(records, fold, count, qm.data_ptr(), qv_ptr, *hyper, stream)
+            _native.check(st, "non-fused 4-bit AdamW step on tensors of more than two dimensions")
+            plan.commit(k, 0, count)
+            return
+        if kind == _native.WALK_ND_ANY:
             # the kernels for any column count write their codes to new arrays: one launch's worth of them at a time
-            whole = kind == _native.WALK_ND
-            size, chunk = (_native.NONFUSED_RANK1_TENSOR.itemsize, count) if whole else (_native.RANK1_ANY_TENSOR.itemsize, most)
-            for i in range(0, count, chunk):
-                n = min(chunk, count - i)
+            size = _native.RANK1_ANY_TENSOR.itemsize
+            for i in range(0, count, most):
+                n = min(most, count - i)
                 plan.prepare(k, i, n)
                 for pass_no, table in ((1, records + i * size), (2, second + i * size)):
-                    if whole:
-                        st = lib.lpmm_nonfused_adamw4bit_rank1_pass_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, pass_no, stream)
-                    else:
-                        st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, _native.RANK1_CODES4, 128, qm.data_ptr(), 4, None,
-                                                                          qv_ptr, 4, None, *hyper, pass_no, stream)
+                    st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, _native.RANK1_CODES4, 128, qm.data_ptr(), 4, None,
+                                                                      qv_ptr, 4, None, *hyper, pass_no, stream)
                     _native.check(st, f"non-fused 4-bit AdamW step on tensors of more than two dimensions, pass {pass_no}")
                     if pass_no == 1:
                         st = lib.lpmm_rank1_small_fold_scale_multi(fold + i * _native.RANK1_SMALL_VECTOR.itemsize, n, stream)
