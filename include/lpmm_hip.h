@@ -205,6 +205,15 @@ int lpmm_rank1_stats_nd(const float *x, int ndim, const int64_t *shape, float *c
 int lpmm_rank1_row_scale_nd(const float *const *stats, int ndim, const int64_t *shape, float *row_scale,
                             void *stream);
 
+/* A whole rank-1 quantisation of a contiguous tensor of 2..LPMM_RANK1_ND_MAX dimensions in one call: its statistics, of more than two
+ * dimensions the scale of a row (both as above), and the codes (lpmm_quant_rank1, for bits other than 4
+ * lpmm_quant_rank1_bits_table with `table`); and the way back from codes and statistics.  work: NULL for two dimensions, otherwise
+ * device memory for numel / shape[ndim-1] floats. */
+int lpmm_quant_rank1_nd(const float *x, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap, int bits,
+                        const void *table, uint8_t *codes, void *stream);
+int lpmm_dequant_rank1_nd(const uint8_t *codes, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap,
+                          int bits, float *out, void *stream);
+
 /* Statistics and scale of short vectors, many per call (no counterpart in the reference).  For
  * each record: stats[i][j] = max |x| over the elements of the vector x (row-major, shape[0..ndim))
  * whose i-th index is j, written in full, and scale[e] = the minimum of element e's statistics (NaN

@@ -502,6 +502,69 @@ extern "C" int lpmm_rank1_row_scale_nd(const float *const *stats, int ndim, cons
     return launch_status();
 }
 
+// 2-D view of a tensor whose dimensions are the caller's: false where it has none
+static bool rank1_view(int ndim, const int64_t *shape, int64_t *rows, int64_t *cols)
+{
+    int64_t n = 1;
+    for (int i = 0; i < ndim; ++i) {
+        if (shape[i] <= 0 || n > INT64_MAX / shape[i])
+            return false;
+        n *= shape[i];
+    }
+    *cols = shape[ndim - 1];
+    *rows = n / *cols;
+    return true;
+}
+
+extern "C" int lpmm_quant_rank1_nd(const float *x, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap,
+                                   int bits, const void *table, uint8_t *codes, void *stream)
+{
+    if (ndim < 2 || ndim > kNdMax)
+        return LPMM_ERR_ARG;
+    LPMM_REQUIRE_PTR(shape);
+    LPMM_REQUIRE_PTR(stats);
+    int64_t rows, cols;
+    if (!rank1_view(ndim, shape, &rows, &cols))
+        return LPMM_ERR_SIZE;
+    const float *rowmax = stats[0], *colmax = stats[ndim - 1];
+    int st;
+    if (ndim == 2) {
+        st = lpmm_rank1_stats(x, rows, cols, stats[0], stats[1], stream);
+    } else {
+        LPMM_REQUIRE_PTR(work);
+        // long last dimension: the 2-D kernel plus a fold of its row maxima, whose place the scales take
+        st = lpmm_rank1_stats_nd(x, ndim, shape, stats, cols >= 32 ? work : nullptr, stream);
+        if (st == LPMM_OK)
+            st = lpmm_rank1_row_scale_nd(stats, ndim, shape, work, stream);
+        rowmax = work;
+    }
+    if (st != LPMM_OK)
+        return st;
+    return bits == 4 ? lpmm_quant_rank1(x, rows, cols, rowmax, colmax, qmap, codes, stream)
+                     : lpmm_quant_rank1_bits_table(x, rows, cols, rowmax, colmax, qmap, bits, table, codes, stream);
+}
+
+extern "C" int lpmm_dequant_rank1_nd(const uint8_t *codes, int ndim, const int64_t *shape, float *const *stats, float *work,
+                                     const float *qmap, int bits, float *out, void *stream)
+{
+    if (ndim < 2 || ndim > kNdMax)
+        return LPMM_ERR_ARG;
+    LPMM_REQUIRE_PTR(shape);
+    LPMM_REQUIRE_PTR(stats);
+    int64_t rows, cols;
+    if (!rank1_view(ndim, shape, &rows, &cols))
+        return LPMM_ERR_SIZE;
+    const float *rowmax = stats[0], *colmax = stats[ndim - 1];
+    if (ndim > 2) {
+        const int st = lpmm_rank1_row_scale_nd(stats, ndim, shape, work, stream);
+        if (st != LPMM_OK)
+            return st;
+        rowmax = work;
+    }
+    return bits == 4 ? lpmm_dequant_rank1(codes, rowmax, colmax, qmap, rows, cols, out, stream)
+                     : lpmm_dequant_rank1_bits(codes, rowmax, colmax, qmap, bits, rows, cols, out, stream);
+}
+
 int lpmm::check_small_vectors(const lpmm_rank1_small_vector *vectors, int64_t count)
 {
     for (int64_t i = 0; i < count; ++i) {

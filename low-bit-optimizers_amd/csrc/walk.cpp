@@ -1,8 +1,11 @@
 // The host side of a step on a model whose optimizer states exist: one walk over a parameter group's tensors
 // that writes the records of the multi-tensor launches.  In Python the same walk is dozens of attribute and
-// dictionary reads a tensor -- 3 to 15 us a tensor, against 0.4 here, while the kernels take 1 us for a tensor of a
+// dictionary reads a tensor -- 3 to 15 us a tensor, against 0.15 here, while the kernels take 1 us for a tensor of a
 // million values -- and bound every model of small tensors: fifty tensors of a few thousand to a million values
 // 186 -> 43 us a step, the 203 of a wide ResNet-152 1634 -> 1054, GPT-2-XL's 580 1.8 -> 0.23 ms of host time.
+// What counts here is dictionary reads: names compared by address (read), a parameter's hash without its call into Python
+// (hash_of), one allocation for a launch's scratch (prepare): 52 tensors 10.3 -> 7.2 us, and with fewer attribute reads in Python
+// their fused step 31.8 -> 25.1 us, 576 tensors of width 64 on the two-pass route 277 -> 209, 18 float16 matrices 70 -> 49.
 // lpmm/optim/adamw.py and sgd.py keep that walk for what is not served here: first steps, other data types,
 // strided operands, other routes; and for every error.
 //
@@ -43,9 +46,10 @@ struct Names {
         *max_dims, *work, *scale_of, *row, *momentum_buffer, *momentum_buffer_qstate, *dtype;
 } N;
 
-// dict[key] = value, once the launch is on the stream; strong references
+// dict[key] = value, once the launch is on the stream; strong references.  hash: of a key that is a parameter, else -1
 struct Swap {
     PyObject *dict, *key, *value;
+    Py_hash_t hash = -1;
 };
 
 // memory of a record, allocated when its launch is next (prepare): n floats of this step's scratch, or the array that
@@ -117,6 +121,58 @@ PyObject *get(PyObject *dict, PyObject *key)  // borrowed; null where absent (a 
     return dict != nullptr && PyDict_Check(dict) ? PyDict_GetItemWithError(dict, key) : nullptr;
 }
 
+// Values of `count` names in a dictionary of a few entries (borrowed; null where absent): one pass over the entries, whose keys are
+// as a rule these very strings.  Only a dictionary that holds other keys as well, or equal strings that are other objects (from a
+// file), is searched name by name.
+template <int COUNT>
+void read(PyObject *dict, PyObject *const (&names)[COUNT], PyObject *(&values)[COUNT])
+{
+    for (int i = 0; i < COUNT; ++i)
+        values[i] = nullptr;
+    if (dict == nullptr || !PyDict_Check(dict))
+        return;
+    PyObject *key, *value;
+    Py_ssize_t at = 0, found = 0;
+    while (PyDict_Next(dict, &at, &key, &value))
+        for (int i = 0; i < COUNT; ++i)
+            if (key == names[i]) {
+                values[i] = value;
+                ++found;
+                break;
+            }
+    if (found != PyDict_GET_SIZE(dict))
+        for (int i = 0; i < COUNT; ++i)
+            if (values[i] == nullptr)
+                values[i] = PyDict_GetItemWithError(dict, names[i]);
+}
+
+// A tensor's hash, its id: torch computes it in Python, 0.1 us a time.  (Were it another one, nothing would be found with this and the
+// tensor would go to the loops in Python.)
+Py_hash_t hash_of(PyObject *tensor)
+{
+    const Py_hash_t id = (Py_hash_t)(uintptr_t)tensor;
+    return id == -1 ? -2 : id;
+}
+PyObject *of_parameter(PyObject *dict, PyObject *p)  // dict[p]; borrowed, or null
+{
+    return dict != nullptr && PyDict_Check(dict) ? _PyDict_GetItem_KnownHash(dict, p, hash_of(p)) : nullptr;
+}
+
+// the settings of a state, state[name + "_qstate"]
+struct QState {
+    PyObject *enable, *overhead, *qmap;
+
+    explicit QState(PyObject *qstate)
+    {
+        PyObject *const names[] = {N.enable, N.overhead, N.qmap};
+        PyObject *of[3];
+        read(qstate, names, of);
+        enable = of[0];
+        overhead = of[1];
+        qmap = of[2];
+    }
+};
+
 bool on_gpu(const at::Tensor &t)
 {
     return t.defined() && t.is_cuda() && t.layout() == at::kStrided &&
@@ -153,6 +209,7 @@ struct Walk {
     Plan *plan;
     PyObject *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
     Settings s;
+    size_t most;  // records of a batch: the group's tensors, fewer at first where they are many
     int64_t (*workspace_bytes)(int64_t, int64_t);  // lpmm_factored_workspace_bytes
 
     // a dense tensor of n values beside p and of its type (parameters on the kernels are float or half)
@@ -173,11 +230,7 @@ struct Walk {
                    : nullptr;
     }
     // the scales of `groups` groups
-    static Ref scales(PyObject *qstate, PyObject **overhead, const at::Tensor &p, int64_t groups)
-    {
-        *overhead = get(qstate, N.overhead);
-        return reals_of(get(*overhead, N.max1), p, groups);
-    }
+    static Ref scales(PyObject *overhead, const at::Tensor &p, int64_t groups) { return reals_of(get(overhead, N.max1), p, groups); }
     // one tensor per dimension
     template <typename T>
     bool statistics(PyObject *list, const at::Tensor &p, T **out)
@@ -200,6 +253,8 @@ struct Walk {
             if (b.kind == kind && b.device == device && b.qm == qm && b.qv == qv && b.flag == flag)
                 return b;
         plan->batches->push_back(Batch{kind, device, flag, qm, qv, {}, {}, {}, {}, {}, {}});
+        plan->batches->back().records.reserve(most * kRecordBytes[kind]);
+        plan->batches->back().items.reserve(most);
         for (PyObject *map : {qm, qv})
             if (map != nullptr) {
                 Py_INCREF(map);
@@ -256,7 +311,7 @@ struct Walk {
         return item;
     }
 
-    int enabled(PyObject *p, PyObject *qstate)  // -1: not decided here
+    int enabled(PyObject *p, PyObject *e)  // e: of the state's settings; -1: not decided here
     {
         if (override_ != nullptr && PyDict_GET_SIZE(override_) != 0) {
             PyObject *id = PyLong_FromVoidPtr(p);
@@ -267,7 +322,6 @@ struct Walk {
             if (o != nullptr)
                 return PyObject_IsTrue(o);
         }
-        PyObject *e = get(qstate, N.enable);
         return e != nullptr ? PyObject_IsTrue(e) : -1;
     }
 
@@ -275,13 +329,15 @@ struct Walk {
     static void next_codes(Item &item, size_t at, PyObject *st, PyObject *name, const at::Tensor &codes)
     {
         item.need[item.needs++] = Need{at, 0, item.swaps, codes};
-        item.swap[item.swaps++] = Swap{st, name, nullptr};
+        item.swap[item.swaps++] = Swap{st, name, nullptr, -1};
     }
     static void scratch(Item &item, size_t at, int64_t n) { item.need[item.needs++] = Need{at, n, -1, at::Tensor()}; }
 
     bool adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
-    bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
-    bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
+    bool factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const Ref &step, PyObject *mo,
+                  PyObject *row_of, const QState &m_of);
+    bool half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, PyObject *mo, PyObject *vo,
+              const QState &m_of, const QState &v_of, int en_m, int en_v);
     bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const Ref &mc,
              const Ref &ms, const Ref &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
     bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const Ref &any_mc,
@@ -289,7 +345,10 @@ struct Walk {
     bool sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
 };
 
-void swap_later(Item &item, PyObject *dict, PyObject *key, PyObject *value) { item.swap[item.swaps++] = Swap{dict, key, value}; }
+void swap_later(Item &item, PyObject *dict, PyObject *key, PyObject *value, Py_hash_t hash = -1)
+{
+    item.swap[item.swaps++] = Swap{dict, key, value, hash};
+}
 
 // true: a record was added.  Every return before that leaves the plan as it was.
 bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
@@ -297,22 +356,25 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     if (!g.defined() || !on_gpu(p) || !on_gpu(g) || p.device() != g.device() || p.numel() != g.numel() ||
         g.scalar_type() != p.scalar_type())
         return false;
-    const Ref step = tensor_of(get(st, N.step));
+    PyObject *const names[] = {N.step, N.exp_avg, N.exp_avg_qstate, N.exp_avg_sq, N.exp_avg_sq_qstate, N.exp_avg_sq_row};
+    PyObject *state_of[6];
+    read(st, names, state_of);
+    const Ref step = tensor_of(state_of[0]);
     if (step == nullptr || !step->is_cpu() || step->scalar_type() != at::kFloat || step->dim() != 0)
         return false;
-    const bool is_factored = get(st, N.exp_avg_sq_row) != nullptr;
-    if (!floats(p))
-        return halfs(p) && !s.fused && !is_factored && half(po, p, g, st);
-    if (is_factored)
-        return factored(po, p, g, st);
-    if (s.fused == 2)
+    const bool is_factored = state_of[5] != nullptr;
+    if (floats(p) ? !is_factored && s.fused == 2 : !halfs(p) || s.fused || is_factored)
         return false;
-    PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
-    PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
-    const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
+    PyObject *const mo = state_of[1], *const vo = state_of[3];
+    const QState m_of(state_of[2]), v_of(state_of[4]);
+    if (is_factored)
+        return factored(po, p, g, st, step, mo, state_of[5], m_of);
+    const int en_m = enabled(po, m_of.enable), en_v = enabled(po, v_of.enable);
     if (en_m < 0 || en_v < 0)
         return false;
-    Item item = item_of(po, g, tensor_of(get(st, N.step)));
+    Item item = item_of(po, g, step);
+    if (!floats(p))
+        return half(po, p, g, st, item, mo, vo, m_of, v_of, en_m, en_v);
     const int64_t n = p.numel();
     if (!en_m && !en_v) {
         const Ref m = reals_like(mo, p), v = reals_like(vo, p);
@@ -322,14 +384,14 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         add(batch(kPlain, p, nullptr, nullptr), r, item);
         return true;
     }
-    PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap);
+    PyObject *const qm = m_of.qmap, *const qv = v_of.qmap;
     const Ref map_m = tensor_of(qm), map_v = tensor_of(qv);
     const Ref vc = codes(vo, p, s.fused ? (n + 1) / 2 : packed(n, 128, s.bits_rank1));
     if (map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) || vc == nullptr || !en_v)
         return false;
-    PyObject *oh_m = nullptr, *oh_v = nullptr;
+    PyObject *const oh_m = m_of.overhead, *const oh_v = v_of.overhead;
     if (s.fused || s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
-        const Ref vs = scales(qs_v, &oh_v, p, (n + 127) / 128);
+        const Ref vs = scales(oh_v, p, (n + 127) / 128);
         if (vs == nullptr)
             return false;
         if (!en_m) {
@@ -340,7 +402,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
             add(batch(kFlatM32, p, nullptr, qv), r, item);
             return true;
         }
-        const Ref mc = codes(mo, p, s.fused ? (n + 1) / 2 : packed(n, 128, false)), ms = scales(qs_m, &oh_m, p, (n + 127) / 128);
+        const Ref mc = codes(mo, p, s.fused ? (n + 1) / 2 : packed(n, 128, false)), ms = scales(oh_m, p, (n + 127) / 128);
         if (!(s.fused ? n % 2 == 0 : s.m_group128 != 0) || mc == nullptr || ms == nullptr)
             return false;
         lpmm_adamw4bit_tensor r;
@@ -355,7 +417,6 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         add(batch(s.fused ? kFused4 : kFlat, p, qm, qv), r, item);
         return true;
     }
-    oh_v = get(qs_v, N.overhead);
     PyObject *cur = get(oh_v, N.max_dims);
     if (!(s.v_rank1 || s.bits_rank1) || cur == nullptr || p.dim() < 2 || p.size(0) == 0)
         return false;
@@ -371,7 +432,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         if (s.m_group <= 0)
             return false;
         mc = codes(mo, p, packed(n, s.m_group, s.bits_rank1));
-        ms = scales(qs_m, &oh_m, p, (n + s.m_group - 1) / s.m_group);
+        ms = scales(oh_m, p, (n + s.m_group - 1) / s.m_group);
         if (mc == nullptr || ms == nullptr)
             return false;
         r.m_codes = use<uint8_t>(mc);
@@ -384,7 +445,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     if (p.dim() > 2)
         return en_m && s.m_group128 && s.v_rank1 && served &&
                nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, vc, oh_v, qm, qv);
-    PyObject *nxt = get(spare_stats, po);
+    PyObject *nxt = of_parameter(spare_stats, po);
     float *now[2], *next[2];
     if (!statistics(cur, p, now) || !statistics(nxt, p, next))
         return false;
@@ -392,7 +453,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     r.v_colmax = now[1];
     r.v_rowmax_next = next[0];
     r.v_colmax_next = next[1];
-    swap_later(item, spare_stats, po, cur);
+    swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     if (!en_m) {
         const Ref m = reals_like(mo, p);
@@ -426,13 +487,13 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         item.swaps = 0;
         return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, vc, oh_m, oh_v, qm, qv);
     }
-    PyObject *spare = get(spare_scales, po);
+    PyObject *spare = of_parameter(spare_scales, po);
     const Ref ms_next = reals_of(spare, p, ms->numel());
     if (!((s.m_wide && whole) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
         return false;
     lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        use<float>(ms_next), r.v_codes, r.v_rowmax,
                                   r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
-    swap_later(item, spare_scales, po, get(oh_m, N.max1));
+    swap_later(item, spare_scales, po, get(oh_m, N.max1), hash_of(po));
     swap_later(item, oh_m, N.max1, spare);
     add(batch(kRank1Wide, p, qm, qv, ragged), w, item);
     return true;
@@ -442,7 +503,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
 bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const Ref &mc,
                const Ref &ms, const Ref &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv)
 {
-    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *spare = get(spare_scales, po);
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = of_parameter(spare_stats, po), *spare = of_parameter(spare_scales, po);
     void *now[2], *next[2];
     const Ref ms_next = ms != nullptr ? reals_of(spare, p, ms->numel()) : nullptr;
     if (!statistics(cur, p, now) || !statistics(nxt, p, next) || (ms != nullptr && ms_next == nullptr))
@@ -461,14 +522,14 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
     r.cols = p.size(1);
     if (kind == LPMM_RANK1_HALF)
         scratch(item, offsetof(lpmm_rank1_any_tensor, work), r.rows + r.cols + (p.numel() + 127) / 128);
-    swap_later(item, spare_stats, po, cur);
+    swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, *vc);
     if (ms != nullptr) {
         r.m_max1 = use<>(ms);
         r.m_max1_next = use<>(ms_next);
         next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *mc);
-        swap_later(item, spare_scales, po, get(oh_m, N.max1));
+        swap_later(item, spare_scales, po, get(oh_m, N.max1), hash_of(po));
         swap_later(item, oh_m, N.max1, spare);
     }
     add(batch(kAny, p, qm, qv, kind), r, item);
@@ -476,18 +537,19 @@ bool Walk::any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
 }
 
 // a matrix with a factored second moment, its first moment 4-bit in groups of 128 values or not quantised
-bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
+bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, const Ref &step, PyObject *mo,
+                    PyObject *row_of, const QState &m_of)
 {
     if (p.dim() != 2 || p.numel() == 0 || workspace_bytes == nullptr)
         return false;
     const int64_t rows = p.size(0), cols = p.size(1), n = p.numel();
-    PyObject *qs = get(st, N.exp_avg_qstate), *mo = get(st, N.exp_avg), *qm = get(qs, N.qmap), *oh = nullptr;
-    const Ref row = reals_of(get(st, N.exp_avg_sq_row), p, rows), col = reals_of(get(st, N.exp_avg_sq_col), p, cols);
+    PyObject *const qm = m_of.qmap;
+    const Ref row = reals_of(row_of, p, rows), col = reals_of(get(st, N.exp_avg_sq_col), p, cols);
     const Ref map = tensor_of(qm);
-    const int en = enabled(po, qs);
+    const int en = enabled(po, m_of.enable);
     if (en < 0 || row == nullptr || col == nullptr || map == nullptr || !floats(*map))
         return false;
-    Item item = item_of(po, g, tensor_of(get(st, N.step)));
+    Item item = item_of(po, g, step);
     lpmm_factored_tensor r;
     memset(&r, 0, sizeof r);
     r.p = ptr<float>(p);
@@ -497,7 +559,7 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
     r.rows = rows;
     r.cols = cols;
     if (en) {
-        const Ref mc = codes(mo, p, packed(n, 128, false)), ms = scales(qs, &oh, p, (n + 127) / 128);
+        const Ref mc = codes(mo, p, packed(n, 128, false)), ms = scales(m_of.overhead, p, (n + 127) / 128);
         if (!s.m_group128 || mc == nullptr || ms == nullptr)
             return false;
         r.m_codes = use<uint8_t>(mc);
@@ -515,13 +577,10 @@ bool Walk::factored(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyOb
 }
 
 // float16 parameters on the non-fused path (lpmm/optim/adamw.py: _half_kernel_kind)
-bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st)
+bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, PyObject *mo, PyObject *vo,
+                const QState &m_of, const QState &v_of, int en_m, int en_v)
 {
-    PyObject *qs_m = get(st, N.exp_avg_qstate), *qs_v = get(st, N.exp_avg_sq_qstate);
-    PyObject *mo = get(st, N.exp_avg), *vo = get(st, N.exp_avg_sq);
-    const int en_m = enabled(po, qs_m), en_v = enabled(po, qs_v);
     const int64_t n = p.numel(), groups = (n + 127) / 128;
-    Item item = item_of(po, g, tensor_of(get(st, N.step)));
     if (en_m == 0 && en_v == 0) {
         const Ref m = reals_like(mo, p), v = reals_like(vo, p);
         if (m == nullptr || v == nullptr || m->sizes() != p.sizes() || v->sizes() != p.sizes())
@@ -530,15 +589,15 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
         add(batch(kHalfPlain, p, nullptr, nullptr), r, item);
         return true;
     }
-    PyObject *qm = get(qs_m, N.qmap), *qv = get(qs_v, N.qmap), *oh_m = nullptr, *oh_v = get(qs_v, N.overhead);
+    PyObject *const qm = m_of.qmap, *const qv = v_of.qmap, *const oh_m = m_of.overhead, *const oh_v = v_of.overhead;
     const Ref map_m = tensor_of(qm), map_v = tensor_of(qv);
-    const Ref mc = codes(mo, p, packed(n, 128, false)), vc = codes(vo, p, packed(n, 128, false)), ms = scales(qs_m, &oh_m, p, groups);
+    const Ref mc = codes(mo, p, packed(n, 128, false)), vc = codes(vo, p, packed(n, 128, false)), ms = scales(oh_m, p, groups);
     PyObject *const half_type = reinterpret_cast<PyObject *>(torch::getTHPDtype(at::kHalf));
     if (en_m != 1 || en_v != 1 || !s.m_group128 || map_m == nullptr || map_v == nullptr || !floats(*map_m) || !floats(*map_v) ||
         mc == nullptr || vc == nullptr || ms == nullptr || get(oh_m, N.dtype) != half_type || get(oh_v, N.dtype) != half_type)
         return false;
     if (s.v_group128 || (s.v_rank1 && p.dim() == 1)) {
-        const Ref vs = scales(qs_v, &oh_v, p, groups);
+        const Ref vs = scales(oh_v, p, groups);
         if (vs == nullptr)
             return false;
         lpmm_adamw4bit_f16_tensor r = {ptr(p), ptr(g), use<uint8_t>(mc), use<uint8_t>(vc), use<>(ms), use<>(vs), n, 0.0f, 0.0f};
@@ -550,11 +609,11 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
     const int64_t rows = p.size(0), cols = p.size(1);
     if (cols % 128 != 0 || !aligned16(ptr(p)) || !aligned16(ptr(g)))
         return (cols >= 32 || rows <= 32768) && any(po, p, g, st, item, LPMM_RANK1_HALF, mc, ms, vc, oh_m, oh_v, qm, qv);
-    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po);
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = of_parameter(spare_stats, po);
     void *now[2], *next[2];
     if (!statistics(cur, p, now) || !statistics(nxt, p, next))
         return false;
-    swap_later(item, spare_stats, po, cur);
+    swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     lpmm_nonfused_rank1_f16_tensor r = {ptr(p), ptr(g), use<uint8_t>(mc), use<>(ms), use<uint8_t>(vc), now[0], now[1], next[0], next[1],
                                         nullptr, rows, cols, 0.0f, 0.0f};
@@ -571,7 +630,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     const int dims = (int)p.dim();
     if (dims > LPMM_RANK1_ND_MAX || (r.rows < 16 && p.numel() > (1 << 20)) || r.cols > (1 << 16))
         return false;
-    PyObject *cur = get(oh_v, N.max_dims), *nxt = get(spare_stats, po), *scratch = get(nd_scratch, po);
+    PyObject *cur = get(oh_v, N.max_dims), *nxt = of_parameter(spare_stats, po), *scratch = of_parameter(nd_scratch, po);
     PyObject *row = get(scratch, N.row);
     const int64_t pitch = (r.cols + 31) / 32 * 32;  // _nd_pitch
     const Ref work = reals_of(get(scratch, N.work), p, 3 * pitch);
@@ -601,7 +660,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     r.v_colmax = rows + old_row * pitch;
     r.v_colmax_next = rows + raw_row * pitch;
     // any_mc: a column count for the general kernels, which also need the next scales
-    PyObject *spare = get(spare_scales, po);
+    PyObject *spare = of_parameter(spare_scales, po);
     const Ref ms_next = any_mc != nullptr ? reals_of(spare, p, (p.numel() + 127) / 128) : nullptr;
     if (any_mc != nullptr && ms_next == nullptr)
         return false;
@@ -609,7 +668,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     if (row_obj == nullptr)
         return false;
     plan->others->push_back(row_obj);
-    swap_later(item, spare_stats, po, cur);
+    swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     swap_later(item, scratch, N.scale_of, nxt);
     swap_later(item, scratch, N.row, row_obj);
@@ -623,7 +682,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
                                r.v_rowmax_next, r.v_colmax_next, nullptr, r.rows, r.cols, 0.0f, 0.0f};
     next_codes(item, offsetof(lpmm_rank1_any_tensor, m_codes_next), st, N.exp_avg, *any_mc);
     next_codes(item, offsetof(lpmm_rank1_any_tensor, v_codes_next), st, N.exp_avg_sq, *vc);
-    swap_later(item, spare_scales, po, get(oh_m, N.max1));
+    swap_later(item, spare_scales, po, get(oh_m, N.max1), hash_of(po));
     swap_later(item, oh_m, N.max1, spare);
     Batch &b = batch(kNdAny, p, qm, qv);
     add(b, w, item);
@@ -637,9 +696,13 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
 {
     if (!g.defined() || !floats(p) || !floats(g) || p.device() != g.device() || p.numel() != g.numel())
         return false;
-    PyObject *qs = get(st, N.momentum_buffer_qstate), *bo = get(st, N.momentum_buffer);
+    PyObject *const names[] = {N.momentum_buffer, N.momentum_buffer_qstate};
+    PyObject *state_of[2];
+    read(st, names, state_of);
+    PyObject *const bo = state_of[0];
+    const QState of(state_of[1]);
     Item item = item_of(po, g, nullptr);
-    const int en = enabled(po, qs);
+    const int en = enabled(po, of.enable);
     if (en < 0)
         return false;
     if (!en) {
@@ -650,8 +713,8 @@ bool Walk::sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject 
         add(batch(kSgdPlain, p, nullptr, nullptr), r, item);
         return true;
     }
-    PyObject *oh = nullptr, *qm = get(qs, N.qmap);
-    const Ref map = tensor_of(qm), mc = codes(bo, p, packed(p.numel(), 128, false)), ms = scales(qs, &oh, p, (p.numel() + 127) / 128);
+    PyObject *const qm = of.qmap;
+    const Ref map = tensor_of(qm), mc = codes(bo, p, packed(p.numel(), 128, false)), ms = scales(of.overhead, p, (p.numel() + 127) / 128);
     if (!s.m_group128 || map == nullptr || !floats(*map) || mc == nullptr || ms == nullptr)
         return false;
     lpmm_sgd4bit_tensor r = {ptr<float>(p), ptr<float>(g), use<uint8_t>(mc), use<float>(ms), p.numel(), 0, 0};
@@ -805,10 +868,30 @@ PyObject *plan_prepare(PyObject *self, PyObject *args)
         return nullptr;
     const size_t bytes = kRecordBytes[b->kind];
     const auto floats = at::TensorOptions().dtype(at::kFloat).device(at::Device(at::kCUDA, (at::DeviceIndex)b->device));
+    // scratch of little size comes out of one allocation for all (1 us each otherwise), at the alignment the allocator gives
+    constexpr int64_t kLittle = 1 << 18, kAlign = 128;  // floats
+    const auto little = [](const Need &need) { return !need.like.defined() && need.n > 0 && need.n < kLittle; };
+    int64_t all = 0, used = 0;
+    for (Py_ssize_t i = first; i < end; ++i)
+        for (uint32_t j = b->items[i].needs; j < b->items[i].needs_end; ++j)
+            if (little(b->needs[j]))
+                all += (b->needs[j].n + kAlign - 1) / kAlign * kAlign;
+    at::Tensor block;
+    if (all != 0)
+        block = at::empty({all}, floats);
     for (Py_ssize_t i = first; i < end; ++i) {
         Record &item = b->items[i];
         for (uint32_t j = item.needs; j < item.needs_end; ++j) {
             Need &need = b->needs[j];
+            if (little(need)) {
+                const void *const p = ptr<float>(block) + used;
+                used += (need.n + kAlign - 1) / kAlign * kAlign;
+                item.scratch = block;
+                memcpy(&b->records[i * bytes + need.at], &p, sizeof p);
+                if (!b->second.empty())
+                    memcpy(&b->second[i * bytes + need.at], &p, sizeof p);
+                continue;
+            }
             const at::Tensor t = need.like.defined() ? at::empty_like(need.like) : at::empty({need.n}, floats);
             if (need.like.defined()) {
                 PyObject *o = THPVariable_Wrap(t);
@@ -849,7 +932,8 @@ PyObject *plan_commit(PyObject *self, PyObject *args)
             if (b->swaps[j].value == nullptr) {
                 PyErr_SetString(PyExc_RuntimeError, "records that were not prepared");
                 return nullptr;
-            } else if (PyDict_SetItem(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value) != 0) {
+            } else if (b->swaps[j].hash != -1 ? _PyDict_SetItem_KnownHash(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value, b->swaps[j].hash) != 0
+                                              : PyDict_SetItem(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value) != 0) {
                 return nullptr;
             }
     }
@@ -896,6 +980,7 @@ PyObject *collect(PyObject *, PyObject *args)
             return nullptr;
         plan->batches->reserve(16);
         w.plan = plan;
+        w.most = (size_t)(PyList_GET_SIZE(params) < 1024 ? PyList_GET_SIZE(params) : 1024);
         w.state = state;
         w.override_ = override_;
         w.spare_stats = spare_stats;
@@ -911,7 +996,7 @@ PyObject *collect(PyObject *, PyObject *args)
                 if (!g.defined() && own)
                     continue;
                 if (serve && own) {
-                    PyObject *st = PyDict_GetItemWithError(state, po);
+                    PyObject *st = of_parameter(state, po);
                     if (st != nullptr && PyDict_Check(st) && PyDict_GET_SIZE(st) != 0)
                         served = is_sgd ? w.sgd(po, p, g, st) : w.adamw(po, p, g, st);
                 }

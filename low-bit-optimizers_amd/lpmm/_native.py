@@ -47,6 +47,8 @@ PROTOTYPES = {
     "lpmm_dequant_rank1": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp]),
     "lpmm_rank1_stats_nd": (_int, [_vp, _int, _vp, _vp, _vp, _vp]),
     "lpmm_rank1_row_scale_nd": (_int, [_vp, _int, _vp, _vp, _vp]),
+    "lpmm_quant_rank1_nd": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _int, _vp, _vp, _vp]),
+    "lpmm_dequant_rank1_nd": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _int, _vp, _vp]),
     "lpmm_pack_nonlinear": (_int, [_vp, _vp, _int, _i64, _vp, _vp]),
     "lpmm_pack_nonlinear_sr": (_int, [_vp, _vp, _int, _i64, ctypes.c_uint64, ctypes.c_uint64, _vp, _vp]),
     "lpmm_unpack_nonlinear": (_int, [_vp, _vp, _int, _i64, _vp, _vp]),
@@ -183,9 +185,15 @@ def walk():
     return _walk
 
 
+_factored_workspace = None
+
+
 def factored_workspace():
     """Address of lpmm_factored_workspace_bytes, which the walk calls."""
-    return ctypes.cast(lib().lpmm_factored_workspace_bytes, ctypes.c_void_p).value
+    global _factored_workspace
+    if _factored_workspace is None:
+        _factored_workspace = ctypes.cast(lib().lpmm_factored_workspace_bytes, ctypes.c_void_p).value
+    return _factored_workspace
 
 
 # kinds of records a walk makes (enum Kind of csrc/walk.cpp)
@@ -201,6 +209,9 @@ def check(status, what):
 
 
 def current_stream(device):
+    """Handle of torch's current stream on a device (an index, or a torch.device).  Read directly: the Stream object that
+    torch.cuda.current_stream makes on the way costs 1 to 2 us, of 11 for a whole call on a small tensor."""
     import torch
 
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device if isinstance(device, int) else device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

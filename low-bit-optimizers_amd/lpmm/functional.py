@@ -130,6 +130,12 @@ def _shape_array(shape):
     return (ctypes.c_int64 * len(shape))(*shape)
 
 
+def _empty_statistics(shape, device):
+    """A float32 tensor per dimension, its length there and one elsewhere."""
+    ones = (1,) * len(shape)
+    return [torch.empty(ones[:i] + (d,) + ones[i + 1:], dtype=torch.float32, device=device) for i, d in enumerate(shape)]
+
+
 def get_sm3_statistics(x, **kwargs):
     """max|x| over all dimensions but one, for each dimension (keepdim shapes).  float32 CUDA
     tensors of 2..8 dimensions take HIP kernels that read x once."""
@@ -139,52 +145,26 @@ def get_sm3_statistics(x, **kwargs):
         rows, cols = xc.shape
         rowmax = torch.empty((rows, 1), dtype=torch.float32, device=x.device)
         colmax = torch.empty((1, cols), dtype=torch.float32, device=x.device)
-        with torch.cuda.device(x.device):
+        with torch.cuda.device(x.get_device()):
             st = _native.lib().lpmm_rank1_stats(xc.data_ptr(), rows, cols, rowmax.data_ptr(), colmax.data_ptr(),
-                                                _native.current_stream(x.device))
+                                                _native.current_stream(x.get_device()))
         _native.check(st, "rank1_stats")
         return [rowmax, colmax]
     if 2 < x.dim() <= RANK1_ND_MAX and on_hip:
         xc = x.contiguous()
         shape = tuple(xc.shape)
-        stats = []
-        for i, d in enumerate(shape):
-            keep = [1] * len(shape)
-            keep[i] = d
-            stats.append(torch.empty(keep, dtype=torch.float32, device=x.device))
+        stats = _empty_statistics(shape, x.device)
         work = None
         if shape[-1] >= 32:  # long last dimension: the 2-D kernel plus a fold of its row maxima
             work = torch.empty((xc.numel() // shape[-1],), dtype=torch.float32, device=x.device)
-        with torch.cuda.device(x.device):
+        with torch.cuda.device(x.get_device()):
             st = _native.lib().lpmm_rank1_stats_nd(xc.data_ptr(), len(shape), _shape_array(shape), _ptr_array(stats),
                                                    work.data_ptr() if work is not None else None,
-                                                   _native.current_stream(x.device))
+                                                   _native.current_stream(x.get_device()))
         _native.check(st, "rank1_stats_nd")
         return stats
     qx = x.abs()
     return [_max_reduce_except_dim(qx, i) for i in range(x.dim())]
-
-
-def _row_scale_nd(max_dims, shape):
-    """For a tensor of more than two dimensions: per row of its (numel / shape[-1], shape[-1])
-    view the smallest statistic of the leading dimensions.  With the last dimension's
-    statistics as column maxima the 2-D kernels then scale by min over all dimensions, which
-    is _compute_sm3_scale_tensor (lpmm/functional.py:503-509)."""
-    if len(shape) > RANK1_ND_MAX:
-        raise NotImplementedError(f"rank-1 scaling of a {len(shape)}-D tensor: the kernels take up to "
-                                  f"{RANK1_ND_MAX} dimensions")
-    dev = max_dims[0].device
-    stats = [m.to(torch.float32).contiguous() for m in max_dims]
-    for m, d in zip(stats, shape):
-        if m.numel() != d:
-            raise ValueError(f"max_dims do not belong to a tensor of shape {tuple(shape)}")
-    rows = math.prod(shape[:-1])
-    row_scale = torch.empty((rows,), dtype=torch.float32, device=dev)
-    with torch.cuda.device(dev):
-        st = _native.lib().lpmm_rank1_row_scale_nd(_ptr_array(stats), len(shape), _shape_array(tuple(shape)),
-                                                   row_scale.data_ptr(), _native.current_stream(dev))
-    _native.check(st, "rank1_row_scale_nd")
-    return row_scale, stats[-1]
 
 
 def _compute_sm3_scale_tensor(max_dims):
@@ -299,8 +279,8 @@ def quant_group_(x, qmap, gp_sz, codes=None, max1=None, b=4):
     if max1 is None:
         max1 = torch.empty((groups, 1), dtype=torch.float32, device=x.device)
     lib = _native.lib()
-    with torch.cuda.device(x.device):
-        stream = _native.current_stream(x.device)
+    with torch.cuda.device(x.get_device()):
+        stream = _native.current_stream(x.get_device())
         if b == 4:
             st = lib.lpmm_quant_group(x.data_ptr(), n, gp_sz, qmap.data_ptr(), codes.data_ptr(), max1.data_ptr(),
                                       stream)
@@ -316,25 +296,16 @@ def quant_rank1_(x, qmap, codes=None, b=4):
     """'rank1' scaling of a contiguous float32 CUDA tensor of two or more dimensions:
     statistics kernel(s), then normalise + search + pack kernel (more than two dimensions: on
     the (numel / shape[-1], shape[-1]) view with the leading dimensions' minima as row scale)."""
-    max_dims = get_sm3_statistics(x)
-    if x.dim() == 2:
-        rows, cols = x.shape
-        rowmax, colmax = max_dims
-    else:
-        rows, cols = x.numel() // x.shape[-1], x.shape[-1]
-        rowmax, colmax = _row_scale_nd(max_dims, x.shape)
+    shape, dev = tuple(x.shape), x.device
+    max_dims = _empty_statistics(shape, dev)
+    work = torch.empty((x.numel() // shape[-1],), dtype=torch.float32, device=dev) if len(shape) > 2 else None
     if codes is None:
-        codes = torch.empty((packed_nbytes(rows * cols, b),), dtype=torch.int8, device=x.device)
-    lib = _native.lib()
-    with torch.cuda.device(x.device):
-        stream = _native.current_stream(x.device)
-        if b == 4:
-            st = lib.lpmm_quant_rank1(x.data_ptr(), rows, cols, rowmax.data_ptr(), colmax.data_ptr(),
-                                      qmap.data_ptr(), codes.data_ptr(), stream)
-        else:
-            st = lib.lpmm_quant_rank1_bits_table(x.data_ptr(), rows, cols, rowmax.data_ptr(), colmax.data_ptr(),
-                                                 qmap.data_ptr(), b, code_table(qmap, b).data_ptr(),
-                                                 codes.data_ptr(), stream)
+        codes = torch.empty((packed_nbytes(x.numel(), b),), dtype=torch.int8, device=dev)
+    table = None if b == 4 else code_table(qmap, b).data_ptr()
+    with torch.cuda.device(x.get_device()):
+        st = _native.lib().lpmm_quant_rank1_nd(
+            x.data_ptr(), len(shape), _shape_array(shape), _ptr_array(max_dims), None if work is None else work.data_ptr(),
+            qmap.data_ptr(), b, table, codes.data_ptr(), _native.current_stream(x.get_device()))
     _native.check(st, "quant_rank1")
     return codes, max_dims
 
@@ -407,8 +378,8 @@ def vectorwise_dequant(qx, denormalized=True, **kwargs):
         n = shape.numel()
         if gp_sz % 128 == 0 and kwargs["max1"].dtype is torch.float32:
             x = torch.empty(shape, dtype=torch.float32, device=dev)
-            with torch.cuda.device(dev):
-                stream = _native.current_stream(dev)
+            with torch.cuda.device(codes.get_device()):
+                stream = _native.current_stream(codes.get_device())
                 if b == 4:
                     st = lib.lpmm_dequant_group(codes.data_ptr(), kwargs["max1"].data_ptr(), qmap.data_ptr(), n,
                                                 gp_sz, x.data_ptr(), stream)
@@ -423,21 +394,18 @@ def vectorwise_dequant(qx, denormalized=True, **kwargs):
         max_dims = kwargs["max_dims"]
         if (2 <= len(scaled_shape) <= RANK1_ND_MAX and numel(scaled_shape) > 0
                 and all(m.dtype is torch.float32 for m in max_dims)):
-            if len(scaled_shape) == 2:
-                rows, cols = scaled_shape
-                rowmax, colmax = max_dims
-            else:
-                rows, cols = numel(scaled_shape[:-1]), scaled_shape[-1]
-                rowmax, colmax = _row_scale_nd(max_dims, scaled_shape)
+            dims, work = len(scaled_shape), None
+            if dims > 2:
+                max_dims = [m.contiguous() for m in max_dims]
+                for m, d in zip(max_dims, scaled_shape):
+                    if m.numel() != d:
+                        raise ValueError(f"max_dims do not belong to a tensor of shape {tuple(scaled_shape)}")
+                work = torch.empty((numel(scaled_shape[:-1]),), dtype=torch.float32, device=dev)
             x = torch.empty(scaled_shape, dtype=torch.float32, device=dev)
-            with torch.cuda.device(dev):
-                stream = _native.current_stream(dev)
-                if b == 4:
-                    st = lib.lpmm_dequant_rank1(codes.data_ptr(), rowmax.data_ptr(), colmax.data_ptr(),
-                                                qmap.data_ptr(), rows, cols, x.data_ptr(), stream)
-                else:
-                    st = lib.lpmm_dequant_rank1_bits(codes.data_ptr(), rowmax.data_ptr(), colmax.data_ptr(),
-                                                     qmap.data_ptr(), b, rows, cols, x.data_ptr(), stream)
+            with torch.cuda.device(codes.get_device()):
+                st = lib.lpmm_dequant_rank1_nd(
+                    codes.data_ptr(), dims, _shape_array(scaled_shape), _ptr_array(max_dims), None if work is None else work.data_ptr(),
+                    qmap.data_ptr(), b, x.data_ptr(), _native.current_stream(codes.get_device()))
             _native.check(st, "dequant_rank1")
         else:
             x = nonlinear_dequant(codes, qmap, b, shape=scaled_shape, round_type=kwargs["round_type"])

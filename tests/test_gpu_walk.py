@@ -480,3 +480,25 @@ def test_scratch_vectors_share_no_cache_line(serve, monkeypatch):
         work, cols = opt._nd_scratch[p]["work"], p.numel() // p.shape[0]
         assert work.dtype is torch.float32 and work.shape[0] == 3 and work.shape[1] >= cols
         assert all(work[r].data_ptr() % 128 == 0 for r in range(3))
+
+
+@pytest.mark.parametrize("case", ["fused", "default", "half", "sgd"])
+def test_states_under_equal_keys_that_are_other_strings(case):
+    """A state's names are compared by address first; dictionaries with other strings of the same text, or with further
+    entries, are served alike."""
+    sides = [_build(case, np.random.default_rng(7)) for _ in range(2)]
+    for step in range(3):
+        for k, (params, opt) in enumerate(sides):
+            rng = np.random.default_rng(8 + step)
+            for p in params:
+                p.grad = torch.from_numpy(rng.standard_normal(p.shape) * 0.1).to(p.dtype).cuda()
+            if step == 1 and k == 1:
+                def other(d):
+                    return {"".join(list(key)): other(v) if isinstance(v, dict) else v for key, v in d.items()} | {"further": 0}
+                for p in params:
+                    opt.state[p] = other(opt.state[p])
+            opt.step()
+    for p, q in zip(sides[0][0], sides[1][0]):
+        assert torch.equal(p.detach(), q.detach())
+        a, b = _state(sides[0][1], p), {k: v for k, v in opt.state[q].items() if torch.is_tensor(v)}
+        assert all(torch.equal(a[k], v) for k, v in b.items())
