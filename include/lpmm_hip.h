@@ -573,6 +573,25 @@ int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensor
                                              const void *table_v, double beta1, double beta2, double lr,
                                              double weight_decay, double eps, int passes, void *stream);
 
+/* The two-pass steps on one kind of quantised tensors together with tensors with fp32 states (lpmm_nonfused_update_multi), which go
+ * with the launch that clears the next statistics, as far as they fit.  Either may be empty.  kind: whose records `tensors`
+ * holds, with the limits that its own entry point states -- lpmm_nonfused_rank1_tensor for _MATRIX, _BITS (bits_m, bits_v and the
+ * tables; 4 and NULL elsewhere) and _ND (with folds), lpmm_rank1_v4bit_tensor for _FLOAT_M, lpmm_rank1_mgroup_tensor for _GROUPS
+ * (m_group_size; 128 elsewhere), lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
+enum {
+    LPMM_STEP_MATRIX = 0,
+    LPMM_STEP_BITS = 1,
+    LPMM_STEP_ND = 2,
+    LPMM_STEP_FLOAT_M = 3,
+    LPMM_STEP_GROUPS = 4,
+    LPMM_STEP_ANY = 8
+};
+int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors, const lpmm_rank1_small_vector *folds, int64_t count,
+                                        const lpmm_adamw_fp32_tensor *plain, int64_t plain_count, int64_t m_group_size,
+                                        const float *qmap_m, int bits_m, const void *table_m, const float *qmap_v, int bits_v,
+                                        const void *table_v, double beta1, double beta2, double lr, double weight_decay, double eps,
+                                        void *stream);
+
 /* lpmm_nonfused_adamw4bit_rank1_step_multi for code widths of 5 to 8 bits (lpmm/configs/
  * default_{5,6,7,8}b.yml): qmap_m / qmap_v hold 2^bits_m / 2^bits_v entries; the code arrays hold
  * one code per byte (lpmm/cpp_extension/quantization_kernel.cu:516-533, :656-669):

@@ -887,6 +887,7 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
     }
 
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
+    NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
     MultiFa args;
     args.decay = c.decay;
     args.w1 = c.w1;
@@ -932,7 +933,7 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
             d.vec_g = aligned_to(t.g, 16) && t.cols % 4 == 0;
             d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16);
             d.kind = t.m_max1 == nullptr ? kFlatFloat : t.cols % 8 == 0 && aligned_to(t.col, 16) ? kFlatRows : kFlatAny;
-            const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, t.step);
+            const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             d.rbc2_sqrt = h.rbc2_sqrt;

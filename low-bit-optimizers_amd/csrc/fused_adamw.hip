@@ -18,7 +18,7 @@
 // use the correctly rounded reciprocal plus one fma correction step; both give the same
 // results as the generic search and the plain division, which remain as the fallback for
 // any other map.
-#include "lpmm_update.hpp"
+#include "lpmm_plain.hpp"
 
 #include <hip/hip_fp16.h>
 #include <math.h>
@@ -51,6 +51,7 @@ constexpr uint32_t fused_lds_bytes()
     return (ALLFULL ? LPMM_FUSED_LDS_KB_WHOLE : LPMM_FUSED_LDS_KB_RAGGED) * 1024u;
 }
 static_assert(fused_lds_bytes<true>() >= kLdsBytes && fused_lds_bytes<false>() >= kLdsBytes, "tables do not fit");
+static_assert(kThreads == kPlainThreads, "tile_fp32 runs in these kernels");
 static_assert(kThreads == kEncEntries, "lds_fill_load / lds_fill_store: one encode-table entry per thread");
 // Optional pause (units of 64 cycles) of every wave of the straight-line variant before its first load.
 // It paid 0.8 % while consecutive tiles went to different XCDs (6 units); with the tile order below it
@@ -156,27 +157,6 @@ using FusedStep4 = FusedArith;
 #else
 using FusedStep4 = FusedArith4;
 #endif
-
-struct NonFusedArith {
-    // code buffers are padded to whole tiles plus one byte, as the reference's packing
-    // operator lays them out: every nibble of an existing group is written, groups past the
-    // tensor hold the code of 0.0
-    static constexpr bool kPadded = true;
-    NfHyper h;
-    template <class M, class T>
-    __device__ __forceinline__ NonFusedArith(const M &a, const T &t)
-    {
-        h.decay = a.s[0];
-        h.w1 = a.s[1];
-        h.b2 = a.s[2];
-        h.w2 = a.s[3];
-        h.eps = a.s[4];
-        h.neg_step_size = t.k[0];
-        h.bc2_sqrt = t.k[1];
-        h.rbc2_sqrt = t.k[2];
-    }
-    __device__ __forceinline__ void elt(float &p, float g, float &m, float &v) const { nonfused_elt(p, g, m, v, h); }
-};
 
 static_assert(sizeof(Multi4) + 2 * sizeof(void *) <= 4096, "kernel arguments exceed 4 KB");
 
@@ -431,56 +411,6 @@ __global__ __launch_bounds__(kThreads) void adamw4bit_kernel(const Multi4 args, 
 // ---------------------------------------------------------------------------------------
 // fp32-state step (lpmm/cpp_extension/fused_adamw_kernel.cu:52-78).
 // ---------------------------------------------------------------------------------------
-struct TensorF {
-    float *p;
-    const float *g;
-    float *m;
-    float *v;
-    int64_t n;
-    float k[4];  // per-tensor scalars, as in Tensor4
-};
-
-constexpr int kMultiFMax = 64;
-constexpr int kTileF = 1024;  // 256 threads x 4 elements
-
-struct MultiF {
-    TensorF t[kMultiFMax];
-    uint32_t tile_start[kMultiFMax + 1];
-    int count;
-    float s[7];
-};
-
-static_assert(sizeof(MultiF) <= 4096, "kernel arguments exceed 4 KB");
-
-// fp32 states, either arithmetic (the FusedArith / NonFusedArith constructors only read the
-// scalars, which Multi4 and MultiF name alike)
-template <class Arith>
-__device__ __forceinline__ void tile_fp32(const MultiF &args, uint32_t tile)
-{
-    int lo = 0, hi = args.count;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (args.tile_start[mid] <= tile)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    const TensorF &t = args.t[lo];
-    const Arith h(args, t);
-    const int64_t tile0 = (int64_t)(tile - args.tile_start[lo]) * kTileF;
-#pragma unroll
-    for (int k = 0; k < kTileF / kThreads; ++k) {
-        const int64_t i = tile0 + k * kThreads + threadIdx.x;
-        if (i < t.n) {
-            float p = t.p[i], m = t.m[i], v = t.v[i];
-            h.elt(p, t.g[i], m, v);
-            t.p[i] = p;
-            t.m[i] = m;
-            t.v[i] = v;
-        }
-    }
-}
-
 template <class Arith>
 __global__ __launch_bounds__(kThreads) void adamw_fp32_kernel(const MultiF args)
 {
@@ -586,6 +516,7 @@ static Launch4 fill4(Multi4 &args, const lpmm_adamw4bit_tensor *tensors, int64_t
     int k = 0;
     uint64_t tiles = 0;
     bool aligned = true, allfull = true;
+    float step = 0.0f;
     args.tile_start[0] = 0;
     while (i < count && k < LPMM_MULTI_MAX) {
         const lpmm_adamw4bit_tensor &t = tensors[i];
@@ -607,7 +538,10 @@ static Launch4 fill4(Multi4 &args, const lpmm_adamw4bit_tensor *tensors, int64_t
         d.ms = t.m_scale;
         d.vs = t.v_scale;
         d.n = t.n;
-        per_tensor(t.step, d.k);
+        if (k != 0 && t.step == step)
+            memcpy(d.k, args.t[k - 1].k, sizeof d.k);
+        else
+            per_tensor(step = t.step, d.k);
         tiles += nt;
         args.tile_start[++k] = (uint32_t)tiles;
         ++i;
@@ -671,13 +605,7 @@ extern "C" int lpmm_nonfused_adamw4bit_step_multi(const lpmm_adamw4bit_tensor *t
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
     const float scalars[7] = {c.decay, c.w1, c.b2, c.w2, c.eps, 0.0f, 0.0f};
     return step_multi4<NonFusedArith>(tensors, count, qmap_m, qmap_v, scalars,
-                                      [=](float step, float (&k)[4]) {
-                                          const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, step);
-                                          k[0] = h.neg_step_size;
-                                          k[1] = h.bc2_sqrt;
-                                          k[2] = h.rbc2_sqrt;
-                                          k[3] = 0.0f;
-                                      },
+                                      [=](float step, float (&k)[4]) { NonFusedArith::per_tensor(beta1, beta2, lr, weight_decay, eps, step, k); },
                                       stream);
 }
 
@@ -697,60 +625,6 @@ extern "C" int lpmm_adamw4bit_step(float *p, const float *g, uint8_t *m_codes, u
     t.step = step;
     t.reserved = 0.0f;
     return lpmm_adamw4bit_step_multi(&t, 1, qmap_m, qmap_v, beta1, beta2, lr, weight_decay, eps, stream);
-}
-
-static int check_fp32(const lpmm_adamw_fp32_tensor *tensors, int64_t count, uintptr_t elt_align)
-{
-    LPMM_REQUIRE_PTR(tensors);
-    for (int64_t i = 0; i < count; ++i) {
-        const lpmm_adamw_fp32_tensor &t = tensors[i];
-        if (t.n < 0 || (t.n + kTileF - 1) / kTileF > 0x7fffffffLL)
-            return LPMM_ERR_SIZE;
-        if (t.n == 0)
-            continue;
-        LPMM_REQUIRE_PTR(t.p);
-        LPMM_REQUIRE_PTR(t.g);
-        LPMM_REQUIRE_PTR(t.m);
-        LPMM_REQUIRE_PTR(t.v);
-        LPMM_REQUIRE_ALIGN(t.p, elt_align);
-        LPMM_REQUIRE_ALIGN(t.g, elt_align);
-        LPMM_REQUIRE_ALIGN(t.m, elt_align);
-        LPMM_REQUIRE_ALIGN(t.v, elt_align);
-    }
-    return LPMM_OK;
-}
-
-// As fill4: the launch's tiles.
-template <class PerTensor>
-static uint32_t fill_fp32(MultiF &args, const lpmm_adamw_fp32_tensor *tensors, int64_t count, int64_t &i, PerTensor per_tensor)
-{
-    int k = 0;
-    uint64_t tiles = 0;
-    args.tile_start[0] = 0;
-    while (i < count && k < kMultiFMax) {
-        const lpmm_adamw_fp32_tensor &t = tensors[i];
-        if (t.n == 0) {
-            ++i;
-            continue;
-        }
-        const uint64_t nt = (uint64_t)((t.n + kTileF - 1) / kTileF);
-        if (tiles + nt > 0x7fffffffULL)
-            break;
-        TensorF &d = args.t[k];
-        d.p = t.p;
-        d.g = t.g;
-        d.m = t.m;
-        d.v = t.v;
-        d.n = t.n;
-        per_tensor(t.step, d.k);
-        tiles += nt;
-        args.tile_start[++k] = (uint32_t)tiles;
-        ++i;
-    }
-    args.count = k;
-    for (int j = k + 1; j <= kMultiFMax; ++j)
-        args.tile_start[j] = (uint32_t)tiles;
-    return (uint32_t)tiles;
 }
 
 template <class Arith, bool HALF = false, class PerTensor>
@@ -840,11 +714,7 @@ extern "C" int lpmm_nonfused_adamw4bit_fp32_step_multi(const lpmm_adamw4bit_tens
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
     const float scalars[7] = {c.decay, c.w1, c.b2, c.w2, c.eps, 0.0f, 0.0f};
     const auto per_tensor = [=](float step, float (&k)[4]) {
-        const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, step);
-        k[0] = h.neg_step_size;
-        k[1] = h.bc2_sqrt;
-        k[2] = h.rbc2_sqrt;
-        k[3] = 0.0f;
+        NonFusedArith::per_tensor(beta1, beta2, lr, weight_decay, eps, step, k);
     };
     return step_joined<NonFusedArith, NonFusedArith>(tensors, count, plain, plain_count, qmap_m, qmap_v, scalars, per_tensor, per_tensor,
                                                      stream);
@@ -877,11 +747,7 @@ extern "C" int lpmm_nonfused_update_multi(const lpmm_adamw_fp32_tensor *tensors,
     const float scalars[7] = {c.decay, c.w1, c.b2, c.w2, c.eps, 0.0f, 0.0f};
     return step_multi_fp32<NonFusedArith>(tensors, count, scalars,
                                           [=](float step, float (&k)[4]) {
-                                              const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, step);
-                                              k[0] = h.neg_step_size;
-                                              k[1] = h.bc2_sqrt;
-                                              k[2] = h.rbc2_sqrt;
-                                              k[3] = 0.0f;
+                                              NonFusedArith::per_tensor(beta1, beta2, lr, weight_decay, eps, step, k);
                                           },
                                           stream);
 }

@@ -96,6 +96,27 @@ inline NfHyper make_nf_hyper(double beta1, double beta2, double lr, double wd, d
     return h;
 }
 
+// The same for the tensors of a call one after another: the two powers of a step count, 0.1 us, are taken again only where it changes.
+class NfHypers {
+public:
+    NfHypers(double beta1, double beta2, double lr, double wd, double eps) : beta1_(beta1), beta2_(beta2), lr_(lr), wd_(wd), eps_(eps) {}
+    const NfHyper &at(float step)
+    {
+        if (!any_ || step != step_) {
+            h_ = make_nf_hyper(beta1_, beta2_, lr_, wd_, eps_, step);
+            step_ = step;
+            any_ = true;
+        }
+        return h_;
+    }
+
+private:
+    double beta1_, beta2_, lr_, wd_, eps_;
+    float step_ = 0.0f;
+    bool any_ = false;
+    NfHyper h_;
+};
+
 __device__ __forceinline__ float lerp_w(float a, float b, float w)
 {
     return (fabsf(w) < 0.5f) ? __builtin_fmaf(w, b - a, a) : __builtin_fmaf(w - 1.0f, b - a, b);

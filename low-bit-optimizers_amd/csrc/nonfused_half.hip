@@ -629,6 +629,7 @@ static int half_step_multi(const lpmm_adamw4bit_f16_tensor *tensors, int64_t cou
         LPMM_REQUIRE_ALIGN(t.v_max1, 2);
     }
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
+    NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
     MultiH args;
     args.decay = c.decay;
     args.w1 = c.w1;
@@ -668,7 +669,7 @@ static int half_step_multi(const lpmm_adamw4bit_f16_tensor *tensors, int64_t cou
             d.ms = static_cast<h16 *>(t.m_max1);
             d.vs = static_cast<h16 *>(t.v_max1);
             d.n = t.n;
-            const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, t.step);
+            const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             d.rbc2_sqrt = h.rbc2_sqrt;
@@ -882,6 +883,7 @@ extern "C" int lpmm_nonfused_update_f16_multi(const lpmm_adamw_fp32_tensor *tens
         LPMM_REQUIRE_ALIGN(t.v, 2);
     }
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
+    NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
     MultiHPlain args;
     args.decay = c.decay;
     args.w1 = c.w1;
@@ -907,7 +909,7 @@ extern "C" int lpmm_nonfused_update_f16_multi(const lpmm_adamw_fp32_tensor *tens
             d.m = reinterpret_cast<h16 *>(t.m);
             d.v = reinterpret_cast<h16 *>(t.v);
             d.n = t.n;
-            const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, t.step);
+            const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             tiles += nt;

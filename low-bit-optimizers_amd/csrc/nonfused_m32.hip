@@ -197,6 +197,7 @@ extern "C" int lpmm_nonfused_adamw_v4bit_step_multi(const lpmm_adamw_v4bit_tenso
         LPMM_REQUIRE_ALIGN(t.v_max1, 4);
     }
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
+    NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
     MultiV4 args;
     args.decay = c.decay;
     args.w1 = c.w1;
@@ -224,7 +225,7 @@ extern "C" int lpmm_nonfused_adamw_v4bit_step_multi(const lpmm_adamw_v4bit_tenso
             d.vc = t.v_codes;
             d.vs = t.v_max1;
             d.n = t.n;
-            const NfHyper h = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, t.step);
+            const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             d.rbc2_sqrt = h.rbc2_sqrt;

@@ -232,6 +232,12 @@ __device__ __forceinline__ uint32_t load_u16_for(const uint16_t *p) { return KEE
 template <bool KEEP>
 __device__ __forceinline__ uint32_t load_u32_for(const uint32_t *p) { return KEEP ? *p : load_u32(p); }
 
+// Tensors with fp32 states that go with the launches of a call; `next`: the first that has not gone yet.
+struct PlainSet {
+    const lpmm_adamw_fp32_tensor *tensors;
+    int64_t count, next;
+};
+
 // One launch's tensors with the tile shapes of either pass (they differ: pass_rows_policy), and its workgroups.
 struct R1Launch {
     MultiR1 update, requant;
@@ -269,7 +275,8 @@ int launch_small_vectors(const lpmm_rank1_small_vector *const *vectors, int64_t 
 // float work arrays (rank1_any_half sets them up and writes the halfs out)
 int rank1_any_step_multi(const lpmm_rank1_any_tensor *tensors, int64_t count, AnyKind kind, uint32_t m_lg, const float *qmap_m,
                          int bits_m, const void *table_m, const float *qmap_v, int bits_v, const void *table_v, double beta1,
-                         double beta2, double lr, double weight_decay, double eps, int passes, void *stream);
+                         double beta2, double lr, double weight_decay, double eps, int passes, void *stream,
+                         PlainSet *plain = nullptr);
 int rank1_any_half(const lpmm_rank1_any_tensor *tensors, int64_t count, const float *qmap_m, const float *qmap_v, double beta1,
                    double beta2, double lr, double weight_decay, double eps, void *stream);
 int rank1_step_multi_half(const lpmm_nonfused_rank1_tensor *tensors, int64_t count, const float *qmap_m,

@@ -751,18 +751,42 @@ PyObject *plan_rest(PyObject *self, void *)
     return rest;
 }
 
-// The tensors with fp32 states that share the launches of the quantised tensors b (lpmm_adamw4bit_fp32_step_multi and its
-// non-fused form), or null.  Decided here: a loop over the batches in Python cost every step 1.0 us, of 34 on three layers of width 128.
+// Can a batch's launches take tensors with fp32 states along, and how well: 2, the one-pass kernels, 1, the launch that clears the
+// two-pass kernels' statistics, 0.
+int takes_plain(const Batch &b)
+{
+    switch (b.kind) {
+    case kFused4:
+    case kFlat:
+        return 2;
+    case kRank1:
+    case kNd:
+    case kRank1M32:
+    case kRank1Bits:
+    case kRank1Wide:
+        return b.items.empty() ? 0 : 1;
+    case kAny:
+        return b.flag != LPMM_RANK1_HALF ? 1 : 0;
+    default:
+        return 0;
+    }
+}
+
+// The tensors with fp32 states that share the launches of the quantised tensors b (lpmm_adamw4bit_fp32_step_multi, its
+// non-fused form, lpmm_nonfused_rank1_fp32_step_multi), or null; they go with the first batch that takes them best.
+// Decided here: a loop over the batches in Python cost every step 1.0 us, of 34 on three layers of width 128.
 const Batch *joined(const std::vector<Batch> &batches, const Batch &b)
 {
-    if (b.kind != kFused4 && b.kind != kFlat)
+    const int best = takes_plain(b);
+    if (best == 0)
         return nullptr;
     const Batch *plain = nullptr;
     for (const Batch &other : batches) {
         if (other.device != b.device)
             continue;
-        if (other.kind == b.kind && &other < &b)
-            return nullptr;  // they go with the first of several
+        const int takes = takes_plain(other);
+        if (takes > best || (takes == best && &other < &b))
+            return nullptr;
         if (other.kind == kPlain)
             plain = &other;
     }
@@ -794,8 +818,8 @@ void join_matrices(std::vector<Batch> &batches)
 
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
-// that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's, and
-// flag 1 in the latter's own batch.
+// that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
+// a fold, in that of the flag), and flag 1 in the latter's own batch.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
     Plan *plan = reinterpret_cast<Plan *>(self);
@@ -825,10 +849,11 @@ PyObject *plan_start(PyObject *self, PyObject *)
             for (const Batch &other : *plan->batches)
                 elsewhere = elsewhere || joined(*plan->batches, other) == &b;
         PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,
-                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : b.flag, (Py_ssize_t)b.items.size(),
+                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.flag,
+                                    (Py_ssize_t)b.items.size(),
                                     (unsigned long long)(uintptr_t)b.records.data(),
                                     (unsigned long long)(uintptr_t)(plain != nullptr ? plain->records.data() : b.second.data()),
-                                    plain != nullptr ? (unsigned long long)plain->items.size()
+                                    plain != nullptr && b.kind != kNd ? (unsigned long long)plain->items.size()
                                                      : (unsigned long long)(uintptr_t)b.fold.data());
         if (t == nullptr || PyList_Append(out, t) != 0) {
             Py_XDECREF(t);

@@ -68,6 +68,8 @@ PROTOTYPES = {
     "lpmm_nonfused_adamw4bit_f16_step_multi": (_int, [_vp, _i64, _vp, _vp] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw4bit_rank1_f16_step_multi": (_int, [_vp, _i64, _vp, _vp] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw4bit_rank1_pass_multi": (_int, [_vp, _i64, _vp, _vp] + [_d] * 5 + [_int, _vp]),
+    "lpmm_nonfused_rank1_fp32_step_multi": (_int, [_int, _vp, _vp, _i64, _vp, _i64, _i64, _vp, _int, _vp, _vp, _int, _vp]
+                                            + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw4bit_rank1_nd_step_multi": (_int, [_vp, _vp, _i64, _vp, _vp] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw_v4bit_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
     "lpmm_nonfused_adamw_v4bit_rank1_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
@@ -200,6 +202,10 @@ def factored_workspace():
 (WALK_FUSED4, WALK_PLAIN, WALK_FLAT, WALK_RANK1, WALK_ND, WALK_FLAT_M32, WALK_RANK1_M32, WALK_RANK1_BITS, WALK_RANK1_WIDE, WALK_SGD4,
  WALK_SGD_PLAIN, WALK_ANY, WALK_ND_ANY, WALK_HALF_PLAIN, WALK_HALF_FLAT, WALK_HALF_RANK1, WALK_FACTORED,
  WALK_FACTORED_ANY) = range(18)
+
+
+# the two-pass steps by kind of record (LPMM_STEP_* of include/lpmm_hip.h); WALK_ANY: plus the kind of its records
+STEP_OF = {WALK_RANK1: 0, WALK_RANK1_BITS: 1, WALK_ND: 2, WALK_RANK1_M32: 3, WALK_RANK1_WIDE: 4, WALK_ANY: 8}
 
 
 def check(status, what):

@@ -269,8 +269,8 @@ class AdamW(LowBitOptimizer):
         hyper = (beta1, beta2, group["lr"], group["weight_decay"], group["eps"])
         lib = _native.lib()
         for k, (kind, index, qm, qv, flag, count, records, second, fold) in enumerate(plan.start()):
-            if flag and kind == _native.WALK_PLAIN:
-                continue  # these go with the quantised tensors
+            if count == 0 or (flag and kind == _native.WALK_PLAIN):
+                continue  # these go with other tensors
             with torch.cuda.device(index):
                 stream = _native.current_stream(index)
                 qm_ptr, qv_ptr = (None if q is None else q.data_ptr() for q in (qm, qv))
@@ -309,18 +309,10 @@ class AdamW(LowBitOptimizer):
 
     @staticmethod
     def _launch_walk_rank1(plan, k, kind, qm, qv, flag, count, records, second, fold, hyper, routes, stream):
-        """Two passes: a state's statistics (and wide scales) are the new ones once its launch is on the stream."""
+        """Two passes: a state's statistics (and wide scales) are the new ones once its launch is on the stream.  second, fold: address
+        and number of the tensors with fp32 states that go along (beside a fold: second, flag)."""
         lib, most = _native.lib(), _native.RANK1_MULTI_MAX
         qv_ptr = qv.data_ptr()
-
-        def code_tables():
-            return [code_table(q, md["b"]).data_ptr() for q, md in ((qm, routes.m), (qv, routes.v))]
-
-        if kind == _native.WALK_ND:
-            st = lib.lpmm_nonfused_adamw4bit_rank1_nd_step_multi(records, fold, count, qm.data_ptr(), qv_ptr, *hyper, stream)
-            _native.check(st, "non-fused 4-bit AdamW step on tensors of more than two dimensions")
-            plan.commit(k, 0, count)
-            return
         if kind == _native.WALK_ND_ANY:
             # the kernels for any column count write their codes to new arrays: one launch's worth of them at a time
             size = _native.RANK1_ANY_TENSOR.itemsize
@@ -336,45 +328,55 @@ class AdamW(LowBitOptimizer):
                         _native.check(st, "rank1_small_fold_scale_multi")
                 plan.commit(k, i, n)
             return
-        if kind == _native.WALK_RANK1:
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw4bit_rank1_step_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, stream)
-            size = _native.NONFUSED_RANK1_TENSOR.itemsize
-        elif kind == _native.WALK_RANK1_M32:
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw_v4bit_rank1_step_multi(table, n, qv_ptr, *hyper, stream)
-            size = _native.RANK1_V4BIT_TENSOR.itemsize
-        elif kind == _native.WALK_ANY:
-            bits, tables, group = (4, 4), (None, None), 128
-            if flag == _native.RANK1_CODES8:
-                bits, tables = (routes.m["b"], routes.v["b"]), code_tables()
-            elif flag == _native.RANK1_CODES4:
+        if kind == _native.WALK_HALF_RANK1 or (kind == _native.WALK_ANY and flag == _native.RANK1_HALF):
+            half_any = kind == _native.WALK_ANY
+            size = (_native.RANK1_ANY_TENSOR if half_any else _native.NONFUSED_RANK1_F16_TENSOR).itemsize
+            for i in range(0, count, most):
+                n = min(most, count - i)
+                plan.prepare(k, i, n)
+                if half_any:
+                    st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(records + i * size, n, flag, 128, qm.data_ptr(), 4, None, qv_ptr, 4,
+                                                                      None, *hyper, 3, stream)
+                else:
+                    st = lib.lpmm_nonfused_adamw4bit_rank1_f16_step_multi(records + i * size, n, qm.data_ptr(), qv_ptr, *hyper, stream)
+                _native.check(st, "non-fused AdamW step on float16 parameters (rank-1 second moment)")
+                plan.commit(k, i, n)
+            return
+        step, plain, plain_count, folds, group, size = _native.STEP_OF[kind], second, fold, None, 128, 0
+        bits, most = kind == _native.WALK_RANK1_BITS, count
+        if kind == _native.WALK_ND:
+            plain_count, folds = flag, fold
+        elif kind == _native.WALK_RANK1_WIDE:
+            group = routes.m["gp_sz"]
+        elif kind == _native.WALK_ANY:  # new codes: one launch's worth at a time
+            step += flag
+            bits, most, size = flag == _native.RANK1_CODES8, _native.RANK1_MULTI_MAX, _native.RANK1_ANY_TENSOR.itemsize
+            if flag == _native.RANK1_CODES4:
                 group = routes.m["gp_sz"]
-
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, flag, group, qm.data_ptr(), bits[0], tables[0], qv_ptr,
-                                                                    bits[1], tables[1], *hyper, 3, stream)
-            size = _native.RANK1_ANY_TENSOR.itemsize
-        elif kind == _native.WALK_HALF_RANK1:
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw4bit_rank1_f16_step_multi(table, n, qm.data_ptr(), qv_ptr, *hyper, stream)
-            size = _native.NONFUSED_RANK1_F16_TENSOR.itemsize
-        elif kind == _native.WALK_RANK1_BITS:
-            tables = code_tables()
-
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw_bits_rank1_step_multi_table(
-                    table, n, qm.data_ptr(), routes.m["b"], tables[0], qv_ptr, routes.v["b"], tables[1], *hyper, stream)
-            size = _native.NONFUSED_RANK1_TENSOR.itemsize
-        else:
-            def run(table, n):
-                return lib.lpmm_nonfused_adamw4bit_rank1_mgroup_step_multi(table, n, qm.data_ptr(), qv_ptr, routes.m["gp_sz"],
-                                                                           *hyper, stream)
-            size = _native.RANK1_MGROUP_TENSOR.itemsize
+        qm_ptr = qm.data_ptr() if qm is not None else None
+        coding = (qm_ptr, 4, None, qv_ptr, 4, None)
+        if bits:
+            coding = (qm_ptr, routes.m["b"], code_table(qm, routes.m["b"]).data_ptr(),
+                      qv_ptr, routes.v["b"], code_table(qv, routes.v["b"]).data_ptr())
         for i in range(0, count, most):
-            n = min(most, count - i)
+            n, table = min(most, count - i), records + i * size
             plan.prepare(k, i, n)
-            _native.check(run(records + i * size, n), "non-fused AdamW step (rank-1 second moment)")
+            if plain_count:
+                st = lib.lpmm_nonfused_rank1_fp32_step_multi(step, table, folds, n, plain, plain_count, group, *coding, *hyper, stream)
+                plain_count = 0
+            elif kind == _native.WALK_ND:
+                st = lib.lpmm_nonfused_adamw4bit_rank1_nd_step_multi(table, folds, n, qm_ptr, qv_ptr, *hyper, stream)
+            elif kind == _native.WALK_RANK1:
+                st = lib.lpmm_nonfused_adamw4bit_rank1_step_multi(table, n, qm_ptr, qv_ptr, *hyper, stream)
+            elif kind == _native.WALK_RANK1_M32:
+                st = lib.lpmm_nonfused_adamw_v4bit_rank1_step_multi(table, n, qv_ptr, *hyper, stream)
+            elif kind == _native.WALK_RANK1_BITS:
+                st = lib.lpmm_nonfused_adamw_bits_rank1_step_multi_table(table, n, *coding, *hyper, stream)
+            elif kind == _native.WALK_RANK1_WIDE:
+                st = lib.lpmm_nonfused_adamw4bit_rank1_mgroup_step_multi(table, n, qm_ptr, qv_ptr, group, *hyper, stream)
+            else:
+                st = lib.lpmm_nonfused_adamw_rank1_any_step_multi(table, n, flag, group, *coding, *hyper, 3, stream)
+            _native.check(st, "non-fused AdamW step (rank-1 second moment)")
             plan.commit(k, i, n)
 
     # ---- fused path (lpmm/optim/adamw.py:439-561) ---------------------------------------

@@ -502,3 +502,39 @@ def test_states_under_equal_keys_that_are_other_strings(case):
         assert torch.equal(p.detach(), q.detach())
         a, b = _state(sides[0][1], p), {k: v for k, v in opt.state[q].items() if torch.is_tensor(v)}
         assert all(torch.equal(a[k], v) for k, v in b.items())
+
+
+@pytest.mark.parametrize("config,shape", [("default.yml", (17, 256)), ("default.yml", (17, 32, 3, 3)), ("default.yml", (34, 192)),
+                                          ("default.yml", (33, 130)), ("2nd_moment_only_default.yml", (17, 256)),
+                                          ("1st_moment_group_256.yml", (17, 256)), ("default_8b.yml", (17, 256)),
+                                          ("default_8b.yml", (33, 130))])
+@pytest.mark.parametrize("matrices,vectors", [(1, 1), (33, 63), (97, 129)])
+def test_float_states_beside_the_clearing(config, shape, matrices, vectors, monkeypatch):
+    """Tensors with fp32 states go with the launch that clears the two-pass kernels' statistics: more of either than one launch takes
+    (192 ranges, two a matrix; 64 tensors), against the loops."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    sides = []
+    for _ in range(2):
+        gen = torch.Generator(device="cuda").manual_seed(3)
+        shapes = [(2 + 37 * k % 3000,) for k in range(vectors)] + [shape] * matrices
+        params = [torch.nn.Parameter(torch.randn(s, device="cuda", generator=gen) * 0.1) for s in shapes]
+        sides.append((params, lpmm.optim.AdamW(params, lr=1e-2, eps=1e-3, qconfig=path)))
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    for step in range(3):
+        grads = [torch.randn(p.shape, device="cuda", generator=gen) * 0.1 for p in sides[0][0]]
+        for serve, (params, opt) in zip((True, False), sides):
+            for p, g in zip(params, grads):
+                p.grad = g
+            with monkeypatch.context() as patch:
+                native = _Native(_native, serve)
+                patch.setattr(adamw, "_native", native)
+                opt.step()
+                assert step < 2 or native.rest == (0 if serve else len(params))
+    for p, q in zip(sides[0][0], sides[1][0]):
+        assert torch.equal(p, q)
+        a, b = _state(sides[0][1], p), _state(sides[1][1], q)
+        assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
