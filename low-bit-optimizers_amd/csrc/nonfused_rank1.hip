@@ -35,6 +35,7 @@
 #include "rank1_tiles.hpp"
 
 #include <cstring>
+#include <type_traits>
 
 namespace lpmm {
 
@@ -161,8 +162,8 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
 #endif
 // 4 waves per SIMD, up to 128 registers: the first pass's operands stay live across the prologue and
 // the lane's column statistics across the passes (with 5 or 6 the compiler spills or re-reads)
-template <int MODE, bool FOLD, bool KEEP>
-__global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
+template <int MODE, bool FOLD, bool KEEP, int N>
+__global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(const MultiR1N<N> args, const float *__restrict__ qmap_m,
                                                                 const float *__restrict__ qmap_v)
 {
     __shared__ __align__(16) uint32_t lds[(kColExtra + kMaxWide * kRedSlotWords * 4) / 4 + kRowSlots];
@@ -323,8 +324,8 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
 }
 
 // MWIDE: the first moment's groups are wider than 128 values; its codes are written here too.
-template <bool MWIDE, bool FOLD>
-__global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1 args, const float *__restrict__ qmap_m,
+template <bool MWIDE, bool FOLD, int N>
+__global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<N> args, const float *__restrict__ qmap_m,
                                                                  const float *__restrict__ qmap_v)
 {
     __shared__ __align__(16) uint32_t lds[(kColExtra + 2 * kColBytes) / 4];
@@ -684,20 +685,20 @@ static Matrix matrix_of(int64_t rows, int64_t cols, bool can_fold)
     return fold ? Matrix{rows / 2, 2 * blocks - 1, true} : Matrix{rows, blocks, false};
 }
 
-template <int MODE, bool FOLD>
-static void launch_rank1_passes(const R1Launch &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
+template <int MODE, bool FOLD, int N>
+static void launch_rank1_passes(const R1LaunchN<N> &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
 {
     if (passes & 1) {
-        const auto update = l.keep ? rank1_update_kernel<MODE, FOLD, true> : rank1_update_kernel<MODE, FOLD, false>;
+        const auto update = l.keep ? rank1_update_kernel<MODE, FOLD, true, N> : rank1_update_kernel<MODE, FOLD, false, N>;
         hipLaunchKernelGGL(update, dim3(l.update_tiles), dim3(kThreads), 0, stream, l.update, qmap_m, qmap_v);
     }
     if (passes & 2)
-        hipLaunchKernelGGL((rank1_requant_kernel<MODE == kMCodesWide, FOLD>), dim3(l.requant_tiles), dim3(kThreads), 0, stream,
+        hipLaunchKernelGGL((rank1_requant_kernel<MODE == kMCodesWide, FOLD, N>), dim3(l.requant_tiles), dim3(kThreads), 0, stream,
                            l.requant, qmap_m, qmap_v);
 }
 
-template <int MODE>
-static void launch_rank1(const R1Launch &l, bool folded, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
+template <int MODE, int N>
+static void launch_rank1(const R1LaunchN<N> &l, bool folded, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
 {
     if constexpr (MODE == kMCodes128)
         if (folded)
@@ -845,21 +846,22 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
 
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
     NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
-    R1Launch l;
-    MultiR1 &args = l.update;
-    args.decay = c.decay;
-    args.w1 = c.w1;
-    args.b2 = c.b2;
-    args.w2 = c.w2;
-    args.eps = c.eps;
     int64_t i = 0;
-    while (i < count) {
+    // one launch's worth of tensors from i on
+    const auto launch = [&](auto &l) -> int {
+        constexpr int kMost = std::decay_t<decltype(l)>::kMax;
+        auto &args = l.update;
+        args.decay = c.decay;
+        args.w1 = c.w1;
+        args.b2 = c.b2;
+        args.w2 = c.w2;
+        args.eps = c.eps;
         int k = 0;
         // what this launch will hold decides its tiles' rows
         LaunchKind kind = {half_io, M32, bits_m != 4, 0, {false, false}};
         const auto each = [&](auto &&f) {
             int k = 0;
-            for (int64_t j = i; j < count && k < kR1Max; ++j)
+            for (int64_t j = i; j < count && k < kMost; ++j)
                 if (tensors[j].rows != 0 && tensors[j].cols != 0) {
                     f(tensors[j]);
                     ++k;
@@ -883,14 +885,14 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             kind.spread[1] = blocks[1] < kSpreadBelow;
         }
         uint64_t tiles = 0, tiles2 = 0;
-        uint32_t start2[kR1Max + 1] = {0};
-        TileShape shape2[kR1Max];
-        float *scale2[kR1Max];  // the column statistics of the second pass
-        const lpmm_rank1_small_vector *between[kR1Max];
+        uint32_t start2[kMost + 1] = {0};
+        TileShape shape2[kMost];
+        float *scale2[kMost];  // the column statistics of the second pass
+        const lpmm_rank1_small_vector *between[kMost];
         int betweens = 0;
         bool folded = false;  // does a tensor of this launch have folded rows
         args.tile_start[0] = 0;
-        while (i < count && k < kR1Max) {
+        while (i < count && k < kMost) {
             const Record &t = tensors[i];
             if (t.rows == 0 || t.cols == 0) {
                 ++i;
@@ -939,10 +941,10 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         if (k == 0) {
             if (i < count)
                 return LPMM_ERR_SIZE;  // a single tensor with more tiles than a grid holds
-            continue;
+            return LPMM_OK;
         }
         args.count = k;
-        for (int j = k + 1; j <= kR1Max; ++j) {
+        for (int j = k + 1; j <= kMost; ++j) {
             args.tile_start[j] = (uint32_t)tiles;
             start2[j] = (uint32_t)tiles2;
         }
@@ -955,18 +957,28 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         l.update_tiles = (uint32_t)tiles;
         l.requant_tiles = (uint32_t)tiles2;
         l.keep = kind.values <= kKeepValues;
-        if (general) {
-            const AnyKind any = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
-            launch_rank1_any(l, *out, qmap_m, qmap_v, any, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
-                             static_cast<const uint32_t *>(table_v), passes, s);
-        } else if (half_io) {
-            launch_rank1_half(l, qmap_m, qmap_v, s);
-        } else if (ragged || (MODE == kMCodesWide && m_lg == 0)) {
-            launch_rank1_ragged(l, qmap_m, qmap_v, s);
-        } else if (bits_m != 4) {
-            launch_rank1_bits(l, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
-                              static_cast<const uint32_t *>(table_v), s);
-        } else if (betweens != 0) {
+        if constexpr (kMost == kR1Max) {
+            if (general) {
+                const AnyKind any = half_io ? kAnyHalf : M32 ? kAnyFloatM : bits_m != 4 ? kAnyBits : kAnyCodes4;
+                launch_rank1_any(l, *out, qmap_m, qmap_v, any, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
+                                 static_cast<const uint32_t *>(table_v), passes, s);
+                return launch_status();
+            }
+            if (half_io) {
+                launch_rank1_half(l, qmap_m, qmap_v, s);
+                return launch_status();
+            }
+            if (ragged || (MODE == kMCodesWide && m_lg == 0)) {
+                launch_rank1_ragged(l, qmap_m, qmap_v, s);
+                return launch_status();
+            }
+            if (bits_m != 4) {
+                launch_rank1_bits(l, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
+                                  static_cast<const uint32_t *>(table_v), s);
+                return launch_status();
+            }
+        }
+        if (betweens != 0) {
             launch_rank1<MODE>(l, folded, qmap_m, qmap_v, 1, s);
             const int st = launch_small_vectors(between, betweens, s);
             if (st != LPMM_OK)
@@ -975,7 +987,29 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         } else {
             launch_rank1<MODE>(l, MODE == kMCodes128 && folded, qmap_m, qmap_v, passes, s);
         }
-        const int st = launch_status();
+        return launch_status();
+    };
+    // More tensors a launch where they are small: a launch's start and end, 8 to 10 us of both passes, are then a good part of it.
+    // Steps with 32 -> 64 a launch: 64 of 512 x 512 71.5 -> 67, of 800 x 1024 (52M values) 187 -> 174, of 1024 x 1024 229.5 -> 221, of 1024 x
+    // 2048 426 -> 422; 128 of 448 x 448 132 -> 120, of 192 x 128 x 3 x 3 156 -> 140; from 200M values on nothing, from 270M on 1 to 2 %
+    // slower: the second pass finds less of what the first has read.
+    constexpr double kManyValues = 80e6;
+    const bool own_kernels = MODE == kMCodes128 && !general && !half_io && bits_m == 4;
+    R1Launch l;
+    R1LaunchN<kR1Many> many;
+    while (i < count) {
+        double values = 0;
+        int held = 0;
+        for (int64_t j = i; own_kernels && j < count && held < kR1Many; ++j)
+            if (tensors[j].rows != 0 && tensors[j].cols != 0) {
+                values += (double)tensors[j].rows * (double)tensors[j].cols;
+                ++held;
+            }
+        int st;
+        if constexpr (MODE == kMCodes128)
+            st = held > kR1Max && values <= kManyValues ? launch(many) : launch(l);
+        else
+            st = launch(l);
         if (st != LPMM_OK)
             return st;
     }

@@ -10,6 +10,7 @@ constexpr int kThreads = 256;
 constexpr int kEltsPerLane = 8;
 constexpr int kDppRows = kThreads / 16;  // 128-column groups a workgroup handles per pass
 constexpr int kR1Max = 32;               // tensors per launch
+constexpr int kR1Many = 64;              // of small ones, in the kernels of nonfused_rank1.hip
 // Tile policy: widest tile (lg of 128-column groups), tensor rows per workgroup (more where one pass
 // of a narrow tile covers more), workgroups taken to be resident together.
 #ifndef LPMM_R1_LG
@@ -75,22 +76,27 @@ struct TensorR1 {
 // codes, bit-identically, and writes its codes -- what both passes do for the second moment).
 enum MomentMode { kMCodes128 = 0, kMFloat = 1, kMCodesWide = 2 };
 
-struct MultiR1 {
-    TensorR1 t[kR1Max];
-    uint32_t tile_start[kR1Max + 1];  // prefix sum of tiles per tensor; unused slots hold the total
+template <int N>
+struct MultiR1N {
+    static constexpr int kMax = N;
+    TensorR1 t[N];
+    uint32_t tile_start[N + 1];  // prefix sum of tiles per tensor; unused slots hold the total
     int count;
     float decay, w1, b2, w2, eps;
 };
+using MultiR1 = MultiR1N<kR1Max>;
 
 static_assert(sizeof(MultiR1) + 3 * sizeof(void *) + 2 * sizeof(int) <= 4096, "kernel arguments exceed 4 KB");
-static_assert(kR1Max <= kWave, "one tile_start entry per lane");
+static_assert(sizeof(MultiR1N<kR1Many>) + 2 * sizeof(void *) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
+static_assert(kR1Max <= kWave && kR1Many <= kWave, "one tile_start entry per lane");
 
 // tensor of this workgroup (uniform): the number of later tensors whose first tile is not
 // after this one
-__device__ __forceinline__ int find_tensor(const MultiR1 &args)
+template <int N>
+__device__ __forceinline__ int find_tensor(const MultiR1N<N> &args)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const bool started = lane + 1 < kR1Max && args.tile_start[lane + 1] <= blockIdx.x;
+    const bool started = lane + 1 < N && args.tile_start[lane + 1] <= blockIdx.x;
     return __popcll(__ballot(started));
 }
 
@@ -239,11 +245,14 @@ struct PlainSet {
 };
 
 // One launch's tensors with the tile shapes of either pass (they differ: pass_rows_policy), and its workgroups.
-struct R1Launch {
-    MultiR1 update, requant;
+template <int N>
+struct R1LaunchN {
+    static constexpr int kMax = N;
+    MultiR1N<N> update, requant;
     uint32_t update_tiles, requant_tiles;
     bool keep;  // the update pass leaves what the second pass reads again in the cache
 };
+using R1Launch = R1LaunchN<kR1Max>;
 
 // The launches of the other kernel families (defined next to their kernels).
 void launch_rank1_bits(const R1Launch &l, const float *qmap_m, const float *qmap_v, int bits_m,
