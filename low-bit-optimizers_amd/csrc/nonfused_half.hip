@@ -448,7 +448,7 @@ __global__ __launch_bounds__(kThreads, 6) void rank1_update_half_kernel(const Mu
             atomicMax(red + k * 16, __float_as_uint((float)vtop[k >> 1][k & 1]));
     }
     __syncthreads();
-    flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
+    flush_row_maxima(rowred, t.tile, q, drow, t.rows, t.row_new);
     // column j of the tile = element k of lane l of slot s
     for (int j = threadIdx.x; j < q.wide * kGroup; j += kThreads) {
         const int w = j & (kGroup - 1);

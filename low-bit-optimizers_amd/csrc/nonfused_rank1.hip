@@ -34,6 +34,7 @@
 #include "lpmm_plain.hpp"
 #include "rank1_tiles.hpp"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -115,19 +116,43 @@ static void launch_clear_plain(const ClearRanges<kClearMax> &ranges, int n, uint
                            ranges_from<kClearJoined>(ranges), args, blocks, clears);
 }
 
+// What a kernel's tensors may be beside matrices of whole column blocks: double rows, which end with a whole row, or rows of several tensor
+// rows, the last of which may be a part (rank1_tiles.hpp: Fold).
+enum FoldKind : int { kNoFold = 0, kDoubles = 1, kWraps = 2 };
+
 // operands of one pass of a DPP row, as loaded
 struct PassRegs {
     float4 a0, a1, b0, b1;
     float4 c0, c1;  // fp32 first moment only
     uint32_t m0, m1, v0, v1;
-    float sm, ro, ro1;  // ro1: the second half's row statistic (folded rows; otherwise ro)
+    float sm, ro, ro1;  // ro1: the second tensor row's statistic (folded rows; otherwise ro)
 };
 
-template <int MODE, bool FOLD, bool KEEP>
-__device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uint32_t cg, int lane16, int64_t r, PassRegs &x)
+template <int MODE, int FOLD, bool KEEP>
+__device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, const FoldSpan &span, uint32_t cg, int lane16, int64_t r,
+                                           PassRegs &x)
 {
     const int64_t grp = r * f.col_blocks + cg;
     const int64_t gbase = grp * kGroup;
+    if (FOLD == kWraps) {
+        // runs beyond the end read the last one
+        const int64_t last = f.values - 4, oa = gbase + lane16 * 4, ob = oa + 64;
+        const int64_t a = oa < last ? oa : last, b = ob < last ? ob : last;
+        x.a0 = load4(t.p + a);
+        x.a1 = load4(t.p + b);
+        x.b0 = load4_for<KEEP>(t.g + a);
+        x.b1 = load4_for<KEEP>(t.g + b);
+        x.m0 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (a >> 1)));
+        x.m1 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (b >> 1)));
+        x.sm = t.ms[a >> 7];
+        x.v0 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (a >> 1)));
+        x.v1 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (b >> 1)));
+        int64_t r0, r1;
+        fold_rows(f, span, r, r0, r1);
+        x.ro = t.row_old[r0];
+        x.ro1 = t.row_old[r1];
+        return;
+    }
     const float *pp = t.p + gbase + lane16 * 4;
     const float *gp = t.g + gbase + lane16 * 4;
     x.a0 = load4(pp);
@@ -148,10 +173,10 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
     x.v0 = load_u16_for<KEEP>(vcp);
     x.v1 = load_u16_for<KEEP>(vcp + 16);
     if (FOLD) {
-        int64_t r0, r1;
-        fold_rows(f, r, cg, r0, r1);
-        x.ro = t.row_old[r0];
-        x.ro1 = t.row_old[r1];
+        uint32_t halves[2];
+        double_halves(f, cg, halves);
+        x.ro = t.row_old[(r << f.lg) + halves[0]];
+        x.ro1 = t.row_old[(r << f.lg) + halves[1]];
     } else {
         x.ro = x.ro1 = t.row_old[r];
     }
@@ -162,18 +187,20 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, uin
 #endif
 // 4 waves per SIMD, up to 128 registers: the first pass's operands stay live across the prologue and
 // the lane's column statistics across the passes (with 5 or 6 the compiler spills or re-reads)
-template <int MODE, bool FOLD, bool KEEP, int N>
+template <int MODE, int FOLD, bool KEEP, int N>
 __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(const MultiR1N<N> args, const float *__restrict__ qmap_m,
                                                                 const float *__restrict__ qmap_v)
 {
-    __shared__ __align__(16) uint32_t lds[(kColExtra + kMaxWide * kRedSlotWords * 4) / 4 + kRowSlots];
+    constexpr int kSlots = FOLD == kWraps ? kFoldSlots : kRowSlots;
+    static_assert(!FOLD || MODE == kMCodes128, "folded rows: 4-bit first moments in groups of 128 values");
+    __shared__ __align__(16) uint32_t lds[(kColExtra + kMaxWide * kRedSlotWords * 4) / 4 + kSlots];
     uint32_t *colred = lds + kColExtra / 4;
     uint32_t *rowred = colred + kMaxWide * kRedSlotWords;
     const int lo = find_tensor(args);
     const TensorR1 &t = args.t[lo];
     const uint32_t tl = blockIdx.x - args.tile_start[lo];
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
-    const Fold f = fold_of<FOLD>(t);
+    const Fold f = fold_of<FOLD != kNoFold>(t);
     const Geometry q = geometry(t.tile, f.col_blocks, tl, drow);
     const int64_t cols = (int64_t)f.col_blocks * kGroup;
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
@@ -196,12 +223,14 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
     // No branch around the first pass's loads: behind one the compiler waits for all of them before the LDS writes, as the path without
     // them has nothing else to count.  A DPP row without work loads what is there.
     PassRegs x;
-    pass_fetch<MODE, FOLD, KEEP>(t, f, row_live ? q.cg : f.col_blocks - 1u, lane16, q.row0 < f.rows ? q.row0 : f.rows - 1, x);
+    const uint32_t cg = row_live ? q.cg : f.col_blocks - 1u;
+    const FoldSpan span = FOLD == kWraps ? fold_span(f, cg) : FoldSpan{0, kGroup};
+    pass_fetch<MODE, FOLD, KEEP>(t, f, span, cg, lane16, q.row0 < f.rows ? q.row0 : f.rows - 1, x);
     lds_fill_store(lds, fill);
     for (int j = threadIdx.x; j < kMaxWide * (int)kRedSlotWords; j += kThreads)
         colred[j] = 0u;
-    if (threadIdx.x < kRowSlots)
-        rowred[threadIdx.x] = 0u;
+    for (int j = threadIdx.x; j < kSlots; j += kThreads)
+        rowred[j] = 0u;
 #pragma unroll
     for (int i = 0; i < kColPerThread; ++i)
         lds[kColOld / 4 + threadIdx.x + i * kThreads] = co_in[i];
@@ -219,7 +248,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
 
     if (MODE == kMCodes128 && tl == 0) {
         const float z[kEltsPerLane] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        const int64_t n = f.rows * cols;
+        const int64_t n = (f.values + kGroup - 1) / kGroup * kGroup;
         write_padding(t.mc, n, (n + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP,
                       encode8_plain(lds, kLdsQ0, kind_m, z));
     }
@@ -228,21 +257,27 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
     if (row_live) {
         const uint32_t co_off = kColOld + (slot * kGroup + lane16 * 4) * 4;
         uint32_t *red = colred + slot * kRedSlotWords + lane16;
+        // folded rows: do the lane's two runs take the second of the two row statistics
+        const bool second_a = FOLD == kWraps && (uint32_t)(4 * lane16) >= span.split;
+    const bool second_b = FOLD == kDoubles || (FOLD == kWraps && (uint32_t)(64 + 4 * lane16) >= span.split);
+        const uint32_t in_tile = FOLD != kWraps ? 0u : span.first - fold_span(f, q.col_tile * (uint32_t)q.wide).first;
         // a lane keeps its eight columns through all passes: their statistics come out of LDS once
         float co[kEltsPerLane];
         unpack8(lds_read<float4>(lds, co_off), lds_read<float4>(lds, co_off + 256), co);
+        const float least = t.tile.drop_nan ? 0.0f : __builtin_nanf("");  // of a column's values
 #pragma unroll 1
         for (int it = 0; it < q.passes; ++it) {
             const int64_t r = q.row0 + it * q.step;
-            if (r >= f.rows)
-                break;
-            if (it > 0)
-                pass_fetch<MODE, FOLD, KEEP>(t, f, q.cg, lane16, r, x);
             const int64_t grp = r * f.col_blocks + q.cg;
             const int64_t gbase = grp * kGroup;
+            if (r >= f.rows || (FOLD == kWraps && gbase >= f.values))
+                break;
+            if (it > 0)
+                pass_fetch<MODE, FOLD, KEEP>(t, f, span, q.cg, lane16, r, x);
+            const bool live_a = FOLD != kWraps || gbase + 4 * lane16 < f.values, live_b = FOLD != kWraps || gbase + 4 * lane16 + 64 < f.values;
             float *pp = t.p + gbase + lane16 * 4;
             const uint32_t wv = x.v0 | (x.v1 << 16);
-            const float ro = x.ro, ro1 = FOLD ? x.ro1 : x.ro;
+            const float ro_a = second_a ? x.ro1 : x.ro, ro_b = second_b ? x.ro1 : x.ro;
             float pv[kEltsPerLane], gv[kEltsPerLane], m[kEltsPerLane], v[kEltsPerLane];
             unpack8(x.a0, x.a1, pv);
             unpack8(x.b0, x.b1, gv);
@@ -253,20 +288,35 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                 unpack8(x.c0, x.c1, m);
 
             const Nibbles nv = split_nibbles(wv);
-            float amax_m = 0.0f, vmax = 0.0f, vmax1 = 0.0f;  // vmax1: the second half's (folded rows)
+            float amax_m = 0.0f, vmax = 0.0f, vmax1 = 0.0f;  // vmax1: the second tensor row's (folded rows)
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
                 if (!M32)
                     m[k] = decode_nibble(lds, kLdsQ0, nm, k) * sm;
-                const float rk = (FOLD && k >= 4) ? ro1 : ro;
+                const float rk = k >= 4 ? ro_b : ro_a;
                 v[k] = decode_nibble(lds, kLdsQ1, nv, k) * ((co[k] < rk) ? co[k] : rk);
+            }
+            if (FOLD == kWraps && !live_b) {
+                // beyond the end: the zeros that fill up the last group
+#pragma unroll
+                for (int k = 0; k < kEltsPerLane; ++k)
+                    if (k >= 4 || !live_a)
+                        gv[k] = m[k] = v[k] = 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < kEltsPerLane; ++k) {
                 nonfused_elt(pv[k], gv[k], m[k], v[k], h);
                 amax_m = fmaxf(amax_m, fabsf(m[k]));
                 if (FOLD && k >= 4)
                     vmax1 = fmaxf(vmax1, v[k]);
                 else
                     vmax = fmaxf(vmax, v[k]);
-                atomicMax(red + k * 16, __float_as_uint(v[k]));
+                atomicMax(red + k * 16, __float_as_uint(FOLD == kWraps ? fmaxf(v[k], least) : v[k]));
+            }
+            if (FOLD == kWraps) {
+                const float a = vmax, b = vmax1;
+                vmax = fmaxf(second_a ? 0.0f : a, second_b ? 0.0f : b);
+                vmax1 = fmaxf(second_a ? a : 0.0f, second_b ? b : 0.0f);
             }
             uint32_t cm = 0;
             if (M32) {
@@ -279,8 +329,10 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
             if (FOLD)
                 vmax1 = row16_max(vmax1);
 
-            store4(pp, make_float4(pv[0], pv[1], pv[2], pv[3]));
-            store4(pp + 64, make_float4(pv[4], pv[5], pv[6], pv[7]));
+            if (live_a)
+                store4(pp, make_float4(pv[0], pv[1], pv[2], pv[3]));
+            if (live_b)
+                store4(pp + 64, make_float4(pv[4], pv[5], pv[6], pv[7]));
             if (M32) {
                 float *mp = reinterpret_cast<float *>(t.mc) + gbase + lane16 * 4;
                 store4(mp, make_float4(m[0], m[1], m[2], m[3]));
@@ -295,13 +347,17 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                 atomic_max_nonneg(t.ms_new + (grp >> t.m_lg), amax_m);
             }
             if (lane16 == 0) {
-                // the maxima of a tensor row meet in LDS (rank1_tiles.hpp); folded rows: a half goes to the
-                // tensor row it lies in
-                uint32_t *slot = rowred + row_slot(t.tile, it, drow);
-                if (FOLD) {
-                    const bool h0 = f.on && q.cg * kGroup >= f.real_cols, h1 = f.on && q.cg * kGroup + 64 >= f.real_cols;
-                    atomicMax(slot + (h0 ? 1 : 0), __float_as_uint(vmax));
-                    atomicMax(slot + (h1 ? 1 : 0), __float_as_uint(vmax1));
+                // the maxima of a tensor row meet in LDS (rank1_tiles.hpp)
+                uint32_t *slot = rowred + row_slot(t.tile, it, drow) * (FOLD == kWraps ? 2 : 1);
+                if (FOLD == kDoubles) {
+                    uint32_t halves[2];
+                    double_halves(f, q.cg, halves);
+                    atomicMax(slot + halves[0], __float_as_uint(vmax));
+                    atomicMax(slot + halves[1], __float_as_uint(vmax1));
+                } else if (FOLD) {
+                    atomicMax(slot + in_tile, __float_as_uint(vmax));
+                    if (span.split < (uint32_t)kGroup)
+                        atomicMax(slot + in_tile + 1, __float_as_uint(vmax1));
                 } else {
                     atomicMax(slot, __float_as_uint(vmax));
                 }
@@ -310,7 +366,10 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
     }
     // the column maxima meet in LDS: nothing below depends on the global stores still in flight
     lds_barrier();
-    flush_row_maxima(rowred, t.tile, q, drow, f.rows, FOLD && f.on, t.row_new);
+    if (FOLD == kWraps)
+        flush_row_maxima_fold(rowred, t.tile, q, drow, f, t.row_new);
+    else
+        flush_row_maxima(rowred, t.tile, q, drow, f.rows, t.row_new, f.lg);
     // column j of the tile = element k of lane l of slot s
     for (int j = threadIdx.x; j < q.wide * kGroup; j += kThreads) {
         const int w = j & (kGroup - 1);
@@ -323,8 +382,17 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
     }
 }
 
+// The runs of a lane beyond the end of the tensor: the second, and the first with it.
+__device__ __forceinline__ void zero_beyond(float (&x)[kEltsPerLane], bool both)
+{
+#pragma unroll
+    for (int k = 0; k < kEltsPerLane; ++k)
+        if (k >= 4 || both)
+            x[k] = 0.0f;
+}
+
 // MWIDE: the first moment's groups are wider than 128 values; its codes are written here too.
-template <bool MWIDE, bool FOLD, int N>
+template <bool MWIDE, int FOLD, int N>
 __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<N> args, const float *__restrict__ qmap_m,
                                                                  const float *__restrict__ qmap_v)
 {
@@ -341,7 +409,7 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
     const TensorR1 &t = args.t[lo];
     const uint32_t tl = blockIdx.x - args.tile_start[lo];
     const int lane16 = threadIdx.x & 15, drow = threadIdx.x >> 4;
-    const Fold f = fold_of<FOLD>(t);
+    const Fold f = fold_of<FOLD != kNoFold>(t);
     const Geometry q = geometry(t.tile, f.col_blocks, tl, drow);
     const int64_t cols = (int64_t)f.col_blocks * kGroup;
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
@@ -361,7 +429,7 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
 
     if (tl == 0) {
         const float z[kEltsPerLane] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        const int64_t n = f.rows * cols;
+        const int64_t n = FOLD ? (f.values + kGroup - 1) / kGroup * kGroup : f.values;
         const int64_t n_pack = (n + LPMM_PACK_GROUP - 1) / LPMM_PACK_GROUP * LPMM_PACK_GROUP;
         write_padding(t.vc, n, n_pack, encode8_plain(lds, kVMap, kind, z));
         if (MWIDE) {
@@ -403,17 +471,30 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
     // the group's 64 code bytes move as one dword per lane (whole lines per access; with the
     // arithmetic taken out this pass is 11 % faster than with two 16-bit accesses per lane)
     const uint32_t code_dword = code_dword_of_lane(lane16), code_sel = code_swap_selector(lane16);
+    const FoldSpan span = FOLD == kWraps ? fold_span(f, q.cg) : FoldSpan{0, kGroup};
+    uint32_t halves[2] = {0u, 0u};
+    if (FOLD == kDoubles)
+        double_halves(f, q.cg, halves);
+    // folded rows: do the lane's two runs take the second of the two row statistics
+    const bool second_a = FOLD == kWraps && (uint32_t)(4 * lane16) >= span.split;
+    const bool second_b = FOLD == kDoubles || (FOLD == kWraps && (uint32_t)(64 + 4 * lane16) >= span.split);
+    const float most = FOLD == kWraps && t.tile.drop_nan ? 1.0f : __builtin_nanf("");
 #pragma unroll 1
     for (int it = 0; it < q.passes; ++it) {
         const int64_t r = q.row0 + it * q.step;
-        if (r >= f.rows)
-            break;
         const int64_t gbase = (r * f.col_blocks + q.cg) * kGroup;
-        const float *gp = t.g + gbase + lane16 * 4;
-        int64_t r0 = r, r1 = r;  // the tensor rows of the DPP row's two halves
-        if (FOLD)
-            fold_rows(f, r, q.cg, r0, r1);
-        const float4 b0 = load4(gp), b1 = load4(gp + 64);
+        if (r >= f.rows || (FOLD == kWraps && gbase >= f.values))
+            break;
+        const int64_t oa = gbase + lane16 * 4, ob = oa + 64, last = f.values - 4;
+        int64_t r0 = r, r1 = r;  // the tensor rows of the DPP row
+        if (FOLD == kWraps) {
+            fold_rows(f, span, r, r0, r1);
+        } else if (FOLD) {
+            r0 = (r << f.lg) + halves[0];
+            r1 = (r << f.lg) + halves[1];
+        }
+        // runs beyond the end read the last one
+        const float4 b0 = load4(t.g + (FOLD == kWraps && oa > last ? last : oa)), b1 = load4(t.g + (FOLD == kWraps && ob > last ? last : ob));
         uint32_t *vcp = reinterpret_cast<uint32_t *>(t.vc + (gbase >> 1)) + code_dword;
         const uint32_t in_v = load_u32(vcp);
         const float ro = t.row_old[r0], rn = t.row_new[r0];
@@ -441,17 +522,18 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
         // of the step; the plain variant would go from 74 to 82 registers and lose a wave per SIMD.)
         constexpr bool kBitMin = FOLD || MWIDE;
         const bool fast = kind == kMapStdV && __all(cols_safe && rc_safe(rn) && rc_safe(rn1) && ro == ro && ro1 == ro1);
+        const float ro_a = second_a ? ro1 : ro, ro_b = second_b ? ro1 : ro, rn_a = second_a ? rn1 : rn, rn_b = second_b ? rn1 : rn;
         if (kBitMin && fast) {
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
-                const float rk = (FOLD && k >= 4) ? ro1 : ro;
+                const float rk = k >= 4 ? ro_b : ro_a;
                 v[k] = decode_nibble(lds, kVMap, nv, k) * __uint_as_float(min(__float_as_uint(co[k]), __float_as_uint(rk)));
                 nonfused_second_moment(v[k], gv[k], h);
             }
         } else {
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
-                const float rk = (FOLD && k >= 4) ? ro1 : ro;
+                const float rk = k >= 4 ? ro_b : ro_a;
                 v[k] = decode_nibble(lds, kVMap, nv, k) * ((co[k] < rk) ? co[k] : rk);
                 nonfused_second_moment(v[k], gv[k], h);
             }
@@ -471,10 +553,10 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
         if (fast) {
             // the correctly rounded reciprocal of whichever statistic is the scale, then one
             // multiply and two fmas: the correctly rounded quotient (v <= scale by construction)
-            const float rcr = rcp_exact(rn), rcr1 = FOLD ? rcp_exact(rn1) : rcr;
+            const float rcr = rcp_exact(rn_a), rcr1 = FOLD ? rcp_exact(rn_b) : rcr;
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
-                const float rnk = (FOLD && k >= 4) ? rn1 : rn, rck = (FOLD && k >= 4) ? rcr1 : rcr;
+                const float rnk = k >= 4 ? rn_b : rn_a, rck = (FOLD && k >= 4) ? rcr1 : rcr;
                 if (kBitMin) {
                     const float sk = __uint_as_float(min(__float_as_uint(cn[k]), __float_as_uint(rnk)));
                     const float rk = __uint_as_float(max(__float_as_uint(rcn[k]), __float_as_uint(rck)));
@@ -484,13 +566,23 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
                     x[k] = div_by_rc(v[k], by_col ? cn[k] : rnk, by_col ? rcn[k] : rck);
                 }
             }
+            if (FOLD == kWraps) {
+                // a NaN whose column's statistic leaves it out: code 15
+#pragma unroll
+                for (int k = 0; k < kEltsPerLane; ++k)
+                    x[k] = fminf(x[k], most);
+                if (ob > last)
+                    zero_beyond(x, oa > last);
+            }
             w = encode8_std_v(x);
         } else {
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k) {
-                const float rnk = (FOLD && k >= 4) ? rn1 : rn;
+                const float rnk = k >= 4 ? rn_b : rn_a;
                 x[k] = v[k] / ((cn[k] < rnk) ? cn[k] : rnk);
             }
+            if (FOLD == kWraps && ob > last)
+                zero_beyond(x, oa > last);
             w = encode8_plain(lds, kVMap, kind, x);
         }
         store_u32(vcp, swap_code_halves(w, code_sel));
@@ -566,9 +658,24 @@ static uint64_t shape_tiles(int64_t rows, uint32_t col_blocks, TileShape &ts, ui
             comb = (comb + kCombMultiple - 1) / kCombMultiple * kCombMultiple;
     }
     ts.lg_wide = b.lg_wide;
+    ts.drop_nan = 0;
     ts.tile_rows = b.tile_rows;
     ts.comb = (uint32_t)comb;
     return (b.rows + comb - 1) / comb * comb * b.col_tiles;
+}
+
+// The matrix that a pass's tiles cover; can_fold: column counts that are no multiple of 128 are folded (and satisfy can_fold_rows).
+struct Matrix {
+    int64_t rows;
+    uint32_t col_blocks, lg;
+};
+
+static Matrix matrix_of(int64_t rows, int64_t cols, bool can_fold)
+{
+    if (!can_fold || cols % kGroup == 0)
+        return {rows, (uint32_t)((cols + kGroup - 1) / kGroup), 0};
+    const uint32_t lg = fold_lg((uint32_t)cols);
+    return {(rows + ((int64_t)1 << lg) - 1) >> lg, (uint32_t)(cols >> (7 - lg)), lg};
 }
 
 // What a launch is, as far as its tile shapes depend on it.
@@ -619,8 +726,13 @@ constexpr uint64_t kSpreadBelow = 1024;
 // 36.6 / 18.4; 8 of 1024 x 1024 28.7 / 16.4, 21.0 / 11.0, 19.0 / 8.9, 19.6 / 10.2; 24 of 512 x 512 27.9 / 15.5, 20.5 / 11.0, 16.5 /
 // 8.3, 15.7 / 7.9; update of 39877 x 128 22.6, 29.0 (a column's row blocks).  Any column count likewise: 2001 x 3001 49.5 / 82, 29.7, 30.2, 30.3 / 35.8;
 // 6 of 4096 x 4100 297, 288, 292, 306.
-static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, int64_t rows, uint32_t col_blocks, bool odd_cols)
+static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, const Matrix &m, bool odd_cols)
 {
+    const bool fold = m.lg != 0;
+    const uint32_t col_blocks = m.col_blocks;
+    const double values = (double)m.rows * (double)col_blocks * kGroup;
+    // a row block has as many atomics on a column as the fold has rows; double rows count as one
+    const int64_t rows = fold ? m.rows << (m.lg - 1) : m.rows;
     if (l.half_io && requant)
         return l.values < 6.5e6 ? kPolicyRows / 4 : l.values < 14e6 ? kPolicyRows / 2 : l.values < 26e6 ? kPolicyRows : kPolicyRowsHalf;
     const bool single = choose_lg_wide(col_blocks) == 0;  // tiles of one column group
@@ -642,7 +754,6 @@ static uint32_t pass_rows_policy(const LaunchKind &l, bool requant, bool fold, i
     else
         tile_rows = rows <= 256 * (int64_t)(kPolicyRows / 4) && !(l.bits && l.values >= 14e6) ? kPolicyRows / 4
                     : rows <= 400 * (int64_t)(kPolicyRows / 2) ? kPolicyRows / 2 : kPolicyRows;
-    const double values = (double)rows * (double)col_blocks * kGroup;
     const double most = values / kValuesPerRowBlock > 512 ? values / kValuesPerRowBlock : 512;
     while (tile_rows < kPolicyRowsMost && (double)rows > most * tile_rows)
         tile_rows *= 2;
@@ -668,24 +779,14 @@ static float *next_scales(const lpmm_nonfused_rank1_tensor &) { return nullptr; 
 static float *next_scales(const lpmm_rank1_v4bit_tensor &) { return nullptr; }
 static float *next_scales(const lpmm_rank1_mgroup_tensor &t) { return t.m_max1_next; }
 
-// a tensor that the kernels take as double rows
-static bool folds(int64_t rows, int64_t cols) { return cols % kGroup == 64 && rows % 2 == 0; }
-
-// The matrix that a pass's tiles cover; can_fold: column counts that are no multiple of 128 are folded (and satisfy folds).
-struct Matrix {
-    int64_t rows;
-    uint32_t col_blocks;
-    bool fold;
-};
-
-static Matrix matrix_of(int64_t rows, int64_t cols, bool can_fold)
+// Tensors that the kernels take as double rows; wraps: as rows of up to 32 too, with any row count (a group then lies in at most two
+// tensor rows; the indexes within a row of the matrix have 32 bits).
+static bool can_fold_rows(int64_t rows, int64_t cols, bool wraps)
 {
-    const uint32_t blocks = (uint32_t)((cols + kGroup - 1) / kGroup);
-    const bool fold = can_fold && cols % kGroup != 0;
-    return fold ? Matrix{rows / 2, 2 * blocks - 1, true} : Matrix{rows, blocks, false};
+    return (cols % kGroup == 64 && rows % 2 == 0) || (wraps && cols % 4 == 0 && (cols >= kGroup || cols == 64) && cols <= (1 << 24));
 }
 
-template <int MODE, bool FOLD, int N>
+template <int MODE, int FOLD, int N>
 static void launch_rank1_passes(const R1LaunchN<N> &l, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
 {
     if (passes & 1) {
@@ -698,18 +799,19 @@ static void launch_rank1_passes(const R1LaunchN<N> &l, const float *qmap_m, cons
 }
 
 template <int MODE, int N>
-static void launch_rank1(const R1LaunchN<N> &l, bool folded, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
+static void launch_rank1(const R1LaunchN<N> &l, int folded, const float *qmap_m, const float *qmap_v, int passes, hipStream_t stream)
 {
     if constexpr (MODE == kMCodes128)
-        if (folded)
-            return launch_rank1_passes<MODE, true>(l, qmap_m, qmap_v, passes, stream);
-    launch_rank1_passes<MODE, false>(l, qmap_m, qmap_v, passes, stream);
+        if (folded != kNoFold)
+            return folded == kDoubles ? launch_rank1_passes<MODE, kDoubles>(l, qmap_m, qmap_v, passes, stream)
+                                      : launch_rank1_passes<MODE, kWraps>(l, qmap_m, qmap_v, passes, stream);
+    launch_rank1_passes<MODE, kNoFold>(l, qmap_m, qmap_v, passes, stream);
 }
 
 // The checks of a call's records.  general: they are for any column count and alignment; can_fold: see rank1_step_multi.
 template <int MODE, class Record>
 static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v, bool general, bool half_io,
-                       bool can_fold)
+                       bool can_fold, bool wraps = false)
 {
     const int64_t real_bytes = general && half_io ? 2 : 4, vec_bytes = general ? real_bytes : 16;
     constexpr bool M32 = MODE == kMFloat;
@@ -722,7 +824,7 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
         const Record &t = tensors[i];
         if (t.rows < 0 || t.cols < 0)
             return LPMM_ERR_SIZE;
-        if (!general && t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && folds(t.rows, t.cols)))
+        if (!general && t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && can_fold_rows(t.rows, t.cols, wraps)))
             return LPMM_ERR_SIZE;
         if (t.rows == 0 || t.cols == 0)
             continue;
@@ -766,13 +868,13 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
 // Validation, batching into launches of at most kR1Max tensors, and the launches.
 // m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
 // folds: a record per tensor, of ndim 0 where the tensor is a matrix (lpmm_nonfused_adamw4bit_rank1_nd_step_multi).
-// plain: tensors with fp32 states that go with the clearing, as many as its launches take.
+// plain: tensors with fp32 states that go with the clearing, as many as its launches take.  wraps: see can_fold_rows.
 template <int MODE, class Record>
 static int rank1_step_multi(const Record *tensors, int64_t count, const float *qmap_m, const float *qmap_v,
                             uint32_t m_lg, double beta1, double beta2, double lr, double weight_decay, double eps,
                             void *stream, int bits_m = 4, int bits_v = 4, const void *table_m = nullptr,
                             const void *table_v = nullptr, int passes = 3, bool half_io = false, const NewCodes *out = nullptr,
-                            const lpmm_rank1_small_vector *folds = nullptr, PlainSet *plain = nullptr)
+                            const lpmm_rank1_small_vector *folds = nullptr, PlainSet *plain = nullptr, bool wraps = false)
 {
     // passes: 1 = the first pass alone (with the clearing of the next statistics), 2 = the second alone,
     // 3 = both; one at a time only where the launches below are this file's own, or general ones: any column count,
@@ -789,7 +891,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     if (count == 0)
         return LPMM_OK;
     if (!general) {
-        const int bad = check_rank1<MODE>(tensors, count, qmap_m, qmap_v, false, half_io, can_fold);
+        const int bad = check_rank1<MODE>(tensors, count, qmap_m, qmap_v, false, half_io, can_fold, wraps);
         if (bad != LPMM_OK)
             return bad;
     }
@@ -877,7 +979,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             each([&](const Record &t) {
                 const Matrix m = matrix_of(t.rows, t.cols, can_fold);
                 for (int pass = 0; pass < 2; ++pass) {
-                    const Blocks b = blocks_of(m.rows, m.col_blocks, pass_rows_policy(kind, pass == 1, m.fold, m.rows, m.col_blocks, t.cols & 1));
+                    const Blocks b = blocks_of(m.rows, m.col_blocks, pass_rows_policy(kind, pass == 1, m, t.cols & 1));
                     blocks[pass] += b.rows * b.col_tiles;
                 }
             });
@@ -890,7 +992,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         float *scale2[kMost];  // the column statistics of the second pass
         const lpmm_rank1_small_vector *between[kMost];
         int betweens = 0;
-        bool folded = false;  // does a tensor of this launch have folded rows
+        int folded = kNoFold;  // what the launch's tensors need
         args.tile_start[0] = 0;
         while (i < count && k < kMost) {
             const Record &t = tensors[i];
@@ -902,9 +1004,9 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             TensorR1 &d = args.t[k];
             const Matrix m = matrix_of(t.rows, t.cols, can_fold);
             const bool odd = t.cols & 1;
-            const uint64_t nt = shape_tiles(m.rows, m.col_blocks, d.tile, pass_rows_policy(kind, false, m.fold, m.rows, m.col_blocks, odd),
+            const uint64_t nt = shape_tiles(m.rows, m.col_blocks, d.tile, pass_rows_policy(kind, false, m, odd),
                                             kind.spread[0]);
-            const uint64_t nt2 = shape_tiles(m.rows, m.col_blocks, shape2[k], pass_rows_policy(kind, true, m.fold, m.rows, m.col_blocks, odd),
+            const uint64_t nt2 = shape_tiles(m.rows, m.col_blocks, shape2[k], pass_rows_policy(kind, true, m, odd),
                                              kind.spread[1]);
             if (tiles + nt > 0x7fffffffULL || tiles2 + nt2 > 0x7fffffffULL)
                 break;
@@ -922,13 +1024,17 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             d.rows = t.rows;
             d.col_blocks = col_blocks;
             d.col_tail = (uint32_t)(t.cols - (int64_t)(col_blocks - 1) * kGroup);
+            // what the kernels for any column count took before
+            d.tile.drop_nan = shape2[k].drop_nan =
+                m.lg != 0 && !can_fold_rows(t.rows, t.cols, false) && (t.cols % 8 != 0 || (folds != nullptr && folds[i].ndim != 0));
             const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
             d.rbc2_sqrt = h.rbc2_sqrt;
             tiles += nt;
             tiles2 += nt2;
-            folded = folded || m.fold;
+            if (m.lg != 0)
+                folded = std::max(folded, (int)(can_fold_rows(t.rows, t.cols, false) ? kDoubles : kWraps));
             scale2[k] = d.col_new;
             if (folds != nullptr && folds[i].ndim != 0) {
                 scale2[k] = folds[i].scale;
@@ -985,7 +1091,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
                 return st;
             launch_rank1<MODE>(l, folded, qmap_m, qmap_v, 2, s);
         } else {
-            launch_rank1<MODE>(l, MODE == kMCodes128 && folded, qmap_m, qmap_v, passes, s);
+            launch_rank1<MODE>(l, MODE == kMCodes128 ? folded : kNoFold, qmap_m, qmap_v, passes, s);
         }
         return launch_status();
     };
@@ -1070,7 +1176,7 @@ static int nd_step_multi(const lpmm_nonfused_rank1_tensor *tensors, const lpmm_r
         LPMM_REQUIRE_ALIGN(v.scale, 16);
     }
     return rank1_step_multi<kMCodes128>(tensors, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, 4, 4, nullptr,
-                                        nullptr, 3, false, nullptr, folds, plain);
+                                        nullptr, 3, false, nullptr, folds, plain, true);
 }
 
 extern "C" int lpmm_nonfused_adamw4bit_rank1_nd_step_multi(const lpmm_nonfused_rank1_tensor *tensors,
@@ -1309,7 +1415,7 @@ extern "C" int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors
         case LPMM_STEP_MATRIX:
         case LPMM_STEP_BITS:
             st = rank1_step_multi<kMCodes128>(matrices, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, bits_m,
-                                              bits_v, table_m, table_v, 3, false, nullptr, nullptr, &set);
+                                              bits_v, table_m, table_v, 3, false, nullptr, nullptr, &set, kind == LPMM_STEP_MATRIX);
             break;
         case LPMM_STEP_ND:
             st = nd_step_multi(matrices, folds, count, qmap_m, qmap_v, beta1, beta2, lr, weight_decay, eps, stream, &set);

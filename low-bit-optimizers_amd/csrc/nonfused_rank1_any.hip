@@ -484,7 +484,7 @@ __global__ __launch_bounds__(kThreads, 4) void rank1_update_any_kernel(const Mul
             atomicMax(colred + (drow & (q.wide - 1)) * kGroup + piece_at<VEC>(first, lane16, k), vtop[k]);
     }
     __syncthreads();
-    flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
+    flush_row_maxima(rowred, t.tile, q, drow, t.rows, t.row_new);
     const int64_t tile_c0 = (int64_t)q.col_tile * q.wide * kGroup;
     for (int j = threadIdx.x; j < q.wide * kGroup; j += kThreads)
         if (tile_c0 + j < cols)

@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void rank1_update_bits_kernel(const Multi
         }
     }
     __syncthreads();
-    flush_row_maxima(rowred, t.tile, q, drow, t.rows, false, t.row_new);
+    flush_row_maxima(rowred, t.tile, q, drow, t.rows, t.row_new);
     // column j of the tile = element k of lane l of slot s
     for (int j = threadIdx.x; j < q.wide * kGroup; j += kThreads) {
         const int w = j & (kGroup - 1);

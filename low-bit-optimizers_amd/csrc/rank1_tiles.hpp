@@ -44,7 +44,8 @@ constexpr uint32_t kRedSlotWords = kGroup + 16;
 // A workgroup covers tile_rows rows x (128 << lg_wide) columns: per pass, (16 >> lg_wide) rows of
 // (1 << lg_wide) adjacent groups each.
 struct TileShape {
-    uint32_t lg_wide : 8;
+    uint32_t lg_wide : 4;
+    uint32_t drop_nan : 4;    // kernels with folded rows: column maxima leave NaNs out, as those of the kernels for any column count do
     uint32_t tile_rows : 24;  // max(the policy's rows, rows of one pass)
     uint32_t comb;            // row blocks whose passes interleave
 };
@@ -147,49 +148,84 @@ __device__ __forceinline__ uint32_t xcd_neighbours(uint32_t index, uint32_t tile
     return block0 + kBlock <= tiles ? block0 + (in % kXcds) * kXcdNeighbours + in / kXcds : index;
 }
 
-// Folded rows.  A tensor of R x C values with C = 64 modulo 128 and R even is the same memory as
-// the row-major matrix of R / 2 double rows of 2 C values, and 2 C is a multiple of 128: the
+// Folded rows.  A tensor of R x C values whose C is no multiple of 128 but of 2^t, 2 <= t < 7, is the same memory as the
+// row-major matrix of rows of 2^lg C values, lg = 7 - t, which are a multiple of 128: the
 // 128-value groups of the first moment, cut from the flattened tensor (lpmm/functional.py:404-422),
-// never straddle a double row, so the kernels for whole column blocks apply to that matrix (GPT-2-XL's
-// d = 1600 and 3 d = 4800).  What changes is where a value's statistics sit: a DPP row's 128 values
-// are two halves of 64 (a lane's first and second run of four), half h of column block cg of double
-// row r lies in tensor row 2 r + (128 cg + 64 h >= C) at column (128 cg + 64 h) mod C.  The record
-// keeps the tensor's own shape (col_blocks = ceil(C / 128), col_tail = 64); kernels instantiated
+// never straddle such a row, so the kernels for whole column blocks apply to that matrix (GPT-2-XL's
+// d = 1600 and 3 d = 4800: double rows; 408 columns: rows of sixteen).  Where R is no multiple of 2^lg the last row of the matrix, and
+// in it the last group, is a part.  What changes is where a value's statistics sit: value c of a row of the matrix
+// lies in tensor row (r << lg) + c / C at column c mod C, and a DPP row's 128 values lie in one or two tensor rows, split at a run of
+// four (C is 64 or at least 128).  The record
+// keeps the tensor's own shape (col_blocks = ceil(C / 128), col_tail = C - 128 (col_blocks - 1)); kernels instantiated
 // with FOLD read it this way, tensors with whole column blocks in the same launch as before.
+// The first moment is then written where it is computed, all tiles but the last are full, and one kind of launch serves nearly every model,
+// where the kernels for any column count (nonfused_rank1_any.hip) and for multiples of 8 (nonfused_rank1_ragged.hip), which split the
+// groups' maxima between rows and write the first moment in the second pass, took 19 bytes a value, launches and new
+// code arrays of their own.  Steps in us: 50257 x 1600 345 -> 278, 31426 x 408 71 -> 62, six of 4096 x 4100 460 -> 343, 1000000 x 136 765 ->
+// 578, thirty of 88 x 88 x 3 x 3 111 -> 48 (the host in both), sixty of 56 x 56 x 3 x 3 208 -> 69.  Double rows keep kernels of their own (whole
+// last rows, halves instead of runs): GPT-2-XL's 192 matrices take 4928 us with them, 4962 to 5025 without.
 struct Fold {
-    bool on;
     uint32_t real_cols, col_blocks;  // columns of the tensor; column blocks of the matrix the kernel works on
+    uint32_t lg;
     int64_t rows;                    // rows of that matrix
+    int64_t tensor_rows, values;
 };
+
+// 7 - t of a column count that folds
+__host__ __device__ __forceinline__ uint32_t fold_lg(uint32_t cols) { return 7u - (uint32_t)__builtin_ctz(cols); }
 
 template <bool FOLD>
 __device__ __forceinline__ Fold fold_of(const TensorR1 &t)
 {
     Fold f;
-    f.on = FOLD && t.col_tail != (uint32_t)kGroup;
     f.real_cols = (t.col_blocks - 1) * kGroup + t.col_tail;
-    f.col_blocks = f.on ? 2 * t.col_blocks - 1 : t.col_blocks;
-    f.rows = f.on ? t.rows >> 1 : t.rows;
+    f.lg = FOLD && t.col_tail != (uint32_t)kGroup ? fold_lg(f.real_cols) : 0u;
+    f.col_blocks = f.lg != 0 ? f.real_cols >> (7u - f.lg) : t.col_blocks;
+    f.tensor_rows = t.rows;
+    f.rows = FOLD ? (t.rows + ((int64_t)1 << f.lg) - 1) >> f.lg : t.rows;
+    f.values = t.rows * f.real_cols;
     return f;
 }
 
-// column of the tensor for column c of the matrix (c < 2 C)
-__device__ __forceinline__ uint32_t fold_col(const Fold &f, uint32_t c) { return c >= f.real_cols ? c - f.real_cols : c; }
+// column of the tensor for column c of the matrix
+__device__ __forceinline__ uint32_t fold_col(const Fold &f, uint32_t c) { return f.lg != 0 ? c % f.real_cols : c; }
 
-// Tensor rows of the two halves of column block cg in row r of the matrix.  No branch: a pass's loads of the row statistics stay among
-// its other loads, ahead of the first wait.
-__device__ __forceinline__ void fold_rows(const Fold &f, int64_t r, uint32_t cg, int64_t &r0, int64_t &r1)
+// Column block cg of the matrix: the first tensor row it lies in, counted within a row of the matrix, and how many of its values do (128
+// or more: all).
+struct FoldSpan {
+    uint32_t first, split;
+};
+__device__ __forceinline__ FoldSpan fold_span(const Fold &f, uint32_t cg)
 {
-    const int on = f.on ? 1 : 0;
-    r0 = (r << on) + (on & (cg * kGroup >= f.real_cols ? 1 : 0));
-    r1 = (r << on) + (on & (cg * kGroup + 64 >= f.real_cols ? 1 : 0));
+    FoldSpan s;
+    s.first = f.lg != 0 ? cg * kGroup / f.real_cols : 0u;
+    s.split = (s.first + 1u) * f.real_cols - cg * kGroup;
+    return s;
+}
+
+// The one or two tensor rows of a column block in row r of the matrix (of the last ones, where there are none).  No branch: a pass's loads
+// of the row statistics stay among its other loads, ahead of the first wait.
+__device__ __forceinline__ void fold_rows(const Fold &f, const FoldSpan &s, int64_t r, int64_t &r0, int64_t &r1)
+{
+    const int64_t last = f.tensor_rows - 1;
+    r0 = (r << f.lg) + s.first;
+    r1 = r0 + (s.split < (uint32_t)kGroup ? 1 : 0);
+    r0 = r0 < last ? r0 : last;
+    r1 = r1 < last ? r1 : last;
+}
+
+// Double rows: the tensor rows of the two halves of column block cg in row r, half h in the second one where halves[h] is 1.
+__device__ __forceinline__ void double_halves(const Fold &f, uint32_t cg, uint32_t (&halves)[2])
+{
+    halves[0] = f.lg != 0 && cg * kGroup >= f.real_cols ? 1u : 0u;
+    halves[1] = f.lg != 0 && cg * kGroup + 64 >= f.real_cols ? 1u : 0u;
 }
 
 // Row maxima of a tile.  An atomic maximum on global memory goes out to the fabric (the L2s of
 // the XCDs are not coherent with each other), and the passes of a tile produce one per tensor row,
 // column group and pass: 0.008 per element, a tenth of the first pass's DRAM transactions together
 // with its partial writes.  So the maxima of a tile's rows meet in LDS first -- slot 2 * (row of
-// the tile) + (tensor row of a double row: folded rows only) -- and one global atomic per row and
+// the tile) + (tensor row of a double row) -- and one global atomic per row and
 // tile follows the passes, issued by neighbouring threads for neighbouring rows (LLaMA-7B-shaped
 // set 21.23 -> 20.85 ms per step, GPT-2-XL-shaped set 6.30 -> 5.71 ms).
 constexpr int kRowSlots = 2 * (int)kPolicyRowsMost;
@@ -201,9 +237,9 @@ __device__ __forceinline__ int row_slot(const TileShape &ts, int pass, int drow)
     return 2 * (pass * (kDppRows >> ts.lg_wide) + (drow >> ts.lg_wide));
 }
 
-// after the passes and a barrier: rows = rows of the matrix the tile works on; fold: its rows are double rows
+// after the passes and a barrier: rows = rows of the matrix the tile works on; lg: 1 where they are double rows
 __device__ __forceinline__ void flush_row_maxima(const uint32_t *rowred, const TileShape &ts, const Geometry &q, int drow,
-                                                 int64_t rows, bool fold, float *__restrict__ row_new)
+                                                 int64_t rows, float *__restrict__ row_new, uint32_t lg = 0)
 {
     if (threadIdx.x >= (uint32_t)kRowSlots)
         return;
@@ -212,8 +248,25 @@ __device__ __forceinline__ void flush_row_maxima(const uint32_t *rowred, const T
     const int pass = local / pr, in_pass = local - pass * pr;
     // the first row of the tile's first pass: row0 of this thread's DPP row less its place in the pass
     const int64_t r = (q.row0 - (drow >> ts.lg_wide)) + (int64_t)pass * q.step + in_pass;
-    if (pass < q.passes && r < rows && (half == 0 || fold))
-        atomic_max_nonneg(row_new + (fold ? 2 * r + half : r), __uint_as_float(rowred[threadIdx.x]));
+    if (pass < q.passes && r < rows && half < (1 << lg))
+        atomic_max_nonneg(row_new + (r << lg) + half, __uint_as_float(rowred[threadIdx.x]));
+}
+
+// Folded rows other than double ones: four slots a row of the tile, for the up to three tensor rows that 256 columns lie in.
+constexpr int kFoldSlots = 4 * (int)kPolicyRowsMost;
+__device__ __forceinline__ void flush_row_maxima_fold(const uint32_t *rowred, const TileShape &ts, const Geometry &q, int drow, const Fold &f,
+                                                      float *__restrict__ row_new)
+{
+    const int pr = kDppRows >> ts.lg_wide;
+    const uint32_t c0 = q.col_tile * (uint32_t)q.wide * kGroup, first = fold_span(f, q.col_tile * (uint32_t)q.wide).first;
+    for (int s = threadIdx.x; s < kFoldSlots; s += kThreads) {
+        const int local = s >> 2, pass = local / pr, in_pass = local - pass * pr;
+        const uint32_t in = first + (uint32_t)(s & 3);  // of the tensor rows of a row of the matrix
+        const int64_t r = (q.row0 - (drow >> ts.lg_wide)) + (int64_t)pass * q.step + in_pass, row = (r << f.lg) + in;
+        if (pass < q.passes && r < f.rows && in < (1u << f.lg) && (uint64_t)in * f.real_cols < (uint64_t)c0 + (uint32_t)q.wide * kGroup &&
+            row < f.tensor_rows)
+            atomic_max_nonneg(row_new + row, __uint_as_float(rowred[s]));
+    }
 }
 
 // Codes of a plain 0.0 into the padding [n, n_padded) of a packed array and 0 into the extra

@@ -43,7 +43,7 @@ constexpr size_t kRecordBytes[kKinds] = {
 
 struct Names {
     PyObject *step, *exp_avg, *exp_avg_sq, *exp_avg_qstate, *exp_avg_sq_qstate, *exp_avg_sq_row, *exp_avg_sq_col, *enable, *overhead, *qmap, *max1,
-        *max_dims, *work, *scale_of, *row, *momentum_buffer, *momentum_buffer_qstate, *dtype;
+        *max_dims, *work, *scale_of, *row, *wraps, *momentum_buffer, *momentum_buffer_qstate, *dtype;
 } N;
 
 // dict[key] = value, once the launch is on the stream; strong references.  hash: of a key that is a parameter, else -1
@@ -66,7 +66,7 @@ struct Item {
     PyObject *step = nullptr;
     const at::Tensor *grad = nullptr;
     size_t held = 0;  // its objects in the plan's begin here
-    Swap swap[8];
+    Swap swap[9];
     int swaps = 0, needs = 0;
     Need need[3];
 };
@@ -87,6 +87,7 @@ struct Batch {
     std::vector<Record> items;
     std::vector<Swap> swaps;
     std::vector<Need> needs;
+    bool wraps = false;  // kRank1: a tensor that the kernels take as rows of several of its own
 };
 
 struct Plan {
@@ -340,7 +341,7 @@ struct Walk {
               const QState &m_of, const QState &v_of, int en_m, int en_v);
     bool any(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st, Item &item, int kind, const Ref &mc,
              const Ref &ms, const Ref &vc, PyObject *oh_m, PyObject *oh_v, PyObject *qm, PyObject *qv);
-    bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const Ref &any_mc,
+    bool nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, Ref any_mc, bool may_wrap,
             PyObject *oh_m, const Ref &vc, PyObject *oh_v, PyObject *qm, PyObject *qv);
     bool sgd(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject *st);
 };
@@ -441,10 +442,21 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     // the kernels that take 16 bytes an access; other operands go to the kernels for any column count
     const bool aligned = aligned16(r.p) && aligned16(r.g);
     const bool whole = aligned && r.cols % 128 == 0, folds = aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
+    // Rows of several tensor rows (Fold, rank1_tiles.hpp; the entry points that take them are those beside fp32 states and folds), in
+    // place.  A tensor's first step here still goes the way of the steps in Python, whose kernels leave new scales, and of some columns
+    // new codes, in arrays of their own: which tensors of a state a second step replaces is what callers know.  nd_scratch says
+    // that it is done: True for a matrix, its entry "wraps" for others.
+    const bool may_wrap = en_m && s.m_group128 && s.v_rank1 && aligned && !whole && !folds && r.cols % 4 == 0 &&
+                          (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
+    const bool wraps = may_wrap && p.dim() == 2 && of_parameter(nd_scratch, po) == Py_True;
+    const auto wraps_next = [&] {
+        if (may_wrap)
+            swap_later(item, nd_scratch, po, Py_True, hash_of(po));
+    };
     const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
     if (p.dim() > 2)
         return en_m && s.m_group128 && s.v_rank1 && served &&
-               nd(po, p, item, r, st, whole || folds ? nullptr : mc, oh_m, vc, oh_v, qm, qv);
+               nd(po, p, item, r, st, whole || folds ? Ref() : mc, may_wrap, oh_m, vc, oh_v, qm, qv);
     PyObject *nxt = of_parameter(spare_stats, po);
     float *now[2], *next[2];
     if (!statistics(cur, p, now) || !statistics(nxt, p, next))
@@ -478,13 +490,16 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         add(batch(kRank1Bits, p, qm, qv), r, item);
         return true;
     }
-    if (s.m_group128 && (whole || folds)) {
-        add(batch(kRank1, p, qm, qv), r, item);
+    if (s.m_group128 && (whole || folds || wraps)) {
+        Batch &b = batch(kRank1, p, qm, qv);
+        add(b, r, item);
+        b.wraps = b.wraps || wraps;
         return true;
     }
     const bool ragged = aligned && !whole && r.cols % 8 == 0;
     if (!whole && !ragged) {
         item.swaps = 0;
+        wraps_next();
         return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, vc, oh_m, oh_v, qm, qv);
     }
     PyObject *spare = of_parameter(spare_scales, po);
@@ -495,6 +510,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
                                   r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
     swap_later(item, spare_scales, po, get(oh_m, N.max1), hash_of(po));
     swap_later(item, oh_m, N.max1, spare);
+    wraps_next();
     add(batch(kRank1Wide, p, qm, qv, ragged), w, item);
     return true;
 }
@@ -624,7 +640,7 @@ bool Walk::half(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObject
 
 // a tensor of 3 to 8 dimensions on its shape[0] x rest view, where the fold between the passes takes one workgroup
 // and the column scale the last step left still holds (lpmm/optim/adamw.py: _rank1_nd_steps)
-bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, const Ref &any_mc,
+bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1_tensor &r, PyObject *st, Ref any_mc, bool may_wrap,
               PyObject *oh_m, const Ref &vc, PyObject *oh_v, PyObject *qm, PyObject *qv)
 {
     const int dims = (int)p.dim();
@@ -632,6 +648,8 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         return false;
     PyObject *cur = get(oh_v, N.max_dims), *nxt = of_parameter(spare_stats, po), *scratch = of_parameter(nd_scratch, po);
     PyObject *row = get(scratch, N.row);
+    if (may_wrap && get(scratch, N.wraps) == Py_True)
+        any_mc = nullptr;
     const int64_t pitch = (r.cols + 31) / 32 * 32;  // _nd_pitch
     const Ref work = reals_of(get(scratch, N.work), p, 3 * pitch);
     float *now[LPMM_RANK1_ND_MAX], *next[LPMM_RANK1_ND_MAX];
@@ -672,6 +690,8 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     swap_later(item, oh_v, N.max_dims, nxt);
     swap_later(item, scratch, N.scale_of, nxt);
     swap_later(item, scratch, N.row, row_obj);
+    if (may_wrap && any_mc != nullptr)
+        swap_later(item, scratch, N.wraps, Py_True);
     if (any_mc == nullptr) {
         Batch &b = batch(kNd, p, qm, qv);
         add(b, r, item);
@@ -819,7 +839,7 @@ void join_matrices(std::vector<Batch> &batches)
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
 // that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
-// a fold, in that of the flag), and flag 1 in the latter's own batch.
+// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1: flag 1 where tensors wrap.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
     Plan *plan = reinterpret_cast<Plan *>(self);
@@ -849,7 +869,7 @@ PyObject *plan_start(PyObject *self, PyObject *)
             for (const Batch &other : *plan->batches)
                 elsewhere = elsewhere || joined(*plan->batches, other) == &b;
         PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,
-                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.flag,
+                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.wraps ? 1 : b.flag,
                                     (Py_ssize_t)b.items.size(),
                                     (unsigned long long)(uintptr_t)b.records.data(),
                                     (unsigned long long)(uintptr_t)(plain != nullptr ? plain->records.data() : b.second.data()),
@@ -1070,6 +1090,7 @@ PyMODINIT_FUNC PyInit__walk()
     LPMM_NAME(work);
     LPMM_NAME(scale_of);
     LPMM_NAME(row);
+    LPMM_NAME(wraps);
     LPMM_NAME(dtype);
     LPMM_NAME(momentum_buffer);
     LPMM_NAME(momentum_buffer_qstate);
