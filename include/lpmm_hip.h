@@ -734,6 +734,12 @@ typedef struct lpmm_sgd_fp32_tensor {
 int lpmm_sgd_fp32_step_multi(const lpmm_sgd_fp32_tensor *tensors, int64_t count, double momentum, double dampening,
                              double lr, double weight_decay, int nesterov, int maximize, void *stream);
 
+/* Both kinds of tensors of a parameter group: up to 64 of the latter go with each launch of up to 64 of the former.  Either array may be
+ * empty. */
+int lpmm_sgd4bit_fp32_step_multi(const lpmm_sgd4bit_tensor *tensors, int64_t count, const lpmm_sgd_fp32_tensor *plain,
+                                 int64_t plain_count, const float *qmap, double momentum, double dampening, double lr,
+                                 double weight_decay, int nesterov, int maximize, void *stream);
+
 /* ---------------------------------------------------------------------------------------
  * Diagnostic (no counterpart in the reference): compares the library's near-exact sqrt and
  * division sequences (hardware approximation + one fma correction of the residual) with the

@@ -22,6 +22,8 @@
 // 15.3, 16.6, 16.6, 20.7 ms), and a straight-line variant for launches of whole tiles gains nothing.
 #include "lpmm_update.hpp"
 
+#include <type_traits>
+
 namespace lpmm {
 
 constexpr int kSgdThreads = 256;
@@ -70,9 +72,82 @@ __device__ __forceinline__ float sgd_elt(float p, float g, float &b, const Multi
     return __builtin_fmaf(a.neg_lr, u, p);
 }
 
-__global__ __launch_bounds__(kSgdThreads) void sgd4bit_kernel(const MultiSgd args, const float *__restrict__ qmap)
+// ---------------------------------------------------------------------------------------
+// The same chain on a float buffer: tensors whose buffer is not quantised (4096 values or fewer
+// by default: biases, norm weights).  As three or four torch operations each they took most of a
+// small model's step -- host time and launches, not bytes (the 51 vectors of a wide ResNet-152 among its 203
+// tensors: 150 launches and 0.25 ms of GPU time one after another; in one launch the whole step goes from
+// 1110-1120 to 466-470 us).  One tile
+// of 1024 values per workgroup: the tensors are short, and four values a thread are one 16-byte
+// access per operand where the pointers allow it.
+// ---------------------------------------------------------------------------------------
+constexpr int kSgdPlainTile = kSgdThreads * 4;
+
+struct TensorSgdPlain {
+    float *p;
+    const float *g;
+    float *buf;
+    int64_t n;
+    uint32_t first_step;
+    uint32_t vec;  // p, g and buf allow 16-byte accesses
+};
+
+struct MultiSgdPlain {
+    TensorSgdPlain t[kSgdMax];
+    uint32_t tile_start[kSgdMax + 1];
+    MultiSgd::Scalars k;
+};
+static_assert(sizeof(MultiSgdPlain) <= 4096, "kernel arguments exceed 4 KB");
+
+__device__ __forceinline__ void sgd_plain_tile(const MultiSgdPlain &args, uint32_t tile)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const bool started = lane + 1 < kSgdMax && args.tile_start[lane + 1] <= tile;
+    const int lo = __popcll(__ballot(started));
+    const TensorSgdPlain &t = args.t[lo];
+    const bool first = t.first_step != 0;
+    const int64_t i = (int64_t)(tile - args.tile_start[lo]) * kSgdPlainTile + threadIdx.x * 4;
+    if (i >= t.n)
+        return;
+    if (t.vec != 0 && i + 4 <= t.n) {
+        const float4 a = load4(t.p + i), b = load4(t.g + i);
+        float4 c = first ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : load4(t.buf + i);
+        float4 o;
+        o.x = sgd_elt(a.x, b.x, c.x, args.k, first);
+        o.y = sgd_elt(a.y, b.y, c.y, args.k, first);
+        o.z = sgd_elt(a.z, b.z, c.z, args.k, first);
+        o.w = sgd_elt(a.w, b.w, c.w, args.k, first);
+        store4(t.p + i, o);
+        store4(t.buf + i, c);
+    } else {
+        for (int64_t j = i; j < i + 4 && j < t.n; ++j) {
+            float b = first ? 0.0f : t.buf[j];
+            t.p[j] = sgd_elt(t.p[j], t.g[j], b, args.k, first);
+            t.buf[j] = b;
+        }
+    }
+}
+
+__global__ __launch_bounds__(kSgdThreads) void sgd_plain_kernel(const MultiSgdPlain args) { sgd_plain_tile(args, blockIdx.x); }
+
+// Both kinds in one launch, the quantised tensors' tiles first: a launch costs the host 2.7 us and the device as much again.  Steps apart ->
+// joined: three layers of width 256 (5M values) 27 -> 21, 48 of width 128 111 -> 101, four of width 384 28 -> 21, twelve of width 768 (85M)
+// 178.5 -> 176, a wide ResNet-152 465 -> 463.
+struct NoPlain {};
+
+// Plain: NoPlain, or the records of the tensors whose tiles follow the quantised ones' `tiles`.  (One kernel of two instances: the same
+// body in a function that two kernels call takes 85 registers instead of 70, and 5 to 8 % more time.)
+template <class Plain>
+__global__ __launch_bounds__(kSgdThreads) void sgd4bit_kernel(const MultiSgd args, const float *__restrict__ qmap, const Plain plain,
+                                                              uint32_t tiles)
 {
     __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
+    if constexpr (std::is_same_v<Plain, MultiSgdPlain>) {
+        if (blockIdx.x >= tiles) {
+            sgd_plain_tile(plain, blockIdx.x - tiles);
+            return;
+        }
+    }
     // tensor of this workgroup (uniform): the number of later tensors whose first tile is not after this one
     const int lane = threadIdx.x & (kWave - 1);
     const bool started = lane + 1 < kSgdMax && args.tile_start[lane + 1] <= blockIdx.x;
@@ -165,62 +240,7 @@ __global__ __launch_bounds__(kSgdThreads) void sgd4bit_kernel(const MultiSgd arg
     if (lane16 == 0)
         t.ms[grp] = amax;
 }
-
-// ---------------------------------------------------------------------------------------
-// The same chain on a float buffer: tensors whose buffer is not quantised (4096 values or fewer
-// by default: biases, norm weights).  As three or four torch operations each they took most of a
-// small model's step -- host time and launches, not bytes (the 51 vectors of a wide ResNet-152 among its 203
-// tensors: 150 launches and 0.25 ms of GPU time one after another; in one launch the whole step goes from
-// 1110-1120 to 466-470 us).  One tile
-// of 1024 values per workgroup: the tensors are short, and four values a thread are one 16-byte
-// access per operand where the pointers allow it.
-// ---------------------------------------------------------------------------------------
-constexpr int kSgdPlainTile = kSgdThreads * 4;
-
-struct TensorSgdPlain {
-    float *p;
-    const float *g;
-    float *buf;
-    int64_t n;
-    uint32_t first_step;
-    uint32_t vec;  // p, g and buf allow 16-byte accesses
-};
-
-struct MultiSgdPlain {
-    TensorSgdPlain t[kSgdMax];
-    uint32_t tile_start[kSgdMax + 1];
-    MultiSgd::Scalars k;
-};
-static_assert(sizeof(MultiSgdPlain) <= 4096, "kernel arguments exceed 4 KB");
-
-__global__ __launch_bounds__(kSgdThreads) void sgd_plain_kernel(const MultiSgdPlain args)
-{
-    const int lane = threadIdx.x & (kWave - 1);
-    const bool started = lane + 1 < kSgdMax && args.tile_start[lane + 1] <= blockIdx.x;
-    const int lo = __popcll(__ballot(started));
-    const TensorSgdPlain &t = args.t[lo];
-    const bool first = t.first_step != 0;
-    const int64_t i = (int64_t)(blockIdx.x - args.tile_start[lo]) * kSgdPlainTile + threadIdx.x * 4;
-    if (i >= t.n)
-        return;
-    if (t.vec != 0 && i + 4 <= t.n) {
-        const float4 a = load4(t.p + i), b = load4(t.g + i);
-        float4 c = first ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : load4(t.buf + i);
-        float4 o;
-        o.x = sgd_elt(a.x, b.x, c.x, args.k, first);
-        o.y = sgd_elt(a.y, b.y, c.y, args.k, first);
-        o.z = sgd_elt(a.z, b.z, c.z, args.k, first);
-        o.w = sgd_elt(a.w, b.w, c.w, args.k, first);
-        store4(t.p + i, o);
-        store4(t.buf + i, c);
-    } else {
-        for (int64_t j = i; j < i + 4 && j < t.n; ++j) {
-            float b = first ? 0.0f : t.buf[j];
-            t.p[j] = sgd_elt(t.p[j], t.g[j], b, args.k, first);
-            t.buf[j] = b;
-        }
-    }
-}
+static_assert(sizeof(MultiSgd) + sizeof(MultiSgdPlain) + 2 * sizeof(void *) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
 
 }  // namespace lpmm
 
@@ -240,14 +260,8 @@ static MultiSgd::Scalars sgd_scalars(double momentum, double dampening, double l
     return k;
 }
 
-extern "C" int lpmm_sgd4bit_step_multi(const lpmm_sgd4bit_tensor *tensors, int64_t count, const float *qmap,
-                                       double momentum, double dampening, double lr, double weight_decay,
-                                       int nesterov, int maximize, void *stream)
+static int check_sgd4(const lpmm_sgd4bit_tensor *tensors, int64_t count, const float *qmap)
 {
-    if (count < 0)
-        return LPMM_ERR_SIZE;
-    if (count == 0)
-        return LPMM_OK;
     LPMM_REQUIRE_PTR(tensors);
     LPMM_REQUIRE_PTR(qmap);
     LPMM_REQUIRE_ALIGN(qmap, 4);
@@ -266,40 +280,106 @@ extern "C" int lpmm_sgd4bit_step_multi(const lpmm_sgd4bit_tensor *tensors, int64
         LPMM_REQUIRE_ALIGN(t.m_codes, 2);
         LPMM_REQUIRE_ALIGN(t.m_max1, 4);
     }
+    return LPMM_OK;
+}
+
+// One launch's records from tensors[i] on: its tiles (0: none left).
+static uint32_t fill_sgd4(MultiSgd &args, const lpmm_sgd4bit_tensor *tensors, int64_t count, int64_t &i)
+{
+    int k = 0;
+    uint64_t tiles = 0;
+    args.tile_start[0] = 0;
+    while (i < count && k < kSgdMax) {
+        const lpmm_sgd4bit_tensor &t = tensors[i];
+        if (t.n == 0) {
+            ++i;
+            continue;
+        }
+        const uint64_t nt = (uint64_t)((t.n + kSgdTile - 1) / kSgdTile);
+        if (tiles + nt > 0x7fffffffULL)
+            break;
+        TensorSgd &d = args.t[k];
+        d.p = t.p;
+        d.g = t.g;
+        d.mc = t.m_codes;
+        d.ms = t.m_max1;
+        d.n = t.n;
+        d.first_step = t.first_step != 0;
+        d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16);
+        tiles += nt;
+        args.tile_start[++k] = (uint32_t)tiles;
+        ++i;
+    }
+    for (int j = k + 1; j <= kSgdMax; ++j)
+        args.tile_start[j] = (uint32_t)tiles;
+    return (uint32_t)tiles;
+}
+
+static int check_sgd_plain(const lpmm_sgd_fp32_tensor *tensors, int64_t count)
+{
+    LPMM_REQUIRE_PTR(tensors);
+    for (int64_t i = 0; i < count; ++i) {
+        const lpmm_sgd_fp32_tensor &t = tensors[i];
+        if (t.n < 0 || (t.n + kSgdPlainTile - 1) / kSgdPlainTile > 0x7fffffffLL)
+            return LPMM_ERR_SIZE;
+        if (t.n == 0)
+            continue;
+        LPMM_REQUIRE_PTR(t.p);
+        LPMM_REQUIRE_PTR(t.g);
+        LPMM_REQUIRE_PTR(t.buf);
+        LPMM_REQUIRE_ALIGN(t.p, 4);
+        LPMM_REQUIRE_ALIGN(t.g, 4);
+        LPMM_REQUIRE_ALIGN(t.buf, 4);
+    }
+    return LPMM_OK;
+}
+
+static uint32_t fill_sgd_plain(MultiSgdPlain &args, const lpmm_sgd_fp32_tensor *tensors, int64_t count, int64_t &i)
+{
+    int k = 0;
+    uint64_t tiles = 0;
+    args.tile_start[0] = 0;
+    while (i < count && k < kSgdMax) {
+        const lpmm_sgd_fp32_tensor &t = tensors[i];
+        const uint64_t nt = (uint64_t)((t.n + kSgdPlainTile - 1) / kSgdPlainTile);
+        if (tiles + nt > 0x7fffffffULL)
+            break;
+        ++i;
+        if (nt == 0)
+            continue;
+        TensorSgdPlain &d = args.t[k];
+        d.p = t.p;
+        d.g = t.g;
+        d.buf = t.buf;
+        d.n = t.n;
+        d.first_step = t.first_step != 0;
+        d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16) && aligned_to(t.buf, 16);
+        tiles += nt;
+        args.tile_start[++k] = (uint32_t)tiles;
+    }
+    for (int j = k + 1; j <= kSgdMax; ++j)
+        args.tile_start[j] = (uint32_t)tiles;
+    return (uint32_t)tiles;
+}
+
+extern "C" int lpmm_sgd4bit_step_multi(const lpmm_sgd4bit_tensor *tensors, int64_t count, const float *qmap,
+                                       double momentum, double dampening, double lr, double weight_decay,
+                                       int nesterov, int maximize, void *stream)
+{
+    if (count < 0)
+        return LPMM_ERR_SIZE;
+    if (count == 0)
+        return LPMM_OK;
+    const int bad = check_sgd4(tensors, count, qmap);
+    if (bad != LPMM_OK)
+        return bad;
     MultiSgd args;
     args.k = sgd_scalars(momentum, dampening, lr, weight_decay, nesterov, maximize);
-    int64_t i = 0;
-    while (i < count) {
-        int k = 0;
-        uint64_t tiles = 0;
-        args.tile_start[0] = 0;
-        while (i < count && k < kSgdMax) {
-            const lpmm_sgd4bit_tensor &t = tensors[i];
-            if (t.n == 0) {
-                ++i;
-                continue;
-            }
-            const uint64_t nt = (uint64_t)((t.n + kSgdTile - 1) / kSgdTile);
-            if (tiles + nt > 0x7fffffffULL)
-                break;
-            TensorSgd &d = args.t[k];
-            d.p = t.p;
-            d.g = t.g;
-            d.mc = t.m_codes;
-            d.ms = t.m_max1;
-            d.n = t.n;
-            d.first_step = t.first_step != 0;
-            d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16);
-            tiles += nt;
-            args.tile_start[++k] = (uint32_t)tiles;
-            ++i;
-        }
-        if (k == 0)
+    for (int64_t i = 0; i < count;) {
+        const uint32_t tiles = fill_sgd4(args, tensors, count, i);
+        if (tiles == 0)
             continue;
-        for (int j = k + 1; j <= kSgdMax; ++j)
-            args.tile_start[j] = (uint32_t)tiles;
-        hipLaunchKernelGGL(sgd4bit_kernel, dim3((uint32_t)tiles), dim3(kSgdThreads), 0, (hipStream_t)stream, args,
-                           qmap);
+        hipLaunchKernelGGL(sgd4bit_kernel<NoPlain>, dim3(tiles), dim3(kSgdThreads), 0, (hipStream_t)stream, args, qmap, NoPlain(), tiles);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;
@@ -315,53 +395,54 @@ extern "C" int lpmm_sgd_fp32_step_multi(const lpmm_sgd_fp32_tensor *tensors, int
         return LPMM_ERR_SIZE;
     if (count == 0)
         return LPMM_OK;
-    LPMM_REQUIRE_PTR(tensors);
-    for (int64_t i = 0; i < count; ++i) {
-        const lpmm_sgd_fp32_tensor &t = tensors[i];
-        if (t.n < 0 || (t.n + kSgdPlainTile - 1) / kSgdPlainTile > 0x7fffffffLL)
-            return LPMM_ERR_SIZE;
-        if (t.n == 0)
-            continue;
-        LPMM_REQUIRE_PTR(t.p);
-        LPMM_REQUIRE_PTR(t.g);
-        LPMM_REQUIRE_PTR(t.buf);
-        LPMM_REQUIRE_ALIGN(t.p, 4);
-        LPMM_REQUIRE_ALIGN(t.g, 4);
-        LPMM_REQUIRE_ALIGN(t.buf, 4);
-    }
+    const int bad = check_sgd_plain(tensors, count);
+    if (bad != LPMM_OK)
+        return bad;
     MultiSgdPlain args;
     args.k = sgd_scalars(momentum, dampening, lr, weight_decay, nesterov, maximize);
-    int64_t i = 0;
-    while (i < count) {
-        int k = 0;
-        uint64_t tiles = 0;
-        args.tile_start[0] = 0;
-        while (i < count && k < kSgdMax) {
-            const lpmm_sgd_fp32_tensor &t = tensors[i];
-            const uint64_t nt = (uint64_t)((t.n + kSgdPlainTile - 1) / kSgdPlainTile);
-            if (tiles + nt > 0x7fffffffULL)
-                break;
-            ++i;
-            if (nt == 0)
-                continue;
-            TensorSgdPlain &d = args.t[k];
-            d.p = t.p;
-            d.g = t.g;
-            d.buf = t.buf;
-            d.n = t.n;
-            d.first_step = t.first_step != 0;
-            d.vec = aligned_to(t.p, 16) && aligned_to(t.g, 16) && aligned_to(t.buf, 16);
-            tiles += nt;
-            args.tile_start[++k] = (uint32_t)tiles;
-        }
-        if (k == 0)
+    for (int64_t i = 0; i < count;) {
+        const uint32_t tiles = fill_sgd_plain(args, tensors, count, i);
+        if (tiles == 0)
             continue;
-        for (int j = k + 1; j <= kSgdMax; ++j)
-            args.tile_start[j] = (uint32_t)tiles;
-        hipLaunchKernelGGL(sgd_plain_kernel, dim3((uint32_t)tiles), dim3(kSgdThreads), 0, (hipStream_t)stream, args);
+        hipLaunchKernelGGL(sgd_plain_kernel, dim3(tiles), dim3(kSgdThreads), 0, (hipStream_t)stream, args);
         const int st = launch_status();
         if (st != LPMM_OK)
             return st;
     }
     return LPMM_OK;
+}
+
+extern "C" int lpmm_sgd4bit_fp32_step_multi(const lpmm_sgd4bit_tensor *tensors, int64_t count, const lpmm_sgd_fp32_tensor *plain,
+                                            int64_t plain_count, const float *qmap, double momentum, double dampening, double lr,
+                                            double weight_decay, int nesterov, int maximize, void *stream)
+{
+    if (count < 0 || plain_count < 0)
+        return LPMM_ERR_SIZE;
+    int st = count == 0 ? LPMM_OK : check_sgd4(tensors, count, qmap);
+    if (st == LPMM_OK && plain_count != 0)
+        st = check_sgd_plain(plain, plain_count);
+    if (st != LPMM_OK)
+        return st;
+    MultiSgd args;
+    MultiSgdPlain args_plain;
+    args.k = args_plain.k = sgd_scalars(momentum, dampening, lr, weight_decay, nesterov, maximize);
+    int64_t i = 0, j = 0;
+    while (i < count && j < plain_count) {
+        const int64_t from = i, from_plain = j;
+        const uint32_t tiles = fill_sgd4(args, tensors, count, i), tiles_plain = fill_sgd_plain(args_plain, plain, plain_count, j);
+        if (tiles == 0 || tiles_plain == 0 || (uint64_t)tiles + tiles_plain > 0x7fffffffULL) {
+            i = from;
+            j = from_plain;
+            break;
+        }
+        hipLaunchKernelGGL(sgd4bit_kernel<MultiSgdPlain>, dim3(tiles + tiles_plain), dim3(kSgdThreads), 0, (hipStream_t)stream, args, qmap,
+                           args_plain, tiles);
+        st = launch_status();
+        if (st != LPMM_OK)
+            return st;
+    }
+    st = lpmm_sgd4bit_step_multi(tensors + i, count - i, qmap, momentum, dampening, lr, weight_decay, nesterov, maximize, stream);
+    return st != LPMM_OK ? st
+                         : lpmm_sgd_fp32_step_multi(plain + j, plain_count - j, momentum, dampening, lr, weight_decay, nesterov, maximize,
+                                                    stream);
 }

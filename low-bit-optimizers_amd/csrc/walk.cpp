@@ -778,6 +778,7 @@ int takes_plain(const Batch &b)
     switch (b.kind) {
     case kFused4:
     case kFlat:
+    case kSgd4:
         return 2;
     case kRank1:
     case kNd:
@@ -793,7 +794,7 @@ int takes_plain(const Batch &b)
 }
 
 // The tensors with fp32 states that share the launches of the quantised tensors b (lpmm_adamw4bit_fp32_step_multi, its
-// non-fused form, lpmm_nonfused_rank1_fp32_step_multi), or null; they go with the first batch that takes them best.
+// non-fused form, lpmm_nonfused_rank1_fp32_step_multi, lpmm_sgd4bit_fp32_step_multi), or null; they go with the first batch that takes them best.
 // Decided here: a loop over the batches in Python cost every step 1.0 us, of 34 on three layers of width 128.
 const Batch *joined(const std::vector<Batch> &batches, const Batch &b)
 {
@@ -807,7 +808,7 @@ const Batch *joined(const std::vector<Batch> &batches, const Batch &b)
         const int takes = takes_plain(other);
         if (takes > best || (takes == best && &other < &b))
             return nullptr;
-        if (other.kind == kPlain)
+        if (other.kind == (b.kind == kSgd4 ? kSgdPlain : kPlain))
             plain = &other;
     }
     return plain;
@@ -865,7 +866,7 @@ PyObject *plan_start(PyObject *self, PyObject *)
         }
         const Batch *const plain = joined(*plan->batches, b);
         bool elsewhere = false;
-        if (b.kind == kPlain)
+        if (b.kind == kPlain || b.kind == kSgdPlain)
             for (const Batch &other : *plan->batches)
                 elsewhere = elsewhere || joined(*plan->batches, other) == &b;
         PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,

@@ -158,10 +158,15 @@ class SGD(LowBitOptimizer):
             if plan.served:
                 hyper = (momentum, dampening, group["lr"], group["weight_decay"], int(bool(group["nesterov"])),
                          int(bool(group["maximize"])))
-                for kind, index, qmap, _, _, count, records, _, _ in plan.start():
+                for kind, index, qmap, _, flag, count, records, plain, plain_count in plan.start():
+                    if flag:
+                        continue  # these go with the quantised tensors
                     with torch.cuda.device(index):
                         stream = _native.current_stream(index)
-                        if kind == _native.WALK_SGD4:
+                        if plain_count:
+                            st = _native.lib().lpmm_sgd4bit_fp32_step_multi(records, count, plain, plain_count, qmap.data_ptr(), *hyper,
+                                                                            stream)
+                        elif kind == _native.WALK_SGD4:
                             st = _native.lib().lpmm_sgd4bit_step_multi(records, count, qmap.data_ptr(), *hyper, stream)
                         else:
                             st = _native.lib().lpmm_sgd_fp32_step_multi(records, count, *hyper, stream)

@@ -239,3 +239,26 @@ def test_sgd_on_float_buffers_matches_oracle(oracle, hyper):
             assert got.dtype == torch.float32 and got.shape == params[i].shape
             assert np.array_equal(to_np(got), b) and np.array_equal(to_np(params[i]), h), (i, h.size, step)
             assert not to_np(stores[i][: i % 3]).any()
+
+
+@pytest.mark.parametrize("matrices,vectors", [(1, 1), (65, 3), (3, 130), (64, 64)])
+def test_float_buffers_beside_quantised_ones(matrices, vectors):
+    """One call for both kinds of tensors (lpmm_sgd4bit_fp32_step_multi), more of either than one launch takes (64), against a call
+    for each."""
+    import lpmm
+
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    start = [torch.randn(s, device="cuda", generator=gen) * 0.1 for s in [(2 + 37 * k % 3000,) for k in range(vectors)] + [(4100 + 13 * k,) for k in range(matrices)]]
+    both, apart = [[torch.nn.Parameter(s.clone()) for s in start] for _ in range(2)]
+    hyper = dict(lr=1e-2, momentum=0.9, weight_decay=1e-3, nesterov=True)
+    opts = [[lpmm.optim.SGD(both, **hyper)], [lpmm.optim.SGD(apart[:vectors], **hyper), lpmm.optim.SGD(apart[vectors:], **hyper)]]
+    for step in range(4):
+        for p, q in zip(both, apart):
+            p.grad = q.grad = torch.randn(p.shape, device="cuda", generator=gen)
+        for side in opts:
+            for opt in side:
+                opt.step()
+    assert all(torch.equal(p, q) for p, q in zip(both, apart))
+    for p, q in zip(both, apart):
+        a, b = opts[0][0].state[p], opts[1][0 if q.numel() < 4000 else 1].state[q]
+        assert torch.equal(a["momentum_buffer"], b["momentum_buffer"])
