@@ -654,7 +654,7 @@ int lpmm_factored_update(float *p, const float *g, uint8_t *m_codes, float *m_ma
 
 /* Both passes for a list of row-major R x C tensors whose column count is a multiple of 128
  * and whose first moment is quantised (4-bit, 'group', gp_sz 128): statistics and update of
- * all tensors in four launches per group of up to 24 tensors
+ * all tensors in three or four launches per group of up to 24 tensors (48 small ones)
  * instead of four per tensor.  Same results as
  * lpmm_factored_stats followed by lpmm_factored_update.  workspace: device scratch of
  * lpmm_factored_workspace_bytes(rows, cols) bytes per tensor, 8-byte aligned, not shared
@@ -679,8 +679,8 @@ int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int64_t count,
 
 /* The same for any column count and natural alignment, and for fp32 first moments: a record whose m_max1 is NULL
  * has m_codes pointing to float[rows * cols], updated in place (first_step is not read).  What
- * lpmm_factored_stats, lpmm_factored_update and lpmm_factored_update_fp32m compute, in four launches for up to
- * 24 tensors. */
+ * lpmm_factored_stats, lpmm_factored_update and lpmm_factored_update_fp32m compute, in three or four launches
+ * for up to 24 tensors (48 small ones). */
 int lpmm_factored_any_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
                                  double beta1, double beta2, double lr, double weight_decay, double eps,
                                  void *stream);

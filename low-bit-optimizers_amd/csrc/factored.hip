@@ -10,6 +10,8 @@
 // Row/column means of g*g are summed in double in a fixed order and rounded once.
 #include "lpmm_update.hpp"
 
+#include <type_traits>
+
 #include <mutex>
 
 namespace lpmm {
@@ -125,18 +127,20 @@ __global__ __launch_bounds__(kFThreads) void factored_partial_kernel(const float
 
 // Pass B: fold the partials in a fixed order and update the EMAs
 // (row.mul_(beta2).add_(mean, alpha=1-beta2): fma(mean, 1-beta2, row*beta2)).
-// Workgroups [0, row_blocks) take 256 rows each and leave the sum of their new row values in
-// rowblock[b]; the remaining workgroups take 64 columns each.
+// Workgroups [0, row_groups) take the rows, the others 64 columns each: 256 rows a workgroup, whose new values' sum they
+// leave in rowblock[b], or (ONE_ROW_GROUP: row_groups is 1) all rows in one, 256 at a time, and their mean.
+template <bool ONE_ROW_GROUP>
 __device__ __forceinline__ void finalize_body(const double *__restrict__ colpart, const double *__restrict__ rowpart,
                                               double *__restrict__ rowblock, int64_t R, int64_t C, int tiles_y,
-                                              int tiles_x, int row_blocks, float *__restrict__ row,
-                                              float *__restrict__ col, float b2, float w2, uint32_t bx)
+                                              int tiles_x, int row_groups, float *__restrict__ row,
+                                              float *__restrict__ col, float b2, float w2, uint32_t bx,
+                                              float *__restrict__ row_mean_all = nullptr)
 {
-    if ((int)bx >= row_blocks) {
+    if ((int)bx >= row_groups) {
         // 64 columns per workgroup; the partials of a column are split over 4 threads, each
         // summing its contiguous quarter 8 loads at a time, and folded in a fixed order
         __shared__ double s_col[kFThreads];
-        const int64_t c = (int64_t)(bx - row_blocks) * 64 + (threadIdx.x & 63);
+        const int64_t c = (int64_t)(bx - row_groups) * 64 + (threadIdx.x & 63);
         const int quarter = threadIdx.x >> 6;
         const int per = (tiles_y + 3) / 4;
         const int t0 = quarter * per, t1 = (t0 + per < tiles_y) ? t0 + per : tiles_y;
@@ -164,26 +168,38 @@ __device__ __forceinline__ void finalize_body(const double *__restrict__ colpart
         return;
     }
     __shared__ double s_sum[kFThreads];
-    const int64_t r = (int64_t)bx * kFThreads + threadIdx.x;
-    double mine = 0.0;
-    if (r < R) {
-        double s = 0.0;
-        for (int t = 0; t < tiles_x; ++t)
-            s += rowpart[(int64_t)t * R + r];
-        const float mean = (float)(s / (double)C);
-        const float nr = __builtin_fmaf(mean, w2, row[r] * b2);
-        row[r] = nr;
-        mine = (double)nr;
-    }
-    s_sum[threadIdx.x] = mine;
-    __syncthreads();
-    for (int o = kFThreads / 2; o > 0; o >>= 1) {
-        if (threadIdx.x < o)
-            s_sum[threadIdx.x] += s_sum[threadIdx.x + o];
+    double all = 0.0;
+    const int64_t end = ONE_ROW_GROUP ? R : (int64_t)(bx + 1) * kFThreads;
+    for (int64_t r0 = (int64_t)bx * kFThreads; r0 < end; r0 += kFThreads) {
+        const int64_t r = r0 + threadIdx.x;
+        double mine = 0.0;
+        if (r < R) {
+            double s = 0.0;
+            for (int t = 0; t < tiles_x; ++t)
+                s += rowpart[(int64_t)t * R + r];
+            const float mean = (float)(s / (double)C);
+            const float nr = __builtin_fmaf(mean, w2, row[r] * b2);
+            row[r] = nr;
+            mine = (double)nr;
+        }
+        s_sum[threadIdx.x] = mine;
         __syncthreads();
+        for (int o = kFThreads / 2; o > 0; o >>= 1) {
+            if (threadIdx.x < o)
+                s_sum[threadIdx.x] += s_sum[threadIdx.x + o];
+            __syncthreads();
+        }
+        if (ONE_ROW_GROUP) {
+            all += s_sum[0];
+            __syncthreads();
+        }
     }
-    if (threadIdx.x == 0)
-        rowblock[bx] = s_sum[0];
+    if (threadIdx.x == 0) {
+        if (ONE_ROW_GROUP)
+            *row_mean_all = (float)(all / (double)R);
+        else
+            rowblock[bx] = s_sum[0];
+    }
 }
 
 __global__ __launch_bounds__(kFThreads) void factored_finalize_kernel(const double *__restrict__ colpart,
@@ -193,7 +209,7 @@ __global__ __launch_bounds__(kFThreads) void factored_finalize_kernel(const doub
                                                                       int row_blocks, float *__restrict__ row,
                                                                       float *__restrict__ col, float b2, float w2)
 {
-    finalize_body(colpart, rowpart, rowblock, R, C, tiles_y, tiles_x, row_blocks, row, col, b2, w2, blockIdx.x);
+    finalize_body<false>(colpart, rowpart, rowblock, R, C, tiles_y, tiles_x, row_blocks, row, col, b2, w2, blockIdx.x);
 }
 
 // Pass C: mean(row) from the per-workgroup sums, in order.
@@ -475,7 +491,7 @@ __global__ __launch_bounds__(kFThreads) void factored_update_fp32m_kernel(
 // a prefix sum of workgroup counts kept in the kernel arguments and then does exactly what
 // the single-tensor kernels above do.
 // ---------------------------------------------------------------------------------------
-constexpr int kFaMax = 24;  // tensors per launch group
+constexpr int kFaMax = 24, kFaMany = 48;  // tensors per launch group: usual ones; small ones
 
 struct TensorFa {
     float *p;
@@ -491,13 +507,20 @@ struct TensorFa {
     int64_t R, C;
     int64_t n_padded;
     uint32_t tiles_x, tiles_y;  // statistics tiles
-    uint32_t row_blocks;        // finalize: workgroups that take rows; the rest take 64 columns each
+    uint32_t row_groups;        // finalize: workgroups that take rows; the rest take 64 columns each
     uint32_t upd_x;             // update: 2048-element tiles of the tensor
     uint32_t first_step : 1;
     // general launch groups: g allows 16-byte loads in the statistics pass, p and g in the update; the update's kind
     uint32_t vec_g : 1, vec : 1, kind : 2;
     float neg_step_size, bc2_sqrt, rbc2_sqrt;
 };
+
+// Groups of 48 where they hold few values, and, of tensors of at most 1024 rows, means by the workgroup that has all rows (the same sums
+// in the same order) in place of a launch: on small matrices a launch, 4.4 us on the device and 2.7 on the host, is what a step
+// consists of.  Steps in us, 24 a group and four launches -> this: 33 layers of an MLP of width 384 219 -> 192, 48 of width 128 148 -> 116, 48 of
+// width 256 169 -> 132, twelve of width 768 208 -> 193, 24 of width 512 202 -> 187; beyond these sizes the same.
+constexpr double kFaManyValues = 64e6;
+constexpr int64_t kOneGroupRows = 1024;
 
 // updates of a general launch group: fp32 first moment, a multiple of 8 columns, any other column count
 enum FlatKind : uint32_t { kFlatFloat = 0, kFlatRows = 1, kFlatAny = 2 };
@@ -508,25 +531,30 @@ enum FlatKind : uint32_t { kFlatFloat = 0, kFlatRows = 1, kFlatAny = 2 };
 // LLaMA-7B MLP shapes against 10.4 with groups bounded by the tensor count alone and streaming
 // loads in the statistics pass).
 
+template <int N>
 struct MultiFa {
-    TensorFa t[kFaMax];
+    static constexpr int kMax = N;
+    TensorFa t[N];
     // prefix sums of workgroups per tensor for the three big kernels; unused slots hold the total
-    uint32_t start_stats[kFaMax + 1], start_fin[kFaMax + 1], start_upd[kFaMax + 1];
+    uint32_t start_stats[N + 1], start_fin[N + 1], start_upd[N + 1];
     int count;
     float decay, w1, b2, w2, eps;
 };
 
-static_assert(sizeof(MultiFa) + sizeof(void *) <= 4096, "kernel arguments exceed 4 KB");
-static_assert(kFaMax <= kWave, "one prefix-sum entry per lane");
+static_assert(sizeof(MultiFa<kFaMax>) + sizeof(void *) <= 4096, "kernel arguments exceed 4 KB");
+static_assert(sizeof(MultiFa<kFaMany>) + sizeof(void *) <= kMostKernargBytes, "kernel arguments exceed 8 KB");
+static_assert(kFaMany <= kWave, "one prefix-sum entry per lane");
 
-__device__ __forceinline__ int find_slot(const uint32_t (&start)[kFaMax + 1], uint32_t block)
+template <int N>
+__device__ __forceinline__ int find_slot(const uint32_t (&start)[N], uint32_t block)
 {
     const int lane = threadIdx.x & (kWave - 1);
-    const bool started = lane + 1 < kFaMax && start[lane + 1] <= block;
+    const bool started = lane + 1 < N - 1 && start[lane + 1] <= block;
     return __popcll(__ballot(started));
 }
 
-__global__ __launch_bounds__(kFThreads) void factored_partial_multi_kernel(const MultiFa args)
+template <int N>
+__global__ __launch_bounds__(kFThreads) void factored_partial_multi_kernel(const MultiFa<N> args)
 {
     const int i = find_slot(args.start_stats, blockIdx.x);
     const TensorFa &t = args.t[i];
@@ -535,26 +563,29 @@ __global__ __launch_bounds__(kFThreads) void factored_partial_multi_kernel(const
     partial_body(t.g, t.R, t.C, t.colpart, t.rowpart, true, bx, by);
 }
 
-__global__ __launch_bounds__(kFThreads) void factored_finalize_multi_kernel(const MultiFa args)
+template <int N, bool ONE_ROW_GROUP>
+__global__ __launch_bounds__(kFThreads) void factored_finalize_multi_kernel(const MultiFa<N> args)
 {
     const int i = find_slot(args.start_fin, blockIdx.x);
     const TensorFa &t = args.t[i];
-    finalize_body(t.colpart, t.rowpart, t.rowblock, t.R, t.C, (int)t.tiles_y, (int)t.tiles_x, (int)t.row_blocks,
-                  t.row, t.col, args.b2, args.w2, blockIdx.x - args.start_fin[i]);
+    finalize_body<ONE_ROW_GROUP>(t.colpart, t.rowpart, t.rowblock, t.R, t.C, (int)t.tiles_y, (int)t.tiles_x, (int)t.row_groups,
+                                 t.row, t.col, args.b2, args.w2, blockIdx.x - args.start_fin[i], t.mean);
 }
 
-__global__ void factored_mean_multi_kernel(const MultiFa args)
+template <int N>
+__global__ void factored_mean_multi_kernel(const MultiFa<N> args)
 {
     const TensorFa &t = args.t[blockIdx.x];
     if (threadIdx.x == 0) {
         double s = 0.0;
-        for (uint32_t b = 0; b < t.row_blocks; ++b)
+        for (uint32_t b = 0; b < t.row_groups; ++b)
             s += t.rowblock[b];
         *t.mean = (float)(s / (double)t.R);
     }
 }
 
-__global__ __launch_bounds__(kFThreads) void factored_update_multi_kernel(const MultiFa args,
+template <int N>
+__global__ __launch_bounds__(kFThreads) void factored_update_multi_kernel(const MultiFa<N> args,
                                                                           const float *__restrict__ qmap_m)
 {
     const uint32_t block = blockIdx.x;
@@ -574,11 +605,12 @@ __global__ __launch_bounds__(kFThreads) void factored_update_multi_kernel(const 
                         t.first_step != 0, local);
 }
 
-// General launch groups: any column count and alignment, fp32 first moments.  One launch each for up to 24 tensors
+// General launch groups: any column count and alignment, fp32 first moments.  One launch each for the tensors of a group
 // in place of four per tensor, whose gaps and host time took most of a step on small matrices (three layers of
 // width 248: 295 -> 51 us a step; 48 layers of width 64, half of whose matrices keep fp32 first moments: 3110 -> 326).
 // The bodies are those of the single-tensor kernels: same results.
-__global__ __launch_bounds__(kFThreads) void factored_partial_any_multi_kernel(const MultiFa args)
+template <int N>
+__global__ __launch_bounds__(kFThreads) void factored_partial_any_multi_kernel(const MultiFa<N> args)
 {
     const int i = find_slot(args.start_stats, blockIdx.x);
     const TensorFa &t = args.t[i];
@@ -587,7 +619,8 @@ __global__ __launch_bounds__(kFThreads) void factored_partial_any_multi_kernel(c
     partial_body(t.g, t.R, t.C, t.colpart, t.rowpart, t.vec_g != 0, bx, by);
 }
 
-__global__ __launch_bounds__(kFThreads) void factored_update_any_multi_kernel(const MultiFa args,
+template <int N>
+__global__ __launch_bounds__(kFThreads) void factored_update_any_multi_kernel(const MultiFa<N> args,
                                                                               const float *__restrict__ qmap_m)
 {
     __shared__ __align__(16) uint32_t lds[kLdsBytes / 4];
@@ -888,22 +921,23 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
 
     const NfHyper c = make_nf_hyper(beta1, beta2, lr, weight_decay, eps, 1.0);
     NfHypers hypers(beta1, beta2, lr, weight_decay, eps);
-    MultiFa args;
-    args.decay = c.decay;
-    args.w1 = c.w1;
-    args.b2 = c.b2;
-    args.w2 = c.w2;
-    args.eps = c.eps;
     int64_t i = 0;
-    while (i < count) {
+    // one launch group from tensors[i] on
+    const auto launch = [&](auto &args, bool one_row_group) -> int {
+        constexpr int kMost = std::decay_t<decltype(args)>::kMax;
+        args.decay = c.decay;
+        args.w1 = c.w1;
+        args.b2 = c.b2;
+        args.w2 = c.w2;
+        args.eps = c.eps;
         int k = 0;
         uint64_t n_stats = 0, n_fin = 0, n_upd = 0;
         args.start_stats[0] = args.start_fin[0] = args.start_upd[0] = 0;
-        while (i < count && k < kFaMax) {
+        while (i < count && k < kMost) {
             const lpmm_factored_tensor &t = tensors[i];
             const uint64_t ty = (uint64_t)((t.rows + kSRows - 1) / kSRows), tx = (uint64_t)((t.cols + kSCols - 1) / kSCols);
             const uint64_t row_blocks = (uint64_t)((t.rows + kFThreads - 1) / kFThreads);
-            const uint64_t fin = row_blocks + (uint64_t)((t.cols + 63) / 64);
+            const uint64_t fin = (one_row_group ? 1 : row_blocks) + (uint64_t)((t.cols + 63) / 64);
             const uint64_t ux = general ? (uint64_t)((t.rows * t.cols + kFTile - 1) / kFTile) : update_tiles(t.rows, t.cols);
             if (n_stats + tx * ty > 0x7fffffffULL || n_fin + fin > 0x7fffffffULL ||
                 n_upd + ux > 0x7fffffffULL) {
@@ -927,7 +961,7 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
             d.n_padded = round_up(t.rows * t.cols, kFTile);
             d.tiles_x = (uint32_t)tx;
             d.tiles_y = (uint32_t)ty;
-            d.row_blocks = (uint32_t)row_blocks;
+            d.row_groups = one_row_group ? 1u : (uint32_t)row_blocks;
             d.upd_x = (uint32_t)ux;
             d.first_step = t.first_step != 0;
             d.vec_g = aligned_to(t.g, 16) && t.cols % 4 == 0;
@@ -947,23 +981,40 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
             ++i;
         }
         args.count = k;
-        for (int j = k + 1; j <= kFaMax; ++j) {
+        for (int j = k + 1; j <= kMost; ++j) {
             args.start_stats[j] = (uint32_t)n_stats;
             args.start_fin[j] = (uint32_t)n_fin;
             args.start_upd[j] = (uint32_t)n_upd;
         }
         hipStream_t s = (hipStream_t)stream;
         if (general)
-            hipLaunchKernelGGL(factored_partial_any_multi_kernel, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
+            hipLaunchKernelGGL(factored_partial_any_multi_kernel<kMost>, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
         else
-            hipLaunchKernelGGL(factored_partial_multi_kernel, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
-        hipLaunchKernelGGL(factored_finalize_multi_kernel, dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
-        hipLaunchKernelGGL(factored_mean_multi_kernel, dim3((uint32_t)k), dim3(kWave), 0, s, args);
+            hipLaunchKernelGGL(factored_partial_multi_kernel<kMost>, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
+        if (one_row_group) {
+            hipLaunchKernelGGL((factored_finalize_multi_kernel<kMost, true>), dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
+        } else {
+            hipLaunchKernelGGL((factored_finalize_multi_kernel<kMost, false>), dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
+            hipLaunchKernelGGL(factored_mean_multi_kernel<kMost>, dim3((uint32_t)k), dim3(kWave), 0, s, args);
+        }
         if (general)
-            hipLaunchKernelGGL(factored_update_any_multi_kernel, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
+            hipLaunchKernelGGL(factored_update_any_multi_kernel<kMost>, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
         else
-            hipLaunchKernelGGL(factored_update_multi_kernel, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
-        const int st = launch_status();
+            hipLaunchKernelGGL(factored_update_multi_kernel<kMost>, dim3((uint32_t)n_upd), dim3(kFThreads), 0, s, args, qmap_m);
+        return launch_status();
+    };
+    MultiFa<kFaMax> args;
+    MultiFa<kFaMany> many;
+    while (i < count) {
+        // what the next groups would hold
+        double values = 0;
+        int64_t rows = 0, held = 0;
+        for (int64_t j = i; j < count && held < kFaMany; ++j, ++held) {
+            values += (double)tensors[j].rows * (double)tensors[j].cols;
+            rows = tensors[j].rows > rows ? tensors[j].rows : rows;
+        }
+        const bool one_row_group = rows <= kOneGroupRows;
+        const int st = held > kFaMax && values <= kFaManyValues ? launch(many, one_row_group) : launch(args, one_row_group);
         if (st != LPMM_OK)
             return st;
     }

@@ -840,7 +840,8 @@ void join_matrices(std::vector<Batch> &batches)
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
 // that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
-// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1: flag 1 where tensors wrap.
+// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1: flag 1 where tensors wrap;
+// the factored kinds: how many to launch at a time, whose scratch is then held.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
     Plan *plan = reinterpret_cast<Plan *>(self);
@@ -869,9 +870,15 @@ PyObject *plan_start(PyObject *self, PyObject *)
         if (b.kind == kPlain || b.kind == kSgdPlain)
             for (const Batch &other : *plan->batches)
                 elsewhere = elsewhere || joined(*plan->batches, other) == &b;
+        int flag = elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.wraps ? 1 : b.flag;
+        if (b.kind == kFactored || b.kind == kFactoredAny) {
+            int64_t scratch = 0;  // floats
+            for (const Need &need : b.needs)
+                scratch += need.n;
+            flag = scratch <= (1 << 24) ? 48 : 24;
+        }
         PyObject *t = Py_BuildValue("(iiOOinKKK)", (int)b.kind, b.device, b.qm != nullptr ? b.qm : Py_None,
-                                    b.qv != nullptr ? b.qv : Py_None, elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.wraps ? 1 : b.flag,
-                                    (Py_ssize_t)b.items.size(),
+                                    b.qv != nullptr ? b.qv : Py_None, flag, (Py_ssize_t)b.items.size(),
                                     (unsigned long long)(uintptr_t)b.records.data(),
                                     (unsigned long long)(uintptr_t)(plain != nullptr ? plain->records.data() : b.second.data()),
                                     plain != nullptr && b.kind != kNd ? (unsigned long long)plain->items.size()

@@ -291,7 +291,7 @@ class AdamW(LowBitOptimizer):
                     st = lib.lpmm_nonfused_adamw_v4bit_step_multi(records, count, qv_ptr, *hyper, stream)
                 elif kind in (_native.WALK_FACTORED, _native.WALK_FACTORED_ANY):
                     run = lib.lpmm_factored_step_multi if kind == _native.WALK_FACTORED else lib.lpmm_factored_any_step_multi
-                    size, most = _native.FACTORED_TENSOR.itemsize, _native.FACTORED_MULTI_MAX
+                    size, most = _native.FACTORED_TENSOR.itemsize, flag
                     for i in range(0, count, most):
                         n = min(most, count - i)
                         plan.prepare(k, i, n)

@@ -307,3 +307,29 @@ def test_factored_any_step_multi_equals_single_tensor_calls(qmaps):
     bad[1] = 0
     table = np.array([tuple(bad)], dtype=_native.FACTORED_TENSOR)
     assert lib.lpmm_factored_any_step_multi(table.ctypes.data, 1, dqm.data_ptr(), *hyper, _stream()) != 0
+
+
+@pytest.mark.parametrize("count,rows,cols", [(25, 64, 128), (49, 64, 96), (30, 256, 128), (30, 257, 128), (25, 1024, 72), (25, 1025, 128), (2, 1500, 128)])
+def test_groups_of_small_tensors(count, rows, cols):
+    """More than 24 tensors in a group, and means without their launch (up to 1024 rows), on either kind of kernels, against the
+    single-tensor entry points (one tensor of more than 1024 rows beside each would change the route, not the result)."""
+    import lpmm
+
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    start = [torch.randn(rows, cols, device="cuda", generator=gen) * 0.1 for _ in range(count)]
+    tall = torch.randn(1300, cols, device="cuda", generator=gen) * 0.1
+    many, few = [[torch.nn.Parameter(s.clone()) for s in start] for _ in range(2)]
+    tails = [torch.nn.Parameter(tall.clone()) for _ in few]
+    make = lambda ps: lpmm.optim.AdamW(ps, lr=1e-2, factor_second_moment=True, fused=True)  # noqa: E731
+    opt, apart = make(many), [make([p, t]) for p, t in zip(few, tails)]
+    for step in range(4):
+        for p, q, t in zip(many, few, tails):
+            p.grad = q.grad = torch.randn(rows, cols, device="cuda", generator=gen)
+            t.grad = torch.ones_like(t)
+        for o in [opt] + apart:
+            o.step()
+    for k, (p, q) in enumerate(zip(many, few)):
+        assert torch.equal(p, q)
+        a, b = opt.state[p], apart[k].state[q]
+        for name in ("exp_avg", "exp_avg_sq_row", "exp_avg_sq_col"):
+            assert torch.equal(a[name], b[name]), name
