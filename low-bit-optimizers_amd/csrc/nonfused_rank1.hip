@@ -865,6 +865,32 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
     return LPMM_OK;
 }
 
+// Where the launch that begins with tensors[i] ends: after `most` tensors that are not empty, or, from 48M values on, where tensors that
+// wrap meet others: the kernel for both takes 1 to 3 % longer than the others' own, so that a large launch holds one kind (GPT-2-XL's
+// 50257 x 1600 embedding with 31 of its matrices, and too large a launch for the cache: 5255 -> 5207 us a step).  A launch
+// of its own for a few small ones would cost more.
+template <class Record>
+static int64_t launch_end(const Record *tensors, int64_t i, int64_t count, int most, bool can_fold)
+{
+    const auto wraps = [&](const Record &t) { return can_fold && t.cols % kGroup != 0 && !can_fold_rows(t.rows, t.cols, false); };
+    double values = 0;
+    int k = 0;
+    bool any_wraps = false, any_other = false;
+    for (; i < count && k < most; ++i) {
+        const Record &t = tensors[i];
+        if (t.rows == 0 || t.cols == 0)
+            continue;
+        const bool w = wraps(t);
+        if (values >= 48e6 && (w ? !any_wraps : !any_other))
+            break;
+        any_wraps = any_wraps || w;
+        any_other = any_other || !w;
+        values += (double)t.rows * (double)t.cols;
+        ++k;
+    }
+    return i;
+}
+
 // Validation, batching into launches of at most kR1Max tensors, and the launches.
 // m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
 // folds: a record per tensor, of ndim 0 where the tensor is a matrix (lpmm_nonfused_adamw4bit_rank1_nd_step_multi).
@@ -959,15 +985,13 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         args.w2 = c.w2;
         args.eps = c.eps;
         int k = 0;
+        const int64_t end = launch_end(tensors, i, count, kMost, can_fold);
         // what this launch will hold decides its tiles' rows
         LaunchKind kind = {half_io, M32, bits_m != 4, 0, {false, false}};
         const auto each = [&](auto &&f) {
-            int k = 0;
-            for (int64_t j = i; j < count && k < kMost; ++j)
-                if (tensors[j].rows != 0 && tensors[j].cols != 0) {
+            for (int64_t j = i; j < end; ++j)
+                if (tensors[j].rows != 0 && tensors[j].cols != 0)
                     f(tensors[j]);
-                    ++k;
-                }
         };
         int held = 0;
         each([&](const Record &t) {
@@ -994,7 +1018,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         int betweens = 0;
         int folded = kNoFold;  // what the launch's tensors need
         args.tile_start[0] = 0;
-        while (i < count && k < kMost) {
+        while (i < end) {
             const Record &t = tensors[i];
             if (t.rows == 0 || t.cols == 0) {
                 ++i;
@@ -1045,7 +1069,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             ++i;
         }
         if (k == 0) {
-            if (i < count)
+            if (i < end)
                 return LPMM_ERR_SIZE;  // a single tensor with more tiles than a grid holds
             return LPMM_OK;
         }
