@@ -142,9 +142,14 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, con
         x.a1 = load4(t.p + b);
         x.b0 = load4_for<KEEP>(t.g + a);
         x.b1 = load4_for<KEEP>(t.g + b);
-        x.m0 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (a >> 1)));
-        x.m1 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (b >> 1)));
-        x.sm = t.ms[a >> 7];
+        if (MODE == kMFloat) {
+            x.c0 = load4(reinterpret_cast<const float *>(t.mc) + a);
+            x.c1 = load4(reinterpret_cast<const float *>(t.mc) + b);
+        } else {
+            x.m0 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (a >> 1)));
+            x.m1 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (b >> 1)));
+            x.sm = t.ms[a >> 7];
+        }
         x.v0 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (a >> 1)));
         x.v1 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (b >> 1)));
         int64_t r0, r1;
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                                                                 const float *__restrict__ qmap_v)
 {
     constexpr int kSlots = FOLD == kWraps ? kFoldSlots : kRowSlots;
-    static_assert(!FOLD || MODE == kMCodes128, "folded rows: 4-bit first moments in groups of 128 values");
+    static_assert(!FOLD || MODE != kMCodesWide, "folded rows: first moments in groups of 128 values, or fp32");
     __shared__ __align__(16) uint32_t lds[(kColExtra + kMaxWide * kRedSlotWords * 4) / 4 + kSlots];
     uint32_t *colred = lds + kColExtra / 4;
     uint32_t *rowred = colred + kMaxWide * kRedSlotWords;
@@ -335,8 +340,10 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                 store4(pp + 64, make_float4(pv[4], pv[5], pv[6], pv[7]));
             if (M32) {
                 float *mp = reinterpret_cast<float *>(t.mc) + gbase + lane16 * 4;
-                store4(mp, make_float4(m[0], m[1], m[2], m[3]));
-                store4(mp + 64, make_float4(m[4], m[5], m[6], m[7]));
+                if (live_a)
+                    store4(mp, make_float4(m[0], m[1], m[2], m[3]));
+                if (live_b)
+                    store4(mp + 64, make_float4(m[4], m[5], m[6], m[7]));
             } else if (MODE == kMCodes128) {
                 uint16_t *mcp = reinterpret_cast<uint16_t *>(t.mc + (gbase >> 1)) + lane16;
                 store_u16(mcp, cm & 0xFFFFu);
@@ -805,6 +812,9 @@ static void launch_rank1(const R1LaunchN<N> &l, int folded, const float *qmap_m,
         if (folded != kNoFold)
             return folded == kDoubles ? launch_rank1_passes<MODE, kDoubles>(l, qmap_m, qmap_v, passes, stream)
                                       : launch_rank1_passes<MODE, kWraps>(l, qmap_m, qmap_v, passes, stream);
+    if constexpr (MODE == kMFloat)
+        if (folded != kNoFold)
+            return launch_rank1_passes<MODE, kWraps>(l, qmap_m, qmap_v, passes, stream);
     launch_rank1_passes<MODE, kNoFold>(l, qmap_m, qmap_v, passes, stream);
 }
 
@@ -911,7 +921,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     constexpr bool M32 = MODE == kMFloat;
     // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
     // served as double rows (rank1_tiles.hpp)
-    const bool can_fold = MODE == kMCodes128 && bits_m == 4 && !half_io;
+    // (fp32 first moments: as rows of any number, where the caller may)
+    const bool can_fold = bits_m == 4 && !half_io && !general && (MODE == kMCodes128 || (M32 && wraps));
     if (count < 0)
         return LPMM_ERR_SIZE;
     if (count == 0)
@@ -1050,7 +1061,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             d.col_tail = (uint32_t)(t.cols - (int64_t)(col_blocks - 1) * kGroup);
             // what the kernels for any column count took before
             d.tile.drop_nan = shape2[k].drop_nan =
-                m.lg != 0 && !can_fold_rows(t.rows, t.cols, false) && (t.cols % 8 != 0 || (folds != nullptr && folds[i].ndim != 0));
+                m.lg != 0 && (M32 || (!can_fold_rows(t.rows, t.cols, false) && (t.cols % 8 != 0 || (folds != nullptr && folds[i].ndim != 0))));
             const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
@@ -1115,7 +1126,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
                 return st;
             launch_rank1<MODE>(l, folded, qmap_m, qmap_v, 2, s);
         } else {
-            launch_rank1<MODE>(l, MODE == kMCodes128 ? folded : kNoFold, qmap_m, qmap_v, passes, s);
+            launch_rank1<MODE>(l, folded, qmap_m, qmap_v, passes, s);
         }
         return launch_status();
     };
@@ -1446,7 +1457,7 @@ extern "C" int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors
             break;
         case LPMM_STEP_FLOAT_M:
             st = rank1_step_multi<kMFloat>(static_cast<const lpmm_rank1_v4bit_tensor *>(tensors), count, qmap_v, qmap_v, 0, beta1, beta2,
-                                           lr, weight_decay, eps, stream, 4, 4, nullptr, nullptr, 3, false, nullptr, nullptr, &set);
+                                           lr, weight_decay, eps, stream, 4, 4, nullptr, nullptr, 3, false, nullptr, nullptr, &set, true);
             break;
         case LPMM_STEP_GROUPS:
             st = rank1_step_multi<kMCodesWide>(static_cast<const lpmm_rank1_mgroup_tensor *>(tensors), count, qmap_m, qmap_v,

@@ -87,7 +87,7 @@ struct Batch {
     std::vector<Record> items;
     std::vector<Swap> swaps;
     std::vector<Need> needs;
-    bool wraps = false;  // kRank1: a tensor that the kernels take as rows of several of its own
+    bool wraps = false;  // kRank1, kRank1M32: a tensor that the kernels take as rows of several of its own
 };
 
 struct Plan {
@@ -441,12 +441,13 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     }
     // the kernels that take 16 bytes an access; other operands go to the kernels for any column count
     const bool aligned = aligned16(r.p) && aligned16(r.g);
-    const bool whole = aligned && r.cols % 128 == 0, folds = aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
+    const bool whole = aligned && r.cols % 128 == 0, folds = en_m && aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
     // Rows of several tensor rows (Fold, rank1_tiles.hpp; the entry points that take them are those beside fp32 states and folds), in
     // place.  A tensor's first step here still goes the way of the steps in Python, whose kernels leave new scales, and of some columns
     // new codes, in arrays of their own: which tensors of a state a second step replaces is what callers know.  nd_scratch says
     // that it is done: True for a matrix, its entry "wraps" for others.
-    const bool may_wrap = en_m && s.m_group128 && s.v_rank1 && aligned && !whole && !folds && r.cols % 4 == 0 &&
+    const Ref m32 = en_m ? Ref() : reals_like(mo, p);
+    const bool may_wrap = (en_m ? s.m_group128 != 0 : m32 != nullptr && aligned16(ptr(*m32))) && s.v_rank1 && aligned && !whole && !folds && r.cols % 4 == 0 &&
                           (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
     const bool wraps = may_wrap && p.dim() == 2 && of_parameter(nd_scratch, po) == Py_True;
     const auto wraps_next = [&] {
@@ -468,18 +469,21 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     if (!en_m) {
-        const Ref m = reals_like(mo, p);
+        const Ref &m = m32;
         if (!s.v_rank1 || m == nullptr)
             return false;
-        if (!whole) {
+        if (!whole && !wraps) {
             item.swaps = 0;
+            wraps_next();
             return served && any(po, p, g, st, item, LPMM_RANK1_FLOAT_M, m, nullptr, vc, nullptr, oh_v, qm, qv);
         }
         if (!aligned16(ptr(*m)))
             return false;
         lpmm_rank1_v4bit_tensor f = {r.p, r.g, use<float>(m), r.v_codes, r.v_rowmax, r.v_colmax, r.v_rowmax_next, r.v_colmax_next,
                                      r.rows, r.cols, 0.0f, 0.0f};
-        add(batch(kRank1M32, p, nullptr, qv), f, item);
+        Batch &b = batch(kRank1M32, p, nullptr, qv);
+        add(b, f, item);
+        b.wraps = b.wraps || wraps;
         return true;
     }
     if (s.bits_rank1) {
@@ -840,7 +844,7 @@ void join_matrices(std::vector<Batch> &batches)
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
 // that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
-// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1: flag 1 where tensors wrap;
+// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1, kRank1M32: flag 1 where tensors wrap;
 // the factored kinds: how many to launch at a time, whose scratch is then held.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
