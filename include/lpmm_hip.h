@@ -577,7 +577,7 @@ int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensor
  * with the launch that clears the next statistics, as far as they fit.  Either may be empty.  kind: whose records `tensors`
  * holds, with the limits that its own entry point states -- lpmm_nonfused_rank1_tensor for _MATRIX, _BITS (bits_m, bits_v and the
  * tables; 4 and NULL elsewhere) and _ND (with folds), lpmm_rank1_v4bit_tensor for _FLOAT_M, lpmm_rank1_mgroup_tensor for _GROUPS
- * (m_group_size; 128 elsewhere).  _MATRIX, _FLOAT_M and _ND also take column counts that are 64 or from 128 to 2^24 and a multiple of 4, with
+ * (m_group_size; 128 elsewhere).  _MATRIX, _BITS, _FLOAT_M and _ND also take column counts that are 64 or from 128 to 2^24 and a multiple of 4, with
  * any row count.  lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
 enum {
     LPMM_STEP_MATRIX = 0,

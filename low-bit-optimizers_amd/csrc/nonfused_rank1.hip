@@ -921,8 +921,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     constexpr bool M32 = MODE == kMFloat;
     // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
     // served as double rows (rank1_tiles.hpp)
-    // (fp32 first moments: as rows of any number, where the caller may)
-    const bool can_fold = bits_m == 4 && !half_io && !general && (MODE == kMCodes128 || (M32 && wraps));
+    // (byte codes and fp32 first moments: as rows of any number, where the caller may)
+    const bool can_fold = !half_io && !general && (MODE == kMCodes128 ? bits_m == 4 || wraps : M32 && wraps);
     if (count < 0)
         return LPMM_ERR_SIZE;
     if (count == 0)
@@ -1061,7 +1061,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
             d.col_tail = (uint32_t)(t.cols - (int64_t)(col_blocks - 1) * kGroup);
             // what the kernels for any column count took before
             d.tile.drop_nan = shape2[k].drop_nan =
-                m.lg != 0 && (M32 || (!can_fold_rows(t.rows, t.cols, false) && (t.cols % 8 != 0 || (folds != nullptr && folds[i].ndim != 0))));
+                m.lg != 0 && (M32 || bits_m != 4 || (!can_fold_rows(t.rows, t.cols, false) && (t.cols % 8 != 0 || (folds != nullptr && folds[i].ndim != 0))));
             const NfHyper &h = hypers.at(t.step);
             d.neg_step_size = h.neg_step_size;
             d.bc2_sqrt = h.bc2_sqrt;
@@ -1114,7 +1114,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
                 return launch_status();
             }
             if (bits_m != 4) {
-                launch_rank1_bits(l, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
+                launch_rank1_bits(l, folded != kNoFold, qmap_m, qmap_v, bits_m, bits_v, static_cast<const uint32_t *>(table_m),
                                   static_cast<const uint32_t *>(table_v), s);
                 return launch_status();
             }
@@ -1450,7 +1450,7 @@ extern "C" int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors
         case LPMM_STEP_MATRIX:
         case LPMM_STEP_BITS:
             st = rank1_step_multi<kMCodes128>(matrices, count, qmap_m, qmap_v, 0, beta1, beta2, lr, weight_decay, eps, stream, bits_m,
-                                              bits_v, table_m, table_v, 3, false, nullptr, nullptr, &set, kind == LPMM_STEP_MATRIX);
+                                              bits_v, table_m, table_v, 3, false, nullptr, nullptr, &set, true);
             break;
         case LPMM_STEP_ND:
             st = nd_step_multi(matrices, folds, count, qmap_m, qmap_v, beta1, beta2, lr, weight_decay, eps, stream, &set);

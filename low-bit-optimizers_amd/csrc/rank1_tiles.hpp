@@ -163,7 +163,8 @@ __device__ __forceinline__ uint32_t xcd_neighbours(uint32_t index, uint32_t tile
 // groups' maxima between rows and write the first moment in the second pass, took 19 bytes a value, launches and new
 // code arrays of their own.  Steps in us: 50257 x 1600 345 -> 278, 31426 x 408 71 -> 62, six of 4096 x 4100 460 -> 343, 1000000 x 136 765 ->
 // 578, thirty of 88 x 88 x 3 x 3 111 -> 48 (the host in both), sixty of 56 x 56 x 3 x 3 208 -> 69;
-// fp32 first moment: 50257 x 1600 363 -> 341, six of 4096 x 4100 499 -> 434, 24 of 200 x 200 60 -> 36.  Double rows keep kernels of their own (whole
+// fp32 first moment: 50257 x 1600 363 -> 341, six of 4096 x 4100 499 -> 434, 24 of 200 x 200 60 -> 36;
+// 8 bits: 50257 x 1600 370 -> 307, six of 4096 x 4100 524 -> 385, 24 of 200 x 200 87 -> 37.  Double rows keep kernels of their own (whole
 // last rows, halves instead of runs): GPT-2-XL's 192 matrices take 4928 us with them, 4962 to 5025 without.
 struct Fold {
     uint32_t real_cols, col_blocks;  // columns of the tensor; column blocks of the matrix the kernel works on
@@ -309,7 +310,7 @@ struct R1LaunchN {
 using R1Launch = R1LaunchN<kR1Max>;
 
 // The launches of the other kernel families (defined next to their kernels).
-void launch_rank1_bits(const R1Launch &l, const float *qmap_m, const float *qmap_v, int bits_m,
+void launch_rank1_bits(const R1Launch &l, bool wraps, const float *qmap_m, const float *qmap_v, int bits_m,
                        int bits_v, const uint32_t *table_m, const uint32_t *table_v, hipStream_t stream);
 void launch_rank1_ragged(const R1Launch &l, const float *qmap_m, const float *qmap_v, hipStream_t stream);
 // any column count and alignment (nonfused_rank1_any.hip)

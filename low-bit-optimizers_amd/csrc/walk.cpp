@@ -87,7 +87,7 @@ struct Batch {
     std::vector<Record> items;
     std::vector<Swap> swaps;
     std::vector<Need> needs;
-    bool wraps = false;  // kRank1, kRank1M32: a tensor that the kernels take as rows of several of its own
+    bool wraps = false;  // kRank1, kRank1M32, kRank1Bits: a tensor that the kernels take as rows of several of its own
 };
 
 struct Plan {
@@ -441,13 +441,14 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     }
     // the kernels that take 16 bytes an access; other operands go to the kernels for any column count
     const bool aligned = aligned16(r.p) && aligned16(r.g);
-    const bool whole = aligned && r.cols % 128 == 0, folds = en_m && aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
+    const bool whole = aligned && r.cols % 128 == 0, folds = en_m && s.m_group128 && aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
     // Rows of several tensor rows (Fold, rank1_tiles.hpp; the entry points that take them are those beside fp32 states and folds), in
     // place.  A tensor's first step here still goes the way of the steps in Python, whose kernels leave new scales, and of some columns
     // new codes, in arrays of their own: which tensors of a state a second step replaces is what callers know.  nd_scratch says
     // that it is done: True for a matrix, its entry "wraps" for others.
     const Ref m32 = en_m ? Ref() : reals_like(mo, p);
-    const bool may_wrap = (en_m ? s.m_group128 != 0 : m32 != nullptr && aligned16(ptr(*m32))) && s.v_rank1 && aligned && !whole && !folds && r.cols % 4 == 0 &&
+    const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 : m32 != nullptr && aligned16(ptr(*m32))) &&
+                          (s.v_rank1 || s.bits_rank1) && aligned && !whole && !folds && r.cols % 4 == 0 &&
                           (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
     const bool wraps = may_wrap && p.dim() == 2 && of_parameter(nd_scratch, po) == Py_True;
     const auto wraps_next = [&] {
@@ -487,11 +488,14 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         return true;
     }
     if (s.bits_rank1) {
-        if (!whole) {
+        if (!whole && !wraps) {
             item.swaps = 0;
+            wraps_next();
             return served && any(po, p, g, st, item, LPMM_RANK1_CODES8, mc, ms, vc, oh_m, oh_v, qm, qv);
         }
-        add(batch(kRank1Bits, p, qm, qv), r, item);
+        Batch &b = batch(kRank1Bits, p, qm, qv);
+        add(b, r, item);
+        b.wraps = b.wraps || wraps;
         return true;
     }
     if (s.m_group128 && (whole || folds || wraps)) {
@@ -844,7 +848,7 @@ void join_matrices(std::vector<Batch> &batches)
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
 // that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
-// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1, kRank1M32: flag 1 where tensors wrap;
+// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1, kRank1M32, kRank1Bits: flag 1 where tensors wrap;
 // the factored kinds: how many to launch at a time, whose scratch is then held.
 PyObject *plan_start(PyObject *self, PyObject *)
 {

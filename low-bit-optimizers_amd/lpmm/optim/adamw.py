@@ -361,7 +361,7 @@ class AdamW(LowBitOptimizer):
         for i in range(0, count, most):
             n, table = min(most, count - i), records + i * size
             plan.prepare(k, i, n)
-            if plain_count or (flag and kind in (_native.WALK_RANK1, _native.WALK_RANK1_M32)):
+            if plain_count or (flag and kind != _native.WALK_ANY and kind != _native.WALK_RANK1_WIDE):
                 st = lib.lpmm_nonfused_rank1_fp32_step_multi(step, table, folds, n, plain, plain_count, group, *coding, *hyper, stream)
                 plain_count = 0
             elif kind == _native.WALK_ND:
