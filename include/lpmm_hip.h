@@ -578,13 +578,14 @@ int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensor
  * holds, with the limits that its own entry point states -- lpmm_nonfused_rank1_tensor for _MATRIX, _BITS (bits_m, bits_v and the
  * tables; 4 and NULL elsewhere) and _ND (with folds), lpmm_rank1_v4bit_tensor for _FLOAT_M, lpmm_rank1_mgroup_tensor for _GROUPS
  * (m_group_size; 128 elsewhere).  _MATRIX, _BITS, _FLOAT_M and _ND also take column counts that are 64 or from 128 to 2^24 and a multiple of 4, with
- * any row count.  lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
+ * any row count; _GROUPS_WRAP takes the records of _GROUPS with those and with multiples of 128 (_GROUPS: any multiple of 8).  lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
 enum {
     LPMM_STEP_MATRIX = 0,
     LPMM_STEP_BITS = 1,
     LPMM_STEP_ND = 2,
     LPMM_STEP_FLOAT_M = 3,
     LPMM_STEP_GROUPS = 4,
+    LPMM_STEP_GROUPS_WRAP = 5,
     LPMM_STEP_ANY = 8
 };
 int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors, const lpmm_rank1_small_vector *folds, int64_t count,

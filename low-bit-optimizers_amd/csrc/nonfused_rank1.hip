@@ -148,7 +148,7 @@ __device__ __forceinline__ void pass_fetch(const TensorR1 &t, const Fold &f, con
         } else {
             x.m0 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (a >> 1)));
             x.m1 = load_u16(reinterpret_cast<const uint16_t *>(t.mc + (b >> 1)));
-            x.sm = t.ms[a >> 7];
+            x.sm = t.ms[MODE == kMCodesWide ? (a >> 7) >> t.m_lg : a >> 7];
         }
         x.v0 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (a >> 1)));
         x.v1 = load_u16_for<KEEP>(reinterpret_cast<const uint16_t *>(t.vc + (b >> 1)));
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
                                                                 const float *__restrict__ qmap_v)
 {
     constexpr int kSlots = FOLD == kWraps ? kFoldSlots : kRowSlots;
-    static_assert(!FOLD || MODE != kMCodesWide, "folded rows: first moments in groups of 128 values, or fp32");
+    static_assert(FOLD != kDoubles || MODE == kMCodes128, "double rows: 4-bit first moments in groups of 128 values");
     __shared__ __align__(16) uint32_t lds[(kColExtra + kMaxWide * kRedSlotWords * 4) / 4 + kSlots];
     uint32_t *colred = lds + kColExtra / 4;
     uint32_t *rowred = colred + kMaxWide * kRedSlotWords;
@@ -552,6 +552,8 @@ __global__ __launch_bounds__(kThreads) void rank1_requant_kernel(const MultiR1N<
 #pragma unroll
             for (int k = 0; k < kEltsPerLane; ++k)
                 m[k] = lerp_w(decode_nibble(lds, kLdsQ0, nm, k) * ms_old, gv[k], h.w1);
+            if (FOLD == kWraps && ob > last)
+                zero_beyond(m, oa > last);
             store_u32(mcp, swap_code_halves(encode8_scaled(lds, kLdsQ0, kind_m, m, ms_new), code_sel));
         }
         uint32_t w;
@@ -812,7 +814,7 @@ static void launch_rank1(const R1LaunchN<N> &l, int folded, const float *qmap_m,
         if (folded != kNoFold)
             return folded == kDoubles ? launch_rank1_passes<MODE, kDoubles>(l, qmap_m, qmap_v, passes, stream)
                                       : launch_rank1_passes<MODE, kWraps>(l, qmap_m, qmap_v, passes, stream);
-    if constexpr (MODE == kMFloat)
+    if constexpr (MODE != kMCodes128)
         if (folded != kNoFold)
             return launch_rank1_passes<MODE, kWraps>(l, qmap_m, qmap_v, passes, stream);
     launch_rank1_passes<MODE, kNoFold>(l, qmap_m, qmap_v, passes, stream);
@@ -834,7 +836,7 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
         const Record &t = tensors[i];
         if (t.rows < 0 || t.cols < 0)
             return LPMM_ERR_SIZE;
-        if (!general && t.cols % (MODE == kMCodesWide ? 8 : kGroup) != 0 && !(can_fold && can_fold_rows(t.rows, t.cols, wraps)))
+        if (!general && t.cols % (MODE == kMCodesWide && !can_fold ? 8 : kGroup) != 0 && !(can_fold && can_fold_rows(t.rows, t.cols, wraps)))
             return LPMM_ERR_SIZE;
         if (t.rows == 0 || t.cols == 0)
             continue;
@@ -921,8 +923,8 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
     constexpr bool M32 = MODE == kMFloat;
     // 4-bit codes in 128-value groups: a column count of 64 modulo 128 with an even row count is
     // served as double rows (rank1_tiles.hpp)
-    // (byte codes and fp32 first moments: as rows of any number, where the caller may)
-    const bool can_fold = !half_io && !general && (MODE == kMCodes128 ? bits_m == 4 || wraps : M32 && wraps);
+    // (byte codes, fp32 first moments and wide groups: as rows of any number, where the caller may)
+    const bool can_fold = !half_io && !general && (wraps || (MODE == kMCodes128 && bits_m == 4));
     if (count < 0)
         return LPMM_ERR_SIZE;
     if (count == 0)
@@ -932,11 +934,11 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
         if (bad != LPMM_OK)
             return bad;
     }
-    // column counts that are no multiple of 128 (wide-group records only): every tensor of the call
+    // column counts that are no multiple of 128 (wide-group records only) and do not fold: every tensor of the call
     // then takes the kernels for ragged rows
     bool ragged = false;
     for (int64_t i = 0; i < count; ++i)
-        ragged = ragged || (MODE == kMCodesWide && tensors[i].cols % kGroup != 0);
+        ragged = ragged || (MODE == kMCodesWide && tensors[i].cols % kGroup != 0 && !can_fold);
 
     hipStream_t s = (hipStream_t)stream;
     if (passes & 1) {
@@ -1109,7 +1111,7 @@ static int rank1_step_multi(const Record *tensors, int64_t count, const float *q
                 launch_rank1_half(l, qmap_m, qmap_v, s);
                 return launch_status();
             }
-            if (ragged || (MODE == kMCodesWide && m_lg == 0)) {
+            if (ragged || (MODE == kMCodesWide && m_lg == 0 && folded == kNoFold)) {
                 launch_rank1_ragged(l, qmap_m, qmap_v, s);
                 return launch_status();
             }
@@ -1439,7 +1441,7 @@ extern "C" int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors
     if (table_v != nullptr)
         LPMM_REQUIRE_ALIGN(table_v, 16);
     const int m_lg = lg_of_group(m_group_size);
-    if (m_lg < 0 || (m_lg != 0 && kind != LPMM_STEP_GROUPS && kind != LPMM_STEP_ANY + LPMM_RANK1_CODES4))
+    if (m_lg < 0 || (m_lg != 0 && kind != LPMM_STEP_GROUPS && kind != LPMM_STEP_GROUPS_WRAP && kind != LPMM_STEP_ANY + LPMM_RANK1_CODES4))
         return LPMM_ERR_SIZE;
     PlainSet set = {plain, plain_count, 0};
     const auto matrices = static_cast<const lpmm_nonfused_rank1_tensor *>(tensors);
@@ -1460,9 +1462,10 @@ extern "C" int lpmm_nonfused_rank1_fp32_step_multi(int kind, const void *tensors
                                            lr, weight_decay, eps, stream, 4, 4, nullptr, nullptr, 3, false, nullptr, nullptr, &set, true);
             break;
         case LPMM_STEP_GROUPS:
+        case LPMM_STEP_GROUPS_WRAP:
             st = rank1_step_multi<kMCodesWide>(static_cast<const lpmm_rank1_mgroup_tensor *>(tensors), count, qmap_m, qmap_v,
                                                (uint32_t)m_lg, beta1, beta2, lr, weight_decay, eps, stream, 4, 4, nullptr, nullptr, 3,
-                                               false, nullptr, nullptr, &set);
+                                               false, nullptr, nullptr, &set, kind == LPMM_STEP_GROUPS_WRAP);
             break;
         case LPMM_STEP_ANY + LPMM_RANK1_CODES4:
         case LPMM_STEP_ANY + LPMM_RANK1_FLOAT_M:

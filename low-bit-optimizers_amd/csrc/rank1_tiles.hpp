@@ -164,7 +164,8 @@ __device__ __forceinline__ uint32_t xcd_neighbours(uint32_t index, uint32_t tile
 // code arrays of their own.  Steps in us: 50257 x 1600 345 -> 278, 31426 x 408 71 -> 62, six of 4096 x 4100 460 -> 343, 1000000 x 136 765 ->
 // 578, thirty of 88 x 88 x 3 x 3 111 -> 48 (the host in both), sixty of 56 x 56 x 3 x 3 208 -> 69;
 // fp32 first moment: 50257 x 1600 363 -> 341, six of 4096 x 4100 499 -> 434, 24 of 200 x 200 60 -> 36;
-// 8 bits: 50257 x 1600 370 -> 307, six of 4096 x 4100 524 -> 385, 24 of 200 x 200 87 -> 37.  Double rows keep kernels of their own (whole
+// 8 bits: 50257 x 1600 370 -> 307, six of 4096 x 4100 524 -> 385, 24 of 200 x 200 87 -> 37; groups of 256: 50257 x 1600
+// 337 -> 293, six of 4096 x 4100 456 -> 369.  Double rows keep kernels of their own (whole
 // last rows, halves instead of runs): GPT-2-XL's 192 matrices take 4928 us with them, 4962 to 5025 without.
 struct Fold {
     uint32_t real_cols, col_blocks;  // columns of the tensor; column blocks of the matrix the kernel works on

@@ -87,7 +87,7 @@ struct Batch {
     std::vector<Record> items;
     std::vector<Swap> swaps;
     std::vector<Need> needs;
-    bool wraps = false;  // kRank1, kRank1M32, kRank1Bits: a tensor that the kernels take as rows of several of its own
+    bool wraps = false;  // kRank1, kRank1M32, kRank1Bits, kRank1Wide: a tensor that the kernels take as rows of several of its own
 };
 
 struct Plan {
@@ -447,7 +447,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     // new codes, in arrays of their own: which tensors of a state a second step replaces is what callers know.  nd_scratch says
     // that it is done: True for a matrix, its entry "wraps" for others.
     const Ref m32 = en_m ? Ref() : reals_like(mo, p);
-    const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 : m32 != nullptr && aligned16(ptr(*m32))) &&
+    const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 || s.m_wide : m32 != nullptr && aligned16(ptr(*m32))) &&
                           (s.v_rank1 || s.bits_rank1) && aligned && !whole && !folds && r.cols % 4 == 0 &&
                           (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
     const bool wraps = may_wrap && p.dim() == 2 && of_parameter(nd_scratch, po) == Py_True;
@@ -504,22 +504,25 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
         b.wraps = b.wraps || wraps;
         return true;
     }
-    const bool ragged = aligned && !whole && r.cols % 8 == 0;
-    if (!whole && !ragged) {
+    const bool ragged = aligned && !whole && !wraps && r.cols % 8 == 0;
+    if (!whole && !ragged && !wraps) {
         item.swaps = 0;
         wraps_next();
         return served && (s.m_wide || s.m_group128) && any(po, p, g, st, item, LPMM_RANK1_CODES4, mc, ms, vc, oh_m, oh_v, qm, qv);
     }
     PyObject *spare = of_parameter(spare_scales, po);
     const Ref ms_next = reals_of(spare, p, ms->numel());
-    if (!((s.m_wide && whole) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
+    if (!((s.m_wide && (whole || wraps)) || ((s.m_wide || s.m_group128) && ragged)) || ms_next == nullptr)
         return false;
     lpmm_rank1_mgroup_tensor w = {r.p,        r.g,        r.m_codes,       r.m_max1,        use<float>(ms_next), r.v_codes, r.v_rowmax,
                                   r.v_colmax, r.v_rowmax_next, r.v_colmax_next, r.rows, r.cols, 0.0f, 0.0f};
     swap_later(item, spare_scales, po, get(oh_m, N.max1), hash_of(po));
     swap_later(item, oh_m, N.max1, spare);
-    wraps_next();
-    add(batch(kRank1Wide, p, qm, qv, ragged), w, item);
+    if (!wraps)
+        wraps_next();
+    Batch &b = batch(kRank1Wide, p, qm, qv, ragged);
+    add(b, w, item);
+    b.wraps = b.wraps || wraps;
     return true;
 }
 
@@ -848,7 +851,7 @@ void join_matrices(std::vector<Batch> &batches)
 // advances the step counts, completes the records; the batches: (kind, device, first map, second map, flag, count,
 // address of the records, address of the second pass's records or 0, address of the fold records or 0).  Quantised tensors
 // that others share launches with: the latter's records in the place of a second pass's, their count in that of the fold's (beside
-// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1, kRank1M32, kRank1Bits: flag 1 where tensors wrap;
+// a fold, in that of the flag), and flag 1 in the latter's own batch.  kRank1, kRank1M32, kRank1Bits, kRank1Wide: flag 1 where tensors wrap;
 // the factored kinds: how many to launch at a time, whose scratch is then held.
 PyObject *plan_start(PyObject *self, PyObject *)
 {
@@ -878,7 +881,7 @@ PyObject *plan_start(PyObject *self, PyObject *)
         if (b.kind == kPlain || b.kind == kSgdPlain)
             for (const Batch &other : *plan->batches)
                 elsewhere = elsewhere || joined(*plan->batches, other) == &b;
-        int flag = elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.wraps ? 1 : b.flag;
+        int flag = elsewhere ? 1 : plain != nullptr && b.kind == kNd ? (int)plain->items.size() : b.wraps ? 1 : b.kind == kRank1Wide ? 0 : b.flag;
         if (b.kind == kFactored || b.kind == kFactoredAny) {
             int64_t scratch = 0;  // floats
             for (const Need &need : b.needs)

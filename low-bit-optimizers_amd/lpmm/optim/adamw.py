@@ -348,6 +348,7 @@ class AdamW(LowBitOptimizer):
             plain_count, folds = flag, fold
         elif kind == _native.WALK_RANK1_WIDE:
             group = routes.m["gp_sz"]
+            step += bool(flag)  # LPMM_STEP_GROUPS_WRAP
         elif kind == _native.WALK_ANY:  # new codes: one launch's worth at a time
             step += flag
             bits, most, size = flag == _native.RANK1_CODES8, _native.RANK1_MULTI_MAX, _native.RANK1_ANY_TENSOR.itemsize
@@ -361,7 +362,7 @@ class AdamW(LowBitOptimizer):
         for i in range(0, count, most):
             n, table = min(most, count - i), records + i * size
             plan.prepare(k, i, n)
-            if plain_count or (flag and kind != _native.WALK_ANY and kind != _native.WALK_RANK1_WIDE):
+            if plain_count or (flag and kind != _native.WALK_ANY):
                 st = lib.lpmm_nonfused_rank1_fp32_step_multi(step, table, folds, n, plain, plain_count, group, *coding, *hyper, stream)
                 plain_count = 0
             elif kind == _native.WALK_ND:
