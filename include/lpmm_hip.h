@@ -374,7 +374,7 @@ int lpmm_nonfused_adamw4bit_rank1_pass_multi(const lpmm_nonfused_rank1_tensor *t
                                              double beta2, double lr, double weight_decay, double eps,
                                              int pass, void *stream);
 
-/* Both passes on tensors of more than two dimensions, and what lies between them, launch by launch: pass 1 on up to 32 tensors,
+/* Both passes on tensors of more than two dimensions, and what lies between them, launch by launch: pass 1 on up to 32 tensors (64 small ones),
  * lpmm_rank1_small_fold_scale_multi on their vectors, pass 2, so that the second pass of a launch finds in the cache what its first
  * has read.  tensors: the records of pass 1; folds[i]: the vector of tensors[i], x its v_colmax_next (cols values), scale what
  * pass 2 divides by (16-byte aligned, another array than v_colmax); ndim 0: a matrix, whose column maxima are its statistics. */
@@ -578,7 +578,8 @@ int lpmm_nonfused_adamw_rank1_any_step_multi(const lpmm_rank1_any_tensor *tensor
  * holds, with the limits that its own entry point states -- lpmm_nonfused_rank1_tensor for _MATRIX, _BITS (bits_m, bits_v and the
  * tables; 4 and NULL elsewhere) and _ND (with folds), lpmm_rank1_v4bit_tensor for _FLOAT_M, lpmm_rank1_mgroup_tensor for _GROUPS
  * (m_group_size; 128 elsewhere).  _MATRIX, _BITS, _FLOAT_M and _ND also take column counts that are 64 or from 128 to 2^24 and a multiple of 4, with
- * any row count; _GROUPS_WRAP takes the records of _GROUPS with those and with multiples of 128 (_GROUPS: any multiple of 8).  lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
+ * any row count; _GROUPS_WRAP takes the records of _GROUPS with those and with multiples of 128 (_GROUPS: any multiple of 8).
+ * lpmm_rank1_any_tensor for _ANY + LPMM_RANK1_CODES4, _FLOAT_M or _CODES8. */
 enum {
     LPMM_STEP_MATRIX = 0,
     LPMM_STEP_BITS = 1,
@@ -685,6 +686,12 @@ int lpmm_factored_step_multi(const lpmm_factored_tensor *tensors, int64_t count,
 int lpmm_factored_any_step_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m,
                                  double beta1, double beta2, double lr, double weight_decay, double eps,
                                  void *stream);
+
+/* Either of the two (any: lpmm_factored_any_step_multi) together with tensors with fp32 states, which go with the launch that finishes the
+ * statistics, as far as they fit: lpmm_adamw_fp32_step_multi (plain_fused) or lpmm_nonfused_update_multi.  Either may be empty. */
+int lpmm_factored_fp32_step_multi(const lpmm_factored_tensor *tensors, int64_t count, int any, const lpmm_adamw_fp32_tensor *plain,
+                                  int64_t plain_count, int plain_fused, const float *qmap_m, double beta1, double beta2, double lr,
+                                  double weight_decay, double eps, void *stream);
 
 /* The same pass with an fp32 first moment (m read and written as floats): tensors at or
  * under the quantisation threshold, or first-moment quantisation disabled

@@ -8,8 +8,9 @@
 // the hardware approximations with one fma correction of the residual (correctly rounded
 // except for a vanishing fraction of inputs; the parameter never feeds back into a state).
 // Row/column means of g*g are summed in double in a fixed order and rounded once.
-#include "lpmm_update.hpp"
+#include "lpmm_plain.hpp"
 
+#include <string.h>
 #include <type_traits>
 
 #include <mutex>
@@ -572,6 +573,23 @@ __global__ __launch_bounds__(kFThreads) void factored_finalize_multi_kernel(cons
                                  t.row, t.col, args.b2, args.w2, blockIdx.x - args.start_fin[i], t.mean);
 }
 
+// The same with tensors that have fp32 states, whose own launch this one saves (4 us on the device, 4 to 5 on the host): the first `tiles`
+// workgroups finish statistics.  Steps on three layers of an MLP of width 64 38 -> 32 us, of width 384 53 -> 46.
+template <bool ONE_ROW_GROUP, class Arith>
+__global__ __launch_bounds__(kFThreads) void factored_finalize_plain_kernel(const MultiFa<kFaMax> args, const MultiF plain, uint32_t tiles)
+{
+    if (blockIdx.x >= tiles) {
+        tile_fp32<Arith>(plain, blockIdx.x - tiles);
+        return;
+    }
+    const int i = find_slot(args.start_fin, blockIdx.x);
+    const TensorFa &t = args.t[i];
+    finalize_body<ONE_ROW_GROUP>(t.colpart, t.rowpart, t.rowblock, t.R, t.C, (int)t.tiles_y, (int)t.tiles_x, (int)t.row_groups,
+                                 t.row, t.col, args.b2, args.w2, blockIdx.x - args.start_fin[i], t.mean);
+}
+static_assert(sizeof(MultiFa<kFaMax>) + sizeof(MultiF) + 8 <= kMostKernargBytes, "kernel arguments exceed 8 KB");
+static_assert(kFThreads == kPlainThreads, "tile_fp32 runs in these kernels");
+
 template <int N>
 __global__ void factored_mean_multi_kernel(const MultiFa<N> args)
 {
@@ -883,7 +901,8 @@ extern "C" int lpmm_factored_update_fp32m(float *p, const float *g, float *m, co
 
 // general: any column count and natural alignment; a tensor without m_max1 has an fp32 first moment
 static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, const float *qmap_m, double beta1,
-                          double beta2, double lr, double weight_decay, double eps, bool general, void *stream)
+                          double beta2, double lr, double weight_decay, double eps, bool general, void *stream,
+                          PlainSet *plain = nullptr, bool plain_fused = false)
 {
     const uintptr_t align = general ? 4 : 16;
     if (count < 0)
@@ -991,10 +1010,42 @@ static int factored_multi(const lpmm_factored_tensor *tensors, int64_t count, co
             hipLaunchKernelGGL(factored_partial_any_multi_kernel<kMost>, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
         else
             hipLaunchKernelGGL(factored_partial_multi_kernel<kMost>, dim3((uint32_t)n_stats), dim3(kFThreads), 0, s, args);
-        if (one_row_group) {
+        bool joined = false;
+        if constexpr (kMost == kFaMax) {
+            MultiF args_f;
+            if (plain != nullptr && plain->next < plain->count) {
+                const int64_t first = plain->next;
+                const float b1 = (float)beta1, b2 = (float)beta2, e = (float)eps;
+                uint32_t tiles;
+                if (plain_fused) {
+                    const float scalars[7] = {b1, b2, 1 - b1, 1 - b2, (float)lr, (float)weight_decay, e};
+                    memcpy(args_f.s, scalars, sizeof args_f.s);
+                    tiles = fill_fp32(args_f, plain->tensors, plain->count, plain->next,
+                                      [=](float step, float(&k)[4]) { FusedArith::per_tensor(b1, b2, e, step, k); });
+                } else {
+                    const float scalars[7] = {c.decay, c.w1, c.b2, c.w2, c.eps, 0.0f, 0.0f};
+                    memcpy(args_f.s, scalars, sizeof args_f.s);
+                    tiles = fill_fp32(args_f, plain->tensors, plain->count, plain->next, [=](float step, float(&k)[4]) {
+                        NonFusedArith::per_tensor(beta1, beta2, lr, weight_decay, eps, step, k);
+                    });
+                }
+                joined = tiles != 0 && tiles <= 0x7fffffffu - (uint32_t)n_fin;
+                if (joined) {
+                    const auto kernel = plain_fused ? (one_row_group ? factored_finalize_plain_kernel<true, FusedArith>
+                                                                     : factored_finalize_plain_kernel<false, FusedArith>)
+                                                    : (one_row_group ? factored_finalize_plain_kernel<true, NonFusedArith>
+                                                                     : factored_finalize_plain_kernel<false, NonFusedArith>);
+                    hipLaunchKernelGGL(kernel, dim3((uint32_t)n_fin + tiles), dim3(kFThreads), 0, s, args, args_f, (uint32_t)n_fin);
+                } else if (tiles != 0) {
+                    plain->next = first;  // they go alone
+                }
+            }
+        }
+        if (!joined && one_row_group)
             hipLaunchKernelGGL((factored_finalize_multi_kernel<kMost, true>), dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
-        } else {
+        else if (!joined)
             hipLaunchKernelGGL((factored_finalize_multi_kernel<kMost, false>), dim3((uint32_t)n_fin), dim3(kFThreads), 0, s, args);
+        if (!one_row_group) {
             hipLaunchKernelGGL(factored_mean_multi_kernel<kMost>, dim3((uint32_t)k), dim3(kWave), 0, s, args);
         }
         if (general)
@@ -1033,4 +1084,24 @@ extern "C" int lpmm_factored_any_step_multi(const lpmm_factored_tensor *tensors,
                                             void *stream)
 {
     return factored_multi(tensors, count, qmap_m, beta1, beta2, lr, weight_decay, eps, true, stream);
+}
+
+extern "C" int lpmm_factored_fp32_step_multi(const lpmm_factored_tensor *tensors, int64_t count, int any, const lpmm_adamw_fp32_tensor *plain,
+                                             int64_t plain_count, int plain_fused, const float *qmap_m, double beta1, double beta2,
+                                             double lr, double weight_decay, double eps, void *stream)
+{
+    if (count < 0 || plain_count < 0)
+        return LPMM_ERR_SIZE;
+    if (plain_count != 0) {
+        const int bad = check_fp32(plain, plain_count, 4);
+        if (bad != LPMM_OK)
+            return bad;
+    }
+    PlainSet set = {plain, plain_count, 0};
+    const int st = factored_multi(tensors, count, qmap_m, beta1, beta2, lr, weight_decay, eps, any != 0, stream, &set, plain_fused != 0);
+    if (st != LPMM_OK)
+        return st;
+    return plain_fused ? lpmm_adamw_fp32_step_multi(plain + set.next, plain_count - set.next, (float)beta1, (float)beta2, (float)lr,
+                                                    (float)weight_decay, (float)eps, stream)
+                       : lpmm_nonfused_update_multi(plain + set.next, plain_count - set.next, beta1, beta2, lr, weight_decay, eps, stream);
 }

@@ -93,34 +93,6 @@ static_assert(LPMM_MULTI_MAX % 8 == 0, "coarse table");
 
 // The arithmetics the kernels are instantiated with.  They read the shared scalars from
 // Multi4::s / MultiF::s and the per-tensor ones from Tensor4::k / TensorF::k.
-struct FusedArith {
-    // code buffers hold exactly ceil(n/2) bytes; a last odd element leaves its high nibble 0
-    static constexpr bool kPadded = false;
-    Hyper h;
-    template <class M, class T>
-    __device__ __forceinline__ FusedArith(const M &a, const T &t)
-    {
-        h.beta1 = a.s[0];
-        h.beta2 = a.s[1];
-        h.omb1 = a.s[2];
-        h.omb2 = a.s[3];
-        h.lr = a.s[4];
-        h.wd = a.s[5];
-        h.eps = a.s[6];
-        h.c1 = t.k[0];   // 1 - beta1^step
-        h.c2s = t.k[1];  // sqrt(1 - beta2^step)
-        h.rc2s = t.k[2]; // 1 / c2s, correctly rounded (host division)
-    }
-    __device__ __forceinline__ void elt(float &p, float g, float &m, float &v) const { p = adamw_elt(p, g, m, v, h); }
-    // per-tensor scalars of a tensor at step `step`, as the reference computes them per thread
-    static void per_tensor(float beta1, float beta2, float eps, float step, float (&k)[4])
-    {
-        bias_corrections(beta1, beta2, step, &k[0], &k[1]);
-        k[2] = 1.0f / k[1];
-        k[3] = 0.0f;
-    }
-};
-
 // The 4-bit step: the moments as FusedArith computes them, the parameter with the folded update.
 struct FusedArith4 {
     static constexpr bool kPadded = false;

@@ -1,5 +1,6 @@
 // Tensors with fp32 states as part of a launch: records, tiles and checks of what fused_adamw.hip launches alone or beside quantised
-// tensors and nonfused_rank1.hip beside the clearing before its first pass; and the non-fused arithmetic.
+// tensors, nonfused_rank1.hip beside the clearing before its first pass and factored.hip beside the end of its statistics; and either
+// arithmetic.
 #pragma once
 #include "lpmm_update.hpp"
 
@@ -8,6 +9,34 @@
 namespace lpmm {
 
 constexpr int kPlainThreads = 256;
+
+struct FusedArith {
+    // code buffers hold exactly ceil(n/2) bytes; a last odd element leaves its high nibble 0
+    static constexpr bool kPadded = false;
+    Hyper h;
+    template <class M, class T>
+    __device__ __forceinline__ FusedArith(const M &a, const T &t)
+    {
+        h.beta1 = a.s[0];
+        h.beta2 = a.s[1];
+        h.omb1 = a.s[2];
+        h.omb2 = a.s[3];
+        h.lr = a.s[4];
+        h.wd = a.s[5];
+        h.eps = a.s[6];
+        h.c1 = t.k[0];   // 1 - beta1^step
+        h.c2s = t.k[1];  // sqrt(1 - beta2^step)
+        h.rc2s = t.k[2]; // 1 / c2s, correctly rounded (host division)
+    }
+    __device__ __forceinline__ void elt(float &p, float g, float &m, float &v) const { p = adamw_elt(p, g, m, v, h); }
+    // per-tensor scalars of a tensor at step `step`, as the reference computes them per thread
+    static void per_tensor(float beta1, float beta2, float eps, float step, float (&k)[4])
+    {
+        bias_corrections(beta1, beta2, step, &k[0], &k[1]);
+        k[2] = 1.0f / k[1];
+        k[3] = 0.0f;
+    }
+};
 
 struct NonFusedArith {
     // code buffers are padded to whole tiles plus one byte, as the reference's packing
@@ -37,6 +66,12 @@ struct NonFusedArith {
         k[2] = h.rbc2_sqrt;
         k[3] = 0.0f;
     }
+};
+
+// Tensors with fp32 states that go with the launches of a call; `next`: the first that has not gone yet.
+struct PlainSet {
+    const lpmm_adamw_fp32_tensor *tensors;
+    int64_t count, next;
 };
 
 struct TensorF {

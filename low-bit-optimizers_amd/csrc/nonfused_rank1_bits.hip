@@ -240,7 +240,8 @@ __global__ __launch_bounds__(kThreads) void rank1_update_bits_kernel(const Multi
         const int w = j & (kGroup - 1);
         const int k = ((w >> 6) << 2) | (w & 3), l = (w >> 2) & 15;
         if (tile_c0 + j < cols)
-            atomic_max_nonneg(t.col_new + (WRAPS ? fold_col(f, (uint32_t)(tile_c0 + j)) : tile_c0 + j), __uint_as_float(colred[(j >> 7) * kRedSlotWords + k * 16 + l]));
+            atomic_max_nonneg(t.col_new + (WRAPS ? fold_col(f, (uint32_t)(tile_c0 + j)) : tile_c0 + j),
+                              __uint_as_float(colred[(j >> 7) * kRedSlotWords + k * 16 + l]));
     }
 }
 

@@ -294,11 +294,7 @@ __device__ __forceinline__ uint32_t load_u16_for(const uint16_t *p) { return KEE
 template <bool KEEP>
 __device__ __forceinline__ uint32_t load_u32_for(const uint32_t *p) { return KEEP ? *p : load_u32(p); }
 
-// Tensors with fp32 states that go with the launches of a call; `next`: the first that has not gone yet.
-struct PlainSet {
-    const lpmm_adamw_fp32_tensor *tensors;
-    int64_t count, next;
-};
+struct PlainSet;  // lpmm_plain.hpp
 
 // One launch's tensors with the tile shapes of either pass (they differ: pass_rows_policy), and its workgroups.
 template <int N>

@@ -783,7 +783,7 @@ PyObject *plan_rest(PyObject *self, void *)
 }
 
 // Can a batch's launches take tensors with fp32 states along, and how well: 2, the one-pass kernels, 1, the launch that clears the
-// two-pass kernels' statistics, 0.
+// two-pass kernels' statistics or the one that finishes the factored ones', 0.
 int takes_plain(const Batch &b)
 {
     switch (b.kind) {
@@ -796,6 +796,8 @@ int takes_plain(const Batch &b)
     case kRank1M32:
     case kRank1Bits:
     case kRank1Wide:
+    case kFactored:
+    case kFactoredAny:
         return b.items.empty() ? 0 : 1;
     case kAny:
         return b.flag != LPMM_RANK1_HALF ? 1 : 0;
@@ -805,7 +807,7 @@ int takes_plain(const Batch &b)
 }
 
 // The tensors with fp32 states that share the launches of the quantised tensors b (lpmm_adamw4bit_fp32_step_multi, its
-// non-fused form, lpmm_nonfused_rank1_fp32_step_multi, lpmm_sgd4bit_fp32_step_multi), or null; they go with the first batch that takes them best.
+// non-fused form, lpmm_nonfused_rank1_fp32_step_multi, lpmm_factored_fp32_step_multi, lpmm_sgd4bit_fp32_step_multi), or null; they go with the first batch that takes them best.
 // Decided here: a loop over the batches in Python cost every step 1.0 us, of 34 on three layers of width 128.
 const Batch *joined(const std::vector<Batch> &batches, const Batch &b)
 {

@@ -86,6 +86,7 @@ PROTOTYPES = {
     "lpmm_factored_any_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 5 + [_vp]),
     "lpmm_factored_update_fp32m": (_int, [_vp] * 6 + [_i64, _i64] + [_d] * 6 + [_vp]),
     "lpmm_sgd4bit_step_multi": (_int, [_vp, _i64, _vp] + [_d] * 4 + [_int, _int, _vp]),
+    "lpmm_factored_fp32_step_multi": (_int, [_vp, _i64, _int, _vp, _i64, _int, _vp] + [_d] * 5 + [_vp]),
     "lpmm_sgd4bit_fp32_step_multi": (_int, [_vp, _i64, _vp, _i64, _vp] + [_d] * 4 + [_int] * 2 + [_vp]),
     "lpmm_sgd_fp32_step_multi": (_int, [_vp, _i64] + [_d] * 4 + [_int, _int, _vp]),
     "lpmm_stream_probe": (_int, [_int] + [_vp] * 6 + [_i64, _i64, _vp]),

@@ -295,7 +295,12 @@ class AdamW(LowBitOptimizer):
                     for i in range(0, count, most):
                         n = min(most, count - i)
                         plan.prepare(k, i, n)
-                        _native.check(run(records + i * size, n, qm_ptr, *hyper, stream), "factored step")
+                        if fold and i == 0:
+                            st = lib.lpmm_factored_fp32_step_multi(records, n, kind == _native.WALK_FACTORED_ANY, second, fold,
+                                                                   bool(group["fused"]), qm_ptr, *hyper, stream)
+                        else:
+                            st = run(records + i * size, n, qm_ptr, *hyper, stream)
+                        _native.check(st, "factored step")
                         plan.commit(k, i, n)
                     continue
                 elif kind == _native.WALK_HALF_PLAIN:

@@ -333,3 +333,27 @@ def test_groups_of_small_tensors(count, rows, cols):
         a, b = opt.state[p], apart[k].state[q]
         for name in ("exp_avg", "exp_avg_sq_row", "exp_avg_sq_col"):
             assert torch.equal(a[name], b[name]), name
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("matrices,vectors,rows", [(1, 1, 96), (24, 64, 96), (3, 70, 1100), (26, 5, 96)])
+def test_float_states_beside_the_statistics(matrices, vectors, rows, fused):
+    """Tensors with fp32 states go with the launch that finishes the factored ones' statistics: either arithmetic, with and without the
+    launch for the means, more of them than one launch takes (64), against optimizers of their own."""
+    import lpmm
+
+    gen = torch.Generator(device="cuda").manual_seed(10)
+    start = [torch.randn(s, device="cuda", generator=gen) * 0.1
+             for s in [(2 + 37 * k % 3000,) for k in range(vectors)] + [(rows, 128 if k % 2 else 72) for k in range(matrices)]]
+    both, apart = [[torch.nn.Parameter(s.clone()) for s in start] for _ in range(2)]
+    make = lambda ps: lpmm.optim.AdamW(ps, lr=1e-2, factor_second_moment=True, fused=fused)  # noqa: E731
+    opt, others = make(both), [make(apart[:vectors]), make(apart[vectors:])]
+    for step in range(4):
+        for p, q in zip(both, apart):
+            p.grad = q.grad = torch.randn(p.shape, device="cuda", generator=gen)
+        for o in [opt] + others:
+            o.step()
+    for k, (p, q) in enumerate(zip(both, apart)):
+        assert torch.equal(p, q), k
+        a, b = opt.state[p], others[k >= vectors].state[q]
+        assert all(torch.equal(a[n], b[n]) for n in a if torch.is_tensor(a[n]))

@@ -248,7 +248,8 @@ def test_float_buffers_beside_quantised_ones(matrices, vectors):
     import lpmm
 
     gen = torch.Generator(device="cuda").manual_seed(3)
-    start = [torch.randn(s, device="cuda", generator=gen) * 0.1 for s in [(2 + 37 * k % 3000,) for k in range(vectors)] + [(4100 + 13 * k,) for k in range(matrices)]]
+    start = [torch.randn(s, device="cuda", generator=gen) * 0.1
+             for s in [(2 + 37 * k % 3000,) for k in range(vectors)] + [(4100 + 13 * k,) for k in range(matrices)]]
     both, apart = [[torch.nn.Parameter(s.clone()) for s in start] for _ in range(2)]
     hyper = dict(lr=1e-2, momentum=0.9, weight_decay=1e-3, nesterov=True)
     opts = [[lpmm.optim.SGD(both, **hyper)], [lpmm.optim.SGD(apart[:vectors], **hyper), lpmm.optim.SGD(apart[vectors:], **hyper)]]
