@@ -395,6 +395,8 @@ def vectorwise_dequant(qx, denormalized=True, **kwargs):
         if (2 <= len(scaled_shape) <= RANK1_ND_MAX and numel(scaled_shape) > 0
                 and all(m.dtype is torch.float32 for m in max_dims)):
             dims, work = len(scaled_shape), None
+            if len(max_dims) != dims:  # the library reads as many addresses as there are dimensions
+                raise ValueError(f"{len(max_dims)} statistics do not belong to a tensor of shape {tuple(scaled_shape)}")
             if dims > 2:
                 max_dims = [m.contiguous() for m in max_dims]
                 for m, d in zip(max_dims, scaled_shape):

@@ -462,3 +462,32 @@ def test_every_shipped_configuration_merges_to_the_reference_settings():
         assert q.M.QUANT_TYPE.DEFAULT == "nonlinear" and q.SQM.QUANT_TYPE.DEFAULT == "power-1"
         assert q.M.ROUND_TYPE == "real-nearest" and q.SQM.ROUND_TYPE == "real-nearest"
         assert q.M.SIGNED is True and q.SQM.SIGNED is False and q.M.THRESHOLD == 4096
+
+
+@pytest.mark.parametrize("shape", [(6, 40), (6, 5, 40), (2, 3, 5, 8)])
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("count", [-1, 0, 1])
+def test_rank1_dequantise_takes_one_statistic_a_dimension(shape, bits, count, monkeypatch):
+    """A rank-1 state with a statistic too few or too many, as a truncated or foreign state dictionary holds it, is refused before the
+    library sees an address; the library is a stand-in that takes them."""
+    from lpmm import _native, functional
+
+    class Reached(Exception):
+        pass
+
+    class Lib:
+        def lpmm_dequant_rank1_nd(self, codes, dims, shape, stats, *rest):
+            assert dims == len(shape) == len(stats)
+            raise Reached
+
+    monkeypatch.setattr(functional, "_require_supported", lambda kwargs, x: None)
+    monkeypatch.setattr(torch.cuda, "device", lambda index: torch.no_grad())
+    monkeypatch.setattr(_native, "lib", Lib)
+    monkeypatch.setattr(_native, "current_stream", lambda index: 0)
+    stats = [torch.ones([d if i == k else 1 for k in range(len(shape))]) for i, d in enumerate(shape)]
+    stats = stats[:-1] if count < 0 else stats + stats[:count]
+    size = torch.Size(shape)
+    kw = dict(qmap=torch.zeros(2 ** bits), b=bits, scale_type="rank1", quant_type="power-1", round_type="real-nearest", gp_sz=128, signed=False,
+              dtype=torch.float32, stride=None, dim=len(shape), max1=None, max_dims=stats, scaled_shape=size, shape=size)
+    with pytest.raises(ValueError, match="statistics do not belong") if count else pytest.raises(Reached):
+        functional.vectorwise_dequant(torch.zeros(functional.packed_nbytes(size.numel(), bits), dtype=torch.int8), **kw)
