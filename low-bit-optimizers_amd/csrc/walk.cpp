@@ -450,7 +450,6 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 || s.m_wide : m32 != nullptr && aligned16(ptr(*m32))) &&
                           (s.v_rank1 || s.bits_rank1) && aligned && !whole && !folds && r.cols % 4 == 0 &&
                           (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
-    const bool wraps = may_wrap && p.dim() == 2 && of_parameter(nd_scratch, po) == Py_True;
     const auto wraps_next = [&] {
         if (may_wrap)
             swap_later(item, nd_scratch, po, Py_True, hash_of(po));
@@ -467,6 +466,8 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     r.v_colmax = now[1];
     r.v_rowmax_next = next[0];
     r.v_colmax_next = next[1];
+    // (their entry points take column statistics at 16 bytes, those for any column count at any float)
+    const bool wraps = may_wrap && of_parameter(nd_scratch, po) == Py_True && aligned16(r.v_colmax) && aligned16(r.v_colmax_next);
     swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     if (!en_m) {
