@@ -200,6 +200,19 @@ int64_t packed(int64_t n, int64_t group, bool bytes)
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
+// Does a matrix gain as rows of 2^lg tensor rows (Fold, rank1_tiles.hpp), which are as many times wider?  The kernels take tiles of 16 such
+// rows and 256 columns: with fewer rows there are up to 32 times as many tiles, and 5.5 ns each, mostly empty.  So it has 16, or at
+// most 512 tiles side by side, which cost less than the host saves.  Steps by the kernels for any column count -> as such rows, us: one of 1 x 1000004 72 -> 701,
+// of 31 x 50004 35 -> 88, of 64 x 50008 32 -> 82; sixteen of 256 x 20004 (8 rows) 384 -> 457, of 512 x 20004 (16) 745 -> 676; of 64 x 5004 (626
+// tiles side by side) 74 -> 94, of 64 x 5008 (313) 42 -> 41, of 64 x 1004 (126) 76 -> 35.
+bool worth_folding(int64_t rows, int64_t cols)
+{
+    int lg = 0;
+    while ((cols << lg) % 128 != 0)
+        ++lg;
+    return rows >= (int64_t)16 << lg || (cols << lg) / 128 <= 1024;
+}
+
 struct Settings {
     int fused;  // 0: the non-fused path, 1: the fused operators, 2: settings the fused operators warn about or refuse
     int m_group128, v_group128, v_rank1, m_wide, bits_rank1;
@@ -449,7 +462,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const Ref m32 = en_m ? Ref() : reals_like(mo, p);
     const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 || s.m_wide : m32 != nullptr && aligned16(ptr(*m32))) &&
                           (s.v_rank1 || s.bits_rank1) && aligned && !whole && !folds && r.cols % 4 == 0 &&
-                          (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24);
+                          (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24) && worth_folding(r.rows, r.cols);
     const auto wraps_next = [&] {
         if (may_wrap)
             swap_later(item, nd_scratch, po, Py_True, hash_of(po));

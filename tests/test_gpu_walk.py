@@ -538,3 +538,41 @@ def test_float_states_beside_the_clearing(config, shape, matrices, vectors, monk
         assert torch.equal(p, q)
         a, b = _state(sides[0][1], p), _state(sides[1][1], q)
         assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
+
+
+@pytest.mark.parametrize("config", ["default.yml", "2nd_moment_only_default.yml", "default_8b.yml", "1st_moment_group_256.yml"])
+@pytest.mark.parametrize("shape,in_place", [((1, 100004), False), ((31, 20004), False), ((127, 20008), False), ((511, 4100), False),
+                                            ((512, 4100), True), ((31, 4092), True), ((3, 8184), True)])
+def test_few_rows_of_many_columns(shape, in_place, config, monkeypatch):
+    """Rows of several tensor rows pay where the matrix has at least 16 of them, or no more than 512 tiles side by side: other shapes stay
+    with the kernels that they had, which leave new codes (of an fp32 first moment those of the second) or scales in other arrays."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    start = torch.randn(shape, device="cuda", generator=gen) * 0.1
+    sides = []
+    for _ in range(2):
+        p = torch.nn.Parameter(start.clone())
+        sides.append((p, lpmm.optim.AdamW([p], lr=1e-2, eps=1e-3, qconfig=path)))
+    for step in range(4):
+        grad = torch.randn(shape, device="cuda", generator=gen) * 0.1
+        held = dict(sides[0][1].state[sides[0][0]])
+        scales = held["exp_avg_qstate"]["overhead"].get("max1") if step else None
+        for serve, (p, opt) in zip((True, False), sides):
+            p.grad = grad
+            with monkeypatch.context() as patch:
+                native = _Native(_native, serve)
+                patch.setattr(adamw, "_native", native)
+                opt.step()
+                assert step < 2 or native.rest == (0 if serve else 1)
+        if step >= 2:
+            state = sides[0][1].state[sides[0][0]]
+            same = state["exp_avg_sq"] is held["exp_avg_sq"] and (
+                config.startswith("1st") or state["exp_avg_qstate"]["overhead"].get("max1") is scales)
+            assert same == in_place or (config.startswith("1st") and shape[1] % 8 == 0)  # those go by other kernels, in place too
+    assert torch.equal(sides[0][0], sides[1][0])
+    a, b = (_state(opt, p) for p, opt in sides)
+    assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
