@@ -912,9 +912,7 @@ class AdamW(LowBitOptimizer):
         state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), 4))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
-        nxt = self._spare_stats.get(p)
-        if nxt is None or nxt[0].device != dev or nxt[0].dtype is not torch.float16:
-            nxt = [torch.empty_like(cur[0]), torch.empty_like(cur[1])]
+        nxt = self._spare_pair(p, cur)
         work = torch.empty(((rows + 3) // 4 * 4 + cols + ((rows * cols + 127) // 128 if with_groups else 0),),
                            dtype=torch.float32, device=dev)
 
@@ -1042,9 +1040,7 @@ class AdamW(LowBitOptimizer):
         state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), b))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
-        nxt = self._spare_stats.get(p)
-        if nxt is None or nxt[0].device != dev:
-            nxt = [torch.empty_like(cur[0]), torch.empty_like(cur[1])]
+        nxt = self._spare_pair(p, cur)
 
         def commit():
             self._spare_stats[p] = cur
@@ -1100,10 +1096,7 @@ class AdamW(LowBitOptimizer):
                 else:
                     mc, ms, ms_next = self._group_state_pair(p, state, batch)
                 vc, cur, nxt = self._rank1_nd_state(p, state, batch)
-                scratch = self._nd_scratch.get(p)
-                if scratch is None or scratch["work"].device != p.device:
-                    scratch = self._nd_scratch[p] = {
-                        "work": torch.empty((3, _nd_pitch(cols)), dtype=torch.float32, device=p.device), "scale_of": None, "row": 0}
+                scratch = self._nd_scratch_of(p, cols)
                 work = scratch["work"]
                 # rows of `work`: the column scale of the current statistics, the column maxima of the new
                 # second moment, the column scale of the next statistics.  The last step's third row is this
@@ -1192,9 +1185,7 @@ class AdamW(LowBitOptimizer):
         state["exp_avg_sq"] = whole_codes(state["exp_avg_sq"], packed_nbytes(p.numel(), 4))
         oh = qs_v["overhead"]
         cur = oh["max_dims"]
-        nxt = self._spare_stats.get(p)
-        if nxt is None or len(nxt) != len(cur) or nxt[0].device != dev:
-            nxt = [torch.empty_like(t) for t in cur]
+        nxt = self._spare_pair(p, cur)
 
         def commit():
             self._spare_stats[p] = cur
@@ -1214,6 +1205,13 @@ class AdamW(LowBitOptimizer):
             d = self.__dict__["_nd_scratch_by_param"] = {}
         return d
 
+    def _nd_scratch_of(self, p, cols):
+        scratch = self._nd_scratch.get(p)
+        if scratch is None or scratch["work"].device != p.device or scratch["work"].shape != (3, _nd_pitch(cols)):
+            scratch = self._nd_scratch[p] = {
+                "work": torch.empty((3, _nd_pitch(cols)), dtype=torch.float32, device=p.device), "scale_of": None, "row": 0}
+        return scratch
+
     @property
     def _spare_stats(self):
         # second pair of row/column statistics per parameter; not part of the optimizer state
@@ -1222,6 +1220,15 @@ class AdamW(LowBitOptimizer):
         if d is None:
             d = self.__dict__["_spare_stats_by_param"] = {}
         return d
+
+    def _spare_pair(self, p, cur):
+        """Where the next statistics go: the spare ones, if they are as the current ones (a parameter may have been given another
+        shape and a fresh state), else new ones."""
+        nxt = self._spare_stats.get(p)
+        if nxt is None or len(nxt) != len(cur) or any(
+                a.numel() != b.numel() or a.device != b.device or a.dtype != b.dtype for a, b in zip(nxt, cur)):
+            nxt = [torch.empty_like(t) for t in cur]
+        return nxt
 
     @property
     def _spare_scales(self):

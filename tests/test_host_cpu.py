@@ -491,3 +491,32 @@ def test_rank1_dequantise_takes_one_statistic_a_dimension(shape, bits, count, mo
               dtype=torch.float32, stride=None, dim=len(shape), max1=None, max_dims=stats, scaled_shape=size, shape=size)
     with pytest.raises(ValueError, match="statistics do not belong") if count else pytest.raises(Reached):
         functional.vectorwise_dequant(torch.zeros(functional.packed_nbytes(size.numel(), bits), dtype=torch.int8), **kw)
+
+
+@pytest.mark.parametrize("first,second", [((66, 33, 2, 2), (40, 132)), ((40, 132), (40, 200)), ((200, 40), (132, 132)), ((40, 132), (66, 33, 4)),
+                                          ((66, 33, 2), (66, 34, 2)), ((66, 8, 8), (66, 64, 1))])
+@pytest.mark.parametrize("half", [False, True])
+def test_spare_statistics_of_a_parameter_that_changed_its_shape(first, second, half):
+    """A parameter given another shape and a fresh state: what the kernels write the next statistics to, and the vectors between the
+    passes, have the new sizes."""
+    import lpmm
+    from lpmm.optim.adamw import _Batch, _nd_pitch
+
+    p = torch.nn.Parameter(torch.zeros(first, dtype=torch.float16 if half else torch.float32))
+    opt = lpmm.optim.AdamW([p])
+    for shape in (first, second, second):
+        if half and len(shape) != 2:
+            continue
+        p.data = torch.zeros(shape, dtype=p.dtype)
+        opt.state.clear()
+        state, _ = opt._state_of(opt.param_groups[0], p)
+        for step in range(2):
+            batch = _Batch()
+            (opt._rank1_state_f16 if half else opt._rank1_state if len(shape) == 2 else opt._rank1_nd_state)(p, state, batch)
+            batch.launched()
+            stats = state["exp_avg_sq_qstate"]["overhead"]["max_dims"]
+            for pair in (stats, opt._spare_stats[p]):
+                assert [t.numel() for t in pair] == list(shape) and all(t.dtype == p.dtype for t in pair)
+        if len(shape) > 2:
+            cols = p.numel() // shape[0]
+            assert opt._nd_scratch_of(p, cols)["work"].shape == (3, _nd_pitch(cols)) and opt._nd_scratch_of(p, cols) is opt._nd_scratch[p]
