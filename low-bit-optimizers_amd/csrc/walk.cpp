@@ -43,7 +43,7 @@ constexpr size_t kRecordBytes[kKinds] = {
 
 struct Names {
     PyObject *step, *exp_avg, *exp_avg_sq, *exp_avg_qstate, *exp_avg_sq_qstate, *exp_avg_sq_row, *exp_avg_sq_col, *enable, *overhead, *qmap, *max1,
-        *max_dims, *work, *scale_of, *row, *wraps, *momentum_buffer, *momentum_buffer_qstate, *dtype;
+        *max_dims, *work, *scale_of, *row, *momentum_buffer, *momentum_buffer_qstate, *dtype;
 } N;
 
 // dict[key] = value, once the launch is on the stream; strong references.  hash: of a key that is a parameter, else -1
@@ -221,7 +221,7 @@ struct Settings {
 
 struct Walk {
     Plan *plan;
-    PyObject *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
+    PyObject *state, *override_, *spare_stats, *spare_scales, *nd_scratch, *in_place;
     Settings s;
     size_t most;  // records of a batch: the group's tensors, fewer at first where they are many
     int64_t (*workspace_bytes)(int64_t, int64_t);  // lpmm_factored_workspace_bytes
@@ -456,16 +456,15 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     const bool aligned = aligned16(r.p) && aligned16(r.g);
     const bool whole = aligned && r.cols % 128 == 0, folds = en_m && s.m_group128 && aligned && r.cols % 128 == 64 && r.rows % 2 == 0;
     // Rows of several tensor rows (Fold, rank1_tiles.hpp; the entry points that take them are those beside fp32 states and folds), in
-    // place.  A tensor's first step here still goes the way of the steps in Python, whose kernels leave new scales, and of some columns
-    // new codes, in arrays of their own: which tensors of a state a second step replaces is what callers know.  nd_scratch says
-    // that it is done: True for a matrix, its entry "wraps" for others.
+    // place.  A state's first step here still goes the way of the steps in Python, whose kernels leave new scales, and of some columns
+    // new codes, in arrays of their own.  in_place says for which state that is done: the second moment's overhead.
     const Ref m32 = en_m ? Ref() : reals_like(mo, p);
     const bool may_wrap = (en_m ? s.m_group128 || s.bits_rank1 || s.m_wide : m32 != nullptr && aligned16(ptr(*m32))) &&
                           (s.v_rank1 || s.bits_rank1) && aligned && !whole && !folds && r.cols % 4 == 0 &&
                           (r.cols >= 128 || r.cols == 64) && r.cols <= (1 << 24) && worth_folding(r.rows, r.cols);
     const auto wraps_next = [&] {
         if (may_wrap)
-            swap_later(item, nd_scratch, po, Py_True, hash_of(po));
+            swap_later(item, in_place, po, oh_v, hash_of(po));
     };
     const bool served = r.cols >= 32 || r.rows <= 32768;  // _any_columns
     if (p.dim() > 2)
@@ -480,7 +479,7 @@ bool Walk::adamw(PyObject *po, const at::Tensor &p, const at::Tensor &g, PyObjec
     r.v_rowmax_next = next[0];
     r.v_colmax_next = next[1];
     // (their entry points take column statistics at 16 bytes, those for any column count at any float)
-    const bool wraps = may_wrap && of_parameter(nd_scratch, po) == Py_True && aligned16(r.v_colmax) && aligned16(r.v_colmax_next);
+    const bool wraps = may_wrap && of_parameter(in_place, po) == oh_v && aligned16(r.v_colmax) && aligned16(r.v_colmax_next);
     swap_later(item, spare_stats, po, cur, hash_of(po));
     swap_later(item, oh_v, N.max_dims, nxt);
     if (!en_m) {
@@ -673,7 +672,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
         return false;
     PyObject *cur = get(oh_v, N.max_dims), *nxt = of_parameter(spare_stats, po), *scratch = of_parameter(nd_scratch, po);
     PyObject *row = get(scratch, N.row);
-    if (may_wrap && get(scratch, N.wraps) == Py_True)
+    if (may_wrap && of_parameter(in_place, po) == oh_v)
         any_mc = nullptr;
     const int64_t pitch = (r.cols + 31) / 32 * 32;  // _nd_pitch
     const Ref work = reals_of(get(scratch, N.work), p, 3 * pitch);
@@ -716,7 +715,7 @@ bool Walk::nd(PyObject *po, const at::Tensor &p, Item &item, lpmm_nonfused_rank1
     swap_later(item, scratch, N.scale_of, nxt);
     swap_later(item, scratch, N.row, row_obj);
     if (may_wrap && any_mc != nullptr)
-        swap_later(item, scratch, N.wraps, Py_True);
+        swap_later(item, in_place, po, oh_v, hash_of(po));
     if (any_mc == nullptr) {
         Batch &b = batch(kNd, p, qm, qv);
         add(b, r, item);
@@ -1032,17 +1031,18 @@ PyGetSetDef plan_getset[] = {{"served", plan_served, nullptr, "are there records
 PyTypeObject PlanType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
 // collect(sgd, params, state, override, spare_stats, spare_scales, nd_scratch, serve, settings,
-// address of lpmm_factored_workspace_bytes or 0)
+// address of lpmm_factored_workspace_bytes or 0, in_place)
 PyObject *collect(PyObject *, PyObject *args)
 {
     int is_sgd, serve;
-    PyObject *params, *state, *override_, *spare_stats, *spare_scales, *nd_scratch;
+    PyObject *params, *state, *override_, *spare_stats, *spare_scales, *nd_scratch, *in_place;
     Walk w;
     int m_group;
     unsigned long long workspace;
-    if (!PyArg_ParseTuple(args, "iO!O!O!O!O!O!p(iiiiiii)K", &is_sgd, &PyList_Type, &params, &PyDict_Type, &state, &PyDict_Type,
+    if (!PyArg_ParseTuple(args, "iO!O!O!O!O!O!p(iiiiiii)KO!", &is_sgd, &PyList_Type, &params, &PyDict_Type, &state, &PyDict_Type,
                           &override_, &PyDict_Type, &spare_stats, &PyDict_Type, &spare_scales, &PyDict_Type, &nd_scratch, &serve,
-                          &w.s.fused, &w.s.m_group128, &w.s.v_group128, &w.s.v_rank1, &w.s.m_wide, &w.s.bits_rank1, &m_group, &workspace))
+                          &w.s.fused, &w.s.m_group128, &w.s.v_group128, &w.s.v_rank1, &w.s.m_wide, &w.s.bits_rank1, &m_group, &workspace,
+                          &PyDict_Type, &in_place))
         return nullptr;
     w.s.m_group = m_group;
     w.workspace_bytes = reinterpret_cast<int64_t (*)(int64_t, int64_t)>((uintptr_t)workspace);
@@ -1066,6 +1066,7 @@ PyObject *collect(PyObject *, PyObject *args)
         w.spare_stats = spare_stats;
         w.spare_scales = spare_scales;
         w.nd_scratch = nd_scratch;
+        w.in_place = in_place;
         for (Py_ssize_t i = 0; i < PyList_GET_SIZE(params); ++i) {
             PyObject *po = PyList_GET_ITEM(params, i);
             bool served = false;
@@ -1125,7 +1126,6 @@ PyMODINIT_FUNC PyInit__walk()
     LPMM_NAME(work);
     LPMM_NAME(scale_of);
     LPMM_NAME(row);
-    LPMM_NAME(wraps);
     LPMM_NAME(dtype);
     LPMM_NAME(momentum_buffer);
     LPMM_NAME(momentum_buffer_qstate);

@@ -261,7 +261,7 @@ class AdamW(LowBitOptimizer):
             True,
             (0 if not fused else 1 if routes.fused4 else 2, routes.m_group128, routes.v_group128, routes.v_rank1,
              routes.m_group_wide, routes.bits_rank1, routes.m_group),
-            _native.factored_workspace())
+            _native.factored_workspace(), self._in_place)
 
     def _launch_walk(self, group, plan, routes):
         """The launches of the walk's records: those that _step_fused and _step_single make."""
@@ -1211,6 +1211,15 @@ class AdamW(LowBitOptimizer):
             scratch = self._nd_scratch[p] = {
                 "work": torch.empty((3, _nd_pitch(cols)), dtype=torch.float32, device=p.device), "scale_of": None, "row": 0}
         return scratch
+
+    @property
+    def _in_place(self):
+        # per matrix and tensor of more than two dimensions whose rows fold (csrc/walk.cpp): the second moment's overhead of the
+        # state that the walk has taken once, and takes in place from then on; a fresh or loaded state has another
+        d = self.__dict__.get("_in_place_by_param")
+        if d is None:
+            d = self.__dict__["_in_place_by_param"] = {}
+        return d
 
     @property
     def _spare_stats(self):

@@ -71,7 +71,7 @@ class SGD(LowBitOptimizer):
             plain = {}  # device -> records of the kernel on float buffers
             # tensors whose buffers exist; the loop below has the others, and every error
             plan = _native.walk().collect(1, group["params"], self.state, self.override_q_enable, {}, {}, {}, momentum != 0,
-                                          (0, one_pass_config, False, False, False, False, 128), 0)
+                                          (0, one_pass_config, False, False, False, False, 128), 0, {})
             for p in plan.rest:
                 if p.grad is None:
                     continue

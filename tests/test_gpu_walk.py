@@ -576,3 +576,37 @@ def test_few_rows_of_many_columns(shape, in_place, config, monkeypatch):
     assert torch.equal(sides[0][0], sides[1][0])
     a, b = (_state(opt, p) for p, opt in sides)
     assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
+
+
+def test_a_parameter_that_becomes_another_tensor():
+    """A matrix of rows of several tensor rows, then a tensor of more than two dimensions, then a matrix again, with a fresh state each
+    time; and a state from a file: its first step leaves new arrays, as any state's does."""
+    import lpmm
+
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", "default.yml")
+    p = torch.nn.Parameter(torch.randn(40, 132, device="cuda", generator=gen))
+    opt = lpmm.optim.AdamW([p], lr=1e-2, eps=1e-3, qconfig=path)
+
+    def steps(optimizer, q, count):
+        out = []
+        for _ in range(count):
+            gen.manual_seed(8)
+            before = optimizer.state[q].get("exp_avg_sq") if q in optimizer.state else None
+            q.grad = torch.randn(q.shape, device="cuda", generator=gen)
+            optimizer.step()
+            out.append(optimizer.state[q]["exp_avg_sq"] is before)
+        return out
+
+    assert steps(opt, p, 4) == [False, False, True, True]
+    for shape in [(66, 33, 2, 2), (40, 132), (33, 44, 3)]:
+        p.grad = None
+        p.data = torch.randn(shape, device="cuda", generator=gen)
+        del opt.state[p]
+        q = torch.nn.Parameter(p.detach().clone())
+        other = lpmm.optim.AdamW([q], lr=1e-2, eps=1e-3, qconfig=path)
+        assert steps(opt, p, 4) == steps(other, q, 4) == [False, False, True, True]
+        assert torch.equal(p, q)
+        opt.load_state_dict(copy.deepcopy(opt.state_dict()))
+        # of more than two dimensions the loops take the first one
+        assert steps(opt, p, 4) == [False, len(shape) == 2, True, True]
