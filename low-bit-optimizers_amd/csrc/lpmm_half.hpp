@@ -182,15 +182,26 @@ __device__ __forceinline__ float half_quotient(float x, h16 dh)
     return ZERO && d == 0.0f ? q : c;
 }
 
-// The parameter of two elements from their updated moments.  The hardware's half root is the correctly rounded one for every
-// half from 0 to infinity on gfx950 (all of them are compared by the tests).  IEEE: divisions as the
+// The correctly rounded root of a half from 0 to infinity: on gfx950 the hardware's half root, for every one of them (all are compared
+// by the tests).  Elsewhere (ARCH of the Makefile) the float root rounded to half, which may be 1 ulp off: the root of a half lies at
+// least 0.5 ulp of a float away from a tie.
+__device__ __forceinline__ h16 half_root(h16 x)
+{
+#if defined(__gfx950__)
+    return (h16)__builtin_amdgcn_sqrth(x);
+#else
+    return (h16)__builtin_amdgcn_sqrtf((float)x);
+#endif
+}
+
+// The parameter of two elements from their updated moments.  IEEE: divisions as the
 // compiler writes them, for kernels that arithmetic does not bound: infinite second moments (with beta2 = 0.999
 // gradients above 8090, where (1 - beta2) g^2 passes 65504) divide as in the chain too.
 template <bool ZERO, bool IEEE>
 __device__ __forceinline__ v2h half_param(v2h p, v2h m, v2h v, const NfHyper &h, const MixConst &c)
 {
     const v2h pi = round2(mix_mul(p.x, h.decay, c), mix_mul(p.y, h.decay, c));
-    v2h d = {(h16)__builtin_amdgcn_sqrth(v.x), (h16)__builtin_amdgcn_sqrth(v.y)};
+    v2h d = {half_root(v.x), half_root(v.y)};
     float q[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {  // div_by_rc(d, bc2_sqrt, rbc2_sqrt)
