@@ -147,16 +147,31 @@ void read(PyObject *dict, PyObject *const (&names)[COUNT], PyObject *(&values)[C
                 values[i] = PyDict_GetItemWithError(dict, names[i]);
 }
 
-// A tensor's hash, its id: torch computes it in Python, 0.1 us a time.  (Were it another one, nothing would be found with this and the
-// tensor would go to the loops in Python.)
+// A tensor's hash, its id: torch computes it in Python, 0.1 us a time.  (Were it another one, no state would be found with this and
+// every tensor would go to the loops in Python.)
 Py_hash_t hash_of(PyObject *tensor)
 {
     const Py_hash_t id = (Py_hash_t)(uintptr_t)tensor;
     return id == -1 ? -2 : id;
 }
+// The dictionary calls that take a hash are private to the interpreter from Python 3.13 on, which gets the public ones.
 PyObject *of_parameter(PyObject *dict, PyObject *p)  // dict[p]; borrowed, or null
 {
-    return dict != nullptr && PyDict_Check(dict) ? _PyDict_GetItem_KnownHash(dict, p, hash_of(p)) : nullptr;
+    if (dict == nullptr || !PyDict_Check(dict))
+        return nullptr;
+#if PY_VERSION_HEX < 0x030d0000
+    return _PyDict_GetItem_KnownHash(dict, p, hash_of(p));
+#else
+    return PyDict_GetItemWithError(dict, p);
+#endif
+}
+int set_item(const Swap &swap)  // dict[key] = value
+{
+#if PY_VERSION_HEX < 0x030d0000
+    if (swap.hash != -1)
+        return _PyDict_SetItem_KnownHash(swap.dict, swap.key, swap.value, swap.hash);
+#endif
+    return PyDict_SetItem(swap.dict, swap.key, swap.value);
 }
 
 // the settings of a state, state[name + "_qstate"]
@@ -1011,8 +1026,7 @@ PyObject *plan_commit(PyObject *self, PyObject *args)
             if (b->swaps[j].value == nullptr) {
                 PyErr_SetString(PyExc_RuntimeError, "records that were not prepared");
                 return nullptr;
-            } else if (b->swaps[j].hash != -1 ? _PyDict_SetItem_KnownHash(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value, b->swaps[j].hash) != 0
-                                              : PyDict_SetItem(b->swaps[j].dict, b->swaps[j].key, b->swaps[j].value) != 0) {
+            } else if (set_item(b->swaps[j]) != 0) {
                 return nullptr;
             }
     }

@@ -53,3 +53,9 @@ def test_steps_without_the_module(monkeypatch):
             torchs.step()
     assert len(warned) == 1 and torch.allclose(p, q)
     assert lpmm.optim.AdamW([torch.nn.Parameter(torch.zeros(3))]).step() is None
+
+
+def test_a_tensors_hash_is_its_address():
+    """The walk looks states up with it (hash_of), and dictionaries keep what it is given."""
+    for t in (torch.zeros(3), torch.nn.Parameter(torch.zeros(3)), torch.nn.Parameter(torch.zeros(0))):
+        assert hash(t) == id(t)
