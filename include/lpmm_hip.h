@@ -208,7 +208,7 @@ int lpmm_rank1_row_scale_nd(const float *const *stats, int ndim, const int64_t *
 /* A whole rank-1 quantisation of a contiguous tensor of 2..LPMM_RANK1_ND_MAX dimensions in one call: its statistics, of more than two
  * dimensions the scale of a row (both as above), and the codes (lpmm_quant_rank1, for bits other than 4
  * lpmm_quant_rank1_bits_table with `table`); and the way back from codes and statistics.  work: NULL for two dimensions, otherwise
- * device memory for numel / shape[ndim-1] floats. */
+ * device memory for numel / shape[ndim-1] floats.  What these calls would refuse is refused with nothing written. */
 int lpmm_quant_rank1_nd(const float *x, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap, int bits,
                         const void *table, uint8_t *codes, void *stream);
 int lpmm_dequant_rank1_nd(const uint8_t *codes, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap,

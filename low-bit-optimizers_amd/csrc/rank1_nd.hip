@@ -516,6 +516,31 @@ static bool rank1_view(int ndim, const int64_t *shape, int64_t *rows, int64_t *c
     return true;
 }
 
+// What the calls that a whole quantisation consists of would refuse, before the first of them launches anything.
+static int check_rank1_nd(const float *values, int ndim, float *const *stats, const float *work, const float *qmap, int bits,
+                          const void *table, const uint8_t *codes, uintptr_t codes4_align)
+{
+    if (bits < 1 || bits > 8)
+        return LPMM_ERR_SIZE;
+    for (int i = 0; i < ndim; ++i) {
+        LPMM_REQUIRE_PTR(stats[i]);
+        LPMM_REQUIRE_ALIGN(stats[i], 4);
+    }
+    if (ndim > 2) {
+        LPMM_REQUIRE_PTR(work);
+        LPMM_REQUIRE_ALIGN(work, 4);
+    }
+    LPMM_REQUIRE_PTR(values);
+    LPMM_REQUIRE_PTR(qmap);
+    LPMM_REQUIRE_PTR(codes);
+    LPMM_REQUIRE_ALIGN(values, 4);
+    LPMM_REQUIRE_ALIGN(qmap, 4);
+    LPMM_REQUIRE_ALIGN(codes, bits == 4 ? codes4_align : 8);
+    if (bits != 4 && table != nullptr)
+        LPMM_REQUIRE_ALIGN(table, 16);
+    return LPMM_OK;
+}
+
 extern "C" int lpmm_quant_rank1_nd(const float *x, int ndim, const int64_t *shape, float *const *stats, float *work, const float *qmap,
                                    int bits, const void *table, uint8_t *codes, void *stream)
 {
@@ -526,12 +551,14 @@ extern "C" int lpmm_quant_rank1_nd(const float *x, int ndim, const int64_t *shap
     int64_t rows, cols;
     if (!rank1_view(ndim, shape, &rows, &cols))
         return LPMM_ERR_SIZE;
+    const int bad = check_rank1_nd(x, ndim, stats, work, qmap, bits, table, codes, 4);
+    if (bad != LPMM_OK)
+        return bad;
     const float *rowmax = stats[0], *colmax = stats[ndim - 1];
     int st;
     if (ndim == 2) {
         st = lpmm_rank1_stats(x, rows, cols, stats[0], stats[1], stream);
     } else {
-        LPMM_REQUIRE_PTR(work);
         // long last dimension: the 2-D kernel plus a fold of its row maxima, whose place the scales take
         st = lpmm_rank1_stats_nd(x, ndim, shape, stats, cols >= 32 ? work : nullptr, stream);
         if (st == LPMM_OK)
@@ -554,6 +581,9 @@ extern "C" int lpmm_dequant_rank1_nd(const uint8_t *codes, int ndim, const int64
     int64_t rows, cols;
     if (!rank1_view(ndim, shape, &rows, &cols))
         return LPMM_ERR_SIZE;
+    const int bad = check_rank1_nd(out, ndim, stats, work, qmap, bits, nullptr, codes, 1);
+    if (bad != LPMM_OK)
+        return bad;
     const float *rowmax = stats[0], *colmax = stats[ndim - 1];
     if (ndim > 2) {
         const int st = lpmm_rank1_row_scale_nd(stats, ndim, shape, work, stream);

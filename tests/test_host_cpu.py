@@ -520,3 +520,42 @@ def test_spare_statistics_of_a_parameter_that_changed_its_shape(first, second, h
         if len(shape) > 2:
             cols = p.numel() // shape[0]
             assert opt._nd_scratch_of(p, cols)["work"].shape == (3, _nd_pitch(cols)) and opt._nd_scratch_of(p, cols) is opt._nd_scratch[p]
+
+
+@pytest.mark.parametrize("shape", [(12, 40), (3, 4, 40), (3, 5, 2, 7)])
+@pytest.mark.parametrize("bits", [4, 2, 8])
+@pytest.mark.parametrize("back", [False, True])
+def test_errors_of_whole_rank1_quantisations(shape, bits, back):
+    """lpmm_quant_rank1_nd and lpmm_dequant_rank1_nd are several calls to the device: what the last would refuse is refused before the
+    first (whose status is another on a machine without a GPU)."""
+    from lpmm import _native
+
+    lib, memory = _native.lib(), np.zeros(4096, np.uint8)  # never read: only the addresses count
+    base = (memory.ctypes.data + 63) // 64 * 64
+    stats = [base + 64 * i for i in range(len(shape))]
+    fine = dict(values=base + 512, shape=shape, dims=len(shape), stats=stats, work=base + 1024 if len(shape) > 2 else None, qmap=base + 1536, bits=bits,
+                table=None, codes=base + 2048)
+
+    def call(**kw):
+        a = {**fine, **kw}
+        sizes = None if a["shape"] is None else (ctypes.c_int64 * len(a["shape"]))(*a["shape"])
+        pointers = None if a["stats"] is None else (ctypes.c_void_p * len(a["stats"]))(*a["stats"])
+        if back:
+            return lib.lpmm_dequant_rank1_nd(a["codes"], a["dims"], sizes, pointers, a["work"], a["qmap"], a["bits"], a["values"], None)
+        return lib.lpmm_quant_rank1_nd(a["values"], a["dims"], sizes, pointers, a["work"], a["qmap"], a["bits"], a["table"], a["codes"], None)
+
+    assert call(dims=1) == 5 and call(dims=9) == 5
+    for name in ("values", "shape", "stats", "qmap", "codes") + (("work",) if len(shape) > 2 else ()):
+        assert call(**{name: None}) == 1, name
+    for name in ("values", "qmap") + (("work",) if len(shape) > 2 else ()):
+        assert call(**{name: fine[name] + 2}) == 2, name
+    for i in range(len(shape)):
+        assert call(stats=stats[:i] + [None] + stats[i + 1:]) == 1 and call(stats=stats[:i] + [stats[i] + 1] + stats[i + 1:]) == 2
+        assert call(shape=shape[:i] + (0,) + shape[i + 1:]) == 3 and call(shape=shape[:i] + (-4,) + shape[i + 1:]) == 3
+    assert call(shape=(1 << 40,) * len(shape)) == 3
+    assert call(bits=0) == 3 and call(bits=9) == 3
+    if bits != 4:
+        assert call(codes=fine["codes"] + 4) == 2
+        assert back or call(table=base + 8) == 2
+    elif not back:
+        assert call(codes=fine["codes"] + 2) == 2
