@@ -522,6 +522,180 @@ def test_spare_statistics_of_a_parameter_that_changed_its_shape(first, second, h
             assert opt._nd_scratch_of(p, cols)["work"].shape == (3, _nd_pitch(cols)) and opt._nd_scratch_of(p, cols) is opt._nd_scratch[p]
 
 
+HYPER = (0.9, 0.999, 1e-3, 0.01, 1e-8)
+
+
+def _records(dtype, count, **values):
+    """Records whose pointers are distinct addresses of a buffer that nothing reads; the buffer has to be kept."""
+    memory = np.zeros(64 * 32 * count + 64, np.uint8)
+    base = (memory.ctypes.data + 63) // 64 * 64
+    records = np.zeros(count, dtype)
+    for i in range(count):
+        for j, name in enumerate(n for n in dtype.names if dtype[n] == np.dtype("<u8")):
+            records[i][name] = base + 64 * (32 * i + j)
+        for name, value in values.items():
+            records[i][name] = value
+    return records, memory, base
+
+
+def _spoil(record, field, change):
+    record[field] = {"null": 0, "shift": record[field] + 2, "shift4": record[field] + 4}.get(change, change) if not (
+        isinstance(change, str) and change in record.dtype.names) else record[change]
+
+
+# kind of the two-pass steps (LPMM_STEP_* of the header): its records, columns that it takes, columns that it refuses
+STEPS = {0: ("NONFUSED_RANK1_TENSOR", (128, 64, 132, 1600), (130, 60, 12)), 1: ("NONFUSED_RANK1_TENSOR", (128, 132), (130, 60)),
+         2: ("NONFUSED_RANK1_TENSOR", (128, 132), (130, 60)), 3: ("RANK1_V4BIT_TENSOR", (128, 132), (130, 60)),
+         4: ("RANK1_MGROUP_TENSOR", (128, 8, 200), (12, 130)), 5: ("RANK1_MGROUP_TENSOR", (128, 132), (130, 8, 60)),
+         8: ("RANK1_ANY_TENSOR", (128, 61), ()), 9: ("RANK1_ANY_TENSOR", (128, 61), ()), 10: ("RANK1_ANY_TENSOR", (128, 61), ())}
+
+
+@pytest.mark.parametrize("kind", list(STEPS))
+def test_errors_of_the_two_pass_steps_beside_float_states(kind):
+    """lpmm_nonfused_rank1_fp32_step_multi: every record of either array is looked at before the first launch (which has a status of its
+    own on a machine without a GPU)."""
+    from lpmm import _native
+
+    name, taken, refused = STEPS[kind]
+    lib, dtype = _native.lib(), getattr(_native, name)
+    bits = 8 if kind in (1, 10) else 4
+    plain, keep_plain, base = _records(_native.ADAMW_FP32_TENSOR, 3, n=100, step=1.0)
+
+    def call(records, count=None, plain=plain, plain_count=3, group=128, bits=(bits, bits), tables=(None, None), maps=(base, base), folds=None):
+        folds = None if folds is None else folds.ctypes.data
+        return lib.lpmm_nonfused_rank1_fp32_step_multi(
+            kind, None if records is None else records.ctypes.data, folds, len(records) if count is None else count,
+            None if plain is None else plain.ctypes.data, plain_count, group, maps[0], bits[0], tables[0], maps[1], bits[1], tables[1], *HYPER, None)
+
+    def fresh(cols=taken[0]):
+        records, *keep = _records(dtype, 40, rows=70, cols=cols, step=1.0)
+        return records, (np.zeros(40, _native.RANK1_SMALL_VECTOR) if kind == 2 else None), keep  # ndim 0: matrices
+
+    records, folds, keep = fresh()
+    assert call(None, 3, folds=folds) == 1 and call(records, -1, folds=folds) == 3 and call(records, plain_count=-1, folds=folds) == 3
+    assert call(records, plain=None, folds=folds) == 1
+    assert call(records, bits=(9 if bits == 8 else 5, bits), folds=folds) == 5 and call(records, bits=(bits, 3), folds=folds) == 5
+    assert call(records, tables=(base + 8, None), folds=folds) == 2 and call(records, tables=(None, base + 4), folds=folds) == 2
+    assert call(records, group=192, folds=folds) == 3 and call(records, group=8192, folds=folds) == 3
+    if kind not in (4, 5, 8):  # those take wide groups of the first moment
+        assert call(records, group=256, folds=folds) == 3
+    assert call(records, maps=(base, None), folds=folds) == 1 and call(records, maps=(base, base + 2), folds=folds) == 2
+    if kind == 2:
+        assert call(records) == 1  # without the vectors
+    for field, change, status in (("p", "null", 1), ("n", -1, 3), ("g", "shift", 2), ("v", "null", 1)):
+        bad = plain.copy()
+        _spoil(bad[2], field, change)
+        assert call(records, plain=bad, folds=folds) == status, field
+    whole = kind < 8
+    for field, change, status in (("p", "null", 1), ("g", "shift4" if whole else "shift", 2), ("v_codes", "shift", 2), ("v_rowmax", "null", 1),
+                                  ("v_rowmax_next", "v_rowmax", 5), ("v_colmax_next", "v_colmax", 5), ("rows", -1, 3), ("cols", -1, 3),
+                                  ("v_colmax", "shift4" if whole else "shift", 2), ("v_colmax_next", "shift4" if whole else "shift", 2)):
+        for cols in taken:
+            records, folds, keep = fresh(cols)
+            _spoil(records[39], field, change)  # beyond what one launch takes
+            assert call(records, folds=folds) == status, (field, cols)
+    for cols in refused:
+        records, folds, keep = fresh()
+        records[39]["cols"] = cols
+        assert call(records, folds=folds) == 3, cols
+
+
+def test_errors_of_kinds_that_there_are_not():
+    from lpmm import _native
+
+    records, keep, base = _records(_native.RANK1_ANY_TENSOR, 1, rows=70, cols=61, step=1.0)
+    for kind in (-1, 6, 7, 11, 12):  # 11: float16 has no such call
+        assert _native.lib().lpmm_nonfused_rank1_fp32_step_multi(kind, records.ctypes.data, None, 1, None, 0, 128, base, 4, None, base, 4, None,
+                                                                 *HYPER, None) == 5
+
+
+def test_errors_of_the_steps_on_tensors_of_more_than_two_dimensions():
+    """lpmm_nonfused_adamw4bit_rank1_nd_step_multi: a vector between the passes that is not its tensor's."""
+    from lpmm import _native
+
+    lib = _native.lib()
+    records, keep, base = _records(_native.NONFUSED_RANK1_TENSOR, 40, rows=70, cols=9 * 128, step=1.0)
+    folds, keep_folds, _ = _records(_native.RANK1_SMALL_VECTOR, 40, ndim=2)
+    stats = np.zeros(4096, np.float32)
+    scales = (stats.ctypes.data + 63) // 64 * 64
+    folds["shape"][:, :2], folds["stats"][:, :2], folds["x"], folds["scale"] = (128, 9), scales + 4096, records["v_colmax_next"], scales
+
+    def call(records=records, folds=folds, count=40):
+        return lib.lpmm_nonfused_adamw4bit_rank1_nd_step_multi(None if records is None else records.ctypes.data,
+                                                               None if folds is None else folds.ctypes.data, count, base, base, *HYPER, None)
+
+    assert call(count=0) == 0 and call(None, None, 0) == 0 and call(count=-1) == 3 and call(None) == 1 and call(folds=None) == 1
+    for field, value, status in (("x", scales + 1024, 5), ("x", 0, 1), ("scale", scales + 4, 2), ("scale", 0, 1), ("ndim", 8, 5), ("ndim", -1, 5)):
+        bad = folds.copy()
+        bad[39][field] = value
+        assert call(folds=bad) == status, field
+    for shape, status in (((128, 8), 3), ((0, 9), 3), ((8192, 9), 3)):
+        bad = folds.copy()
+        bad["shape"][39, :2] = shape
+        assert call(folds=bad) == status, shape
+    bad = folds.copy()
+    bad["scale"][39] = bad["x"][39]  # in the place of what the second pass still needs
+    assert call(folds=bad) == 5
+    bad = folds.copy()
+    bad["scale"][39] = records["v_colmax"][39]
+    assert call(folds=bad) == 5
+    bad = folds.copy()
+    bad["stats"][39, 1] = 0
+    assert call(folds=bad) == 1
+    bad = records.copy()
+    bad["v_codes"][39] = 0
+    assert call(bad) == 1
+
+
+@pytest.mark.parametrize("general", [0, 1])
+@pytest.mark.parametrize("plain_fused", [0, 1])
+def test_errors_of_the_factored_steps_beside_float_states(general, plain_fused):
+    from lpmm import _native
+
+    lib = _native.lib()
+    plain, keep_plain, base = _records(_native.ADAMW_FP32_TENSOR, 3, n=100, step=1.0)
+    records, keep, _ = _records(_native.FACTORED_TENSOR, 60, rows=70, cols=128, step=1.0)
+
+    def call(records=records, count=60, plain=plain, plain_count=3, qmap=base):
+        return lib.lpmm_factored_fp32_step_multi(None if records is None else records.ctypes.data, count, general,
+                                                 None if plain is None else plain.ctypes.data, plain_count, plain_fused, qmap, *HYPER, None)
+
+    assert call(count=-1) == 3 and call(plain_count=-1) == 3 and call(None) == 1 and call(plain=None) == 1 and call(qmap=None) == 1
+    assert call(None, 0, None, 0) == 0  # nothing to do
+    for field, change, status in (("m", "null", 1), ("n", -1, 3), ("g", "shift", 2)):
+        bad = plain.copy()
+        _spoil(bad[2], field, change)
+        assert call(plain=bad) == status and call(None, 0, bad) == status, field
+    for field, change, status in (("p", "null", 1), ("row", "shift", 2), ("workspace", "shift4", 2), ("rows", 0, 3), ("cols", -1, 3),
+                                  ("col", "shift" if general else "shift4", 2)) + (() if general else (("cols", 136, 3), ("m_max1", "null", 1))):
+        bad = records.copy()
+        _spoil(bad[59], field, change)
+        assert call(bad) == status, field
+
+
+def test_errors_of_the_sgd_steps_beside_float_buffers():
+    from lpmm import _native
+
+    lib = _native.lib()
+    plain, keep_plain, base = _records(_native.SGD_FP32_TENSOR, 70, n=100)
+    records, keep, _ = _records(_native.SGD4BIT_TENSOR, 70, n=5000)
+
+    def call(records=records, count=70, plain=plain, plain_count=70, qmap=base):
+        return lib.lpmm_sgd4bit_fp32_step_multi(None if records is None else records.ctypes.data, count, None if plain is None else plain.ctypes.data,
+                                                plain_count, qmap, 0.9, 0.0, 0.1, 0.0, 0, 0, None)
+
+    assert call(count=-1) == 3 and call(plain_count=-1) == 3 and call(None) == 1 and call(plain=None) == 1 and call(qmap=None) == 1
+    assert call(None, 0, None, 0, None) == 0  # nothing to do
+    for field, change, status in (("buf", "null", 1), ("n", -1, 3), ("g", "shift", 2)):
+        bad = plain.copy()
+        _spoil(bad[69], field, change)
+        assert call(plain=bad) == status and call(None, 0, bad) == status, field
+    for field, change, status in (("m_codes", "null", 1), ("n", -1, 3), ("m_max1", "shift", 2)):
+        bad = records.copy()
+        _spoil(bad[69], field, change)
+        assert call(bad) == status and call(bad, plain=None, plain_count=0) == status, field
+
+
 @pytest.mark.parametrize("shape", [(12, 40), (3, 4, 40), (3, 5, 2, 7)])
 @pytest.mark.parametrize("bits", [4, 2, 8])
 @pytest.mark.parametrize("back", [False, True])
