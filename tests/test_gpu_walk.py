@@ -540,6 +540,112 @@ def test_float_states_beside_the_clearing(config, shape, matrices, vectors, monk
         assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
 
 
+@pytest.mark.parametrize("config", ["default.yml", "2nd_moment_only_default.yml", "default_8b.yml", "default_5b.yml",
+                                    "1st_moment_group_256.yml", "1st_moment_group_1024.yml"])
+@pytest.mark.parametrize("shape", [(1, 5000), (5, 1004), (33, 132), (70, 64), (31, 192), (97, 136), (64, 140), (129, 160), (257, 200), (1000, 408),
+                                   (16, 576), (2047, 1600), (300, 3076), (33, 33, 2, 2), (88, 88, 3, 3), (45, 17, 8), (352, 132, 1, 1)])
+def test_rows_of_several_tensor_rows(shape, config, monkeypatch):
+    """Column counts of 4 to 64 modulo 128 on the kernels for whole column blocks (rank1_tiles.hpp: Fold), whole and partial last rows and
+    groups, against the kernels for any column count, which the loops take; rows of zeros (0 / 0 in scales and codes), a
+    not-a-number and an infinity among the gradients."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+
+    float_m, in_place, wide = config.startswith("2nd"), config == "default.yml", config.startswith("1st")
+    if not in_place and len(shape) > 2:
+        pytest.skip("such tensors go by the loops")
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    gen = torch.Generator(device="cuda").manual_seed(41)
+    start = [torch.randn(s, device="cuda", generator=gen) * 0.1 for s in (shape, (64, 256))]
+    sides = []
+    for _ in range(2):
+        params = [torch.nn.Parameter(s.clone()) for s in start]
+        sides.append((params, lpmm.optim.AdamW(params, lr=1e-2, eps=1e-3, qconfig=path)))
+    for step in range(5):
+        grads = [torch.randn(s.shape, device="cuda", generator=gen) * 0.1 for s in start]
+        rows = grads[0].view(shape[0], -1)
+        rows.mul_(torch.randn(shape[0], 1, device="cuda", generator=gen).exp())
+        rows[shape[0] // 2:: 5] = 0
+        if step < 2:
+            rows[:, ::7] = 0
+        if step == 3:
+            rows[-1, -1], rows[0, 1] = float("inf"), float("nan")
+        for serve, (params, opt) in zip((True, False), sides):
+            for p, g in zip(params, grads):
+                p.grad = g
+            with monkeypatch.context() as patch:
+                native = _Native(_native, serve)
+                patch.setattr(adamw, "_native", native)
+                opt.step()
+                assert step < 2 or native.rest == (0 if serve else len(params))
+        # the second step replaces scales and codes as the loops' kernels do, those after it write in place
+        state = sides[0][1].state[sides[0][0][0]]
+        held = state["exp_avg_sq"] if float_m else state["exp_avg_qstate"]["overhead"]["max1"]
+        cols = start[0].numel() // shape[0]
+        if wide:  # their scales trade places on every step
+            held = state["exp_avg"]
+        if start[0].numel() > 4096 and not (wide and cols % 8 == 0) and (not in_place or cols % 128 != 64 or shape[0] % 2):
+            assert step == 0 or (held is last) == (step >= 2)
+        last = held
+        if step in (2, 4):
+            for p, q in zip(*(params for params, _ in sides)):
+                assert torch.equal(p.nan_to_num(), q.nan_to_num())
+                a, b = _state(sides[0][1], p), _state(sides[1][1], q)
+                assert a.keys() == b.keys()
+                for k in a:
+                    assert torch.equal(a[k].nan_to_num(), b[k].nan_to_num()) if a[k].is_floating_point() else torch.equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("config,shape", [("default.yml", (33, 132)), ("2nd_moment_only_default.yml", (33, 132)),
+                                          ("2nd_moment_only_default.yml", (65, 200)), ("default_8b.yml", (33, 132)),
+                                          ("default_8b.yml", (65, 200)), ("1st_moment_group_256.yml", (33, 132))])
+@pytest.mark.parametrize("odd", ["state", "spare"])
+def test_column_statistics_at_any_float(config, shape, odd, monkeypatch):
+    """Column statistics behind an odd number of row statistics in one buffer, as a caller may hold them: such a matrix stays with the
+    kernels for any column count on every step, the others' own state or their spare one."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    start = torch.randn(shape, device="cuda", generator=gen) * 0.1
+    sides = []
+    for _ in range(2):
+        p = torch.nn.Parameter(start.clone())
+        sides.append((p, lpmm.optim.AdamW([p], lr=1e-2, eps=1e-3, qconfig=path)))
+
+    def moved(stats):
+        rows, cols = shape
+        flat = torch.empty(rows + cols, device="cuda")
+        assert flat[rows:].data_ptr() % 16 != 0
+        views = [flat[:rows].view(rows, 1), flat[rows:].view(1, cols)]
+        for view, s in zip(views, stats):
+            view.copy_(s)
+        return views
+
+    for step in range(6):
+        grad = torch.randn(shape, device="cuda", generator=gen) * 0.1
+        for serve, (p, opt) in zip((True, False), sides):
+            if step == 1 and serve:
+                oh = opt.state[p]["exp_avg_sq_qstate"]["overhead"]
+                if odd == "state":
+                    oh["max_dims"] = moved(oh["max_dims"])
+                else:
+                    opt._spare_stats[p] = moved(opt._spare_stats[p])
+            p.grad = grad
+            with monkeypatch.context() as patch:
+                native = _Native(_native, serve)
+                patch.setattr(adamw, "_native", native)
+                opt.step()
+                assert step < 2 or native.rest == (0 if serve else 1)
+        assert torch.equal(sides[0][0], sides[1][0])
+        a, b = (_state(opt, p) for p, opt in sides)
+        assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a)
+
+
 @pytest.mark.parametrize("config", ["default.yml", "2nd_moment_only_default.yml", "default_8b.yml", "1st_moment_group_256.yml"])
 @pytest.mark.parametrize("shape,in_place", [((1, 100004), False), ((31, 20004), False), ((127, 20008), False), ((511, 4100), False),
                                             ((512, 4100), True), ((31, 4092), True), ((3, 8184), True)])
