@@ -5,6 +5,8 @@
 //   dequant BITS ROWS COLS              the way back
 //   rank1 MODE ROWS COLS [ROWS COLS]... one step on these matrices; MODE: codes4, float_m (fp32 first moment), codes8 or
 //                                       half (float16)
+//   beside MODE ROWS COLS [ROWS COLS]...  the same but for half, by the entry point for steps beside tensors with fp32 states (of which
+//                                       there are none); groups as well (first moment in groups of 256 values)
 //   any ROWS COLS [ROWS COLS]...        one step with 4-bit codes by the kernels for any column count
 // and one line of output its status and the grids, "x,y" each.
 // Build: g++ -O1 -rdynamic -D__HIP_PLATFORM_AMD__ -I<rocm>/include -I<include> launches.cpp -llpmm_hip
@@ -53,11 +55,12 @@ static char *made_up()
     return reinterpret_cast<char *>(at += uintptr_t(1) << 30);
 }
 
-static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, int64_t>> &shapes)
+static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, int64_t>> &shapes, bool beside = false)
 {
     std::vector<lpmm_nonfused_rank1_tensor> coded;
     std::vector<lpmm_rank1_v4bit_tensor> plain;
     std::vector<lpmm_nonfused_rank1_f16_tensor> halfs;
+    std::vector<lpmm_rank1_mgroup_tensor> groups;
     for (const auto &[rows, cols] : shapes) {
         lpmm_nonfused_rank1_tensor t;
         lpmm_rank1_v4bit_tensor f;
@@ -78,11 +81,20 @@ static int rank1(const std::string &mode, const std::vector<std::pair<int64_t, i
         f.step = t.step = 1.0f;
         coded.push_back(t);
         plain.push_back(f);
+        groups.push_back({t.p, t.g, t.m_codes, t.m_max1, (float *)made_up(), t.v_codes, t.v_rowmax, t.v_colmax, t.v_rowmax_next,
+                          t.v_colmax_next, rows, cols, 1.0f, 0.0f});
         halfs.push_back({t.p, t.g, t.m_codes, t.m_max1, t.v_codes, t.v_rowmax, t.v_colmax, t.v_rowmax_next, t.v_colmax_next,
                          (float *)made_up(), rows, cols, 1.0f, 0.0f});
     }
     const float *map = (const float *)made_up();
     const int64_t n = (int64_t)shapes.size();
+    if (beside) {
+        const int kind = mode == "codes4" ? LPMM_STEP_MATRIX : mode == "codes8" ? LPMM_STEP_BITS : mode == "float_m" ? LPMM_STEP_FLOAT_M : LPMM_STEP_GROUPS_WRAP;
+        const void *records = mode == "float_m" ? (const void *)plain.data() : mode == "groups" ? (const void *)groups.data() : coded.data();
+        const int bits = mode == "codes8" ? 8 : 4;
+        return lpmm_nonfused_rank1_fp32_step_multi(kind, records, nullptr, n, nullptr, 0, mode == "groups" ? 256 : 128, map, bits, nullptr, map,
+                                                   bits, nullptr, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
+    }
     if (mode == "float_m")
         return lpmm_nonfused_adamw_v4bit_rank1_step_multi(plain.data(), n, map, 0.9, 0.999, 1e-3, 0.01, 1e-8, nullptr);
     if (mode == "half")
@@ -150,6 +162,7 @@ int main()
         const int status = call == "stats"   ? lpmm_rank1_stats((const float *)made_up(), r, c, (float *)made_up(), (float *)made_up(),
                                                                 nullptr)
                            : call == "rank1" ? rank1(mode, shapes)
+                           : call == "beside" ? rank1(mode, shapes, true)
                            : call == "any"   ? any_columns(shapes)
                                              : quantiser(call == "dequant", std::stoi(mode), r, c);
         printf("%d", status);

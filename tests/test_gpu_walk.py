@@ -716,3 +716,36 @@ def test_a_parameter_that_becomes_another_tensor():
         opt.load_state_dict(copy.deepcopy(opt.state_dict()))
         # of more than two dimensions the loops take the first one
         assert steps(opt, p, 4) == [False, len(shape) == 2, True, True]
+
+
+@pytest.mark.parametrize("config", ["default.yml", "2nd_moment_only_default.yml", "default_8b.yml", "1st_moment_group_256.yml"])
+def test_launches_that_end_between_kinds_of_matrices(config, monkeypatch):
+    """Whole column blocks, double rows and rows of several tensor rows in turn, beyond the 48M values from which on a launch ends where
+    tensors that wrap meet others: every one of them is stepped, once, as by the loops."""
+    import lpmm
+    import lpmm.optim.adamw as adamw
+    from lpmm import _native
+
+    path = os.path.join(os.path.dirname(lpmm.config.__file__), "configs", config)
+    whole, double, wraps = (4096, 4096), (4096, 4160), (4095, 4100)
+    shapes = [whole, whole, whole, wraps, whole, double, wraps, (33, 132), wraps, double, double, whole, (17, 256), whole, wraps]
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    sides = []
+    for _ in range(2):
+        gen.manual_seed(12)
+        params = [torch.nn.Parameter(torch.randn(s, device="cuda", generator=gen) * 0.1) for s in shapes]
+        sides.append((params, lpmm.optim.AdamW(params, lr=1e-2, eps=1e-3, qconfig=path)))
+    for step in range(4):
+        grads = [torch.randn(s, device="cuda", generator=gen) * 0.1 for s in shapes]
+        for serve, (params, opt) in zip((True, False), sides):
+            for p, g in zip(params, grads):
+                p.grad = g
+            with monkeypatch.context() as patch:
+                native = _Native(_native, serve)
+                patch.setattr(adamw, "_native", native)
+                opt.step()
+                assert step < 2 or native.rest == (0 if serve else len(params))
+    for i, (p, q) in enumerate(zip(*(params for params, _ in sides))):
+        assert torch.equal(p, q), i
+        a, b = _state(sides[0][1], p), _state(sides[1][1], q)
+        assert a.keys() == b.keys() and all(torch.equal(a[k], b[k]) for k in a), i

@@ -216,6 +216,19 @@ def test_second_pass_tiles_of_odd_columns(launches):
         assert status == 0 and blocks * tiles <= grids[2][0] < (blocks + 256 // tiles) * tiles, (values_of, grids)
 
 
+def test_where_launches_end_between_kinds_of_matrices(launches):
+    """A launch ends at 32 tensors (4-bit codes: 64 of at most 80M values in all), and from 48M values on before the first tensor that
+    wraps among others or the other way round; double rows count as others.  In calls: the clearing, then two passes a launch."""
+    whole, double, wraps = " 4096 4096", " 4096 4160", " 4096 4100"  # 17M values each
+    for mode in ("codes4", "float_m", "codes8", "groups"):
+        cases = {3 * whole + wraps: 2, 2 * whole + wraps + whole + wraps: 1, 3 * double + wraps: 2, 3 * whole + double: 1, 3 * wraps + double: 2,
+                 3 * wraps + whole + 2 * wraps: 2, 3 * whole + wraps + 2 * whole + double: 2, 3 * whole + 3 * wraps + whole: 3, wraps: 1,
+                 33 * " 512 512": 1 if mode == "codes4" else 2, 64 * " 512 516": 1 if mode == "codes4" else 2,
+                 65 * " 512 516": 2 if mode == "codes4" else 3}
+        for (shapes, count), (status, grids) in zip(cases.items(), launches(*(f"beside {mode}{shapes}" for shapes in cases))):
+            assert status == 0 and len(grids) == 1 + 2 * count, (mode, shapes, grids)
+
+
 def test_remainders_of_small_float16_launches(launches):
     """55 row blocks of 128 rows, 17 resident beside 15 column tiles: launches of few workgroups take four groups of 17, the last one's
     rows spread over all of its blocks; others take groups of equal size."""
