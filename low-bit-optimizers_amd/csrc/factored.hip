@@ -574,7 +574,8 @@ __global__ __launch_bounds__(kFThreads) void factored_finalize_multi_kernel(cons
 }
 
 // The same with tensors that have fp32 states, whose own launch this one saves (4 us on the device, 4 to 5 on the host): the first `tiles`
-// workgroups finish statistics.  Steps on three layers of an MLP of width 64 38 -> 32 us, of width 384 53 -> 46.
+// workgroups finish statistics.  Steps on three layers of an MLP of width 64 38 -> 32 us, of width 384 53 -> 46.  (Beside groups of 48, whose
+// arguments and theirs would exceed 8 KB, they keep a launch of their own.)
 template <bool ONE_ROW_GROUP, class Arith>
 __global__ __launch_bounds__(kFThreads) void factored_finalize_plain_kernel(const MultiFa<kFaMax> args, const MultiF plain, uint32_t tiles)
 {

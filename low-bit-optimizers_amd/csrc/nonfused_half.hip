@@ -23,7 +23,7 @@
 // are decoded by one read and the normalised halfs encoded as halfs, maxima over a lane's columns stay in registers through its
 // passes instead of going to LDS one by one, and addresses advance by one addition each.  Kernels of the usual constants (USUAL)
 // have no branch in the chain.  VALU instructions an element, before and after the decoding, encoding and roots of halfs: update 48 -> 37,
-// second pass 19 -> 15.  Four decoder layers of width 4096 (8.1e8 values), a step: 1737 -> 1570 us (the memory system's: 1360);
+// second pass 19 -> 14.  Four decoder layers of width 4096 (8.1e8 values), a step: 1737 -> 1570 us (the memory system's: 1360);
 // the one pass on a LLaMA-7B-shaped set (6.7e9 values) 13.4 -> 11.3 ms a step.  Six waves per SIMD for the update: within 1 % of four,
 // five and seven.
 #include "lpmm_half.hpp"

@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kThreads, LPMM_R1_WAVES) void rank1_update_kernel(c
         uint32_t *red = colred + slot * kRedSlotWords + lane16;
         // folded rows: do the lane's two runs take the second of the two row statistics
         const bool second_a = FOLD == kWraps && (uint32_t)(4 * lane16) >= span.split;
-    const bool second_b = FOLD == kDoubles || (FOLD == kWraps && (uint32_t)(64 + 4 * lane16) >= span.split);
+        const bool second_b = FOLD == kDoubles || (FOLD == kWraps && (uint32_t)(64 + 4 * lane16) >= span.split);
         const uint32_t in_tile = FOLD != kWraps ? 0u : span.first - fold_span(f, q.col_tile * (uint32_t)q.wide).first;
         // a lane keeps its eight columns through all passes: their statistics come out of LDS once
         float co[kEltsPerLane];
@@ -729,8 +729,9 @@ constexpr uint64_t kSpreadBelow = 1024;
 //     50, 59 (1235 workgroups, a fifth more than are resident together), 52; ten of 1001 x 1003 54, 58, 51; but 2001 x 3001 40, 34, 36.
 // The float16 update is bound by its arithmetic, so that large launches take tall tiles, which spread a tile's set-up; small ones
 // leave the chip idle with them.  Update / second pass with tiles of 128, 64, 32, 16 rows: 20 of 4096 x 11008 (902M values) 1323 / 495, 1333 /
-// 518, 1391 / 509, 1507 / 743; 8 of 4096 x 4096 233 / 91, 225 / 90; 4 of them 102 / 47, 97 / 42, 103 / 43 (128 rows all the same:
-// from 26M values on launches keep the groups of kSpreadBelow); one 35.8 / 18.7, 31.1 / 14.0,
+// 518, 1391 / 509, 1507 / 743; 8 of 4096 x 4096 233 / 91, 225 / 90; 4 of them 102 / 47, 97 / 42, 103 / 43 (so that up to
+// some 200M values 64 rows would take 3 to 7 % less; from 26M on the rows are 128 all the same, with which the groups of kSpreadBelow were
+// measured: 6974 x 3840); one 35.8 / 18.7, 31.1 / 14.0,
 // 30.2 / 14.6, 32.6 / 16.4; 24 of 512 x 2048 45.8 / 21.9, 41.5 / 18.3, 42.7 / 19.5; 32 of 256 x 2304 43.6 / 20.7, 35.8 / 15.9, 33.6 / 16.2,
 // 36.6 / 18.4; 8 of 1024 x 1024 28.7 / 16.4, 21.0 / 11.0, 19.0 / 8.9, 19.6 / 10.2; 24 of 512 x 512 27.9 / 15.5, 20.5 / 11.0, 16.5 /
 // 8.3, 15.7 / 7.9; update of 39877 x 128 22.6, 29.0 (a column's row blocks).  Any column count likewise: 2001 x 3001 49.5 / 82, 29.7, 30.2, 30.3 / 35.8;
@@ -877,10 +878,14 @@ static int check_rank1(const Record *tensors, int64_t count, const float *qmap_m
     return LPMM_OK;
 }
 
-// Where the launch that begins with tensors[i] ends: after `most` tensors that are not empty, or, from 48M values on, where tensors that
-// wrap meet others: the kernel for both takes 1 to 3 % longer than the others' own, so that a large launch holds one kind (GPT-2-XL's
+// Where the launch that begins with tensors[i] ends: after `most` tensors that are not empty, or, from 48M values on, where the first of
+// the tensors that wrap meets others or the other way round, double rows among the others.  4-bit first moments in groups of 128: the kernel
+// for both takes 1 to 3 % longer than the others' own, so that a large launch holds one kind (GPT-2-XL's
 // 50257 x 1600 embedding with 31 of its matrices, and too large a launch for the cache: 5255 -> 5207 us a step).  A launch
-// of its own for a few small ones would cost more.
+// of its own for a few small ones would cost more.  The other first moments have no kernel of their own for double rows, and there the line is no
+// better and no worse than one between kernels (double rows among those that wrap).  Steps with this one -> that one, fp32 / 8 bits / groups of 256: eight of
+// 4096 x 4096, then eight of 4096 x 4160 1163 / 995 / 961 -> 1120 / 975 / 921, but four, then two 424 / 367 / 355 -> 426 / 381 / 349; four of 4096 x
+// 4160, then two of 4096 x 4100 443 / 387 / 384 -> 431 / 378 / 371, but eight of each (beyond the cache) 1140 / 996 / 973 -> 1166 / 1009 / 1003.
 template <class Record>
 static int64_t launch_end(const Record *tensors, int64_t i, int64_t count, int most, bool can_fold)
 {
@@ -903,7 +908,7 @@ static int64_t launch_end(const Record *tensors, int64_t i, int64_t count, int m
     return i;
 }
 
-// Validation, batching into launches of at most kR1Max tensors, and the launches.
+// Validation, batching into launches of at most kR1Max tensors (4-bit codes of both moments: kR1Many small ones), and the launches.
 // m_lg: the first moment's group holds 128 << m_lg values (MODE kMCodesWide only).
 // folds: a record per tensor, of ndim 0 where the tensor is a matrix (lpmm_nonfused_adamw4bit_rank1_nd_step_multi).
 // plain: tensors with fp32 states that go with the clearing, as many as its launches take.  wraps: see can_fold_rows.

@@ -158,6 +158,7 @@ __device__ __forceinline__ uint32_t xcd_neighbours(uint32_t index, uint32_t tile
 // four (C is 64 or at least 128).  The record
 // keeps the tensor's own shape (col_blocks = ceil(C / 128), col_tail = C - 128 (col_blocks - 1)); kernels instantiated
 // with FOLD read it this way, tensors with whole column blocks in the same launch as before.
+// Made for tensors of many rows: fewer than 16 rows of the matrix leave its tiles mostly empty (walk.cpp: worth_folding, says which go here).
 // The first moment is then written where it is computed, all tiles but the last are full, and one kind of launch serves nearly every model,
 // where the kernels for any column count (nonfused_rank1_any.hip) and for multiples of 8 (nonfused_rank1_ragged.hip), which split the
 // groups' maxima between rows and write the first moment in the second pass, took 19 bytes a value, launches and new

@@ -217,9 +217,9 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 // Does a matrix gain as rows of 2^lg tensor rows (Fold, rank1_tiles.hpp), which are as many times wider?  The kernels take tiles of 16 such
 // rows and 256 columns: with fewer rows there are up to 32 times as many tiles, and 5.5 ns each, mostly empty.  So it has 16, or at
-// most 512 tiles side by side, which cost less than the host saves.  Steps by the kernels for any column count -> as such rows, us: one of 1 x 1000004 72 -> 701,
-// of 31 x 50004 35 -> 88, of 64 x 50008 32 -> 82; sixteen of 256 x 20004 (8 rows) 384 -> 457, of 512 x 20004 (16) 745 -> 676; of 64 x 5004 (626
-// tiles side by side) 74 -> 94, of 64 x 5008 (313) 42 -> 41, of 64 x 1004 (126) 76 -> 35.
+// most 512 tiles side by side, which cost less than the host saves.  Steps by the kernels for any column count -> as such rows, us:
+// one of 1 x 1000004 72 -> 701, of 31 x 50004 35 -> 88, of 64 x 50008 32 -> 82; sixteen of 256 x 20004 (8 rows) 384 -> 457, of
+// 512 x 20004 (16) 745 -> 676; of 64 x 5004 (626 tiles side by side) 74 -> 94, of 64 x 5008 (313) 42 -> 41, of 64 x 1004 (126) 76 -> 35.
 bool worth_folding(int64_t rows, int64_t cols)
 {
     int lg = 0;
